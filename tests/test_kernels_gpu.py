@@ -516,6 +516,34 @@ def test_gemm_simple(mnk):
     assert np.abs(f64(o2) - ab @ wb.T).max() < 1e-6 * K ** 0.5 * 8
 
 
+# rows at which the kernel or its tile changes, k inside and at the ends of blocks, segments and rounds of
+# segments, workgroups' tiles that end inside the matrix (the last two: tiles of 64 and of 128)
+@pytest.mark.parametrize("mnk", [(1, 7, 256), (8, 23, 260), (9, 33, 2052), (16, 17, 1028), (17, 40, 516), (33, 19, 2304),
+                                 (64, 50, 100), (130, 70, 1540), (130, 4100, 300), (1100, 5570, 68)])
+@pytest.mark.parametrize("types", [("float32", "float32"), ("bfloat16", "float32"), ("bfloat16", "bfloat16")])
+def test_gemm_simple_at_the_edges_of_its_tiles(mnk, types):
+    from transformer_amd import kernels
+    M, N, K = mnk
+    own = np.random.default_rng([M, N, K])
+    a, w = rounded(own.normal(size=(M, K)), types[0]), rounded(own.normal(size=(N, K)), types[1])
+    want = a @ w.T
+    ad, wd = dev(a, DT[types[0]]), dev(w, DT[types[1]])
+    out = torch.full((M, N + 3), 7.0, device=DEV)
+    kernels.gemm_simple(ad, wd, out[:, 1:N + 1])
+    assert np.abs(f64(out[:, 1:N + 1]) - want).max() < 1e-6 * K ** 0.5 * 8
+    assert (out[:, 0] == 7).all() and (out[:, N + 1:] == 7).all()
+    one = torch.empty(1, N, device=DEV)          # the same bits alone, and from rows that start anywhere
+    kernels.gemm_simple(ad[M - 1:], wd, one)
+    assert torch.equal(one[0], out[M - 1, 1:N + 1])
+    odd = torch.empty(M, K + 3, dtype=ad.dtype, device=DEV)[:, 1:K + 1].copy_(ad)
+    got = torch.empty(M, N, device=DEV)
+    kernels.gemm_simple(odd, wd, got)
+    assert torch.equal(got, out[:, 1:N + 1])
+    both = torch.empty(2, M, N, device=DEV)      # side by side
+    kernels.gemm_simple_batched(ad.expand(2, M, K), wd.expand(2, N, K), both)
+    assert torch.equal(both[0], got) and torch.equal(both[1], got)
+
+
 @pytest.mark.parametrize("mnk", [(1, 16, 128), (3, 130, 104), (8, 301, 1000), (16, 48, 4104), (5, 1000, 72),
                                  (8, 16 * 1024 + 5, 2048), (3, 16 * 2050, 1096), (16, 16 * 1030, 4096)])
 @pytest.mark.parametrize("waves", [0, 4, 8, 16])

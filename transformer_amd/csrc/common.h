@@ -111,6 +111,19 @@ __device__ __forceinline__ void ta_sums2(float& w, float& r) {
   r = __uint_as_float(c[1]);
 }
 
+// 16 bytes per lane from memory to LDS without a register in between: lane i's piece lands at `lds` + 16 i (`lds`
+// the same in all lanes). Written as an instruction because the compiler answers its own builtin with a wait for
+// everything in flight before the next read of LDS. The caller waits: ta_wait_loads<n>() until at most n of the
+// wave's loads are on their way, then a barrier; and no wave ends with one still in flight.
+__device__ __forceinline__ void ta_load_to_lds16(const void* src, void* lds) {
+  const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to) : "m0", "memory");
+}
+template <int N>
+__device__ __forceinline__ void ta_wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 // ---------------------------------------------------------------- host side
 int ta_fail(const char* fmt, ...);            // records the message, returns 1
 int ta_check_launch(const char* what);        // hipGetLastError -> message

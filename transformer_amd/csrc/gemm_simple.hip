@@ -1,74 +1,331 @@
-// C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) with float32 accumulation on the vector
-// ALU: the matrix product of the true 32-bit path, and the fallback for storage
-// types and shapes that no faster kernel takes.
+// C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits on the matrix cores: the product of the true
+// 32-bit path, and the fallback for storage types and shapes that no faster kernel takes.
 //
-// Every output element is one chain of fused multiply-adds over k = 0..K-1 in
-// ascending order, whatever M, N or the tiling: a row of A gives the same bits
-// alone or inside any batch.
+// The float32 matrix instructions are chains of fused multiply-adds: v_mfma_f32_16x16x4_f32 and
+// v_mfma_f32_32x32x2_f32 give the bits of fmaf over their 4 (2) k-slots in ascending order, denormals
+// included. Every output element is therefore summed in one order that depends on K alone, whatever
+// M, N, the kernel or the tile:
+//   k is cut into segments of 256 and these into blocks of 16; a segment's chain starts at zero and takes
+//   its blocks in ascending order, and of a block k = 0 4 8 12, 1 5 9 13, 2 6 10 14, 3 7 11 15; the
+//   segments' sums are added in ascending order.
+// So a row of A gives the same bits alone or inside any batch. The order inside a block is the one in
+// which a lane that has read 4 consecutive k holds them: no operand is turned round.
+// Segments (instead of one chain over K) let few rows be split over waves; they also round less.
+//
+// Two kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_tiles: a tile
+// of 128 x 128 or 64 x 64 a workgroup, operands through LDS.
 #include "common.h"
 
-#define BM 64
-#define BN 64
-#define BK 16
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-template <typename T, typename TW, typename TC>
-__global__ __launch_bounds__(256) void gemm_simple_kernel(const T* __restrict__ A, int lda,
-                                                          const TW* __restrict__ W, int ldw,
-                                                          const float* __restrict__ bias,
-                                                          TC* __restrict__ C, int ldc, int M,
-                                                          int N, int K, long long sa, long long sw,
-                                                          long long sc) {
+#define SEG 256      // k per segment
+#define BLK 16       // k per block
+
+__device__ float4 gemm_zeros;      // where a piece past K is read from (never written: zero)
+
+// 4 consecutive k of a row as floats. VEC: rows are 4-element aligned and K is a multiple of 4, so a piece
+// lies wholly inside K or wholly outside. NT: read once, past the caches.
+template <typename T, bool VEC, bool NT>
+__device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
+  if (VEC) {
+    if (sizeof(T) == 4) {
+      const f32x4* p = k < K ? reinterpret_cast<const f32x4*>(row + k) : reinterpret_cast<const f32x4*>(&gemm_zeros);
+      return NT ? __builtin_nontemporal_load(p) : *p;
+    }
+    const u32x2* p = k < K ? reinterpret_cast<const u32x2*>(row + k) : reinterpret_cast<const u32x2*>(&gemm_zeros);
+    const u32x2 v = NT ? __builtin_nontemporal_load(p) : *p;
+    return f32x4{__uint_as_float(v[0] << 16), __uint_as_float(v[0] & 0xffff0000u), __uint_as_float(v[1] << 16),
+                 __uint_as_float(v[1] & 0xffff0000u)};
+  }
+  f32x4 v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = k + j < K ? to_f32(row[k + j]) : 0.f;
+  return v;
+}
+
+// Few rows (up to 16 * RT of them a workgroup), bound by reading W. A lane reads 4 consecutive k of a row of W and
+// of RT rows of A, which are the operands of 4 matrix instructions as they are (a row's four lanes cover 64
+// bytes); while one chunk of BC blocks is multiplied the next is on its way. The waves take the segments in
+// turn and leave the partial tiles in LDS, where they are added in ascending order after every round.
+// 16,384 x 2,048 at 1 / 4 / 16 rows: 30 / 33 / 38 us (4.5 TB/s of W at one row; 220 us by one thread an output on
+// the vector ALU), 2,048 x 8,192: 14.4 / 16.7 / 34.7 us (530).
+// PAIR (up to 8 rows): a matrix instruction multiplies two segments side by side, 8 columns of W each, of
+// whose 16 x 16 products the two squares on the diagonal are used. A workgroup then owns 8 columns: a matrix of
+// 2,048 rows keeps 256 CUs reading instead of 128.
+template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool VEC>
+__global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __restrict__ A, int lda,
+                                                                   const TW* __restrict__ W, int ldw,
+                                                                   const float* __restrict__ bias,
+                                                                   TC* __restrict__ C, int ldc, int M, int N, int K,
+                                                                   long long sa, long long sw, long long sc) {
+  static_assert(!PAIR || RT == 1, "two segments in one tile");
   A += (size_t)blockIdx.z * sa;
   W += (size_t)blockIdx.z * sw;
   C += (size_t)blockIdx.z * sc;
-  __shared__ float As[BK][BM + 4];
-  __shared__ float Ws[BK][BN + 4];
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  float acc[4][4];
+  constexpr int COLS = PAIR ? 8 : 16, ROWS = PAIR ? 8 : 16 * RT;   // of the workgroup's tile
+  constexpr int TURN = PAIR ? 2 * WAVES : WAVES;                   // segments per round
+  constexpr int CPS = SEG / (BC * BLK);                            // chunks per segment
+  constexpr int OUT = (ROWS * COLS + WAVES * 64 - 1) / (WAVES * 64);
+  __shared__ __attribute__((aligned(16))) float part[2][TURN][ROWS * COLS];
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  const int r = lane % 16, kb = lane / 16;
+  const int n0 = blockIdx.x * COLS, m0 = blockIdx.y * ROWS;
+  const int first = PAIR ? 2 * wave + r / 8 : wave;                // this lane's segment of a round
+  // rows past N or M read another row and feed outputs that are never stored
+  const TW* wrow = W + (size_t)(n0 + r % COLS < N ? n0 + r % COLS : N - 1) * ldw;
+  const T* arow[RT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+  for (int i = 0; i < RT; ++i) {
+    const int m = m0 + 16 * i + (PAIR ? r % 8 : r);
+    arow[i] = A + (size_t)(m < M ? m : m0) * lda;
+  }
+  const int segs = (K + SEG - 1) / SEG, rounds = (segs + TURN - 1) / TURN;
 
-  // each thread stages 4 elements of A and 4 of W per k-slab: row = tid / 4, k = (tid % 4) * 4 ..
-  const int lr = threadIdx.x / 4, lk = (threadIdx.x % 4) * 4;
-  for (int k0 = 0; k0 < K; k0 += BK) {
+  f32x4 wreg[2][BC], areg[2][RT][BC];
+  // chunk c of this lane: chunk c % CPS of its segment of round c / CPS; past K: zeros from one address
+  auto load = [&](int set, int c) {
+    const int k0 = ((c / CPS) * TURN + first) * SEG + (c % CPS) * BC * BLK + 4 * kb;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int k = k0 + lk + e;
-      const int am = m0 + lr, wn = n0 + lr;
-      As[lk + e][lr] = (am < M && k < K) ? to_f32(A[(size_t)am * lda + k]) : 0.f;
-      Ws[lk + e][lr] = (wn < N && k < K) ? to_f32(W[(size_t)wn * ldw + k]) : 0.f;
+    for (int i = 0; i < BC; ++i) {
+      wreg[set][i] = load_piece<TW, VEC, (RT < 4)>(wrow, k0 + i * BLK, K);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) areg[set][t][i] = load_piece<T, VEC, false>(arow[t], k0 + i * BLK, K);
+    }
+  };
+  f32x4 acc[RT];
+  auto multiply = [&](int set) {
+#pragma unroll
+    for (int i = 0; i < BC; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wreg[set][i][j], areg[set][t][i][j], acc[t], 0, 0, 0);
+  };
+  float total[OUT];
+#pragma unroll
+  for (int e = 0; e < OUT; ++e) total[e] = 0.f;
+
+  load(0, 0);
+  for (int round = 0; round < rounds; ++round) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    static_assert(CPS % 2 == 0, "chunks of a segment in pairs");
+#pragma unroll
+    for (int c = 0; c < CPS; c += 2) {
+      load(1, round * CPS + c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(0, round * CPS + c + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // a lane holds columns 4 kb .. + 3 of row r of each tile
+    auto* to = part[round & 1];
+    if (PAIR) {
+      if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[first][(r % 8) * 8 + 4 * (kb % 2)]) = acc[0];
+    } else {
+#pragma unroll
+      for (int t = 0; t < RT; ++t) *reinterpret_cast<f32x4*>(&to[wave][t * 256 + r * 16 + 4 * kb]) = acc[t];
     }
     __syncthreads();
+    const int live = segs - round * TURN < TURN ? segs - round * TURN : TURN;
 #pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      float a[4], w[4];
+    for (int e = 0; e < OUT; ++e) {
+      const int at = (int)threadIdx.x + WAVES * 64 * e;
+      if (at < ROWS * COLS)
+        for (int w = 0; w < live; ++w) total[e] += to[w][at];
+    }
+  }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
+  for (int e = 0; e < OUT; ++e) {
+    const int at = (int)threadIdx.x + WAVES * 64 * e;
+    const int m = m0 + at / COLS, n = n0 + at % COLS;
+    if (at < ROWS * COLS && m < M && n < N)
+      C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
+  }
+}
+
+// Many rows, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
+// bytes of operands). 4 waves in 2 x 2 share a tile of 64 TT x 64 TT; each owns TT x TT tiles of 32 x 32. 32 k at a
+// time go through LDS, double buffered: row by row in 8 pieces of 16 bytes, permuted by the row number so that the
+// eight lanes that are served together meet no bank twice. float32 operands go from memory to LDS without passing
+// through registers (a wave's 64 pieces land side by side, so the permutation is in the addresses they are read
+// from); other types are converted on the way. Half h of a wave multiplies pieces h and h + 2 of a block's four,
+// element by element: the order above. 1,021 x 16,384 x 2,048: 548 us (125 TFLOP/s; 630 through registers,
+// 1,880 on the vector ALU); the instruction alone reaches 154.
+template <typename T, typename TW, typename TC, int TT, bool VEC>
+__global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict__ A, int lda,
+                                                            const TW* __restrict__ W, int ldw,
+                                                            const float* __restrict__ bias,
+                                                            TC* __restrict__ C, int ldc, int M, int N, int K,
+                                                            long long sa, long long sw, long long sc) {
+  A += (size_t)blockIdx.z * sa;
+  W += (size_t)blockIdx.z * sw;
+  C += (size_t)blockIdx.z * sc;
+  constexpr bool DIRECT = VEC && sizeof(T) == 4 && sizeof(TW) == 4;
+  constexpr int BT = 64 * TT;                    // rows and columns of the tile
+  constexpr int PER = BT * 8 / 256;              // pieces of an operand that a thread brings
+  constexpr int ST = DIRECT && TT == 1 ? 4 : 2;  // LDS buffers: ST - 1 steps are on their way
+  __shared__ f32x4 As[ST][BT * 8], Ws[ST][BT * 8];
+  const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
+  const int n0 = blockIdx.x * BT, m0 = blockIdx.y * BT;
+  const int lrow = threadIdx.x / 8;              // 32 rows of 128 bytes at a time
+  const int place = threadIdx.x % 8;             // piece of the row in LDS (DIRECT) or in memory
+  const int piece = DIRECT ? place ^ (lrow & 7) : place;
+  const T* asrc[PER];
+  const TW* wsrc[PER];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
+  for (int i = 0; i < PER; ++i) {
+    const int row = lrow + 32 * i;
+    asrc[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda + piece * 4;
+    wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw + piece * 4;
+  }
+  f32x4 ain[DIRECT ? 1 : PER], win[DIRECT ? 1 : PER];
+  // 32 k from k0 on, into LDS buffer `buf` or the registers
+  auto fetch = [&](int buf, int k0) {
+    if constexpr (DIRECT) {
+      const bool whole = k0 + 32 <= K;           // else the last step of a K that is no multiple of 32
+      const bool in = k0 + piece * 4 < K;        // past K: zeros from one address
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < PER; ++i) {
+        const void *a = asrc[i] + k0, *w = wsrc[i] + k0;
+        if (!whole) {
+          a = in ? a : (const void*)&gemm_zeros;
+          w = in ? w : (const void*)&gemm_zeros;
+        }
+        ta_load_to_lds16(a, &As[buf][(32 * i + 8 * wave) * 8]);
+        ta_load_to_lds16(w, &Ws[buf][(32 * i + 8 * wave) * 8]);
+      }
+    } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+      for (int i = 0; i < PER; ++i) {
+        ain[i] = load_piece<T, VEC, false>(asrc[i] - piece * 4, k0 + piece * 4, K);
+        win[i] = load_piece<TW, VEC, false>(wsrc[i] - piece * 4, k0 + piece * 4, K);
+      }
+    }
+  };
+  // the next step's k are in LDS for the whole workgroup, which has done with this step's buffer
+  auto arrive = [&](int buf) {
+    if constexpr (DIRECT) {
+      ta_wait_loads<2 * PER * (ST - 2)>();
+    } else {
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int row = lrow + 32 * i, at = row * 8 + (place ^ (row & 7));
+        As[buf][at] = ain[i];
+        Ws[buf][at] = win[i];
+      }
     }
     __syncthreads();
-  }
+  };
+  const int half = lane / 32, r = lane % 32;
+  const int am = (wave % 2) * 32 * TT + r, wn = (wave / 2) * 32 * TT + r;    // this lane's rows in As and Ws
+  f32x16 total[TT][TT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+  for (int i = 0; i < TT; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float v = acc[i][j];
-      if (bias) v += bias[n];
-      C[(size_t)m * ldc + n] = from_f32<TC>(v);
+    for (int j = 0; j < TT; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) total[i][j][e] = 0.f;
+
+  const int steps = (K + 31) / 32;
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s) fetch(s, (s < steps ? s : steps - 1) * 32);
+  arrive(0);
+  for (int s = 0; s < steps;) {
+    f32x16 acc[TT][TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+      for (int j = 0; j < TT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    const int end = s + SEG / 32 < steps ? s + SEG / 32 : steps;
+    for (; s < end; ++s) {
+      const int buf = s % ST, ahead = s + ST - 1;
+      fetch(ahead % ST, (ahead < steps ? ahead : steps - 1) * 32);      // behind the last step: once more, unused
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        f32x4 a[TT][2], w[TT][2];
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const int at = (4 * b + 2 * p + half) ^ (r & 7);
+            a[i][p] = As[buf][(am + 32 * i) * 8 + at];
+            w[i][p] = Ws[buf][(wn + 32 * i) * 8 + at];
+          }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int x = 0; x < TT; ++x)
+#pragma unroll
+              for (int y = 0; y < TT; ++y)
+                acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x][p][j], w[y][p][j], acc[x][y], 0, 0, 0);
+      }
+      arrive((s + 1) % ST);
     }
+#pragma unroll
+    for (int x = 0; x < TT; ++x)
+#pragma unroll
+      for (int y = 0; y < TT; ++y)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) total[x][y][e] += acc[x][y][e];
   }
+  if constexpr (DIRECT) ta_wait_loads<0>();      // nothing may land in LDS that is another's
+  // accumulator: register e of a lane is row 8 (e / 4) + 4 half + e % 4 of the tile, column r
+#pragma unroll
+  for (int y = 0; y < TT; ++y) {
+    const int n = n0 + wn + 32 * y;
+    if (n >= N) continue;
+    const float add = bias ? bias[n] : 0.f;
+#pragma unroll
+    for (int x = 0; x < TT; ++x)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + (wave % 2) * 32 * TT + 32 * x + 8 * (e / 4) + 4 * half + e % 4;
+        if (m < M) C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[x][y][e] + add : total[x][y][e]);
+      }
+  }
+}
+
+template <typename T, typename TW, typename TC, bool VEC>
+static void launch(hipStream_t stream, const void* A_, int lda, long long sa, const void* W_, int ldw, long long sw,
+                   const float* bias, void* C_, int ldc, long long sc, int M, int N, int K, int batch) {
+  const T* A = (const T*)A_;
+  const TW* W = (const TW*)W_;
+  TC* C = (TC*)C_;
+  auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
+  // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
+  // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 210, 256 rows 170 against 210, 512 rows 209 by tiles
+  // against 340). Tiles of 128 take two workgroups on every CU to fill.
+  if (M > 64 && tiles(64) >= 192) {
+    if (tiles(128) >= 384)
+      gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+    else
+      gemm_tiles_kernel<T, TW, TC, 1, VEC><<<dim3((N + 63) / 64, (M + 63) / 64, batch), 256, 0, stream>>>(
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+    return;
+  }
+#define FEW(WAVES, RT, BC, PAIR)                                                                               \
+  gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, VEC>                                                    \
+      <<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch), WAVES * 64, 0, stream>>>( \
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
+  // four waves a workgroup and 16 KB on their way in each: several workgroups share a CU and fill each other's
+  // starts and ends (16,384 x 2,048 at 16 rows: 38 us; 44 with eight waves and twice the loads)
+  if (M <= 8) FEW(4, 1, 4, true);
+  else if (M <= 16) FEW(4, 1, 4, false);
+  else if (M <= 32) FEW(4, 2, 2, false);
+  else FEW(4, 4, 2, false);
+#undef FEW
 }
 
 // in_dtype: type of A; w_dtype: type of W (a bfloat16 engine keeps a matrix that its file
@@ -82,11 +339,17 @@ extern "C" int ta_gemm_simple_batched(hipStream_t stream, int in_dtype, int w_dt
              "ta_gemm_simple: bad sizes M=%d N=%d K=%d batch=%d", M, N, K, batch);
   TA_REQUIRE(lda >= K && ldw >= K && ldc >= N, "ta_gemm_simple: leading dimensions too small");
   if (M == 0) return 0;
-  dim3 g((N + BN - 1) / BN, (M + BM - 1) / BM, batch), b(256);
-  TA_REQUIRE(g.y <= 65535, "ta_gemm_simple: M=%d too large for one launch", M);
-#define LAUNCH(T, TW, TC)                                                                        \
-  gemm_simple_kernel<T, TW, TC><<<g, b, 0, stream>>>((const T*)A, lda, (const TW*)W, ldw, bias,   \
-                                                     (TC*)C, ldc, M, N, K, sa, sw, sc)
+  TA_REQUIRE((M + 63) / 64 <= 65535 && K <= (1 << 30), "ta_gemm_simple: M=%d K=%d too large for one launch", M, K);
+  // rows that start on 4 elements and hold whole pieces of 4
+  auto aligned = [&](const void* p, int dtype, long long ld, long long stride) {
+    return (uintptr_t)p % (dtype == TA_F32 ? 16 : 8) == 0 && ld % 4 == 0 && stride % 4 == 0;
+  };
+  const bool vec = K % 4 == 0 && aligned(A, in_dtype, lda, sa) && aligned(W, w_dtype, ldw, sw);
+#define LAUNCH(T, TW, TC)                                                                                   \
+  do {                                                                                                      \
+    if (vec) launch<T, TW, TC, true>(stream, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch);     \
+    else launch<T, TW, TC, false>(stream, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch);        \
+  } while (0)
   if (in_dtype == TA_F32 && w_dtype == TA_F32 && out_dtype == TA_F32) LAUNCH(float, float, float);
   else if (in_dtype == TA_BF16 && w_dtype == TA_BF16 && out_dtype == TA_BF16) LAUNCH(bf16_t, bf16_t, bf16_t);
   else if (in_dtype == TA_BF16 && w_dtype == TA_BF16 && out_dtype == TA_F32) LAUNCH(bf16_t, bf16_t, float);

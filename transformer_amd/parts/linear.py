@@ -1,8 +1,9 @@
 """y = x @ W^T, the matrix product every part uses.
 
 float32 engine: the hand-written product of csrc/gemm_simple.hip, whose every
-output element is one ascending-k chain of fused multiply-adds; no library and
-no reduced-precision matrix mode is involved anywhere in that path.
+output element is summed by fused multiply-adds in one order that depends on k
+alone; no library and no reduced-precision matrix mode is involved anywhere in
+that path.
 
 bfloat16 engine: the vendor library through ``torch.mm`` (the reference's
 engine also hands its products to a library: the external ``mat_mul`` operator,
