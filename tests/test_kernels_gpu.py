@@ -235,6 +235,78 @@ def test_attention_generic(dtype, shape):
     assert np.abs(got - want).max() < tol(dtype)
 
 
+# nh, nkv, dk, dv, lengths of the caches, (softcap, sink, gate, window, keep_first, chunk): both kinds of widths of
+# each kernel, groups of 1, 5 and 20 heads, ends on and off a page's edge, every option
+F32_SHAPES = [
+    (8, 2, 128, 128, [1, 64, 65, 300, 700], {}),
+    (4, 4, 64, 64, [127, 128, 640], {"softcap": 5.0, "sink": "unit"}),
+    (5, 1, 48, 16, [33, 200], {"window": 70, "keep_first": 5, "sink": "learned", "gate": True}),
+    (20, 1, 96, 112, [10, 190], {"chunk": 50, "gate": True}),
+    (6, 3, 16, 128, [130, 512], {"window": 64}),
+]
+
+
+@pytest.mark.parametrize("shape", F32_SHAPES, ids=[f"h{s[0]}kv{s[1]}k{s[2]}v{s[3]}" for s in F32_SHAPES])
+def test_float32_attention_page_by_page(shape):
+    """A sequence's last tokens, as a prompt that continues it and one by one with and without scratch: the same
+    bits, and the plain attention's numbers. Cache places behind the end hold NaN."""
+    from transformer_amd import kernels
+    from transformer_amd.parts.linear import Workspace
+    nh, nkv, dk, dv, lengths, opt = shape
+    own = np.random.default_rng([nh, dk, dv])
+    group, B, tail = nh // nkv, len(lengths), 3
+    tails = [min(tail, n) for n in lengths]
+    need = [-(-n // 64) for n in lengths]
+    order = own.permutation(sum(need) + 2)
+    table = np.zeros((B, max(need) + 1), dtype=np.int32)
+    kc, vc = np.full((len(order), nkv, 64, dk), np.nan), np.full((len(order), nkv, dv, 64), np.nan)
+    ks, vs, used = [], [], 0
+    for b, n in enumerate(lengths):
+        table[b, :need[b]] = order[used:used + need[b]]
+        used += need[b]
+        ks.append(own.normal(size=(n, nkv, dk)).astype(np.float32)); vs.append(own.normal(size=(n, nkv, dv)).astype(np.float32))
+        for p in range(n):
+            kc[table[b, p // 64], :, p % 64], vc[table[b, p // 64], :, :, p % 64] = ks[b][p], vs[b][p]
+    nt = sum(tails)
+    q, g = own.normal(size=(nt, nh * dk)).astype(np.float32), own.normal(size=(nt, nh * dv)).astype(np.float32)
+    learned = own.normal(size=nh).astype(np.float32)
+    sink = {"unit": "unit", "learned": dev(learned), None: None}[opt.get("sink")]
+    scale = 1.5 / math.sqrt(dk)
+
+    def step(rows, counts, before, ws):
+        out = torch.full((len(rows), nh * dv), float("nan"), device=DEV)
+        cu = np.concatenate([[0], np.cumsum(counts)])
+        kernels.attention_sink(dev(q[rows]), out, dev(kc), dev(vc), dev(table, torch.int32), dev(cu, torch.int32),
+                               dev(before, torch.int32), max(counts), nh, nkv, dk, dv, scale, opt.get("window"),
+                               opt.get("softcap"), sink, dev(g[rows]) if opt.get("gate") else None,
+                               keep_first=opt.get("keep_first", 0), chunk=opt.get("chunk"), ws=ws)
+        return out
+
+    start = np.concatenate([[0], np.cumsum(tails)])
+    whole = step(list(range(nt)), tails, [n - t for n, t in zip(lengths, tails)], None)
+    # the last token of each, its pages in waves of their own, and by the prompts' kernel
+    rows = [int(start[b + 1]) - 1 for b in range(B)]
+    for ws in (Workspace(DEV), None):
+        alone = step(rows, [1] * B, [n - 1 for n in lengths], ws)
+        assert torch.equal(alone, whole[rows])
+    for b, n in enumerate(lengths):
+        for i in range(tails[b]):
+            at, row = n - tails[b] + i, int(start[b]) + i
+            j = np.arange(n)
+            first = at // opt["chunk"] * opt["chunk"] if "chunk" in opt else max(0, at + 1 - opt.get("window", n))
+            see = (j <= at) & ((j >= first) | (j < opt.get("keep_first", 0)))
+            for h in range(nh):
+                x = ks[b][:, h // group].astype(np.float64) @ q[row, h * dk:(h + 1) * dk] * scale
+                if "softcap" in opt:
+                    x = opt["softcap"] * np.tanh(x / opt["softcap"])
+                e = np.where(see, np.exp(x), 0.0)
+                total = e.sum() + {"unit": 1.0, "learned": np.exp(float(learned[h])), None: 0.0}[opt.get("sink")]
+                want = (e / total) @ vs[b][:, h // group]
+                if opt.get("gate"):
+                    want = want / (1 + np.exp(-g[row, h * dv:(h + 1) * dv].astype(np.float64)))
+                assert np.abs(f64(whole[row, h * dv:(h + 1) * dv]) - want).max() < 2e-5
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_attention_far_key_among_hundreds(dtype):
     # sequence 1, its only query, key 3 of 800, head 5: the output must be that key's value

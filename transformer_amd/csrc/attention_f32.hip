@@ -1,0 +1,384 @@
+// Causal grouped-query attention over the paged cache in 32 bits on the matrix cores, for key and value
+// widths that are multiples of 16 up to 128: what attention_generic.hip computes, options included, for the
+// float32 engine's usual heads (other widths and storage types stay there).
+//
+// The float32 matrix instructions are chains of fused multiply-adds, so a row's result can be defined
+// without them: pages of 64 keys are taken one by one, each with a maximum, a sum of exponentials and a sum
+// of values of its own, and joined in ascending order:
+//   M' = max(M, m), a = exp(M - M'), b = exp(m - M'); L = b l + a L; O = b o + a O.
+// A page's numbers depend on the row's query and that page alone. So they may be formed anywhere: prompts walk
+// a row's pages in one wave, single tokens hand every page to a wave of its own and join the pages in a second
+// kernel, and both give the same bits, whatever the batch and the cut into steps.
+//
+// 16 rows (query token, query head of the kv head's group) a wave, v_mfma_f32_16x16x4_f32. Lane (r, kb), r < 16,
+// kb < 4: scores K Q^T leave it row r's keys 16 t + 4 kb + i (t, i < 4), which is the layout in which the second
+// product V^T P^T wants the weights; both operands of either product are runs of 4 consecutive numbers of a key
+// or value row.
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct F32Attention {
+  const float* q;
+  float* out;
+  const float *k, *v;          // one layer: [pages][nkv][64][dh], [pages][nkv][dv][64]
+  const int *table, *cu_q, *pos0;
+  const float *sink, *gate;
+  float* parts;                // single tokens: [B][nh][max_blocks][dv] sums, then [B][nh][max_blocks][2] maxima and sums
+  int q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window, sink_mode, gate_stride, gate_dv, keep, chunk;
+  float scale, softcap;
+};
+
+// what a row sees: keys start .. end - 1 and the first `keep`
+struct Span {
+  int start, end, keep;
+  __device__ __forceinline__ bool key(int k) const { return (k >= start || k < keep) && k < end; }
+  __device__ __forceinline__ bool page(int p) const { return p * 64 < end && (p * 64 + 64 > start || p * 64 < keep); }
+};
+
+template <int NB, bool EXACT, typename KF>
+__device__ __forceinline__ void page_scores(const f32x4* qf, int nb, KF kfrag, f32x4* s) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+    if (EXACT || d < nb) {
+      f32x4 k[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) k[t] = kfrag(t, d);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][j], qf[d][j], s[t], 0, 0, 0);
+    }
+}
+
+// scores -> weights relative to the page's maximum m, and their sum l
+__device__ __forceinline__ void page_softmax(const F32Attention& p, const Span& see, int key0, f32x4* s, float& m, float& l) {
+  m = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x = s[t][i] * p.scale;
+      if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
+      s[t][i] = see.key(key0 + 16 * t + i) ? x : -INFINITY;
+      m = fmaxf(m, s[t][i]);
+    }
+  m = fmaxf(m, __shfl_xor(m, 16, TA_WAVE));
+  m = fmaxf(m, __shfl_xor(m, 32, TA_WAVE));
+  l = 0.f;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s[t][i] = s[t][i] == -INFINITY ? 0.f : expf(s[t][i] - m);
+      l += s[t][i];
+    }
+  l += __shfl_xor(l, 16, TA_WAVE);
+  l += __shfl_xor(l, 32, TA_WAVE);
+}
+
+// o[d] = the page's sum of values, columns 16 d + 4 kb + i of row r. Keys from `live` on (of the page) were never
+// written and count as zero.
+template <int NB, bool EXACT, typename VF>
+__device__ __forceinline__ void page_values(const f32x4* e, int nb, int live, int kb, VF vfrag, f32x4* o) {
+#pragma unroll
+  for (int d = 0; d < NB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int d = 0; d < NB; ++d)
+      if (EXACT || d < nb) {
+        f32x4 v = vfrag(t, d);
+        if (live < 64) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = 16 * t + 4 * kb + j < live ? v[j] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], e[t][j], o[d], 0, 0, 0);
+      }
+}
+
+// factors with which what was joined so far and a page's numbers enter the sums
+__device__ __forceinline__ void join(float& M, float m, float& a, float& b) {
+  const float n = fmaxf(M, m);
+  a = M == n ? 1.f : expf(M - n);
+  b = m == n ? 1.f : expf(m - n);
+  M = n;
+}
+
+// what stands between the sums and the result: the sink's term, the division, a gate per head
+__device__ __forceinline__ float last_factor(const F32Attention& p, float M, float L, int head, size_t token, float& rescale) {
+  rescale = 1.f;
+  if (p.sink_mode != 0) {
+    const float sv = p.sink_mode == 2 ? p.sink[head] : 0.f;
+    const float n = fmaxf(M, sv);
+    rescale = expf(M - n);               // M = -inf (no key seen) gives 0
+    L = L * rescale + expf(sv - n);
+  }
+  float inv = L > 0.f ? 1.0f / L : 0.f;
+  if (p.gate && p.gate_dv == 0) inv *= 1.0f / (1.0f + expf(-p.gate[token * p.gate_stride + head]));
+  return inv;
+}
+__device__ __forceinline__ float gated(const F32Attention& p, float x, int head, size_t token, int col) {
+  if (p.gate && col < p.gate_dv) x *= 1.0f / (1.0f + expf(-p.gate[token * p.gate_stride + (size_t)head * p.gate_dv + col]));
+  return x;
+}
+
+// Prompts: 64 rows of one (sequence, kv head) a workgroup, 16 a wave; a page's keys and its values go through LDS
+// once for the four. The next page's keys are on their way during the softmax and the second product, its values
+// during the next scores; two workgroups share a CU. Bound by the matrix instructions: 256 of 32 cycles per
+// page and wave. 1,021 tokens, 16 heads of 128 over 4 kv heads: 102 us (807 on the vector ALU).
+template <int NB, bool EXACT>
+__global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32Attention p) {
+  __shared__ f32x4 Ks[64 * 4 * NB], Vs[16 * NB * 16];
+  const int group = p.nh / p.nkv, b = blockIdx.z, kvh = blockIdx.y;
+  const int q0 = p.cu_q[b], qlen = p.cu_q[b + 1] - q0, nrows = qlen * group;
+  const int blocks = (nrows + 63) / 64;
+  if ((int)blockIdx.x >= blocks) return;
+  const int row0 = (blocks - 1 - (int)blockIdx.x) * 64;            // the longest first
+  const int pos0 = p.pos0[b];
+  const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE, r = lane % 16, kb = lane / 16;
+  const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
+
+  const int last = row0 + 63 < nrows - 1 ? row0 + 63 : nrows - 1;
+  const Span all = {ta_first_key(pos0 + row0 / group + 1, p.window, p.chunk), pos0 + last / group + 1, p.keep};
+  const int row = row0 + 16 * wave + r;
+  const bool ok = row < nrows;
+  const int qi = ok ? row / group : 0, head = kvh * group + (ok ? row % group : 0);
+  Span see = {ta_first_key(pos0 + qi + 1, p.window, p.chunk), pos0 + qi + 1, p.keep};
+  if (!ok) see = {0, 0, 0};
+  // the wave's own rows
+  const int wfirst = row0 + 16 * wave, wlast = wfirst + 15 < nrows - 1 ? wfirst + 15 : nrows - 1;
+  const bool wlive = wfirst < nrows;
+  const Span mine = {ta_first_key(pos0 + wfirst / group + 1, p.window, p.chunk), wlive ? pos0 + wlast / group + 1 : 0, p.keep};
+
+  f32x4 qf[NB], O[NB];
+  const float* qrow = p.q + (size_t)(q0 + qi) * p.q_stride + (size_t)head * p.dh;
+#pragma unroll
+  for (int d = 0; d < NB; ++d) {
+    if (EXACT || d < nkb) qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
+    O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  float M = -INFINITY, L = 0.f;
+
+  // pieces of 16 bytes, permuted inside a row by the row's number
+  const int* table = p.table + (size_t)b * p.max_blocks;
+  const int kper = 4 * nkb, kmask = nkb % 4 == 0 ? 15 : nkb % 2 == 0 ? 7 : 3;
+  auto bring_keys = [&](int page) {
+    const float* from = p.k + ((size_t)table[page] * p.nkv + kvh) * 64 * p.dh;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (EXACT || i < nkb) {
+        const int at = i * 256 + (int)threadIdx.x, row_ = at / kper, piece = (at - row_ * kper) ^ (row_ & kmask);
+        ta_load_to_lds16(from + (size_t)row_ * p.dh + piece * 4, &Ks[i * 256 + wave * 64]);
+      }
+  };
+  auto bring_values = [&](int page) {
+    const float* from = p.v + ((size_t)table[page] * p.nkv + kvh) * 64 * p.dv;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      if (EXACT || i < nvb) {
+        const int at = i * 256 + (int)threadIdx.x, row_ = at / 16, piece = (at % 16) ^ (row_ & 15);
+        ta_load_to_lds16(from + (size_t)row_ * 64 + piece * 4, &Vs[i * 256 + wave * 64]);
+      }
+  };
+  auto next_page = [&](int page) {
+    do ++page; while (page * 64 < all.end && !all.page(page));
+    return page;
+  };
+
+  int page = next_page(-1);
+  bring_keys(page);
+  bring_values(page);
+  while (page * 64 < all.end) {
+    const int next = next_page(page);
+    const bool more = next * 64 < all.end;
+    const bool use = mine.page(page);
+    // the keys have come: they were asked for before the values
+    if (EXACT) ta_wait_loads<NB>(); else ta_wait_loads<0>();
+    __syncthreads();
+    f32x4 s[4];
+    if (use) {
+      page_scores<NB, EXACT>(qf, nkb, [&](int t, int d) {
+        return Ks[(16 * t + r) * kper + ((4 * d + kb) ^ (r & kmask))];
+      }, s);
+    }
+    __syncthreads();                               // everybody has done with the keys
+    if (more) bring_keys(next);
+    float m = -INFINITY, l = 0.f;
+    if (use) page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
+    if (EXACT && more) ta_wait_loads<NB>(); else ta_wait_loads<0>();          // the values
+    __syncthreads();
+    f32x4 o[NB];
+    if (use) {
+      const int live = all.end - page * 64;
+      page_values<NB, EXACT>(s, nvb, live, kb, [&](int t, int d) {
+        return Vs[(16 * d + r) * 16 + ((4 * t + kb) ^ r)];
+      }, o);
+    }
+    __syncthreads();                               // everybody has done with the values
+    if (more) bring_values(next);
+    if (use) {
+      float a, c;
+      join(M, m, a, c);
+      L = fmaf(l, c, L * a);
+#pragma unroll
+      for (int d = 0; d < NB; ++d)
+        if (EXACT || d < nvb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) O[d][i] = fmaf(o[d][i], c, O[d][i] * a);
+    }
+    page = next;
+  }
+  if (!ok) return;
+  const size_t token = (size_t)(q0 + qi);
+  float rescale;
+  const float inv = last_factor(p, M, L, head, token, rescale);
+  float* orow = p.out + token * p.out_stride + (size_t)head * p.dv;
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+    if (EXACT || d < nvb) {
+      f32x4 x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = gated(p, O[d][i] * rescale * inv, head, token, 16 * d + 4 * kb + i);
+      *reinterpret_cast<f32x4*>(orow + 16 * d + 4 * kb) = x;
+    }
+}
+
+// Single tokens: a wave takes one page of one (sequence, kv head, 16 of the group's heads), operands straight from
+// memory: all of a page's 64 KB are asked for at once. Pages the sequence does not have end at once: the grid
+// follows the page table's width, so that a recorded launch fits every length. 4 sequences of 50 to 300 keys, 16
+// heads over 4 kv heads: 14.3 us and 4.7 to join (279 by one workgroup per sequence and kv head).
+template <int NB, bool EXACT>
+__global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
+  const int group = p.nh / p.nkv, tiles = (group + 15) / 16, b = blockIdx.z, kvh = blockIdx.y / tiles, h0 = blockIdx.y % tiles * 16;
+  const int lane = threadIdx.x % TA_WAVE, r = lane % 16, kb = lane / 16;
+  const int page = blockIdx.x * 4 + threadIdx.x / TA_WAVE;
+  const int end = p.pos0[b] + 1;
+  Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
+  if (page >= p.max_blocks || !see.page(page)) return;
+  const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
+  const bool ok = h0 + r < group;
+  const int head = kvh * group + (ok ? h0 + r : 0);
+  const size_t at = ((size_t)p.table[(size_t)b * p.max_blocks + page] * p.nkv + kvh) * 64;
+  const float *kp = p.k + at * p.dh, *vp = p.v + at * p.dv;
+  const float* qrow = p.q + (size_t)p.cu_q[b] * p.q_stride + (size_t)head * p.dh;
+  f32x4 kf[4][NB], vf[4][NB], qf[NB];
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+    if (EXACT || d < nkb) {
+      qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) kf[t][d] = *reinterpret_cast<const f32x4*>(kp + (size_t)(16 * t + r) * p.dh + 16 * d + 4 * kb);
+    }
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int d = 0; d < NB; ++d)
+      if (EXACT || d < nvb) vf[t][d] = *reinterpret_cast<const f32x4*>(vp + (size_t)(16 * d + r) * 64 + 16 * t + 4 * kb);
+  __builtin_amdgcn_sched_barrier(0);               // or the values are asked for behind the scores
+  f32x4 s[4], o[NB];
+  float m, l;
+  page_scores<NB, EXACT>(qf, nkb, [&](int t, int d) { return kf[t][d]; }, s);
+  page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
+  page_values<NB, EXACT>(s, nvb, end - page * 64, kb, [&](int t, int d) { return vf[t][d]; }, o);
+  if (!ok) return;
+  const size_t unit = ((size_t)b * p.nh + head) * p.max_blocks + page;
+  float* sums = p.parts + unit * p.dv;
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+    if (EXACT || d < nvb) *reinterpret_cast<f32x4*>(sums + 16 * d + 4 * kb) = o[d];
+  if (kb == 0) {
+    float* ml = p.parts + (size_t)gridDim.z * p.nh * p.max_blocks * p.dv + unit * 2;
+    ml[0] = m;
+    ml[1] = l;
+  }
+}
+
+// The pages of a single token's row joined in ascending order, eight asked for at a time; a thread a column.
+__global__ __launch_bounds__(128) void attn_f32_join_kernel(F32Attention p) {
+  const int head = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+  const int end = p.pos0[b] + 1;
+  const Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
+  const size_t unit = ((size_t)b * p.nh + head) * p.max_blocks;
+  const float* sums = p.parts + unit * p.dv;
+  const float* ml = p.parts + (size_t)gridDim.y * p.nh * p.max_blocks * p.dv + unit * 2;
+  const int pages = (end + 63) / 64 < p.max_blocks ? (end + 63) / 64 : p.max_blocks;
+  float M = -INFINITY, L = 0.f, O = 0.f;
+  for (int p0 = 0; p0 < pages; p0 += 8) {
+    float o[8], m[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bool in = p0 + i < pages && see.page(p0 + i);
+      const int at = in ? p0 + i : pages - 1;        // the last page is always seen
+      o[i] = sums[(size_t)at * p.dv + (d < p.dv ? d : 0)];
+      m[i] = ml[2 * at];
+      l[i] = ml[2 * at + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (p0 + i < pages && see.page(p0 + i)) {
+        float a, c;
+        join(M, m[i], a, c);
+        L = fmaf(l[i], c, L * a);
+        O = fmaf(o[i], c, O * a);
+      }
+  }
+  if (d >= p.dv) return;
+  const size_t token = (size_t)p.cu_q[b];
+  float rescale;
+  const float inv = last_factor(p, M, L, head, token, rescale);
+  p.out[token * p.out_stride + (size_t)head * p.dv + d] = gated(p, O * rescale * inv, head, token, d);
+}
+
+// Floats of scratch that ta_attention_f32 wants for a step of single tokens.
+extern "C" long long ta_attention_f32_scratch(int batch, int nh, int max_blocks, int dv) {
+  return (long long)batch * nh * max_blocks * (dv + 2);
+}
+
+// As ta_attention_generic_sink, float32, dh and dv multiples of 16 up to 128, rows that start on 16 bytes. parts:
+// scratch of ta_attention_f32_scratch floats for steps in which every sequence brings one token (max_qlen 1), or
+// null: the kernel for prompts then serves these too, with the same bits.
+extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride, void* out, int out_stride,
+                                const void* kcache, const void* vcache, const int* block_table, int max_blocks,
+                                const int* cu_q, const int* pos0, int batch, int max_qlen, int nh, int nkv, int dh,
+                                int dv, float scale, int window, float softcap, int sink_mode, const float* sink,
+                                const void* gate, int gate_stride, int gate_dv, int keep, int chunk, float* parts) {
+  TA_REQUIRE(batch >= 0 && max_qlen >= 0, "ta_attention_f32: bad batch=%d max_qlen=%d", batch, max_qlen);
+  TA_REQUIRE(sink_mode >= 0 && sink_mode <= 2 && (sink_mode != 2 || sink != nullptr) && softcap >= 0.f,
+             "ta_attention_f32: sink mode %d, cap %f", sink_mode, softcap);
+  TA_REQUIRE(gate == nullptr || (gate_dv >= 0 && gate_dv <= dv && gate_stride >= nh * (gate_dv > 0 ? gate_dv : 1)),
+             "ta_attention_f32: gate rows of %d", gate_stride);
+  TA_REQUIRE(keep >= 0 && (keep == 0 || window > 0), "ta_attention_f32: %d kept keys beside a window of %d", keep, window);
+  TA_REQUIRE(chunk >= 0 && (chunk == 0 || window <= 0), "ta_attention_f32: chunks of %d beside a window of %d", chunk, window);
+  TA_REQUIRE(nh > 0 && nkv > 0 && nh % nkv == 0, "ta_attention_f32: %d heads do not divide into %d kv heads", nh, nkv);
+  TA_REQUIRE(dh % 16 == 0 && dh >= 16 && dh <= 128 && dv % 16 == 0 && dv >= 16 && dv <= 128,
+             "ta_attention_f32: key width %d / value width %d", dh, dv);
+  TA_REQUIRE(q_stride >= nh * dh && out_stride >= nh * dv && q_stride % 4 == 0 && out_stride % 4 == 0 &&
+                 ((uintptr_t)q | (uintptr_t)out | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)parts) % 16 == 0,
+             "ta_attention_f32: rows of %d and %d floats or their start", q_stride, out_stride);
+  TA_REQUIRE(max_blocks > 0 && batch <= 65535 && (long long)nkv * ((nh / nkv + 15) / 16) <= 65535,
+             "ta_attention_f32: grid of %d sequences, %d kv heads, %d pages", batch, nkv, max_blocks);
+  if (batch == 0 || max_qlen == 0) return 0;
+  const F32Attention p = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, cu_q, pos0,
+                          sink, (const float*)gate, parts, q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window,
+                          sink_mode, gate_stride, gate_dv, keep, chunk, scale, softcap};
+  const int group = nh / nkv, most = dh > dv ? dh : dv;
+#define PICK(kernel, grid)                                                        \
+  do {                                                                            \
+    if (dh == 128 && dv == 128) kernel<8, true><<<grid, 256, 0, stream>>>(p);     \
+    else if (dh == 64 && dv == 64) kernel<4, true><<<grid, 256, 0, stream>>>(p);  \
+    else if (most <= 64) kernel<4, false><<<grid, 256, 0, stream>>>(p);           \
+    else kernel<8, false><<<grid, 256, 0, stream>>>(p);                           \
+  } while (0)
+  if (max_qlen == 1 && parts != nullptr) {
+    PICK(attn_f32_pages_kernel, dim3((max_blocks + 3) / 4, nkv * ((group + 15) / 16), batch));
+    attn_f32_join_kernel<<<dim3(nh, batch), 128, 0, stream>>>(p);
+  } else {
+    PICK(attn_f32_rows_kernel, dim3((unsigned)(((long long)max_qlen * group + 63) / 64), nkv, batch));
+  }
+#undef PICK
+  return ta_check_launch("ta_attention_f32");
+}

@@ -1,6 +1,7 @@
 // Causal grouped-query attention over the paged cache, float32 arithmetic on the
 // vector ALU, for any key width and any value width up to 256 (the two may differ)
-// and both storage types. It serves prompts and single tokens alike.
+// and both storage types. It serves prompts and single tokens alike. (float32 heads whose widths are multiples
+// of 16 up to 128 go to attention_f32.hip.)
 //
 // A workgroup owns 16 "rows" of one (sequence, kv head): row = (query token,
 // query head inside the kv head's group), so the heads of a group share every

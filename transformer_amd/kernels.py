@@ -214,8 +214,10 @@ def rope_kv_write(qkv: torch.Tensor, num_q_heads: int, num_kv_heads: int, head_d
 def attention_generic(q: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor,
                       vcache: torch.Tensor, block_table: torch.Tensor, cu_q: torch.Tensor,
                       pos0: torch.Tensor, max_qlen: int, num_heads: int, num_kv_heads: int,
-                      head_dim: int, scale: float, window: Optional[int] = None):
-    """Causal attention of each sequence's new tokens over its cached keys.
+                      head_dim: int, scale: float, window: Optional[int] = None, ws=None):
+    """Causal attention of each sequence's new tokens over its cached keys, in 32 bits. ws: a
+    workspace for the partial rows of a float32 step of single tokens (without one such a step
+    runs the prompts' kernel, with the same bits).
 
     q: [nt, >= nh*dh] (a view whose rows may be wider, e.g. the qkv buffer);
     out: [nt, nh*dh]; kcache [pages, nkv, PAGE, dh], vcache [pages, nkv, dh, PAGE];
@@ -234,6 +236,9 @@ def attention_generic(q: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor,
     B = pos0.numel()
     if cu_q.numel() != B + 1 or block_table.dim() != 2 or block_table.shape[0] != B:
         raise KernelError("attention: cu_q / pos0 / block_table disagree about the batch size")
+    if f32_attention_takes(q, out, kcache, vcache, head_dim, head_dim):
+        return _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads,
+                              num_kv_heads, head_dim, head_dim, scale, window, ws)
     _check(library().ta_attention_generic(
         _stream(), c_int(_code(q.dtype)), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache),
         _ptr(vcache), _ptr(block_table), c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0),
@@ -242,12 +247,43 @@ def attention_generic(q: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor,
     return out
 
 
+def f32_attention_takes(q, out, kcache, vcache, key_dim: int, value_dim: int) -> bool:
+    """Whether the 32-bit matrix-core attention takes these heads: float32, key and value widths that are
+    multiples of 16 up to 128 (a page's keys and values then fit 64 KB of LDS), rows on 16 bytes. The widths
+    decide for a model once and for all, so that its prompts and its single tokens give the same bits; a step
+    of the engine brings rows that qualify whenever the widths do."""
+    return q.dtype == torch.float32 and key_dim % 16 == 0 and 16 <= key_dim <= 128 and value_dim % 16 == 0 \
+        and 16 <= value_dim <= 128 and q.stride(0) % 4 == 0 and out.stride(0) % 4 == 0 \
+        and all(t.data_ptr() % 16 == 0 for t in (q, out, kcache, vcache))
+
+
+# the most partial rows that a float32 step of single tokens leaves in its workspace (floats)
+_F32_PARTS = 1 << 26
+
+
+def _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads, num_kv_heads, key_dim,
+                   value_dim, scale, window, ws, cap=0.0, mode=0, sink=None, gate=None, gs=0, gd=0, keep=0, chunk=0):
+    B, parts = pos0.numel(), None
+    if max_qlen == 1 and ws is not None:
+        need = library().ta_attention_f32_scratch
+        need.restype = c_longlong
+        floats = need(c_int(B), c_int(num_heads), c_int(block_table.shape[1]), c_int(value_dim))
+        if floats <= _F32_PARTS:
+            parts = ws.take("attention.f32_parts", (floats,), torch.float32)
+    _check(library().ta_attention_f32(
+        _stream(), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache), _ptr(vcache), _ptr(block_table),
+        c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0), c_int(B), c_int(max_qlen), c_int(num_heads),
+        c_int(num_kv_heads), c_int(key_dim), c_int(value_dim), c_float(scale), c_int(window or 0), c_float(cap),
+        c_int(mode), _ptr(sink), _ptr(gate), c_int(gs), c_int(gd), c_int(keep), c_int(chunk), _ptr(parts)))
+    return out
+
+
 def attention(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, max_kv_len, num_heads,
-              num_kv_heads, head_dim, scale, window=None):
+              num_kv_heads, head_dim, scale, window=None, ws=None):
     """Picks the attention kernel for the step's shape and storage type: bfloat16
     with a head size that is a multiple of 32 runs on the matrix cores (one kernel
     for prompts, one for single tokens that slices the keys); everything else, and
-    all of float32, runs the vector-ALU kernel."""
+    all of float32, runs the 32-bit kernels (``attention_generic``, which is given ``ws``)."""
     if q.dtype == torch.bfloat16 and head_dim % 32 == 0 and 32 <= head_dim <= 256:
         if max_qlen == 1 and keys_kernel_fits(num_heads, num_kv_heads, head_dim):
             return attention_keys(q, out, kcache, vcache, block_table, cu_q, pos0, max_kv_len,
@@ -255,7 +291,7 @@ def attention(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, max_kv_
         return attention_rows(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen,
                               num_heads, num_kv_heads, head_dim, scale, window)
     return attention_generic(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads,
-                             num_kv_heads, head_dim, scale, window)
+                             num_kv_heads, head_dim, scale, window, ws)
 
 
 def _attention_args(q, out, kcache, vcache, block_table, cu_q, pos0, num_heads, num_kv_heads,
@@ -1091,7 +1127,7 @@ def qk_prepare(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, key_dim: in
 
 
 def attention_generic_dv(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads,
-                         num_kv_heads, key_dim, value_dim, scale, window=None):
+                         num_kv_heads, key_dim, value_dim, scale, window=None, ws=None):
     """``attention_generic`` for values of another width than the keys: q [nt, >= nh*dk],
     out [nt, nh*dv], kcache [pages, nkv, PAGE, dk], vcache [pages, nkv, dv, PAGE]."""
     _dev(q, "q", contiguous=False); _dev(out, "out", q.dtype, contiguous=False)
@@ -1107,6 +1143,9 @@ def attention_generic_dv(q, out, kcache, vcache, block_table, cu_q, pos0, max_ql
     B = pos0.numel()
     if cu_q.numel() != B + 1 or block_table.dim() != 2 or block_table.shape[0] != B:
         raise KernelError("attention: cu_q / pos0 / block_table disagree about the batch size")
+    if f32_attention_takes(q, out, kcache, vcache, key_dim, value_dim):
+        return _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads,
+                              num_kv_heads, key_dim, value_dim, scale, window, ws)
     _check(library().ta_attention_generic_dv(
         _stream(), c_int(_code(q.dtype)), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache),
         _ptr(vcache), _ptr(block_table), c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0),
@@ -1835,7 +1874,7 @@ def qk_rotate_store(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, key_di
 def attention_sink(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads, num_kv_heads, key_dim,
                    value_dim, scale, window=None, softcap: Optional[float] = None, sink=None,
                    gate: Optional[torch.Tensor] = None, gate_dim: Optional[int] = None, keep_first: int = 0,
-                   chunk: Optional[int] = None):
+                   chunk: Optional[int] = None, ws=None):
     """``attention_generic_dv`` with the options of a capped, sunk and gated softmax. softcap: score <-
     softcap * tanh(score / softcap) after the scale. sink: None; "unit": the denominator holds one more
     term exp(0) = 1; a float32 tensor [heads]: one more term exp(sink[head]). gate: rows [nt, >= heads *
@@ -1861,6 +1900,10 @@ def attention_sink(q, out, kcache, vcache, block_table, cu_q, pos0, max_qlen, nu
     if not 0 <= gd <= value_dim:
         raise KernelError(f"attention: gate columns per head {gd} outside [0, {value_dim}]")
     cap, mode, sink_t, gate, gs = _sink_args("attention", q, num_heads, gd, softcap, sink, gate)
+    if f32_attention_takes(q, out, kcache, vcache, key_dim, value_dim):
+        return _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads,
+                              num_kv_heads, key_dim, value_dim, scale, window, ws, cap, mode, sink_t, gate, gs, gd,
+                              _kept(keep_first, window), _chunk(chunk, window))
     _check(library().ta_attention_generic_sink(
         _stream(), c_int(_code(q.dtype)), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache),
         _ptr(vcache), _ptr(block_table), c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0),

@@ -129,7 +129,7 @@ class CachedAttention(Part):
                                            bias=self.w.get("qkv.bias"))
         kernels.attention(qkv, o, kc, vc, meta.block_table, ctx.cu_q, ctx.pos0, ctx.max_qlen,
                           ctx.max_kv_len, self.nq, self.nkv, self.dh, float(self.spec.scale),
-                          self.spec.window)
+                          self.spec.window, ws=ctx.ws)
         return self._out(o, ctx, fold, into)
 
 
@@ -232,7 +232,7 @@ class NormedAttention(Part):
         if not self._on_matrix_cores():
             o = ctx.ws.take("attention.o", (nt, self.nq * self.dv), self.dtype)
             kernels.attention_generic_dv(qkv, o, kc, vc, meta.block_table, ctx.cu_q, ctx.pos0, ctx.max_qlen,
-                                         self.nq, self.nkv, self.dk, self.dv, float(s.scale), s.window)
+                                         self.nq, self.nkv, self.dk, self.dv, float(s.scale), s.window, ws=ctx.ws)
             return linear_delta(o, self.w["out.weight"], ctx.ws, "attention.delta"), None
         o = ctx.ws.take("attention.o", (nt, self.nq * self.dk), self.dtype)
         planner = self.step_planner()
@@ -415,7 +415,7 @@ class SinkAttention(Part):
             o = ctx.ws.take("attention.o", (nt, self.nq * vd), self.dtype)
             kernels.attention_sink(qkv, o, kc, vc, meta.block_table, ctx.cu_q, ctx.pos0, ctx.max_qlen, self.nq,
                                    self.nkv, self.dk, vd, float(s.scale), s.window, s.softcap, sink, gate, self.gate_dim,
-                                   keep_first=s.keep_first, chunk=s.chunk)
+                                   keep_first=s.keep_first, chunk=s.chunk, ws=ctx.ws)
             return finish(o, w, ctx.ws, "attention.delta", fold, into)
         # matrix cores: scores and sums in float32, the softmax weights kept at 32 bits by three pieces
         o = ctx.ws.take("attention.o", (nt, self.nq * self.dk), self.dtype)
