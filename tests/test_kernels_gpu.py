@@ -905,6 +905,40 @@ def test_sample_rows_on_16_byte_boundaries_and_others_choose_alike(vocab):
         assert torch.equal(a, b), (T, k, p_, (a != b).nonzero().flatten().tolist())
 
 
+@pytest.mark.parametrize("vocab", [4095, 4097, 8192, 40963])
+def test_sample_in_parts_of_a_row_chooses_as_the_whole_row(vocab):
+    """Rows whose parts end at, before and behind a multiple of 4,096; thresholds inside one step of logit / T, on a
+    step's edge, among equals in several parts, more equals than a part may gather, 16 units and more under the
+    maximum, parts of nothing but -inf: the kernel that walks unaligned rows chooses the same tokens."""
+    from transformer_amd import kernels
+    own = np.random.default_rng(vocab)
+    n = 24
+    l = (own.normal(size=(n, vocab)) * 2.5).astype(np.float32)
+    l[1] = np.round(l[1] * 4) / 4                              # equal logits on the steps' edges
+    l[2, ::7] = 9.0                                            # equals in every part
+    l[3, :] = -3.0
+    l[4, :4000] = -np.inf
+    l[5, :] = -np.inf
+    l[5, vocab - 1] = 1.5
+    l[6] *= 40
+    l[7] *= 0.01
+    l[8] += 1e4
+    l[9, -3:] = 20.0
+    u = own.random(n).astype(np.float32)
+    u[10:12] = 0.0, 1.0 - 2.0 ** -24
+    ld = (vocab + 11) // 4 * 4
+    aligned = torch.zeros(n, ld, device=DEV)[:, 4:4 + vocab]
+    shifted = torch.zeros(n, ld, device=DEV)[:, 1:1 + vocab]
+    aligned.copy_(dev(l)); shifted.copy_(dev(l))
+    a, b = (torch.empty(n, dtype=torch.int32, device=DEV) for _ in range(2))
+    scratch = torch.full((kernels.sample_scratch(n, vocab),), 255, dtype=torch.uint8, device=DEV)
+    for T, k, p_ in ((1.0, vocab, 1.0), (0.8, 40, 0.95), (1.1, vocab, 0.9), (0.05, vocab, 0.99), (30.0, vocab, 0.5), (1.0, 1, 1.0),
+                     (1.0, vocab - 1, 1.0), (2.0, 3000, 0.9999), (1.0, vocab, 0.0)):
+        kernels.sample(aligned, dev(u), a, T, k, p_, scratch)
+        kernels.sample(shifted, dev(u), b, T, k, p_)
+        assert torch.equal(a, b), (T, k, p_, (a != b).nonzero().flatten().tolist())
+
+
 def test_sample_frequencies():
     from transformer_amd import kernels
     l = np.log(np.array([0.5, 0.25, 0.125, 0.0625, 0.0625], dtype=np.float64)).astype(np.float32)

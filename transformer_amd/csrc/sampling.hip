@@ -386,34 +386,61 @@ __device__ __forceinline__ u64 wave_sum_u64(u64 v) {
 
 // a mass no row reaches (2^17 tokens of 2^40 each are 2^57), with room to add to it
 #define NO_MASS_LIMIT ((u64)1 << 62)
-#define CAND_PER_WAVE 256  // tokens near the maximum that a wave's share of the row may hold
-#define NEAR_BINS 96       // steps of 1/9 counted one by one: down to e^-10.7 of the largest probability
+#define STEPS 128          // steps of 1/8 of a unit of logit / T that a part counts one by one: 16 units down from its largest
+#define STEPS_PER_UNIT 8.0f
+#define PART 4096          // tokens of a row that one workgroup looks at
+#define PART_THREADS 256
+#define MAX_PARTS 256       // of a row: a million tokens
+#define PART_CAND 512      // tokens of the steps that hold the threshold, per part
+#define ROW_CAND 4096      // and per row
+#define MASS_MARGIN 1e-4   // sums relative to a part's maximum are this close to the row's own (3e-6 measured from the formats)
 
-// distance from the maximum in steps of 1/9 of (max - logit) / T; 255 holds all that is further
-__device__ __forceinline__ int near_bin(float l, float m, float inv_t) {
-  const float d = (m - l) * inv_t * 9.0f;
-  return d < 255.0f ? (int)d : 255;
+// The step a logit lies in, counted up from 0 at logit 0: a rising function of the logit.
+__device__ __forceinline__ int step_of(float l, float inv_t) {
+  return (int)floorf(fminf(fmaxf(l * inv_t * STEPS_PER_UNIT, -1e9f), 1e9f));
 }
 
-// One digit of the threshold key: the highest bin with which the count reaches k_lim or
-// the mass p_lim. The last digit also settles how many tokens of the threshold value are
+// One digit of the threshold key, by one wave (a lane four bins): the highest bin with which the count
+// reaches k_lim or the mass p_lim. The last digit also settles how many tokens of the threshold value are
 // kept (the lower indices among equals).
 __device__ void choose_digit(SelectState& st, const uint32_t* h_cnt, const u64* h_mass, int shift,
                              bool last, uint32_t k_lim, u64 p_lim) {
-  uint32_t ca = st.count_above;
-  u64 ma = st.mass_above;
-  int chosen = -1;
-  for (int bin = 255; bin >= 0; --bin) {
-    if (h_cnt[bin] == 0) continue;
-    if (ca + h_cnt[bin] >= k_lim || ma + h_mass[bin] >= p_lim) {
-      chosen = bin;
-      break;
-    }
-    ca += h_cnt[bin];
-    ma += h_mass[bin];
+  const int lane = threadIdx.x % TA_WAVE;
+  uint32_t c[4], cs = 0;
+  u64 q[4], qs = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    c[i] = h_cnt[255 - 4 * lane - i];
+    q[i] = h_mass[255 - 4 * lane - i];
+    cs += c[i];
+    qs += q[i];
   }
+  u64 ci = cs, qi = qs;                            // sums up to and with this lane
+#pragma unroll
+  for (int o = 1; o < TA_WAVE; o <<= 1) {
+    const u64 cu = shfl_up_u64(ci, o), qu = shfl_up_u64(qi, o);
+    if (lane >= o) {
+      ci += cu;
+      qi += qu;
+    }
+  }
+  uint32_t ca = st.count_above + (uint32_t)ci - cs;
+  u64 ma = st.mass_above + qi - qs;
+  int hit = -1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (hit < 0) {
+      if (c[i] && (ca + c[i] >= k_lim || ma + q[i] >= p_lim)) hit = i;
+      else {
+        ca += c[i];
+        ma += q[i];
+      }
+    }
+  const u64 found = __ballot(hit >= 0);
   // p_lim <= total, so the lowest non-empty bin reaches it at the latest
-  if (chosen < 0) chosen = 0;
+  const int who = found ? __ffsll((unsigned long long)found) - 1 : TA_WAVE - 1;
+  if (lane != who) return;
+  const int chosen = hit >= 0 ? 255 - 4 * lane - hit : 0;
   st.count_above = ca;
   st.mass_above = ma;
   st.prefix |= (uint32_t)chosen << shift;
@@ -432,12 +459,11 @@ __device__ void choose_digit(SelectState& st, const uint32_t* h_cnt, const u64* 
   }
 }
 
-// The same choice for rows that start on 16-byte boundaries: every pass over the row brings
-// sixteen bytes per lane. A pass that one thread walks four bytes at a time is a chain of
-// its own loads; with vectors a pass is bound by what one CU can pull out of the L2, where
-// the row (half a megabyte at 128 K tokens) stays after the first pass. All sums are integer
-// sums and the sweeps keep the order of the indices, so this kernel and the one above choose
-// the same token.
+// The same choice by one workgroup for a row that starts on a 16-byte boundary, every pass over the row bringing
+// sixteen bytes per lane: what is left for rows whose threshold the parts below cannot enclose (more than
+// PART_CAND tokens of a part within a step of it, as when thousands are equal, or a threshold more than 16 units of
+// logit / T under the maximum). All sums are integer sums and the sweeps keep the order of the indices, so every way
+// chooses the same token.
 #define VEC_STEPS 64      // steps of 256 tokens whose sums a wave remembers (16 waves: 262,144 tokens)
 struct Four {
   float v[4];
@@ -462,10 +488,8 @@ __device__ __forceinline__ Four load_four_if(const float* __restrict__ row, int 
   return load_four(row, j < groups ? j : 0, j < groups ? vocab : 0);
 }
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
-    const float* __restrict__ logits, size_t ld, int vocab, float inv_t, int top_k, float top_p,
-    const float* __restrict__ uniform, int* __restrict__ out) {
-  const float* row = logits + (size_t)blockIdx.x * ld;
+__device__ void sample_whole_row(const float* __restrict__ row, int vocab, float inv_t, int top_k, float top_p,
+                                 float uniform, int* __restrict__ out) {
   const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
   const int groups = (vocab + 3) / 4;                  // runs of four tokens
   __shared__ float s_f[SAMPLE_WAVES];
@@ -478,11 +502,6 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
   __shared__ u64 s_total;
   __shared__ int s_pick;
   __shared__ u64 s_step[SAMPLE_WAVES][VEC_STEPS];      // kept mass of each step of a wave's range
-  // tokens near the maximum, gathered in index order: wave w's share of the row in cand_*[w]
-  __shared__ float cand_l[SAMPLE_WAVES][CAND_PER_WAVE];
-  __shared__ int cand_i[SAMPLE_WAVES][CAND_PER_WAVE];
-  __shared__ int s_ccnt[SAMPLE_WAVES];
-  __shared__ int s_small;
 
   // ---- max
   float m = -INFINITY;
@@ -517,7 +536,6 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
     st.tie_count = 0xffffffffu;   // "every token of the threshold value is kept"
     st.tie_mass = 0;
     s_pick = 0;
-    s_small = 0;
   }
   for (int i = threadIdx.x; i < 256; i += SAMPLE_THREADS) {
     h_cnt[i] = 0;
@@ -525,231 +543,25 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
   }
   __syncthreads();
 
-  // ---- with a cut: the tokens by their distance from the maximum, in steps of 1/9 of a
-  // unit of (max - logit) / T. The sums give the total mass, and the step in which the count
-  // reaches top_k or the mass reaches top_p bounds the kept set: usually a few hundred
-  // tokens, which are then gathered into LDS and cut and drawn from there, so the row is
-  // read three times in all instead of nine. When that step lies far from the maximum or
-  // the tokens do not fit, the digits of the threshold are found over the whole row as in
-  // the kernel above.
+  // ---- total mass, which only the cut by mass asks for
   if (cut) {
-    // steps from NEAR_BINS on are lumped into the last one, summed in registers: most tokens
-    // lie there, and the cut almost never does
-    uint32_t far_cnt = 0;
-    u64 far_mass = 0;
-    const bool need_total = top_p < 1.0f;    // top-k alone never asks for the mass of the far tokens
-    for (int j = threadIdx.x; j < groups; j += 4 * SAMPLE_THREADS) {
-      Four f[4];
+    u64 tot = 0;
+    if (top_p < 1.0f)
+      for (int j = threadIdx.x; j < groups; j += SAMPLE_THREADS) {
+        const Four f = load_four(row, j, vocab);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) f[u] = load_four_if(row, j + u * SAMPLE_THREADS, groups, vocab);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (!f[u].ok[e]) continue;
-          const int bin = near_bin(f[u].v[e], m, inv_t);
-          if (bin < NEAR_BINS) {             // such a token has mass left by a wide margin
-            atomicAdd(&h_cnt[bin], 1u);
-            atomicAdd(&h_mass[bin], fixed_mass(f[u].v[e], m, inv_t));
-          } else {
-            ++far_cnt;
-            if (need_total) far_mass += fixed_mass(f[u].v[e], m, inv_t);
-          }
-        }
-    }
-    far_cnt = (uint32_t)wave_sum_u64(far_cnt);
-    far_mass = wave_sum_u64(far_mass);
-    if (lane == 0 && far_cnt) {
-      atomicAdd(&h_cnt[255], far_cnt);
-      atomicAdd(&h_mass[255], far_mass);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      u64 t = 0;
-      for (int bin = 0; bin < 256; ++bin) t += h_mass[bin];
-      s_total = t;
-      const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
-      u64 p_lim = (u64)ceil((double)top_p * (double)t);
-      if (p_lim < 1) p_lim = 1;
-      if (p_lim > t) p_lim = t;
-      if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;   // the far tokens' mass was not summed; nothing is cut by mass
-      uint32_t ca = 0;
-      u64 ma = 0;
-      int last = 255;
-      for (int bin = 0; bin < 256; ++bin) {
-        ca += h_cnt[bin];
-        ma += h_mass[bin];
-        if (ca >= k_lim || ma >= p_lim) {
-          last = bin;
-          break;
-        }
+        for (int e = 0; e < 4; ++e) tot += f.ok[e] ? fixed_mass(f.v[e], m, inv_t) : 0;
       }
-      s_pick = last;                          // borrowed until the draw: the last step that matters
-      s_small = t > 0 && last < NEAR_BINS && ca <= (uint32_t)(SAMPLE_WAVES * CAND_PER_WAVE);
-    }
+    tot = wave_sum_u64(tot);
+    if (lane == 0) atomicAdd(&s_total, tot);
     __syncthreads();
   }
   const u64 total = s_total;
-  const int near_last = s_pick;
-  __syncthreads();
-  if (threadIdx.x == 0) s_pick = 0;
 
-  // ---- gather the tokens of the steps up to that one, wave by wave in index order
   const int span = ((groups + SAMPLE_WAVES - 1) / SAMPLE_WAVES + TA_WAVE - 1) / TA_WAVE * TA_WAVE;
   const int lo = wave * span;
   const int hi = (lo + span < groups) ? lo + span : groups;
   const u64 lanes_below = ((u64)1 << lane) - 1;
-  if (cut && s_small) {
-    int have = 0;
-    for (int j0 = lo; j0 < hi; j0 += TA_WAVE) {
-      const int j = j0 + lane;
-      Four f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f.v[e] = -INFINITY;
-        f.ok[e] = false;
-      }
-      if (j < hi) f = load_four(row, j, vocab);
-      bool take[4];
-      int before = 0, all = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        take[e] = f.ok[e] && near_bin(f.v[e], m, inv_t) <= near_last;
-        const u64 b = __ballot(take[e]);
-        before += __popcll(b & lanes_below);
-        all += __popcll(b);
-      }
-      int at = have + before;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (take[e]) {
-          if (at < CAND_PER_WAVE) {
-            cand_l[wave][at] = f.v[e];
-            cand_i[wave][at] = 4 * j + e;
-          }
-          ++at;
-        }
-      have += all;
-    }
-    if (lane == 0) s_ccnt[wave] = have;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int ok = 1;
-      for (int w = 0; w < SAMPLE_WAVES; ++w)
-        if (s_ccnt[w] > CAND_PER_WAVE) ok = 0;         // a wave's share did not fit: the long way
-      s_small = ok;
-    }
-    __syncthreads();
-  }
-
-  if (cut && s_small) {
-    // ---- the cut among the gathered tokens (they hold every token at or above the threshold)
-    const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
-    u64 p_lim = (u64)ceil((double)top_p * (double)total);
-    if (p_lim < 1) p_lim = 1;
-    if (p_lim > total) p_lim = total;
-    if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;      // see above: only top_k cuts
-    const int mine = s_ccnt[wave];
-    for (int pass = 0; pass < 4; ++pass) {
-      const int shift = 24 - 8 * pass;
-      for (int i = threadIdx.x; i < 256; i += SAMPLE_THREADS) {
-        h_cnt[i] = 0;
-        h_mass[i] = 0;
-      }
-      __syncthreads();
-      const uint32_t prefix = st.prefix, mask = st.mask;
-      for (int c = lane; c < mine; c += TA_WAVE) {
-        const float l = cand_l[wave][c];
-        const uint32_t key = order_key(l);
-        if ((key & mask) == prefix) {
-          const int bin = (key >> shift) & 255;
-          atomicAdd(&h_cnt[bin], 1u);
-          atomicAdd(&h_mass[bin], fixed_mass(l, m, inv_t));
-        }
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) choose_digit(st, h_cnt, h_mass, shift, pass == 3, k_lim, p_lim);
-      __syncthreads();
-    }
-    const uint32_t thr = st.prefix;
-    const uint32_t n_tie = st.tie_count;
-    // ---- the draw, in index order: wave by wave, and inside a wave as gathered
-    uint32_t ties = 0;
-    for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
-      const int c = c0 + lane;
-      ties += __popcll(__ballot(c < mine && order_key(cand_l[wave][c]) == thr));
-    }
-    if (lane == 0) s_c[wave] = ties;
-    __syncthreads();
-    uint32_t tie_base = 0;
-    for (int w = 0; w < wave; ++w) tie_base += s_c[w];
-    u64 kept = 0;
-    {
-      uint32_t rank = tie_base;
-      for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
-        const int c = c0 + lane;
-        bool keep = false, tie = false;
-        float l = 0.f;
-        if (c < mine) {
-          l = cand_l[wave][c];
-          const uint32_t key = order_key(l);
-          tie = key == thr;
-          keep = key > thr;
-        }
-        const u64 b = __ballot(tie);
-        if (tie && rank + __popcll(b & lanes_below) < n_tie) keep = true;
-        rank += __popcll(b);
-        if (keep) kept += fixed_mass(l, m, inv_t);
-      }
-    }
-    kept = wave_sum_u64(kept);
-    if (lane == 0) s_q[wave] = kept;
-    __syncthreads();
-    u64 mass_base = 0, kept_total = 0;
-    for (int w = 0; w < SAMPLE_WAVES; ++w) {
-      if (w < wave) mass_base += s_q[w];
-      kept_total += s_q[w];
-    }
-    u64 target = (u64)((double)uniform[blockIdx.x] * (double)kept_total);
-    if (kept_total > 0 && target >= kept_total) target = kept_total - 1;
-    if (kept_total > 0 && target >= mass_base && target < mass_base + s_q[wave]) {
-      uint32_t rank = tie_base;
-      u64 run = mass_base;
-      for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
-        const int c = c0 + lane;
-        bool keep = false, tie = false;
-        float l = 0.f;
-        if (c < mine) {
-          l = cand_l[wave][c];
-          const uint32_t key = order_key(l);
-          tie = key == thr;
-          keep = key > thr;
-        }
-        const u64 b = __ballot(tie);
-        if (tie && rank + __popcll(b & lanes_below) < n_tie) keep = true;
-        rank += __popcll(b);
-        const u64 q = keep ? fixed_mass(l, m, inv_t) : 0;
-        u64 inc = q;
-#pragma unroll
-        for (int o = 1; o < TA_WAVE; o <<= 1) {
-          const u64 up = shfl_up_u64(inc, o);
-          if (lane >= o) inc += up;
-        }
-        const bool hit = q > 0 && run + inc > target && run + inc - q <= target;
-        if (__ballot(hit)) {
-          if (hit) s_pick = cand_i[wave][c];
-          break;
-        }
-        uint32_t lo32 = (uint32_t)inc, hi32 = (uint32_t)(inc >> 32);
-        lo32 = __shfl(lo32, TA_WAVE - 1, TA_WAVE);
-        hi32 = __shfl(hi32, TA_WAVE - 1, TA_WAVE);
-        run += ((u64)hi32 << 32) | lo32;
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) out[blockIdx.x] = s_pick;
-    return;
-  }
 
   // ---- threshold of the kept set (only when top-k or top-p cut anything)
   if (cut) {
@@ -757,7 +569,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
     u64 p_lim = (u64)ceil((double)top_p * (double)total);
     if (p_lim < 1) p_lim = 1;
     if (p_lim > total) p_lim = total;
-    if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;      // see above: only top_k cuts
+    if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;      // the mass was not summed: only top_k cuts
     for (int pass = 0; pass < 4; ++pass) {
       const int shift = 24 - 8 * pass;
       for (int i = threadIdx.x; i < 256; i += SAMPLE_THREADS) {
@@ -779,7 +591,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
         }
       }
       __syncthreads();
-      if (threadIdx.x == 0) choose_digit(st, h_cnt, h_mass, shift, pass == 3, k_lim, p_lim);
+      if (wave == 0) choose_digit(st, h_cnt, h_mass, shift, pass == 3, k_lim, p_lim);
       __syncthreads();
     }
   }
@@ -863,7 +675,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
     if (w < wave) mass_base += s_q[w];
     kept_total += s_q[w];
   }
-  u64 target = (u64)((double)uniform[blockIdx.x] * (double)kept_total);
+  u64 target = (u64)((double)uniform * (double)kept_total);
   if (kept_total > 0 && target >= kept_total) target = kept_total - 1;
 
   // sweep 3: the wave whose range holds the target finds the token
@@ -928,22 +740,561 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_vec_kernel(
   }
 #undef KEEP_FOUR
   __syncthreads();
+  if (threadIdx.x == 0) *out = s_pick;
+}
+
+// Rows that start on a 16-byte boundary are dealt out in parts of 4,096 tokens, one workgroup each, so that eight rows
+// keep 256 CUs busy and not eight: a row is bound by instructions per token, not by memory. Three kernels:
+//   parts   each part's maximum, and its tokens and their mass (relative to that maximum) by steps of 1/8 of a
+//           unit of logit / T;
+//   gather  from all parts' steps the step that holds the threshold, or the two between which the margin of the
+//           relative masses leaves it; what lies above it is kept: its mass and count, exactly; what lies in
+//           it is gathered in index order;
+//   draw    one workgroup a row: the threshold among the gathered tokens by the digits of their keys, the part that
+//           holds the drawn mass, the token in it.
+// 8 rows of 128,256 tokens, top-k 40 and top-p 0.95: 125 us by one workgroup a row (which gathered whole kept sets of a
+// few thousand tokens), 29 us in parts
+// (5 + 10 + 15); 64 rows 51 us, 256 rows 125, one row without a cut 16.
+struct PartRecord {
+  float2 mass[STEPS / 2];    // of two steps each, relative to the part's maximum
+  uint32_t cnt[STEPS / 2];   // tokens of two steps each, 16 bits of them (a part has 4,096)
+  u64 above, total;          // exact: of the tokens above the steps in question; of all
+  double rest;               // of all its tokens, relative to the part's maximum
+  float max;
+  uint32_t above_n;
+  int lo, hi;                // the steps in question, counted down from the row's largest; lo < 0: not enclosed
+  int n;                     // gathered
+  float cand_l[PART_CAND];   // in index order
+};
+
+// group u (of four) of this thread in its part
+__device__ __forceinline__ int part_group(int part, int u) { return part * (PART / 4) + u * PART_THREADS + (int)threadIdx.x; }
+
+__global__ __launch_bounds__(PART_THREADS) void sample_parts_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                    float inv_t, int cut, int by_mass,
+                                                                    PartRecord* __restrict__ records) {
+  const float* row = logits + (size_t)blockIdx.y * ld;
+  PartRecord& rec = records[(size_t)blockIdx.y * gridDim.x + blockIdx.x];
+  const int groups = (vocab + 3) / 4, wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  __shared__ float s_f[PART_THREADS / TA_WAVE];
+  __shared__ uint32_t cnt[STEPS];
+  __shared__ u64 mass[STEPS], rest;
+  for (int i = threadIdx.x; i < STEPS; i += PART_THREADS) {
+    cnt[i] = 0;
+    mass[i] = 0;
+  }
+  if (threadIdx.x == 0) rest = 0;
+  Four f[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) f[u] = load_four_if(row, part_group(blockIdx.x, u), groups, vocab);
+  float m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = fmaxf(m, f[u].v[e]);
+  m = wave_max(m);
+  if (lane == 0) s_f[wave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < PART_THREADS / TA_WAVE; ++w) m = fmaxf(m, s_f[w]);
+  if (threadIdx.x == 0) rec.max = m;
+  if (!cut) return;
+  const int top = step_of(m, inv_t);
+  u64 all = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (!f[u].ok[e]) continue;
+      const int at = top - step_of(f[u].v[e], inv_t);
+      const u64 q = by_mass ? fixed_mass(f[u].v[e], m, inv_t) : 0;
+      all += q;
+      if (at < STEPS) {
+        atomicAdd(&cnt[at], 1u);
+        if (by_mass) atomicAdd(&mass[at], q);
+      }
+    }
+  if (by_mass) {
+    all = wave_sum_u64(all);
+    if (lane == 0) atomicAdd(&rest, all);
+  }
+  __syncthreads();
+  if (threadIdx.x < STEPS / 2) {
+    const int i = 2 * threadIdx.x;
+    rec.cnt[threadIdx.x] = cnt[i] | (cnt[i + 1] << 16);
+    rec.mass[threadIdx.x] = float2{(float)mass[i], (float)mass[i + 1]};
+  }
+  if (threadIdx.x == 0) rec.rest = (double)rest;
+}
+
+// the row's maximum from its parts'
+__device__ __forceinline__ float row_max(const PartRecord* rec, int parts) {
+  float m = -INFINITY;
+  for (int p = threadIdx.x % TA_WAVE; p < parts; p += TA_WAVE) m = fmaxf(m, rec[p].max);
+  return wave_max(m);
+}
+
+__global__ __launch_bounds__(PART_THREADS) void sample_gather_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                     float inv_t, int top_k, float top_p, int cut,
+                                                                     PartRecord* __restrict__ records) {
+  const float* row = logits + (size_t)blockIdx.y * ld;
+  PartRecord* all = records + (size_t)blockIdx.y * gridDim.x;
+  PartRecord& rec = all[blockIdx.x];
+  const int parts = gridDim.x, groups = (vocab + 3) / 4;
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  constexpr int WAVES = PART_THREADS / TA_WAVE;
+  __shared__ u64 s_c[WAVES][TA_WAVE][3];
+  __shared__ double s_q[WAVES][TA_WAVE][3], s_rest[WAVES];
+  __shared__ int s_lo, s_hi, s_n[4][WAVES];
+  __shared__ u64 s_above[WAVES], s_total[WAVES];
+  __shared__ uint32_t s_above_n[WAVES];
+  Four f[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) f[u] = load_four_if(row, part_group(blockIdx.x, u), groups, vocab);
+  const float m = row_max(all, parts);
+  const int top = step_of(m, inv_t);
+  const bool by_mass = top_p < 1.0f;
+  if (cut) {
+    // the row's steps from the parts': a step is the same interval of logits in all of them, so a part's are
+    // moved by the difference of the largest ones. A wave takes every fourth part, a lane two steps; where a part
+    // is moved by an odd number its pairs fall on two lanes' steps
+    u64 c[3] = {0, 0, 0};                            // this lane's steps 2 lane, 2 lane + 1, and what belongs one further
+    double q[3] = {0.0, 0.0, 0.0}, t = 0.0;
+    for (int p0 = wave; p0 < parts; p0 += 8 * WAVES) {
+      uint32_t cn[8];
+      float2 qn[8];
+      float pm[8];
+      double rest[8];
+      int off[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pm[i] = all[p0 + i * WAVES < parts ? p0 + i * WAVES : p0].max;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const PartRecord& r = all[p0 + i * WAVES < parts ? p0 + i * WAVES : p0];
+        off[i] = top - step_of(pm[i], inv_t);
+        const int at = lane - off[i] / 2;            // pair of the part whose first step is 2 lane (or one further)
+        const bool in = p0 + i * WAVES < parts && at >= 0;
+        cn[i] = r.cnt[in ? at : 0];
+        qn[i] = r.mass[in ? at : 0];
+        rest[i] = r.rest;
+        if (!in) {
+          cn[i] = 0;
+          qn[i] = float2{0.f, 0.f};
+        }
+        if (p0 + i * WAVES >= parts) rest[i] = 0.0;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float w = __builtin_amdgcn_exp2f((pm[i] - m) * inv_t * 1.44269504088896341f);
+        const bool odd = off[i] & 1;
+        const uint32_t ca = cn[i] & 0xffffu, cb = cn[i] >> 16;
+        c[0] += odd ? 0 : ca;
+        c[1] += odd ? ca : cb;
+        c[2] += odd ? cb : 0;
+        if (by_mass) {
+          const double qa = (double)qn[i].x * w, qb = (double)qn[i].y * w;
+          q[0] += odd ? 0.0 : qa;
+          q[1] += odd ? qa : qb;
+          q[2] += odd ? qb : 0.0;
+          t += rest[i] * w;
+        }
+      }
+    }
+    s_c[wave][lane][0] = c[0];
+    s_c[wave][lane][1] = c[1];
+    s_c[wave][lane][2] = c[2];
+    s_q[wave][lane][0] = q[0];
+    s_q[wave][lane][1] = q[1];
+    s_q[wave][lane][2] = q[2];
+    if (lane == 0) s_rest[wave] = t;                 // the same in all lanes
+    __syncthreads();
+    if (wave == 0) {                                 // a lane two steps
+      u64 c0 = 0, c = 0;
+      double q0 = 0.0, q = 0.0;
+      t = 0.0;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) {
+        c0 += s_c[w][lane][0] + (lane ? s_c[w][lane - 1][2] : 0);
+        c += s_c[w][lane][1];
+        q0 += s_q[w][lane][0] + (lane ? s_q[w][lane - 1][2] : 0.0);
+        q += s_q[w][lane][1];
+        t += s_rest[w];
+      }
+      const u64 c1 = c;
+      const double q1 = q;
+      c += c0;
+      q += q0;
+#pragma unroll
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const u64 cu = shfl_up_u64(c, o);
+        const double qu = __shfl_up(q, o, TA_WAVE);
+        if (lane >= o) {
+          c += cu;
+          q += qu;
+        }
+      }
+      const double want = (double)top_p * t;
+      auto reaches = [&](u64 cn, double qn, double factor) {
+        return cn >= (u64)top_k || (by_mass && qn >= want * factor);
+      };
+      c0 = c - c1;                                   // up to and with the first of the two
+      q0 = q - q1;
+      auto first = [&](double factor) {
+        const u64 b0 = __ballot(reaches(c0, q0, factor)), b1 = __ballot(reaches(c, q, factor));
+        const u64 any = b0 | b1;
+        if (!any) return STEPS;
+        const int who = __ffsll((unsigned long long)any) - 1;
+        return 2 * who + ((b0 >> who) & 1 ? 0 : 1);
+      };
+      const int lo = first(1.0 - MASS_MARGIN), hi = first(1.0 + MASS_MARGIN);
+      if (lane == 0) {
+        s_lo = hi < STEPS && m > -INFINITY && m < INFINITY ? lo : -1;
+        s_hi = hi;
+      }
+    }
+    __syncthreads();
+  }
+  const int lo = cut ? s_lo : STEPS, hi = cut ? s_hi : STEPS;
+  // this part: what is kept for certain, and what is in question
+  u64 above = 0, total = 0;
+  uint32_t above_n = 0;
+  int before[4], mine[4];
+  u64 take[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    int all_ = 0;
+    before[u] = mine[u] = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool ok = f[u].ok[e];
+      const u64 q = ok ? fixed_mass(f[u].v[e], m, inv_t) : 0;
+      const int at = top - step_of(f[u].v[e], inv_t);
+      total += q;
+      const bool keep = ok && (!cut || at < lo);
+      above += keep ? q : 0;
+      above_n += keep;
+      take[u][e] = __ballot(ok && cut && at >= lo && at <= hi);
+      before[u] += __popcll(take[u][e] & (((u64)1 << lane) - 1));
+      all_ += __popcll(take[u][e]);
+    }
+    if (lane == 0) s_n[u][wave] = all_;
+  }
+  above = wave_sum_u64(above);
+  total = wave_sum_u64(total);
+  above_n = (uint32_t)wave_sum_u64(above_n);
+  if (lane == 0) {
+    s_above[wave] = above;
+    s_total[wave] = total;
+    s_above_n[wave] = above_n;
+  }
+  __syncthreads();
+  int base = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (w == wave) {
+        int at = base + before[u];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((take[u][e] >> lane) & 1) {
+            if (at < PART_CAND) rec.cand_l[at] = f[u].v[e];
+            ++at;
+          }
+      }
+      base += s_n[u][w];
+    }
+  if (threadIdx.x == 0) {
+    u64 a = 0, t = 0;
+    uint32_t n = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      a += s_above[w];
+      t += s_total[w];
+      n += s_above_n[w];
+    }
+    rec.above = a;
+    rec.total = t;
+    rec.above_n = n;
+    rec.lo = lo;
+    rec.hi = hi;
+    rec.n = base;
+  }
+}
+
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                     float inv_t, int top_k, float top_p, int cut, int parts,
+                                                                     const PartRecord* __restrict__ records,
+                                                                     const float* __restrict__ uniform, int* __restrict__ out) {
+  const float* row = logits + (size_t)blockIdx.x * ld;
+  const PartRecord* all = records + (size_t)blockIdx.x * parts;
+  const int groups = (vocab + 3) / 4;
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  const u64 lanes_below = ((u64)1 << lane) - 1;
+  __shared__ float cand_l[ROW_CAND];
+  __shared__ uint32_t s_ties[SAMPLE_WAVES];
+  __shared__ uint32_t h_cnt[256];
+  __shared__ u64 h_mass[256];
+  __shared__ SelectState st;
+  __shared__ int s_ok, s_cands, s_part, s_pick, s_lo, s_hi;
+  __shared__ u64 s_total, s_target, s_base, s_wave[SAMPLE_WAVES];
+  __shared__ uint32_t s_tie_base;
+  __shared__ float s_max;
+  __shared__ int s_first[MAX_PARTS];                 // first gathered token of a part
+  __shared__ u64 s_kept[MAX_PARTS];                  // mass that a part keeps
+
+  // ---- what the parts say: 16 waves read their records side by side, one adds up
+  if (threadIdx.x == 0) s_ok = 1;
+  if (wave == 0) {
+    const float m = row_max(all, parts);
+    if (lane == 0) {
+      s_max = m;
+      s_lo = all[0].lo;
+      s_hi = all[0].hi;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int run = 0;
+    u64 total = 0, above = 0;
+    uint32_t above_n = 0;
+    bool ok = true;
+    for (int p0 = 0; p0 < parts; p0 += TA_WAVE) {
+      const int p = p0 + lane;
+      const bool in = p < parts;
+      const PartRecord& r = all[in ? p : 0];
+      const int n = in ? r.n : 0;
+      total += in ? r.total : 0;
+      above += in ? r.above : 0;
+      above_n += in ? r.above_n : 0;
+      ok = ok && n <= PART_CAND;
+      int inc = n;
+#pragma unroll
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const int up = __shfl_up(inc, o, TA_WAVE);
+        if (lane >= o) inc += up;
+      }
+      if (in) {
+        s_first[p] = run + inc - n;
+        s_kept[p] = r.above;
+      }
+      run += __shfl(inc, TA_WAVE - 1, TA_WAVE);
+    }
+    total = wave_sum_u64(total);
+    above = wave_sum_u64(above);
+    above_n = (uint32_t)wave_sum_u64(above_n);
+    ok = __ballot(!ok) == 0;
+    if (lane == 0) {
+      s_total = total;
+      s_cands = run;
+      s_ok = ok && run <= ROW_CAND && total > 0 && s_lo >= 0;
+      st.prefix = 0;
+      st.mask = 0;
+      st.count_above = above_n;
+      st.mass_above = above;
+      st.tie_count = 0xffffffffu;
+      st.tie_mass = 0;
+      s_pick = 0;
+      s_part = -1;
+      s_tie_base = 0;
+    }
+  }
+  __syncthreads();
+  if (!s_ok) {
+    sample_whole_row(row, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
+    return;
+  }
+  const float m = s_max;
+  const int cands = s_cands, lo = s_lo, hi = s_hi, top = step_of(m, inv_t);
+  if (cut) {
+    for (int p = wave; p < parts; p += SAMPLE_WAVES)
+      for (int c = lane; c < all[p].n; c += TA_WAVE) cand_l[s_first[p] + c] = all[p].cand_l[c];
+    // ---- the threshold among the gathered tokens
+    const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
+    u64 p_lim = (u64)ceil((double)top_p * (double)s_total);
+    if (p_lim < 1) p_lim = 1;
+    if (p_lim > s_total) p_lim = s_total;
+    if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;
+    for (int pass = 0; pass < 4; ++pass) {
+      const int shift = 24 - 8 * pass;
+      if (threadIdx.x < 256) {
+        h_cnt[threadIdx.x] = 0;
+        h_mass[threadIdx.x] = 0;
+      }
+      __syncthreads();
+      const uint32_t prefix = st.prefix, mask = st.mask;
+      for (int c = threadIdx.x; c < cands; c += SAMPLE_THREADS) {
+        const float l = cand_l[c];
+        const uint32_t key = order_key(l);
+        if ((key & mask) == prefix) {
+          atomicAdd(&h_cnt[(key >> shift) & 255], 1u);
+          atomicAdd(&h_mass[(key >> shift) & 255], fixed_mass(l, m, inv_t));
+        }
+      }
+      __syncthreads();
+      if (wave == 0) choose_digit(st, h_cnt, h_mass, shift, pass == 3, k_lim, p_lim);
+      __syncthreads();
+    }
+  }
+  const uint32_t thr = st.prefix, n_tie = st.tie_count;
+  // ---- what every part keeps of its gathered tokens. Waves take the parts in turn; the ties of a row are
+  // ranked in index order, so their numbers per part come first
+  if (cut) {
+    __shared__ uint32_t s_part_ties[MAX_PARTS];
+    for (int p = wave; p < parts; p += SAMPLE_WAVES) {
+      const int n = all[p].n;
+      uint32_t ties = 0;
+      u64 kept = 0;
+      for (int c0 = 0; c0 < n; c0 += TA_WAVE) {
+        const bool in = c0 + lane < n;
+        const float l = in ? cand_l[s_first[p] + c0 + lane] : 0.f;
+        const uint32_t key = order_key(l);
+        ties += __popcll(__ballot(in && key == thr));
+        if (in && key > thr) kept += fixed_mass(l, m, inv_t);
+      }
+      kept = wave_sum_u64(kept);
+      if (lane == 0) {
+        s_part_ties[p] = ties;
+        s_kept[p] += kept;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      u64 sum = 0;
+      uint32_t rank = 0;
+      for (int p = 0; p < parts; ++p) {
+        const uint32_t t = s_part_ties[p], room = n_tie > rank ? n_tie - rank : 0;
+        s_kept[p] += (u64)(t < room ? t : room) * st.tie_mass;
+        s_part_ties[p] = rank;
+        rank += t;
+        sum += s_kept[p];
+      }
+      s_total = sum;
+      u64 target = (u64)((double)uniform[blockIdx.x] * (double)sum);
+      if (sum > 0 && target >= sum) target = sum - 1;
+      u64 run = 0;
+      for (int p = 0; p < parts; ++p) {
+        if (target < run + s_kept[p]) {
+          s_part = p;
+          s_base = run;
+          s_tie_base = s_part_ties[p];
+          break;
+        }
+        run += s_kept[p];
+      }
+      s_target = target;
+    }
+  } else if (threadIdx.x == 0) {
+    u64 target = (u64)((double)uniform[blockIdx.x] * (double)s_total), run = 0;
+    if (target >= s_total) target = s_total - 1;
+    for (int p = 0; p < parts; ++p) {
+      if (target < run + s_kept[p]) {
+        s_part = p;
+        s_base = run;
+        break;
+      }
+      run += s_kept[p];
+    }
+    s_target = target;
+  }
+  __syncthreads();
+  if (s_part < 0) {
+    if (threadIdx.x == 0) out[blockIdx.x] = 0;
+    return;
+  }
+  // ---- the token in that part: one group of four a thread, in index order
+  const int j = s_part * (PART / 4) + (int)threadIdx.x;
+  const Four f = load_four_if(row, j, groups, vocab);
+  bool keep[4], tie[4];
+  uint32_t ties_before = 0, ties_all = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int at = top - step_of(f.v[e], inv_t);
+    const bool asked = cut && f.ok[e] && at >= lo && at <= hi;
+    const uint32_t key = order_key(f.v[e]);
+    tie[e] = asked && key == thr;
+    keep[e] = f.ok[e] && (!cut || at < lo || (asked && key > thr));
+    const u64 b = __ballot(tie[e]);
+    ties_before += __popcll(b & lanes_below);
+    ties_all += __popcll(b);
+  }
+  if (lane == 0) s_ties[wave] = ties_all;
+  __syncthreads();
+  uint32_t rank = s_tie_base + ties_before;
+  for (int w = 0; w < wave; ++w) rank += s_ties[w];
+  u64 q[4], mine = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (tie[e]) {
+      keep[e] = rank < n_tie;
+      ++rank;
+    }
+    q[e] = keep[e] ? fixed_mass(f.v[e], m, inv_t) : 0;
+    mine += q[e];
+  }
+  u64 inc = mine;
+#pragma unroll
+  for (int o = 1; o < TA_WAVE; o <<= 1) {
+    const u64 up = shfl_up_u64(inc, o);
+    if (lane >= o) inc += up;
+  }
+  if (lane == TA_WAVE - 1) s_wave[wave] = inc;
+  __syncthreads();
+  u64 run = s_base;
+  for (int w = 0; w < wave; ++w) run += s_wave[w];
+  const u64 target = s_target;
+  if (mine > 0 && run + inc > target && run + inc - mine <= target) {
+    u64 at = run + inc - mine;
+    int pick = 4 * j;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (q[e] > 0 && at + q[e] > target && at <= target) pick = 4 * j + e;
+      at += q[e];
+    }
+    s_pick = pick;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = s_pick;
 }
 
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                     float inv_t, int top_k, float top_p,
+                                                                     const float* __restrict__ uniform, int* __restrict__ out) {
+  sample_whole_row(logits + (size_t)blockIdx.x * ld, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
+}
+
+static int sample_parts(int vocab) { return (vocab + PART - 1) / PART; }
+
+// Bytes of scratch that lets ta_sample deal rows out in parts (0: rows of this vocabulary are not).
+extern "C" long long ta_sample_scratch(int n, int vocab) {
+  if (n <= 0 || n > 65535 || vocab <= 0 || sample_parts(vocab) > MAX_PARTS) return 0;
+  const long long bytes = (long long)n * sample_parts(vocab) * (long long)sizeof(PartRecord);
+  return bytes <= (256ll << 20) ? bytes : 0;     // thousands of rows fill the chip one workgroup each
+}
+
+// scratch: ta_sample_scratch bytes on an 8-byte boundary, or null: one workgroup takes a row then.
 extern "C" int ta_sample(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
                          float temperature, int top_k, float top_p, const float* uniform,
-                         int* out) {
+                         int* out, void* scratch) {
   TA_REQUIRE(n >= 0 && vocab > 0 && ld >= vocab, "ta_sample: bad sizes n=%d vocab=%d ld=%lld", n, vocab, ld);
   TA_REQUIRE(temperature > 0.f, "ta_sample: temperature %g must be > 0 (0 means argmax)", (double)temperature);
   TA_REQUIRE(top_k >= 1, "ta_sample: top_k %d < 1", top_k);
   TA_REQUIRE(top_p >= 0.f && top_p <= 1.f, "ta_sample: top_p %g outside [0, 1]", (double)top_p);
+  TA_REQUIRE((uintptr_t)scratch % 8 == 0, "ta_sample: scratch does not start on 8 bytes");
   if (n == 0) return 0;
-  if (((uintptr_t)logits % 16) == 0 && ld % 4 == 0)
-    sample_vec_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, 1.0f / temperature,
-                                                        top_k, top_p, uniform, out);
-  else
-    sample_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, 1.0f / temperature,
-                                                    top_k, top_p, uniform, out);
+  const float inv_t = 1.0f / temperature;
+  if (((uintptr_t)logits % 16) != 0 || ld % 4 != 0) {
+    sample_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
+  } else if (scratch == nullptr || ta_sample_scratch(n, vocab) == 0) {
+    sample_rows_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
+  } else {
+    const int parts = sample_parts(vocab), cut = top_k < vocab || top_p < 1.0f;
+    PartRecord* rec = (PartRecord*)scratch;
+    const dim3 g(parts, n);
+    sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec);
+    sample_gather_kernel<<<g, PART_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, cut, rec);
+    sample_draw_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, cut, parts, rec,
+                                                         uniform, out);
+  }
   return ta_check_launch("ta_sample");
 }

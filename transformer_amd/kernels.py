@@ -834,18 +834,33 @@ def argmax(logits: torch.Tensor, out: torch.Tensor):
     return out
 
 
+def sample_scratch(rows: int, vocab: int) -> int:
+    """Bytes of scratch with which ``sample`` deals rows out among workgroups (0: it does not)."""
+    need = library().ta_sample_scratch
+    need.restype = c_longlong
+    return int(need(c_int(rows), c_int(vocab)))
+
+
 def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, temperature: float,
-           top_k: int, top_p: float):
-    """Draws one token per row from softmax(logits / temperature) cut by top_k / top_p."""
+           top_k: int, top_p: float, scratch: Optional[torch.Tensor] = None):
+    """Draws one token per row from softmax(logits / temperature) cut by top_k / top_p. scratch: uint8 of at least
+    ``sample_scratch`` bytes that nothing else uses meanwhile; without it the call allocates its own."""
     _dev(logits, "logits", torch.float32, contiguous=False); _dev(out, "out", torch.int32)
     _dev(uniform, "uniform", torch.float32)
     n, ld = _rows2d(logits, "logits")
     if out.numel() != n or uniform.numel() != n:
         raise KernelError("sample: out and uniform must hold one entry per row")
     vocab = logits.shape[1]
+    need = sample_scratch(n, vocab)
+    if scratch is None:
+        scratch = torch.empty(need, dtype=torch.uint8, device=logits.device) if need else None
+    else:
+        _dev(scratch, "scratch", torch.uint8)
+        if scratch.numel() < need:
+            raise KernelError(f"sample: {scratch.numel()} bytes of scratch, {need} are needed")
     _check(library().ta_sample(_stream(), _ptr(logits), c_longlong(ld), c_int(n), c_int(vocab),
                                c_float(temperature), c_int(min(int(top_k), vocab)),
-                               c_float(top_p), _ptr(uniform), _ptr(out)))
+                               c_float(top_p), _ptr(uniform), _ptr(out), _ptr(scratch)))
     return out
 
 

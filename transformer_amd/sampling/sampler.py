@@ -49,6 +49,7 @@ class Sampler:
         self.args, self.seed, self.device = args, int(seed), torch.device(device)
         self._ring = [None] * self.RING
         self._turn = 0
+        self._scratch = [None] * self.RING
 
     def _buffers(self, n: int):
         i = self._turn
@@ -75,8 +76,12 @@ class Sampler:
                                             zip(sequences, drawn)], dtype=np.float32)
             u_dev.copy_(u_host, non_blocking=True)
             k = self.args.top_k if self.args.top_k is not None else logits.shape[1]
+            need = kernels.sample_scratch(n, logits.shape[1])
+            i = (self._turn - 1) % self.RING              # of the buffers just taken
+            if self._scratch[i] is None or self._scratch[i].numel() < need:
+                self._scratch[i] = torch.empty(need, dtype=torch.uint8, device=self.device)
             kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
-                           float(self.args.top_p))
+                           float(self.args.top_p), self._scratch[i])
         out_host.copy_(out, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
