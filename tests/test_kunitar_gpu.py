@@ -214,6 +214,53 @@ def test_experts_products_in_every_form(form, geom):
         _close(got, want, "bfloat16" if out_dtype == torch.bfloat16 else "float32", f"{out_dtype}")
 
 
+# experts, router outputs, top, tokens, N, K: one token, the most that are routed in one launch and one more, columns that
+# end inside the 32 or 64 of a workgroup, k inside and behind a wave's share
+@pytest.mark.parametrize("geom", [(5, 5, 3, 1, 40, 72), (64, 72, 6, 16, 33, 200), (8, 8, 2, 17, 96, 1032), (3, 4, 4, 6, 130, 2056)])
+def test_few_tokens_are_routed_and_multiplied_as_in_single_steps(geom):
+    """Routing and plan in one launch, and the experts' first product from the tokens' own rows (weighed, with its
+    activation, as gate and up joined), against the launches they stand for: the same bits for every pair."""
+    from transformer_amd import kernels
+    E, R, top, nt, N, K = geom
+    own = np.random.default_rng(E + nt)
+    z = _t(own.standard_normal((nt, R)).astype(np.float32))
+    corr = _t(0.3 * own.standard_normal(R).astype(np.float32))
+    rows = kernels.moe_max_rows(nt * top, E)
+    i32 = lambda *n: torch.full(n, -7, dtype=torch.int32, device=DEV)
+    got = [], []
+    for one, keep in ((True, got[0]), (False, got[1])):
+        chosen, weight = i32(nt, top), torch.empty(nt, top, device=DEV)
+        row_pair, tile_expert, pair_row = i32(rows), i32(rows // 16), i32(nt * top)
+        if one:
+            kernels.moe_route_plan(z, R, top, chosen, weight, E, row_pair, tile_expert, pair_row, "softmax", True,
+                                   correction=corr, factor=1.7)
+        else:
+            kernels.moe_route(z, R, top, chosen, weight, "softmax", True, correction=corr, factor=1.7)
+            kernels.moe_plan(chosen, E, row_pair, tile_expert, pair_row)
+        keep += [chosen, weight, tile_expert, row_pair, pair_row]
+    for a, b in zip(got[0][:3], got[1][:3]):
+        assert torch.equal(a, b)
+    chosen, weight, tile_expert, row_pair, pair_row = got[0]
+    pr, rp, ch = _np(pair_row).astype(int), _np(row_pair).astype(int), _np(chosen).astype(int).reshape(-1)
+    assert (pr[ch >= E] == -1).all() and (rp[pr[ch < E]] == np.nonzero(ch < E)[0]).all() and (rp >= 0).sum() == (ch < E).sum()
+    assert (_np(tile_expert).astype(int)[pr[ch < E] // 16] == ch[ch < E]).all()
+    h = _t(_bf(own.standard_normal((nt, K))), torch.bfloat16)
+    w = _t(_bf(own.standard_normal((E, 2 * N, K)) / np.sqrt(K)), torch.bfloat16)
+    live = torch.tensor(pr[ch < E], device=DEV)
+    for on in (None, weight):
+        a = kernels.moe_gather(h, top, row_pair, on, torch.empty(rows, K, dtype=torch.bfloat16, device=DEV))
+        pre = kernels.moe_gemm(a, w, tile_expert, torch.zeros(rows, 2 * N, dtype=torch.bfloat16, device=DEV), None, form="split_k")
+        plain = torch.empty(rows, 2 * N, dtype=torch.bfloat16, device=DEV)
+        kernels.moe_gemm(a, w, tile_expert, plain, "relu2", form="split_k")
+        out = kernels.moe_gemm_tokens(h, top, row_pair, on, w, tile_expert, torch.empty_like(plain), "relu2")
+        assert torch.equal(out[live], plain[live])
+        joined = torch.empty(rows, N, dtype=torch.bfloat16, device=DEV)
+        kernels.moe_gemm_tokens(h, top, row_pair, on, w, tile_expert, joined, glu=True)
+        assert torch.equal(joined[live], kernels.glu(pre, torch.empty_like(joined))[live])
+        kernels.moe_gemm_tokens(h, top, row_pair, on, w, tile_expert, joined, glu=True, limits=(0.8, 1.702, 1.0))
+        assert torch.equal(joined[live], kernels.glu_limit(pre, torch.empty_like(joined), 0.8)[live])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("geom", [(3, 20, 8, 8, 48, 33), (1, 16, 16, 16, 16, 1), (5, 7, 6, 4, 19, 9), (2, 12, 8, 8, 48, None),
                                   (8, 64, 32, 32, 128, 150), (4, 16, 0, 0, 300, 70)])

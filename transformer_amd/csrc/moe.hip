@@ -31,15 +31,30 @@
 // counts as its largest score, and only experts of the `keep` best groups (the lowest index
 // among equals) can be chosen. correction [E] or null: the choice compares score + correction, the
 // weights are the scores without it. factor: the weights are multiplied by it last.
-__global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__ logits, int ld, int E, int top,
-                                                       int mode, int renorm, int* __restrict__ chosen,
-                                                       float* __restrict__ weight,
-                                                       const float* __restrict__ bias, int groups, int keep,
-                                                       const float* __restrict__ correction, float factor) {
-  extern __shared__ float sc[];           // [E], then a score per group [groups], then the plain scores [E]
-  float* plain = sc + E + groups;         // (with a correction only)
-  const size_t t = blockIdx.x;
-  const int lane = threadIdx.x;
+struct MoeRoute {
+  const float* logits;
+  int ld, E, top, mode, renorm;
+  const float* bias;
+  int groups, keep;
+  const float* correction;
+  float factor;
+  // floats of LDS that a token takes: a score per expert, one per group, and with a correction the plain scores
+  __host__ __device__ int lds() const { return E + groups + (correction ? E : 0); }
+};
+
+// the wave's LDS writes before this are seen by its reads behind it
+__device__ __forceinline__ void moe_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// one wave routes token t; chosen and weight are the token's own `top` places
+__device__ void moe_route_token(const MoeRoute& p, size_t t, float* sc, int* chosen, float* weight) {
+  const float *logits = p.logits, *bias = p.bias, *correction = p.correction;
+  const int ld = p.ld, E = p.E, top = p.top, mode = p.mode, groups = p.groups, keep = p.keep;
+  float* plain = sc + E + groups;
+  const int lane = threadIdx.x % TA_WAVE;
   float mx = -INFINITY;
   for (int e = lane; e < E; e += 64) mx = fmaxf(mx, logits[t * ld + e] + (bias ? bias[e] : 0.f));
   mx = wave_max(mx);
@@ -58,7 +73,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       sc[e] = s + correction[e];
     }
   }
-  __syncthreads();
+  moe_wave_sync();
   if (groups > 1) {
     float* gs = sc + E;
     const int size = E / groups;
@@ -67,7 +82,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       for (int e = g * size; e < (g + 1) * size; ++e) best = fmaxf(best, sc[e]);
       gs[g] = best;
     }
-    __syncthreads();
+    moe_wave_sync();
     // a group stays when fewer than `keep` groups come before it in the order (score down, index up)
     for (int g = lane; g < groups; g += 64) {
       const float mine = gs[g];
@@ -76,7 +91,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       if (ahead >= keep)
         for (int e = g * size; e < (g + 1) * size; ++e) sc[e] = -INFINITY;
     }
-    __syncthreads();
+    moe_wave_sync();
   }
   float total = 0.f;
   for (int j = 0; j < top; ++j) {
@@ -94,18 +109,24 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
     }
     const float w = correction ? plain[at] : mode == 0 ? best : best / sum;
     if (lane == 0) {
-      chosen[t * top + j] = at;
-      weight[t * top + j] = renorm ? w : w * factor;
+      chosen[j] = at;
+      weight[j] = p.renorm ? w : w * p.factor;
     }
     total += w;
-    __syncthreads();
+    moe_wave_sync();
     if (lane == 0) sc[at] = -INFINITY;
-    __syncthreads();
+    moe_wave_sync();
   }
-  if (renorm) {
-    __syncthreads();
-    for (int j = lane; j < top; j += 64) weight[t * top + j] = weight[t * top + j] / total * factor;
+  if (p.renorm) {
+    moe_wave_sync();
+    for (int j = lane; j < top; j += 64) weight[j] = weight[j] / total * p.factor;
   }
+}
+
+__global__ __launch_bounds__(64) void moe_route_kernel(MoeRoute p, int* __restrict__ chosen, float* __restrict__ weight) {
+  extern __shared__ float sc[];
+  const size_t t = blockIdx.x;
+  moe_route_token(p, t, sc, chosen + t * p.top, weight + t * p.top);
 }
 
 extern "C" int ta_moe_route(hipStream_t stream, const float* logits, const float* bias, int ld, int nt, int E,
@@ -118,8 +139,8 @@ extern "C" int ta_moe_route(hipStream_t stream, const float* logits, const float
   if (nt == 0) return 0;
   const size_t lds = ((size_t)E + groups + (correction ? E : 0)) * sizeof(float);
   TA_REQUIRE(lds <= 65536, "ta_moe_route: %d experts in %d groups do not fit the LDS", E, groups);
-  moe_route_kernel<<<nt, 64, lds, stream>>>(logits, ld, E, top, mode, renorm, chosen, weight, bias, groups, keep,
-                                            correction, factor);
+  const MoeRoute p = {logits, ld, E, top, mode, renorm, bias, groups, keep, correction, factor};
+  moe_route_kernel<<<nt, 64, lds, stream>>>(p, chosen, weight);
   return ta_check_launch("ta_moe_route");
 }
 
@@ -189,6 +210,97 @@ extern "C" int ta_moe_plan(hipStream_t stream, const int* chosen, int pairs, int
   moe_plan_kernel<<<1, 1024, (size_t)(2 * E + 1) * sizeof(int), stream>>>(chosen, pairs, E, max_rows, row_pair,
                                                                         tile_expert, pair_row);
   return ta_check_launch("ta_moe_plan");
+}
+
+// Routing and ordering for a step of few tokens in one launch: a workgroup of 16 waves, a wave a token, then the
+// plan as above with the experts' runs added up by one wave. 4 tokens of 32 experts: 7.0 us, where the two launches
+// take 5.4 + 3.9 and the trip between them.
+#define MOE_FEW_TOKENS 16
+#define MOE_FEW_EXPERTS 256
+__global__ __launch_bounds__(1024) void moe_route_plan_kernel(MoeRoute p, int nt, int experts, int max_rows,
+                                                              int* __restrict__ chosen, float* __restrict__ weight,
+                                                              int* __restrict__ row_pair, int* __restrict__ tile_expert,
+                                                              int* __restrict__ pair_row) {
+  extern __shared__ float moe_few[];      // a token's scores for every wave, then count [experts], start [experts + 1], chosen [pairs]
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE, pairs = nt * p.top;
+  int* count = reinterpret_cast<int*>(moe_few + MOE_FEW_TOKENS * p.lds());
+  int* start = count + experts;
+  int* mine = start + experts + 1;
+  for (int e = threadIdx.x; e < experts; e += 1024) count[e] = 0;
+  for (int i = threadIdx.x; i < max_rows; i += 1024) row_pair[i] = -1;
+  if (wave < nt) {
+    moe_route_token(p, wave, moe_few + wave * p.lds(), mine + wave * p.top, weight + wave * p.top);
+    moe_wave_sync();
+    for (int j = lane; j < p.top; j += TA_WAVE) chosen[wave * p.top + j] = mine[wave * p.top + j];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < pairs; i += 1024)
+    if (mine[i] < experts) atomicAdd(&count[mine[i]], 1);
+  __syncthreads();
+  if (wave == 0) {
+    int run = 0;
+    for (int e0 = 0; e0 < experts; e0 += TA_WAVE) {
+      const int e = e0 + lane;
+      const int n = e < experts ? (count[e] + MOE_TILE - 1) / MOE_TILE * MOE_TILE : 0;
+      int inc = n;
+#pragma unroll
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const int up = __shfl_up(inc, o, TA_WAVE);
+        if (lane >= o) inc += up;
+      }
+      if (e < experts) {
+        start[e] = run + inc - n;
+        count[e] = 0;
+      }
+      run += __shfl(inc, TA_WAVE - 1, TA_WAVE);
+    }
+    if (lane == 0) start[experts] = run;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < max_rows / MOE_TILE; i += 1024) {
+    const int r = i * MOE_TILE;
+    int e = -1;
+    if (r < start[experts]) {
+      int lo = 0, hi = experts - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start[mid] <= r) lo = mid; else hi = mid - 1;
+      }
+      e = lo;
+    }
+    tile_expert[i] = e;
+  }
+  for (int i = threadIdx.x; i < pairs; i += 1024) {
+    const int e = mine[i];
+    int r = -1;
+    if (e < experts) {
+      r = start[e] + atomicAdd(&count[e], 1);
+      row_pair[r] = i;
+    }
+    pair_row[i] = r;
+  }
+}
+
+// Whether ta_moe_route_plan takes a step of this many tokens.
+extern "C" int ta_moe_few_tokens(int nt, int E, int top) {
+  return nt >= 1 && nt <= MOE_FEW_TOKENS && E <= MOE_FEW_EXPERTS && top <= 32;
+}
+
+// ta_moe_route over E scores a token, then ta_moe_plan for `experts` experts with matrices (E or fewer).
+extern "C" int ta_moe_route_plan(hipStream_t stream, const float* logits, const float* bias, int ld, int nt, int E,
+                                 int top, int mode, int renorm, int groups, int keep, const float* correction,
+                                 float factor, int* chosen, float* weight, int experts, int max_rows, int* row_pair,
+                                 int* tile_expert, int* pair_row) {
+  TA_REQUIRE(ta_moe_few_tokens(nt, E, top) && E >= 1 && top >= 1 && top <= E && ld >= E && (mode == 0 || mode == 1),
+             "ta_moe_route_plan: bad sizes nt=%d experts=%d top=%d ld=%d", nt, E, top, ld);
+  TA_REQUIRE(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (E / groups),
+             "ta_moe_route_plan: %d experts in %d groups of which %d stay do not hold %d choices", E, groups, keep, top);
+  TA_REQUIRE(experts >= 1 && experts <= E && max_rows == ta_moe_max_rows(nt * top, experts),
+             "ta_moe_route_plan: %d rows for %d pairs of %d experts", max_rows, nt * top, experts);
+  const MoeRoute p = {logits, ld, E, top, mode, renorm, bias, groups, keep, correction, factor};
+  const size_t lds = ((size_t)MOE_FEW_TOKENS * p.lds() + 2 * experts + 1 + nt * top) * sizeof(float);
+  moe_route_plan_kernel<<<1, 1024, lds, stream>>>(p, nt, experts, max_rows, chosen, weight, row_pair, tile_expert, pair_row);
+  return ta_check_launch("ta_moe_route_plan");
 }
 
 // ------------------------------------------------------------------ gathering the rows
@@ -393,53 +505,102 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16_t* __rest
   }
 }
 
-// Few tiles (a step of few tokens): a workgroup owns ONE tile of 16 rows and 64 columns and its
-// four waves divide K, so that four times as many loads of the expert's matrix are on their way;
-// the partial tiles are added in wave order through LDS.
-template <typename TC>
-__global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(const bf16_t* __restrict__ A,
-                                                                   const bf16_t* __restrict__ W,
+__device__ uint4 moe_zeros;             // where a piece past K is read from (never written: zero)
+
+// Few tiles (a step of few tokens), bound by reading the chosen experts' matrices: a workgroup owns ONE tile of 16
+// rows and 64 rows of the matrix and its four waves divide K; the partial tiles are added in wave order through
+// LDS. While 128 k are multiplied the next are on their way (16 KB a wave).
+// row_pair (or null: A holds the ordered rows): the tile's rows are read from the tokens' rows h, each times its
+// pair's weight, rounded as moe_gather rounds it: a step of few tokens needs no ordered copy.
+// GLU: the matrix holds gate rows, then up rows; the workgroup takes 32 of each and joins them.
+struct MoeRows {
+  const bf16_t* A;
+  const int* row_pair;
+  const float* weight;
+  int top;
+};
+template <typename TC, bool GLU>
+__global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows, const bf16_t* __restrict__ W,
                                                                    const int* __restrict__ tile_expert,
-                                                                   TC* __restrict__ C, int N, int K, int act) {
+                                                                   TC* __restrict__ C, int N, int K, int act, TaGlu glu) {
   __shared__ float red[4][16][65];
   const int e = tile_expert[blockIdx.y];
   if (e < 0) return;                                    // the whole workgroup: tiles past the last expert's rows
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int r = lane % 16, kb = lane / 16;
-  const int n0 = blockIdx.x * 64;
+  constexpr int COLS = GLU ? 32 : 64;                   // of C
+  const int n0 = blockIdx.x * COLS;
   const size_t r0 = (size_t)blockIdx.y * MOE_TILE;
-  const bf16_t* We = W + (size_t)e * N * K;
+  const bf16_t* We = W + (size_t)e * (GLU ? 2 : 1) * N * K;
   const int steps = (K + 31) / 32;
   const int kbeg = 32 * (steps * wave / 4), kend = 32 * (steps * (wave + 1) / 4);
-  const bf16_t* arow = A + (r0 + r) * K + kb * 8;
-  const bf16_t* wrow[4];
-  bool wok[4];
+  const int pair = rows.row_pair ? rows.row_pair[r0 + r] : 0;    // asked for before the matrix, needed behind it
+  const bf16_t* wrow[4];                                // rows past N: another row, whose products are not stored
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    const int n = n0 + 16 * t + r;
-    wok[t] = n < N;
-    wrow[t] = We + (size_t)(wok[t] ? n : 0) * K + kb * 8;
+    const int n = n0 + (GLU ? 16 * (t % 2) : 16 * t) + r;
+    wrow[t] = We + (size_t)((n < N ? n : N - 1) + (GLU && t >= 2 ? N : 0)) * K + kb * 8;
   }
   moe_floatx4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
   constexpr int DEPTH = 4;                              // steps of 32 k asked for together
-  for (int k0 = kbeg; k0 < kend; k0 += 32 * DEPTH) {
-    MoeFrag af[DEPTH], wf[DEPTH][4];
+  MoeFrag af[2][DEPTH], wf[2][DEPTH][4];
+  auto load_matrix = [&](int set, int k0) {
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) {
       const int k = k0 + 32 * u;
       const bool kok = k < kend && k + kb * 8 < K;
-      af[u].q = kok ? *reinterpret_cast<const moe_u32x4*>(arow + k) : moe_zero4();
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        wf[u][t].q = (kok && wok[t]) ? __builtin_nontemporal_load(reinterpret_cast<const moe_u32x4*>(wrow[t] + k)) : moe_zero4();
+        wf[set][u][t].q = __builtin_nontemporal_load(
+            reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(wrow[t] + k) : (const void*)&moe_zeros));
     }
+  };
+  load_matrix(0, kbeg);
+  __builtin_amdgcn_sched_barrier(0);
+  const bf16_t* arow = rows.A + (r0 + r) * K + kb * 8;
+  float factor = 1.f;
+  if (rows.row_pair) {                                  // a row that only fills the tile: any token's, never read again
+    arow = rows.A + (size_t)(pair >= 0 ? pair / rows.top : 0) * K + kb * 8;
+    if (rows.weight) factor = pair >= 0 ? rows.weight[pair] : 0.f;
+  }
+  const bool weighs = rows.row_pair && rows.weight;
+  auto load_rows = [&](int set, int k0) {
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u)
+    for (int u = 0; u < DEPTH; ++u) {
+      const int k = k0 + 32 * u;
+      const bool kok = k < kend && k + kb * 8 < K;
+      af[set][u].q = *reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(arow + k) : (const void*)&moe_zeros);
+    }
+  };
+  auto multiply = [&](int set) {
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) {
+      if (weighs) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t x = af[set][u].q[i];
+          af[set][u].q[i] = f32x2_to_bf16x2_bits(__uint_as_float(x << 16) * factor, __uint_as_float(x & 0xffff0000u) * factor);
+        }
+      }
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][t].v, af[u].v, acc[t], 0, 0, 0);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][u][t].v, af[set][u].v, acc[t], 0, 0, 0);
+    }
+  };
+  load_rows(0, kbeg);
+  for (int k0 = kbeg; k0 < kend; k0 += 64 * DEPTH) {
+    load_matrix(1, k0 + 32 * DEPTH);
+    load_rows(1, k0 + 32 * DEPTH);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_matrix(0, k0 + 64 * DEPTH);
+    load_rows(0, k0 + 64 * DEPTH);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -447,10 +608,18 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(const bf16_t*
     for (int j = 0; j < 4; ++j) red[wave][r][16 * t + 4 * kb + j] = acc[t][j];
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = threadIdx.x + 256 * i, row = idx / 64, col = idx % 64;
-    const float v = (red[0][row][col] + red[1][row][col]) + (red[2][row][col] + red[3][row][col]);
-    if (n0 + col < N) C[(r0 + row) * N + n0 + col] = from_f32<TC>(moe_act(act, v));
+  for (int i = 0; i < COLS / 16; ++i) {
+    const int idx = threadIdx.x + 256 * i, row = idx / COLS, col = idx % COLS;
+    float v = (red[0][row][col] + red[1][row][col]) + (red[2][row][col] + red[3][row][col]);
+    if (GLU) {
+      const int up = col + 32;
+      const float u = (red[0][row][up] + red[1][row][up]) + (red[2][row][up] + red[3][row][up]);
+      // the product of its own stores gate and up in the engine's type
+      v = ta_glu(glu, to_f32(from_f32<bf16_t>(v)), to_f32(from_f32<bf16_t>(u)));
+    } else {
+      v = moe_act(act, v);
+    }
+    if (n0 + col < N) C[(r0 + row) * N + n0 + col] = from_f32<TC>(v);
   }
 }
 
@@ -630,6 +799,33 @@ static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A,
   return ta_check_launch("ta_moe_gemm");
 }
 
+// Whether the experts' product of this many ordered rows takes the form for few tiles (bfloat16).
+extern "C" int ta_moe_few_rows(int max_rows, int N, int K) {
+  return K % 8 == 0 && (long long)(max_rows / MOE_TILE) * ((N + 255) / 256) < 1024;
+}
+
+// The first product of the experts of a step of few tokens, from the tokens' rows h [nt, K]: C [max_rows, N] in
+// bfloat16. glu: W is [E, 2 N, K], gate rows then up rows, joined by silu (limit 0) or the limited form; else W is
+// [E, N, K] and `act` as in ta_moe_gemm. weight (or null): of the pairs, acts on the rows.
+extern "C" int ta_moe_gemm_tokens(hipStream_t stream, const void* h, int nt, const int* row_pair, const float* weight, int top,
+                                  const void* W, const int* tile_expert, void* C, int max_rows, int N, int K, int act, int glu,
+                                  float limit, float slope, float shift) {
+  TA_REQUIRE(nt >= 1 && top >= 1 && max_rows >= 0 && max_rows % MOE_TILE == 0 && N > 0 && K > 0 && K % 8 == 0 && act >= 0 && act <= 4 &&
+                 (uintptr_t)h % 16 == 0 && (uintptr_t)W % 16 == 0,
+             "ta_moe_gemm_tokens: bad sizes rows=%d N=%d K=%d act=%d", max_rows, N, K, act);
+  if (max_rows == 0) return 0;
+  const MoeRows rows = {(const bf16_t*)h, row_pair, weight, top};
+  const TaGlu g = {limit, slope, shift};
+  const int tiles = max_rows / MOE_TILE;
+  if (glu)
+    moe_gemm_mfma_splitk_kernel<bf16_t, true><<<dim3((N + 31) / 32, tiles), 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert,
+                                                                                            (bf16_t*)C, N, K, 0, g);
+  else
+    moe_gemm_mfma_splitk_kernel<bf16_t, false><<<dim3((N + 63) / 64, tiles), 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert,
+                                                                                             (bf16_t*)C, N, K, act, g);
+  return ta_check_launch("ta_moe_gemm_tokens");
+}
+
 // form: 0 = chosen by the shape; 1 = the waves divide K (few tiles); 2 = runs of tiles with operands
 // straight from memory; 3 = operands through LDS (many tiles). 1 to 3 take bfloat16 with K % 8 == 0.
 extern "C" int ta_moe_gemm_form(hipStream_t stream, int dtype, int out_dtype, const void* A, const void* W,
@@ -642,14 +838,16 @@ extern "C" int ta_moe_gemm_form(hipStream_t stream, int dtype, int out_dtype, co
   const int tiles = max_rows / MOE_TILE;
   if (dtype == TA_BF16 && K % 8 == 0) {
     if (out_dtype != TA_BF16 && out_dtype != TA_F32) return ta_fail("ta_moe_gemm: unknown output type %d", out_dtype);
-    const bool few = (long long)tiles * ((N + 255) / 256) < 1024;
+    const bool few = ta_moe_few_rows(max_rows, N, K);
     if (form == 3 || (form == 0 && !few)) return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, max_rows, tiles, N, K, act);
     if (form == 1 || (form == 0 && few)) {   // too few workgroups to fill the CUs: the waves divide K
       dim3 gk((N + 63) / 64, tiles);
+      const MoeRows rows = {(const bf16_t*)A, nullptr, nullptr, 1};
+      const TaGlu none = {0.f, 1.f, 0.f};
       if (out_dtype == TA_BF16)
-        moe_gemm_mfma_splitk_kernel<bf16_t><<<gk, 256, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, (bf16_t*)C, N, K, act);
+        moe_gemm_mfma_splitk_kernel<bf16_t, false><<<gk, 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert, (bf16_t*)C, N, K, act, none);
       else
-        moe_gemm_mfma_splitk_kernel<float><<<gk, 256, 0, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, (float*)C, N, K, act);
+        moe_gemm_mfma_splitk_kernel<float, false><<<gk, 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert, (float*)C, N, K, act, none);
       return ta_check_launch("ta_moe_gemm");
     }
     dim3 g((N + 255) / 256, (tiles + 3) / 4);
@@ -679,7 +877,10 @@ extern "C" int ta_moe_gemm(hipStream_t stream, int dtype, int out_dtype, const v
 }
 
 // ------------------------------------------------------------------ putting the rows back
-template <typename T>
+// A thread V columns of a token. V 4: rows of whole 16-byte pieces; the rows of up to four pairs are asked for together
+// and a token's columns are dealt out to several workgroups, so that a step of few tokens is one trip to memory and
+// not `top` times the columns of a thread (2 tokens, 4,096 columns, top 6: 20 us in one workgroup a token, 5 now).
+template <typename T, int V>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ rows, int d, int top,
                                                           const int* __restrict__ pair_row,
                                                           const float* __restrict__ weight,
@@ -688,34 +889,47 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
                                                           float* __restrict__ delta,
                                                           const float* __restrict__ extra, int xplanes, size_t xplane,
                                                           const T* __restrict__ h) {
-  extern __shared__ float cmb[];          // [top] rows of the token's pairs, [top] their weights
-  int* prow = reinterpret_cast<int*>(cmb);
-  float* pw = cmb + top;
+  typedef float vec __attribute__((ext_vector_type(V)));
   const size_t t = blockIdx.x;
-  for (int j = threadIdx.x; j < top; j += 256) {
-    prow[j] = pair_row[t * top + j];
-    pw[j] = weight ? weight[t * top + j] : 1.f;
-  }
+  const int c = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (c >= d) return;
+  const size_t at = t * d + c;
   float sg = 1.f;
   if (shared && shared_gate) sg = 1.0f / (1.0f + expf(-shared_gate[t * gate_ld]));
-  __syncthreads();
-  for (int c = threadIdx.x; c < d; c += 256) {
-    float s = 0.f;
-    const float own = h ? to_f32(h[t * d + c]) : 0.f;        // what an identity expert gives
-    for (int j = 0; j < top; ++j) {
-      const int r = prow[j];
-      const float y = rows[(size_t)(r >= 0 ? r : 0) * d + c];
-      s = fmaf(r >= 0 ? y : own, pw[j], s);
-    }
-    if (shared) {
-      float v = shared[t * d + c];
-      for (int p = 1; p < planes; ++p) v += shared[t * d + c + p * plane];
-      s += sg * v;
-    }
-    if (extra)      // what another sublayer adds to the stream beside this one, planes in order
-      for (int p = 0; p < xplanes; ++p) s += extra[t * d + c + p * xplane];
-    delta[t * d + c] = s;
+  vec s, own;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    s[i] = 0.f;
+    own[i] = h ? to_f32(h[at + i]) : 0.f;                    // what an identity expert gives
   }
+  for (int j0 = 0; j0 < top; j0 += 4) {
+    vec y[4];
+    float w[4];
+    int r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const size_t pair = t * top + (j0 + j < top ? j0 + j : j0);
+      r[j] = pair_row[pair];
+      w[j] = weight ? weight[pair] : 1.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = *reinterpret_cast<const vec*>(rows + (size_t)(r[j] >= 0 ? r[j] : 0) * d + c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (j0 + j < top) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) s[i] = fmaf(r[j] >= 0 ? y[j][i] : own[i], w[j], s[i]);
+      }
+  }
+  if (shared) {
+    vec v = *reinterpret_cast<const vec*>(shared + at);
+    for (int p = 1; p < planes; ++p) v += *reinterpret_cast<const vec*>(shared + at + p * plane);
+#pragma unroll
+    for (int i = 0; i < V; ++i) s[i] = fmaf(sg, v[i], s[i]);
+  }
+  if (extra)      // what another sublayer adds to the stream beside this one, planes in order
+    for (int p = 0; p < xplanes; ++p) s += *reinterpret_cast<const vec*>(extra + at + p * xplane);
+  *reinterpret_cast<vec*>(delta + at) = s;
 }
 
 // rows: [max_rows, d] float32, the experts' results in the planned order. weight: null when it
@@ -735,9 +949,19 @@ extern "C" int ta_moe_combine(hipStream_t stream, const float* rows, int d, int 
              "ta_moe_combine: %d planes of the further addend", xplanes);
   if (nt == 0) return 0;
 #define MOE_COMBINE(T)                                                                                          \
-  moe_combine_kernel<T><<<nt, 256, (size_t)2 * top * sizeof(float), stream>>>(                                  \
-      rows, d, top, pair_row, weight, shared, planes, (size_t)plane, shared_gate, gate_ld, delta, extra, xplanes, \
-      (size_t)xplane, (const T*)h)
+  do {                                                                                                          \
+    if (vec)                                                                                                    \
+      moe_combine_kernel<T, 4><<<dim3(nt, (d / 4 + 255) / 256), 256, 0, stream>>>(                              \
+          rows, d, top, pair_row, weight, shared, planes, (size_t)plane, shared_gate, gate_ld, delta, extra, xplanes, \
+          (size_t)xplane, (const T*)h);                                                                         \
+    else                                                                                                        \
+      moe_combine_kernel<T, 1><<<dim3(nt, (d + 255) / 256), 256, 0, stream>>>(                                  \
+          rows, d, top, pair_row, weight, shared, planes, (size_t)plane, shared_gate, gate_ld, delta, extra, xplanes, \
+          (size_t)xplane, (const T*)h);                                                                         \
+  } while (0)
+  const bool vec = d % 4 == 0 && plane % 4 == 0 && xplane % 4 == 0 &&
+                   ((uintptr_t)rows | (uintptr_t)shared | (uintptr_t)extra | (uintptr_t)delta) % 16 == 0;
+  TA_REQUIRE((d + 255) / 256 <= 65535, "ta_moe_combine: rows of %d", d);
   if (h_dtype == TA_F32) MOE_COMBINE(float); else MOE_COMBINE(bf16_t);
 #undef MOE_COMBINE
   return ta_check_launch("ta_moe_combine");

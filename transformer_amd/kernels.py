@@ -1711,16 +1711,8 @@ def moe_max_rows(pairs: int, experts: int) -> int:
     return n
 
 
-def moe_route(logits: torch.Tensor, experts: int, top: int, chosen: torch.Tensor, weight: torch.Tensor,
-              score: str = "sigmoid", renormalize: bool = False, bias: Optional[torch.Tensor] = None,
-              groups: int = 1, keep_groups: int = 1, correction: Optional[torch.Tensor] = None, factor: float = 1.0):
-    """chosen [nt, top] int32, weight [nt, top] float32: the ``top`` largest scores of the
-    first ``experts`` columns of logits [nt, >= experts] float32 (lowest index among equals).
-    bias [experts] float32: added to the logits first. "softmax" with ``renormalize`` is the
-    softmax over the chosen logits alone. groups > 1: the experts form that many equal groups of
-    neighbours, a group counts as its largest score, and only experts of the ``keep_groups`` best
-    groups can be chosen. correction [experts] float32: the choice compares score + correction, the weights
-    are the scores without it. factor: multiplies the weights (behind ``renormalize``)."""
+def _check_route(logits, experts, top, chosen, weight, score, bias, groups, keep_groups, correction) -> int:
+    """Checks what a routing is given; returns the logits' row stride."""
     _dev(logits, "logits", torch.float32, contiguous=False)
     nt, ld = _rows2d(logits, "logits")
     _dev(chosen, "chosen", torch.int32); _dev(weight, "weight", torch.float32)
@@ -1737,24 +1729,66 @@ def moe_route(logits: torch.Tensor, experts: int, top: int, chosen: torch.Tensor
         _dev(correction, "correction", torch.float32)
         if correction.shape != (experts,):
             raise KernelError(f"moe_route: correction is {tuple(correction.shape)}, expected {(experts,)}")
+    return ld
+
+
+def moe_route(logits: torch.Tensor, experts: int, top: int, chosen: torch.Tensor, weight: torch.Tensor,
+              score: str = "sigmoid", renormalize: bool = False, bias: Optional[torch.Tensor] = None,
+              groups: int = 1, keep_groups: int = 1, correction: Optional[torch.Tensor] = None, factor: float = 1.0):
+    """chosen [nt, top] int32, weight [nt, top] float32: the ``top`` largest scores of the
+    first ``experts`` columns of logits [nt, >= experts] float32 (lowest index among equals).
+    bias [experts] float32: added to the logits first. "softmax" with ``renormalize`` is the
+    softmax over the chosen logits alone. groups > 1: the experts form that many equal groups of
+    neighbours, a group counts as its largest score, and only experts of the ``keep_groups`` best
+    groups can be chosen. correction [experts] float32: the choice compares score + correction, the weights
+    are the scores without it. factor: multiplies the weights (behind ``renormalize``)."""
+    ld = _check_route(logits, experts, top, chosen, weight, score, bias, groups, keep_groups, correction)
+    nt = logits.shape[0]
     _check(library().ta_moe_route(_stream(), _ptr(logits), _ptr(bias), c_int(ld), c_int(nt), c_int(experts),
                                   c_int(top), c_int(_ROUTE_MODES[score]), c_int(int(renormalize)), c_int(groups),
                                   c_int(keep_groups), _ptr(correction), c_float(factor), _ptr(chosen), _ptr(weight)))
     return chosen, weight
 
 
-def moe_plan(chosen: torch.Tensor, experts: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
-             pair_row: torch.Tensor):
-    """Orders the (token, choice) pairs by expert; see ``moe_max_rows`` for row_pair's size. A choice of
-    ``experts`` or more gets no row (pair_row -1): an expert without matrices."""
+def _check_plan(chosen, experts, row_pair, tile_expert, pair_row) -> int:
+    """Checks the tables of an ordering; returns the ordered rows."""
     _dev(chosen, "chosen", torch.int32); _dev(row_pair, "row_pair", torch.int32)
     _dev(tile_expert, "tile_expert", torch.int32); _dev(pair_row, "pair_row", torch.int32)
     pairs = chosen.numel()
     rows = moe_max_rows(pairs, experts)
     if row_pair.numel() != rows or tile_expert.numel() != rows // 16 or pair_row.numel() != pairs:
         raise KernelError(f"moe_plan: {pairs} pairs of {experts} experts need {rows} rows")
+    return rows
+
+
+def moe_plan(chosen: torch.Tensor, experts: int, row_pair: torch.Tensor, tile_expert: torch.Tensor,
+             pair_row: torch.Tensor):
+    """Orders the (token, choice) pairs by expert; see ``moe_max_rows`` for row_pair's size. A choice of
+    ``experts`` or more gets no row (pair_row -1): an expert without matrices."""
+    rows = _check_plan(chosen, experts, row_pair, tile_expert, pair_row)
+    pairs = chosen.numel()
     _check(library().ta_moe_plan(_stream(), _ptr(chosen), c_int(pairs), c_int(experts), c_int(rows), _ptr(row_pair),
                                  _ptr(tile_expert), _ptr(pair_row)))
+
+
+def moe_route_plan(logits: torch.Tensor, outputs: int, top: int, chosen: torch.Tensor, weight: torch.Tensor, experts: int,
+                   row_pair: torch.Tensor, tile_expert: torch.Tensor, pair_row: torch.Tensor, score: str = "sigmoid",
+                   renormalize: bool = False, bias: Optional[torch.Tensor] = None, groups: int = 1, keep_groups: int = 1,
+                   correction: Optional[torch.Tensor] = None, factor: float = 1.0) -> None:
+    """``moe_route`` over the ``outputs`` of the router, then ``moe_plan`` for its first ``experts``: one launch where
+    the step has few tokens (up to 16, of up to 256 outputs and 32 choices), two otherwise."""
+    nt = logits.shape[0]
+    if not library().ta_moe_few_tokens(c_int(nt), c_int(outputs), c_int(top)):
+        moe_route(logits, outputs, top, chosen, weight, score, renormalize, bias=bias, groups=groups,
+                  keep_groups=keep_groups, correction=correction, factor=factor)
+        moe_plan(chosen, experts, row_pair, tile_expert, pair_row)
+        return
+    ld = _check_route(logits, outputs, top, chosen, weight, score, bias, groups, keep_groups, correction)
+    rows = _check_plan(chosen, experts, row_pair, tile_expert, pair_row)
+    _check(library().ta_moe_route_plan(
+        _stream(), _ptr(logits), _ptr(bias), c_int(ld), c_int(nt), c_int(outputs), c_int(top), c_int(_ROUTE_MODES[score]),
+        c_int(int(renormalize)), c_int(groups), c_int(keep_groups), _ptr(correction), c_float(factor), _ptr(chosen),
+        _ptr(weight), c_int(experts), c_int(rows), _ptr(row_pair), _ptr(tile_expert), _ptr(pair_row)))
 
 
 def moe_gather(h: torch.Tensor, top: int, row_pair: torch.Tensor, weight, out: torch.Tensor) -> torch.Tensor:
@@ -1787,6 +1821,37 @@ def moe_gemm(a: torch.Tensor, w: torch.Tensor, tile_expert: torch.Tensor, out: t
     _check(library().ta_moe_gemm_form(_stream(), c_int(_code(a.dtype)), c_int(_code(out.dtype)), _ptr(a), _ptr(w),
                                       _ptr(tile_expert), _ptr(out), c_int(rows), c_int(w.shape[1]), c_int(K),
                                       c_int(_MOE_ACTS[act]), c_int(_MOE_FORMS[form])))
+    return out
+
+
+def moe_takes_tokens(h: torch.Tensor, rows: int, w: torch.Tensor) -> bool:
+    """Whether the experts' first product reads the tokens' rows themselves (``moe_gemm_tokens``): bfloat16 steps whose
+    ordered rows are few enough for the form that divides k; more rows are cheaper ordered first, since every
+    column block of the product reads them again."""
+    return h.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and h.is_contiguous() and h.data_ptr() % 16 == 0 and \
+        w.data_ptr() % 16 == 0 and bool(library().ta_moe_few_rows(c_int(rows), c_int(w.shape[1]), c_int(w.shape[2])))
+
+
+def moe_gemm_tokens(h: torch.Tensor, top: int, row_pair: torch.Tensor, weight, w: torch.Tensor, tile_expert: torch.Tensor,
+                    out: torch.Tensor, act: Optional[str] = None, glu: bool = False,
+                    limits: Optional[Sequence[float]] = None) -> torch.Tensor:
+    """``moe_gather`` and the experts' first ``moe_gemm`` in one: h [nt, K], out [rows, N] bfloat16. glu: w is [E, 2 N, K]
+    (gate rows, up rows) and out = silu(gate) * up, or with limits = (limit, slope, shift) joined as ``glu_limit``
+    does; else w is [E, N, K] and ``act`` is applied. weight (or None) [nt, top] acts on the rows."""
+    _dev(h, "h", torch.bfloat16); _dev(w, "w", torch.bfloat16); _dev(out, "out", torch.bfloat16)
+    _dev(row_pair, "row_pair", torch.int32); _dev(tile_expert, "tile_expert", torch.int32)
+    (nt, K), (rows, N) = h.shape, out.shape
+    if weight is not None:
+        _dev(weight, "weight", torch.float32)
+        if weight.numel() != nt * top:
+            raise KernelError(f"moe_gemm_tokens: {weight.numel()} weights for {nt} tokens x {top}")
+    if act not in _MOE_ACTS or (glu and act is not None) or w.dim() != 3 or w.shape[2] != K or \
+            w.shape[1] != (2 * N if glu else N) or row_pair.numel() != rows or tile_expert.numel() * 16 != rows:
+        raise KernelError(f"moe_gemm_tokens: h {tuple(h.shape)} w {tuple(w.shape)} out {tuple(out.shape)} act {act!r}")
+    _check(library().ta_moe_gemm_tokens(
+        _stream(), _ptr(h), c_int(nt), _ptr(row_pair), _ptr(weight), c_int(top), _ptr(w), _ptr(tile_expert), _ptr(out),
+        c_int(rows), c_int(N), c_int(K), c_int(_MOE_ACTS[act]), c_int(int(glu)),
+        *[c_float(v) for v in (limits or (0.0, 1.0, 0.0))]))
     return out
 
 

@@ -215,24 +215,29 @@ class RoutedMLP(Part):
         logits = linear(h, self.w["router.weight"], ws.take("moe.logits", (nt, R + int(self.gated_shared)), torch.float32))
         chosen = ws.take("moe.chosen", (nt, top), torch.int32)
         weight = ws.take("moe.weight", (nt, top), torch.float32)
-        kernels.moe_route(logits, R, top, chosen, weight, s.score, s.renormalize, bias=self.w.get("router.bias"),
-                          groups=self.groups, keep_groups=self.keep_groups, correction=self.w.get("router.correction"),
-                          factor=float(getattr(s, "factor", 1.0)))
-        if getattr(ctx, "dump", None) is not None:
-            ctx.dump("experts", chosen)
         rows = kernels.moe_max_rows(nt * top, E)
         row_pair = ws.take("moe.row_pair", (rows,), torch.int32)
         tile_expert = ws.take("moe.tile_expert", (rows // 16,), torch.int32)
         pair_row = ws.take("moe.pair_row", (nt * top,), torch.int32)
-        kernels.moe_plan(chosen, E, row_pair, tile_expert, pair_row)
+        kernels.moe_route_plan(logits, R, top, chosen, weight, E, row_pair, tile_expert, pair_row, s.score, s.renormalize,
+                               bias=self.w.get("router.bias"), groups=self.groups, keep_groups=self.keep_groups,
+                               correction=self.w.get("router.correction"), factor=float(getattr(s, "factor", 1.0)))
+        if getattr(ctx, "dump", None) is not None:
+            ctx.dump("experts", chosen)
         on_input = s.weight_on == "input"
-        a = kernels.moe_gather(h, top, row_pair, weight if on_input else None, ws.take("moe.a", (rows, d), self.dtype))
         first, k = ("gate_up", 2) if self.two else ("up", 1)
         up = self.w[f"experts.{first}.weight"].view(E, k * ff, d)
         down = self.w["experts.down.weight"].view(E, d, ff)
         if up.dtype != self.dtype:
             raise PartError(f"the experts' matrices are {up.dtype}, the engine computes in {self.dtype}")
-        mid = self._first(a, up, tile_expert, ws, "moe.mid", ff, getattr(s, "limit", 0.0))
+        acts = weight if on_input else None
+        if kernels.moe_takes_tokens(h, rows, up) and not (self.glu and s.activation != "silu"):
+            limits = (float(s.limit), float(s.gate_slope), float(s.up_shift)) if self.limited else None
+            mid = kernels.moe_gemm_tokens(h, top, row_pair, acts, up, tile_expert, ws.take("moe.mid", (rows, ff), self.dtype),
+                                          None if self.two else s.activation, glu=self.two, limits=limits)
+        else:
+            a = kernels.moe_gather(h, top, row_pair, acts, ws.take("moe.a", (rows, d), self.dtype))
+            mid = self._first(a, up, tile_expert, ws, "moe.mid", ff, getattr(s, "limit", 0.0))
         out = kernels.moe_gemm(mid, down, tile_expert, ws.take("moe.out", (rows, d), torch.float32))
         shared = None
         if s.shared_intermediate is not None:
