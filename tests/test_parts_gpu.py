@@ -171,6 +171,24 @@ def test_a_long_k_product_of_a_short_prompt_is_left_in_planes(rows):
         assert np.abs(f64(x) - (x0 + want)).max() < tol
 
 
+@pytest.mark.parametrize("rows", [1024, 1030, 1300])
+def test_a_product_over_a_long_k_in_whole_rounds_and_a_rest(rows):
+    """16,384 columns fill the CUs once with 1,024 rows: the rows of every call join the stream at their own place."""
+    from transformer_amd.parts.linear import Workspace, library_rows, linear_delta
+    n, k = 16384, 10240
+    assert library_rows(rows, n, k) == ([rows] if rows == 1024 else [1024, rows - 1024] if rows == 1300 else [1024, 6])
+    assert library_rows(9000, 4096, 11008) == [8192, 808] and library_rows(4915, 4096, 14336) == [4915]
+    assert library_rows(5000, 4096, 8192) == [5000] and sum(library_rows(70001, 8192, 28672)) == 70001
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    x = torch.randn(rows, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn(n, k, generator=g, device=DEV) * 0.01).bfloat16()
+    stream = torch.randn(rows, n, generator=g, device=DEV)
+    want = stream + x.float() @ w.float().t()
+    assert linear_delta(x, w, Workspace(DEV), "t", into=stream) is None
+    # float32 sums of 10,240 products of order 0.01 in two orders
+    assert (stream - want).abs().max() < 1e-6 * k ** 0.5 * 8
+
+
 # ---------------------------------------------------------------- a toy mixer with state
 @dataclass(frozen=True)
 class RunningSumSpec:

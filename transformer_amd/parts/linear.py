@@ -98,6 +98,31 @@ def library_planes(rows: int, weight: torch.Tensor) -> int:
     return planes
 
 
+def library_rows(rows: int, n: int, k: int) -> list:
+    """Row counts of the calls in which the vendor library is given a float32 product of many rows over a long k.
+
+    Its tiles of 256 x 256 fill the 256 CUs in rounds, and it runs at 1.3 to 1.45 PFLOP/s while the last round is
+    nearly full, nearly half or nearly a quarter full (it then cuts that round along k by 1, 2 or 4). Between those,
+    and with more than two rounds, it falls to half for k from about 10,000 on: 4,096 columns over k = 11,008 take
+    258 us at 3,904 rows, 592 at 4,128, 330 at 4,800, 638 at 5,248, 399 at 5,920, 743 at 7,040, 905 at 9,000; in two
+    calls, whole rounds and the rest, 282 us at 4,128, 376 at 5,248, 462 at 7,040, 623 at 9,000 (where it does well by
+    itself two calls cost up to 7 % more). The same holds for 4,096 columns over 14,336 and for 8,192 over 28,672; over
+    k = 8,192 one call is as good everywhere."""
+    full = 256 * (256 * 256 // max(256, n))            # rows whose tiles fill the CUs once
+    if k < 10240 or n % 256 or rows <= full:
+        return [rows]
+    calls = []
+    while rows > 2 * full:
+        calls.append(2 * full)
+        rows -= 2 * full
+    rest = rows - full
+    if rest > 0 and not any(part - full // 8 < rest <= part for part in (full // 4, full // 2, full)):
+        calls += [full, rest]
+    else:
+        calls.append(rows)
+    return calls
+
+
 def adds_in_place(rows: int, weight: torch.Tensor) -> bool:
     """Whether ``linear_delta`` can add this product to the residual stream by itself: the
     vendor library's product in one plane, which takes what it adds to as its third operand."""
@@ -123,7 +148,11 @@ def linear_delta(x: torch.Tensor, weight: torch.Tensor, ws: Workspace, name: str
                 or into.dtype != torch.float32:
             raise kernels.KernelError(f"linear_delta: cannot add {tuple(x.shape)} x {tuple(weight.shape)} "
                                       f"in place into {tuple(into.shape)} {into.dtype}")
-        torch.addmm(into, x, weight.t(), out_dtype=torch.float32, out=into)
+        at = 0
+        for rows in library_rows(nt, n, x.shape[1]):
+            part = into[at:at + rows]
+            torch.addmm(part, x[at:at + rows], weight.t(), out_dtype=torch.float32, out=part)
+            at += rows
         return None
     if x.dtype == torch.bfloat16 and nt > 0 and kernels.mid_takes(nt, weight) \
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
