@@ -144,6 +144,44 @@ def test_rope_kv_write(dtype, dh, style, many):
         assert np.isnan(rest_k).all() and np.isnan(rest_v).all()                # nothing else touched
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("nq,nkv,dh,style,cache", [(3, 2, 48, "half", True), (2, 2, 128, "interleaved", True),
+                                                   (4, 1, 16, "interleaved", True), (2, 1, 64, "half", False), (2, 1, 256, "half", True)])
+def test_rope_kv_write_of_prompts(dtype, nq, nkv, dh, style, cache):
+    """64 tokens and more: whole groups of places, groups cut by a page's end, by the end of a sequence and by the
+    end of a block of 64 tokens, tokens that are not stored; nothing but their places is written."""
+    from transformer_amd import kernels
+    own = np.random.default_rng([nq, dh])
+    dest = [5 * 64 + i for i in range(64)] + [2 * 64 + i for i in range(7)] + [4 * 64 + 13 + i for i in range(51)] + \
+        [0 * 64 + i for i in range(9)] + [-1, -1] + [1 * 64 + 5, 1 * 64 + 6]
+    nt, pages = len(dest), 7
+    pos = own.integers(0, 5000, nt).tolist()
+    qkv = rounded(own.normal(size=(nt, nq + 2 * nkv, dh)), dtype)
+    bias = own.normal(size=((nq + 2 * nkv), dh)).astype(np.float32) * 0.1
+    inv = P.rope_inv_freq(dh, 12345.0)
+    ang = kernels.rope_table(dev(pos, torch.int32), dev(inv), torch.empty(nt, dh // 2, 2, device=DEV))
+    for b in (None, bias):
+        t = dev(qkv.reshape(nt, -1), DT[dtype])
+        kc = torch.full((pages, nkv, 64, dh), float("nan"), dtype=DT[dtype], device=DEV)
+        vc = torch.full((pages, nkv, dh, 64), float("nan"), dtype=DT[dtype], device=DEV)
+        kernels.rope_kv_write(t, nq, nkv, dh, ang, style == "interleaved", dev(dest, torch.int32) if cache else None,
+                              kc if cache else None, vc if cache else None, None if b is None else dev(b.reshape(-1)))
+        src = qkv + (0 if b is None else b[None].astype(np.float64))
+        want = np.concatenate([P.rope(src[:, :nq + nkv], pos, 12345.0, style), src[:, nq + nkv:]], axis=1)
+        got, e = f64(t).reshape(nt, nq + 2 * nkv, dh), tol(dtype, 3)
+        assert np.abs(got - want).max() < e
+        if not cache:
+            continue
+        kcn, vcn = f64(kc), f64(vc).transpose(0, 1, 3, 2)
+        stored = [(i, d_) for i, d_ in enumerate(dest) if d_ >= 0]
+        for i, d_ in stored:
+            assert np.array_equal(kcn[d_ // 64, :, d_ % 64], got[i, nq:nq + nkv])
+            assert np.array_equal(vcn[d_ // 64, :, d_ % 64], got[i, nq + nkv:])
+        written = np.zeros((pages, 64), dtype=bool)
+        written[[d_ // 64 for _, d_ in stored], [d_ % 64 for _, d_ in stored]] = True
+        assert np.isnan(kcn.transpose(0, 2, 1, 3)[~written]).all() and np.isnan(vcn.transpose(0, 2, 1, 3)[~written]).all()
+
+
 def test_rope_without_rotation_only_stores():
     from transformer_amd import kernels
     qkv = rng.normal(size=(2, 4 * 16)).astype(np.float32)

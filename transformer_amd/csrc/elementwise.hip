@@ -530,6 +530,170 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
   }
 }
 
+// Prompts of 64 tokens and more, heads of whole 16 elements: bound by its bytes (q and k read and written, k and v
+// stored once more). q and k: a thread takes two runs of eight elements that hold each other's partners (style 0:
+// elements j..j+7 and those dh/2 further on; style 1: sixteen in a row) and asks for all it needs at once. v:
+// a workgroup takes 64 tokens of one kv head through LDS and stores the transposed page line by line: groups of
+// 16 bytes of neighbouring places, eight lanes a line of 128, where the kernel above wrote 8 bytes every 128 (a
+// line then went to memory in sixteen pieces). 4,454 tokens of 32 + 32 + 32 heads of 128: 201 -> 43.5 us (5.8 TB/s); 8,159 of 32 +
+// 8 + 8: 105 -> 36; 2,011: 18.6 -> 11.5.
+template <typename T> struct Run8 {
+  Vec4<T> a, b;
+  __device__ __forceinline__ void load(const T* p) {
+    if constexpr (sizeof(T) == 2) {
+      const uint4 v = *reinterpret_cast<const uint4*>(p);
+      a.v = make_uint2(v.x, v.y);
+      b.v = make_uint2(v.z, v.w);
+    } else {
+      a.load(p);
+      b.load(p + 4);
+    }
+  }
+  __device__ __forceinline__ void store(T* p) const {
+    if constexpr (sizeof(T) == 2) {
+      *reinterpret_cast<uint4*>(p) = make_uint4(a.v.x, a.v.y, b.v.x, b.v.y);
+    } else {
+      a.store(p);
+      b.store(p + 4);
+    }
+  }
+  __device__ __forceinline__ float get(int i) const { return i < 4 ? a.get(i) : b.get(i - 4); }
+  __device__ __forceinline__ void set(const float* x) {
+    a.set(x[0], x[1], x[2], x[3]);
+    b.set(x[4], x[5], x[6], x[7]);
+  }
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
+    T* __restrict__ qkv, const float* __restrict__ bias, const int* __restrict__ dest,
+    const float2* __restrict__ cs, int style, T* __restrict__ kcache, T* __restrict__ vcache,
+    int nt, int nq, int nkv, int dh, int turn_blocks) {
+  const size_t width = (size_t)(nq + 2 * nkv) * dh;
+  const bool cache = kcache != nullptr && dest != nullptr;
+  if ((int)blockIdx.x < turn_blocks) {
+    // ---- q and k heads
+    const int half = dh / 2, per_head = dh / 16;
+    const long long it = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (it >= (long long)nt * (nq + nkv) * per_head) return;
+    const int u = (int)(it % per_head);
+    const long long th = it / per_head;
+    const int h = (int)(th % (nq + nkv)), t = (int)(th / (nq + nkv));
+    const int o0 = style == 0 ? 8 * u : 16 * u, o1 = style == 0 ? 8 * u + half : 16 * u + 8;
+    T* v = qkv + (size_t)t * width + (size_t)h * dh;
+    const int sl = cache && h >= nq ? dest[t] : -1;
+    Run8<T> x0, x1;
+    x0.load(v + o0);
+    x1.load(v + o1);
+    float2 k[8];
+    if (cs) {
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const float4 c2 = *reinterpret_cast<const float4*>(cs + (size_t)t * half + 8 * u + e);
+        k[e] = make_float2(c2.x, c2.y);
+        k[e + 1] = make_float2(c2.z, c2.w);
+      }
+    }
+    float a[8], c[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      a[e] = x0.get(e);
+      c[e] = x1.get(e);
+      if (bias) {
+        a[e] += bias[(size_t)h * dh + o0 + e];
+        c[e] += bias[(size_t)h * dh + o1 + e];
+      }
+    }
+    if (cs) {
+      if (style == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float r0 = a[e] * k[e].x - c[e] * k[e].y, r1 = a[e] * k[e].y + c[e] * k[e].x;
+          a[e] = r0;
+          c[e] = r1;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+          const float2 ka = k[e / 2], kc = k[4 + e / 2];
+          const float a0 = a[e] * ka.x - a[e + 1] * ka.y, a1 = a[e] * ka.y + a[e + 1] * ka.x;
+          const float c0 = c[e] * kc.x - c[e + 1] * kc.y, c1 = c[e] * kc.y + c[e + 1] * kc.x;
+          a[e] = a0;
+          a[e + 1] = a1;
+          c[e] = c0;
+          c[e + 1] = c1;
+        }
+      }
+    }
+    x0.set(a);
+    x1.set(c);
+    if (bias || cs) {
+      x0.store(v + o0);
+      x1.store(v + o1);
+    }
+    if (sl >= 0) {
+      T* kc = kcache + (((size_t)(sl / TA_PAGE) * nkv + (h - nq)) * TA_PAGE + sl % TA_PAGE) * dh;
+      x0.store(kc + o0);
+      x1.store(kc + o1);
+    }
+    return;
+  }
+  // ---- v heads
+  extern __shared__ __attribute__((aligned(16))) unsigned char rope_lds[];
+  T* tile = reinterpret_cast<T*>(rope_lds);              // [64][dh + 2]
+  __shared__ int slot[64], first[65], groups_s;
+  constexpr int RUN = 16 / (int)sizeof(T);
+  const int unit = blockIdx.x - turn_blocks, g = unit % nkv, t0 = unit / nkv * 64;
+  const int ntok = nt - t0 < 64 ? nt - t0 : 64, ld = dh + 2;
+  const float* vb = bias ? bias + (size_t)(nq + nkv + g) * dh : nullptr;
+  if (threadIdx.x < 64) {
+    const int i = threadIdx.x;
+    const int sl = cache && i < ntok ? dest[t0 + i] : -1;
+    slot[i] = sl;
+    const int before = __shfl_up(sl, 1, TA_WAVE);
+    const bool starts = i < ntok && (i == 0 || sl != before + 1 || sl % RUN == 0);
+    const unsigned long long mask = __ballot(starts);
+    if (starts) first[__popcll(mask & (((unsigned long long)1 << i) - 1))] = i;
+    if (i == 0) {
+      groups_s = __popcll(mask);
+      first[__popcll(mask)] = ntok;
+    }
+  }
+  const int pieces = dh / 8;
+  for (int it = threadIdx.x; it < ntok * pieces; it += 256) {
+    const int i = it / pieces, o = it % pieces * 8;
+    T* from = qkv + (size_t)(t0 + i) * width + (size_t)(nq + nkv + g) * dh + o;
+    Run8<T> x;
+    x.load(from);
+    if (vb) {
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = x.get(e) + vb[o + e];
+      x.set(y);
+      x.store(from);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) tile[i * ld + o + e] = from_f32<T>(x.get(e));
+  }
+  __syncthreads();
+  if (!cache) return;
+  const int groups = groups_s;
+  for (int it = threadIdx.x; it < groups * dh; it += 256) {
+    const int q = it % groups, d = it / groups;
+    const int i0 = first[q], n = first[q + 1] - i0, sl = slot[i0];
+    if (sl < 0) continue;
+    T* to = vcache + (((size_t)(sl / TA_PAGE) * nkv + g) * dh + d) * TA_PAGE + sl % TA_PAGE;
+    if (n == RUN && sl % RUN == 0) {
+      struct alignas(16) { T x[RUN]; } line;
+#pragma unroll
+      for (int e = 0; e < RUN; ++e) line.x[e] = tile[(i0 + e) * ld + d];
+      *reinterpret_cast<uint4*>(to) = *reinterpret_cast<const uint4*>(&line);
+    } else {
+      for (int e = 0; e < n; ++e) to[e] = tile[(i0 + e) * ld + d];
+    }
+  }
+}
+
 extern "C" int ta_rope_kv_write(hipStream_t stream, int dtype, void* qkv, const float* bias,
                                 const int* dest, const float* cs, int style, void* kcache,
                                 void* vcache, int nt, int nq, int nkv, int dh) {
@@ -539,6 +703,21 @@ extern "C" int ta_rope_kv_write(hipStream_t stream, int dtype, void* qkv, const 
   TA_REQUIRE((kcache == nullptr) == (vcache == nullptr), "ta_rope_kv_write: K and V cache must come together");
   if (nt == 0) return 0;
   const bool aligned = ((uintptr_t)qkv % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && ((uintptr_t)vcache % 16) == 0;
+  const size_t tile = 64 * (size_t)(dh + 2) * (dtype == TA_F32 ? 4 : 2);       // of values on their way through LDS
+  if (nt >= 64 && dh % 16 == 0 && tile <= 40960 && aligned && ((uintptr_t)cs % 16) == 0 &&
+      (dtype == TA_F32 || dtype == TA_BF16)) {
+    const long long turns = ((long long)nt * (nq + nkv) * (dh / 16) + 255) / 256;
+    const long long lines = (kcache != nullptr && dest != nullptr) || bias ? (long long)((nt + 63) / 64) * nkv : 0;
+    TA_REQUIRE(turns + lines <= 2147483647ll, "ta_rope_kv_write: %d tokens of %d heads are too many for one launch", nt, nq + 2 * nkv);
+    const dim3 gl((unsigned)(turns + lines));
+    if (dtype == TA_F32)
+      rope_kv_write_lines_kernel<float><<<gl, 256, tile, stream>>>((float*)qkv, bias, dest, (const float2*)cs, style,
+                                                                   (float*)kcache, (float*)vcache, nt, nq, nkv, dh, (int)turns);
+    else
+      rope_kv_write_lines_kernel<bf16_t><<<gl, 256, tile, stream>>>((bf16_t*)qkv, bias, dest, (const float2*)cs, style,
+                                                                    (bf16_t*)kcache, (bf16_t*)vcache, nt, nq, nkv, dh, (int)turns);
+    return ta_check_launch("ta_rope_kv_write");
+  }
   if (nt >= 8 && dh % 8 == 0 && aligned && (dtype == TA_F32 || dtype == TA_BF16)) {
     const int groups = (nt + 3) / 4;
     int parts = 1;
