@@ -156,8 +156,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
 // eight lanes that are served together meet no bank twice. float32 operands go from memory to LDS without passing
 // through registers (a wave's 64 pieces land side by side, so the permutation is in the addresses they are read
 // from); other types are converted on the way. Half h of a wave multiplies pieces h and h + 2 of a block's four,
-// element by element: the order above. 1,021 x 16,384 x 2,048: 548 us (125 TFLOP/s; 630 through registers,
-// 1,880 on the vector ALU); the instruction alone reaches 154.
+// element by element: the order above. 1,021 x 16,384 x 2,048: 535 us (128 TFLOP/s; 630 through registers,
+// 1,880 on the vector ALU); the instruction alone reaches 154. With the barrier at a step's end instead of in its
+// middle 553, and 1,021 x 3,072 x 2,048 141 where it now takes 130.
 template <typename T, typename TW, typename TC, int TT, bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict__ A, int lda,
                                                             const TW* __restrict__ W, int ldw,
@@ -186,22 +187,26 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
     wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw + piece * 4;
   }
   f32x4 ain[DIRECT ? 1 : PER], win[DIRECT ? 1 : PER];
-  // 32 k from k0 on, into LDS buffer `buf` or the registers
-  auto fetch = [&](int buf, int k0) {
+  // step s's 32 k: into LDS buffer `buf` (DIRECT, piece i of each operand; the pointers walk along) or the registers
+  const int steps = (K + 31) / 32;
+  auto send = [&](int i, int buf, int s) {
     if constexpr (DIRECT) {
-      const bool whole = k0 + 32 <= K;           // else the last step of a K that is no multiple of 32
-      const bool in = k0 + piece * 4 < K;        // past K: zeros from one address
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const void *a = asrc[i] + k0, *w = wsrc[i] + k0;
-        if (!whole) {
-          a = in ? a : (const void*)&gemm_zeros;
-          w = in ? w : (const void*)&gemm_zeros;
-        }
-        ta_load_to_lds16(a, &As[buf][(32 * i + 8 * wave) * 8]);
-        ta_load_to_lds16(w, &Ws[buf][(32 * i + 8 * wave) * 8]);
+      const void *a = asrc[i], *w = wsrc[i];
+      if (s + 1 >= steps && K % 32 != 0) {       // past K: zeros from one address
+        const bool in = (steps - 1) * 32 + piece * 4 < K;
+        a = in ? a : (const void*)&gemm_zeros;
+        w = in ? w : (const void*)&gemm_zeros;
       }
-    } else {
+      ta_load_to_lds16(a, &As[buf][(32 * i + 8 * wave) * 8]);
+      ta_load_to_lds16(w, &Ws[buf][(32 * i + 8 * wave) * 8]);
+      const int on = s + 1 < steps ? 32 : 0;     // behind the last step: the same once more, unused
+      asrc[i] += on;
+      wsrc[i] += on;
+    }
+  };
+  auto fetch = [&](int s) {
+    if constexpr (!DIRECT) {
+      const int k0 = (s < steps ? s : steps - 1) * 32;
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         ain[i] = load_piece<T, VEC, false>(asrc[i] - piece * 4, k0 + piece * 4, K);
@@ -209,11 +214,8 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
       }
     }
   };
-  // the next step's k are in LDS for the whole workgroup, which has done with this step's buffer
-  auto arrive = [&](int buf) {
-    if constexpr (DIRECT) {
-      ta_wait_loads<2 * PER * (ST - 2)>();
-    } else {
+  auto stash = [&](int buf) {
+    if constexpr (!DIRECT) {
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         const int row = lrow + 32 * i, at = row * 8 + (place ^ (row & 7));
@@ -221,63 +223,77 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
         Ws[buf][at] = win[i];
       }
     }
-    __syncthreads();
   };
   const int half = lane / 32, r = lane % 32;
   const int am = (wave % 2) * 32 * TT + r, wn = (wave / 2) * 32 * TT + r;    // this lane's rows in As and Ws
-  f32x16 total[TT][TT];
+  f32x16 total[TT][TT], acc[TT][TT];
 #pragma unroll
   for (int i = 0; i < TT; ++i)
 #pragma unroll
     for (int j = 0; j < TT; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) total[i][j][e] = 0.f;
-
-  const int steps = (K + 31) / 32;
-#pragma unroll
-  for (int s = 0; s < ST - 1; ++s) fetch(s, (s < steps ? s : steps - 1) * 32);
-  arrive(0);
-  for (int s = 0; s < steps;) {
-    f32x16 acc[TT][TT];
+      for (int e = 0; e < 16; ++e) total[i][j][e] = acc[i][j][e] = 0.f;
+  // a block's operands, one of a step's two while the other is multiplied
+  f32x4 a[2][TT][2], w[2][TT][2];
+  auto read = [&](int set, int buf) {
 #pragma unroll
     for (int i = 0; i < TT; ++i)
 #pragma unroll
-      for (int j = 0; j < TT; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    const int end = s + SEG / 32 < steps ? s + SEG / 32 : steps;
-    for (; s < end; ++s) {
-      const int buf = s % ST, ahead = s + ST - 1;
-      fetch(ahead % ST, (ahead < steps ? ahead : steps - 1) * 32);      // behind the last step: once more, unused
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        f32x4 a[TT][2], w[TT][2];
-#pragma unroll
-        for (int i = 0; i < TT; ++i)
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const int at = (4 * b + 2 * p + half) ^ (r & 7);
-            a[i][p] = As[buf][(am + 32 * i) * 8 + at];
-            w[i][p] = Ws[buf][(wn + 32 * i) * 8 + at];
-          }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int x = 0; x < TT; ++x)
-#pragma unroll
-              for (int y = 0; y < TT; ++y)
-                acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x][p][j], w[y][p][j], acc[x][y], 0, 0, 0);
+      for (int p = 0; p < 2; ++p) {
+        const int at = (4 * set + 2 * p + half) ^ (r & 7);
+        a[set][i][p] = As[buf][(am + 32 * i) * 8 + at];
+        w[set][i][p] = Ws[buf][(wn + 32 * i) * 8 + at];
       }
-      arrive((s + 1) % ST);
+  };
+  auto multiply = [&](int set, int j) {          // a quarter of the block
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int x = 0; x < TT; ++x)
+#pragma unroll
+        for (int y = 0; y < TT; ++y)
+          acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][x][p][j], w[set][y][p][j], acc[x][y], 0, 0, 0);
+  };
+
+#pragma unroll
+  for (int s = 0; s < ST; ++s) {
+    fetch(s);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) send(i, s, s);
+    stash(s);
+  }
+  if constexpr (DIRECT) ta_wait_loads<2 * PER * (ST - 1)>();
+  __syncthreads();
+  read(0, 0);
+  // The barrier stands in the middle of a step: in front of it a step's second block is read, behind it the
+  // step's buffer is free for the step ST further on, and the next step's first block is read while the second
+  // is multiplied, so that no wave waits for LDS right behind a barrier. What is sent for goes out between the
+  // products.
+  for (int s = 0; s < steps; ++s) {
+    const int buf = s % ST;
+    fetch(s + ST);
+    read(1, buf);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) multiply(0, j);
+    if constexpr (DIRECT) ta_wait_loads<2 * PER * (ST - 2)>();                // the next step's k have come
+    __syncthreads();
+    stash(buf);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) send(i, buf, s + ST);
+    read(0, (s + 1) % ST);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) multiply(1, j);
+    if ((s + 1) % (SEG / 32) == 0 || s + 1 == steps) {
+#pragma unroll
+      for (int x = 0; x < TT; ++x)
+#pragma unroll
+        for (int y = 0; y < TT; ++y)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            total[x][y][e] += acc[x][y][e];
+            acc[x][y][e] = 0.f;
+          }
     }
-#pragma unroll
-    for (int x = 0; x < TT; ++x)
-#pragma unroll
-      for (int y = 0; y < TT; ++y)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) total[x][y][e] += acc[x][y][e];
   }
   if constexpr (DIRECT) ta_wait_loads<0>();      // nothing may land in LDS that is another's
   // accumulator: register e of a lane is row 8 (e / 4) + 4 half + e % 4 of the tile, column r
@@ -304,7 +320,7 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   TC* C = (TC*)C_;
   auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
   // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
-  // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 210, 256 rows 170 against 210, 512 rows 209 by tiles
+  // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
   // against 340). Tiles of 128 take two workgroups on every CU to fill.
   if (M > 64 && tiles(64) >= 192) {
     if (tiles(128) >= 384)
