@@ -117,7 +117,8 @@ __device__ __forceinline__ void ta_sums2(float& w, float& r) {
 // wave's loads are on their way, then a barrier; and no wave ends with one still in flight.
 __device__ __forceinline__ void ta_load_to_lds16(const void* src, void* lds) {
   const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to) : "m0", "memory");
+  // a scalar write of m0 wants one wait state before a load to LDS reads it
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to) : "m0", "memory");
 }
 template <int N>
 __device__ __forceinline__ void ta_wait_loads() {
