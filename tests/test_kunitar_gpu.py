@@ -214,6 +214,31 @@ def test_experts_products_in_every_form(form, geom):
         _close(got, want, "bfloat16" if out_dtype == torch.bfloat16 else "float32", f"{out_dtype}")
 
 
+# tiles of the experts, N, K: experts of one tile side by side, of 15 to 17 and 33 (blocks of 16 begin at an expert's first
+# tile, workgroups own those that begin at four tiles), columns around 256 and not in fours, k around 32 and short of the
+# steps that are sent ahead
+@pytest.mark.parametrize("geom", [((1, 1, 1, 1, 1, 2, 3), 256, 32), ((15, 16, 17, 1, 33), 257, 136), ((3, 0, 64, 5, 11), 130, 264),
+                                  ((2, 9, 12), 516, 8), ((16, 48), 8, 96)])
+def test_experts_blocks_through_lds_equal_operands_from_memory(geom):
+    """The form for many tiles against the one without LDS: the same instruction over the same ascending k, the same bits;
+    rows behind the last expert's keep what they held, and operands off 16 bytes take the other form."""
+    from transformer_amd import kernels
+    runs, N, K = geom
+    own = np.random.default_rng(N + K)
+    tiles = [e for e, n in enumerate(runs) for _ in range(n)]
+    tile_expert = torch.tensor(tiles + [-1] * 5, dtype=torch.int32, device=DEV)
+    rows = 16 * len(tile_expert)
+    a = _t(_bf(own.standard_normal((rows, K))), torch.bfloat16)
+    w = _t(_bf(own.standard_normal((len(runs), N, K)) / np.sqrt(K)), torch.bfloat16)
+    loose = torch.empty(w.numel() + 4, dtype=torch.bfloat16, device=DEV)[4:].view(w.shape).copy_(w)
+    for out_dtype, act in ((torch.float32, None), (torch.bfloat16, None), (torch.bfloat16, "relu2")):
+        want = kernels.moe_gemm(a, w, tile_expert, torch.full((rows, N), 7.0, dtype=out_dtype, device=DEV), act, form="direct")
+        assert (want[16 * len(tiles):] == 7.0).all()
+        for matrix in (w, loose):
+            got = kernels.moe_gemm(a, matrix, tile_expert, torch.full((rows, N), 7.0, dtype=out_dtype, device=DEV), act, form="lds")
+            assert torch.equal(got, want), (out_dtype, act)
+
+
 # experts, router outputs, top, tokens, N, K: one token, the most that are routed in one launch and one more, columns that
 # end inside the 32 or 64 of a workgroup, k inside and behind a wave's share
 @pytest.mark.parametrize("geom", [(5, 5, 3, 1, 40, 72), (64, 72, 6, 16, 33, 200), (8, 8, 2, 17, 96, 1032), (3, 4, 4, 6, 130, 2056)])

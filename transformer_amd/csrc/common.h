@@ -120,6 +120,12 @@ __device__ __forceinline__ void ta_load_to_lds16(const void* src, void* lds) {
   // a scalar write of m0 wants one wait state before a load to LDS reads it
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(to) : "m0", "memory");
 }
+// The same from `base` (one for the wave) + `offset` bytes. A base that a vector instruction has just written (the
+// compiler may read it from a register's first lane right here) wants five wait states.
+__device__ __forceinline__ void ta_load_to_lds16(const void* base, uint32_t offset, void* lds) {
+  const uint32_t to = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(to) : "m0", "memory");
+}
 template <int N>
 __device__ __forceinline__ void ta_wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

@@ -623,155 +623,202 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   }
 }
 
-// Many tiles (a prompt): operands through LDS. A workgroup owns eight neighbouring tiles of 16
-// rows and 128 columns; the runs of one expert among them are multiplied one after the other.
-// Every thread brings whole 16-byte pieces of the rows of A and of the expert's matrix (eight
-// lanes a row: whole cache lines), a step of 64 k ahead of the one being multiplied, into one of
-// two LDS buffers (rows 72 elements apart, so that the operand reads of 16 rows meet 16
-// different bank groups); a wave multiplies 64 x 64 of the 128 x 128 (4 x 4 operand tiles: every
-// LDS read feeds four products).
-#define ML_BM 128
-#define ML_BN 128
-#define ML_BK 64
-#define ML_LD 72
+// Many tiles (a prompt): operands through LDS. An expert's tiles of 16 rows are cut, from its first one on, into
+// blocks of up to 16, so that its matrix is read once for every 256 rows. A workgroup of eight waves owns 256 columns
+// of the blocks that begin at four neighbouring tiles (about one block where the experts have four tiles or more; few
+// or none have rows for several), and what is sent for runs on from one block into the next. The operands go from
+// memory to LDS without passing through registers, 32 k at a time, four steps ahead into five buffers (160 KB). A
+// row's four pieces of 16 bytes are permuted by half the row number, so that eight rows' reads meet no bank twice. The
+// waves stand in 2 x 4; each multiplies half of the block's tiles by 64 columns. What bounds it: few rows an expert, the
+// experts' matrices from memory (3.9 TB/s); many, the loads and the reads of LDS around the products (0.67 PFLOP/s).
+// 64 experts of 2,816 x 4,096, 6 of 72 a token (128 rows of eight tiles by 128 columns through registers before):
+// 600 tokens 384 us (487), 1,200 436 (623), 2,943 711 (912), 5,800 1,070 (1,438); of 4,096 x 1,408 into float32,
+// 2,943 tokens 378 (513).
+#define ML_BM 256
+#define ML_BN 256
+#define ML_BK 32
+#define ML_ST 5
+#define ML_TILES (ML_BM / MOE_TILE)
+#define ML_OWN 4
 
-template <typename TC>
-__global__ __launch_bounds__(256, 2) void moe_gemm_lds_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+static __device__ const moe_u32x4 ml_zeros = {0, 0, 0, 0};
+
+// 32 k of a block: UU tiles of rows from `rows` on by 64 columns from `cols` on
+template <int UU>
+static __device__ __forceinline__ void ml_multiply(moe_floatx4 (&acc)[UU][4], const moe_u32x4* As, const moe_u32x4* Ws, int rows, int cols,
+                                                   int r, int kb) {
+  MoeFrag af[UU], wf[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) wf[v].q = Ws[(cols + 16 * v + r) * 4 + (kb ^ ((r >> 1) & 3))];
+#pragma unroll
+  for (int u = 0; u < UU; ++u) af[u].q = As[(rows + 16 * u + r) * 4 + (kb ^ ((r >> 1) & 3))];
+  __builtin_amdgcn_sched_barrier(0);                    // every read goes out before the first product waits for one
+#pragma unroll
+  for (int u = 0; u < UU; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      // register j of a lane: column 4 * (lane / 16) + j of the tile, row lane % 16
+      acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[v].v, af[u].v, acc[u][v], 0, 0, 0);
+}
+
+template <typename TC, bool ACT>
+__global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                            const int* __restrict__ tile_expert, int tiles, int max_rows,
                                                            TC* __restrict__ C, int N, int K, int act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ml_lds[];
-  bf16_t* As = reinterpret_cast<bf16_t*>(ml_lds);                       // [2][ML_BM][ML_LD]
-  bf16_t* Ws = As + 2 * ML_BM * ML_LD;                                  // [2][ML_BN][ML_LD]
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int r = lane % 16, kb = lane / 16, wr = wave / 2, wc = wave % 2;
-  // Which (group of eight tiles, block of 128 columns) this workgroup takes. Workgroups go to the
-  // eight XCDs in turn, and each XCD has an L2 of its own: the workgroups that one XCD gets one
-  // after the other take two neighbouring groups of tiles (mostly one expert) through all blocks
-  // of columns, block by block, so that the expert's panel of 128 columns is read from memory once
-  // for both groups and the groups' rows once for all blocks.
+  moe_u32x4* As = reinterpret_cast<moe_u32x4*>(ml_lds);                 // [ML_ST][ML_BM * 4]
+  moe_u32x4* Ws = As + ML_ST * ML_BM * 4;                               // [ML_ST][ML_BN * 4]
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
+  const int r = lane % 16, kb = lane / 16, wr = wave / 4, wc = wave % 4;
   const int ncol = (N + ML_BN - 1) / ML_BN;
-  const int xcd = blockIdx.x % 8, seq = blockIdx.x / 8;
-  const int unit = (seq / (2 * ncol)) * 8 + xcd, within = seq % (2 * ncol);
-  const int group = 2 * unit + within % 2;
-  const int n0 = (within / 2) * ML_BN;
-  int t = group * 8;
-  if (t >= tiles) return;
-  const int t_end = t + 8 < tiles ? t + 8 : tiles;
-  const int nk = (K + ML_BK - 1) / ML_BK;
-  while (t < t_end) {
-    const int e = tile_expert[t];
-    if (e < 0) return;                                  // the whole workgroup: tiles past the last expert's rows
-    int run = 1;
-    while (t + run < t_end && tile_expert[t + run] == e) ++run;
-    const int R = run * MOE_TILE;
-    const size_t r0 = (size_t)t * MOE_TILE;
-    const bf16_t* We = W + (size_t)e * N * K;
-    // this thread's four pieces of A and of W in a step: row p / 8, piece p % 8, p = tid + 256 i
-    const bf16_t* asrc[4];
-    const bf16_t* wsrc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int p = tid + 256 * i, row = p / 8, pc = p % 8;
-      const size_t ar = r0 + (row < R ? row : R - 1);                   // rows past the run: read again, never stored
-      const int wn = n0 + row < N ? n0 + row : N - 1;                   // columns past N likewise
-      asrc[i] = A + ar * K + pc * 8;
-      wsrc[i] = We + (size_t)wn * K + pc * 8;
+  const int window = __builtin_amdgcn_readfirstlane((int)(blockIdx.x / (unsigned)ncol));
+  const int n0 = ((int)blockIdx.x - window * ncol) * ML_BN, t0 = window * ML_OWN;
+  int e = tile_expert[t0];
+  if (e < 0) return;                                    // tiles past the last expert's rows
+  // the first tile of e's run
+  int first = t0;
+  while (true) {
+    const int i = first - 1 - lane;
+    const unsigned long long other = __ballot(i < 0 || tile_expert[i < 0 ? 0 : i] != e);
+    if (other) {
+      first -= __ffsll(other) - 1;
+      break;
     }
-    // Three steps' pieces wait in registers on their way from memory (a trip takes several times
-    // as long as a step's products); the barrier between steps waits for LDS traffic only, not
-    // for these loads.
-    struct Pieces {
-      moe_u32x4 a[4], w[4];
-    };
-    auto fetch = [&](Pieces& q, int step) {
-      const int k0 = step * ML_BK;
-      if (step >= nk) return;
-      if (k0 + ML_BK <= K) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          q.a[i] = *reinterpret_cast<const moe_u32x4*>(asrc[i] + k0);
-          q.w[i] = *reinterpret_cast<const moe_u32x4*>(wsrc[i] + k0);
-        }
-      } else {                                                          // the last, partial step
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const bool kok = k0 + ((tid + 256 * i) % 8) * 8 < K;
-          q.a[i] = kok ? *reinterpret_cast<const moe_u32x4*>(asrc[i] + k0) : moe_zero4();
-          q.w[i] = kok ? *reinterpret_cast<const moe_u32x4*>(wsrc[i] + k0) : moe_zero4();
-        }
-      }
-    };
-    auto stash = [&](const Pieces& q, int buf) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = tid + 256 * i, row = p / 8, pc = p % 8;
-        *reinterpret_cast<moe_u32x4*>(As + (buf * ML_BM + row) * ML_LD + pc * 8) = q.a[i];
-        *reinterpret_cast<moe_u32x4*>(Ws + (buf * ML_BN + row) * ML_LD + pc * 8) = q.w[i];
-      }
-    };
-    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    moe_floatx4 acc[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[u][v] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
-    const bool busy = 64 * wr < R;                      // a run of at most 64 rows leaves two waves only loading
-    auto multiply = [&](int buf) {
-      if (!busy) return;
-#pragma unroll
-      for (int kk = 0; kk < ML_BK; kk += 32) {
-        MoeFrag af[4], wf[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          af[u].q = *reinterpret_cast<const moe_u32x4*>(As + (buf * ML_BM + 64 * wr + 16 * u + r) * ML_LD + kk + 8 * kb);
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          wf[v].q = *reinterpret_cast<const moe_u32x4*>(Ws + (buf * ML_BN + 64 * wc + 16 * v + r) * ML_LD + kk + 8 * kb);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int v = 0; v < 4; ++v)
-            // register j of a lane: column 4 * (lane / 16) + j of the tile, row lane % 16
-            acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[v].v, af[u].v, acc[u][v], 0, 0, 0);
-      }
-    };
-    Pieces p0, p1, p2;
-    fetch(p0, 0);
-    fetch(p1, 1);
-    fetch(p2, 2);
-    stash(p0, 0);
-    fetch(p0, 3);
-    lds_barrier();
-    // step s multiplies buffer s & 1; the pieces of step s + 1 (in set (s + 1) % 3) then go to the
-    // other buffer and their set asks for step s + 4
-    for (int step = 0; step < nk; step += 3) {
-      multiply(step & 1);
-      if (step + 1 < nk) { stash(p1, (step + 1) & 1); fetch(p1, step + 4); }
-      lds_barrier();
-      if (step + 1 >= nk) break;
-      multiply((step + 1) & 1);
-      if (step + 2 < nk) { stash(p2, (step + 2) & 1); fetch(p2, step + 5); }
-      lds_barrier();
-      if (step + 2 >= nk) break;
-      multiply((step + 2) & 1);
-      if (step + 3 < nk) { stash(p0, (step + 3) & 1); fetch(p0, step + 6); }
-      lds_barrier();
-    }
-    if (busy) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (64 * wr + 16 * u >= R) break;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int n = n0 + 64 * wc + 16 * v + 4 * kb + j;
-            if (n < N) C[(r0 + 64 * wr + 16 * u + r) * N + n] = from_f32<TC>(moe_act(act, acc[u][v][j]));
-          }
-      }
-    }
-    t += run;
+    first -= 64;
   }
+  // The blocks that begin at this workgroup's tiles: five bits each, their tiles (none: 0)
+  unsigned blocks = 0;
+#pragma unroll
+  for (int i = 0; i < ML_OWN; ++i) {
+    const int t = t0 + i, here = t < tiles ? tile_expert[t] : -1;
+    if (here < 0) break;
+    if (here != e) e = here, first = t;
+    if ((t - first) % ML_TILES == 0) {
+      const int ahead = t + lane;
+      const unsigned long long other = __ballot(lane >= ML_TILES || ahead >= tiles || tile_expert[ahead < tiles ? ahead : t] != e);
+      blocks |= (unsigned)(__ffsll(other) - 1) << (5 * i);
+    }
+  }
+  blocks = __builtin_amdgcn_readfirstlane(blocks);
+  if (blocks == 0) return;
+  auto next_block = [&](int i) {                        // the first one from i on, or ML_OWN
+    const unsigned left = blocks >> (5 * i);
+    return __builtin_amdgcn_readfirstlane(left ? i + (__ffs(left) - 1) / 5 : ML_OWN);
+  };
+  auto run_of = [&](int i) { return (int)(blocks >> (5 * i) & 31u); };
+  const int nk = (K + ML_BK - 1) / ML_BK;
+
+  // The sender: block `sent`, step `ks` of it. A wave brings 16 rows at a time: rows 16 (wave + 8 i).
+  const int srow = lane / 4, piece = lane % 4 ^ ((srow >> 1) & 3);
+  const bf16_t *abase, *wbase;                          // of the block, at step ks
+  uint32_t aoff[2], woff[2];                            // bytes from there on
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 16 * (wave + 8 * i) + srow;
+    woff[i] = ((uint32_t)(n0 + row < N ? row : N - 1 - n0) * K + piece * 8) * 2;   // columns past N: read again, never stored
+  }
+  int sent = next_block(0), ks = 0;
+  auto aim = [&]() {
+    const int R = run_of(sent) * MOE_TILE;
+    abase = A + (size_t)(t0 + sent) * MOE_TILE * K;
+    wbase = W + ((size_t)__builtin_amdgcn_readfirstlane(tile_expert[t0 + sent]) * N + n0) * K;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = 16 * (wave + 8 * i) + srow;
+      aoff[i] = ((uint32_t)(row < R ? row : R - 1) * K + piece * 8) * 2;           // rows past the block likewise
+    }
+  };
+  auto send = [&](int buf) {
+    if (ks + 1 < nk || K % ML_BK == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        ta_load_to_lds16(abase, aoff[i], &As[buf * ML_BM * 4 + 64 * (wave + 8 * i)]);
+        ta_load_to_lds16(wbase, woff[i], &Ws[buf * ML_BN * 4 + 64 * (wave + 8 * i)]);
+      }
+    } else {                                                            // the last, partial step: past K zeros
+      const bool in = ks * ML_BK + piece * 8 < K;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        ta_load_to_lds16(in ? (const char*)abase + aoff[i] : (const char*)&ml_zeros, &As[buf * ML_BM * 4 + 64 * (wave + 8 * i)]);
+        ta_load_to_lds16(in ? (const char*)wbase + woff[i] : (const char*)&ml_zeros, &Ws[buf * ML_BN * 4 + 64 * (wave + 8 * i)]);
+      }
+    }
+    if (ks + 1 < nk) {
+      ++ks;
+      abase += ML_BK;
+      wbase += ML_BK;
+    } else if (next_block(sent + 1) < ML_OWN) {                         // on into the next block
+      sent = next_block(sent + 1);
+      ks = 0;
+      aim();
+    }                                                                   // else the last step again, unused
+  };
+  aim();
+#pragma unroll
+  for (int s = 0; s < ML_ST - 1; ++s) send(s);
+
+  int buf = 0;
+  for (int i = next_block(0); i < ML_OWN; i = next_block(i + 1)) {
+    const int run = run_of(i), half = (run + 1) / 2;
+    auto block = [&](auto width) {
+      constexpr int U = decltype(width)::value;         // tiles of a wave
+      // all of a wave's, which the compiler no longer sees behind the stores of the block before
+      auto same = [](uint64_t x) {
+        const uint32_t high = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)), low = __builtin_amdgcn_readfirstlane((uint32_t)x);
+        return (uint64_t)high << 32 | low;
+      };
+      sent = __builtin_amdgcn_readfirstlane(sent);
+      ks = __builtin_amdgcn_readfirstlane(ks);
+      buf = __builtin_amdgcn_readfirstlane(buf);
+      abase = reinterpret_cast<const bf16_t*>(same((uint64_t)abase));
+      wbase = reinterpret_cast<const bf16_t*>(same((uint64_t)wbase));
+      moe_floatx4 acc[U][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[u][v] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int step = 0; step < nk; ++step) {
+        ta_wait_loads<4 * (ML_ST - 2)>();                 // this step's pieces; C's stores, if any, only make it wait longer
+        __syncthreads();                                  // everyone's; and all have read the buffer that is sent for now
+        send(buf == 0 ? ML_ST - 1 : buf - 1);
+        ml_multiply<U>(acc, As + buf * ML_BM * 4, Ws + buf * ML_BN * 4, 16 * U * wr, 64 * wc, r, kb);
+        buf = buf + 1 == ML_ST ? 0 : buf + 1;
+      }
+      TC* out = C + ((size_t)(t0 + i) * MOE_TILE + r) * N;
+      const bool whole = N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;   // a lane's four columns are stored at once
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int tile = U * wr + u;
+        if (tile >= run) break;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int n = n0 + 64 * wc + 16 * v + 4 * kb;
+          TC x[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[j] = from_f32<TC>(ACT ? moe_act(act, acc[u][v][j]) : acc[u][v][j]);
+          TC* o = out + (size_t)tile * MOE_TILE * N + n;
+          if (whole) {
+            struct alignas(4 * sizeof(TC)) Four { TC x[4]; };
+            if (n < N) *reinterpret_cast<Four*>(o) = Four{{x[0], x[1], x[2], x[3]}};
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              if (n + j < N) o[j] = x[j];
+          }
+        }
+      }
+    };
+    switch (half) {
+      case 1: block(std::integral_constant<int, 1>{}); break;
+      case 2: block(std::integral_constant<int, 2>{}); break;
+      case 3:
+      case 4: block(std::integral_constant<int, 4>{}); break;
+      case 5:
+      case 6: block(std::integral_constant<int, 6>{}); break;
+      default: block(std::integral_constant<int, 8>{}); break;
+    }
+  }
+  ta_wait_loads<0>();                                   // what was sent for and not used has landed before the LDS is given back
 }
 
 // A: [max_rows, K] ordered rows; W: [E, N, K]; C: [max_rows, N], float32 or the type of A;
@@ -779,12 +826,11 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_lds_kernel(const bf16_t* __re
 // rows are skipped and their rows of C keep what they held.
 static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A, const void* W, const int* tile_expert,
                                void* C, int max_rows, int tiles, int N, int K, int act) {
-  const size_t lds = (size_t)2 * (ML_BM + ML_BN) * ML_LD * sizeof(bf16_t);
-  const int ncol = (N + ML_BN - 1) / ML_BN, groups = (tiles + 7) / 8, units = (groups + 1) / 2;
-  dim3 g((unsigned)((units + 7) / 8 * 8 * 2 * ncol));      // see the kernel: eight XCDs take units of 2 groups x all column blocks
-#define ML_RUN(TC)                                                                                               \
+  const size_t lds = (size_t)ML_ST * (ML_BM + ML_BN) * ML_BK * sizeof(bf16_t);
+  const unsigned g = (unsigned)((N + ML_BN - 1) / ML_BN) * (unsigned)((tiles + ML_OWN - 1) / ML_OWN);
+#define ML_RUN(TC, ACT)                                                                                          \
   do {                                                                                                           \
-    auto kern = moe_gemm_lds_kernel<TC>;                                                                         \
+    auto kern = moe_gemm_lds_kernel<TC, ACT>;                                                                    \
     static bool allowed = false;                        /* asked for once, not at every launch */                \
     if (!allowed) {                                                                                              \
       const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                            \
@@ -792,9 +838,13 @@ static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A,
       if (err != hipSuccess) return ta_fail("ta_moe_gemm: %zu bytes of LDS refused (%s)", lds, hipGetErrorString(err)); \
       allowed = true;                                                                                            \
     }                                                                                                            \
-    kern<<<g, 256, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, tiles, max_rows, (TC*)C, N, K, act); \
+    kern<<<g, 512, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, tiles, max_rows, (TC*)C, N, K, act); \
   } while (0)
-  if (out_dtype == TA_BF16) ML_RUN(bf16_t); else ML_RUN(float);
+  if (out_dtype == TA_BF16) {
+    if (act) ML_RUN(bf16_t, true); else ML_RUN(bf16_t, false);
+  } else {
+    if (act) ML_RUN(float, true); else ML_RUN(float, false);
+  }
 #undef ML_RUN
   return ta_check_launch("ta_moe_gemm");
 }
@@ -839,7 +889,9 @@ extern "C" int ta_moe_gemm_form(hipStream_t stream, int dtype, int out_dtype, co
   if (dtype == TA_BF16 && K % 8 == 0) {
     if (out_dtype != TA_BF16 && out_dtype != TA_F32) return ta_fail("ta_moe_gemm: unknown output type %d", out_dtype);
     const bool few = ta_moe_few_rows(max_rows, N, K);
-    if (form == 3 || (form == 0 && !few)) return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, max_rows, tiles, N, K, act);
+    const bool aligned = ((uintptr_t)A | (uintptr_t)W) % 16 == 0;   // else operands straight from memory
+    if ((form == 3 || (form == 0 && !few)) && aligned)
+      return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, max_rows, tiles, N, K, act);
     if (form == 1 || (form == 0 && few)) {   // too few workgroups to fill the CUs: the waves divide K
       dim3 gk((N + 63) / 64, tiles);
       const MoeRows rows = {(const bf16_t*)A, nullptr, nullptr, 1};
