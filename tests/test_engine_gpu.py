@@ -62,6 +62,31 @@ def test_last_32_tokens_one_by_one(name, dtype):
     cache.free_slot(s)
 
 
+@pytest.mark.parametrize("name", ["A", "C", "D"])
+def test_float32_bits_do_not_depend_on_who_shares_a_step(name):
+    """A prompt whole, in pieces of 64 and 9 tokens and one by one, and beside 69 others: the same logits bit for bit,
+    then the same single tokens alone and in a step of 70."""
+    from transformer_amd import Entry
+    model, toks = G.engine(name, "float32"), G.tokens(name, 74, 70)
+    cache = model.new_cache(16384, max_slots=72)
+
+    def run(cuts, others=0):
+        slots = [cache.alloc_slot() for _ in range(1 + others)]
+        out, at = [], 0
+        for n in cuts:
+            beside = [Entry(s, G.tokens(name, 74, 200 + i)[at:at + n], [0]) for i, s in enumerate(slots[1:])]
+            out.append(_logits(model, cache, [Entry(slots[0], toks[at:at + n], range(n))] + beside)[:n])
+            at += n
+        for s in slots:
+            cache.free_slot(s)
+        return np.concatenate(out)
+
+    want = run([70, 1, 1, 1, 1])
+    for got in (run([64, 6, 1, 1, 1, 1]), run([9] * 7 + [7, 1, 1, 1, 1]), run([1] * 74), run([70, 1, 1, 1, 1], 69),
+                run([1] * 74, 69)):
+        assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("name,dtype", CASES)
 def test_unequal_batches_one_after_another_in_reused_slots(name, dtype):
     from transformer_amd import Entry

@@ -273,6 +273,34 @@ def test_attention_generic(dtype, shape):
     assert np.abs(got - want).max() < tol(dtype)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dh,style", [(16, "half"), (48, "interleaved"), (128, "half"), (128, "interleaved")])
+def test_rope_kv_write_gives_a_token_the_same_bits_at_any_count(dtype, dh, style):
+    """A token's rotated queries and keys in calls of 131, 64, 9 and one token: three kernels, one rounding."""
+    from transformer_amd import kernels
+    own = np.random.default_rng([dh, len(style)])
+    nq, nkv, nt = 3, 2, 131
+    pos = own.integers(0, 100000, nt).tolist()
+    qkv = dev(rounded(own.normal(size=(nt, (nq + 2 * nkv) * dh)), dtype), DT[dtype])
+    bias = dev(own.normal(size=(nq + 2 * nkv) * dh).astype(np.float32))
+    dest = dev(own.permutation(4 * 64)[:nt], torch.int32)
+    inv = dev(P.rope_inv_freq(dh, 500000.0))
+    ang = kernels.rope_table(dev(pos, torch.int32), inv, torch.empty(nt, dh // 2, 2, device=DEV))
+    for b in (None, bias):
+        results = []
+        for step in (nt, 64, 9, 1):
+            rows = qkv.clone()
+            kc = torch.zeros(4, nkv, 64, dh, dtype=DT[dtype], device=DEV)
+            vc = torch.zeros(4, nkv, dh, 64, dtype=DT[dtype], device=DEV)
+            for t in range(0, nt, step):
+                kernels.rope_kv_write(rows[t:t + step], nq, nkv, dh, ang[t:t + step].contiguous(), style == "interleaved",
+                                      dest[t:t + step], kc, vc, b)
+            results.append((rows, kc, vc))
+        for got in results[1:]:
+            for x, y in zip(got, results[0]):
+                assert torch.equal(x, y)
+
+
 # nh, nkv, dk, dv, lengths of the caches, (softcap, sink, gate, window, keep_first, chunk): both kinds of widths of
 # each kernel, groups of 1, 5 and 20 heads, ends on and off a page's edge, every option
 F32_SHAPES = [

@@ -351,6 +351,15 @@ extern "C" int ta_rope_table(hipStream_t stream, const int* pos, const float* in
   return ta_rope_table_scaled(stream, pos, inv_freq, cs, nt, half, 1.0f);
 }
 
+// The pair (a, c) turned by the angle of (cosine, sine) k. The three kernels below take the same token at different
+// counts of tokens, so what is rounded is written out: left to the compiler, a product that two branches share is
+// kept and the other one of its sum contracted, and a key then depends on how many tokens share its step.
+__device__ __forceinline__ void rotate_pair(float& a, float& c, float2 k) {
+  const float r0 = fmaf(a, k.x, -(c * k.y)), r1 = fmaf(c, k.x, a * k.y);
+  a = r0;
+  c = r1;
+}
+
 // qkv: [nt, nq + 2*nkv, dh]. Per token t:
 //   q heads: (+bias) rotated in place
 //   k heads: (+bias) rotated, written to the K cache at dest[t] (and back in place)
@@ -386,13 +395,8 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, const float* __restric
         a += b[i0];
         c += b[i1];
       }
-      float r0 = a, r1 = c;
-      if (ct) {
-        const float2 k = ct[j];
-        r0 = a * k.x - c * k.y;
-        r1 = a * k.y + c * k.x;
-      }
-      const T o0 = from_f32<T>(r0), o1 = from_f32<T>(r1);
+      if (ct) rotate_pair(a, c, ct[j]);
+      const T o0 = from_f32<T>(a), o1 = from_f32<T>(c);
       v[i0] = o0;
       v[i1] = o1;
       if (kc) {
@@ -464,22 +468,12 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
       const float2* ct = cs + (size_t)t * half;
       if (style == 0) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float2 k = ct[4 * u + e];
-          const float r0 = a[e] * k.x - c[e] * k.y, r1 = a[e] * k.y + c[e] * k.x;
-          a[e] = r0;
-          c[e] = r1;
-        }
+        for (int e = 0; e < 4; ++e) rotate_pair(a[e], c[e], ct[4 * u + e]);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
-          const float2 ka = ct[4 * u + e / 2], kc2 = ct[4 * u + 2 + e / 2];
-          const float a0 = a[e] * ka.x - a[e + 1] * ka.y, a1 = a[e] * ka.y + a[e + 1] * ka.x;
-          const float c0 = c[e] * kc2.x - c[e + 1] * kc2.y, c1 = c[e] * kc2.y + c[e + 1] * kc2.x;
-          a[e] = a0;
-          a[e + 1] = a1;
-          c[e] = c0;
-          c[e + 1] = c1;
+          rotate_pair(a[e], a[e + 1], ct[4 * u + e / 2]);
+          rotate_pair(c[e], c[e + 1], ct[4 * u + 2 + e / 2]);
         }
       }
     }
@@ -607,21 +601,12 @@ __global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
     if (cs) {
       if (style == 0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float r0 = a[e] * k[e].x - c[e] * k[e].y, r1 = a[e] * k[e].y + c[e] * k[e].x;
-          a[e] = r0;
-          c[e] = r1;
-        }
+        for (int e = 0; e < 8; ++e) rotate_pair(a[e], c[e], k[e]);
       } else {
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
-          const float2 ka = k[e / 2], kc = k[4 + e / 2];
-          const float a0 = a[e] * ka.x - a[e + 1] * ka.y, a1 = a[e] * ka.y + a[e + 1] * ka.x;
-          const float c0 = c[e] * kc.x - c[e + 1] * kc.y, c1 = c[e] * kc.y + c[e + 1] * kc.x;
-          a[e] = a0;
-          a[e + 1] = a1;
-          c[e] = c0;
-          c[e + 1] = c1;
+          rotate_pair(a[e], a[e + 1], k[e / 2]);
+          rotate_pair(c[e], c[e + 1], k[4 + e / 2]);
         }
       }
     }
