@@ -104,12 +104,16 @@ def library_rows(rows: int, n: int, k: int) -> list:
     Its tiles of 256 x 256 fill the 256 CUs in rounds, and it runs at 1.3 to 1.45 PFLOP/s while the last round is
     nearly full, nearly half or nearly a quarter full (it then cuts that round along k by 1, 2 or 4). Between those,
     and with more than two rounds, it falls to half for k from about 10,000 on: 4,096 columns over k = 11,008 take
-    258 us at 3,904 rows, 592 at 4,128, 330 at 4,800, 638 at 5,248, 399 at 5,920, 743 at 7,040, 905 at 9,000; in two
-    calls, whole rounds and the rest, 282 us at 4,128, 376 at 5,248, 462 at 7,040, 623 at 9,000 (where it does well by
-    itself two calls cost up to 7 % more). The same holds for 4,096 columns over 14,336 and for 8,192 over 28,672; over
-    k = 8,192 one call is as good everywhere."""
-    full = 256 * (256 * 256 // max(256, n))            # rows whose tiles fill the CUs once
-    if k < 10240 or n % 256 or rows <= full:
+    258 us at 3,904 rows, 592 at 4,128, 330 at 4,800, 638 at 5,248, 399 at 5,920, 743 at 7,040, 905 at 9,000; in
+    calls of whole rounds and a rest 282 us at 4,128, 376 at 5,248, 462 at 7,040, 623 at 9,000.
+    Measured at 4,096, 8,192 and 16,384 columns, k from 10,240 to 28,672, 1 to 10 rounds: 1.05 to 2.1 times as fast
+    in calls, at worst 4 % slower. Other widths do not fill the CUs in whole rounds (5,120 columns: 240 of 256) and
+    lose (6,144 over 14,336 at 8,192 rows: 1,037 us in one call, 1,623 in calls), as do 4,096 columns over 28,672 at
+    some counts; over k = 8,192 one call is as good everywhere."""
+    if n not in (4096, 8192, 16384) or not 10240 <= k <= min(4 * n, 28672):
+        return [rows]
+    full = 256 * (256 * 256 // n)                      # rows whose tiles fill the CUs once
+    if rows <= full:
         return [rows]
     calls = []
     while rows > 2 * full:
