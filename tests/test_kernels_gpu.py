@@ -654,6 +654,33 @@ def test_gemm_simple(mnk):
     assert np.abs(f64(o2) - ab @ wb.T).max() < 1e-6 * K ** 0.5 * 8
 
 
+@pytest.mark.parametrize("counts", [[0, 1, 0, 1, 1, 0], [1, 0, 0], [0, 0, 1]])
+def test_float32_attention_of_sequences_that_bring_no_token(counts):
+    """Single tokens beside sequences without one, first, last and in between: the rows of the others, the same as
+    without them, and nothing behind the last row."""
+    from transformer_amd import kernels
+    from transformer_amd.parts.linear import Workspace
+    own = np.random.default_rng(len(counts))
+    nh, nkv, dh, B, nt = 8, 2, 64, len(counts), sum(counts)
+    kc, vc = dev(own.normal(size=(2 * B, nkv, 64, dh))), dev(own.normal(size=(2 * B, nkv, dh, 64)))
+    table = dev(own.permutation(2 * B).reshape(B, 2), torch.int32)
+    pos = own.integers(3, 128, B)
+    q = dev(own.normal(size=(nt, nh * dh)))
+    live = [b for b, n in enumerate(counts) if n]
+
+    def step(who, ws):
+        out = torch.full((nt + 2, nh * dh), 7.0, device=DEV)
+        cu = np.concatenate([[0], np.cumsum([counts[b] for b in who])])
+        kernels.attention_generic(q, out[:nt], kc, vc, table[who].contiguous(), dev(cu, torch.int32), dev(pos[who], torch.int32),
+                                  1, nh, nkv, dh, 0.125, None, ws)
+        assert (out[nt:] == 7.0).all()
+        return out[:nt]
+
+    want = step(live, None)
+    for ws in (Workspace(DEV), None):
+        assert torch.equal(step(list(range(B)), ws), want)
+
+
 # rows at which the kernel or its tile changes, k inside and at the ends of blocks, segments and rounds of
 # segments, workgroups' tiles that end inside the matrix (the last two: tiles of 64 and of 128)
 @pytest.mark.parametrize("mnk", [(1, 7, 256), (8, 23, 260), (9, 33, 2052), (16, 17, 1028), (17, 40, 516), (33, 19, 2304),

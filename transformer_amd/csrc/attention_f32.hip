@@ -259,6 +259,7 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
   const int end = p.pos0[b] + 1;
   Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
   if (page >= p.max_blocks || !see.page(page)) return;
+  if (p.cu_q[b + 1] == p.cu_q[b]) return;          // a sequence that brings no token has no row
   const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
   const bool ok = h0 + r < group;
   const int head = kvh * group + (ok ? h0 + r : 0);
@@ -300,6 +301,7 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
 // The pages of a single token's row joined in ascending order, eight asked for at a time; a thread a column.
 __global__ __launch_bounds__(128) void attn_f32_join_kernel(F32Attention p) {
   const int head = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+  if (p.cu_q[b + 1] == p.cu_q[b]) return;
   const int end = p.pos0[b] + 1;
   const Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
   const size_t unit = ((size_t)b * p.nh + head) * p.max_blocks;
@@ -339,7 +341,7 @@ extern "C" long long ta_attention_f32_scratch(int batch, int nh, int max_blocks,
 }
 
 // As ta_attention_generic_sink, float32, dh and dv multiples of 16 up to 128, rows that start on 16 bytes. parts:
-// scratch of ta_attention_f32_scratch floats for steps in which every sequence brings one token (max_qlen 1), or
+// scratch of ta_attention_f32_scratch floats for steps in which every sequence brings one token or none (max_qlen 1), or
 // null: the kernel for prompts then serves these too, with the same bits.
 extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride, void* out, int out_stride,
                                 const void* kcache, const void* vcache, const int* block_table, int max_blocks,
