@@ -998,6 +998,21 @@ def test_sample_rows_on_16_byte_boundaries_and_others_choose_alike(vocab):
         assert torch.equal(a, b), (T, k, p_, (a != b).nonzero().flatten().tolist())
 
 
+def test_sample_without_scratch_keeps_its_entry_point():
+    """ta_sample has the ten arguments it always had; ta_sample_parts takes the scratch."""
+    from ctypes import c_float, c_int, c_longlong
+    from transformer_amd import kernels
+    own = np.random.default_rng(10)
+    n, vocab = 5, 8200
+    logits, u = dev(own.normal(size=(n, vocab)) * 3), dev(own.random(n))
+    a, b = (torch.full((n,), -1, dtype=torch.int32, device=DEV) for _ in range(2))
+    kernels.sample(logits, u, a, 0.8, 40, 0.95)
+    kernels._check(kernels.library().ta_sample(
+        kernels._stream(), kernels._ptr(logits), c_longlong(vocab), c_int(n), c_int(vocab), c_float(0.8), c_int(40),
+        c_float(0.95), kernels._ptr(u), kernels._ptr(b)))
+    assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("vocab", [4095, 4097, 8192, 40963])
 def test_sample_in_parts_of_a_row_chooses_as_the_whole_row(vocab):
     """Rows whose parts end at, before and behind a multiple of 4,096; thresholds inside one step of logit / T, on a

@@ -1265,7 +1265,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(const float
 
 static int sample_parts(int vocab) { return (vocab + PART - 1) / PART; }
 
-// Bytes of scratch that lets ta_sample deal rows out in parts (0: rows of this vocabulary are not).
+// Bytes of scratch that lets ta_sample_parts deal rows out in parts (0: rows of this vocabulary are not).
 extern "C" long long ta_sample_scratch(int n, int vocab) {
   if (n <= 0 || n > 65535 || vocab <= 0 || sample_parts(vocab) > MAX_PARTS) return 0;
   const long long bytes = (long long)n * sample_parts(vocab) * (long long)sizeof(PartRecord);
@@ -1273,9 +1273,9 @@ extern "C" long long ta_sample_scratch(int n, int vocab) {
 }
 
 // scratch: ta_sample_scratch bytes on an 8-byte boundary, or null: one workgroup takes a row then.
-extern "C" int ta_sample(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
-                         float temperature, int top_k, float top_p, const float* uniform,
-                         int* out, void* scratch) {
+extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
+                               float temperature, int top_k, float top_p, const float* uniform,
+                               int* out, void* scratch) {
   TA_REQUIRE(n >= 0 && vocab > 0 && ld >= vocab, "ta_sample: bad sizes n=%d vocab=%d ld=%lld", n, vocab, ld);
   TA_REQUIRE(temperature > 0.f, "ta_sample: temperature %g must be > 0 (0 means argmax)", (double)temperature);
   TA_REQUIRE(top_k >= 1, "ta_sample: top_k %d < 1", top_k);
@@ -1297,4 +1297,10 @@ extern "C" int ta_sample(hipStream_t stream, const float* logits, long long ld, 
                                                          uniform, out);
   }
   return ta_check_launch("ta_sample");
+}
+
+// Without scratch: one workgroup a row.
+extern "C" int ta_sample(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
+                         float temperature, int top_k, float top_p, const float* uniform, int* out) {
+  return ta_sample_parts(stream, logits, ld, n, vocab, temperature, top_k, top_p, uniform, out, nullptr);
 }

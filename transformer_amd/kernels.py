@@ -858,9 +858,9 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, tempe
         _dev(scratch, "scratch", torch.uint8)
         if scratch.numel() < need:
             raise KernelError(f"sample: {scratch.numel()} bytes of scratch, {need} are needed")
-    _check(library().ta_sample(_stream(), _ptr(logits), c_longlong(ld), c_int(n), c_int(vocab),
-                               c_float(temperature), c_int(min(int(top_k), vocab)),
-                               c_float(top_p), _ptr(uniform), _ptr(out), _ptr(scratch)))
+    _check(library().ta_sample_parts(_stream(), _ptr(logits), c_longlong(ld), c_int(n), c_int(vocab),
+                                     c_float(temperature), c_int(min(int(top_k), vocab)),
+                                     c_float(top_p), _ptr(uniform), _ptr(out), _ptr(scratch)))
     return out
 
 
