@@ -998,6 +998,29 @@ def test_sample_rows_on_16_byte_boundaries_and_others_choose_alike(vocab):
         assert torch.equal(a, b), (T, k, p_, (a != b).nonzero().flatten().tolist())
 
 
+# rows, vocabulary, top_k, top_p: rows in turns; each of the lines between parts and a workgroup a row from both sides;
+# more tokens than parts are kept for (none of a row's, then one that the gathered tokens settle)
+@pytest.mark.parametrize("n,vocab,k,p,parts", [
+    (272, 128256, 2000, 0.9, True), (273, 128256, 2000, 0.9, False), (187, 128256, 40, 0.95, True), (188, 128256, 40, 0.95, False), (116, 128256, 128256, 1.0, True),
+    (118, 128256, 128256, 1.0, False), (3, 4096, 4096, 1.0, False), (2, 1048576, 1048576, 0.8, True), (2, 1048580, 1048580, 0.8, False),
+    (2, 1100000, 50, 1.0, False), (9000, 300, 40, 0.9, True)])
+def test_sample_by_turns_and_by_a_workgroup_a_row(n, vocab, k, p, parts):
+    """Every route chooses what the kernel that walks unaligned rows token by token chooses, within 24 MB of scratch."""
+    from transformer_amd import kernels
+    g = torch.Generator(device=DEV).manual_seed(n)
+    ld = (vocab + 7) // 4 * 4
+    logits = torch.randn(n, ld, generator=g, device=DEV) * 2.0
+    shifted = torch.empty(n, ld, device=DEV)[:, 1:1 + vocab]
+    shifted.copy_(logits[:, :vocab])
+    u = torch.rand(n, generator=g, device=DEV)
+    a, b = (torch.empty(n, dtype=torch.int32, device=DEV) for _ in range(2))
+    need = kernels.sample_scratch(n, vocab, k, p)
+    assert (need > 0) == parts and need <= 24 << 20 and kernels.sample_scratch(n, vocab) <= 24 << 20
+    kernels.sample(logits[:, :vocab], u, a, 0.9, k, p)
+    kernels.sample(shifted, u, b, 0.9, k, p)
+    assert torch.equal(a, b)
+
+
 def test_sample_without_scratch_keeps_its_entry_point():
     """ta_sample has the ten arguments it always had; ta_sample_parts takes the scratch."""
     from ctypes import c_float, c_int, c_longlong

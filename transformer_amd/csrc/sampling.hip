@@ -459,11 +459,20 @@ __device__ void choose_digit(SelectState& st, const uint32_t* h_cnt, const u64* 
   }
 }
 
+#define CAND_PER_WAVE 256  // tokens near the maximum that a wave's share of the row may hold
+#define NEAR_BINS 96       // steps of 1/9 counted one by one: down to e^-10.7 of the largest probability
+
+// distance from the maximum in steps of 1/9 of (max - logit) / T; 255 holds all that is further
+__device__ __forceinline__ int near_bin(float l, float m, float inv_t) {
+  const float d = (m - l) * inv_t * 9.0f;
+  return d < 255.0f ? (int)d : 255;
+}
+
 // The same choice by one workgroup for a row that starts on a 16-byte boundary, every pass over the row bringing
-// sixteen bytes per lane: what is left for rows whose threshold the parts below cannot enclose (more than
-// PART_CAND tokens of a part within a step of it, as when thousands are equal, or a threshold more than 16 units of
-// logit / T under the maximum). All sums are integer sums and the sweeps keep the order of the indices, so every way
-// chooses the same token.
+// sixteen bytes per lane. GATHER: the kept tokens, where they are few, go through LDS and the row is read three times;
+// without it (rows whose threshold the parts below cannot enclose: more than PART_CAND tokens of a part within a step
+// of it, as when thousands are equal, or a threshold more than 16 units of logit / T under the maximum) up to nine
+// times. All sums are integer sums and the sweeps keep the order of the indices, so every way chooses the same token.
 #define VEC_STEPS 64      // steps of 256 tokens whose sums a wave remembers (16 waves: 262,144 tokens)
 struct Four {
   float v[4];
@@ -488,6 +497,7 @@ __device__ __forceinline__ Four load_four_if(const float* __restrict__ row, int 
   return load_four(row, j < groups ? j : 0, j < groups ? vocab : 0);
 }
 
+template <bool GATHER>
 __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float inv_t, int top_k, float top_p,
                                  float uniform, int* __restrict__ out) {
   const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
@@ -502,6 +512,11 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
   __shared__ u64 s_total;
   __shared__ int s_pick;
   __shared__ u64 s_step[SAMPLE_WAVES][VEC_STEPS];      // kept mass of each step of a wave's range
+  // tokens near the maximum, gathered in index order: wave w's share of the row in cand_*[w]
+  __shared__ float cand_l[GATHER ? SAMPLE_WAVES : 1][GATHER ? CAND_PER_WAVE : 1];
+  __shared__ int cand_i[GATHER ? SAMPLE_WAVES : 1][GATHER ? CAND_PER_WAVE : 1];
+  __shared__ int s_ccnt[SAMPLE_WAVES];
+  __shared__ int s_small;
 
   // ---- max
   float m = -INFINITY;
@@ -536,6 +551,7 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
     st.tie_count = 0xffffffffu;   // "every token of the threshold value is kept"
     st.tie_mass = 0;
     s_pick = 0;
+    s_small = 0;
   }
   for (int i = threadIdx.x; i < 256; i += SAMPLE_THREADS) {
     h_cnt[i] = 0;
@@ -543,8 +559,71 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
   }
   __syncthreads();
 
+  // ---- with a cut: the tokens by their distance from the maximum, in steps of 1/9 of a
+  // unit of (max - logit) / T. The sums give the total mass, and the step in which the count
+  // reaches top_k or the mass reaches top_p bounds the kept set: usually a few hundred
+  // tokens, which are then gathered into LDS and cut and drawn from there, so the row is
+  // read three times in all instead of nine. When that step lies far from the maximum or
+  // the tokens do not fit, the digits of the threshold are found over the whole row.
+  if (GATHER && cut) {
+    // steps from NEAR_BINS on are lumped into the last one, summed in registers: most tokens
+    // lie there, and the cut almost never does
+    uint32_t far_cnt = 0;
+    u64 far_mass = 0;
+    const bool need_total = top_p < 1.0f;    // top-k alone never asks for the mass of the far tokens
+    for (int j = threadIdx.x; j < groups; j += 4 * SAMPLE_THREADS) {
+      Four f[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f[u] = load_four_if(row, j + u * SAMPLE_THREADS, groups, vocab);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (!f[u].ok[e]) continue;
+          const int bin = near_bin(f[u].v[e], m, inv_t);
+          if (bin < NEAR_BINS) {             // such a token has mass left by a wide margin
+            atomicAdd(&h_cnt[bin], 1u);
+            atomicAdd(&h_mass[bin], fixed_mass(f[u].v[e], m, inv_t));
+          } else {
+            ++far_cnt;
+            if (need_total) far_mass += fixed_mass(f[u].v[e], m, inv_t);
+          }
+        }
+    }
+    far_cnt = (uint32_t)wave_sum_u64(far_cnt);
+    far_mass = wave_sum_u64(far_mass);
+    if (lane == 0 && far_cnt) {
+      atomicAdd(&h_cnt[255], far_cnt);
+      atomicAdd(&h_mass[255], far_mass);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      u64 t = 0;
+      for (int bin = 0; bin < 256; ++bin) t += h_mass[bin];
+      s_total = t;
+      const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
+      u64 p_lim = (u64)ceil((double)top_p * (double)t);
+      if (p_lim < 1) p_lim = 1;
+      if (p_lim > t) p_lim = t;
+      if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;   // the far tokens' mass was not summed; nothing is cut by mass
+      uint32_t ca = 0;
+      u64 ma = 0;
+      int last = 255;
+      for (int bin = 0; bin < 256; ++bin) {
+        ca += h_cnt[bin];
+        ma += h_mass[bin];
+        if (ca >= k_lim || ma >= p_lim) {
+          last = bin;
+          break;
+        }
+      }
+      s_pick = last;                          // borrowed until the draw: the last step that matters
+      s_small = t > 0 && last < NEAR_BINS && ca <= (uint32_t)(SAMPLE_WAVES * CAND_PER_WAVE);
+    }
+    __syncthreads();
+  }
   // ---- total mass, which only the cut by mass asks for
-  if (cut) {
+  if (!GATHER && cut) {
     u64 tot = 0;
     if (top_p < 1.0f)
       for (int j = threadIdx.x; j < groups; j += SAMPLE_THREADS) {
@@ -557,11 +636,169 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
     __syncthreads();
   }
   const u64 total = s_total;
+  const int near_last = GATHER ? s_pick : 0;
+  if (GATHER) {
+    __syncthreads();
+    if (threadIdx.x == 0) s_pick = 0;
+  }
 
   const int span = ((groups + SAMPLE_WAVES - 1) / SAMPLE_WAVES + TA_WAVE - 1) / TA_WAVE * TA_WAVE;
   const int lo = wave * span;
   const int hi = (lo + span < groups) ? lo + span : groups;
   const u64 lanes_below = ((u64)1 << lane) - 1;
+
+  // ---- gather the tokens of the steps up to that one, wave by wave in index order
+  if (GATHER && cut && s_small) {
+    int have = 0;
+    for (int j0 = lo; j0 < hi; j0 += TA_WAVE) {
+      const int j = j0 + lane;
+      Four f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f.v[e] = -INFINITY;
+        f.ok[e] = false;
+      }
+      if (j < hi) f = load_four(row, j, vocab);
+      bool take[4];
+      int before = 0, all = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        take[e] = f.ok[e] && near_bin(f.v[e], m, inv_t) <= near_last;
+        const u64 b = __ballot(take[e]);
+        before += __popcll(b & lanes_below);
+        all += __popcll(b);
+      }
+      int at = have + before;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (take[e]) {
+          if (at < CAND_PER_WAVE) {
+            cand_l[wave][at] = f.v[e];
+            cand_i[wave][at] = 4 * j + e;
+          }
+          ++at;
+        }
+      have += all;
+    }
+    if (lane == 0) s_ccnt[wave] = have;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int ok = 1;
+      for (int w = 0; w < SAMPLE_WAVES; ++w)
+        if (s_ccnt[w] > CAND_PER_WAVE) ok = 0;         // a wave's share did not fit: the long way
+      s_small = ok;
+    }
+    __syncthreads();
+  }
+
+  if (GATHER && cut && s_small) {
+    // ---- the cut among the gathered tokens (they hold every token at or above the threshold)
+    const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
+    u64 p_lim = (u64)ceil((double)top_p * (double)total);
+    if (p_lim < 1) p_lim = 1;
+    if (p_lim > total) p_lim = total;
+    if (top_p >= 1.0f) p_lim = NO_MASS_LIMIT;      // see above: only top_k cuts
+    const int mine = s_ccnt[wave];
+    for (int pass = 0; pass < 4; ++pass) {
+      const int shift = 24 - 8 * pass;
+      for (int i = threadIdx.x; i < 256; i += SAMPLE_THREADS) {
+        h_cnt[i] = 0;
+        h_mass[i] = 0;
+      }
+      __syncthreads();
+      const uint32_t prefix = st.prefix, mask = st.mask;
+      for (int c = lane; c < mine; c += TA_WAVE) {
+        const float l = cand_l[wave][c];
+        const uint32_t key = order_key(l);
+        if ((key & mask) == prefix) {
+          const int bin = (key >> shift) & 255;
+          atomicAdd(&h_cnt[bin], 1u);
+          atomicAdd(&h_mass[bin], fixed_mass(l, m, inv_t));
+        }
+      }
+      __syncthreads();
+      if (wave == 0) choose_digit(st, h_cnt, h_mass, shift, pass == 3, k_lim, p_lim);
+      __syncthreads();
+    }
+    const uint32_t thr = st.prefix;
+    const uint32_t n_tie = st.tie_count;
+    // ---- the draw, in index order: wave by wave, and inside a wave as gathered
+    uint32_t ties = 0;
+    for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
+      const int c = c0 + lane;
+      ties += __popcll(__ballot(c < mine && order_key(cand_l[wave][c]) == thr));
+    }
+    if (lane == 0) s_c[wave] = ties;
+    __syncthreads();
+    uint32_t tie_base = 0;
+    for (int w = 0; w < wave; ++w) tie_base += s_c[w];
+    u64 kept = 0;
+    {
+      uint32_t rank = tie_base;
+      for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
+        const int c = c0 + lane;
+        bool keep = false, tie = false;
+        float l = 0.f;
+        if (c < mine) {
+          l = cand_l[wave][c];
+          const uint32_t key = order_key(l);
+          tie = key == thr;
+          keep = key > thr;
+        }
+        const u64 b = __ballot(tie);
+        if (tie && rank + __popcll(b & lanes_below) < n_tie) keep = true;
+        rank += __popcll(b);
+        if (keep) kept += fixed_mass(l, m, inv_t);
+      }
+    }
+    kept = wave_sum_u64(kept);
+    if (lane == 0) s_q[wave] = kept;
+    __syncthreads();
+    u64 mass_base = 0, kept_total = 0;
+    for (int w = 0; w < SAMPLE_WAVES; ++w) {
+      if (w < wave) mass_base += s_q[w];
+      kept_total += s_q[w];
+    }
+    u64 target = (u64)((double)uniform * (double)kept_total);
+    if (kept_total > 0 && target >= kept_total) target = kept_total - 1;
+    if (kept_total > 0 && target >= mass_base && target < mass_base + s_q[wave]) {
+      uint32_t rank = tie_base;
+      u64 run = mass_base;
+      for (int c0 = 0; c0 < mine; c0 += TA_WAVE) {
+        const int c = c0 + lane;
+        bool keep = false, tie = false;
+        float l = 0.f;
+        if (c < mine) {
+          l = cand_l[wave][c];
+          const uint32_t key = order_key(l);
+          tie = key == thr;
+          keep = key > thr;
+        }
+        const u64 b = __ballot(tie);
+        if (tie && rank + __popcll(b & lanes_below) < n_tie) keep = true;
+        rank += __popcll(b);
+        const u64 q = keep ? fixed_mass(l, m, inv_t) : 0;
+        u64 inc = q;
+#pragma unroll
+        for (int o = 1; o < TA_WAVE; o <<= 1) {
+          const u64 up = shfl_up_u64(inc, o);
+          if (lane >= o) inc += up;
+        }
+        const bool hit = q > 0 && run + inc > target && run + inc - q <= target;
+        if (__ballot(hit)) {
+          if (hit) s_pick = cand_i[wave][c];
+          break;
+        }
+        uint32_t lo32 = (uint32_t)inc, hi32 = (uint32_t)(inc >> 32);
+        lo32 = __shfl(lo32, TA_WAVE - 1, TA_WAVE);
+        hi32 = __shfl(hi32, TA_WAVE - 1, TA_WAVE);
+        run += ((u64)hi32 << 32) | lo32;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *out = s_pick;
+    return;
+  }
 
   // ---- threshold of the kept set (only when top-k or top-p cut anything)
   if (cut) {
@@ -1101,7 +1338,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
   }
   __syncthreads();
   if (!s_ok) {
-    sample_whole_row(row, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
+    sample_whole_row<false>(row, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
     return;
   }
   const float m = s_max;
@@ -1260,16 +1497,44 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(const float* __restrict__ logits, size_t ld, int vocab,
                                                                      float inv_t, int top_k, float top_p,
                                                                      const float* __restrict__ uniform, int* __restrict__ out) {
-  sample_whole_row(logits + (size_t)blockIdx.x * ld, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
+  sample_whole_row<true>(logits + (size_t)blockIdx.x * ld, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
 }
 
 static int sample_parts(int vocab) { return (vocab + PART - 1) / PART; }
 
+// Rows that are dealt out in parts at a time, so that the records stay within 24 MB (8,600 rows of one part); more go
+// through in turns.
+static int rows_at_a_time(int vocab) {
+  const long long rows = (24ll << 20) / (sample_parts(vocab) * (long long)sizeof(PartRecord));
+  return rows < 1 ? 1 : rows > 65535 ? 65535 : (int)rows;
+}
+
+// Whether rows are better dealt out in parts than given to a workgroup each (GPU time of a call, us, parts against whole):
+// - nothing is cut: three launches, which pay while few workgroups would walk long rows. 8 x 1,000 13 against 5; 8 x
+//   32,000 14.5 against 14.5; 8 x 128,256 16 against 44; 64 x 128,256 29 against 48; 512 x 128,256 148 against 104. A row
+//   alone costs 5 + 3e-4 a token, parts 12 + 2.1e-6 a token of all rows.
+// - else a workgroup gathers the kept tokens where they are few, and with every CU busy its three passes are cheaper than
+//   the parts' two with the exponential in both. k 40, p 0.95: 100 x 128,256 68 against 110 or so; 188: 101 against 80;
+//   512: 240 against 146; 2,500: 1,164 against 599; 740 x 32,000 108 against 130; 760: 119 against 72; 1,024 x 8,192 61
+//   against 121. Kept tokens that don't fit (a cut by mass alone can keep thousands) are walked nine times: 188 x 128,256,
+//   p 0.9, 109 against 286, 512 257 against 451, but 235 against 129 where dozens are kept: such cuts stay in parts a little
+//   longer.
+static bool in_parts(int n, int vocab, int top_k, float top_p) {
+  if (sample_parts(vocab) > MAX_PARTS) return false;
+  const long long all = (long long)n * vocab;
+  if (top_k >= vocab && top_p >= 1.0f) return all < 145ll * vocab - 3500000;
+  return vocab <= 16384 || all <= (top_k <= 1024 ? 24000000 : 35000000);
+}
+
 // Bytes of scratch that lets ta_sample_parts deal rows out in parts (0: rows of this vocabulary are not).
 extern "C" long long ta_sample_scratch(int n, int vocab) {
-  if (n <= 0 || n > 65535 || vocab <= 0 || sample_parts(vocab) > MAX_PARTS) return 0;
-  const long long bytes = (long long)n * sample_parts(vocab) * (long long)sizeof(PartRecord);
-  return bytes <= (256ll << 20) ? bytes : 0;     // thousands of rows fill the chip one workgroup each
+  if (n <= 0 || vocab <= 0 || sample_parts(vocab) > MAX_PARTS) return 0;
+  const int rows = n < rows_at_a_time(vocab) ? n : rows_at_a_time(vocab);
+  return (long long)rows * sample_parts(vocab) * (long long)sizeof(PartRecord);
+}
+// The same for these cuts: 0 also where a workgroup a row is the better way.
+extern "C" long long ta_sample_scratch_for(int n, int vocab, int top_k, float top_p) {
+  return n > 0 && vocab > 0 && in_parts(n, vocab, top_k, top_p) ? ta_sample_scratch(n, vocab) : 0;
 }
 
 // scratch: ta_sample_scratch bytes on an 8-byte boundary, or null: one workgroup takes a row then.
@@ -1285,16 +1550,21 @@ extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long lon
   const float inv_t = 1.0f / temperature;
   if (((uintptr_t)logits % 16) != 0 || ld % 4 != 0) {
     sample_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
-  } else if (scratch == nullptr || ta_sample_scratch(n, vocab) == 0) {
+  } else if (scratch == nullptr || !in_parts(n, vocab, top_k, top_p)) {
     sample_rows_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
   } else {
     const int parts = sample_parts(vocab), cut = top_k < vocab || top_p < 1.0f;
     PartRecord* rec = (PartRecord*)scratch;
-    const dim3 g(parts, n);
-    sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec);
-    sample_gather_kernel<<<g, PART_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, cut, rec);
-    sample_draw_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, cut, parts, rec,
-                                                         uniform, out);
+    const int turn = rows_at_a_time(vocab);
+    for (int r0 = 0; r0 < n; r0 += turn) {
+      const int rows = n - r0 < turn ? n - r0 : turn;
+      const float* from = logits + (size_t)r0 * ld;
+      const dim3 g(parts, rows);
+      sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec);
+      sample_gather_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, cut, rec);
+      sample_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, cut, parts, rec,
+                                                              uniform + r0, out + r0);
+    }
   }
   return ta_check_launch("ta_sample");
 }

@@ -834,11 +834,14 @@ def argmax(logits: torch.Tensor, out: torch.Tensor):
     return out
 
 
-def sample_scratch(rows: int, vocab: int) -> int:
-    """Bytes of scratch with which ``sample`` deals rows out among workgroups (0: it does not)."""
-    need = library().ta_sample_scratch
+def sample_scratch(rows: int, vocab: int, top_k: Optional[int] = None, top_p: Optional[float] = None) -> int:
+    """Bytes of scratch with which ``sample`` deals rows out among workgroups, at most 24 MB (0: it does not). With
+    top_k and top_p: 0 also where those cuts are better left to a workgroup a row."""
+    need = library().ta_sample_scratch if top_p is None else library().ta_sample_scratch_for
     need.restype = c_longlong
-    return int(need(c_int(rows), c_int(vocab)))
+    if top_p is None:
+        return int(need(c_int(rows), c_int(vocab)))
+    return int(need(c_int(rows), c_int(vocab), c_int(min(int(top_k), vocab)), c_float(top_p)))
 
 
 def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, temperature: float,
@@ -851,7 +854,8 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, tempe
     if out.numel() != n or uniform.numel() != n:
         raise KernelError("sample: out and uniform must hold one entry per row")
     vocab = logits.shape[1]
-    need = sample_scratch(n, vocab)
+    walks = logits.data_ptr() % 16 or ld % 4           # rows off 16 bytes: a workgroup walks one token at a time
+    need = 0 if walks else sample_scratch(n, vocab, top_k, float(top_p))
     if scratch is None:
         scratch = torch.empty(need, dtype=torch.uint8, device=logits.device) if need else None
     else:

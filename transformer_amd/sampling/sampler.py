@@ -76,12 +76,12 @@ class Sampler:
                                             zip(sequences, drawn)], dtype=np.float32)
             u_dev.copy_(u_host, non_blocking=True)
             k = self.args.top_k if self.args.top_k is not None else logits.shape[1]
-            need = kernels.sample_scratch(n, logits.shape[1])
+            need = kernels.sample_scratch(n, logits.shape[1], int(k), float(self.args.top_p))
             i = (self._turn - 1) % self.RING              # of the buffers just taken
-            if self._scratch[i] is None or self._scratch[i].numel() < need:
+            if need and (self._scratch[i] is None or self._scratch[i].numel() < need):
                 self._scratch[i] = torch.empty(need, dtype=torch.uint8, device=self.device)
             kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
-                           float(self.args.top_p), self._scratch[i])
+                           float(self.args.top_p), self._scratch[i] if need else None)
         out_host.copy_(out, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
