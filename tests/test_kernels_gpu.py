@@ -146,9 +146,10 @@ def test_rope_kv_write(dtype, dh, style, many):
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("nq,nkv,dh,style,cache", [(3, 2, 48, "half", True), (2, 2, 128, "interleaved", True),
-                                                   (4, 1, 16, "interleaved", True), (2, 1, 64, "half", False), (2, 1, 256, "half", True)])
+                                                   (4, 1, 16, "interleaved", True), (2, 1, 64, "half", False), (2, 1, 256, "half", True),
+                                                   (1, 43, 96, "half", True)])
 def test_rope_kv_write_of_prompts(dtype, nq, nkv, dh, style, cache):
-    """64 tokens and more: whole groups of places, groups cut by a page's end, by the end of a sequence and by the
+    """64 tokens and more (43 kv heads: enough for the widest part of a head, and a rest): whole groups of places, groups cut by a page's end, by the end of a sequence and by the
     end of a block of 64 tokens, tokens that are not stored; nothing but their places is written."""
     from transformer_amd import kernels
     own = np.random.default_rng([nq, dh])

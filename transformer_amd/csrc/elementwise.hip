@@ -524,13 +524,16 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec_kernel(
   }
 }
 
-// Prompts of 64 tokens and more, heads of whole 16 elements: bound by its bytes (q and k read and written, k and v
+// 64 tokens and more, heads of whole 16 elements: bound by its bytes (q and k read and written, k and v
 // stored once more). q and k: a thread takes two runs of eight elements that hold each other's partners (style 0:
 // elements j..j+7 and those dh/2 further on; style 1: sixteen in a row) and asks for all it needs at once. v:
-// a workgroup takes 64 tokens of one kv head through LDS and stores the transposed page line by line: groups of
-// 16 bytes of neighbouring places, eight lanes a line of 128, where the kernel above wrote 8 bytes every 128 (a
-// line then went to memory in sixteen pieces). 4,454 tokens of 32 + 32 + 32 heads of 128: 201 -> 43.5 us (5.8 TB/s); 8,159 of 32 +
-// 8 + 8: 105 -> 36; 2,011: 18.6 -> 11.5.
+// a workgroup takes 64 tokens of `cols` columns of one kv head (a line of memory, fewer where the chip would stay empty)
+// through LDS and stores the transposed page line by line: groups of 16 bytes of neighbouring places, eight lanes a line
+// of 128, where the kernel above wrote 8 bytes every 128 (a line then went to memory in sixteen pieces). bfloat16, heads
+// of 128, 32 + 32 + 32 of them: 2,048 tokens of a prompt 42.7 -> 20.3 us, 4,454 201 -> 43.5 (5.8 TB/s), 64 6.0 -> 3.6; 32 +
+// 8 + 8: 2,048 16.5 -> 10.2, 64 4.6 -> 3.1; 4 + 1 of 256: 64 3.8 -> 3.0 (6.1 with the whole head to a workgroup). Tokens
+// that land apart (single tokens of many sequences) are stored element by element as above: 64 of 32 + 8 + 8 5.3 -> 4.8
+// (15.4 with the whole head to a workgroup), 64 of 16 + 4 + 4 in float32 4.0 -> 4.4, 512 7.2 -> 7.7.
 template <typename T> struct Run8 {
   Vec4<T> a, b;
   __device__ __forceinline__ void load(const T* p) {
@@ -562,7 +565,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
     T* __restrict__ qkv, const float* __restrict__ bias, const int* __restrict__ dest,
     const float2* __restrict__ cs, int style, T* __restrict__ kcache, T* __restrict__ vcache,
-    int nt, int nq, int nkv, int dh, int turn_blocks) {
+    int nt, int nq, int nkv, int dh, int turn_blocks, int cols) {
   const size_t width = (size_t)(nq + 2 * nkv) * dh;
   const bool cache = kcache != nullptr && dest != nullptr;
   if ((int)blockIdx.x < turn_blocks) {
@@ -625,12 +628,13 @@ __global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
   }
   // ---- v heads
   extern __shared__ __attribute__((aligned(16))) unsigned char rope_lds[];
-  T* tile = reinterpret_cast<T*>(rope_lds);              // [64][dh + 2]
+  T* tile = reinterpret_cast<T*>(rope_lds);              // [64][cols + 2]
   __shared__ int slot[64], first[65], groups_s;
   constexpr int RUN = 16 / (int)sizeof(T);
-  const int unit = blockIdx.x - turn_blocks, g = unit % nkv, t0 = unit / nkv * 64;
-  const int ntok = nt - t0 < 64 ? nt - t0 : 64, ld = dh + 2;
-  const float* vb = bias ? bias + (size_t)(nq + nkv + g) * dh : nullptr;
+  const int per_head = (dh + cols - 1) / cols, unit = blockIdx.x - turn_blocks, part = unit % (per_head * nkv);
+  const int g = part / per_head, d0 = part % per_head * cols, nd = dh - d0 < cols ? dh - d0 : cols, t0 = unit / (per_head * nkv) * 64;
+  const int ntok = nt - t0 < 64 ? nt - t0 : 64, ld = cols + 2;
+  const float* vb = bias ? bias + (size_t)(nq + nkv + g) * dh + d0 : nullptr;
   if (threadIdx.x < 64) {
     const int i = threadIdx.x;
     const int sl = cache && i < ntok ? dest[t0 + i] : -1;
@@ -644,10 +648,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
       first[__popcll(mask)] = ntok;
     }
   }
-  const int pieces = dh / 8;
+  const int pieces = nd / 8;
   for (int it = threadIdx.x; it < ntok * pieces; it += 256) {
     const int i = it / pieces, o = it % pieces * 8;
-    T* from = qkv + (size_t)(t0 + i) * width + (size_t)(nq + nkv + g) * dh + o;
+    T* from = qkv + (size_t)(t0 + i) * width + (size_t)(nq + nkv + g) * dh + d0 + o;
     Run8<T> x;
     x.load(from);
     if (vb) {
@@ -663,11 +667,11 @@ __global__ __launch_bounds__(256) void rope_kv_write_lines_kernel(
   __syncthreads();
   if (!cache) return;
   const int groups = groups_s;
-  for (int it = threadIdx.x; it < groups * dh; it += 256) {
+  for (int it = threadIdx.x; it < groups * nd; it += 256) {
     const int q = it % groups, d = it / groups;
     const int i0 = first[q], n = first[q + 1] - i0, sl = slot[i0];
     if (sl < 0) continue;
-    T* to = vcache + (((size_t)(sl / TA_PAGE) * nkv + g) * dh + d) * TA_PAGE + sl % TA_PAGE;
+    T* to = vcache + (((size_t)(sl / TA_PAGE) * nkv + g) * dh + d0 + d) * TA_PAGE + sl % TA_PAGE;
     if (n == RUN && sl % RUN == 0) {
       struct alignas(16) { T x[RUN]; } line;
 #pragma unroll
@@ -688,19 +692,22 @@ extern "C" int ta_rope_kv_write(hipStream_t stream, int dtype, void* qkv, const 
   TA_REQUIRE((kcache == nullptr) == (vcache == nullptr), "ta_rope_kv_write: K and V cache must come together");
   if (nt == 0) return 0;
   const bool aligned = ((uintptr_t)qkv % 16) == 0 && ((uintptr_t)kcache % 16) == 0 && ((uintptr_t)vcache % 16) == 0;
-  const size_t tile = 64 * (size_t)(dh + 2) * (dtype == TA_F32 ? 4 : 2);       // of values on their way through LDS
-  if (nt >= 64 && dh % 16 == 0 && tile <= 40960 && aligned && ((uintptr_t)cs % 16) == 0 &&
+  if (nt >= 64 && dh % 16 == 0 && aligned && ((uintptr_t)cs % 16) == 0 &&
       (dtype == TA_F32 || dtype == TA_BF16)) {
     const long long turns = ((long long)nt * (nq + nkv) * (dh / 16) + 255) / 256;
-    const long long lines = (kcache != nullptr && dest != nullptr) || bias ? (long long)((nt + 63) / 64) * nkv : 0;
+    const long long groups = (long long)((nt + 63) / 64) * nkv;
+    int cols = dtype == TA_F32 ? 32 : 64;
+    while (cols > 16 && groups * ((dh + cols - 1) / cols) < 256) cols /= 2;
+    const long long lines = (kcache != nullptr && dest != nullptr) || bias ? groups * ((dh + cols - 1) / cols) : 0;
     TA_REQUIRE(turns + lines <= 2147483647ll, "ta_rope_kv_write: %d tokens of %d heads are too many for one launch", nt, nq + 2 * nkv);
+    const size_t tile = 64 * (size_t)(cols + 2) * (dtype == TA_F32 ? 4 : 2);       // of values on their way through LDS
     const dim3 gl((unsigned)(turns + lines));
     if (dtype == TA_F32)
       rope_kv_write_lines_kernel<float><<<gl, 256, tile, stream>>>((float*)qkv, bias, dest, (const float2*)cs, style,
-                                                                   (float*)kcache, (float*)vcache, nt, nq, nkv, dh, (int)turns);
+                                                                   (float*)kcache, (float*)vcache, nt, nq, nkv, dh, (int)turns, cols);
     else
       rope_kv_write_lines_kernel<bf16_t><<<gl, 256, tile, stream>>>((bf16_t*)qkv, bias, dest, (const float2*)cs, style,
-                                                                    (bf16_t*)kcache, (bf16_t*)vcache, nt, nq, nkv, dh, (int)turns);
+                                                                    (bf16_t*)kcache, (bf16_t*)vcache, nt, nq, nkv, dh, (int)turns, cols);
     return ta_check_launch("ta_rope_kv_write");
   }
   if (nt >= 8 && dh % 8 == 0 && aligned && (dtype == TA_F32 || dtype == TA_BF16)) {
