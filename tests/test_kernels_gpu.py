@@ -683,9 +683,11 @@ def test_float32_attention_of_sequences_that_bring_no_token(counts):
 
 
 # rows at which the kernel or its tile changes, k inside and at the ends of blocks, segments and rounds of
-# segments, workgroups' tiles that end inside the matrix (the last two: tiles of 64 and of 128)
+# segments, workgroups' tiles that end inside the matrix (tiles of 64 and of 128), lengths up to which waves end
+# where k does and from which they don't, the longest k whose single rows go to tiles
 @pytest.mark.parametrize("mnk", [(1, 7, 256), (8, 23, 260), (9, 33, 2052), (16, 17, 1028), (17, 40, 516), (33, 19, 2304),
-                                 (64, 50, 100), (130, 70, 1540), (130, 4100, 300), (1100, 5570, 68)])
+                                 (64, 50, 100), (130, 70, 1540), (130, 4100, 300), (1100, 5570, 68), (1, 30, 1792), (7, 30, 1796),
+                                 (12, 20, 768), (40, 33, 772), (3, 12300, 128), (3, 12300, 132), (2, 50, 16)])
 @pytest.mark.parametrize("types", [("float32", "float32"), ("bfloat16", "float32"), ("bfloat16", "bfloat16")])
 def test_gemm_simple_at_the_edges_of_its_tiles(mnk, types):
     from transformer_amd import kernels

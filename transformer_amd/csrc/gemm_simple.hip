@@ -54,7 +54,10 @@ __device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
 // PAIR (up to 8 rows): a matrix instruction multiplies two segments side by side, 8 columns of W each, of
 // whose 16 x 16 products the two squares on the diagonal are used. A workgroup then owns 8 columns: a matrix of
 // 2,048 rows keeps 256 CUs reading instead of 128.
-template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool VEC>
+// SHORT: k does not fill a round of segments. A wave then ends where k does instead of multiplying zeros to the end of
+// its segment: 40 x 5,000 x 64 6.3 us (21 without), 1 x 5,000 x 768 6.9 (10.6). The test between the chunks costs
+// long k 2 to 4 % (8 x 16,384 x 4,096 74.6 us without it, 77.3 with).
+template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool SHORT, bool VEC>
 __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __restrict__ A, int lda,
                                                                    const TW* __restrict__ W, int ldw,
                                                                    const float* __restrict__ bias,
@@ -113,8 +116,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     static_assert(CPS % 2 == 0, "chunks of a segment in pairs");
+    const int seg0 = SHORT ? __builtin_amdgcn_readfirstlane((round * TURN + (PAIR ? 2 * wave : wave)) * SEG) : 0;
 #pragma unroll
     for (int c = 0; c < CPS; c += 2) {
+      if (SHORT && seg0 + c * BC * BLK >= K) break;       // the rest of this wave's segments lies past K
       load(1, round * CPS + c + 1);
       __builtin_amdgcn_sched_barrier(0);
       multiply(0);
@@ -321,8 +326,10 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
   // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
   // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
-  // against 340). Tiles of 128 take two workgroups on every CU to fill.
-  if (M > 64 && tiles(64) >= 192) {
+  // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
+  // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
+  const bool brief = K <= 128;
+  if (tiles(64) >= 192 && (M > 64 || brief)) {
     if (tiles(128) >= 384)
       gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
           A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
@@ -331,16 +338,22 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
           A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
     return;
   }
-#define FEW(WAVES, RT, BC, PAIR)                                                                               \
-  gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, VEC>                                                    \
+#define FEW_(WAVES, RT, BC, PAIR, SHORT)                                                                       \
+  gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, SHORT, VEC>                                             \
       <<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch), WAVES * 64, 0, stream>>>( \
           A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
+#define FEW(WAVES, RT, BC, PAIR)                                                                               \
+  do {                                                                                                         \
+    if (K <= (WAVES * (PAIR ? 2 : 1) - 1) * SEG) FEW_(WAVES, RT, BC, PAIR, true);                              \
+    else FEW_(WAVES, RT, BC, PAIR, false);                                                                     \
+  } while (0)
   // four waves a workgroup and 16 KB on their way in each: several workgroups share a CU and fill each other's
   // starts and ends (16,384 x 2,048 at 16 rows: 38 us; 44 with eight waves and twice the loads)
   if (M <= 8) FEW(4, 1, 4, true);
   else if (M <= 16) FEW(4, 1, 4, false);
   else if (M <= 32) FEW(4, 2, 2, false);
   else FEW(4, 4, 2, false);
+#undef FEW_
 #undef FEW
 }
 
