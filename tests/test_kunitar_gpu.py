@@ -216,9 +216,11 @@ def test_experts_products_in_every_form(form, geom):
 
 # tiles of the experts, N, K: experts of one tile side by side, of 15 to 17 and 33 (blocks of 16 begin at an expert's first
 # tile, workgroups own those that begin at four tiles), columns around 256 and not in fours, k around 32 and short of the
-# steps that are sent ahead
+# steps that are sent ahead; blocks of 8 and (from the sixth on) of 16 tiles, runs over 64 and 4,096 tiles, which are
+# looked at together
 @pytest.mark.parametrize("geom", [((1, 1, 1, 1, 1, 2, 3), 256, 32), ((15, 16, 17, 1, 33), 257, 136), ((3, 0, 64, 5, 11), 130, 264),
-                                  ((2, 9, 12), 516, 8), ((16, 48), 8, 96)])
+                                  ((2, 9, 12), 516, 8), ((16, 48), 8, 96), ((70, 130, 1, 64, 63, 65, 127), 1100, 40),
+                                  ((3,) * 1400, 24, 16), ((5, 4200, 9), 20, 32)])
 def test_experts_blocks_through_lds_equal_operands_from_memory(geom):
     """The form for many tiles against the one without LDS: the same instruction over the same ascending k, the same bits;
     rows behind the last expert's keep what they held, and operands off 16 bytes take the other form."""

@@ -625,15 +625,19 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
 
 // Many tiles (a prompt): operands through LDS. An expert's tiles of 16 rows are cut, from its first one on, into
 // blocks of up to 16, so that its matrix is read once for every 256 rows. A workgroup of eight waves owns 256 columns
-// of the blocks that begin at four neighbouring tiles (about one block where the experts have four tiles or more; few
-// or none have rows for several), and what is sent for runs on from one block into the next. The operands go from
+// of the blocks that begin at four neighbouring tiles (one block where the experts have four tiles or more), and what is
+// sent for runs on from one block into the next. The operands go from
 // memory to LDS without passing through registers, 32 k at a time, four steps ahead into five buffers (160 KB). A
 // row's four pieces of 16 bytes are permuted by half the row number, so that eight rows' reads meet no bank twice. The
 // waves stand in 2 x 4; each multiplies half of the block's tiles by 64 columns. What bounds it: few rows an expert, the
 // experts' matrices from memory (3.9 TB/s); many, the loads and the reads of LDS around the products (0.67 PFLOP/s).
-// 64 experts of 2,816 x 4,096, 6 of 72 a token (128 rows of eight tiles by 128 columns through registers before):
-// 600 tokens 384 us (487), 1,200 436 (623), 2,943 711 (912), 5,800 1,070 (1,438); of 4,096 x 1,408 into float32,
-// 2,943 tokens 378 (513).
+// Workgroups are numbered by the blocks there are: with one for every four tiles, most of them empty, the blocks of long
+// runs fell on every fourth workgroup and so on a part of the XCDs and shader engines: 32 experts of 2,048 x 1,408 at
+// 8,000 tokens of four 612 us, 292 now (412 by the kernel before blocks); of 1,024 x 4,096 547 and 415 (488); 64 experts
+// of 2,816 x 4,096 at 2,943 tokens of six, unevenly routed, 726 and 652 (978), evenly 764 and 777 (949). Finding its
+// number costs a workgroup some 2 us. Some shapes stay slower than by that kernel (128 rows by 128 columns through
+// registers), whose smaller pieces suit narrow matrices of long k: 8 experts of 1,024 x 4,096 at 4,096 tokens of two 171
+// against 151, 64 of 384 x 2,048 at 6,000 of six 176 against 149.
 #define ML_BM 256
 #define ML_BN 256
 #define ML_BK 32
@@ -661,9 +665,81 @@ static __device__ __forceinline__ void ml_multiply(moe_floatx4 (&acc)[UU][4], co
       acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[v].v, af[u].v, acc[u][v], 0, 0, 0);
 }
 
+// Of the windows of ML_OWN tiles in which a block begins, number `want`: its first tile, or -1 if there are fewer, and in
+// `first` the first tile of that tile's run. A run's blocks begin at every `most` tiles (a power of two) from its first
+// on. All eight waves, 4,096 tiles at a time: one trip to memory, three barriers. `lds`: 1.5 KB.
+static __device__ __forceinline__ int ml_find(const int* __restrict__ tile_expert, int tiles, int most, int want, unsigned char* lds, int& first) {
+  unsigned long long* starts_of = reinterpret_cast<unsigned long long*>(lds);            // of 64 chunks of 64 tiles: where runs start
+  unsigned long long* windows_of = starts_of + 64;                                        // the windows with a block's beginning
+  int* last_of = reinterpret_cast<int*>(windows_of + 64);                                 // the last start in them, or -1
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
+  int begun = 0;                                        // the start of the run that reaches into these 4,096
+  for (int base = 0, seen = 0; base < tiles; base += 4096) {
+    int here[8];
+    unsigned long long starts[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int t = base + (wave + 8 * k) * 64 + lane;
+      here[k] = tile_expert[t < tiles ? t : tiles - 1];
+      const int before = tile_expert[t == 0 ? 0 : t <= tiles ? t - 1 : tiles - 1];
+      here[k] = t < tiles ? here[k] : -1;
+      starts[k] = __ballot(t == 0 || here[k] != before);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (lane == 0) {
+        starts_of[wave + 8 * k] = starts[k];
+        last_of[wave + 8 * k] = starts[k] ? base + (wave + 8 * k) * 64 + 63 - __clzll((long long)starts[k]) : -1;
+      }
+    __syncthreads();
+    int reach = last_of[lane];                          // lane c: the last start up to and with chunk c
+#pragma unroll
+    for (int o = 1; o < TA_WAVE; o <<= 1) {
+      const int up = __shfl_up(reach, o, TA_WAVE);
+      if (lane >= o && up > reach) reach = up;
+    }
+    const int before_ = __shfl_up(reach, 1, TA_WAVE), into = lane && before_ >= 0 ? before_ : begun;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int c = wave + 8 * k, t = base + c * 64 + lane;
+      const unsigned long long mine = starts[k] & ((2ull << lane) - 1);
+      const int carried = __builtin_amdgcn_readlane(into, c);              // by all lanes, whichever needs it
+      const int from = mine ? base + c * 64 + 63 - __clzll((long long)mine) : carried;
+      unsigned long long begins = __ballot(here[k] >= 0 && ((t - from) & (most - 1)) == 0);
+      begins |= begins >> 2;
+      if (lane == 0) windows_of[c] = (begins | begins >> 1) & 0x1111111111111111ull;
+    }
+    __syncthreads();
+    const unsigned long long windows = windows_of[lane], runs = starts_of[lane];
+    const int n = __popcll(windows);
+    int upto = n;
+#pragma unroll
+    for (int o = 1; o < TA_WAVE; o <<= 1) {
+      const int up = __shfl_up(upto, o, TA_WAVE);
+      if (lane >= o) upto += up;
+    }
+    __syncthreads();                                    // everyone has read before the LDS is written again
+    const unsigned long long there = __ballot(want - seen < upto);
+    if (there) {
+      const int who = __ffsll(there) - 1;               // the chunk's lane
+      unsigned long long left = windows;
+      for (int k = lane == who ? want - seen - (upto - n) : 0; k > 0; --k) left &= left - 1;
+      const int at = left ? __ffsll(left) - 1 : 0;
+      const unsigned long long mine = runs & ((2ull << at) - 1);
+      const int from = mine ? base + lane * 64 + 63 - __clzll((long long)mine) : into;
+      first = __builtin_amdgcn_readlane(from, who);
+      return __builtin_amdgcn_readlane(base + lane * 64 + at, who);
+    }
+    seen += __builtin_amdgcn_readlane(upto, 63);
+    const int end = __builtin_amdgcn_readlane(reach, 63);
+    if (end >= 0) begun = end;
+  }
+  return -1;
+}
+
 template <typename TC, bool ACT>
 __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                                           const int* __restrict__ tile_expert, int tiles, int max_rows,
+                                                           const int* __restrict__ tile_expert, int tiles, int most,
                                                            TC* __restrict__ C, int N, int K, int act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ml_lds[];
   moe_u32x4* As = reinterpret_cast<moe_u32x4*>(ml_lds);                 // [ML_ST][ML_BM * 4]
@@ -671,31 +747,23 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
   const int r = lane % 16, kb = lane / 16, wr = wave / 4, wc = wave % 4;
   const int ncol = (N + ML_BN - 1) / ML_BN;
-  const int window = __builtin_amdgcn_readfirstlane((int)(blockIdx.x / (unsigned)ncol));
-  const int n0 = ((int)blockIdx.x - window * ncol) * ML_BN, t0 = window * ML_OWN;
+  const int want = __builtin_amdgcn_readfirstlane((int)(blockIdx.x / (unsigned)ncol));
+  const int n0 = ((int)blockIdx.x - want * ncol) * ML_BN;
+  // Windows without a block have no workgroup: a long run's blocks begin at every fourth window, and with a workgroup each
+  // those would all be the same XCD's or shader engine's.
+  int first;
+  const int t0 = ml_find(tile_expert, tiles, most, want, ml_lds, first);
+  if (t0 < 0) return;
   int e = tile_expert[t0];
-  if (e < 0) return;                                    // tiles past the last expert's rows
-  // the first tile of e's run
-  int first = t0;
-  while (true) {
-    const int i = first - 1 - lane;
-    const unsigned long long other = __ballot(i < 0 || tile_expert[i < 0 ? 0 : i] != e);
-    if (other) {
-      first -= __ffsll(other) - 1;
-      break;
-    }
-    first -= 64;
-  }
   // The blocks that begin at this workgroup's tiles: five bits each, their tiles (none: 0)
   unsigned blocks = 0;
 #pragma unroll
   for (int i = 0; i < ML_OWN; ++i) {
     const int t = t0 + i, here = t < tiles ? tile_expert[t] : -1;
-    if (here < 0) break;
     if (here != e) e = here, first = t;
-    if ((t - first) % ML_TILES == 0) {
+    if (here >= 0 && ((t - first) & (most - 1)) == 0) {
       const int ahead = t + lane;
-      const unsigned long long other = __ballot(lane >= ML_TILES || ahead >= tiles || tile_expert[ahead < tiles ? ahead : t] != e);
+      const unsigned long long other = __ballot(lane >= most || ahead >= tiles || tile_expert[ahead < tiles ? ahead : t] != e);
       blocks |= (unsigned)(__ffsll(other) - 1) << (5 * i);
     }
   }
@@ -781,7 +849,7 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
         ta_wait_loads<4 * (ML_ST - 2)>();                 // this step's pieces; C's stores, if any, only make it wait longer
         __syncthreads();                                  // everyone's; and all have read the buffer that is sent for now
         send(buf == 0 ? ML_ST - 1 : buf - 1);
-        ml_multiply<U>(acc, As + buf * ML_BM * 4, Ws + buf * ML_BN * 4, 16 * U * wr, 64 * wc, r, kb);
+        if (n0 + 64 * wc < N) ml_multiply<U>(acc, As + buf * ML_BM * 4, Ws + buf * ML_BN * 4, 16 * U * wr, 64 * wc, r, kb);
         buf = buf + 1 == ML_ST ? 0 : buf + 1;
       }
       TC* out = C + ((size_t)(t0 + i) * MOE_TILE + r) * N;
@@ -825,9 +893,14 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
 // act: 0 none, 1 gelu, 2 gelu (tanh), 3 relu squared, 4 silu. Tiles past the last expert's
 // rows are skipped and their rows of C keep what they held.
 static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A, const void* W, const int* tile_expert,
-                               void* C, int max_rows, int tiles, int N, int K, int act) {
+                               void* C, int tiles, int N, int K, int act) {
   const size_t lds = (size_t)ML_ST * (ML_BM + ML_BN) * ML_BK * sizeof(bf16_t);
-  const unsigned g = (unsigned)((N + ML_BN - 1) / ML_BN) * (unsigned)((tiles + ML_OWN - 1) / ML_OWN);
+  const int ncol = (N + ML_BN - 1) / ML_BN;
+  const unsigned g = (unsigned)ncol * (unsigned)((tiles + ML_OWN - 1) / ML_OWN);
+  // Blocks of 8 where they give every CU one at most (8 experts, tiles x columns x k: 133 x 2,048 x 1,408 71 us by 16 and
+  // 56 by 8, 520 x 512 x 2,048 95 and 77, 258 x 1,408 x 2,048 95 and 77); beyond, a block of 16 costs less than two of 8
+  // (520 x 2,048 x 1,408 84 against 99).
+  const int most = (long long)((tiles + 7) / 8) * ncol <= 256 ? 8 : ML_TILES;
 #define ML_RUN(TC, ACT)                                                                                          \
   do {                                                                                                           \
     auto kern = moe_gemm_lds_kernel<TC, ACT>;                                                                    \
@@ -838,7 +911,7 @@ static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A,
       if (err != hipSuccess) return ta_fail("ta_moe_gemm: %zu bytes of LDS refused (%s)", lds, hipGetErrorString(err)); \
       allowed = true;                                                                                            \
     }                                                                                                            \
-    kern<<<g, 512, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, tiles, max_rows, (TC*)C, N, K, act); \
+    kern<<<g, 512, lds, stream>>>((const bf16_t*)A, (const bf16_t*)W, tile_expert, tiles, most, (TC*)C, N, K, act); \
   } while (0)
   if (out_dtype == TA_BF16) {
     if (act) ML_RUN(bf16_t, true); else ML_RUN(bf16_t, false);
@@ -894,7 +967,7 @@ extern "C" int ta_moe_gemm_form(hipStream_t stream, int dtype, int out_dtype, co
     const bool few = ta_moe_few_rows(max_rows, N, K);
     const bool aligned = ((uintptr_t)A | (uintptr_t)W) % 16 == 0;   // else operands straight from memory
     if ((form == 3 || (form == 0 && !few)) && aligned)
-      return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, max_rows, tiles, N, K, act);
+      return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, tiles, N, K, act);
     if (form == 1 || (form == 0 && few)) {   // too few workgroups to fill the CUs: the waves divide K
       dim3 gk((N + 63) / 64, tiles);
       const MoeRows rows = {(const bf16_t*)A, nullptr, nullptr, 1};
