@@ -533,7 +533,8 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   const size_t r0 = (size_t)blockIdx.y * MOE_TILE;
   const bf16_t* We = W + (size_t)e * (GLU ? 2 : 1) * N * K;
   const int steps = (K + 31) / 32;
-  const int kbeg = 32 * (steps * wave / 4), kend = 32 * (steps * (wave + 1) / 4);
+  const int kbeg = __builtin_amdgcn_readfirstlane(32 * (steps * wave / 4));
+  const int kend = __builtin_amdgcn_readfirstlane(32 * (steps * (wave + 1) / 4));
   const int pair = rows.row_pair ? rows.row_pair[r0 + r] : 0;    // asked for before the matrix, needed behind it
   const bf16_t* wrow[4];                                // rows past N: another row, whose products are not stored
 #pragma unroll
@@ -591,15 +592,20 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   };
   load_rows(0, kbeg);
   for (int k0 = kbeg; k0 < kend; k0 += 64 * DEPTH) {
-    load_matrix(1, k0 + 32 * DEPTH);
-    load_rows(1, k0 + 32 * DEPTH);
+    const bool second = k0 + 32 * DEPTH < kend, third = k0 + 64 * DEPTH < kend;   // nothing is asked for past the wave's k
+    if (second) {
+      load_matrix(1, k0 + 32 * DEPTH);
+      load_rows(1, k0 + 32 * DEPTH);
+    }
     __builtin_amdgcn_sched_barrier(0);
     multiply(0);
     __builtin_amdgcn_sched_barrier(0);
-    load_matrix(0, k0 + 64 * DEPTH);
-    load_rows(0, k0 + 64 * DEPTH);
+    if (third) {
+      load_matrix(0, k0 + 64 * DEPTH);
+      load_rows(0, k0 + 64 * DEPTH);
+    }
     __builtin_amdgcn_sched_barrier(0);
-    multiply(1);
+    if (second) multiply(1);
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
