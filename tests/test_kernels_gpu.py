@@ -682,6 +682,32 @@ def test_float32_attention_of_sequences_that_bring_no_token(counts):
         assert torch.equal(step(list(range(B)), ws), want)
 
 
+# a table so wide that its partial rows go through in turns: of two and one sequences, of one kv head, of three and two
+@pytest.mark.parametrize("nh,nkv,B,width", [(20, 5, 3, 20000), (8, 2, 2, 128000), (40, 5, 1, 38000)])
+def test_float32_attention_of_single_tokens_in_turns(nh, nkv, B, width):
+    """A page table's width decides the scratch, not the sequences' lengths: the bits of a narrow table, within 256 MB
+    or one kv head's rows."""
+    from transformer_amd import kernels
+    from transformer_amd.parts.linear import Workspace
+    own = np.random.default_rng([nh, B])
+    dh = 64
+    kc, vc = dev(own.normal(size=(4 * B, nkv, 64, dh))), dev(own.normal(size=(4 * B, nkv, dh, 64)))
+    narrow = own.permutation(4 * B).reshape(B, 4)
+    wide = np.zeros((B, width), dtype=np.int32)
+    wide[:, :4] = narrow
+    pos = dev(own.integers(3, 256, B), torch.int32)
+    q, cu = dev(own.normal(size=(B, nh * dh))), dev(np.arange(B + 1), torch.int32)
+    got = []
+    for table in (narrow, wide):
+        ws = Workspace(DEV)
+        out = torch.full((B, nh * dh), float("nan"), device=DEV)
+        kernels.attention_generic(q, out, kc, vc, dev(table, torch.int32), cu, pos, 1, nh, nkv, dh, 0.125, None, ws)
+        parts = ws._bufs["attention.f32_parts", torch.float32].numel()
+        assert parts <= max(1 << 26, nh // nkv * table.shape[1] * (dh + 2))
+        got.append(out)
+    assert torch.isfinite(got[0]).all() and torch.equal(got[0], got[1])
+
+
 # rows at which the kernel or its tile changes, k inside and at the ends of blocks, segments and rounds of
 # segments, workgroups' tiles that end inside the matrix (tiles of 64 and of 128), lengths up to which waves end
 # where k does and from which they don't, the longest k whose single rows go to tiles

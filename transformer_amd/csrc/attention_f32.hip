@@ -24,9 +24,12 @@ struct F32Attention {
   const float *k, *v;          // one layer: [pages][nkv][64][dh], [pages][nkv][dv][64]
   const int *table, *cu_q, *pos0;
   const float *sink, *gate;
-  float* parts;                // single tokens: [B][nh][max_blocks][dv] sums, then [B][nh][max_blocks][2] maxima and sums
+  // single tokens: [seqs][heads][max_blocks][dv] sums, then [seqs][heads][max_blocks][2] maxima and sums, of the sequences
+  // from b0 on and the heads of the kv heads from kv0 on
+  float* parts;
   int q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window, sink_mode, gate_stride, gate_dv, keep, chunk;
   float scale, softcap;
+  int b0, kv0, seqs, heads;
 };
 
 // what a row sees: keys start .. end - 1 and the first `keep`
@@ -253,7 +256,8 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
 // heads over 4 kv heads: 14.3 us and 4.7 to join (279 by one workgroup per sequence and kv head).
 template <int NB, bool EXACT>
 __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
-  const int group = p.nh / p.nkv, tiles = (group + 15) / 16, b = blockIdx.z, kvh = blockIdx.y / tiles, h0 = blockIdx.y % tiles * 16;
+  const int group = p.nh / p.nkv, tiles = (group + 15) / 16, b = p.b0 + blockIdx.z;
+  const int kvh = p.kv0 + blockIdx.y / tiles, h0 = blockIdx.y % tiles * 16;
   const int lane = threadIdx.x % TA_WAVE, r = lane % 16, kb = lane / 16;
   const int page = blockIdx.x * 4 + threadIdx.x / TA_WAVE;
   const int end = p.pos0[b] + 1;
@@ -286,13 +290,13 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
   page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
   page_values<NB, EXACT>(s, nvb, end - page * 64, kb, [&](int t, int d) { return vf[t][d]; }, o);
   if (!ok) return;
-  const size_t unit = ((size_t)b * p.nh + head) * p.max_blocks + page;
+  const size_t unit = ((size_t)blockIdx.z * p.heads + head - p.kv0 * group) * p.max_blocks + page;
   float* sums = p.parts + unit * p.dv;
 #pragma unroll
   for (int d = 0; d < NB; ++d)
     if (EXACT || d < nvb) *reinterpret_cast<f32x4*>(sums + 16 * d + 4 * kb) = o[d];
   if (kb == 0) {
-    float* ml = p.parts + (size_t)gridDim.z * p.nh * p.max_blocks * p.dv + unit * 2;
+    float* ml = p.parts + (size_t)p.seqs * p.heads * p.max_blocks * p.dv + unit * 2;
     ml[0] = m;
     ml[1] = l;
   }
@@ -300,13 +304,13 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
 
 // The pages of a single token's row joined in ascending order, eight asked for at a time; a thread a column.
 __global__ __launch_bounds__(128) void attn_f32_join_kernel(F32Attention p) {
-  const int head = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+  const int head = p.kv0 * (p.nh / p.nkv) + blockIdx.x, b = p.b0 + blockIdx.y, d = threadIdx.x;
   if (p.cu_q[b + 1] == p.cu_q[b]) return;
   const int end = p.pos0[b] + 1;
   const Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
-  const size_t unit = ((size_t)b * p.nh + head) * p.max_blocks;
+  const size_t unit = ((size_t)blockIdx.y * p.heads + blockIdx.x) * p.max_blocks;
   const float* sums = p.parts + unit * p.dv;
-  const float* ml = p.parts + (size_t)gridDim.y * p.nh * p.max_blocks * p.dv + unit * 2;
+  const float* ml = p.parts + (size_t)p.seqs * p.heads * p.max_blocks * p.dv + unit * 2;
   const int pages = (end + 63) / 64 < p.max_blocks ? (end + 63) / 64 : p.max_blocks;
   float M = -INFINITY, L = 0.f, O = 0.f;
   for (int p0 = 0; p0 < pages; p0 += 8) {
@@ -335,13 +339,31 @@ __global__ __launch_bounds__(128) void attn_f32_join_kernel(F32Attention p) {
   p.out[token * p.out_stride + (size_t)head * p.dv + d] = gated(p, O * rescale * inv, head, token, d);
 }
 
+// Single tokens go through in turns whose partial rows take 256 MB at most (or one kv head's, if that is more): whole
+// sequences while one fits, else some kv heads of one sequence. (The prompts' kernel, which had such steps before, walks
+// a row's pages one after the other: 8 sequences of 120,000 keys, 32 heads over 8, 11.0 ms, 2.9 in turns; 16 of 60,000
+// 5.5 and 2.6.)
+#define F32_PARTS (1ll << 26)
+static void f32_turn(int batch, int nh, int nkv, int max_blocks, int dv, int& seqs, int& kvs) {
+  const long long unit = (long long)(nh / nkv) * max_blocks * (dv + 2), fit = F32_PARTS / unit > 1 ? F32_PARTS / unit : 1;
+  kvs = fit < nkv ? (int)fit : nkv;
+  seqs = fit / nkv < 1 ? 1 : fit / nkv < batch ? (int)(fit / nkv) : batch;
+}
+
 // Floats of scratch that ta_attention_f32 wants for a step of single tokens.
+extern "C" long long ta_attention_f32_turn_scratch(int batch, int nh, int nkv, int max_blocks, int dv) {
+  if (batch <= 0 || nkv <= 0 || nh < nkv || max_blocks <= 0 || dv <= 0) return 0;
+  int seqs, kvs;
+  f32_turn(batch, nh, nkv, max_blocks, dv, seqs, kvs);
+  return (long long)seqs * kvs * (nh / nkv) * max_blocks * (dv + 2);
+}
+// The most that it wants, whatever the kv heads.
 extern "C" long long ta_attention_f32_scratch(int batch, int nh, int max_blocks, int dv) {
   return (long long)batch * nh * max_blocks * (dv + 2);
 }
 
 // As ta_attention_generic_sink, float32, dh and dv multiples of 16 up to 128, rows that start on 16 bytes. parts:
-// scratch of ta_attention_f32_scratch floats for steps in which every sequence brings one token or none (max_qlen 1), or
+// scratch of ta_attention_f32_turn_scratch floats for steps in which every sequence brings one token or none (max_qlen 1), or
 // null: the kernel for prompts then serves these too, with the same bits.
 extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride, void* out, int out_stride,
                                 const void* kcache, const void* vcache, const int* block_table, int max_blocks,
@@ -364,9 +386,9 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
   TA_REQUIRE(max_blocks > 0 && batch <= 65535 && (long long)nkv * ((nh / nkv + 15) / 16) <= 65535,
              "ta_attention_f32: grid of %d sequences, %d kv heads, %d pages", batch, nkv, max_blocks);
   if (batch == 0 || max_qlen == 0) return 0;
-  const F32Attention p = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, cu_q, pos0,
+  F32Attention p = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, cu_q, pos0,
                           sink, (const float*)gate, parts, q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window,
-                          sink_mode, gate_stride, gate_dv, keep, chunk, scale, softcap};
+                          sink_mode, gate_stride, gate_dv, keep, chunk, scale, softcap, 0, 0, 0, 0};
   const int group = nh / nkv, most = dh > dv ? dh : dv;
 #define PICK(kernel, grid)                                                        \
   do {                                                                            \
@@ -376,8 +398,15 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
     else kernel<8, false><<<grid, 256, 0, stream>>>(p);                           \
   } while (0)
   if (max_qlen == 1 && parts != nullptr) {
-    PICK(attn_f32_pages_kernel, dim3((max_blocks + 3) / 4, nkv * ((group + 15) / 16), batch));
-    attn_f32_join_kernel<<<dim3(nh, batch), 128, 0, stream>>>(p);
+    int kvs;
+    f32_turn(batch, nh, nkv, max_blocks, dv, p.seqs, kvs);
+    p.heads = kvs * group;
+    for (p.b0 = 0; p.b0 < batch; p.b0 += p.seqs)
+      for (p.kv0 = 0; p.kv0 < nkv; p.kv0 += kvs) {
+        const int bs = batch - p.b0 < p.seqs ? batch - p.b0 : p.seqs, ks = nkv - p.kv0 < kvs ? nkv - p.kv0 : kvs;
+        PICK(attn_f32_pages_kernel, dim3((max_blocks + 3) / 4, ks * ((group + 15) / 16), bs));
+        attn_f32_join_kernel<<<dim3(ks * group, bs), 128, 0, stream>>>(p);
+      }
   } else {
     PICK(attn_f32_rows_kernel, dim3((unsigned)(((long long)max_qlen * group + 63) / 64), nkv, batch));
   }

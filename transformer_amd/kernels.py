@@ -257,19 +257,14 @@ def f32_attention_takes(q, out, kcache, vcache, key_dim: int, value_dim: int) ->
         and all(t.data_ptr() % 16 == 0 for t in (q, out, kcache, vcache))
 
 
-# the most partial rows that a float32 step of single tokens leaves in its workspace (floats)
-_F32_PARTS = 1 << 26
-
-
 def _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max_qlen, num_heads, num_kv_heads, key_dim,
                    value_dim, scale, window, ws, cap=0.0, mode=0, sink=None, gate=None, gs=0, gd=0, keep=0, chunk=0):
     B, parts = pos0.numel(), None
     if max_qlen == 1 and ws is not None:
-        need = library().ta_attention_f32_scratch
+        need = library().ta_attention_f32_turn_scratch
         need.restype = c_longlong
-        floats = need(c_int(B), c_int(num_heads), c_int(block_table.shape[1]), c_int(value_dim))
-        if floats <= _F32_PARTS:
-            parts = ws.take("attention.f32_parts", (floats,), torch.float32)
+        floats = need(c_int(B), c_int(num_heads), c_int(num_kv_heads), c_int(block_table.shape[1]), c_int(value_dim))
+        parts = ws.take("attention.f32_parts", (floats,), torch.float32)     # 256 MB at most, or one kv head's rows
     _check(library().ta_attention_f32(
         _stream(), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache), _ptr(vcache), _ptr(block_table),
         c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0), c_int(B), c_int(max_qlen), c_int(num_heads),
