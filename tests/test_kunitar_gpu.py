@@ -241,6 +241,34 @@ def test_experts_blocks_through_lds_equal_operands_from_memory(geom):
             assert torch.equal(got, want), (out_dtype, act)
 
 
+@pytest.mark.parametrize("corrected", [False, True])
+def test_a_token_of_nan_scores_leaves_the_others_routing_alone(corrected):
+    """Tokens of one launch share its LDS: the choices and weights of the tokens around one whose scores are NaN are
+    those that they have alone. The neighbour's last choice is the last expert, whose score stands next to it."""
+    from transformer_amd import kernels
+    own = np.random.default_rng(7)
+    E, top, nt = 24, 24, 15
+    z = own.standard_normal((nt, E)).astype(np.float32)
+    z[:, E - 1] = -4.0
+    z[1::2] = np.nan
+    corr = _t(0.1 * own.standard_normal(E).astype(np.float32)) if corrected else None
+    rows = lambda n: kernels.moe_max_rows(n * top, E)
+
+    def route(zz):
+        n = len(zz)
+        chosen, weight = torch.empty(n, top, dtype=torch.int32, device=DEV), torch.empty(n, top, device=DEV)
+        i32 = lambda m: torch.empty(m, dtype=torch.int32, device=DEV)
+        kernels.moe_route_plan(_t(zz), E, top, chosen, weight, E, i32(rows(n)), i32(rows(n) // 16), i32(n * top), "sigmoid",
+                               False, correction=corr)
+        return chosen, weight
+
+    chosen, weight = route(z)
+    for t in range(0, nt, 2):
+        c, w = route(z[t:t + 1])
+        assert torch.equal(c[0], chosen[t]) and torch.equal(w[0], weight[t]) and torch.isfinite(w).all()
+    assert (chosen[1::2] >= E).all()
+
+
 # experts, router outputs, top, tokens, N, K: one token, the most that are routed in one launch and one more, columns that
 # end inside the 32 or 64 of a workgroup, k inside and behind a wave's share
 @pytest.mark.parametrize("geom", [(5, 5, 3, 1, 40, 72), (64, 72, 6, 16, 33, 200), (8, 8, 2, 17, 96, 1032), (3, 4, 4, 6, 130, 2056)])

@@ -107,14 +107,15 @@ __device__ void moe_route_token(const MoeRoute& p, size_t t, float* sc, int* cho
       const int oa = __shfl_xor(at, o, TA_WAVE);
       if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
     }
-    const float w = correction ? plain[at] : mode == 0 ? best : best / sum;
+    // scores of a token that are all NaN choose nobody: such a token touches no LDS but its own
+    const float w = correction ? (at < E ? plain[at] : 0.f) : mode == 0 ? best : best / sum;
     if (lane == 0) {
       chosen[j] = at;
       weight[j] = p.renorm ? w : w * p.factor;
     }
     total += w;
     moe_wave_sync();
-    if (lane == 0) sc[at] = -INFINITY;
+    if (lane == 0 && at < E) sc[at] = -INFINITY;
     moe_wave_sync();
   }
   if (p.renorm) {
