@@ -110,8 +110,9 @@ def _model_and_plain(dtype):
 
 
 def test_float32_at_the_headline_width_equals_the_plain_model():
-    """Sums of 4,096 to 14,336 float32 terms in ascending order against float64: an error of
-    about sqrt(K) * 2^-24 of the terms' size per product (1e-5 on logits whose spread is 1.3);
+    """Sums of 4,096 to 14,336 float32 terms (segments of 256, whose sums are added in ascending
+    order; blocks of 16 inside them in an order of their own) against float64: an error below
+    sqrt(K) * 2^-24 of the terms' size per product (1e-5 on logits whose spread is 1.3);
     the bound below leaves a factor of ten. A wrong weight row, head or position moves the
     logits by 1e-2 or more."""
     import torch

@@ -311,9 +311,19 @@ F32_SHAPES = [
     (20, 1, 96, 112, [10, 190], {"chunk": 50, "gate": True}),
     (6, 3, 16, 128, [130, 512], {"window": 64}),
 ]
+# the same with many tokens of a sequence: several workgroups of 64 rows, waves of one workgroup that see other pages
+# than their neighbours, a window and kept keys with whole pages between them, chunks that end inside a workgroup's rows
+F32_TAILS = [
+    (8, 2, 128, 128, [300, 700], {"window": 100, "tail": 150}),
+    (4, 4, 64, 64, [200, 520], {"window": 70, "keep_first": 5, "sink": "unit", "tail": 130}),
+    (8, 2, 128, 128, [333, 130], {"chunk": 100, "tail": 90}),
+    (5, 1, 64, 64, [260], {"chunk": 48, "gate": True, "softcap": 3.0, "tail": 100}),
+    (16, 2, 128, 128, [190], {"tail": 75}),
+]
 
 
-@pytest.mark.parametrize("shape", F32_SHAPES, ids=[f"h{s[0]}kv{s[1]}k{s[2]}v{s[3]}" for s in F32_SHAPES])
+@pytest.mark.parametrize("shape", F32_SHAPES + F32_TAILS,
+                         ids=[f"h{s[0]}kv{s[1]}k{s[2]}v{s[3]}t{s[5].get('tail', 3)}" for s in F32_SHAPES + F32_TAILS])
 def test_float32_attention_page_by_page(shape):
     """A sequence's last tokens, as a prompt that continues it and one by one with and without scratch: the same
     bits, and the plain attention's numbers. Cache places behind the end hold NaN."""
@@ -321,7 +331,7 @@ def test_float32_attention_page_by_page(shape):
     from transformer_amd.parts.linear import Workspace
     nh, nkv, dk, dv, lengths, opt = shape
     own = np.random.default_rng([nh, dk, dv])
-    group, B, tail = nh // nkv, len(lengths), 3
+    group, B, tail = nh // nkv, len(lengths), opt.get("tail", 3)
     tails = [min(tail, n) for n in lengths]
     need = [-(-n // 64) for n in lengths]
     order = own.permutation(sum(need) + 2)
@@ -351,11 +361,14 @@ def test_float32_attention_page_by_page(shape):
 
     start = np.concatenate([[0], np.cumsum(tails)])
     whole = step(list(range(nt)), tails, [n - t for n, t in zip(lengths, tails)], None)
-    # the last token of each, its pages in waves of their own, and by the prompts' kernel
-    rows = [int(start[b + 1]) - 1 for b in range(B)]
-    for ws in (Workspace(DEV), None):
-        alone = step(rows, [1] * B, [n - 1 for n in lengths], ws)
-        assert torch.equal(alone, whole[rows])
+    # single tokens of each (the last and, of many, some of other waves and workgroups), their pages in waves of their
+    # own, and by the prompts' kernel
+    for back in {0, 1, 3, 14, 17, 40, 66, tail - 1} if tail > 3 else {0}:
+        taken = [max(t - 1 - back, 0) for t in tails]
+        rows = [int(start[b]) + taken[b] for b in range(B)]
+        for ws in (Workspace(DEV), None):
+            alone = step(rows, [1] * B, [n - t + i for n, t, i in zip(lengths, tails, taken)], ws)
+            assert torch.equal(alone, whole[rows])
     for b, n in enumerate(lengths):
         for i in range(tails[b]):
             at, row = n - tails[b] + i, int(start[b]) + i
