@@ -173,8 +173,8 @@ def main(argv: Optional[Sequence[str]] = None) -> int:
                    help="the engine's type; default: what config.json's torch_dtype says (float32 stays "
                         "float32, everything else computes in bfloat16)")
     g.add_argument("--backend", choices=["hip", "ref"], default="hip",
-                   help="ref: the plain float32 kernels of the device (one sum per output element in "
-                        "ascending order, attention without matrix cores), whatever --dtype says; the "
+                   help="ref: the plain float32 kernels of the device (sums in 32 bits in an order that does "
+                        "not depend on the batch), whatever --dtype says; the "
                         "role of the reference's CPU back-end (models/llama/common-cpu/src/lib.rs:48-67)")
     g.add_argument("--seed", type=int, default=0)
     g.add_argument("--timers", action="store_true",

@@ -161,8 +161,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
 // eight lanes that are served together meet no bank twice. float32 operands go from memory to LDS without passing
 // through registers (a wave's 64 pieces land side by side, so the permutation is in the addresses they are read
 // from); other types are converted on the way. Half h of a wave multiplies pieces h and h + 2 of a block's four,
-// element by element: the order above. 1,021 x 16,384 x 2,048: 535 us (128 TFLOP/s; 630 through registers,
-// 1,880 on the vector ALU); the instruction alone reaches 154. With the barrier at a step's end instead of in its
+// element by element: the order above. 1,021 x 16,384 x 2,048: 535 us back to back (128 TFLOP/s; 566 in a prompt's
+// trace; 630 through registers, 1,880 on the vector ALU); the instruction alone reaches 154. With the barrier at a step's end instead of in its
 // middle 553, and 1,021 x 3,072 x 2,048 141 where it now takes 130.
 template <typename T, typename TW, typename TC, int TT, bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict__ A, int lda,

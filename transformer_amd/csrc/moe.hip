@@ -931,8 +931,8 @@ static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A,
 
 // Whether the experts' product of this many ordered rows takes the form for few tiles (bfloat16). Below the line the
 // blocks of the other form leave CUs idle, above it this one reads an expert's matrix once for every tile. Few against
-// LDS: 124 tiles of 1,024 x 2,048 48 us against 87, 124 of 2,048 x 1,024 48 against 48, 90 of 2,816 x 4,096 305 against
-// 305, 75 of 4,096 x 1,408 168 against 138, 255 of 2,048 x 1,024 82 against 45.
+// LDS, us (tiles, in brackets those with rows): 66 (51) of 4,096 x 1,408 139 and 139, 83 (72) 200 and 246; 81 (64) of 2,816
+// x 4,096 308 and 310, 105 (72) 368 and 333; 80 (66) of 2,048 x 1,024 52 and 40, 255 (239) 151 and 59.
 extern "C" int ta_moe_few_rows(int max_rows, int N, int K) {
   return K % 8 == 0 && (long long)(max_rows / MOE_TILE) * ((N + 255) / 256) < 1024;
 }

@@ -19,8 +19,8 @@ __device__ __forceinline__ uint32_t order_key(float l) {
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 // floor(2^40 * exp((l - m) / T)) from the hardware's exp2 and two 32-bit conversions: the
-// library's expf and a float-to-64-bit conversion are some fifty instructions, and a row of
-// 128 K tokens on one CU is bound by exactly these
+// library's expf and a float-to-64-bit conversion are some fifty instructions, and sampling is
+// bound by what it does for each token, whether a row is one workgroup's or dealt out in parts
 __device__ __forceinline__ u64 fixed_mass(float l, float m, float inv_t) {
   const float w = __builtin_amdgcn_exp2f((l - m) * inv_t * 1.44269504088896341f);   // in [0, 1]
   const float upper = w * 1048576.0f;                    // 2^20; exact, as is what follows

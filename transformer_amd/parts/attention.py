@@ -185,8 +185,9 @@ class NormedAttention(Part):
     # bfloat16 with a key width the matrix-core kernels take and values no wider than the keys:
     # the cache keeps value rows of the keys' width (the rest zero), so that the kernels for
     # equal widths serve prompts and single tokens, and the output projection reads the heads'
-    # rows through a copy of its matrix with zero columns in the same places. Everything else
-    # (float32, other widths) runs the vector-ALU kernel on values of their own width.
+    # rows through a copy of its matrix with zero columns in the same places. Everything else keeps
+    # values of their own width: float32 on the 32-bit matrix instructions where the widths allow
+    # (``kernels.f32_attention_takes``), the rest on the vector ALU.
     def _on_matrix_cores(self) -> bool:
         return (self.dtype == torch.bfloat16 and self.dk % 32 == 0 and 32 <= self.dk <= 256
                 and self.dv <= self.dk and self.width % 8 == 0)     # rows of [q | k | v] start on 16 bytes
@@ -331,7 +332,8 @@ class SinkAttention(Part):
     # serve prompts and single tokens, and the output projection reads the heads' rows through a copy
     # of its matrix with zero columns in the same places (as ``NormedAttention`` does). This depends on
     # the type and the two widths alone, which a layer shares with the readers of its cache. Everything
-    # else (float32, other widths) runs the vector-ALU kernel on values of their own width.
+    # else keeps values of their own width: float32 on the 32-bit matrix instructions where the widths
+    # allow (``kernels.f32_attention_takes``), the rest on the vector ALU.
     def _pads_values(self) -> bool:
         return self.dtype == torch.bfloat16 and self.dk % 32 == 0 and 32 <= self.dk <= 256 and self.dv <= self.dk
 
