@@ -1110,6 +1110,10 @@ def test_sample_in_parts_of_a_row_chooses_as_the_whole_row(vocab):
         kernels.sample(aligned, dev(u), a, T, k, p_, scratch)
         kernels.sample(shifted, dev(u), b, T, k, p_)
         assert torch.equal(a, b), (T, k, p_, (a != b).nonzero().flatten().tolist())
+    for short in (scratch[:8], scratch[:scratch.numel() - 8], scratch[:0]):
+        with pytest.raises(kernels.KernelError, match="are needed"):
+            kernels.sample(aligned, dev(u), a, 0.8, 40, 0.95, short)
+        kernels.sample(shifted, dev(u), b, 0.8, 40, 0.95, short)      # rows that take none
 
 
 def test_sample_frequencies():

@@ -1537,10 +1537,11 @@ extern "C" long long ta_sample_scratch_for(int n, int vocab, int top_k, float to
   return n > 0 && vocab > 0 && in_parts(n, vocab, top_k, top_p) ? ta_sample_scratch(n, vocab) : 0;
 }
 
-// scratch: ta_sample_scratch bytes on an 8-byte boundary, or null: one workgroup takes a row then.
+// scratch: scratch_bytes on an 8-byte boundary, ta_sample_scratch_for of them or more, or null: one workgroup takes a
+// row then.
 extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
                                float temperature, int top_k, float top_p, const float* uniform,
-                               int* out, void* scratch) {
+                               int* out, void* scratch, long long scratch_bytes) {
   TA_REQUIRE(n >= 0 && vocab > 0 && ld >= vocab, "ta_sample: bad sizes n=%d vocab=%d ld=%lld", n, vocab, ld);
   TA_REQUIRE(temperature > 0.f, "ta_sample: temperature %g must be > 0 (0 means argmax)", (double)temperature);
   TA_REQUIRE(top_k >= 1, "ta_sample: top_k %d < 1", top_k);
@@ -1553,6 +1554,8 @@ extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long lon
   } else if (scratch == nullptr || !in_parts(n, vocab, top_k, top_p)) {
     sample_rows_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
   } else {
+    TA_REQUIRE(scratch_bytes >= ta_sample_scratch(n, vocab), "ta_sample: %lld bytes of scratch, %lld are needed", scratch_bytes,
+               ta_sample_scratch(n, vocab));
     const int parts = sample_parts(vocab), cut = top_k < vocab || top_p < 1.0f;
     PartRecord* rec = (PartRecord*)scratch;
     const int turn = rows_at_a_time(vocab);
@@ -1572,5 +1575,5 @@ extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long lon
 // Without scratch: one workgroup a row.
 extern "C" int ta_sample(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
                          float temperature, int top_k, float top_p, const float* uniform, int* out) {
-  return ta_sample_parts(stream, logits, ld, n, vocab, temperature, top_k, top_p, uniform, out, nullptr);
+  return ta_sample_parts(stream, logits, ld, n, vocab, temperature, top_k, top_p, uniform, out, nullptr, 0);
 }

@@ -849,17 +849,18 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, tempe
     if out.numel() != n or uniform.numel() != n:
         raise KernelError("sample: out and uniform must hold one entry per row")
     vocab = logits.shape[1]
-    walks = logits.data_ptr() % 16 or ld % 4           # rows off 16 bytes: a workgroup walks one token at a time
-    need = 0 if walks else sample_scratch(n, vocab, top_k, float(top_p))
-    if scratch is None:
+    if scratch is not None:
+        _dev(scratch, "scratch", torch.uint8)          # its size is checked with the launch
+    if scratch is None or scratch.numel() == 0:
+        walks = logits.data_ptr() % 16 or ld % 4       # rows off 16 bytes: a workgroup walks one token at a time
+        need = 0 if walks else sample_scratch(n, vocab, top_k, float(top_p))
+        if scratch is not None and need:
+            raise KernelError(f"sample: no bytes of scratch, {need} are needed")
         scratch = torch.empty(need, dtype=torch.uint8, device=logits.device) if need else None
-    else:
-        _dev(scratch, "scratch", torch.uint8)
-        if scratch.numel() < need:
-            raise KernelError(f"sample: {scratch.numel()} bytes of scratch, {need} are needed")
     _check(library().ta_sample_parts(_stream(), _ptr(logits), c_longlong(ld), c_int(n), c_int(vocab),
                                      c_float(temperature), c_int(min(int(top_k), vocab)),
-                                     c_float(top_p), _ptr(uniform), _ptr(out), _ptr(scratch)))
+                                     c_float(top_p), _ptr(uniform), _ptr(out), _ptr(scratch),
+                                     c_longlong(0 if scratch is None else scratch.numel())))
     return out
 
 
