@@ -187,6 +187,49 @@ def test_routed_feed_forward_pieces(dtype, geom):
         _close(_np(delta), want, dtype, f"{nt} tokens")
 
 
+# one token, the most that are routed and ordered in one launch, the most whose products divide k, a prompt through LDS
+@pytest.mark.parametrize("nt,few", [(1, True), (16, True), (1980, True), (2011, False)])
+def test_routed_experts_count_token_by_token(nt, few):
+    """The routed experts alone, with matrices of the usual spread, so that nothing stands beside them in the sum: every
+    token within what the engine's type gives, and far outside it where the plain function leaves an expert out.
+
+    Rounded to bfloat16 are a pair's weighted row (2^-9 of each term at most, which the square behind the first product
+    doubles) and the squares (2^-9 again): 3 * 2^-9 of a token's result in the 2-norm, and 4 * 2^-9 is allowed. In 64 bits
+    with these two roundings: 0.0041 at the worst of 2,011 tokens."""
+    from transformer_amd import kernels
+    from transformer_amd.config.spec import RoutedMLPSpec
+    from transformer_amd.parts.base import build_part
+    from transformer_amd.parts.linear import Workspace
+    E, top, ff, d = 8, 2, 1024, 1024
+    rng = np.random.default_rng(nt)
+    router = _bf(2 * rng.standard_normal((E, d)) / np.sqrt(d))
+    up, down = _bf(rng.standard_normal((E, ff, d)) / np.sqrt(d)), _bf(rng.standard_normal((E, d, ff)) / np.sqrt(ff))
+    part = build_part(RoutedMLPSpec(hidden=d, experts=E, top=top, intermediate=ff, shared_intermediate=None), torch.bfloat16, DEV)
+    bound = {"router.weight": router, "experts.up.weight": up.reshape(E * ff, d), "experts.down.weight": down.reshape(E * d, ff)}
+    part.bind({k: _t(v, torch.bfloat16) for k, v in bound.items()})
+    rows = kernels.moe_max_rows(nt * top, E)
+    assert bool(kernels.library().ta_moe_few_rows(rows, ff, d)) == few and bool(kernels.library().ta_moe_few_rows(rows, d, ff)) == few
+
+    class Ctx:
+        ws = Workspace(DEV)
+    h = _bf(rng.standard_normal((nt, d)))
+    got = _np(part.run(_t(h, torch.bfloat16), Ctx)[0])
+    chosen = _np(Ctx.ws.take("moe.chosen", (nt, top), torch.int32)).astype(int)
+    weight = P.sigmoid(h @ router.T)
+    best = np.sort(weight, axis=1)[:, -top:]
+    assert (np.sort(np.take_along_axis(weight, chosen, 1), axis=1) >= best - 1e-5).all()      # but for close calls
+
+    want, off = np.zeros((nt, d)), np.zeros(nt)
+    for e in range(E):
+        who = np.nonzero((chosen == e).any(axis=1))[0]
+        y = P.relu_squared((weight[who, e:e + 1] * h[who]) @ up[e].T) @ down[e].T
+        want[who] += y
+        off[who] = np.maximum(off[who], np.linalg.norm(y, axis=1))
+    norm, error = np.linalg.norm(want, axis=1), np.linalg.norm(got - want, axis=1)
+    assert (error <= 2.0 ** -7 * norm).all()
+    assert (off > 8 * 2.0 ** -7 * norm).all()          # without its larger expert no token would pass
+
+
 @pytest.mark.parametrize("form", ["split_k", "direct", "lds"])
 @pytest.mark.parametrize("geom", [(5, 3, 40, 72, 700), (3, 1, 264, 200, 300), (16, 2, 130, 136, 90), (2, 2, 64, 64, 5)])
 def test_experts_products_in_every_form(form, geom):
