@@ -668,6 +668,17 @@ def test_gemm_simple(mnk):
     assert np.abs(f64(o2) - ab @ wb.T).max() < 1e-6 * K ** 0.5 * 8
 
 
+def test_gemm_simple_over_more_than_two_to_the_thirty():
+    """A row of 2^30 and some elements with itself: whole numbers at both ends, around 2^30 and at the very end."""
+    from transformer_amd import kernels
+    K = 2 ** 30 + 2052
+    a = torch.zeros(1, K, dtype=torch.bfloat16, device=DEV)
+    a[0, [0, 5, 2 ** 30 - 1, 2 ** 30, 2 ** 30 + 7, K - 1]] = dev([1, 2, 3, 4, 5, 6], torch.bfloat16)
+    out = torch.empty(1, 1, device=DEV)
+    kernels.gemm_simple(a, a, out)
+    assert out.item() == 91.0
+
+
 @pytest.mark.parametrize("counts", [[0, 1, 0, 1, 1, 0], [1, 0, 0], [0, 0, 1]])
 def test_float32_attention_of_sequences_that_bring_no_token(counts):
     """Single tokens beside sequences without one, first, last and in between: the rows of the others, the same as

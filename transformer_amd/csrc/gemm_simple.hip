@@ -368,7 +368,8 @@ extern "C" int ta_gemm_simple_batched(hipStream_t stream, int in_dtype, int w_dt
              "ta_gemm_simple: bad sizes M=%d N=%d K=%d batch=%d", M, N, K, batch);
   TA_REQUIRE(lda >= K && ldw >= K && ldc >= N, "ta_gemm_simple: leading dimensions too small");
   if (M == 0) return 0;
-  TA_REQUIRE((M + 63) / 64 <= 65535 && K <= (1 << 30), "ta_gemm_simple: M=%d K=%d too large for one launch", M, K);
+  // the few-rows kernel counts up to two rounds of 8 segments past k
+  TA_REQUIRE((M + 63) / 64 <= 65535 && K <= 2147483647 - 32 * SEG, "ta_gemm_simple: M=%d K=%d too large for one launch", M, K);
   // rows that start on 4 elements and hold whole pieces of 4
   auto aligned = [&](const void* p, int dtype, long long ld, long long stride) {
     return (uintptr_t)p % (dtype == TA_F32 ? 16 : 8) == 0 && ld % 4 == 0 && stride % 4 == 0;
