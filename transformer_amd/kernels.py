@@ -597,7 +597,8 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor
 def gemm_simple(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor,
                 bias: Optional[torch.Tensor] = None):
     """out = a @ w.T (+ bias), float32 accumulation in an order that depends on k's length alone
-    (segments of 256, whose sums are added in ascending order). a and w share a dtype, or a is bfloat16 and w float32 (a matrix that stays as its file stores it)."""
+    (segments of 256, whose sums are added in ascending order). a and w share a dtype, or a is
+    bfloat16 and w float32 (a matrix that stays as its file stores it)."""
     _dev(a, "a", contiguous=False)
     _dev(w, "w", None if (a.dtype == torch.bfloat16 and w.dtype == torch.float32) else a.dtype,
          contiguous=False)
