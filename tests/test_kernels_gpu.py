@@ -762,6 +762,39 @@ def test_gemm_simple_at_the_edges_of_its_tiles(mnk, types):
     assert torch.equal(both[0], got) and torch.equal(both[1], got)
 
 
+# float32, few rows, wide: the kernel that keeps its rows and walks along the columns, at the ends of its row and column tiles
+# (one more tile than workgroups, a last turn of few), segments and numbers of waves, beside sizes it leaves to the others.
+# The sums are held to the bound of the test above; the activation has the bits of the two kernels in turn.
+@pytest.mark.parametrize("mnk", [(1, 2560, 2048), (8, 5114, 516), (9, 5106, 1024), (16, 5120, 1028), (7, 2566, 2052),
+                                 (12, 8200, 2048), (16, 5106, 4096), (3, 2562, 3000), (8, 2552, 2048), (4, 2560, 4100)])
+def test_gemm_walk_along_the_columns(mnk):
+    from transformer_amd import kernels
+    M, N, K = mnk
+    own = np.random.default_rng([M, N, K, 1])
+    a, w, bias = own.normal(size=(M, K)), own.normal(size=(N, K)), own.normal(size=N)
+    ad, wd, bd = dev(a), dev(w), dev(bias)
+    out = torch.full((M, N + 3), 7.0, device=DEV)
+    kernels.gemm_simple(ad, wd, out[:, 1:N + 1], bd)
+    assert np.abs(f64(out[:, 1:N + 1]) - (f64(ad) @ f64(wd).T + f64(bd))).max() < 1e-6 * K ** 0.5 * 8
+    assert (out[:, 0] == 7).all() and (out[:, N + 1:] == 7).all()
+    many = torch.empty(70, N, device=DEV)        # the same bits among many rows, by the tiles' kernel
+    kernels.gemm_simple(ad[torch.arange(70, device=DEV) % M].contiguous(), wd, many, bd)
+    assert torch.equal(many[:M], out[:, 1:N + 1])
+    assert kernels.simple_glu_takes(ad, wd) == (512 < K <= 4096 and -(-N // (8 if M <= 8 else 16)) >= (640 if M <= 8 and K <= 1024 else 320))
+    if not kernels.simple_glu_takes(ad, wd):
+        with pytest.raises(kernels.KernelError):
+            kernels.gemm_simple_glu(ad, wd, torch.empty(M, N // 2, device=DEV))
+        return
+    for b in (None, bd):
+        both, two, one = torch.empty(M, N, device=DEV), torch.empty(M, N // 2, device=DEV), torch.full((M, N // 2 + 2), 7.0, device=DEV)
+        kernels.gemm_simple(ad, wd, both, b)
+        kernels.swiglu(both, two)
+        kernels.gemm_simple_glu(ad, wd, one[:, 1:N // 2 + 1], b)
+        assert torch.equal(one[:, 1:N // 2 + 1], two)
+        assert (one[:, 0] == 7).all() and (one[:, N // 2 + 1:] == 7).all()
+    assert not kernels.simple_glu_takes(ad[:, 1:], wd[:, 1:])    # rows off 16 bytes
+
+
 @pytest.mark.parametrize("mnk", [(1, 16, 128), (3, 130, 104), (8, 301, 1000), (16, 48, 4104), (5, 1000, 72),
                                  (8, 16 * 1024 + 5, 2048), (3, 16 * 2050, 1096), (16, 16 * 1030, 4096)])
 @pytest.mark.parametrize("waves", [0, 4, 8, 16])

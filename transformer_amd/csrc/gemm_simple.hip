@@ -12,8 +12,9 @@
 // which a lane that has read 4 consecutive k holds them: no operand is turned round.
 // Segments (instead of one chain over K) let few rows be split over waves; they also round less.
 //
-// Two kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_tiles: a tile
-// of 128 x 128 or 64 x 64 a workgroup, operands through LDS.
+// Three kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk: the same for
+// wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns.
+// gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS.
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -153,6 +154,123 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
     if (at < ROWS * COLS && m < M && n < N)
       C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
   }
+}
+
+// Up to 8 (PAIR) or 16 rows of A against a wide W over a k of at most one round of segments: every wave keeps its
+// segments of A in registers, the workgroup walks over tiles of 8 (16) columns, and the next tile's k are on their way
+// while the last ones of this are multiplied and added up. Bound by reading W. gemm_few_rows reads A again with every
+// tile, as many bytes as W at 8 rows, and its workgroups, which live for four chunks, start and end all the time:
+// 16,384 x 2,048 at 1 / 4 / 8 / 16 rows 31.6 / 33.5 / 40.2 / 39.0 us there, 25.4 / 25.7 / 26.6 / 28.9 here (5.2 TB/s
+// at 4 rows); 32,000 x 2,048 at 4 rows 67 and 48, 28,672 x 4,096 at 4 rows 116 and 85, 5,000 x 3,000 at 8 rows 27 and 20. One workgroup a CU with 8 KB of W a wave on their way is enough;
+// two or three a CU are up to 4 % slower. W passes the caches like any other read here: past them 3 % slower.
+// GLU: W holds gate rows, then up rows; a tile has half its columns of either and stores silu(gate) * up, with the bits
+// that the product and the activation's kernel give one after the other (a launch and two passes over its rows less).
+template <int WAVES, bool PAIR, bool GLU>
+__global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __restrict__ A, int lda,
+                                                               const float* __restrict__ W, int ldw,
+                                                               const float* __restrict__ bias, float* __restrict__ C,
+                                                               int ldc, int M, int N, int K, int tiles) {
+  constexpr int SIDE = PAIR ? 8 : 16;            // rows and columns of a tile
+  constexpr int TURN = PAIR ? 2 * WAVES : WAVES; // segments
+  constexpr int BC = WAVES > 8 ? 4 : 8;          // blocks per chunk: sixteen waves have 128 registers each
+  constexpr int CH = SEG / (BC * BLK);           // chunks per segment
+  constexpr int HALF = SIDE / 2;
+  static_assert(WAVES * 64 >= SIDE * SIDE, "a thread an output");
+  __shared__ __attribute__((aligned(16))) float part[2][TURN][SIDE * SIDE];
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  const int r = lane % 16, kb = lane / 16, col = r % SIDE;
+  const int seg = PAIR ? 2 * wave + r / 8 : wave, segs = (K + SEG - 1) / SEG;
+  const int k0 = seg * SEG + 4 * kb, n_out = GLU ? N / 2 : N;
+  // columns past the last read another row and feed outputs that are never stored
+  auto rows_of = [&](int tile) {
+    const int n = GLU ? HALF * tile + col % HALF : SIDE * tile + col;
+    return W + (size_t)((n < n_out ? n : n_out - 1) + (GLU && col >= HALF ? n_out : 0)) * ldw;
+  };
+  f32x4 a[CH][BC], w[2][BC];
+  auto load = [&](int c, const float* row) {
+#pragma unroll
+    for (int i = 0; i < BC; ++i) w[c % 2][i] = load_piece<float, true, false>(row, k0 + (c * BC + i) * BLK, K);
+  };
+  int tile = blockIdx.x;
+  const float* row = rows_of(tile);
+  load(0, row);
+  const float* arow = A + (size_t)(col < M ? col : 0) * lda;
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int i = 0; i < BC; ++i) a[c][i] = load_piece<float, true, false>(arow, k0 + (c * BC + i) * BLK, K);
+  const int m = threadIdx.x / SIDE, nn = threadIdx.x % SIDE;
+  for (int turn = 0; tile < tiles; tile += gridDim.x, turn ^= 1) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int c) {
+#pragma unroll
+      for (int i = 0; i < BC; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[c % 2][i][j], a[c][i][j], acc, 0, 0, 0);
+    };
+    static_assert(CH % 2 == 0, "a segment's chunks in two sets of registers in turn");
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      if (c + 1 < CH) {
+        load(c + 1, row);
+      } else {                                   // the next tile's first
+        row = rows_of(tile + (int)gridDim.x < tiles ? tile + (int)gridDim.x : tile);
+        load(0, row);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // a lane holds columns 4 kb .. + 3 of row r
+    auto* to = part[turn];
+    if (PAIR) {
+      if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[seg][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
+    } else {
+      *reinterpret_cast<f32x4*>(&to[seg][r * 16 + 4 * kb]) = acc;
+    }
+    // one barrier a tile: who comes to this half again has passed the other half's, behind which all have read this one
+    __syncthreads();
+    if (threadIdx.x < SIDE * SIDE) {
+      float total = 0.f;
+      for (int s = 0; s < segs; ++s) total += to[s][threadIdx.x];
+      const int n = (GLU ? HALF * tile + nn % HALF : SIDE * tile + nn);
+      if (bias && n < n_out) total += bias[n + (GLU && nn >= HALF ? n_out : 0)];
+      if (GLU) {
+        const float up = __shfl_xor(total, HALF, TA_WAVE);
+        if (m < M && nn < HALF && n < n_out) C[(size_t)m * ldc + n] = total / (1.0f + expf(-total)) * up;
+      } else if (m < M && n < n_out) {
+        C[(size_t)m * ldc + n] = total;
+      }
+    }
+  }
+}
+
+// Whether gemm_walk takes the product: as long a k as its waves' segments and a quarter more tiles than workgroups. With a tile a
+// workgroup it is gemm_few_rows with A read first (2,048 x 2,048 6.3 us there, 6.7 here; 2,304 x 4,096, 288 tiles, at one row
+// 14.8 and 15.2; 3,072 x 2,048, 384 tiles, at 4 rows 10.7 and 9.6). Up to k = 1,024 a workgroup of two waves has too little on its
+// way for a CU, so there are two of them on each. Below k = 512 the waves would have no segment.
+#define WALK_CUS 256
+static int walk_groups(int M, int K) { return M <= 8 && K <= 1024 ? 2 * WALK_CUS : WALK_CUS; }
+static bool walk_takes(int M, int N, int K) {
+  const int side = M <= 8 ? 8 : 16;
+  return M >= 1 && M <= 16 && K > 512 && K <= 4096 && (N + side - 1) / side >= walk_groups(M, K) * 5 / 4;
+}
+template <bool GLU>
+static void walk(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc,
+                 int M, int N, int K) {
+  const int side = M <= 8 ? 8 : 16, tiles = (N + side - 1) / side, grid = walk_groups(M, K);
+#define WALK(WAVES, PAIR) \
+  gemm_walk_kernel<WAVES, PAIR, GLU><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles)
+  if (M <= 8) {
+    if (K <= 1024) WALK(2, true);
+    else if (K <= 2048) WALK(4, true);
+    else WALK(8, true);
+  } else {
+    if (K <= 1024) WALK(4, false);
+    else if (K <= 2048) WALK(8, false);
+    else WALK(16, false);
+  }
+#undef WALK
 }
 
 // Many rows, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
@@ -338,6 +456,11 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
           A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
     return;
   }
+  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
+    if (batch == 1 && walk_takes(M, N, K)) {
+      walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
+      return;
+    }
 #define FEW_(WAVES, RT, BC, PAIR, SHORT)                                                                       \
   gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, SHORT, VEC>                                             \
       <<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch), WAVES * 64, 0, stream>>>( \
@@ -395,4 +518,20 @@ extern "C" int ta_gemm_simple(hipStream_t stream, int in_dtype, int w_dtype, int
                               void* C, int ldc, int M, int N, int K) {
   return ta_gemm_simple_batched(stream, in_dtype, w_dtype, out_dtype, A, lda, 0, W, ldw, 0, bias, C, ldc, 0,
                                 M, N, K, 1);
+}
+
+// Whether ta_gemm_simple_glu takes such a product (float32, rows on 16 bytes).
+extern "C" int ta_gemm_simple_glu_takes(int M, int di, int K) {
+  return di > 0 && di <= 1073741823 && K % 4 == 0 && walk_takes(M, 2 * di, K);
+}
+
+// C[M, di] = silu(A W[:di]^T + bias[:di]) * (A W[di:]^T + bias[di:]), W [2 di, K]: what ta_gemm_simple and ta_swiglu give one
+// after the other, bit for bit.
+extern "C" int ta_gemm_simple_glu(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias,
+                                  float* C, int ldc, int M, int di, int K) {
+  TA_REQUIRE(ta_gemm_simple_glu_takes(M, di, K), "ta_gemm_simple_glu: M=%d di=%d K=%d", M, di, K);
+  TA_REQUIRE(lda >= K && ldw >= K && ldc >= di && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
+             "ta_gemm_simple_glu: rows of %d, %d, %d floats or their start", lda, ldw, ldc);
+  walk<true>(stream, A, lda, W, ldw, bias, C, ldc, M, 2 * di, K);
+  return ta_check_launch("ta_gemm_simple_glu");
 }

@@ -618,6 +618,30 @@ def gemm_simple(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor,
     return out
 
 
+def simple_glu_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_simple_glu`` takes these operands: few float32 rows against a wide [gate rows | up rows]."""
+    return a.dtype == torch.float32 and w.dtype == torch.float32 and a.dim() == 2 and w.dim() == 2 and w.shape[0] % 2 == 0 \
+        and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 \
+        and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+        and bool(library().ta_gemm_simple_glu_takes(c_int(a.shape[0]), c_int(w.shape[0] // 2), c_int(a.shape[1])))
+
+
+def gemm_simple_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out [m, n] = silu(a @ w[:n].T) * (a @ w[n:].T) in float32, with the bits of ``gemm_simple`` and ``swiglu`` in turn."""
+    _dev(a, "a", torch.float32, contiguous=False); _dev(w, "w", torch.float32, contiguous=False)
+    _dev(out, "out", torch.float32, contiguous=False)
+    M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
+    if N % 2 or w.shape[1] != a.shape[1] or Mo != M or out.shape[1] != N // 2:
+        raise KernelError(f"gemm_simple_glu: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    if bias is not None:
+        _dev(bias, "bias", torch.float32)
+        if bias.numel() != N:
+            raise KernelError("gemm_simple_glu: bias must hold one entry per row of w")
+    _check(library().ta_gemm_simple_glu(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(bias), _ptr(out), c_int(ldc),
+                                        c_int(M), c_int(N // 2), c_int(a.shape[1])))
+    return out
+
+
 class RowScale:
     """Rows of activations that an RMS norm has not scaled yet: ``parts`` [tiles, 16] float32
     holds sums of squares per row (16 columns each), and the product that reads the rows

@@ -56,6 +56,9 @@ class SwiGLU(Part):
             # the 8B shape where the vendor library's product and the activation's kernel take 55
             kernels.gemm_mid(h, self.w["gate_up.weight"], act, swiglu=True, bias=self.w.get("gate_up.bias"),
                              limits=self.limits)
+        elif self.limits is None and kernels.simple_glu_takes(h, self.w["gate_up.weight"]):
+            # few float32 rows: the product applies the activation itself, with the same bits
+            kernels.gemm_simple_glu(h, self.w["gate_up.weight"], act, self.w.get("gate_up.bias"))
         else:
             gu = linear(h, self.w["gate_up.weight"],
                         ctx.ws.take("swiglu.gate_up", (nt, 2 * s.intermediate), self.dtype))
