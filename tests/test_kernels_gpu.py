@@ -706,6 +706,32 @@ def test_float32_attention_of_sequences_that_bring_no_token(counts):
         assert torch.equal(step(list(range(B)), ws), want)
 
 
+# more pages than workgroups a row, so that each walks several: even and uneven turns, pages outside a window in between, heads
+# of two tiles of 16, widths that leave a wave without value columns
+@pytest.mark.parametrize("nh,nkv,dk,dv,B,most,opt", [(8, 4, 128, 128, 40, 1300, {}), (4, 4, 64, 64, 34, 1600, {"window": 300, "keep_first": 70}),
+                                                     (34, 2, 64, 32, 33, 1100, {}), (3, 3, 80, 16, 50, 1025, {"chunk": 500})])
+def test_float32_attention_of_single_tokens_over_many_pages(nh, nkv, dk, dv, B, most, opt):
+    """The bits of the prompts' kernel."""
+    from transformer_amd import kernels
+    from transformer_amd.parts.linear import Workspace
+    own = np.random.default_rng([nh, dk, B])
+    pages = -(-most // 64)
+    g = torch.Generator(device=DEV).manual_seed(B)
+    kc = torch.randn(B * pages, nkv, 64, dk, generator=g, device=DEV)
+    vc = torch.randn(B * pages, nkv, dv, 64, generator=g, device=DEV)
+    table = dev(own.permutation(B * pages).reshape(B, pages), torch.int32)
+    pos = own.integers(0, most, B)
+    pos[:3] = most - 1, 0, 511
+    q, cu = torch.randn(B, nh * dk, generator=g, device=DEV), dev(np.arange(B + 1), torch.int32)
+    got = []
+    for ws in (Workspace(DEV), None):
+        out = torch.full((B, nh * dv), float("nan"), device=DEV)
+        kernels.attention_sink(q, out, kc, vc, table, cu, dev(pos, torch.int32), 1, nh, nkv, dk, dv, 0.2, opt.get("window"),
+                               None, None, None, keep_first=opt.get("keep_first", 0), chunk=opt.get("chunk"), ws=ws)
+        got.append(out)
+    assert torch.isfinite(got[1]).all() and torch.equal(got[0], got[1])
+
+
 # a table so wide that its partial rows go through in turns: of two and one sequences, of one kv head, of three and two
 @pytest.mark.parametrize("nh,nkv,B,width", [(20, 5, 3, 20000), (8, 2, 2, 128000), (40, 5, 1, 38000)])
 def test_float32_attention_of_single_tokens_in_turns(nh, nkv, B, width):

@@ -250,55 +250,75 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
     }
 }
 
-// Single tokens: a wave takes one page of one (sequence, kv head, 16 of the group's heads), operands straight from
-// memory: all of a page's 64 KB are asked for at once. Pages the sequence does not have end at once: the grid
-// follows the page table's width, so that a recorded launch fits every length. 4 sequences of 50 to 300 keys, 16
-// heads over 4 kv heads: 14.3 us and 4.7 to join (279 by one workgroup per sequence and kv head).
+// Single tokens: a workgroup takes pages of one (sequence, kv head, 16 of the group's heads), operands straight from
+// memory, all of a page's 64 KB asked for at once. Wave t forms the scores of keys 16 t .. + 15, hands them round through
+// LDS, and sums the values of columns 16 d .. + 15 for d = t, t + 4; weights, maximum and sum are formed by every wave, so
+// that each number comes about as in the prompts' kernel. Bound by the trip to memory. The grid follows the page table's width, so
+// that a recorded launch fits every length; the pages are its slowest index, since workgroups that find no page are then handed out
+// last (with the pages fastest 4 x 200 keys, 16 heads over 4 kv heads, 14.0 us for both kernels where it now takes 9.1).
+// Both kernels, those heads, 4 x 200 / 16 x 300 / 16 x 2,000 keys: 9.1 / 12.3 / 36 us; with a wave a page, which brings 64 KB by
+// itself, 20.6 / 58 / 65; by one workgroup per sequence and kv head 279 (4 of 50 to 300).
 template <int NB, bool EXACT>
 __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
-  const int group = p.nh / p.nkv, tiles = (group + 15) / 16, b = p.b0 + blockIdx.z;
-  const int kvh = p.kv0 + blockIdx.y / tiles, h0 = blockIdx.y % tiles * 16;
-  const int lane = threadIdx.x % TA_WAVE, r = lane % 16, kb = lane / 16;
-  const int page = blockIdx.x * 4 + threadIdx.x / TA_WAVE;
+  __shared__ f32x4 scores[2][4][TA_WAVE];
+  const int group = p.nh / p.nkv, tiles = (group + 15) / 16, b = p.b0 + blockIdx.y;
+  const int kvh = p.kv0 + blockIdx.x / tiles, h0 = blockIdx.x % tiles * 16;
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE, r = lane % 16, kb = lane / 16;
   const int end = p.pos0[b] + 1;
-  Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
-  if (page >= p.max_blocks || !see.page(page)) return;
+  const Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
+  if ((int)blockIdx.z * 64 >= end) return;
   if (p.cu_q[b + 1] == p.cu_q[b]) return;          // a sequence that brings no token has no row
+  constexpr int OWN = NB / 4;                      // blocks of value columns a wave owns
   const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
   const bool ok = h0 + r < group;
   const int head = kvh * group + (ok ? h0 + r : 0);
-  const size_t at = ((size_t)p.table[(size_t)b * p.max_blocks + page] * p.nkv + kvh) * 64;
-  const float *kp = p.k + at * p.dh, *vp = p.v + at * p.dv;
   const float* qrow = p.q + (size_t)p.cu_q[b] * p.q_stride + (size_t)head * p.dh;
-  f32x4 kf[4][NB], vf[4][NB], qf[NB];
+  f32x4 qf[NB];
 #pragma unroll
   for (int d = 0; d < NB; ++d)
-    if (EXACT || d < nkb) {
-      qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) kf[t][d] = *reinterpret_cast<const f32x4*>(kp + (size_t)(16 * t + r) * p.dh + 16 * d + 4 * kb);
-    }
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
+    if (EXACT || d < nkb) qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
+  for (int page = blockIdx.z, turn = 0; page * 64 < end; page += gridDim.z) {
+    if (!see.page(page)) continue;
+    const size_t at = ((size_t)p.table[(size_t)b * p.max_blocks + page] * p.nkv + kvh) * 64;
+    const float *kp = p.k + (at + 16 * wave + r) * p.dh, *vp = p.v + at * p.dv;
+    f32x4 kf[NB], vf[4][OWN];
 #pragma unroll
     for (int d = 0; d < NB; ++d)
-      if (EXACT || d < nvb) vf[t][d] = *reinterpret_cast<const f32x4*>(vp + (size_t)(16 * d + r) * 64 + 16 * t + 4 * kb);
-  __builtin_amdgcn_sched_barrier(0);               // or the values are asked for behind the scores
-  f32x4 s[4], o[NB];
-  float m, l;
-  page_scores<NB, EXACT>(qf, nkb, [&](int t, int d) { return kf[t][d]; }, s);
-  page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
-  page_values<NB, EXACT>(s, nvb, end - page * 64, kb, [&](int t, int d) { return vf[t][d]; }, o);
-  if (!ok) return;
-  const size_t unit = ((size_t)blockIdx.z * p.heads + head - p.kv0 * group) * p.max_blocks + page;
-  float* sums = p.parts + unit * p.dv;
+      if (EXACT || d < nkb) kf[d] = *reinterpret_cast<const f32x4*>(kp + 16 * d + 4 * kb);
 #pragma unroll
-  for (int d = 0; d < NB; ++d)
-    if (EXACT || d < nvb) *reinterpret_cast<f32x4*>(sums + 16 * d + 4 * kb) = o[d];
-  if (kb == 0) {
-    float* ml = p.parts + (size_t)p.seqs * p.heads * p.max_blocks * p.dv + unit * 2;
-    ml[0] = m;
-    ml[1] = l;
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < OWN; ++i)
+        if (EXACT || wave + 4 * i < nvb)
+          vf[t][i] = *reinterpret_cast<const f32x4*>(vp + (size_t)(16 * (wave + 4 * i) + r) * 64 + 16 * t + 4 * kb);
+    __builtin_amdgcn_sched_barrier(0);             // or the values are asked for behind the scores
+    f32x4 own = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < NB; ++d)
+      if (EXACT || d < nkb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) own = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[d][j], qf[d][j], own, 0, 0, 0);
+    // one barrier a page: who writes this half again has passed the other half's, behind which all have read this one
+    scores[turn][wave][lane] = own;
+    __syncthreads();
+    f32x4 s[4], o[OWN];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[t] = scores[turn][t][lane];
+    turn ^= 1;
+    float m, l;
+    page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
+    page_values<OWN, EXACT>(s, (nvb - wave + 3) / 4, end - page * 64, kb, [&](int t, int i) { return vf[t][i]; }, o);
+    if (!ok) continue;
+    const size_t unit = ((size_t)blockIdx.y * p.heads + head - p.kv0 * group) * p.max_blocks + page;
+    float* sums = p.parts + unit * p.dv;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+      if (EXACT || wave + 4 * i < nvb) *reinterpret_cast<f32x4*>(sums + 16 * (wave + 4 * i) + 4 * kb) = o[i];
+    if (wave == 0 && kb == 0) {
+      float* ml = p.parts + (size_t)p.seqs * p.heads * p.max_blocks * p.dv + unit * 2;
+      ml[0] = m;
+      ml[1] = l;
+    }
   }
 }
 
@@ -344,6 +364,10 @@ __global__ __launch_bounds__(128) void attn_f32_join_kernel(F32Attention p) {
 // a row's pages one after the other: 8 sequences of 120,000 keys, 32 heads over 8, 11.0 ms, 2.9 in turns; 16 of 60,000
 // 5.5 and 2.6.)
 #define F32_PARTS (1ll << 26)
+// Workgroups of single tokens: enough for every CU to hold a few, at least 8 a row, each with every so-manieth page (256 / 512 /
+// 1,024 of them: 4 sequences of 4,000 keys, 16 heads of 64 with keys of their own, 47.6 / 46.9 / 42.5 us; 2 of 16,000 150 / 113 /
+// 102; a workgroup per page of a table of 64 pages, most of them empty, 16 sequences of 300 keys over 4 kv heads 28.7, 12.3 here).
+#define F32_PAGE_WGS 1024
 static void f32_turn(int batch, int nh, int nkv, int max_blocks, int dv, int& seqs, int& kvs) {
   const long long unit = (long long)(nh / nkv) * max_blocks * (dv + 2), fit = F32_PARTS / unit > 1 ? F32_PARTS / unit : 1;
   kvs = fit < nkv ? (int)fit : nkv;
@@ -404,7 +428,9 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
     for (p.b0 = 0; p.b0 < batch; p.b0 += p.seqs)
       for (p.kv0 = 0; p.kv0 < nkv; p.kv0 += kvs) {
         const int bs = batch - p.b0 < p.seqs ? batch - p.b0 : p.seqs, ks = nkv - p.kv0 < kvs ? nkv - p.kv0 : kvs;
-        PICK(attn_f32_pages_kernel, dim3((max_blocks + 3) / 4, ks * ((group + 15) / 16), bs));
+        const long long rows = (long long)ks * ((group + 15) / 16) * bs;
+        const int each = (int)((F32_PAGE_WGS + rows - 1) / rows), turn = each < 8 ? 8 : each;
+        PICK(attn_f32_pages_kernel, dim3(ks * ((group + 15) / 16), bs, max_blocks < turn ? max_blocks : turn));
         attn_f32_join_kernel<<<dim3(ks * group, bs), 128, 0, stream>>>(p);
       }
   } else {
