@@ -788,6 +788,34 @@ def test_gemm_simple_at_the_edges_of_its_tiles(mnk, types):
     assert torch.equal(both[0], got) and torch.equal(both[1], got)
 
 
+# float32, two groups of waves: each height of the tiles with rows and columns that end inside a tile, an odd and an even number of
+# segments, k that ends inside a block, a segment of the first and of the second group, right behind the first two
+@pytest.mark.parametrize("mnk", [(65, 16400, 516), (67, 16384, 1024), (743, 2048, 1292), (739, 2020, 1536), (1021, 2048, 772),
+                                 (1000, 2000, 2052), (300, 2100, 1028), (130, 4100, 2000)])
+def test_gemm_groups_of_waves_in_turn(mnk):
+    from transformer_amd import kernels
+    M, N, K = mnk
+    own = np.random.default_rng([M, N, K, 2])
+    a, w, bias = own.normal(size=(M, K)).astype(np.float32), own.normal(size=(N, K)).astype(np.float32), own.normal(size=N)
+    ad, wd, bd = dev(a), dev(w), dev(bias)
+    out = torch.full((M, N + 3), 7.0, device=DEV)
+    kernels.gemm_simple(ad, wd, out[:, 1:N + 1], bd)
+    rows = [0, 31, 32, 63, 64, M - 2, M - 1]
+    want = a[rows].astype(np.float64) @ w.T.astype(np.float64) + f64(bd)
+    assert np.abs(f64(out[rows, 1:N + 1]) - want).max() < 1e-6 * K ** 0.5 * 8
+    assert (out[:, 0] == 7).all() and (out[:, N + 1:] == 7).all()
+    few = torch.empty(7, N, device=DEV)          # the same bits alone
+    kernels.gemm_simple(ad[rows].contiguous(), wd, few, bd)
+    assert torch.equal(few, out[rows, 1:N + 1])
+    got = torch.empty(M, N, device=DEV)          # every row by the general kernel: rows that start anywhere
+    kernels.gemm_simple(torch.empty(M, K + 3, device=DEV)[:, 1:K + 1].copy_(ad), wd, got, bd)
+    assert torch.equal(got, out[:, 1:N + 1])
+    both = torch.empty(2, M, N, device=DEV)      # side by side
+    kernels.gemm_simple_batched(ad.expand(2, M, K), wd.expand(2, N, K), both)
+    kernels.gemm_simple(ad, wd, got)
+    assert torch.equal(both[0], got) and torch.equal(both[1], got)
+
+
 # float32, few rows, wide: the kernel that keeps its rows and walks along the columns, at the ends of its row and column tiles
 # (one more tile than workgroups, a last turn of few), segments and numbers of waves, beside sizes it leaves to the others.
 # The sums are held to the bound of the test above; the activation has the bits of the two kernels in turn.

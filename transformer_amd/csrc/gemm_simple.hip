@@ -12,9 +12,10 @@
 // which a lane that has read 4 consecutive k holds them: no operand is turned round.
 // Segments (instead of one chain over K) let few rows be split over waves; they also round less.
 //
-// Three kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk: the same for
+// Four kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk: the same for
 // wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns.
-// gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS.
+// gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS; gemm_groups: 64, 96 or 128 x 64, two groups
+// of waves that take the segments in turn.
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -249,8 +250,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
 // workgroup it is gemm_few_rows with A read first (2,048 x 2,048 6.3 us there, 6.7 here; 2,304 x 4,096, 288 tiles, at one row
 // 14.8 and 15.2; 3,072 x 2,048, 384 tiles, at 4 rows 10.7 and 9.6). Up to k = 1,024 a workgroup of two waves has too little on its
 // way for a CU, so there are two of them on each. Below k = 512 the waves would have no segment.
-#define WALK_CUS 256
-static int walk_groups(int M, int K) { return M <= 8 && K <= 1024 ? 2 * WALK_CUS : WALK_CUS; }
+#define CUS 256
+static int walk_groups(int M, int K) { return M <= 8 && K <= 1024 ? 2 * CUS : CUS; }
 static bool walk_takes(int M, int N, int K) {
   const int side = M <= 8 ? 8 : 16;
   return M >= 1 && M <= 16 && K > 512 && K <= 4096 && (N + side - 1) / side >= walk_groups(M, K) * 5 / 4;
@@ -435,6 +436,138 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
   }
 }
 
+// Tiles of 32 WM x 64 over k of more than a segment, float32: two groups of 2 WM waves take the segments in turn, each
+// wave one 32 x 32 of the tile, and the second group hands its segment's sums to the first through LDS, which adds them in
+// ascending order. Operands go to LDS as in gemm_tiles, for both groups' 32 k at a time, the barrier in the middle of a step.
+// What it gains over gemm_tiles with 64 x 64 (one group): four waves a SIMD instead of two, whose waits for LDS, loads and
+// barriers fill each other, and a tile's height that fits the CUs: a CU's time follows the rows it is given, on one workgroup
+// or on two (an older workgroup's waves go first and the younger one is left with a CU to itself), so that the host picks
+// the height whose tiles leave the CUs evenly filled. 2,048 columns over k = 8,192: 1,021 rows 292 us (309 to 331 by 64 x 64),
+// 743 rows 233 (305), 300 rows 160 (247 by few rows). The matrix instructions alone take 232 of the 292, LDS reads 20 more; the
+// rest goes with the loads (four further waves that do nothing but load, 64 x 64 and one group: 294).
+template <int WM>
+__global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __restrict__ A, int lda,
+                                                               const float* __restrict__ W, int ldw,
+                                                               const float* __restrict__ bias, float* __restrict__ C,
+                                                               int ldc, int M, int N, int K, long long sa, long long sw,
+                                                               long long sc) {
+  constexpr int WN = 2, WK = 2, ST = 2;          // waves along the columns, groups, LDS buffers
+  constexpr int WAVES = WM * WN * WK, ROWS = 32 * (WM + WN);
+  constexpr int CHUNKS = WK * ROWS / 8, PER = (CHUNKS + WAVES - 1) / WAVES;     // 8 rows of 128 bytes a load
+  A += (size_t)blockIdx.z * sa;
+  W += (size_t)blockIdx.z * sw;
+  C += (size_t)blockIdx.z * sc;
+  __shared__ f32x4 S[ST][WK][ROWS * 8];          // rows of A, then rows of W
+  __shared__ float handed[WM * WN][16][TA_WAVE];
+  const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
+  const int n0 = blockIdx.x * 32 * WN, m0 = blockIdx.y * 32 * WM;
+  const int group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
+  const int segs = (K + SEG - 1) / SEG, rounds = (segs + 1) / 2, steps = rounds * (SEG / 32);
+  // the chunks this wave brings (the last ones of WM = 3 are brought twice, by two waves)
+  const float* src[PER];
+  int to[PER], from_k[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = wave + WAVES * i < CHUNKS ? wave + WAVES * i : CHUNKS - 1;
+    const int of = c / (ROWS / 8), rows8 = c % (ROWS / 8) * 8, row = rows8 + lane / 8;
+    from_k[i] = of * SEG + ((lane % 8) ^ (row & 7)) * 4;
+    if (row < 32 * WM) src[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda + from_k[i];
+    else src[i] = W + (size_t)(n0 + row - 32 * WM < N ? n0 + row - 32 * WM : N - 1) * ldw + from_k[i];
+    to[i] = (of * ROWS + rows8) * 8;
+  }
+  const int inside = K / (WK * SEG) * (SEG / 32);      // steps that lie inside K in both groups
+  auto send = [&](int buf, int s) {
+    if (s >= steps) s = steps - 1;                     // behind the last step: the same once more, unused
+    const int k = s / (SEG / 32) * (WK * SEG) + s % (SEG / 32) * 32;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const void* p = src[i] + k;
+      if (s >= inside) p = from_k[i] + k < K ? p : (const void*)&gemm_zeros;    // past K: zeros from one address
+      ta_load_to_lds16(p, &S[buf][0][to[i]]);
+    }
+  };
+  const int half = lane / 32, r = lane % 32;
+  f32x16 total, acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) total[e] = acc[e] = 0.f;
+  f32x4 a[2][2], w[2][2];
+  auto read = [&](int set, int buf) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int at = (4 * set + 2 * p + half) ^ (r & 7);
+      a[set][p] = S[buf][group][(32 * wm + r) * 8 + at];
+      w[set][p] = S[buf][group][(32 * (WM + wn) + r) * 8 + at];
+    }
+  };
+  auto multiply = [&](int set, int j) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][p][j], w[set][p][j], acc, 0, 0, 0);
+  };
+  auto take_over = [&]() {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) total[e] += handed[wave][e][lane];
+  };
+#pragma unroll
+  for (int s = 0; s < ST; ++s) send(s, s);
+  ta_wait_loads<PER * (ST - 1)>();
+  __syncthreads();
+  read(0, 0);
+  for (int s = 0; s < steps; ++s) {
+    const int buf = s % ST;
+    read(1, buf);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) multiply(0, j);
+    ta_wait_loads<PER * (ST - 2)>();                   // the next step's k have come
+    __syncthreads();
+    // the first step's barrier of a round: the other group's sums of the round before lie in LDS
+    if (group == 0 && s % (SEG / 32) == 0 && s > 0) take_over();
+    send(buf, s + ST);
+    read(0, (s + 1) % ST);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) multiply(1, j);
+    if (s % (SEG / 32) == SEG / 32 - 1) {
+      if (group == 0) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) total[e] += acc[e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) handed[wave - WM * WN][e][lane] = acc[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    }
+  }
+  ta_wait_loads<0>();                                  // nothing may land in LDS that is another's
+  __syncthreads();
+  if (group != 0) return;
+  if (segs % 2 == 0) take_over();                      // an odd number of segments ends with the first group's
+  // accumulator: register e of a lane is row 8 (e / 4) + 4 half + e % 4 of the tile, column r
+  const int n = n0 + 32 * wn + r;
+  if (n >= N) return;
+  const float add = bias ? bias[n] : 0.f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int m = m0 + 32 * wm + 8 * (e / 4) + 4 * half + e % 4;
+    if (m < M) C[(size_t)m * ldc + n] = bias ? total[e] + add : total[e];
+  }
+}
+
+// The height WM of gemm_groups' tiles for a product, or 0 where another kernel takes it. A CU's time is that of the tiles it is
+// given, 36.5 us for 32 rows of 64 columns over k = 8,192 in tiles of 64 rows, 3 % more in tiles of 96, 2 % less in tiles of 128,
+// and 12 % less in gemm_tiles' 128 x 128 once there are enough of those to fill it (1,021 x 16,384 x 2,048: 534 us there, 614 here;
+// 300 rows 265 and 205). Below 129 tiles of 64 x 64 the few-rows kernel's finer workgroups are as fast (2,048 columns over k =
+// 8,192: 256 rows 168 and 161 us, 128 rows 79 and 158), and two segments or fewer give the groups too little (2,048 x 512 x 300
+// 13 us by 64 x 64, 17 here).
+static int groups_height(int M, int N, int K, int batch) {
+  auto tiles = [&](int rows, int cols) { return (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * batch; };
+  if (M <= 64 || K <= 2 * SEG || tiles(64, 64) <= 128) return 0;
+  auto cost = [&](int wm, int each) { return (tiles(32 * wm, 64) + CUS - 1) / CUS * wm * each; };
+  const long long c2 = cost(2, 100), c3 = cost(3, 103), c4 = cost(4, 98);
+  const long long least = c2 < c3 ? (c2 < c4 ? c2 : c4) : (c3 < c4 ? c3 : c4);
+  if (tiles(128, 128) >= 384 && (tiles(128, 128) + CUS - 1) / CUS * 8 * 88 <= least) return 0;
+  return least == c4 ? 4 : least == c2 ? 2 : 3;
+}
+
 template <typename T, typename TW, typename TC, bool VEC>
 static void launch(hipStream_t stream, const void* A_, int lda, long long sa, const void* W_, int ldw, long long sw,
                    const float* bias, void* C_, int ldc, long long sc, int M, int N, int K, int batch) {
@@ -447,6 +580,16 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
   // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
   const bool brief = K <= 128;
+  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
+    if (const int wm = groups_height(M, N, K, batch)) {
+      const dim3 grid((N + 63) / 64, (M + 32 * wm - 1) / (32 * wm), batch);
+#define GROUPS(WM) gemm_groups_kernel<WM><<<grid, WM * 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
+      if (wm == 2) GROUPS(2);
+      else if (wm == 3) GROUPS(3);
+      else GROUPS(4);
+#undef GROUPS
+      return;
+    }
   if (tiles(64) >= 192 && (M > 64 || brief)) {
     if (tiles(128) >= 384)
       gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
