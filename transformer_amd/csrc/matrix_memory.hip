@@ -17,7 +17,7 @@
 //
 // keep is formed as exp(f - (m_t - m_(t-1))): where m_t is the rounded f + m_(t-1), the difference of the
 // two maxima is exact and keep makes up for that rounding.
-#include "common.h"
+#include "chunked.h"
 
 #define MM_FLOOR_EPS 1e-6f      // beside the denominator
 
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void memory_recurrent_kernel(
 // proj: [nt] rows, stride apart, with q and k (H*dk each) and v (H*dv) at columns qoff, koff, voff; q is taken times
 // qscale. keep, write [nt, H] (ta_memory_gates); state [slots, H, dk, dv], n_state [slots, H, dk] float32, moved on.
 // o_out [nt, H, dv] = S_t^T q_t, den_out [nt, H] = n_t . q_t, float32. lanes that share a column (0: chosen by the
-// shape; 16 or 32, where the key width leaves the choice).
+// shape; 16 or 32, where the key width leaves the choice: the walk token by token).
 extern "C" int ta_memory_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int qoff, int koff,
                                    int voff, float qscale, const float* keep, const float* write, float* state,
                                    float* n_state, const int* cu_q, const int* slots, int batch, int nt, int H, int dk,
@@ -292,6 +292,14 @@ extern "C" int ta_memory_recurrent(hipStream_t stream, int dtype, const void* pr
              stride >= voff + H * dv, "ta_memory_recurrent: rows of %d are too short", stride);
   TA_REQUIRE(lanes == 0 || lanes == 16 || lanes == 32, "ta_memory_recurrent: %d lanes", lanes);
   TA_REQUIRE(dtype == TA_F32 || dtype == TA_BF16, "ta_memory_recurrent: unknown dtype %d", dtype);
+  // From a million numbers of state on the walk fills the CUs and is bound by its vector instructions; below, both are
+  // chains of latencies, of which the walk's is the shorter (walk / chunks: 1 x 1,000 tokens of 8 heads of 256 x 512
+  // 261 / 236 us, 4 x 300 236 / 116, 32 x 100 of 8 of 64 x 64 39 / 35, but 8 x 300 of those 47 / 59).
+  if (lanes == 0 && (long long)batch * H * dk * dv >= 1 << 20 && ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
+    const TaChunked c = {proj, stride, qoff, koff, voff, 1, qscale, nullptr, keep, nullptr, write, nullptr, state, cu_q, slots,
+                         H, dk, dv, (size_t)nt * H * dv, 1, o_out, n_state, den_out, false};
+    return ta_chunked_launch(stream, dtype, c, batch, "ta_memory_recurrent");
+  }
   if (lanes == 0) lanes = (long long)batch * H * dv > MM_FEW_COLUMNS ? 16 : 32;
   if (dk <= 64) lanes = 16;
   if (dk > 256) lanes = 32;

@@ -23,9 +23,10 @@
 //   inputs of every sequence kept between steps; used in front of the state space and by the
 //   attention variant that convolves its q, k and v.
 //
-// All state, decays, gates and sums are float32; tokens are walked in the same order however a
-// sequence was cut into steps, so the cut does not change a bit of the result.
-#include "common.h"
+// All state, decays, gates and sums are float32. Tokens are walked in order, except in long steps: `rglru_scan` scans
+// segments side by side and the matrix states go 16 tokens at a time (chunked.hip), counted from the step's first token, so
+// that a cut of the sequence into steps changes the order of 32-bit sums.
+#include "chunked.h"
 
 __device__ __forceinline__ int seq_of_token_r(const int* __restrict__ cu_q, int batch, int t) {
   int lo = 0, hi = batch - 1;
@@ -728,6 +729,14 @@ __global__ __launch_bounds__(256) void gla_recurrent_kernel(
 
 extern "C" int ta_gla_row_parts(int dk) { return (dk + GLA_RT - 1) / GLA_RT; }
 
+// Planes that the recurrence's readout takes at least: chunks leave it whole.
+static int recurrence_planes(bool scalar_decay, bool bonus, int dk, int nt, int batch) {
+  return ta_chunked_long(nt, batch) && ta_chunked_takes(scalar_decay, bonus, dk) ? 1 : ta_gla_row_parts(dk);
+}
+extern "C" int ta_recurrence_planes(int scalar_decay, int bonus, int dk, int nt, int batch) {
+  return recurrence_planes(scalar_decay != 0, bonus != 0, dk, nt, batch);
+}
+
 // proj: [nt, stride] rows holding q (H*dk) at qoff, k (H*dk) at koff, v (H*dv) at voff and the
 // low-rank decay input (rank) at aoff. a2: [H*dk, rank], a2b [H*dk]. alpha: scratch [nt, H*dk]
 // float32. state: [slots, H, dk, dv] float32. o_out: [ta_gla_row_parts(dk), nt, H, dv] float32,
@@ -736,7 +745,7 @@ static int gla_recurrent_launch(hipStream_t stream, int dtype, int wdtype, const
                                 int qoff, int koff, int voff, const void* low, int low_stride, int aoff, int rank,
                                 const void* a2, const float* a2b, float inv_tau, float qscale, float* alpha,
                                 float* state, const int* cu_q, const int* slots, int batch, int nt, int H, int dk,
-                                int dv, float* o_out, int mode, const float* bonus,
+                                int dv, int planes, float* o_out, int mode, const float* bonus,
                                 const float* head_decay = nullptr, int qk_share = 1,
                                 const float* tok_decay = nullptr, const float* tok_kscale = nullptr) {
   TA_REQUIRE(batch > 0 && batch <= 65535 && H > 0 && H <= 65535 && nt >= batch,
@@ -760,7 +769,15 @@ static int gla_recurrent_launch(hipStream_t stream, int dtype, int wdtype, const
 #undef GLA_DECAY
   dim3 g(batch, H, parts * tiles);
   const size_t plane = (size_t)nt * H * dv;
-  const bool few = nt <= 8 * batch;         // at most 8 tokens a sequence on average: short chunks
+  const bool few = nt <= 8 * batch;         // at most 8 tokens a sequence on average: the walk in short turns
+  TA_REQUIRE(planes == parts || planes == recurrence_planes(head_decay || tok_decay, bonus, dk, nt, batch),
+             "ta_gla_recurrent: a readout of %d planes", planes);
+  if (ta_chunked_long(nt, batch) && ta_chunked_takes(head_decay || tok_decay, bonus, dk)) {
+    const bool scalar = head_decay || tok_decay;
+    const TaChunked c = {proj, stride, qoff, koff, voff, qk_share, qscale, scalar ? nullptr : alpha, tok_decay, head_decay,
+                         tok_kscale, bonus, state, cu_q, slots, H, dk, dv, plane, planes, o_out, nullptr, nullptr, false};
+    return ta_chunked_launch(stream, dtype, c, batch, "ta_gla_recurrent");
+  }
 #define GLA_RUN(T, TC, B)                                                                                   \
   gla_recurrent_kernel<T, TC, B><<<g, 256, 0, stream>>>((const T*)proj, stride, qoff, koff, voff, alpha, qscale, \
                                                         state, cu_q, slots, H, dk, dv, tiles, plane, o_out, bonus, \
@@ -784,9 +801,9 @@ extern "C" int ta_gla_recurrent(hipStream_t stream, int dtype, int wdtype, const
                                 int qoff, int koff, int voff, int aoff, int rank, const void* a2,
                                 const float* a2b, float inv_tau, float qscale, float* alpha, float* state,
                                 const int* cu_q, const int* slots, int batch, int nt, int H, int dk, int dv,
-                                float* o_out) {
+                                int planes, float* o_out) {
   return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, proj, stride, aoff, rank, a2,
-                              a2b, inv_tau, qscale, alpha, state, cu_q, slots, batch, nt, H, dk, dv, o_out, 0,
+                              a2b, inv_tau, qscale, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 0,
                               nullptr);
 }
 
@@ -798,10 +815,10 @@ extern "C" int ta_wkv_recurrent(hipStream_t stream, int dtype, int wdtype, const
                                 int qoff, int koff, int voff, const void* low, int low_stride, int rank,
                                 const void* a2, const float* a2b, const float* bonus, float* alpha,
                                 float* state, const int* cu_q, const int* slots, int batch, int nt, int H,
-                                int dk, int dv, float* o_out) {
+                                int dk, int dv, int planes, float* o_out) {
   TA_REQUIRE(bonus != nullptr, "ta_wkv_recurrent: the bonus is required");
   return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, low, low_stride, 0, rank, a2,
-                              a2b, 1.0f, 1.0f, alpha, state, cu_q, slots, batch, nt, H, dk, dv, o_out, 1, bonus);
+                              a2b, 1.0f, 1.0f, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 1, bonus);
 }
 
 // The recurrence with ONE fixed decay per head, S_t = decay_h S_{t-1} + k_t v_t^T, o_t = S_t^T
@@ -809,10 +826,10 @@ extern "C" int ta_wkv_recurrent(hipStream_t stream, int dtype, int wdtype, const
 // ``proj`` as above. No decay input, no scratch for decays.
 extern "C" int ta_decay_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int qoff, int koff,
                                   int voff, const float* head_decay, float qscale, float* state, const int* cu_q,
-                                  const int* slots, int batch, int nt, int H, int dk, int dv, float* o_out) {
+                                  const int* slots, int batch, int nt, int H, int dk, int dv, int planes, float* o_out) {
   TA_REQUIRE(head_decay != nullptr, "ta_decay_recurrent: the heads' decays are required");
   return gla_recurrent_launch(stream, dtype, dtype, proj, stride, qoff, koff, voff, nullptr, 0, 0, 0, nullptr,
-                              nullptr, 1.0f, qscale, nullptr, state, cu_q, slots, batch, nt, H, dk, dv, o_out, 0,
+                              nullptr, 1.0f, qscale, nullptr, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 0,
                               nullptr, head_decay);
 }
 
@@ -1192,10 +1209,10 @@ extern "C" int ta_ssm_steps(hipStream_t stream, int dtype, const void* proj, int
 extern "C" int ta_ssm_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int coff, int boff,
                                 int xoff, int share, const float* decay, const float* dt, float* state,
                                 const int* cu_q, const int* slots, int batch, int nt, int H, int N, int P,
-                                float* o_out) {
+                                int planes, float* o_out) {
   TA_REQUIRE(decay != nullptr && dt != nullptr, "ta_ssm_recurrent: decays and step sizes are required");
   return gla_recurrent_launch(stream, dtype, dtype, proj, stride, coff, boff, xoff, nullptr, 0, 0, 0, nullptr,
-                              nullptr, 1.0f, 1.0f, nullptr, state, cu_q, slots, batch, nt, H, N, P, o_out, 0,
+                              nullptr, 1.0f, 1.0f, nullptr, state, cu_q, slots, batch, nt, H, N, P, planes, o_out, 0,
                               nullptr, nullptr, share, decay, dt);
 }
 

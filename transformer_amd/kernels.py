@@ -1301,6 +1301,19 @@ def gla_row_parts(key_dim: int) -> int:
     return int(library().ta_gla_row_parts(c_int(key_dim)))
 
 
+def recurrence_planes(key_dim: int, nt: int, batch: int, scalar_decay: bool = False, bonus: bool = False) -> int:
+    """Planes of a readout that the recurrences are given at least for a step of nt tokens: one where they go in chunks,
+    else ``gla_row_parts``."""
+    return int(library().ta_recurrence_planes(c_int(int(scalar_decay)), c_int(int(bonus)), c_int(key_dim), c_int(nt),
+                                              c_int(batch)))
+
+
+def _planes_fit(o_out, shape, key_dim, batch, scalar_decay=False, bonus=False) -> bool:
+    """A readout [planes, *shape] in as many planes as ``gla_row_parts`` or ``recurrence_planes`` say."""
+    return o_out.dim() == 4 and tuple(o_out.shape[1:]) == shape and \
+        o_out.shape[0] in (gla_row_parts(key_dim), recurrence_planes(key_dim, shape[0], batch, scalar_decay, bonus))
+
+
 def gla_recurrent(proj: torch.Tensor, heads: int, key_dim: int, value_dim: int, rank: int, a2, a2_bias,
                   tau: float, state: torch.Tensor, cu_q, slots, o_out: torch.Tensor,
                   alpha: torch.Tensor) -> torch.Tensor:
@@ -1308,7 +1321,7 @@ def gla_recurrent(proj: torch.Tensor, heads: int, key_dim: int, value_dim: int, 
     the output gate and the low-rank decay input, in that order. Per head S <- diag(alpha) S +
     k v^T with alpha = sigmoid(a2 @ low + a2_bias)^(1/tau), o = S^T (q / sqrt(dk)). ``state``
     [slots, H, dk, dv] float32; ``alpha`` [nt, H*dk] float32 scratch that receives the decays;
-    o_out [gla_row_parts(dk), nt, H, dv] float32 planes that add up to the readout."""
+    o_out [gla_row_parts(dk) or recurrence_planes(..), nt, H, dv] float32 planes that add up to the readout."""
     _dev(proj, "proj", contiguous=False)
     nt, stride = _rows2d(proj, "proj")
     H, dk, dv = heads, key_dim, value_dim
@@ -1317,7 +1330,7 @@ def gla_recurrent(proj: torch.Tensor, heads: int, key_dim: int, value_dim: int, 
     _dev(o_out, "o_out", torch.float32); _dev(alpha, "alpha", torch.float32)
     if proj.shape[1] != 2 * H * dk + 2 * H * dv + rank or a2.shape != (H * dk, rank) \
             or a2_bias.shape != (H * dk,) or state.dim() != 4 or state.shape[1:] != (H, dk, dv) \
-            or o_out.shape != (gla_row_parts(dk), nt, H, dv) or alpha.shape != (nt, H * dk):
+            or not _planes_fit(o_out, (nt, H, dv), dk, batch) or alpha.shape != (nt, H * dk):
         raise KernelError(f"gla_recurrent: shapes do not fit {H} heads of {dk} / {dv}, rank {rank}: "
                           f"proj {tuple(proj.shape)} a2 {tuple(a2.shape)} state {tuple(state.shape)} "
                           f"o_out {tuple(o_out.shape)} alpha {tuple(alpha.shape)}")
@@ -1326,7 +1339,7 @@ def gla_recurrent(proj: torch.Tensor, heads: int, key_dim: int, value_dim: int, 
         c_int(stride), c_int(0), c_int(H * dk), c_int(2 * H * dk), c_int(2 * H * dk + 2 * H * dv),
         c_int(rank), _ptr(a2), _ptr(a2_bias), c_float(1.0 / tau), c_float(float(dk) ** -0.5), _ptr(alpha),
         _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt), c_int(H), c_int(dk), c_int(dv),
-        _ptr(o_out)))
+        c_int(o_out.shape[0]), _ptr(o_out)))
     return o_out
 
 
@@ -1488,7 +1501,7 @@ def wkv_recurrent(rkvg: torch.Tensor, low: torch.Tensor, heads: int, key_dim: in
     _dev(w2, "w2"); _dev(w0, "w0", torch.float32); _dev(bonus, "bonus", torch.float32)
     _dev(state, "state", torch.float32); _dev(o_out, "o_out", torch.float32); _dev(decay, "decay", torch.float32)
     if nl != nt or w2.shape != (n, rank) or w0.shape != (n,) or bonus.numel() != n or state.dim() != 4 \
-            or state.shape[1:] != (H, dk, dv) or o_out.shape != (gla_row_parts(dk), nt, H, dv) \
+            or state.shape[1:] != (H, dk, dv) or not _planes_fit(o_out, (nt, H, dv), dk, batch, bonus=True) \
             or decay.shape != (nt, n) or 3 * nt * n >= 2 ** 31:
         raise KernelError(f"wkv_recurrent: shapes do not fit {H} heads of {dk}: low {tuple(low.shape)} w2 "
                           f"{tuple(w2.shape)} state {tuple(state.shape)} o_out {tuple(o_out.shape)}")
@@ -1496,7 +1509,7 @@ def wkv_recurrent(rkvg: torch.Tensor, low: torch.Tensor, heads: int, key_dim: in
         _stream(), c_int(_code(rkvg.dtype)), c_int(_wcode(w2, rkvg.dtype, "wkv_recurrent")), _ptr(rkvg), c_int(n),
         c_int(0), c_int(nt * n), c_int(2 * nt * n), _ptr(low), c_int(ls), c_int(rank), _ptr(w2), _ptr(w0),
         _ptr(bonus), _ptr(decay), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt), c_int(H),
-        c_int(dk), c_int(dv), _ptr(o_out)))
+        c_int(dk), c_int(dv), c_int(o_out.shape[0]), _ptr(o_out)))
     return o_out
 
 
@@ -1552,14 +1565,14 @@ def decay_recurrent(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, head
     _dev(decays, "decays", torch.float32); _dev(state, "state", torch.float32); _dev(o_out, "o_out", torch.float32)
     ends = (q_off + H * dk, k_off + H * dk, v_off + H * dv)
     if min(q_off, k_off, v_off) < 0 or max(ends) > proj.shape[1] or decays.shape != (H,) or state.dim() != 4 \
-            or state.shape[1:] != (H, dk, dv) or o_out.shape != (gla_row_parts(dk), nt, H, dv):
+            or state.shape[1:] != (H, dk, dv) or not _planes_fit(o_out, (nt, H, dv), dk, batch, scalar_decay=True):
         raise KernelError(f"decay_recurrent: shapes do not fit {H} heads of {dk} / {dv}: proj {tuple(proj.shape)} "
                           f"offsets {(q_off, k_off, v_off)} decays {tuple(decays.shape)} state {tuple(state.shape)} "
                           f"o_out {tuple(o_out.shape)}")
     _check(library().ta_decay_recurrent(
         _stream(), c_int(_code(proj.dtype)), _ptr(proj), c_int(stride), c_int(q_off), c_int(k_off), c_int(v_off),
         _ptr(decays), c_float(q_scale), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt), c_int(H),
-        c_int(dk), c_int(dv), _ptr(o_out)))
+        c_int(dk), c_int(dv), c_int(o_out.shape[0]), _ptr(o_out)))
     return o_out
 
 
@@ -2205,13 +2218,13 @@ def ssm_recurrent(xbc: torch.Tensor, x_off: int, b_off: int, c_off: int, heads: 
         raise KernelError(f"ssm_recurrent: decay {tuple(decay.shape)} / dt {tuple(dt.shape)}, expected {(nt, heads)}")
     if state.dim() != 4 or tuple(state.shape[1:]) != (heads, state_dim, head_dim):
         raise KernelError(f"ssm_recurrent: state is {tuple(state.shape)}")
-    if tuple(o_out.shape) != (gla_row_parts(state_dim), nt, heads, head_dim):
-        raise KernelError(f"ssm_recurrent: o_out is {tuple(o_out.shape)}")
     batch = _step_tables(cu_q, slots, nt, "ssm_recurrent")
+    if not _planes_fit(o_out, (nt, heads, head_dim), state_dim, batch, scalar_decay=True):
+        raise KernelError(f"ssm_recurrent: o_out is {tuple(o_out.shape)}")
     _check(library().ta_ssm_recurrent(
         _stream(), c_int(_code(xbc.dtype)), _ptr(xbc), c_int(stride), c_int(c_off), c_int(b_off), c_int(x_off),
         c_int(heads // groups), _ptr(decay), _ptr(dt), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt),
-        c_int(heads), c_int(state_dim), c_int(head_dim), _ptr(o_out)))
+        c_int(heads), c_int(state_dim), c_int(head_dim), c_int(o_out.shape[0]), _ptr(o_out)))
     return o_out
 
 

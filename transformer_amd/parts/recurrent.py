@@ -3,8 +3,9 @@
 ``DiagonalRecurrence``: a gated linear recurrence per channel behind a short causal
 convolution (the recurrent block of De et al., "Griffin: Mixing Gated Linear Recurrences with
 Local Attention for Efficient Language Models"). ``GatedLinearAttention``: a matrix state per
-head with a decay per key channel. Both walk a sequence's tokens in order in float32, so the
-result does not depend on how the sequence was cut into steps; a step's products (the input
+head with a decay per key channel. Both pass a sequence's state on from token to token (in long
+steps from segment to segment) in float32, so a cut of the sequence into steps changes the result by
+rounding alone; a step's products (the input
 and output projections) are the framework's usual ones.
 """
 from __future__ import annotations
@@ -98,7 +99,7 @@ class GatedLinearAttention(Part):
         proj = linear(h, self.w["in.weight"], ctx.ws.take("gla.in", (nt, self.width), self.dtype))
         o = kernels.gla_recurrent(proj, H, dk, dv, s.rank, self.w["decay.weight"], self.w["decay.bias"],
                                   float(s.tau), cache.layer_state(layer), ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("gla.o", (kernels.gla_row_parts(dk), nt, H, dv), torch.float32),
+                                  ctx.ws.take("gla.o", (kernels.recurrence_planes(dk, nt, ctx.batch), nt, H, dv), torch.float32),
                                   ctx.ws.take("gla.alpha", (nt, H * dk), torch.float32))
         g = kernels.gla_out(o, proj, H, dk, dv, self.w["norm.weight"], float(s.eps),
                             ctx.ws.take("gla.gated", (nt, H * dv), self.dtype))
@@ -110,8 +111,8 @@ class BonusRecurrence(Part):
 
     Its five inputs are token-shifted rows with a weight vector each; the previous token's row
     is the first of its two pieces of state, the heads' matrices the second. The kernels are
-    those of ``GatedLinearAttention`` with the readout placed before the update (the recurrence
-    walks a sequence's tokens in order in float32; decays and state never leave float32)."""
+    those of ``GatedLinearAttention`` with the readout placed before the update (decays and state never
+    leave float32)."""
     graph_safe = True
     SHIFTS = 5          # r, k, v, gate, decay: the order of the rows of ``mu``
 
@@ -151,7 +152,8 @@ class BonusRecurrence(Part):
         low = linear(mixed[4], self.w["w1.weight"], ctx.ws.take("bonus.low", (nt, s.decay_rank), self.dtype))
         o = kernels.wkv_recurrent(rkvg, low, H, dk, dk, self.w["w2.weight"], self.w["w0"], self.w["bonus"], state,
                                   ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("bonus.o", (kernels.gla_row_parts(dk), nt, H, dk), torch.float32),
+                                  ctx.ws.take("bonus.o", (kernels.recurrence_planes(dk, nt, ctx.batch, bonus=True), nt, H, dk),
+                                              torch.float32),
                                   ctx.ws.take("bonus.decay", (nt, n), torch.float32))
         g = kernels.head_norm_gate(o, rkvg[3], H, dk, self.w["norm.weight"], float(s.eps),
                                    ctx.ws.take("bonus.gated", (nt, n), self.dtype))
@@ -168,8 +170,8 @@ class DecayLinearAttention(Part):
     the queries instead (the readout is linear in both); the norm of the readout per head or
     over all heads at once, with or without a weight; the gate's activation. The recurrence is
     the kernel of ``GatedLinearAttention`` with the head's constant in place of a decay per
-    key channel and token: state, decays and readout stay float32, tokens are walked in order,
-    so a cut of the sequence changes nothing."""
+    key channel and token: state, decays and readout stay float32, a cut
+    of the sequence changes the order of sums alone."""
     graph_safe = True
 
     def __init__(self, spec, dtype, device):
@@ -222,7 +224,8 @@ class DecayLinearAttention(Part):
                                k_inplace=True)
         o = kernels.decay_recurrent(proj, 0, self.nk, 2 * self.nk, H, dk, dv, self.decays, float(s.key_scale),
                                     cache.layer_state(layer), ctx.cu_q, ctx.slots,
-                                    ctx.ws.take("decay_attention.o", (kernels.gla_row_parts(dk), nt, H, dv),
+                                    ctx.ws.take("decay_attention.o",
+                                                (kernels.recurrence_planes(dk, nt, ctx.batch, scalar_decay=True), nt, H, dv),
                                                 torch.float32))
         gate = proj[:, 2 * self.nk + self.nv:]
         gated = ctx.ws.take("decay_attention.gated", (nt, self.nv), self.dtype)
@@ -243,7 +246,7 @@ class StateSpace(Part):
     sizes and decays of every (token, head) in float32; the recurrence is the kernel of
     ``GatedLinearAttention`` with q = C, k = B, v = x, the heads of a group reading the same B and C,
     one decay per (token, head) and the step size as a factor on the key, so state, decays and
-    readout stay float32 and tokens are walked in order; ``kernels.gated_group_norm`` adds D x, gates
+    readout stay float32; ``kernels.gated_group_norm`` adds D x, gates
     with silu(z) and norms the parts of the row."""
     graph_safe = True
 
@@ -294,7 +297,9 @@ class StateSpace(Part):
         kernels.ssm_steps(proj, self.inner + self.conv_width, H, self.w["dt_bias"], self.w["A_log"], dt, decay)
         o = kernels.ssm_recurrent(xbc, 0, self.inner, self.inner + self.gn, H, s.groups, N, P, decay, dt,
                                   cache.layer_state(layer[0]), ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("state_space.o", (kernels.gla_row_parts(N), nt, H, P), torch.float32))
+                                  ctx.ws.take("state_space.o",
+                                              (kernels.recurrence_planes(N, nt, ctx.batch, scalar_decay=True), nt, H, P),
+                                              torch.float32))
         y = kernels.gated_group_norm(o.view(o.shape[0], nt, self.inner), proj, 0, self.w["norm.weight"], float(s.eps),
                                      s.norm_groups, ctx.ws.take("state_space.y", (nt, self.inner), self.dtype),
                                      x=xbc, x_off=0, skip=self.w["D"], head_dim=P)
