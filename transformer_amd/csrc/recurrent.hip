@@ -245,6 +245,105 @@ __global__ __launch_bounds__(256) void rglru_gates_tiled_kernel(
   }
 }
 
+// Few tokens: a workgroup owns 16 channels of a block (32 rows of the two gates) and TT tokens. Eight lanes share a row and
+// ask for its first 256 weights before anything else, so that the trip to memory runs beside the convolution of the block's
+// inputs, which every workgroup of the block forms for itself; sums over the lanes at the end. Bound by the latency of those
+// two: 8 tokens of 16 blocks of 256 in bfloat16 (4 MB) 12 us, where the kernel above walks the block's inputs in
+// turns behind barriers on a quarter of the workgroups (49).
+#define RGF_OC 16
+#define RGF_MOST 256          // tokens of a step, from there on the tiles above (or the library, in bfloat16)
+
+template <typename TW> struct alignas(8 * sizeof(TW)) RgRun { TW x[8]; };
+
+// TAPS: 4, or 0 for any number, which then waits for its taps one by one
+template <typename T, typename TW, int TT, int TAPS>
+__global__ __launch_bounds__(256) void rglru_gates_few_kernel(
+    const T* __restrict__ yx, int stride, int xoff, const float* __restrict__ xbias,
+    const float* __restrict__ taps, const float* __restrict__ conv_bias, int K_,
+    const float* __restrict__ conv_state, const TW* __restrict__ gates_w,
+    const float* __restrict__ gates_b, const float* __restrict__ lam, float c0,
+    const int* __restrict__ cu_q, const int* __restrict__ slots, int batch, int nt, int C, int nb,
+    float* __restrict__ a_out, float* __restrict__ b_out) {
+  extern __shared__ float u[];                 // [TT][bs]
+  const int K = TAPS ? TAPS : K_;
+  __shared__ int s_start[TT], s_slot[TT];
+  __shared__ float s_sum[2 * RGF_OC][TT];
+  const int bs = C / nb, tiles = bs / RGF_OC;
+  const int blk = blockIdx.y / tiles, o0 = (blockIdx.y % tiles) * RGF_OC, t0 = blockIdx.x * TT;
+  const int row = threadIdx.x / 8, l8 = threadIdx.x % 8;     // rows 0..15: recurrence gate, 16..31: input gate
+  const TW* w = gates_w + ((size_t)((row / RGF_OC) * nb + blk) * bs + o0 + row % RGF_OC) * bs + 8 * l8;
+  RgRun<TW> wr[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) wr[j] = *reinterpret_cast<const RgRun<TW>*>(w + (64 * j < bs ? 64 * j : 0));
+  if (threadIdx.x < TT) {
+    const int t = t0 + threadIdx.x < nt ? t0 + threadIdx.x : nt - 1;
+    const int b = seq_of_token_r(cu_q, batch, t);
+    s_start[threadIdx.x] = cu_q[b];
+    s_slot[threadIdx.x] = slots[b];
+  }
+  __syncthreads();
+  // (a token past the step's end computes what the last one does)
+#pragma unroll 4
+  for (int idx = threadIdx.x; idx < TT * bs; idx += 256) {
+    const int tt = idx / bs, c = blk * bs + idx % bs;
+    const int t = t0 + tt < nt ? t0 + tt : nt - 1, start = s_start[tt];
+    const float* cs = conv_state + ((size_t)s_slot[tt] * (K - 1)) * C;
+    const float xb = xbias[c];
+    float acc = conv_bias[c];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      const int tp = t - (K - 1 - j);
+      const bool here = tp >= start;
+      const float a = to_f32(yx[(size_t)(here ? tp : t) * stride + xoff + c]) + xb;
+      const float m = K > 1 ? cs[(size_t)(here ? 0 : K - 1 + (tp - start)) * C + c] : 0.f;
+      acc = fmaf(taps[(size_t)c * K + j], here ? a : m, acc);
+    }
+    u[idx] = acc;
+  }
+  __syncthreads();
+  float acc[TT];
+#pragma unroll
+  for (int t = 0; t < TT; ++t) acc[t] = 0.f;
+  for (int k0 = 0; k0 < bs; k0 += 256) {
+    if (k0 > 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) wr[j] = *reinterpret_cast<const RgRun<TW>*>(w + (k0 + 64 * j < bs ? k0 + 64 * j : 0));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (k0 + 64 * j < bs) {
+        const float* ub = u + k0 + 64 * j + 8 * l8;
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          const float4 x = *reinterpret_cast<const float4*>(ub + t * bs), y = *reinterpret_cast<const float4*>(ub + t * bs + 4);
+          const float us[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[t] = fmaf(to_f32(wr[j].x[e]), us[e], acc[t]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TT; ++t) {
+    float x = acc[t];
+    x += ta_dpp<0xB1>(x);
+    x += ta_dpp<0x4E>(x);
+    x += ta_dpp<0x141>(x);                     // eight lanes
+    if (l8 == 0) s_sum[row][t] = x;
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < TT * RGF_OC; idx += 256) {
+    const int tt = idx / RGF_OC, o = idx % RGF_OC, t = t0 + tt, ob = o0 + o, c = blk * bs + ob;
+    if (t < nt) {
+      const float r = sigmoidf_(s_sum[o][tt] + gates_b[(size_t)blk * bs + ob]);
+      const float g = sigmoidf_(s_sum[RGF_OC + o][tt] + gates_b[(size_t)(nb + blk) * bs + ob]);
+      const float loga = -c0 * r * softplusf_(lam[c]);
+      a_out[(size_t)t * C + c] = expf(loga);
+      b_out[(size_t)t * C + c] = sqrtf(-expm1f(2.0f * loga)) * g * u[tt * bs + ob];
+    }
+  }
+}
+
 // Long steps of a bfloat16 engine take the gates' block-diagonal products to the matrix cores
 // without giving up 32-bit inputs: `rglru_conv_split` leaves u in float32 and as two bfloat16
 // numbers hi + lo = u (to 16 bits of mantissa), the library multiplies both by the bfloat16
@@ -336,6 +435,26 @@ extern "C" int ta_rglru_gates(hipStream_t stream, int dtype, int wdtype, const v
   TA_REQUIRE(nb <= 65535, "ta_rglru_gates: too many blocks");
   const int bs = C / nb;
   const int bsp = (bs + RGT_KC - 1) / RGT_KC * RGT_KC;
+  const int few_tt = nt <= 4 ? 4 : nt <= 8 ? 8 : 16;
+  const size_t lds_few = (size_t)few_tt * bs * sizeof(float);
+  if (nt <= RGF_MOST && bs % 64 == 0 && lds_few <= 60000 && (long long)nb * (bs / RGF_OC) <= 65535 && (uintptr_t)gates_w % 32 == 0) {
+    dim3 gf((nt + few_tt - 1) / few_tt, nb * (bs / RGF_OC));
+#define RGF_LAUNCH_K(T, TW, TT, TAPS)                                                                  \
+  rglru_gates_few_kernel<T, TW, TT, TAPS><<<gf, 256, lds_few, stream>>>((const T*)yx, stride, xoff, xbias, taps, conv_bias, K, \
+      conv_state, (const TW*)gates_w, gates_b, lam, c0, cu_q, slots, batch, nt, C, nb, a_out, b_out)
+#define RGF_LAUNCH(T, TW, TT) \
+  if (K == 4) RGF_LAUNCH_K(T, TW, TT, 4); else RGF_LAUNCH_K(T, TW, TT, 0)
+#define RGF_BY_TT(T, TW) \
+  if (few_tt == 4) { RGF_LAUNCH(T, TW, 4); } else if (few_tt == 8) { RGF_LAUNCH(T, TW, 8); } else { RGF_LAUNCH(T, TW, 16); }
+    if (dtype == TA_F32 && wdtype == TA_F32) { RGF_BY_TT(float, float); }
+    else if (dtype == TA_BF16 && wdtype == TA_BF16) { RGF_BY_TT(bf16_t, bf16_t); }
+    else if (dtype == TA_BF16 && wdtype == TA_F32) { RGF_BY_TT(bf16_t, float); }
+    else return ta_fail("ta_rglru_gates: unsupported dtypes %d / %d", dtype, wdtype);
+#undef RGF_BY_TT
+#undef RGF_LAUNCH
+#undef RGF_LAUNCH_K
+    return ta_check_launch("ta_rglru_gates");
+  }
   const size_t lds_tiled = ((size_t)RGT_TT * bsp + 2 * RGT_KC * RGT_OC) * sizeof(float);
   const int tiles = (bs + RGT_OC - 1) / RGT_OC;
   if (lds_tiled <= 64000 && (long long)nb * tiles <= 65535) {
