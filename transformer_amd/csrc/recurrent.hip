@@ -1089,6 +1089,124 @@ extern "C" int ta_gla_out(hipStream_t stream, int dtype, const float* o, int par
   return ta_gla_out_act(stream, dtype, o, parts, proj, stride, goff, w, 0, eps, nt, H, dv, 0, nullptr, nullptr, out);
 }
 
+// ------------------------------------------------------------------ gla: a step of single tokens
+// Decays, update, readout, the head's norm and its gate in one kernel, a workgroup of dk dv / 16 threads per (head,
+// sequence): a thread keeps four neighbouring columns of four key channels and asks for them before anything else. Bound by
+// the state's way from memory and back: 8 sequences of 32 heads of 128 x 128 (34 MB) 8.9 us, where decays (4.6), recurrence
+// (16.1) and norm (4.7) were kernels of their own; 4 of 32 heads of 64 x 64 8.2 us against 5.1 + 6.0 + 3.9.
+// low: [batch] rows, low_stride apart, of the decay's low-rank input; mode and bonus as above.
+template <typename T, typename TW, bool BONUS>
+__global__ __launch_bounds__(1024) void gla_step_kernel(
+    const T* __restrict__ proj, int stride, int qoff, int koff, int voff, const T* __restrict__ low, int low_stride, int rank,
+    const TW* __restrict__ a2, const float* __restrict__ a2b, float inv_tau, int mode, float qscale,
+    const float* __restrict__ bonus, float* __restrict__ state, const int* __restrict__ slots, int H, int dk, int dv,
+    const T* __restrict__ gate, int gate_stride, const float* __restrict__ w, int wstride, float eps, int gate_act,
+    T* __restrict__ out) {
+  __shared__ float s_q[256], s_k[256], s_a[256], s_u[BONUS ? 256 : 1];
+  __shared__ __attribute__((aligned(16))) float s_o[16][256];      // readouts of the waves' rows
+  __shared__ float s_ss[4];
+  const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, threads = blockDim.x;
+  const int groups = dv / 4, cg = tid % groups, rg = tid / groups, rstep = dk / 4;      // rows rg + rstep i
+  float* st = state + ((size_t)slots[b] * H + h) * dk * (size_t)dv + 4 * cg;
+  float4 S[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) S[i] = *reinterpret_cast<const float4*>(st + (size_t)(rg + rstep * i) * dv);
+  const T* row = proj + (size_t)b * stride;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = to_f32(row[voff + h * dv + 4 * cg + e]);
+  float gv = 0.f, wc = 1.f;
+  if (tid < dv) {
+    gv = to_f32(gate[(size_t)b * gate_stride + h * dv + tid]);
+    if (w) wc = w[h * wstride + tid];
+  }
+  for (int i = tid; i < dk; i += threads) {
+    s_q[i] = to_f32(row[qoff + h * dk + i]) * qscale;
+    s_k[i] = to_f32(row[koff + h * dk + i]);
+    if (BONUS) s_u[BONUS ? i : 0] = bonus[h * dk + i];
+  }
+  // eight lanes a channel
+  for (int i = tid / 8; i < dk; i += threads / 8) {
+    const TW* wr = a2 + (size_t)(h * dk + i) * rank;
+    float z = 0.f;
+    for (int r = tid % 8; r < rank; r += 8) {
+      const float x = to_f32(low[(size_t)b * low_stride + r]);
+      z = fmaf(to_f32(wr[r]), mode == 1 ? tanhf(x) : x, z);
+    }
+    z += ta_dpp<0xB1>(z);
+    z += ta_dpp<0x4E>(z);
+    z += ta_dpp<0x141>(z);
+    z += a2b[h * dk + i];
+    if (tid % 8 == 0)
+      s_a[i] = mode == 1 ? expf(-expf(z)) : expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau);
+  }
+  __syncthreads();
+  float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = rg + rstep * i;
+    const float q = s_q[r], k = s_k[r], a = s_a[r], u = BONUS ? s_u[BONUS ? r : 0] : 0.f;
+    float x[4] = {S[i].x, S[i].y, S[i].z, S[i].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float kv = k * v[e], was = x[e];
+      x[e] = fmaf(a, was, kv);
+      o[e] = fmaf(BONUS ? fmaf(u, kv, was) : x[e], q, o[e]);
+    }
+    *reinterpret_cast<float4*>(st + (size_t)r * dv) = float4{x[0], x[1], x[2], x[3]};
+  }
+  for (int d = groups; d < TA_WAVE; d <<= 1) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], d, TA_WAVE);
+  }
+  if (tid % TA_WAVE < groups) *reinterpret_cast<float4*>(&s_o[tid / TA_WAVE][4 * cg]) = float4{o[0], o[1], o[2], o[3]};
+  __syncthreads();
+  float y = 0.f;
+  const int waves = threads / TA_WAVE;
+  if (tid < dv)
+    for (int i = 0; i < waves; ++i) y += s_o[i][tid];
+  const float ss = wave_sum(y * y);
+  if (tid % TA_WAVE == 0 && tid < dv) s_ss[tid / TA_WAVE] = ss;
+  __syncthreads();
+  if (tid >= dv) return;
+  float sum = s_ss[0];
+  for (int i = 1; i < (dv + TA_WAVE - 1) / TA_WAVE; ++i) sum += s_ss[i];
+  const float f = rsqrtf(sum / (float)dv + eps), sg = 1.0f / (1.0f + expf(-gv));
+  out[(size_t)b * ((size_t)H * dv) + h * dv + tid] = from_f32<T>(y * f * wc * (gate_act == 1 ? sg : gv * sg));
+}
+
+// Heads that the kernel takes: its threads are whole waves, at most 1,024 and at least one per column, and a wave holds
+// whole rows of threads.
+extern "C" int ta_gla_step_fits(int dk, int dv) {
+  return dk >= 16 && dk <= 256 && dk % 4 == 0 && dv >= 16 && dv <= 256 && (dv & (dv - 1)) == 0 &&
+         dk * dv % (16 * TA_WAVE) == 0 && dk * dv <= 16 * 1024;
+}
+
+// proj, q, k, v, a2, a2b, inv_tau, qscale, state: as ta_gla_recurrent's, a row per sequence; low: rows of the low-rank input;
+// bonus: null, or the bonus recurrence with its double-exponential decay; gate, w, wstride, eps, gate_act, out: as
+// ta_gla_out_act's.
+extern "C" int ta_gla_step(hipStream_t stream, int dtype, int wdtype, const void* proj, int stride, int qoff, int koff, int voff,
+                           const void* low, int low_stride, int rank, const void* a2, const float* a2b, float inv_tau,
+                           float qscale, const float* bonus, float* state, const int* slots, int batch, int H, int dk, int dv,
+                           const void* gate, int gate_stride, const float* w, int wstride, float eps, int gate_act, void* out) {
+  TA_REQUIRE(ta_gla_step_fits(dk, dv), "ta_gla_step: heads of %d x %d", dk, dv);
+  TA_REQUIRE(batch > 0 && batch <= 65535 && H > 0 && rank >= 1 && rank <= 8192, "ta_gla_step: batch %d, %d heads, rank %d", batch, H, rank);
+  TA_REQUIRE(gate_act == 0 || gate_act == 1, "ta_gla_step: unknown gate activation %d", gate_act);
+  TA_REQUIRE(wstride == 0 || wstride == dv, "ta_gla_step: weight rows of %d for heads of %d", wstride, dv);
+  TA_REQUIRE((uintptr_t)state % 16 == 0, "ta_gla_step: the state lies off 16 bytes");
+  const dim3 g(H, batch);
+#define GS_RUN(T, TW, B)                                                                                                  \
+  gla_step_kernel<T, TW, B><<<g, dk * dv / 16, 0, stream>>>((const T*)proj, stride, qoff, koff, voff, (const T*)low, low_stride, rank, \
+      (const TW*)a2, a2b, inv_tau, B ? 1 : 0, qscale, bonus, state, slots, H, dk, dv, (const T*)gate, gate_stride, w, wstride, \
+      eps, gate_act, (T*)out)
+  if (dtype == TA_F32 && wdtype == TA_F32) { if (bonus) GS_RUN(float, float, true); else GS_RUN(float, float, false); }
+  else if (dtype == TA_BF16 && wdtype == TA_BF16) { if (bonus) GS_RUN(bf16_t, bf16_t, true); else GS_RUN(bf16_t, bf16_t, false); }
+  else if (dtype == TA_BF16 && wdtype == TA_F32) { if (bonus) GS_RUN(bf16_t, float, true); else GS_RUN(bf16_t, float, false); }
+  else return ta_fail("ta_gla_step: unsupported dtypes %d / %d", dtype, wdtype);
+#undef GS_RUN
+  return ta_check_launch("ta_gla_step");
+}
+
 // ------------------------------------------------------------------ short causal convolution
 // y_t[c] = act(bias_out[c] + sum_j taps[c][j] * u_{t-(K-1-j)}[c]) on a range of columns of the rows of
 // ``in``; u = in + bias_in (a bias that belongs to the projection in front). Inputs before a

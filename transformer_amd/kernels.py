@@ -1360,6 +1360,43 @@ def gla_out(o: torch.Tensor, proj: torch.Tensor, heads: int, key_dim: int, value
     return out
 
 
+def gla_step_fits(key_dim: int, value_dim: int) -> bool:
+    """Whether ``gla_step`` takes heads of this size."""
+    return bool(library().ta_gla_step_fits(c_int(key_dim), c_int(value_dim)))
+
+
+def gla_step(rows: torch.Tensor, q_off: int, k_off: int, v_off: int, low: torch.Tensor, a2, a2_bias, tau: float,
+             q_scale: float, bonus: Optional[torch.Tensor], state: torch.Tensor, slots, gate: torch.Tensor, weight, eps: float,
+             out: torch.Tensor) -> torch.Tensor:
+    """A step of single tokens of ``gla_recurrent`` (or, with ``bonus``, ``wkv_recurrent``) and the norm and gate behind it
+    (``head_norm_gate`` with silu) in one kernel. rows [batch, ..]: q, k, v at element offsets (that may lie behind a
+    row's end: planes), heads x width each; low [batch, rank]; gate, out [batch, H*dv]; weight [dv] or [H*dv]."""
+    _dev(rows, "rows", contiguous=False); _dev(state, "state", torch.float32); _dev(slots, "slots", torch.int32)
+    B, stride = _rows2d(rows, "rows")
+    _dev(low, "low", rows.dtype, contiguous=False); _dev(gate, "gate", rows.dtype, contiguous=False); _dev(out, "out", rows.dtype)
+    _dev(a2, "a2"); _dev(a2_bias, "a2_bias", torch.float32); _dev(weight, "weight", torch.float32)
+    if state.dim() != 4 or not gla_step_fits(*state.shape[2:]):
+        raise KernelError(f"gla_step: state {tuple(state.shape)}")
+    _, H, dk, dv = state.shape
+    (nl, ls), (ng, gs), rank = _rows2d(low, "low"), _rows2d(gate, "gate"), low.shape[1]
+    if bonus is not None:
+        _dev(bonus, "bonus", torch.float32)
+    room = (rows.untyped_storage().nbytes() // rows.element_size()) - rows.storage_offset()
+    if slots.numel() != B or nl != B or ng != B or gate.shape[1] != H * dv or out.shape != (B, H * dv) \
+            or a2.shape != (H * dk, rank) or a2_bias.shape != (H * dk,) or weight.numel() not in (dv, H * dv) \
+            or (bonus is not None and bonus.numel() != H * dk) or min(q_off, k_off, v_off) < 0 \
+            or max(q_off + H * dk, k_off + H * dk, v_off + H * dv) + (B - 1) * stride > room:
+        raise KernelError(f"gla_step: shapes do not fit {H} heads of {dk} / {dv}: rows {tuple(rows.shape)} low "
+                          f"{tuple(low.shape)} gate {tuple(gate.shape)} out {tuple(out.shape)} a2 {tuple(a2.shape)}")
+    _check(library().ta_gla_step(
+        _stream(), c_int(_code(rows.dtype)), c_int(_wcode(a2, rows.dtype, "gla_step")), _ptr(rows), c_int(stride),
+        c_int(q_off), c_int(k_off), c_int(v_off), _ptr(low), c_int(ls), c_int(rank), _ptr(a2), _ptr(a2_bias),
+        c_float(1.0 / tau), c_float(q_scale), _ptr(bonus), _ptr(state), _ptr(slots), c_int(B), c_int(H), c_int(dk), c_int(dv),
+        _ptr(gate), c_int(gs), _ptr(weight), c_int(dv if weight.numel() == H * dv and H > 1 else 0), c_float(eps), c_int(0),
+        _ptr(out)))
+    return out
+
+
 # ------------------------------------------------------------------ results normed before they join the stream
 def postnorm_add(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor, eps: float,
                  xcast: Optional[torch.Tensor] = None, next_weight: Optional[torch.Tensor] = None,

@@ -97,6 +97,13 @@ class GatedLinearAttention(Part):
         s, nt = self.spec, h.shape[0]
         H, dk, dv = s.num_heads, s.key_dim, s.value_dim
         proj = linear(h, self.w["in.weight"], ctx.ws.take("gla.in", (nt, self.width), self.dtype))
+        if ctx.all_single and kernels.gla_step_fits(dk, dv):
+            gates = 2 * H * dk + H * dv
+            g = kernels.gla_step(proj, 0, H * dk, 2 * H * dk, proj[:, gates + H * dv:], self.w["decay.weight"],
+                                 self.w["decay.bias"], float(s.tau), float(dk) ** -0.5, None, cache.layer_state(layer),
+                                 ctx.slots, proj[:, gates:gates + H * dv], self.w["norm.weight"], float(s.eps),
+                                 ctx.ws.take("gla.gated", (nt, H * dv), self.dtype))
+            return linear_delta(g, self.w["out.weight"], ctx.ws, "gla.delta"), None
         o = kernels.gla_recurrent(proj, H, dk, dv, s.rank, self.w["decay.weight"], self.w["decay.bias"],
                                   float(s.tau), cache.layer_state(layer), ctx.cu_q, ctx.slots,
                                   ctx.ws.take("gla.o", (kernels.recurrence_planes(dk, nt, ctx.batch), nt, H, dv), torch.float32),
@@ -150,6 +157,11 @@ class BonusRecurrence(Part):
         for i in range(4):
             linear(mixed[i], w[i], rkvg[i])
         low = linear(mixed[4], self.w["w1.weight"], ctx.ws.take("bonus.low", (nt, s.decay_rank), self.dtype))
+        if ctx.all_single and kernels.gla_step_fits(dk, dk):
+            g = kernels.gla_step(rkvg[0], 0, nt * n, 2 * nt * n, low, self.w["w2.weight"], self.w["w0"], 1.0, 1.0,
+                                 self.w["bonus"], state, ctx.slots, rkvg[3], self.w["norm.weight"], float(s.eps),
+                                 ctx.ws.take("bonus.gated", (nt, n), self.dtype))
+            return linear_delta(g, self.w["out.weight"], ctx.ws, "bonus.delta"), None
         o = kernels.wkv_recurrent(rkvg, low, H, dk, dk, self.w["w2.weight"], self.w["w0"], self.w["bonus"], state,
                                   ctx.cu_q, ctx.slots,
                                   ctx.ws.take("bonus.o", (kernels.recurrence_planes(dk, nt, ctx.batch, bonus=True), nt, H, dk),
