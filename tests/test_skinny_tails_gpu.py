@@ -1,0 +1,64 @@
+"""What the few-rows product does behind its sums: activations, and several products in one launch."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _randn(seed, *shape):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+
+
+@pytest.mark.parametrize("kind", ["gelu", "gelu_tanh", "relu2", "silu"])
+@pytest.mark.parametrize("m,n,k", [(1, 24, 64), (4, 64, 2048), (16, 1000, 136), (3, 10256, 256), (16, 10240, 4096)])
+def test_activation_in_the_product_has_the_bits_of_its_kernel(m, n, k, kind):
+    """One tile and many, k that ends inside a chunk, the kernel that holds its rows (640 tiles and more), side rows that
+    are part of a wider table."""
+    from transformer_amd import kernels as K
+    a, w = _randn(1, m, k), _randn(2, n, k)
+    table = _randn(3, m, n + 40).float()
+    for side in (None, table[:, 8:8 + n]):
+        for dtype in (torch.bfloat16, torch.float32):
+            want = K.gemm_skinny(a, w, torch.empty(m, n, dtype=dtype, device=DEV))
+            K.activation(want, want, kind, side=side)
+            got = K.gemm_skinny_act(a, w, torch.full((m, n), float("nan"), dtype=dtype, device=DEV), kind, side)
+            assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("m,n,k", [(1, 24, 64), (8, 1000, 136), (16, 14336, 4096)])
+def test_gated_activation_in_the_product_has_the_bits_of_its_kernel(m, n, k, kind):
+    from transformer_amd import kernels as K
+    a, w = _randn(4, m, k), _randn(5, 2 * n, k)
+    parts = [K.gemm_skinny(a, w[i * n:(i + 1) * n], torch.empty(m, n, dtype=torch.bfloat16, device=DEV)) for i in range(2)]
+    want = K.glu(torch.cat(parts, 1), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), kind)
+    got = K.gemm_skinny_act(a, w, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), kind, glu=True)
+    # the halves' sums are cut among as many waves as their own shape says: a rounding apart at most
+    assert float((got.float() - want.float()).abs().max()) <= 2 ** -7 * float(want.float().abs().max())
+    assert float((got.float() - want.float()).norm()) <= 2 ** -8 * float(want.float().norm())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("count,m,n,k", [(1, 1, 16, 8), (4, 4, 2048, 2048), (3, 16, 40, 200), (5, 7, 100, 1000)])
+def test_products_in_one_launch_have_the_bits_of_their_own(count, m, n, k, dtype):
+    from transformer_amd import kernels as K
+    a, w = _randn(6, count + 1, m, k)[:count], _randn(7, count, n, k)
+    out = torch.full((count, m, n), float("nan"), dtype=dtype, device=DEV)
+    K.gemm_skinny_many(a, w, out)
+    for i in range(count):
+        assert torch.equal(out[i], K.gemm_skinny(a[i], w[i], torch.empty(m, n, dtype=dtype, device=DEV)))
+
+
+def test_shapes_that_do_not_fit_are_refused():
+    from transformer_amd import kernels as K
+    a, w = _randn(8, 4, 64), _randn(9, 32, 64)
+    out = torch.empty(4, 32, dtype=torch.bfloat16, device=DEV)
+    for call in (lambda: K.gemm_skinny_act(a, w, out[:, :31], "silu"), lambda: K.gemm_skinny_act(a, w, out, "tanh"),
+                 lambda: K.gemm_skinny_act(a, w, out, "relu2", glu=True),
+                 lambda: K.gemm_skinny_act(a, w, out, "silu", side=torch.zeros(4, 31, device=DEV)),
+                 lambda: K.gemm_skinny_many(a.view(1, 4, 64), w.view(2, 16, 64), out.view(1, 4, 32)),
+                 lambda: K.gemm_skinny_many(_randn(1, 1, 17, 64), w.view(1, 32, 64), torch.empty(1, 17, 32, device=DEV))):
+        with pytest.raises(K.KernelError):
+            call()

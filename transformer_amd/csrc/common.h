@@ -45,10 +45,21 @@ template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float f) {
   return r;
 }
 
-// How a product that owns a gate column and an up column joins them: silu(gate) * up, or, with a
+// 0 gelu (erf), 1 gelu (tanh), 2 relu squared, 3 silu
+__device__ __forceinline__ float ta_act(int act, float z) {
+  switch (act) {
+    case 0: return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
+    case 1: return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    case 2: { const float r = fmaxf(z, 0.f); return r * r; }
+    default: return z / (1.0f + expf(-z));
+  }
+}
+
+// How a product that owns a gate column and an up column joins them: silu(gate) * up, gelu_tanh(gate) * up, or, with a
 // limit, g * sigmoid(slope * g) * (u + shift) with g = min(gate, limit), u = clamp(up, -limit, limit).
 struct TaGlu {
-  float limit, slope, shift;      // limit 0: silu
+  float limit, slope, shift;      // limit 0: silu, or
+  int gelu;                       // gelu (tanh)
 };
 __device__ __forceinline__ float ta_glu(const TaGlu& p, float g, float u) {
   if (p.limit > 0.f) {
@@ -56,6 +67,7 @@ __device__ __forceinline__ float ta_glu(const TaGlu& p, float g, float u) {
     u = fminf(fmaxf(u, -p.limit), p.limit);
     return g / (1.0f + expf(-p.slope * g)) * (u + p.shift);
   }
+  if (p.gelu) return ta_act(1, g) * u;
   return g / (1.0f + expf(-g)) * u;
 }
 

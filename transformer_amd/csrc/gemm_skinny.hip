@@ -27,6 +27,11 @@
 // leaves the sum of squares of its 16 columns per row in out_parts[tile][16]. The product
 // behind the norm (scale_parts set) sums these per row in tile order and multiplies its
 // result by rsqrt(sum / size + eps): a row's scale factors out of the dot product.
+//
+// A product whose result goes through an activation (and a row of a side table) applies it to what it stores, and equal
+// products of different rows share a launch: in a recorded step of small products a launch costs 3 to 5 us whatever it
+// does (4 tokens, two layers of a matrix recurrence and two of latent attention over 2,048 columns: 14 launches and some 60 us
+// of 500 less).
 #include "common.h"
 
 struct SkinnyNorm {
@@ -40,12 +45,24 @@ struct SkinnyNorm {
   int ldh;
   float* out_parts;           // [tiles][16]
   TaGlu glu;                  // SWIGLU: how gate and up are joined
+  int act;                    // else 1 + the activation of ta_act, 0: none
+  const float* side;          // [M][side_stride], or null: a factor behind the activation
+  int side_stride;
+  size_t a_step, w_step, c_step;      // from one of the launch's products (blockIdx.y) to the next
 };
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// what becomes of a sum that has been rounded as the product alone would store it
+template <typename TC>
+__device__ __forceinline__ float skinny_act(const SkinnyNorm& nm, float v, int m, int n) {
+  if (sizeof(TC) == 2) v = to_f32(from_f32<bf16_t>(v));
+  v = ta_act(nm.act - 1, v);
+  return nm.side ? v * nm.side[(size_t)m * nm.side_stride + n] : v;
+}
 
 union Frag16 {
   bf16x8 v;
@@ -64,6 +81,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
                                                                  const float* __restrict__ bias,
                                                                  TC* __restrict__ C, int ldc, int M,
                                                                  int n_out, int K, SkinnyNorm nm) {
+  A += blockIdx.y * nm.a_step;
+  W += blockIdx.y * nm.w_step;
+  C += blockIdx.y * nm.c_step;
   constexpr int NT = SWIGLU ? 2 : 1;
   constexpr int SP = 16;       // partial sums of squares a thread asks for ahead of the product
   __shared__ float row_sq[WAVES][16];
@@ -234,6 +254,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     if (threadIdx.x % 16 == 0) nm.out_parts[(size_t)blockIdx.x * 16 + m] = sq;
     return;
   }
+  if (!SWIGLU && nm.act && col_ok) o = skinny_act<TC>(nm, o, m, n);
   if (col_ok) C[(size_t)m * ldc + n] = from_f32<TC>(o);
 }
 
@@ -365,6 +386,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_hold_kernel(const bf16_t* __
             gate = sum;
         } else {
           if (bias) sum += bias[n];
+          if (nm.act) sum = skinny_act<TC>(nm, sum, m, n);
           C[(size_t)m * ldc + n] = from_f32<TC>(sum);
         }
       }
@@ -387,7 +409,7 @@ static int skinny_waves(int n_out, int K) {
 
 static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const void* A, int lda,
                          const void* W, int ldw, const float* bias, void* C, int ldc, int M,
-                         int n_out, int K, int waves, const SkinnyNorm& nm);
+                         int n_out, int K, int waves, const SkinnyNorm& nm, int count = 1);
 
 // out_dtype TA_BF16 or TA_F32. swiglu != 0: W is [2*n_out, K] (gate rows, then up rows),
 // C is [M, n_out] and bias, if given, has 2*n_out entries. Otherwise W is [n_out, K].
@@ -412,7 +434,7 @@ extern "C" int ta_gemm_skinny_norm_bf16(hipStream_t stream, int out_dtype, int s
                                         float* out_parts, float limit, float slope, float shift) {
   TA_REQUIRE(limit >= 0.f && (limit == 0.f || swiglu), "ta_gemm_skinny_norm_bf16: limit %g", (double)limit);
   SkinnyNorm nm = {};
-  nm.glu = TaGlu{limit, slope, shift};
+  nm.glu = TaGlu{limit, slope, shift, 0};
   if (scale_parts) {
     TA_REQUIRE(n_parts > 0 && size > 0, "ta_gemm_skinny_norm_bf16: %d partial sums over a width of %d", n_parts, size);
     nm.scale_parts = scale_parts; nm.n_parts = n_parts; nm.eps = eps; nm.inv_size = 1.0f / (float)size;
@@ -428,9 +450,36 @@ extern "C" int ta_gemm_skinny_norm_bf16(hipStream_t stream, int out_dtype, int s
   return skinny_launch(stream, out_dtype, swiglu, A, lda, W, ldw, bias, C, ldc, M, n_out, K, waves, nm);
 }
 
+// The product with its activation. glu 0: C [M, n_out] = act(A W^T) (* side), act as ta_act's; 1: W is [2 n_out, K], C =
+// act(gate) * up, act 1 (gelu, tanh) or 3 (silu), no side.
+extern "C" int ta_gemm_skinny_act_bf16(hipStream_t stream, int out_dtype, int glu, int act, const void* A, int lda, const void* W,
+                                       int ldw, void* C, int ldc, int M, int n_out, int K, const float* side, int side_stride) {
+  TA_REQUIRE(act >= 0 && act <= 3 && (!glu || ((act == 1 || act == 3) && !side)), "ta_gemm_skinny_act_bf16: activation %d", act);
+  TA_REQUIRE(side == nullptr || side_stride >= n_out, "ta_gemm_skinny_act_bf16: side rows of %d for %d columns", side_stride, n_out);
+  SkinnyNorm nm = {};
+  if (glu) nm.glu.gelu = act == 1;
+  else nm.act = act + 1;
+  nm.side = side;
+  nm.side_stride = side_stride;
+  return skinny_launch(stream, out_dtype, glu, A, lda, W, ldw, nullptr, C, ldc, M, n_out, K, 0, nm);
+}
+
+// count products of one shape in one launch; steps in elements from one's operands and result to the next's.
+extern "C" int ta_gemm_skinny_many_bf16(hipStream_t stream, int out_dtype, const void* A, int lda, long long a_step, const void* W,
+                                        int ldw, long long w_step, void* C, int ldc, long long c_step, int M, int n_out, int K, int count) {
+  TA_REQUIRE(count >= 1 && count <= 65535, "ta_gemm_skinny_many_bf16: %d products", count);
+  TA_REQUIRE(a_step >= 0 && w_step >= 0 && c_step >= 0 && a_step % 8 == 0 && w_step % 8 == 0,
+             "ta_gemm_skinny_many_bf16: operands must start on 16 bytes");
+  SkinnyNorm nm = {};
+  nm.a_step = a_step;
+  nm.w_step = w_step;
+  nm.c_step = c_step;
+  return skinny_launch(stream, out_dtype, 0, A, lda, W, ldw, nullptr, C, ldc, M, n_out, K, 0, nm, count);
+}
+
 static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const void* A, int lda,
                          const void* W, int ldw, const float* bias, void* C, int ldc, int M,
-                         int n_out, int K, int waves, const SkinnyNorm& nm) {
+                         int n_out, int K, int waves, const SkinnyNorm& nm, int count) {
   TA_REQUIRE(M >= 0 && M <= 16, "ta_gemm_skinny_bf16: M=%d outside [0, 16]", M);
   TA_REQUIRE(n_out > 0 && K > 0, "ta_gemm_skinny_bf16: bad sizes N=%d K=%d", n_out, K);
   TA_REQUIRE(K % 8 == 0 && lda % 8 == 0 && ldw % 8 == 0 && lda >= K && ldw >= K && (nm.X || ldc >= n_out),
@@ -439,7 +488,7 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
   TA_REQUIRE(out_dtype == TA_BF16 || out_dtype == TA_F32, "ta_gemm_skinny_bf16: unknown output dtype %d", out_dtype);
   if (M == 0) return 0;
   const int tiles = (n_out + 15) / 16, chunks = (K + 127) / 128;
-  if (waves == 0 && !nm.X && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32) {
+  if (waves == 0 && !nm.X && count == 1 && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32) {
     // about one workgroup per CU and round, at most eight tiles each
     const int steps = (swiglu ? 2 : 1) * tiles;
     const int rounds = (steps + 2047) / 2048;
@@ -465,7 +514,7 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
   if (waves == 0) waves = skinny_waves(n_out, K);
   if (swiglu && waves > 8) waves = 8;          // two tiles per wave: 8 KB of LDS each
   TA_REQUIRE(waves == 4 || waves == 8 || waves == 16, "ta_gemm_skinny_bf16: waves must be 4, 8 or 16, got %d", waves);
-  dim3 g((n_out + 15) / 16), b(waves * 64);
+  dim3 g((n_out + 15) / 16, count), b(waves * 64);
 #define LAUNCH_T(WV, SW, TL, TC, SC, FO)                                                           \
   gemm_skinny_kernel<WV, SW, TL, TC, SC, FO><<<g, b, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, \
                                                                   ldw, bias, (TC*)C, ldc, M, n_out, K, nm)

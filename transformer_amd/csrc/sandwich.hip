@@ -199,22 +199,13 @@ extern "C" int ta_stream_add(hipStream_t stream, int cast_dtype, float* x, const
 }
 
 // ------------------------------------------------------------------ activations
-__device__ __forceinline__ float act_apply(int act, float z) {
-  switch (act) {
-    case 0: return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));                              // gelu
-    case 1: return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));   // gelu (tanh)
-    case 2: { const float r = fmaxf(z, 0.f); return r * r; }                                       // relu squared
-    default: return z / (1.0f + expf(-z));                                                         // silu
-  }
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void activation_kernel(const T* __restrict__ in, int in_stride,
                                                          T* __restrict__ out, int out_stride, int n, int act,
                                                          const float* __restrict__ side, int side_stride) {
   const size_t t = blockIdx.y;
   for (int c = blockIdx.x * 256 + threadIdx.x; c < n; c += gridDim.x * 256) {
-    float v = act_apply(act, to_f32(in[t * in_stride + c]));
+    float v = ta_act(act, to_f32(in[t * in_stride + c]));
     if (side) v *= side[t * side_stride + c];
     out[t * out_stride + c] = from_f32<T>(v);
   }
@@ -233,7 +224,7 @@ __global__ __launch_bounds__(256) void activation_vec_kernel(const T* __restrict
     __builtin_memcpy(a, &raw, 16);
     float v[W];
 #pragma unroll
-    for (int i = 0; i < W; ++i) v[i] = act_apply(act, to_f32(a[i]));
+    for (int i = 0; i < W; ++i) v[i] = ta_act(act, to_f32(a[i]));
 #pragma unroll
     for (int i = 0; i < W; ++i) a[i] = from_f32<T>(v[i]);
     uint4 res;

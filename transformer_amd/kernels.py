@@ -737,6 +737,42 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor], s
     return out
 
 
+def gemm_skinny_act(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str, side: Optional[torch.Tensor] = None,
+                    glu: bool = False) -> torch.Tensor:
+    """``gemm_skinny`` followed by ``activation`` (kind, side), or with ``glu`` by ``glu`` (kind "silu" or "gelu_tanh", w [2*n,
+    k]), in one kernel with the same bits."""
+    _dev(a, "a", torch.bfloat16, contiguous=False); _dev(w, "w", torch.bfloat16, contiguous=False); _dev(out, "out", contiguous=False)
+    M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
+    if kind not in _ACTIVATIONS or (glu and kind not in _GLU_ACTS):
+        raise KernelError(f"gemm_skinny_act: unknown activation {kind!r}")
+    n_out = N // 2 if glu else N
+    if w.shape[1] != a.shape[1] or (glu and (N % 2 or side is not None)) or out.shape != (M, n_out):
+        raise KernelError(f"gemm_skinny_act: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    ss = 0
+    if side is not None:
+        _dev(side, "side", torch.float32, contiguous=False)
+        Ms, ss = _rows2d(side, "side")
+        if side.shape != (M, n_out):
+            raise KernelError(f"gemm_skinny_act: side rows {tuple(side.shape)} for {M} x {n_out}")
+    _check(library().ta_gemm_skinny_act_bf16(
+        _stream(), c_int(_code(out.dtype)), c_int(int(glu)), c_int(_ACTIVATIONS[kind]), _ptr(a), c_int(lda), _ptr(w), c_int(ldw),
+        _ptr(out), c_int(ldc), c_int(M), c_int(n_out), c_int(a.shape[1]), _ptr(side), c_int(ss)))
+    return out
+
+
+def gemm_skinny_many(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """out[i] = a[i] @ w[i].T for every i in one launch: a [count, m, k], w [count, n, k], at most 16 rows each."""
+    _dev(a, "a", torch.bfloat16, contiguous=False); _dev(w, "w", torch.bfloat16, contiguous=False); _dev(out, "out", contiguous=False)
+    if a.dim() != 3 or w.dim() != 3 or tuple(out.shape) != (a.shape[0], a.shape[1], w.shape[1]) or \
+            w.shape[0] != a.shape[0] or w.shape[2] != a.shape[2] or any(t.stride(2) != 1 for t in (a, w, out)):
+        raise KernelError(f"gemm_skinny_many: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    _check(library().ta_gemm_skinny_many_bf16(
+        _stream(), c_int(_code(out.dtype)), _ptr(a), c_int(a.stride(1)), c_longlong(a.stride(0)), _ptr(w), c_int(w.stride(1)),
+        c_longlong(w.stride(0)), _ptr(out), c_int(out.stride(1)), c_longlong(out.stride(0)), c_int(a.shape[1]), c_int(w.shape[1]),
+        c_int(a.shape[2]), c_int(a.shape[0])))
+    return out
+
+
 SKINNY_MAX_ROWS = 16
 MID_MAX_ROWS = 64
 

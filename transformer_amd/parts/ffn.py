@@ -12,7 +12,7 @@ import torch
 from .. import kernels
 from ..weights.loader import Param
 from .base import Part, PartError, register_part
-from .linear import adds_in_place, linear, linear_delta
+from .linear import activated, adds_in_place, linear, linear_delta
 
 
 class SwiGLU(Part):
@@ -97,10 +97,13 @@ class GLU(SwiGLU):
         if self.activation in ("silu", "limited"):
             return super().run(h, ctx, scale=scale, fold=fold, into=into)
         s, nt = self.spec, h.shape[0]
-        gu = linear(h, self.w["gate_up.weight"],
-                    ctx.ws.take("swiglu.gate_up", (nt, 2 * s.intermediate), self.dtype))
-        act = kernels.glu(gu, ctx.ws.take("swiglu.act", (nt, s.intermediate), self.dtype),
-                          self.activation, self.w.get("gate_up.bias"))
+        act = ctx.ws.take("swiglu.act", (nt, s.intermediate), self.dtype)
+        if not s.bias and kernels.skinny_wins(h, self.w["gate_up.weight"]):
+            kernels.gemm_skinny_act(h, self.w["gate_up.weight"], act, self.activation, glu=True)
+        else:
+            gu = linear(h, self.w["gate_up.weight"],
+                        ctx.ws.take("swiglu.gate_up", (nt, 2 * s.intermediate), self.dtype))
+            kernels.glu(gu, act, self.activation, self.w.get("gate_up.bias"))
         if fold is not None:
             kernels.gemm_skinny(act, self.w["down.weight"], None, bias=self.w.get("down.bias"), fold=fold)
             return None
@@ -124,8 +127,7 @@ class MLP(Part):
 
     def run(self, h, ctx):
         s, nt = self.spec, h.shape[0]
-        u = linear(h, self.w["up.weight"], ctx.ws.take("mlp.up", (nt, s.intermediate), self.dtype))
-        kernels.activation(u, u, s.activation)
+        u = activated(h, self.w["up.weight"], ctx.ws.take("mlp.up", (nt, s.intermediate), self.dtype), s.activation)
         return linear_delta(u, self.w["down.weight"], ctx.ws, "mlp.delta"), None
 
 
@@ -197,6 +199,8 @@ class RoutedMLP(Part):
         s, rows = self.spec, a.shape[0]
         k = 2 if self.two else 1
         pre = ws.take(name + ".pre", (rows, k * n), self.dtype)
+        if tile_expert is None and not self.two:
+            return activated(a, w, pre, s.activation)
         if tile_expert is not None:
             kernels.moe_gemm(a, w, tile_expert, pre, None if self.two else s.activation)
         else:
@@ -204,8 +208,6 @@ class RoutedMLP(Part):
         if self.glu:
             return kernels.glu(pre, ws.take(name, (rows, n), self.dtype), s.activation)
         if not self.limited:
-            if tile_expert is None:
-                kernels.activation(pre, pre, s.activation)
             return pre
         return kernels.glu_limit(pre, ws.take(name, (rows, n), self.dtype), float(act_limit),
                                  float(s.gate_slope), float(s.up_shift))

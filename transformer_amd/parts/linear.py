@@ -75,6 +75,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor], s
     return out
 
 
+def activated(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, kind: str,
+              side: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out = act(x @ weight^T) (* side): few rows in one kernel, which applies the activation to what it would store."""
+    if x.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and kernels.skinny_wins(x, weight):
+        return kernels.gemm_skinny_act(x, weight, out, kind, side)
+    return kernels.activation(linear(x, weight, out), out, kind, side=side)
+
+
 def library_planes(rows: int, weight: torch.Tensor) -> int:
     """Planes in which the vendor library leaves a float32 product of 65 to 1,536 rows over a
     long k (the down projection): one batched call multiplies the parts of k side by side, and

@@ -154,8 +154,11 @@ class BonusRecurrence(Part):
                                           self.w["mu"].view(self.SHIFTS, s.hidden), shift_state, ctx.cu_q, ctx.slots)
         rkvg = ctx.ws.take("bonus.rkvg", (4, nt, n), self.dtype)
         w = self.w["rkvg.weight"].view(4, n, s.hidden)
-        for i in range(4):
-            linear(mixed[i], w[i], rkvg[i])
+        if kernels.skinny_wins(mixed[0], w[0]):
+            kernels.gemm_skinny_many(mixed[:4], w, rkvg)         # few rows: one launch for all four
+        else:
+            for i in range(4):
+                linear(mixed[i], w[i], rkvg[i])
         low = linear(mixed[4], self.w["w1.weight"], ctx.ws.take("bonus.low", (nt, s.decay_rank), self.dtype))
         if ctx.all_single and kernels.gla_step_fits(dk, dk):
             g = kernels.gla_step(rkvg[0], 0, nt * n, 2 * nt * n, low, self.w["w2.weight"], self.w["w0"], 1.0, 1.0,

@@ -17,7 +17,7 @@ from .. import kernels
 from ..weights.loader import Param
 from .base import Part, PartError, build_part, register_part, span
 from .embedding import TokenSideTable
-from .linear import linear, linear_delta
+from .linear import activated, linear, linear_delta
 
 
 class TokenSide(Part):
@@ -42,8 +42,8 @@ class TokenSide(Part):
         if rows is None or rows.shape[1] < s.offset + s.dim:
             raise PartError("the token side input needs the step's side-table rows "
                             f"(columns {s.offset}..{s.offset + s.dim})")
-        g = linear(xcast, self.w["gate.weight"], ctx.ws.take("side.gate", (nt, s.dim), self.dtype))
-        kernels.activation(g, g, "gelu_tanh", side=rows[:, s.offset:s.offset + s.dim])
+        g = activated(xcast, self.w["gate.weight"], ctx.ws.take("side.gate", (nt, s.dim), self.dtype), "gelu_tanh",
+                      side=rows[:, s.offset:s.offset + s.dim])
         y = linear(g, self.w["proj.weight"], ctx.ws.take("side.y", (nt, s.hidden), torch.float32))
         kernels.postnorm_add(x, y, self.w["norm.weight"], float(s.eps),
                              next_weight=None if next_norm is None else next_norm.gain(),
