@@ -510,7 +510,10 @@ __device__ uint4 moe_zeros;             // where a piece past K is read from (ne
 
 // Few tiles (a step of few tokens), bound by reading the chosen experts' matrices: a workgroup owns ONE tile of 16
 // rows and 64 rows of the matrix and its four waves divide K; the partial tiles are added in wave order through
-// LDS. While 128 k are multiplied the next are on their way (16 KB a wave).
+// LDS. While 128 k are multiplied the next are on their way (16 KB a wave). The matrix comes in whole lines, sixteen lanes a
+// row's 256 bytes, and takes the operands' layout in the wave's own LDS: read in that layout straight from memory, 16 bytes of
+// sixteen rows at a time, it is the lines a CU touches that bind. 2 tokens of six of 64 experts of 1,408 x 4,096 (gate and up,
+// then down) 49.8 -> 35 and 29.9 -> 22.4 us; 4 of four of 32 of 1,024 x 2,048 16.3 -> 14.0 and 16.2 -> 12.2.
 // row_pair (or null: A holds the ordered rows): the tile's rows are read from the tokens' rows h, each times its
 // pair's weight, rounded as moe_gather rounds it: a step of few tokens needs no ordered copy.
 // GLU: the matrix holds gate rows, then up rows; the workgroup takes 32 of each and joins them.
@@ -524,7 +527,10 @@ template <typename TC, bool GLU>
 __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows, const bf16_t* __restrict__ W,
                                                                    const int* __restrict__ tile_expert,
                                                                    TC* __restrict__ C, int N, int K, int act, TaGlu glu) {
-  __shared__ float red[4][16][65];
+  // a wave's 64 rows x 128 k of the matrix on their way from whole lines to the operands' layout, then its sums
+  __shared__ __attribute__((aligned(16))) uint32_t stage[4][4][1024];
+  typedef float Sums[16][65];
+  Sums* red = reinterpret_cast<Sums*>(&stage[0][0][0]);
   const int e = tile_expert[blockIdx.y];
   if (e < 0) return;                                    // the whole workgroup: tiles past the last expert's rows
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
@@ -537,26 +543,32 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   const int kbeg = __builtin_amdgcn_readfirstlane(32 * (steps * wave / 4));
   const int kend = __builtin_amdgcn_readfirstlane(32 * (steps * (wave + 1) / 4));
   const int pair = rows.row_pair ? rows.row_pair[r0 + r] : 0;    // asked for before the matrix, needed behind it
-  const bf16_t* wrow[4];                                // rows past N: another row, whose products are not stored
+  // loading: instruction i of tile t brings rows 4 i + lane / 16; a row's sixteen lanes bring its 256 bytes, permuted by the
+  // row's number so that the operands' reads meet no bank twice
+  const int lrow = lane / 16, lpiece = lane % 16;
+  const bf16_t* wbase[2] = {We + (size_t)n0 * K, We + (size_t)(GLU ? N + n0 : n0) * K};
+  uint32_t woff[4][4];                                  // rows past N: another row, whose products are not stored
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int n = n0 + (GLU ? 16 * (t % 2) : 16 * t) + r;
-    wrow[t] = We + (size_t)((n < N ? n : N - 1) + (GLU && t >= 2 ? N : 0)) * K + kb * 8;
-  }
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = (GLU ? 16 * (t % 2) : 16 * t) + 4 * i + lrow;
+      woff[t][i] = (uint32_t)(n0 + n < N ? n : N - 1 - n0) * (uint32_t)K + (uint32_t)((lpiece ^ (4 * i + lrow)) * 8);
+    }
   moe_floatx4 acc[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) acc[t] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
   constexpr int DEPTH = 4;                              // steps of 32 k asked for together
-  MoeFrag af[2][DEPTH], wf[2][DEPTH][4];
+  MoeFrag af[2][DEPTH], wf[2][4][4];
   auto load_matrix = [&](int set, int k0) {
 #pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-      const int k = k0 + 32 * u;
-      const bool kok = k < kend && k + kb * 8 < K;
+    for (int i = 0; i < 4; ++i) {
+      const int k = k0 + (lpiece ^ (4 * i + lrow)) * 8;
+      const bool kok = k < kend && k < K;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        wf[set][u][t].q = __builtin_nontemporal_load(
-            reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(wrow[t] + k) : (const void*)&moe_zeros));
+        wf[set][t][i].q = __builtin_nontemporal_load(
+            reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(wbase[GLU && t >= 2] + k0 + woff[t][i]) : (const void*)&moe_zeros));
     }
   };
   load_matrix(0, kbeg);
@@ -578,6 +590,13 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   };
   auto multiply = [&](int set) {
 #pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<moe_u32x4*>(&stage[wave][t][(4 * i + lrow) * 64 + lpiece * 4]) = wf[set][t][i].q;
+    // the wave reads what its other lanes wrote: LDS serves a wave's requests in order
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
     for (int u = 0; u < DEPTH; ++u) {
       if (weighs) {
 #pragma unroll
@@ -587,9 +606,13 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
         }
       }
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][u][t].v, af[set][u].v, acc[t], 0, 0, 0);
+      for (int t = 0; t < 4; ++t) {
+        MoeFrag w;
+        w.q = *reinterpret_cast<const moe_u32x4*>(&stage[wave][t][r * 64 + ((4 * u + kb) ^ r) * 4]);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.v, af[set][u].v, acc[t], 0, 0, 0);
+      }
     }
+    __builtin_amdgcn_wave_barrier();
   };
   load_rows(0, kbeg);
   for (int k0 = kbeg; k0 < kend; k0 += 64 * DEPTH) {
@@ -609,6 +632,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
     if (second) multiply(1);
     __builtin_amdgcn_sched_barrier(0);
   }
+  __syncthreads();                                      // (the waves' sums lie where the others' rows were)
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
