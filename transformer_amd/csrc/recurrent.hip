@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void rglru_gates_tiled_kernel(
 // Few tokens: a workgroup owns 16 channels of a block (32 rows of the two gates) and TT tokens. Eight lanes share a row and
 // ask for its first 256 weights before anything else, so that the trip to memory runs beside the convolution of the block's
 // inputs, which every workgroup of the block forms for itself; sums over the lanes at the end. Bound by the latency of those
-// two: 8 tokens of 16 blocks of 256 in bfloat16 (4 MB) 12 us, where the kernel above walks the block's inputs in
+// two: 8 single tokens of 16 blocks of 256 in bfloat16 (4 MB) 13.4 us, where the kernel above walks the block's inputs in
 // turns behind barriers on a quarter of the workgroups (49).
 #define RGF_OC 16
 #define RGF_MOST 256          // tokens of a step, from there on the tiles above (or the library, in bfloat16)
@@ -277,12 +277,24 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
   for (int j = 0; j < 4; ++j) wr[j] = *reinterpret_cast<const RgRun<TW>*>(w + (64 * j < bs ? 64 * j : 0));
   if (threadIdx.x < TT) {
     const int t = t0 + threadIdx.x < nt ? t0 + threadIdx.x : nt - 1;
-    const int b = seq_of_token_r(cu_q, batch, t);
-    s_start[threadIdx.x] = cu_q[b];
+    const int b = nt == batch ? t : seq_of_token_r(cu_q, batch, t);      // (no sequence brings none)
+    s_start[threadIdx.x] = nt == batch ? t : cu_q[b];
     s_slot[threadIdx.x] = slots[b];
   }
   __syncthreads();
   // (a token past the step's end computes what the last one does)
+  if (nt == batch) {                           // single tokens: all taps but the last fall into the sequence's memory
+#pragma unroll 4
+    for (int idx = threadIdx.x; idx < TT * bs; idx += 256) {
+      const int tt = idx / bs, c = blk * bs + idx % bs, t = t0 + tt < nt ? t0 + tt : nt - 1;
+      const float* cs = conv_state + ((size_t)s_slot[tt] * (K - 1)) * C + c;
+      const float x = to_f32(yx[(size_t)t * stride + xoff + c]) + xbias[c];
+      float acc = conv_bias[c];
+#pragma unroll
+      for (int j = 0; j < K - 1; ++j) acc = fmaf(taps[(size_t)c * K + j], cs[(size_t)j * C], acc);
+      u[idx] = fmaf(taps[(size_t)c * K + K - 1], x, acc);
+    }
+  } else
 #pragma unroll 4
   for (int idx = threadIdx.x; idx < TT * bs; idx += 256) {
     const int tt = idx / bs, c = blk * bs + idx % bs;
