@@ -991,7 +991,7 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
 //           holds the drawn mass, the token in it.
 // 8 rows of 128,256 tokens, top-k 40 and top-p 0.95: 125 us by one workgroup a row (which gathered whole kept sets of a
 // few thousand tokens), 29 us in parts
-// (5 + 10 + 15); 64 rows 51 us, 256 rows 125, one row without a cut 16.
+// (5 + 10 + 15; the draw 12 since it asks for all it needs of the records at once and a wave adds up over the parts); 64 rows 51 us, 256 rows 125, one row without a cut 16.
 struct PartRecord {
   float2 mass[STEPS / 2];    // of two steps each, relative to the part's maximum
   uint32_t cnt[STEPS / 2];   // tokens of two steps each, 16 bits of them (a part has 4,096)
@@ -1004,13 +1004,21 @@ struct PartRecord {
   float cand_l[PART_CAND];   // in index order
 };
 
+// The rows' random numbers in the launch's arguments: the first of the three kernels puts them where the last reads them.
+#define SAMPLE_IN_ARGS 64
+struct SampleUniforms {
+  float u[SAMPLE_IN_ARGS];
+};
+
 // group u (of four) of this thread in its part
 __device__ __forceinline__ int part_group(int part, int u) { return part * (PART / 4) + u * PART_THREADS + (int)threadIdx.x; }
 
 __global__ __launch_bounds__(PART_THREADS) void sample_parts_kernel(const float* __restrict__ logits, size_t ld, int vocab,
                                                                     float inv_t, int cut, int by_mass,
-                                                                    PartRecord* __restrict__ records) {
+                                                                    PartRecord* __restrict__ records, SampleUniforms given,
+                                                                    int n_given, float* __restrict__ uniform) {
   const float* row = logits + (size_t)blockIdx.y * ld;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && (int)threadIdx.x < n_given) uniform[threadIdx.x] = given.u[threadIdx.x];
   PartRecord& rec = records[(size_t)blockIdx.y * gridDim.x + blockIdx.x];
   const int groups = (vocab + 3) / 4, wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
   __shared__ float s_f[PART_THREADS / TA_WAVE];
@@ -1259,10 +1267,35 @@ __global__ __launch_bounds__(PART_THREADS) void sample_gather_kernel(const float
   }
 }
 
+// The first part with which the running sum of what the parts keep exceeds target (-1: none), the sum in front of it in
+// *base. By a whole wave.
+__device__ __forceinline__ int find_part(const u64* kept, int parts, u64 target, u64* base) {
+  const int lane = threadIdx.x % TA_WAVE;
+  u64 run = 0;
+  for (int p0 = 0; p0 < parts; p0 += TA_WAVE) {
+    const u64 mine = p0 + lane < parts ? kept[p0 + lane] : 0;
+    u64 inc = mine;
+#pragma unroll
+    for (int o = 1; o < TA_WAVE; o <<= 1) {
+      const u64 up = shfl_up_u64(inc, o);
+      if (lane >= o) inc += up;
+    }
+    const u64 hit = __ballot(target < run + inc);
+    if (hit) {
+      const int who = __ffsll((unsigned long long)hit) - 1;
+      if (lane == who) *base = run + inc - mine;
+      return p0 + who;
+    }
+    run += (u64)__shfl((unsigned long long)inc, TA_WAVE - 1, TA_WAVE);
+  }
+  return -1;
+}
+
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float* __restrict__ logits, size_t ld, int vocab,
                                                                      float inv_t, int top_k, float top_p, int cut, int parts,
                                                                      const PartRecord* __restrict__ records,
-                                                                     const float* __restrict__ uniform, int* __restrict__ out) {
+                                                                     const float* __restrict__ uniform, int* __restrict__ out,
+                                                                     int* __restrict__ out_host) {
   const float* row = logits + (size_t)blockIdx.x * ld;
   const PartRecord* all = records + (size_t)blockIdx.x * parts;
   const int groups = (vocab + 3) / 4;
@@ -1277,30 +1310,32 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
   __shared__ u64 s_total, s_target, s_base, s_wave[SAMPLE_WAVES];
   __shared__ uint32_t s_tie_base;
   __shared__ float s_max;
-  __shared__ int s_first[MAX_PARTS];                 // first gathered token of a part
+  __shared__ int s_first[MAX_PARTS], s_n[MAX_PARTS]; // first gathered token of a part, its number of them
   __shared__ u64 s_kept[MAX_PARTS];                  // mass that a part keeps
 
-  // ---- what the parts say: 16 waves read their records side by side, one adds up
-  if (threadIdx.x == 0) s_ok = 1;
-  if (wave == 0) {
-    const float m = row_max(all, parts);
-    if (lane == 0) {
-      s_max = m;
-      s_lo = all[0].lo;
-      s_hi = all[0].hi;
-    }
+  // ---- what the parts say: everything that is needed of the records is asked for at once, before it is known how many
+  // tokens a part has gathered; a wave adds up
+  const float uni = uniform[blockIdx.x];
+  constexpr int AHEAD = 2;                           // parts of a wave whose first 64 gathered tokens are on their way
+  float ahead[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) {
+    const int p = wave + i * SAMPLE_WAVES;
+    ahead[i] = cut ? all[p < parts ? p : 0].cand_l[lane] : 0.f;
   }
-  __syncthreads();
   if (wave == 0) {
     int run = 0;
     u64 total = 0, above = 0;
     uint32_t above_n = 0;
     bool ok = true;
+    float m = -INFINITY;
+    const int lo0 = all[0].lo, hi0 = all[0].hi;
     for (int p0 = 0; p0 < parts; p0 += TA_WAVE) {
       const int p = p0 + lane;
       const bool in = p < parts;
       const PartRecord& r = all[in ? p : 0];
       const int n = in ? r.n : 0;
+      m = fmaxf(m, r.max);
       total += in ? r.total : 0;
       above += in ? r.above : 0;
       above_n += in ? r.above_n : 0;
@@ -1313,18 +1348,23 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
       }
       if (in) {
         s_first[p] = run + inc - n;
+        s_n[p] = n;
         s_kept[p] = r.above;
       }
       run += __shfl(inc, TA_WAVE - 1, TA_WAVE);
     }
+    m = wave_max(m);
     total = wave_sum_u64(total);
     above = wave_sum_u64(above);
     above_n = (uint32_t)wave_sum_u64(above_n);
     ok = __ballot(!ok) == 0;
     if (lane == 0) {
+      s_max = m;
+      s_lo = lo0;
+      s_hi = hi0;
       s_total = total;
       s_cands = run;
-      s_ok = ok && run <= ROW_CAND && total > 0 && s_lo >= 0;
+      s_ok = ok && run <= ROW_CAND && total > 0 && lo0 >= 0;
       st.prefix = 0;
       st.mask = 0;
       st.count_above = above_n;
@@ -1338,14 +1378,21 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
   }
   __syncthreads();
   if (!s_ok) {
-    sample_whole_row<false>(row, vocab, inv_t, top_k, top_p, uniform[blockIdx.x], out + blockIdx.x);
+    sample_whole_row<false>(row, vocab, inv_t, top_k, top_p, uni, out + blockIdx.x);
+    __syncthreads();
+    if (threadIdx.x == 0 && out_host) out_host[blockIdx.x] = out[blockIdx.x];
     return;
   }
   const float m = s_max;
   const int cands = s_cands, lo = s_lo, hi = s_hi, top = step_of(m, inv_t);
   if (cut) {
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int p = wave + i * SAMPLE_WAVES;
+      if (p < parts && lane < s_n[p]) cand_l[s_first[p] + lane] = ahead[i];
+    }
     for (int p = wave; p < parts; p += SAMPLE_WAVES)
-      for (int c = lane; c < all[p].n; c += TA_WAVE) cand_l[s_first[p] + c] = all[p].cand_l[c];
+      for (int c = lane + (p < AHEAD * SAMPLE_WAVES ? TA_WAVE : 0); c < s_n[p]; c += TA_WAVE) cand_l[s_first[p] + c] = all[p].cand_l[c];
     // ---- the threshold among the gathered tokens
     const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
     u64 p_lim = (u64)ceil((double)top_p * (double)s_total);
@@ -1379,7 +1426,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
   if (cut) {
     __shared__ uint32_t s_part_ties[MAX_PARTS];
     for (int p = wave; p < parts; p += SAMPLE_WAVES) {
-      const int n = all[p].n;
+      const int n = s_n[p];
       uint32_t ties = 0;
       u64 kept = 0;
       for (int c0 = 0; c0 < n; c0 += TA_WAVE) {
@@ -1396,47 +1443,53 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
       }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      u64 sum = 0;
+    // ranks of the ties, then sums of what is kept, in the parts' order: a wave, 64 parts at a time
+    if (wave == 0) {
       uint32_t rank = 0;
-      for (int p = 0; p < parts; ++p) {
-        const uint32_t t = s_part_ties[p], room = n_tie > rank ? n_tie - rank : 0;
-        s_kept[p] += (u64)(t < room ? t : room) * st.tie_mass;
-        s_part_ties[p] = rank;
-        rank += t;
-        sum += s_kept[p];
-      }
-      s_total = sum;
-      u64 target = (u64)((double)uniform[blockIdx.x] * (double)sum);
-      if (sum > 0 && target >= sum) target = sum - 1;
-      u64 run = 0;
-      for (int p = 0; p < parts; ++p) {
-        if (target < run + s_kept[p]) {
-          s_part = p;
-          s_base = run;
-          s_tie_base = s_part_ties[p];
-          break;
+      u64 sum = 0;
+      for (int p0 = 0; p0 < parts; p0 += TA_WAVE) {
+        const int p = p0 + lane;
+        const uint32_t t = p < parts ? s_part_ties[p] : 0;
+        uint32_t inc = t;
+#pragma unroll
+        for (int o = 1; o < TA_WAVE; o <<= 1) {
+          const uint32_t up = __shfl_up(inc, o, TA_WAVE);
+          if (lane >= o) inc += up;
         }
-        run += s_kept[p];
+        const uint32_t before = rank + inc - t, room = n_tie > before ? n_tie - before : 0;
+        const u64 kept = p < parts ? s_kept[p] + (u64)(t < room ? t : room) * st.tie_mass : 0;
+        if (p < parts) {
+          s_kept[p] = kept;
+          s_part_ties[p] = before;
+        }
+        rank += __shfl(inc, TA_WAVE - 1, TA_WAVE);
+        sum += wave_sum_u64(kept);
       }
+      u64 target = (u64)((double)uni * (double)sum);
+      if (sum > 0 && target >= sum) target = sum - 1;
+      const int p = find_part(s_kept, parts, target, &s_base);
+      if (lane == 0) {
+        s_total = sum;
+        s_target = target;
+        s_part = p;
+        if (p >= 0) s_tie_base = s_part_ties[p];
+      }
+    }
+  } else if (wave == 0) {
+    u64 target = (u64)((double)uni * (double)s_total);
+    if (target >= s_total) target = s_total - 1;
+    const int p = find_part(s_kept, parts, target, &s_base);
+    if (lane == 0) {
+      s_part = p;
       s_target = target;
     }
-  } else if (threadIdx.x == 0) {
-    u64 target = (u64)((double)uniform[blockIdx.x] * (double)s_total), run = 0;
-    if (target >= s_total) target = s_total - 1;
-    for (int p = 0; p < parts; ++p) {
-      if (target < run + s_kept[p]) {
-        s_part = p;
-        s_base = run;
-        break;
-      }
-      run += s_kept[p];
-    }
-    s_target = target;
   }
   __syncthreads();
   if (s_part < 0) {
-    if (threadIdx.x == 0) out[blockIdx.x] = 0;
+    if (threadIdx.x == 0) {
+      out[blockIdx.x] = 0;
+      if (out_host) out_host[blockIdx.x] = 0;
+    }
     return;
   }
   // ---- the token in that part: one group of four a thread, in index order
@@ -1491,7 +1544,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
     s_pick = pick;
   }
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = s_pick;
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = s_pick;
+    if (out_host) out_host[blockIdx.x] = s_pick;
+  }
 }
 
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(const float* __restrict__ logits, size_t ld, int vocab,
@@ -1537,11 +1593,11 @@ extern "C" long long ta_sample_scratch_for(int n, int vocab, int top_k, float to
   return n > 0 && vocab > 0 && in_parts(n, vocab, top_k, top_p) ? ta_sample_scratch(n, vocab) : 0;
 }
 
-// scratch: scratch_bytes on an 8-byte boundary, ta_sample_scratch_for of them or more, or null: one workgroup takes a
-// row then.
-extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
-                               float temperature, int top_k, float top_p, const float* uniform,
-                               int* out, void* scratch, long long scratch_bytes) {
+// given: null, or the n random numbers on the host, which then reach ``uniform`` in the launch's arguments; out_host: null, or
+// where the tokens go as well.
+static int sample_launch(hipStream_t stream, const float* logits, long long ld, int n, int vocab, float temperature, int top_k,
+                         float top_p, float* uniform, int* out, void* scratch, long long scratch_bytes, const float* given,
+                         int* out_host) {
   TA_REQUIRE(n >= 0 && vocab > 0 && ld >= vocab, "ta_sample: bad sizes n=%d vocab=%d ld=%lld", n, vocab, ld);
   TA_REQUIRE(temperature > 0.f, "ta_sample: temperature %g must be > 0 (0 means argmax)", (double)temperature);
   TA_REQUIRE(top_k >= 1, "ta_sample: top_k %d < 1", top_k);
@@ -1549,9 +1605,12 @@ extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long lon
   TA_REQUIRE((uintptr_t)scratch % 8 == 0, "ta_sample: scratch does not start on 8 bytes");
   if (n == 0) return 0;
   const float inv_t = 1.0f / temperature;
+  const bool whole = ((uintptr_t)logits % 16) != 0 || ld % 4 != 0 || scratch == nullptr || !in_parts(n, vocab, top_k, top_p);
+  TA_REQUIRE(!given || (!whole && n <= SAMPLE_IN_ARGS), "ta_sample_given: %d rows that are not dealt out in parts, or more than %d", n,
+             SAMPLE_IN_ARGS);
   if (((uintptr_t)logits % 16) != 0 || ld % 4 != 0) {
     sample_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
-  } else if (scratch == nullptr || !in_parts(n, vocab, top_k, top_p)) {
+  } else if (whole) {
     sample_rows_kernel<<<n, SAMPLE_THREADS, 0, stream>>>(logits, (size_t)ld, vocab, inv_t, top_k, top_p, uniform, out);
   } else {
     TA_REQUIRE(scratch_bytes >= ta_sample_scratch(n, vocab), "ta_sample: %lld bytes of scratch, %lld are needed", scratch_bytes,
@@ -1559,17 +1618,48 @@ extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long lon
     const int parts = sample_parts(vocab), cut = top_k < vocab || top_p < 1.0f;
     PartRecord* rec = (PartRecord*)scratch;
     const int turn = rows_at_a_time(vocab);
+    SampleUniforms args = {};
+    if (given)
+      for (int i = 0; i < n; ++i) args.u[i] = given[i];
     for (int r0 = 0; r0 < n; r0 += turn) {
       const int rows = n - r0 < turn ? n - r0 : turn;
       const float* from = logits + (size_t)r0 * ld;
       const dim3 g(parts, rows);
-      sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec);
+      sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec, args,
+                                                      given && r0 == 0 ? n : 0, uniform);
       sample_gather_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, cut, rec);
       sample_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, cut, parts, rec,
-                                                              uniform + r0, out + r0);
+                                                              uniform + r0, out + r0, out_host ? out_host + r0 : nullptr);
     }
   }
   return ta_check_launch("ta_sample");
+}
+
+// scratch: scratch_bytes on an 8-byte boundary, ta_sample_scratch_for of them or more, or null: one workgroup takes a
+// row then.
+extern "C" int ta_sample_parts(hipStream_t stream, const float* logits, long long ld, int n, int vocab,
+                               float temperature, int top_k, float top_p, const float* uniform,
+                               int* out, void* scratch, long long scratch_bytes) {
+  return sample_launch(stream, logits, ld, n, vocab, temperature, top_k, top_p, const_cast<float*>(uniform), out, scratch,
+                       scratch_bytes, nullptr, nullptr);
+}
+
+// Rows that are dealt out in parts, at most ta_sample_given_rows of them, without a copy to the GPU in front or one back behind:
+// given [n] random numbers on the host (read before the call returns), uniform [n] floats of scratch on the GPU, out_host [n]:
+// pinned host memory that receives the tokens beside out. A copy of a few bytes costs 3 us on the GPU and 5 to ask for:
+// 8 rows of 128,256 through Sampler 40 us a choice with them, 30 to 34 without (42 and 35 of which the host works).
+extern "C" int ta_sample_given_rows() { return SAMPLE_IN_ARGS; }
+extern "C" int ta_sample_given(hipStream_t stream, const float* logits, long long ld, int n, int vocab, float temperature,
+                               int top_k, float top_p, const float* given, float* uniform, int* out, int* out_host,
+                               void* scratch, long long scratch_bytes) {
+  TA_REQUIRE(given && uniform && out_host, "ta_sample_given: the random numbers, their place and the host's tokens are needed");
+  void* seen = nullptr;                              // the GPU's address of the host memory; not pinned: refused here
+  const hipError_t e = hipHostGetDevicePointer(&seen, out_host, 0);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return ta_fail("ta_sample_given: the host's tokens are not in pinned memory: %s", hipGetErrorString(e));
+  }
+  return sample_launch(stream, logits, ld, n, vocab, temperature, top_k, top_p, uniform, out, scratch, scratch_bytes, given, (int*)seen);
 }
 
 // Without scratch: one workgroup a row.

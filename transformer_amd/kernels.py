@@ -925,6 +925,29 @@ def sample(logits: torch.Tensor, uniform: torch.Tensor, out: torch.Tensor, tempe
     return out
 
 
+SAMPLE_GIVEN_ROWS = 64      # rows whose random numbers travel in a launch's arguments (SAMPLE_IN_ARGS of csrc/sampling.hip)
+
+
+def sample_given(logits: torch.Tensor, given: Sequence[float], uniform: torch.Tensor, out: torch.Tensor,
+                 out_host: torch.Tensor, temperature: float, top_k: int, top_p: float, scratch: torch.Tensor):
+    """``sample`` with the random numbers given as host values and the tokens written to pinned memory beside ``out``, so that
+    nothing is copied: at most ``SAMPLE_GIVEN_ROWS`` rows that ``sample_scratch`` deals out (> 0 with the cuts) and that
+    start on 16 bytes. uniform: n floats of scratch on the GPU."""
+    _dev(logits, "logits", torch.float32, contiguous=False); _dev(out, "out", torch.int32)
+    _dev(uniform, "uniform", torch.float32); _dev(scratch, "scratch", torch.uint8)
+    n, ld = _rows2d(logits, "logits")
+    if out.numel() != n or uniform.numel() != n or len(given) != n or n > SAMPLE_GIVEN_ROWS:
+        raise KernelError(f"sample_given: {n} rows, {len(given)} numbers, out {tuple(out.shape)} uniform {tuple(uniform.shape)}")
+    if out_host.is_cuda or out_host.dtype != torch.int32 or out_host.numel() != n or not out_host.is_contiguous() \
+            or not out_host.is_pinned():
+        raise KernelError("sample_given: out_host must be n int32 in pinned host memory")
+    vocab = logits.shape[1]
+    _check(library().ta_sample_given(_stream(), _ptr(logits), c_longlong(ld), c_int(n), c_int(vocab), c_float(temperature),
+                                     c_int(min(int(top_k), vocab)), c_float(top_p), (c_float * n)(*given), _ptr(uniform),
+                                     _ptr(out), _ptr(out_host), _ptr(scratch), c_longlong(scratch.numel())))
+    return out
+
+
 # ------------------------------------------------------------------ random fill
 def fill_normal(out: torch.Tensor, seed: int, stream_id: int, mean: float, std: float):
     """out[i] = mean + std * z_i, z_i standard normal, a function of (seed, stream_id, i)."""

@@ -71,18 +71,25 @@ class Sampler:
         out, u_dev, u_host, out_host = self._buffers(n)
         if self.args.greedy:
             kernels.argmax(logits, out)
+            out_host.copy_(out, non_blocking=True)
         else:
-            u_host.numpy()[:] = np.asarray([uniform(self.seed, s, d) for s, d in
-                                            zip(sequences, drawn)], dtype=np.float32)
-            u_dev.copy_(u_host, non_blocking=True)
+            u = [uniform(self.seed, s, d) for s, d in zip(sequences, drawn)]
             k = self.args.top_k if self.args.top_k is not None else logits.shape[1]
             need = kernels.sample_scratch(n, logits.shape[1], int(k), float(self.args.top_p))
             i = (self._turn - 1) % self.RING              # of the buffers just taken
             if need and (self._scratch[i] is None or self._scratch[i].numel() < need):
                 self._scratch[i] = torch.empty(need, dtype=torch.uint8, device=self.device)
-            kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
-                           float(self.args.top_p), self._scratch[i] if need else None)
-        out_host.copy_(out, non_blocking=True)
+            if need and len(u) == n <= kernels.SAMPLE_GIVEN_ROWS and logits.data_ptr() % 16 == 0 \
+                    and logits.stride(0) % 4 == 0:
+                # the numbers go with the launch, the tokens come back from the kernel that draws them
+                kernels.sample_given(logits, u, u_dev, out, out_host, float(self.args.temperature), int(k),
+                                     float(self.args.top_p), self._scratch[i])
+            else:
+                u_host.numpy()[:] = np.asarray(u, dtype=np.float32)
+                u_dev.copy_(u_host, non_blocking=True)
+                kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
+                               float(self.args.top_p), self._scratch[i] if need else None)
+                out_host.copy_(out, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record()
         return Chosen(out, out_host, ev)
