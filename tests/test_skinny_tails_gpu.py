@@ -62,3 +62,21 @@ def test_shapes_that_do_not_fit_are_refused():
                  lambda: K.gemm_skinny_many(_randn(1, 1, 17, 64), w.view(1, 32, 64), torch.empty(1, 17, 32, device=DEV))):
         with pytest.raises(K.KernelError):
             call()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [4096, 4097, 5120, 5121, 6143, 6144, 7168, 7169])
+@pytest.mark.parametrize("m,k", [(1, 128), (16, 4096), (5, 1000)])
+def test_a_workgroup_a_cu_has_the_bits_of_tiles_of_16(m, k, n, dtype):
+    """20, 24 and 28 columns a workgroup, the last one part of one; with a bias, behind a norm, with an activation."""
+    from transformer_amd import kernels as K
+    a, w, bias = _randn(10, m, k), _randn(11, n, k), _randn(12, n).float()
+    parts = torch.rand(-(-k // 16), 16, generator=torch.Generator(device=DEV).manual_seed(13), device=DEV)
+    scale = K.RowScale(parts, 1e-5, k)
+    for more in ({}, {"bias": bias}, {"scale": scale}, {"bias": bias, "scale": scale}):
+        want = K.gemm_skinny(a, w, torch.empty(m, n, dtype=dtype, device=DEV), waves=4, **more)
+        got = torch.full((m, n + 8), 7.0, dtype=dtype, device=DEV)
+        K.gemm_skinny(a, w, got[:, :n], **more)
+        assert torch.equal(got[:, :n], want) and (got[:, n:] == 7).all()
+    want = K.activation(K.gemm_skinny(a, w, torch.empty(m, n, dtype=dtype, device=DEV), waves=4), want, "relu2")
+    assert torch.equal(K.gemm_skinny_act(a, w, torch.empty(m, n, dtype=dtype, device=DEV), "relu2"), want)

@@ -75,7 +75,9 @@ union Frag16 {
 #define STREAM_LOAD(p) __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p))
 
 
-template <int WAVES, bool SWIGLU, bool TAIL, typename TC, bool SCALE, bool FOLD>
+// COLS: columns of a workgroup, a multiple of 4 (a load brings four rows of W): 16, or what gives every CU one workgroup of
+// a weight that in tiles of 16 would leave some CUs with two (see skinny_cols).
+template <int WAVES, bool SWIGLU, bool TAIL, typename TC, bool SCALE, bool FOLD, int COLS = 16>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ A, int lda,
                                                                  const bf16_t* __restrict__ W, int ldw,
                                                                  const float* __restrict__ bias,
@@ -84,7 +86,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
   A += blockIdx.y * nm.a_step;
   W += blockIdx.y * nm.w_step;
   C += blockIdx.y * nm.c_step;
-  constexpr int NT = SWIGLU ? 2 : 1;
+  static_assert(COLS % 4 == 0 && COLS >= 16 && (COLS == 16 || (!SWIGLU && !FOLD)), "gates and folds go by tiles of 16");
+  constexpr int NT = SWIGLU ? 2 : (COLS + 15) / 16;
   constexpr int SP = 16;       // partial sums of squares a thread asks for ahead of the product
   __shared__ float row_sq[WAVES][16];
   // per wave and tile: 16 rows x 128 k of W (4 KB) on their way from the coalesced load to
@@ -92,7 +95,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
   __shared__ __attribute__((aligned(16))) uint32_t stage[WAVES][NT][1024];
   const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
   const int r = lane % 16, kb = lane / 16;
-  const int n0 = blockIdx.x * 16;
+  const int n0 = blockIdx.x * COLS;
+  // whether load t of tile nt brings rows of the workgroup's; rows that none brings feed outputs that are never stored
+#define LIVE(nt, t) (SWIGLU || 16 * (nt) + 4 * (t) < COLS)
   // loading: instruction t brings rows 4t + lane/16; the 16 lanes of a row bring its 256
   // bytes, permuted by the row number so that the operand reads below meet no bank twice
   const int lrow = lane / 16, lpiece = lane % 16;
@@ -104,7 +109,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     gpiece[t] = lpiece ^ row;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-      wsrc[nt][t] = W + (size_t)(nt * n_out + (n0 + row < n_out ? n0 + row : 0)) * ldw + gpiece[t] * 8;
+      if (SWIGLU)
+        wsrc[nt][t] = W + (size_t)(nt * n_out + (n0 + row < n_out ? n0 + row : 0)) * ldw + gpiece[t] * 8;
+      else
+        wsrc[nt][t] = W + (size_t)(n0 + 16 * nt + row < n_out ? n0 + 16 * nt + row : 0) * ldw + gpiece[t] * 8;
   }
   const bool a_ok = r < M;
   const bf16_t* arow = A + (size_t)(a_ok ? r : 0) * lda;
@@ -138,7 +146,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     _Pragma("unroll") for (int t = 0; t < 4; ++t) {                                           \
       const bool wk_ = live_ && (!TAIL || kc_ + gpiece[t] * 8 < K);                           \
       const bool ak_ = live_ && (!TAIL || kc_ + t * 32 + kb * 8 < K);                         \
-      _Pragma("unroll") for (int nt = 0; nt < NT; ++nt) {                                     \
+      _Pragma("unroll") for (int nt = 0; nt < NT; ++nt) if (LIVE(nt, t)) {                    \
         const u32x4 v_ = STREAM_LOAD(wk_ ? wsrc[nt][t] + kc_ : W);                            \
         wreg[set][nt][t] = (TAIL && !wk_) ? u32x4{0, 0, 0, 0} : v_;                           \
       }                                                                                       \
@@ -152,7 +160,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
 #define MUL_CHUNK(set)                                                                        \
   do {                                                                                        \
     _Pragma("unroll") for (int t = 0; t < 4; ++t)                                             \
-        _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                                     \
+        _Pragma("unroll") for (int nt = 0; nt < NT; ++nt) if (LIVE(nt, t))                    \
             *reinterpret_cast<u32x4*>(&stage[wave][nt][(4 * t + lrow) * 64 + lpiece * 4]) = wreg[set][nt][t]; \
     __builtin_amdgcn_wave_barrier();                                                          \
     _Pragma("unroll") for (int t = 0; t < 4; ++t)                                             \
@@ -198,6 +206,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
   }
 #undef LOAD_CHUNK
 #undef MUL_CHUNK
+#undef LIVE
   if (SCALE) {
     float sq = 0.f;
 #pragma unroll
@@ -235,7 +244,21 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     v[nt] = sum * rs;
     // the unfused path stores the product in the output type before bias and activation
     if (SWIGLU && sizeof(TC) == 2) v[nt] = to_f32(from_f32<bf16_t>(v[nt]));
-    if (bias && col_ok) v[nt] += bias[nt * n_out + n];
+    if (SWIGLU) {
+      if (bias && col_ok) v[nt] += bias[nt * n_out + n];
+    } else if (bias && n + 16 * nt < n_out) {
+      v[nt] += bias[n + 16 * nt];
+    }
+  }
+  if (!SWIGLU) {
+#pragma unroll
+    for (int nt = 1; nt < NT; ++nt) {
+      const int col = n + 16 * nt;
+      if (16 * nt + (int)threadIdx.x % 16 < COLS && col < n_out) {
+        if (nm.act) v[nt] = skinny_act<TC>(nm, v[nt], m, col);
+        C[(size_t)m * ldc + col] = from_f32<TC>(v[nt]);
+      }
+    }
   }
   float o = v[0];
   if (SWIGLU) o = ta_glu(nm.glu, v[0], v[NT - 1]);
@@ -407,6 +430,16 @@ static int skinny_waves(int n_out, int K) {
   return w;
 }
 
+// Columns of a workgroup: what gives each of the 256 CUs one, where tiles of 16 give some of them one and some two, and those
+// set the time. us at 1 / 8 / 16 rows, tiles of 16 against this: 6,144 columns over k = 4,096 10.8 / 12.8 / 14.6 and 9.7 / 10.8 /
+// 11.6, 5,120 over 4,096 10.7 / 11.9 / 13.7 and 8.9 / 9.6 / 10.5, 7,168 over 4,096 12.1 / 13.2 / 15.9 and 11.6 / 12.0 / 12.9, 4,500 over
+// 14,336 30.5 / 35.5 / 43.6 and 22.6 / 25.0 / 30.3. Fewer columns, where some CUs have none, gain nothing from narrower
+// workgroups (3,072 over 4,096 6.6 / 7.1 / 8.1 and 6.8 / 7.3 / 7.9; 768 to 3,072 over 2,048 up to 0.2 slower).
+static int skinny_cols(int n_out) {
+  const int cols = (n_out + 1023) / 1024 * 4;
+  return cols >= 20 && cols <= 28 ? cols : 16;
+}
+
 static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const void* A, int lda,
                          const void* W, int ldw, const float* bias, void* C, int ldc, int M,
                          int n_out, int K, int waves, const SkinnyNorm& nm, int count = 1);
@@ -510,6 +543,29 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
 #undef HOLD
 #undef HOLD_SW
     return ta_check_launch("ta_gemm_skinny_bf16 (many columns)");
+  }
+  if (waves == 0 && !swiglu && !nm.X && count == 1) {
+    const int cols = skinny_cols(n_out);
+    if (cols != 16) {
+      const dim3 gc((n_out + cols - 1) / cols);
+#define COLS_RUN(WV, TL, TC, SC, CO)                                                                                \
+  gemm_skinny_kernel<WV, false, TL, TC, SC, false, CO><<<gc, WV * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, \
+                                                                                  bias, (TC*)C, ldc, M, n_out, K, nm)
+#define COLS_BY(TC, CO)                                                                                                \
+  if (K % 128 == 0) { if (nm.scale_parts) COLS_RUN(4, false, TC, true, CO); else COLS_RUN(4, false, TC, false, CO); } \
+  else { if (nm.scale_parts) COLS_RUN(4, true, TC, true, CO); else COLS_RUN(4, true, TC, false, CO); }
+#define COLS_TYPE(CO) \
+  if (out_dtype == TA_BF16) { COLS_BY(bf16_t, CO) } else { COLS_BY(float, CO) }
+      switch (cols) {
+        case 20: COLS_TYPE(20); break;
+        case 24: COLS_TYPE(24); break;
+        default: COLS_TYPE(28); break;
+      }
+#undef COLS_TYPE
+#undef COLS_BY
+#undef COLS_RUN
+      return ta_check_launch("ta_gemm_skinny_bf16 (a workgroup a CU)");
+    }
   }
   if (waves == 0) waves = skinny_waves(n_out, K);
   if (swiglu && waves > 8) waves = 8;          // two tiles per wave: 8 KB of LDS each
