@@ -87,3 +87,30 @@ def test_gates_of_few_tokens(lens, geom, dtype):
         log = -8.0 * r * torch.nn.functional.softplus(lam.double())
         np.testing.assert_allclose(a[cu[i]:cu[i + 1]].cpu(), log.exp(), atol=1e-5)
         np.testing.assert_allclose(b[cu[i]:cu[i + 1]].cpu(), (-torch.expm1(2 * log)).sqrt() * g * u, atol=2e-5, rtol=2e-5)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("taps", [1, 2, 4, 8])
+@pytest.mark.parametrize("channels", [4, 260, 1028])
+def test_convolution_of_four_channels_a_thread_has_the_bits_of_one(channels, taps, dtype):
+    """Rows that start on whole pieces against the same rows a column further: sequences that end inside, at and behind a
+    thread's sixteen tokens, biases, activation, and the memory that is left behind."""
+    from transformer_amd import kernels as K
+    td, lens = getattr(torch, dtype), [1, 2, 30, 16, 5, 40]
+    nt, C = sum(lens), channels
+    g = torch.Generator(device=DEV).manual_seed(C + taps)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, w, bi, bo, mem = r(nt, C).to(td), r(C, taps), r(C), r(C), r(8, taps - 1, C)
+    cu, slots = _t(np.concatenate([[0], np.cumsum(lens)]), torch.int32), _t([7, 0, 3, 2, 5, 6], torch.int32)
+    got = []
+    for off in (4, 5):
+        rows = torch.zeros(nt, C + 8, dtype=td, device=DEV)
+        rows[:, off:off + C] = x
+        state = mem.clone() if taps > 1 else None
+        out = torch.full((nt, C + 4), 7.0, dtype=td, device=DEV)
+        K.causal_conv(rows, off, C, w, out[:, :C], state, cu, slots, max(lens), bias_in=bi, bias_out=bo, activation="silu")
+        assert (out[:, C:] == 7).all()
+        got.append((out[:, :C], state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.isfinite(got[0][0]).all()
+    if taps > 1:
+        assert torch.equal(got[0][1], got[1][1])
