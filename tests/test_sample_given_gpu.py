@@ -57,3 +57,24 @@ def test_the_sampler_returns_the_same_tokens_on_both_sides(n):
         u = torch.tensor([uniform(5, i, turn) for i in range(n)], device=DEV)
         want = K.sample(logits, u, torch.empty(n, dtype=torch.int32, device=DEV), 0.7, 30, 0.9)
         assert got.result() == want.tolist() == got.device.tolist()
+
+
+def test_host_tokens_stay_until_they_are_written():
+    """A choice behind a few milliseconds of other work, dropped unread with its sampler: the pinned block that its kernel
+    writes to may be anyone's only behind that kernel."""
+    import transformer_amd as ta
+    from transformer_amd.sampling.sampler import Sampler
+    s = Sampler(ta.SampleArgs(0.7, 0.9, 30), seed=5, device=DEV)
+    logits, big = torch.randn(8, 32000, device=DEV), torch.randn(4096, 4096, device=DEV)
+    s.choose(logits, range(8), [0] * 8)
+    for _ in range(3):
+        s.choose_async(logits, range(8), [0] * 8)
+    for _ in range(20):
+        big = torch.mm(big, big).clamp_(-1, 1)
+    c, done = s.choose_async(logits, range(8), [0] * 8), torch.cuda.Event()
+    done.record()
+    at = c._host.data_ptr()
+    del s, c
+    taken = [torch.empty(64, dtype=torch.int32, pin_memory=True) for _ in range(16)]
+    assert done.query() or at not in [t.data_ptr() for t in taken]
+    torch.cuda.synchronize()

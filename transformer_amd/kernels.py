@@ -932,7 +932,8 @@ def sample_given(logits: torch.Tensor, given: Sequence[float], uniform: torch.Te
                  out_host: torch.Tensor, temperature: float, top_k: int, top_p: float, scratch: torch.Tensor):
     """``sample`` with the random numbers given as host values and the tokens written to pinned memory beside ``out``, so that
     nothing is copied: at most ``SAMPLE_GIVEN_ROWS`` rows that ``sample_scratch`` deals out (> 0 with the cuts) and that
-    start on 16 bytes. uniform: n floats of scratch on the GPU."""
+    start on 16 bytes. uniform: n floats of scratch on the GPU. out_host is written when the stream gets there, unknown to
+    torch's pool of pinned memory: the caller keeps it until then."""
     _dev(logits, "logits", torch.float32, contiguous=False); _dev(out, "out", torch.int32)
     _dev(uniform, "uniform", torch.float32); _dev(scratch, "scratch", torch.uint8)
     n, ld = _rows2d(logits, "logits")

@@ -30,12 +30,39 @@ def uniform(seed: int, sequence: int, drawn: int) -> float:
     return (z >> 40) / float(1 << 24)
 
 
+class _Buffers:
+    """What a choice works in. The kernel that draws the tokens stores them straight into ``host``, which torch's pool of
+    pinned memory does not hear of: the block may go back to it, for anyone to take, only behind that kernel."""
+
+    def __init__(self, rows: int, device):
+        self.rows = rows
+        self.device = torch.empty(rows, dtype=torch.int32, device=device)
+        self.uniform = torch.empty(rows, dtype=torch.float32, device=device)
+        self.uniform_host = torch.empty(rows, dtype=torch.float32, pin_memory=True)
+        self.host = torch.empty(rows, dtype=torch.int32, pin_memory=True)
+        self.scratch = None
+        self._last = {}             # the last use on each stream
+
+    def used(self):
+        """Marks the work that the current stream has been given so far as the last to touch these buffers."""
+        stream = torch.cuda.current_stream()
+        event = torch.cuda.Event()
+        event.record(stream)
+        self._last[stream.cuda_stream] = event
+        return event
+
+    def __del__(self):
+        for event in getattr(self, "_last", {}).values():
+            event.synchronize()
+
+
 class Chosen:
     """Tokens that the GPU has been asked to choose: ``device`` holds them (int32) as soon as
     the stream gets there; ``result()`` waits for their copy to the host."""
 
-    def __init__(self, device: torch.Tensor, host: torch.Tensor, event):
-        self.device, self._host, self._event = device, host, event
+    def __init__(self, buffers: _Buffers, rows: int):
+        self.device, self._host = buffers.device[:rows], buffers.host[:rows]
+        self._buffers, self._event = buffers, buffers.used()
 
     def result(self):
         self._event.synchronize()
@@ -49,26 +76,22 @@ class Sampler:
         self.args, self.seed, self.device = args, int(seed), torch.device(device)
         self._ring = [None] * self.RING
         self._turn = 0
-        self._scratch = [None] * self.RING
 
-    def _buffers(self, n: int):
+    def _buffers(self, n: int) -> _Buffers:
         i = self._turn
         self._turn = (i + 1) % self.RING
         b = self._ring[i]
-        if b is None or b[0].numel() < n:
-            cap = max(64, n)
-            b = (torch.empty(cap, dtype=torch.int32, device=self.device),
-                 torch.empty(cap, dtype=torch.float32, device=self.device),
-                 torch.empty(cap, dtype=torch.float32, pin_memory=True),
-                 torch.empty(cap, dtype=torch.int32, pin_memory=True))
-            self._ring[i] = b
-        return b[0][:n], b[1][:n], b[2][:n], b[3][:n]
+        if b is None or b.rows < n:
+            b = self._ring[i] = _Buffers(max(64, n), self.device)
+        return b
 
     def choose_async(self, logits: torch.Tensor, sequences: Sequence[int], drawn: Sequence[int]) -> Chosen:
         """logits: float32 [n, vocab] on the GPU. sequences[i], drawn[i]: the keys of
-        row i's random number. Nothing here waits for the GPU."""
+        row i's random number. Nothing here waits for the GPU, but for a choice of more rows than a buffer has
+        room for while the one that it replaces is still in flight."""
         n = logits.shape[0]
-        out, u_dev, u_host, out_host = self._buffers(n)
+        b = self._buffers(n)
+        out, u_dev, out_host = b.device[:n], b.uniform[:n], b.host[:n]
         if self.args.greedy:
             kernels.argmax(logits, out)
             out_host.copy_(out, non_blocking=True)
@@ -76,23 +99,21 @@ class Sampler:
             u = [uniform(self.seed, s, d) for s, d in zip(sequences, drawn)]
             k = self.args.top_k if self.args.top_k is not None else logits.shape[1]
             need = kernels.sample_scratch(n, logits.shape[1], int(k), float(self.args.top_p))
-            i = (self._turn - 1) % self.RING              # of the buffers just taken
-            if need and (self._scratch[i] is None or self._scratch[i].numel() < need):
-                self._scratch[i] = torch.empty(need, dtype=torch.uint8, device=self.device)
+            if need and (b.scratch is None or b.scratch.numel() < need):
+                b.scratch = torch.empty(need, dtype=torch.uint8, device=self.device)
             if need and len(u) == n <= kernels.SAMPLE_GIVEN_ROWS and logits.data_ptr() % 16 == 0 \
                     and logits.stride(0) % 4 == 0:
                 # the numbers go with the launch, the tokens come back from the kernel that draws them
                 kernels.sample_given(logits, u, u_dev, out, out_host, float(self.args.temperature), int(k),
-                                     float(self.args.top_p), self._scratch[i])
+                                     float(self.args.top_p), b.scratch)
             else:
+                u_host = b.uniform_host[:n]
                 u_host.numpy()[:] = np.asarray(u, dtype=np.float32)
                 u_dev.copy_(u_host, non_blocking=True)
                 kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
-                               float(self.args.top_p), self._scratch[i] if need else None)
+                               float(self.args.top_p), b.scratch if need else None)
                 out_host.copy_(out, non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record()
-        return Chosen(out, out_host, ev)
+        return Chosen(b, n)
 
     def choose(self, logits: torch.Tensor, sequences: Sequence[int], drawn: Sequence[int]):
         """As ``choose_async``, returning the chosen tokens as a list of ints."""
