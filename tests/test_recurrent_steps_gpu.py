@@ -60,9 +60,10 @@ def test_heads_that_a_step_takes_and_refuses():
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("geom", [(2, 64, 4), (3, 128, 1), (1, 256, 4), (2, 320, 2)])
-@pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [2, 1, 5], [1] * 17, [3, 250]])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [2, 1, 5], [1] * 17, [3, 250], [2, 0], [0, 2, 1], [1] * 16 + [0, 2]])
 def test_gates_of_few_tokens(lens, geom, dtype):
-    """Blocks of whole 64 inputs, against the formulas in 64 bits: sums of ``size`` products of order 1 / sqrt(size)."""
+    """Blocks of whole 64 inputs, against the formulas in 64 bits: sums of ``size`` products of order 1 / sqrt(size). As many
+    tokens as sequences, too, where a sequence brings none and another two."""
     from transformer_amd import kernels as K
     nb, size, taps = geom
     C, nt, B = nb * size, sum(lens), len(lens)
@@ -80,6 +81,8 @@ def test_gates_of_few_tokens(lens, geom, dtype):
     x, w = yx[:, C:].double() + xb.double(), gw.double()
     for i in range(B):
         rows = torch.cat([mem[slots[i]].double(), x[cu[i]:cu[i + 1]]])
+        if not lens[i]:
+            continue
         u = torch.stack([cb.double() + (rows[t:t + taps] * tp.double().T).sum(0) for t in range(lens[i])])
         ub = u.view(-1, nb, size)
         r, g = (torch.sigmoid(torch.einsum("tbi,boi->tbo", ub, w[z * nb:(z + 1) * nb]) + gb[z * nb:(z + 1) * nb].double()).reshape(-1, C)

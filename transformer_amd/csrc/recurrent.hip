@@ -264,9 +264,9 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
     const float* __restrict__ gates_b, const float* __restrict__ lam, float c0,
     const int* __restrict__ cu_q, const int* __restrict__ slots, int batch, int nt, int C, int nb,
     float* __restrict__ a_out, float* __restrict__ b_out) {
-  extern __shared__ float u[];                 // [TT][bs]
+  extern __shared__ __attribute__((aligned(16))) float u[];      // [TT][bs], read four at a time
   const int K = TAPS ? TAPS : K_;
-  __shared__ int s_start[TT], s_slot[TT];
+  __shared__ int s_start[TT], s_slot[TT], s_single;
   __shared__ float s_sum[2 * RGF_OC][TT];
   const int bs = C / nb, tiles = bs / RGF_OC;
   const int blk = blockIdx.y / tiles, o0 = (blockIdx.y % tiles) * RGF_OC, t0 = blockIdx.x * TT;
@@ -277,13 +277,25 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
   for (int j = 0; j < 4; ++j) wr[j] = *reinterpret_cast<const RgRun<TW>*>(w + (64 * j < bs ? 64 * j : 0));
   if (threadIdx.x < TT) {
     const int t = t0 + threadIdx.x < nt ? t0 + threadIdx.x : nt - 1;
-    const int b = nt == batch ? t : seq_of_token_r(cu_q, batch, t);      // (no sequence brings none)
-    s_start[threadIdx.x] = nt == batch ? t : cu_q[b];
-    s_slot[threadIdx.x] = slots[b];
+    int start = t, slot = 0;
+    bool alone = false;                        // as many tokens as sequences may still be two of one and none of another
+    if (nt == batch) {
+      slot = slots[t];
+      alone = (cu_q[t] == t) & (cu_q[t + 1] == t + 1);
+    }
+    if (!alone) {
+      const int b = seq_of_token_r(cu_q, batch, t);
+      start = cu_q[b];
+      slot = slots[b];
+    }
+    s_start[threadIdx.x] = start;
+    s_slot[threadIdx.x] = slot;
+    const int all = __all(alone);
+    if (threadIdx.x == 0) s_single = all;
   }
   __syncthreads();
   // (a token past the step's end computes what the last one does)
-  if (nt == batch) {                           // single tokens: all taps but the last fall into the sequence's memory
+  if (__builtin_amdgcn_readfirstlane(s_single)) {      // single tokens: all taps but the last fall into the sequence's memory
 #pragma unroll 4
     for (int idx = threadIdx.x; idx < TT * bs; idx += 256) {
       const int tt = idx / bs, c = blk * bs + idx % bs, t = t0 + tt < nt ? t0 + tt : nt - 1;
