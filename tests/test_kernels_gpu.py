@@ -706,6 +706,34 @@ def test_float32_attention_of_sequences_that_bring_no_token(counts):
         assert torch.equal(step(list(range(B)), ws), want)
 
 
+def test_float32_attention_of_a_position_behind_the_page_table():
+    """Keys count as far as the table is wide: the softmax over its pages in 64 bits, and no partial row behind the scratch that
+    the width asks for, with many more positions than that (two sequences, a table of 2 pages)."""
+    from transformer_amd import kernels
+    own = np.random.default_rng(5)
+    nh, nkv, dh = 4, 2, 64
+    kc, vc = own.normal(size=(4, nkv, 64, dh)), own.normal(size=(4, nkv, dh, 64))
+    table, pos, q = own.permutation(4).reshape(2, 2), [5000, 100], own.normal(size=(2, nh * dh))
+    taken = []
+
+    class Room:
+        def take(self, name, shape, dtype):
+            taken.append((torch.full((shape[0] + 4096,), 3.0, dtype=dtype, device=DEV), shape[0]))
+            return taken[-1][0][:shape[0]]
+
+    out = torch.full((2, nh * dh), float("nan"), device=DEV)
+    kernels.attention_generic(dev(q), out, dev(kc), dev(vc), dev(table, torch.int32), dev([0, 1, 2], torch.int32),
+                              dev(pos, torch.int32), 1, nh, nkv, dh, 0.125, None, Room())
+    scratch, n = taken[0]
+    assert (scratch[n:] == 3.0).all()
+    for b in range(2):
+        live = min(pos[b] + 1, 128)
+        for h in range(nh):
+            k, v = (np.concatenate([c[i, h // 2] if c is kc else c[i, h // 2].T for i in table[b]])[:live] for c in (kc, vc))
+            w = np.exp(k @ q[b, h * dh:(h + 1) * dh] * 0.125)
+            np.testing.assert_allclose(out[b, h * dh:(h + 1) * dh].cpu(), w @ v / w.sum(), atol=2e-5)
+
+
 # more pages than workgroups a row, so that each walks several: even and uneven turns, pages outside a window in between, heads
 # of two tiles of 16, widths that leave a wave without value columns
 @pytest.mark.parametrize("nh,nkv,dk,dv,B,most,opt", [(8, 4, 128, 128, 40, 1300, {}), (4, 4, 64, 64, 34, 1600, {"window": 300, "keep_first": 70}),

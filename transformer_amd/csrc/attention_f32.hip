@@ -266,7 +266,9 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
   const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE, r = lane % 16, kb = lane / 16;
   const int end = p.pos0[b] + 1;
   const Span see = {ta_first_key(end, p.window, p.chunk), end, p.keep};
-  if ((int)blockIdx.z * 64 >= end) return;
+  // no page behind the table's width, which the joining kernel goes by and which p.parts has room for
+  const int pages = (end + 63) / 64 < p.max_blocks ? (end + 63) / 64 : p.max_blocks;
+  if ((int)blockIdx.z >= pages) return;
   if (p.cu_q[b + 1] == p.cu_q[b]) return;          // a sequence that brings no token has no row
   constexpr int OWN = NB / 4;                      // blocks of value columns a wave owns
   const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
 #pragma unroll
   for (int d = 0; d < NB; ++d)
     if (EXACT || d < nkb) qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
-  for (int page = blockIdx.z, turn = 0; page * 64 < end; page += gridDim.z) {
+  for (int page = blockIdx.z, turn = 0; page < pages; page += gridDim.z) {
     if (!see.page(page)) continue;
     const size_t at = ((size_t)p.table[(size_t)b * p.max_blocks + page] * p.nkv + kvh) * 64;
     const float *kp = p.k + (at + 16 * wave + r) * p.dh, *vp = p.v + at * p.dv;
