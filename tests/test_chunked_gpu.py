@@ -144,3 +144,88 @@ def test_a_later_tokens_values_reach_no_earlier_one(bad):
         assert torch.allclose(o[:at], clean[:at], rtol=1e-5, atol=1e-5)
         assert not torch.isfinite(o[at, 0]).all()
         assert torch.allclose(o[:, 1], clean[:, 1], rtol=1e-5, atol=1e-5)
+
+
+def _f32_walk(q, k, v, a, S, bonus=None):
+    """The walk token by token in float32 (one sequence): readouts and the last state."""
+    out = torch.empty(q.shape[0], q.shape[1], v.shape[2], device=DEV)
+    for t in range(q.shape[0]):
+        kv = k[t, :, :, None] * v[t, :, None]
+        before, S = S, torch.addcmul(kv, a[t, :, :, None], S)
+        out[t] = ((S if bonus is None else torch.addcmul(before, bonus[:, :, None], kv)) * q[t, :, :, None]).sum(1)
+    return out, S
+
+
+def _off(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("fade", [0.02, 0.5, 3.0])
+@pytest.mark.parametrize("kind", ["channel", "bonus"])
+def test_chunks_are_no_further_off_than_a_walk_in_32_bits(kind, fade):
+    """Decays that last for hundreds of tokens, for tens and for a few. The products of a chunk's decays must not add up their
+    roundings, nor may a readout be one chain over its channels: either doubles the error. What a chunk adds is one rounding
+    of every decayed key, 2.5e-8 of it on average (2^-24 / sqrt(6)), which the walk of a state that soon forgets has not. A
+    tenth is left for chance (the readout has 500 x 8 x 128 numbers)."""
+    from transformer_amd import kernels as K
+    H, d, n, rank = 8, 128, 500, 4
+    g = torch.Generator(device=DEV).manual_seed(int(100 * fade))
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    state, decay, o = r(1, H, d, d), torch.empty(n, H * d, device=DEV), torch.empty(1, n, H, d, device=DEV)
+    first, args = state[0].clone(), (_t([0, n], torch.int32), _t([0], torch.int32))
+    if kind == "channel":                        # log sigmoid(z) / 1: about -fade
+        proj = r(n, 4 * H * d + rank).bfloat16()
+        z = 0.3 * r(H * d) - np.log(np.expm1(fade))
+        K.gla_recurrent(proj, H, d, d, rank, 0.1 * r(H * d, rank).bfloat16(), z, 1.0, state, *args, o, decay)
+        q, k, v = (x.float().view(n, H, d) for x in proj[:, :3 * H * d].split(H * d, 1))
+        q, u = q * d ** -0.5, None
+    else:
+        rkv, u = r(3, n, H * d).bfloat16(), 0.5 * r(H, d)
+        K.wkv_recurrent(rkv, r(n, rank).bfloat16(), H, d, d, 0.1 * r(H * d, rank).bfloat16(), 0.3 * r(H * d) + np.log(fade), u,
+                        state, *args, o, decay)
+        q, k, v = (x.float().view(n, H, d) for x in rkv)
+    a = decay.view(n, H, d)
+    walked, last = _f32_walk(q, k, v, a, first, u)
+    want, end = _walk(*(x.double().cpu().numpy() for x in (q, k, v, a, first)), None if u is None else u.double().cpu().numpy())
+    want, end = _t(want, torch.float64), _t(end, torch.float64)
+    for got, walk, exact in ((o[0], walked, want), (state[0], last, end)):
+        assert _off(got, exact) <= 1.1 * (_off(walk, exact) ** 2 + 2.5e-8 ** 2) ** 0.5
+
+
+def test_matrix_memory_in_chunks_is_no_further_off_than_its_walk():
+    from transformer_amd import kernels as K
+    H, dk, dv, n = 8, 256, 512, 400
+    g = torch.Generator(device=DEV).manual_seed(7)
+    rows = torch.randn(n, 2 * H * dk + H * dv, generator=g, device=DEV).bfloat16()
+    keep, write = 1 - 0.1 * torch.rand(n, H, generator=g, device=DEV), torch.rand(n, H, generator=g, device=DEV)
+    q, k, v = (x.double().cpu().numpy().reshape(n, H, -1) for x in rows.split([H * dk, H * dk, H * dv], 1))
+    k = k * write.double().cpu().numpy()[:, :, None]
+    v = np.concatenate([v, np.ones((n, H, 1))], 2)                # the normaliser is a column of ones
+    want, end = _walk(q * dk ** -0.5, k, v, np.broadcast_to(keep.double().cpu().numpy()[:, :, None], (n, H, dk)), np.zeros((H, dk, dv + 1)))
+    want, end = _t(want, torch.float64), _t(end, torch.float64)
+    off = []
+    for lanes in (0, 16):
+        state, norm = torch.zeros(1, H, dk, dv, device=DEV), torch.zeros(1, H, dk, device=DEV)
+        o, den = torch.empty(n, H, dv, device=DEV), torch.empty(n, H, device=DEV)
+        K.memory_recurrent(rows, 0, H * dk, 2 * H * dk, dk ** -0.5, keep, write, state, norm, _t([0, n], torch.int32),
+                           _t([0], torch.int32), o, den, lanes=lanes)
+        off.append([_off(o, want[..., :dv]), _off(den, want[..., dv]), _off(state[0], end[..., :dv]), _off(norm[0], end[..., dv])])
+    assert all(a <= 1.1 * b for a, b in zip(*off)), off
+
+
+@pytest.mark.parametrize("column", ["key", "query"])
+def test_an_infinite_number_stays_infinite(column):
+    """Everything positive: sums that an infinite term enters are infinite, as the walk's are, and not undefined."""
+    from transformer_amd import kernels as K
+    H, d, n, rank, at = 2, 64, 60, 4, 21
+    g = torch.Generator(device=DEV).manual_seed(3)
+    proj = torch.rand(n, 4 * H * d + rank, generator=g, device=DEV) + 0.1
+    proj[at, (H * d if column == "key" else 0) + 5] = float("inf")
+    o, decay = torch.empty(2, n, H, d, device=DEV), torch.empty(n, H * d, device=DEV)
+    K.gla_recurrent(proj.bfloat16(), H, d, d, rank, torch.zeros(H * d, rank, device=DEV).bfloat16(), torch.ones(H * d, device=DEV), 2.0,
+                    torch.ones(1, H, d, d, device=DEV), _t([0, n], torch.int32), _t([0], torch.int32), o, decay)
+    inf = torch.zeros(n, H, dtype=torch.bool, device=DEV)
+    inf[at:, 0] = True if column == "key" else inf[at:, 0]
+    inf[at, 0] = True
+    got = o.sum(0)
+    assert (got[inf] == float("inf")).all() and torch.isfinite(got[~inf]).all()

@@ -5,19 +5,27 @@
 //     o_t = S^T (P_t q_t) + sum_{s <= t} A[t][s] v_s,   A[t][s] = sum_i q_t[i] k_s[i] prod_{s < u <= t} a_u[i]
 //     S'  = diag(P_16) S + sum_s (k_s prod_{u > s} a_u) v_s^T
 // which is two products of 16 x dk x dv and one of 16 x 16 x dv where the walk token by token has 16 updates one behind
-// the other. Every factor is a product of decays as the walk forms it (no logarithm, no quotient), so none overflows and a
-// decay of 0 is a decay of 0.
+// the other. Every factor is a product of decays (no logarithm, no quotient), so none overflows and a decay of 0 is a decay
+// of 0.
+//
+// Rounding: sixteen factors in a row add up sixteen roundings, which the walk spreads over S, and a readout that is one chain
+// over a head's channels is twice as far off as the walk's sum over lanes. So products of decays are carried in two numbers,
+// S takes in a chunk as one group of tokens before and one behind its own product, and readouts are chains of four added
+// in pairs. Relative errors against 64 bits, walk / chunks / chunks without that care, in 1e-7: readouts of 32 heads of
+// 128 x 128 1.16 / 1.09 / 2.16, their states 0.86 / 0.76 / 1.16; the bonus form of 64 x 64 0.89 / 0.87 / 1.61 and 0.54 / 0.55 /
+// 0.76; matrix memory of 256 x 512 1.18 / 1.15 / 2.16 and 0.89 / 0.82 / 1.13.
 //
 // A workgroup owns CT value columns of one (sequence, head). Eight waves prepare the next chunk (P_t q_t, the decayed
 // keys, A) on the vector ALU and leave it in LDS in the matrix instructions' order while the other waves, 16 columns each
 // (and half of the key channels where there are more than 128), take this chunk; the accumulators' layout of S is the
 // operands' layout of the readout, so S never leaves its registers.
 //
-// A chunk takes 2 to 5 us (1 to 8 sequences of 32 heads of 128 x 128), of which the matrix instructions need 1.8 at the
-// most: bound by the preparation's chain of reads from LDS, products and sums over lanes. The recurrence of 8 prompts of 176
-// to 653 tokens, 32 heads of 128 x 128: 754 -> 205 us, its norm 83 -> 48, since the readout is left whole; the matrix memory
-// of prompts of 1,386 and 1,557 tokens, 8 heads of 256 x 512: 746 -> 390. Half as many preparing waves 212 and 569;
-// reading a group of tokens ahead of the branches, for every wave, 10 to 30 % slower.
+// A chunk takes 4 to 8 us (1 to 8 sequences of 32 heads of 128 x 128), of which the matrix instructions need 1.8 at the
+// most: bound by the preparation's chain of reads from LDS, products and sums over
+// lanes. 8 x 656 tokens of 32 heads of 128 x 128, decays included: 829 us token by token, 336 in chunks (287 with products of
+// decays in one number), and the norm reads one plane of readouts instead of four; the matrix memory of 2 x 1,536 tokens, 8 heads of
+// 256 x 512: 730 -> 390. Half as many preparing waves cost 1.5 times as much; reading a group of tokens ahead of the branches, for
+// every wave, 10 to 30 % more.
 #include "chunked.h"
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -41,7 +49,8 @@ __device__ __forceinline__ ChRun<T, N> ch_load(const T* p, uint32_t off, int c, 
   return r;
 }
 
-// Where the piece of tokens 4 g .. + 3 lies in a row of 16 (rows of keys, values and A): sixteen lanes that ask for 16 bytes
+// Where the piece of tokens g, g + 4, g + 8, g + 12 lies in a row of 16 (rows of keys, values and A), so that the matrix
+// instructions take the tokens in their order, four at a time: sixteen lanes that ask for 16 bytes
 // each, of neighbouring rows and either of two pieces, meet every bank once.
 __device__ __forceinline__ int ch_place(int row, int g) {
   return 4 * (g ^ ((0x78 >> (2 * ((row >> 2) & 3))) & 3));       // rows in fours: 0, 2, 3, 1
@@ -49,6 +58,21 @@ __device__ __forceinline__ int ch_place(int row, int g) {
 
 // Where channel c of token t lies in a row of queries, for the same reason
 __device__ __forceinline__ int ch_query(int t, int c) { return (c & ~63) + 4 * (((c >> 2) & 15) ^ t) + (c & 3); }
+
+// x is formed here. (Sums of what the matrix instructions left would else be put off to where they are stored, and what they
+// are made of kept in registers until then.)
+__device__ __forceinline__ void ch_now(f32x4_t& x) { asm volatile("" : "+v"(x)); }
+
+// hi + lo, a product of decays to twice 24 bits, times one more. (A sum of hi and lo must not take the product along.)
+__device__ __forceinline__ void ch_fall(float& hi, float& lo, float d) {
+#pragma clang fp contract(off)
+  const float p = hi * d, e = fmaf(hi, d, -p);
+  lo = fmaf(lo, d, e);
+  hi = p;
+}
+// x times such a product, rounded once; xl is x, or 0 for an infinite x, which lo would turn into an undefined one
+__device__ __forceinline__ float ch_times(float x, float xl, float hi, float lo) { return fmaf(x, hi, xl * lo); }
+__device__ __forceinline__ float ch_finite(float x) { return fabsf(x) < INFINITY ? x : 0.f; }
 
 // VEC: known when the kernel is chosen, since a load inside a branch is waited for where the branch ends
 template <typename T, int DK, int CT, int MODE, bool VEC>
@@ -140,24 +164,28 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
     // denominators of the chunk that the other waves work on
     auto normalise = [&](int c) {
       const int cur = c & 1, nxt = cur ^ 1;
-      float d = ig < 16 ? s_a[cur][tt][ig] : 0.f;  // (a row's sum: its pieces lie in another order)
+      float d = 0.f;
 #pragma unroll
       for (int r = 0; r < RUNS; ++r) {
         const run_t x = *(const run_t*)&s_q[cur][tt][ch_query(tt, chan(r))], y = *(const run_t*)&s_n[cur][chan(r)];
+        float run = x[0] * y[0];
 #pragma unroll
-        for (int e = 0; e < RN; ++e) d = fmaf(x[e], y[e], d);
+        for (int e = 1; e < RN; ++e) run = fmaf(x[e], y[e], run);
+        d += run;
       }
+      if (ig < 16) d += s_a[cur][tt][ig];          // (a row's sum: its pieces lie in another order)
       float none = 0.f;
       ta_sums2<32>(d, none);
       const int t = start + TA_CHUNK * c + tt;
       if (ig == 0 && t < end) p.den_out[(size_t)t * p.H + h] = d;
       if (tid < DK) {
-        n *= s_p[cur][0];
+        float keys[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const f32x4_t x = *(const f32x4_t*)&s_k[cur][tid][4 * g];
-          n += (x[0] + x[1]) + (x[2] + x[3]);
+          keys[g] = (x[0] + x[1]) + (x[2] + x[3]);
         }
+        n = fmaf(n, s_p[cur][0], (keys[0] + keys[1]) + (keys[2] + keys[3]));
         s_n[nxt][tid] = n;
       }
     };
@@ -171,15 +199,19 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
       bool odd = false;
 #pragma unroll
       for (int j = 0; j < VC; ++j) {
-        s_v[at][ig * VC + j][ch_place(ig * VC + j, tt / 4) + tt % 4] = vf[j];
+        s_v[at][ig * VC + j][ch_place(ig * VC + j, tt % 4) + tt / 4] = vf[j];
         odd |= !(fabsf(vf[j]) < INFINITY);
       }
       const bool any = __any(odd);
       if (lane == 0) s_odd[at][wave] = any;
-      // r: the product of the decays up to token tt, from there on the key and what the later tokens leave of it
-      float r[PC], dq[PC], acc[16], fall[SCALAR ? 16 : 1], rs = 1.f, ps = 1.f;
+      // r + rl: the product of the decays up to token tt, from there on what the later tokens leave of the key
+      float kl[SCALAR ? 1 : PC], r[PC], rl[PC], dq[PC], acc[16], fall[SCALAR ? 16 : 1], rs = 1.f, rsl = 0.f, ps = 1.f;
 #pragma unroll
-      for (int j = 0; j < PC; ++j) r[j] = 1.f;
+      for (int j = 0; j < PC; ++j) {
+        if (!SCALAR) kl[SCALAR ? 0 : j] = ch_finite(kf[j]);
+        r[j] = 1.f;
+        rl[j] = 0.f;
+      }
 #pragma unroll
       for (int t = 0; t < 16; ++t) acc[t] = 0.f;
       f32x4_t da[SCALAR ? 4 : 1];
@@ -195,14 +227,14 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
           for (int e = 0; e < 2; ++e) {
             const int t = 2 * bq + e;
             if (SCALAR) {
-              rs *= da[SCALAR ? t / 4 : 0][t % 4];
+              ch_fall(rs, rsl, da[SCALAR ? t / 4 : 0][t % 4]);
               fall[SCALAR ? t : 0] = 0.f;
             } else {
 #pragma unroll
               for (int x = 0; x < RUNS; ++x) {
                 const run_t d = *(const run_t*)&r_a[at][SCALAR ? 0 : t][chan(x)];
 #pragma unroll
-                for (int i = 0; i < RN; ++i) r[RN * x + i] *= d[i];
+                for (int i = 0; i < RN; ++i) ch_fall(r[RN * x + i], rl[RN * x + i], d[i]);
               }
             }
           }
@@ -212,10 +244,11 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
             const int t = 2 * bq + e;
             const bool mine = own == e;
             if (SCALAR) {
-              rs *= da[SCALAR ? t / 4 : 0][t % 4];
-              ps = mine ? rs : ps;                 // P_tt
+              ch_fall(rs, rsl, da[SCALAR ? t / 4 : 0][t % 4]);
+              ps = mine ? rs + rsl : ps;           // P_tt
               rs = mine ? 1.f : rs;
-              fall[SCALAR ? t : 0] = rs;
+              rsl = mine ? 0.f : rsl;
+              fall[SCALAR ? t : 0] = rs + rsl;
             }
 #pragma unroll
             for (int x = 0; x < RUNS; ++x) {
@@ -228,18 +261,19 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
                 if (SCALAR) {
                   dq[j] = mine ? qv[i] : dq[j];
                   acc[t] = fmaf(qv[i], kf[j], acc[t]);
-                } else if (BONUS) {
-                  dq[j] = mine ? qv[i] * r[j] : dq[j];
-                  acc[t] = fmaf(qv[i], mine ? u[BONUS ? j : 0] * kf[j] : r[j], acc[t]);
-                  const float f = r[j] * d[i];
-                  if (t == 15 && mine) s_p[at][chan(x) + i] = f;
-                  r[j] = mine ? kf[j] : f;
                 } else {
-                  const float f = r[j] * d[i];
-                  dq[j] = mine ? qv[i] * f : dq[j];
-                  if (t == 15 && mine) s_p[at][chan(x) + i] = f;
-                  r[j] = mine ? kf[j] : f;
-                  acc[t] = fmaf(qv[i], r[j], acc[t]);
+                  if (BONUS) {
+                    dq[j] = mine ? ch_times(qv[i], ch_finite(qv[i]), r[j], rl[j]) : dq[j];
+                    acc[t] = fmaf(qv[i], mine ? u[BONUS ? j : 0] * kf[j] : ch_times(kf[j], kl[SCALAR ? 0 : j], r[j], rl[j]), acc[t]);
+                  }
+                  ch_fall(r[j], rl[j], d[i]);
+                  if (!BONUS) {
+                    dq[j] = mine ? ch_times(qv[i], ch_finite(qv[i]), r[j], rl[j]) : dq[j];
+                    acc[t] = fmaf(qv[i], mine ? kf[j] : ch_times(kf[j], kl[SCALAR ? 0 : j], r[j], rl[j]), acc[t]);
+                  }
+                  if (t == 15 && mine) s_p[at][chan(x) + i] = r[j] + rl[j];
+                  r[j] = mine ? 1.f : r[j];
+                  rl[j] = mine ? 0.f : rl[j];
                 }
               }
             }
@@ -249,8 +283,8 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
           for (int e = 0; e < 2; ++e) {
             const int t = 2 * bq + e;
             if (SCALAR) {
-              rs *= da[SCALAR ? t / 4 : 0][t % 4];
-              fall[SCALAR ? t : 0] = rs;
+              ch_fall(rs, rsl, da[SCALAR ? t / 4 : 0][t % 4]);
+              fall[SCALAR ? t : 0] = rs + rsl;
             }
 #pragma unroll
             for (int x = 0; x < RUNS; ++x) {
@@ -262,12 +296,10 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
                 const int j = RN * x + i;
                 if (SCALAR) {
                   acc[t] = fmaf(qv[i], kf[j], acc[t]);
-                } else if (BONUS) {
-                  acc[t] = fmaf(qv[i], r[j], acc[t]);
-                  r[j] *= d[i];
                 } else {
-                  r[j] *= d[i];
-                  acc[t] = fmaf(qv[i], r[j], acc[t]);
+                  if (BONUS) acc[t] = fmaf(qv[i], ch_times(kf[j], kl[SCALAR ? 0 : j], r[j], rl[j]), acc[t]);
+                  ch_fall(r[j], rl[j], d[i]);
+                  if (!BONUS) acc[t] = fmaf(qv[i], ch_times(kf[j], kl[SCALAR ? 0 : j], r[j], rl[j]), acc[t]);
                 }
               }
             }
@@ -281,7 +313,7 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
         of = ig == t ? (SCALAR ? acc[t] * fall[SCALAR ? t : 0] : acc[t]) : of;
         of = ig == t + 1 ? (SCALAR ? acc[t + 1] * fall[SCALAR ? t + 1 : 0] : acc[t + 1]) : of;
       }
-      if (ig < 16) s_a[at][ig][ch_place(ig, tt / 4) + tt % 4] = ig >= tt ? of : 0.f;
+      if (ig < 16) s_a[at][ig][ch_place(ig, tt % 4) + tt / 4] = ig >= tt ? of : 0.f;
       if (SCALAR && tid == CH_PRODUCERS - 1) s_p[at][0] = ps;
 #pragma unroll
       for (int x = 0; x < RUNS; ++x) {
@@ -290,7 +322,7 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
         for (int i = 0; i < RN; ++i) {
           const int j = RN * x + i;
           y[i] = SCALAR ? dq[j] * ps : dq[j];
-          s_k[at][chan(x) + i][ch_place(chan(x), tt / 4) + tt % 4] = SCALAR ? kf[j] * rs : r[j];
+          s_k[at][chan(x) + i][ch_place(chan(x), tt % 4) + tt / 4] = SCALAR ? ch_times(kf[j], ch_finite(kf[j]), rs, rsl) : ch_times(kf[j], kl[SCALAR ? 0 : j], r[j], rl[j]);
         }
         *(run_t*)&s_q[at][tt][ch_query(tt, chan(x))] = y;
       }
@@ -339,37 +371,65 @@ __global__ __launch_bounds__(CH_PRODUCERS + CT / 16 * (DK > 128 ? 2 : 1) * TA_WA
   for (int c = 0; c < chunks; ++c) {
     const int cur = c & 1;
     const f32x4_t v = *(const f32x4_t*)&s_v[cur][16 * ct + m][piece];
-    f32x4_t o = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t o = zero;
+    // sixteen terms: four chains of four
+    auto dot = [&](const f32x4_t& x, const f32x4_t& y) {
+      f32x4_t c[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], y[j], zero, 0, 0, 0);
+      return (c[0] + c[1]) + (c[2] + c[3]);
+    };
     if (part == 0) {
       if (s_odd[cur][0] | s_odd[cur][1] | s_odd[cur][2] | s_odd[cur][3] | s_odd[cur][4] | s_odd[cur][5] | s_odd[cur][6] | s_odd[cur][7]) {
         // a later token's infinite or undefined value must not reach this token as 0 times it
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           for (int t = 0; t <= 4 * g + r; ++t)
-            o[r] = fmaf(s_a[cur][4 * g + r][ch_place(4 * g, t / 4) + t % 4], s_v[cur][16 * ct + m][ch_place(m, t / 4) + t % 4], o[r]);
+            o[r] = fmaf(s_a[cur][4 * g + r][ch_place(4 * g, t % 4) + t / 4], s_v[cur][16 * ct + m][ch_place(m, t % 4) + t / 4], o[r]);
       } else {
-        const f32x4_t a = *(const f32x4_t*)&s_a[cur][m][piece];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], v[j], o, 0, 0, 0);
+        o = dot(*(const f32x4_t*)&s_a[cur][m][piece], v);
       }
     }
+    // the tiles' sums in pairs, the pairs' in pairs: as short a chain as their number allows. The next tile's operands are on
+    // their way, no others: registers.
+    static_assert(TILES == 4 || TILES == 8, "fours of tiles");
+    auto query = [&](int i) { return *(const f32x4_t*)&s_q[cur][m][ch_query(m, row0 + 16 * i + 4 * g)]; };
+    f32x4_t x = query(0), pairs[2], fours = zero;
 #pragma unroll
     for (int i = 0; i < TILES; ++i) {
-      const f32x4_t q = *(const f32x4_t*)&s_q[cur][m][ch_query(m, row0 + 16 * i + 4 * g)];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (i % 2) o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j], S[i][j], o1, 0, 0, 0);
-        else o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j], S[i][j], o, 0, 0, 0);
+      const f32x4_t mine = x;
+      if (i + 1 < TILES) x = query(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4_t sum = dot(mine, S[i]);
+      ch_now(sum);
+      if (i % 2 == 0) pairs[i / 2 % 2] = sum;
+      else pairs[i / 2 % 2] += sum;
+      if (i % 4 == 3) {
+        const f32x4_t four = pairs[0] + pairs[1];
+        if (i < 4) fours = four;
+        else fours += four;
+        ch_now(fours);
       }
     }
-    o += o1;
+    o += fours;
+    auto key = [&](int i) { return *(const f32x4_t*)&s_k[cur][row0 + 16 * i + m][piece]; };
+    x = key(0);
+    f32x4_t P = s_p[cur][0];
 #pragma unroll
     for (int i = 0; i < TILES; ++i) {
-      const f32x4_t k = *(const f32x4_t*)&s_k[cur][row0 + 16 * i + m][piece];
-      if (SCALAR) S[i] *= s_p[cur][0];
-      else S[i] *= *(const f32x4_t*)&s_p[cur][SCALAR ? 0 : row0 + 16 * i + 4 * g];
+      const f32x4_t mine = x;
+      if (!SCALAR) P = *(const f32x4_t*)&s_p[cur][SCALAR ? 0 : row0 + 16 * i + 4 * g];
+      if (i + 1 < TILES) x = key(i + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      // the first eight tokens by themselves, then S, then the last eight: S that lasts is rounded nine times a chunk where
+      // the walk rounds it sixteen times, S that fades as the walk would
+      f32x4_t fresh = __builtin_amdgcn_mfma_f32_16x16x4f32(mine[0], v[0], zero, 0, 0, 0);
+      fresh = __builtin_amdgcn_mfma_f32_16x16x4f32(mine[1], v[1], fresh, 0, 0, 0);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], v[j], S[i], 0, 0, 0);
+      for (int r = 0; r < 4; ++r) S[i][r] = fmaf(S[i][r], P[r], fresh[r]);
+#pragma unroll
+      for (int j = 2; j < 4; ++j) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(mine[j], v[j], S[i], 0, 0, 0);
     }
     if (RS == 1) {
       store(c, o);
