@@ -51,6 +51,33 @@ def test_a_step_in_one_kernel_equals_its_kernels(geom, bonus, dtype, weights):
     assert torch.equal(s1[[2, 4]], first[[2, 4]])
 
 
+@pytest.mark.parametrize("geom", [(32, 128, 128), (16, 64, 64), (8, 256, 64), (8, 192, 64)])
+def test_a_step_in_one_kernel_is_no_further_off_than_its_kernels(geom):
+    """Against 64 bits, whole rows in float32; a twentieth for chance (64 x H x dv numbers)."""
+    from transformer_amd import kernels as K
+    H, dk, dv = geom
+    B, rank, n = 64, 16, H * dk
+    g = torch.Generator(device=DEV).manual_seed(dk)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    proj, a2, a2b, w, first = r(B, 2 * n + 2 * H * dv + rank), r(n, rank) / 4, 0.3 * r(n), 1 + 0.1 * r(dv), 3 * r(B, H, dk, dv)
+    cu, slots, at = _t(np.arange(B + 1), torch.int32), _t(np.arange(B), torch.int32), 2 * n + H * dv
+    out, alone = torch.empty(B, H * dv, device=DEV), torch.empty(B, H * dv, device=DEV)
+    o, alpha = torch.empty(K.gla_row_parts(dk), B, H, dv, device=DEV), torch.empty(B, n, device=DEV)
+    K.gla_step(proj, 0, n, 2 * n, proj[:, at + H * dv:], a2, a2b, 16.0, dk ** -0.5, None, first.clone(), slots,
+               proj[:, at:at + H * dv], w, 1e-5, out)
+    K.gla_recurrent(proj, H, dk, dv, rank, a2, a2b, 16.0, first.clone(), cu, slots, o, alpha)
+    K.gla_out(o, proj, H, dk, dv, w, 1e-5, alone)
+    x = proj.double()
+    q, k, v = (t.reshape(B, H, -1) for t in x[:, :at].split([n, n, H * dv], 1))
+    a = (torch.sigmoid(x[:, at + H * dv:] @ a2.double().T + a2b.double()) ** (1 / 16)).view(B, H, dk, 1)
+    y = ((a * first.double() + k[..., None] * v[:, :, None]) * q[..., None]).sum(2) * dk ** -0.5
+    y = y * torch.rsqrt((y * y).mean(-1, keepdim=True) + 1e-5) * w.double()
+    gate = x[:, at:at + H * dv]
+    want = y.reshape(B, -1) * gate * torch.sigmoid(gate)
+    off, walk = (float((t.double() - want).norm() / want.norm()) for t in (out, alone))
+    assert off <= 1.05 * walk
+
+
 def test_heads_that_a_step_takes_and_refuses():
     from transformer_amd import kernels as K
     takes = [(64, 64), (128, 128), (16, 64), (256, 64), (64, 256), (32, 32)]

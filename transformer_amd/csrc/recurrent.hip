@@ -1165,7 +1165,7 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(
       s_a[i] = mode == 1 ? expf(-expf(z)) : expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau);
   }
   __syncthreads();
-  float o[4] = {0.f, 0.f, 0.f, 0.f};
+  float o[4], pair[2][4] = {};
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = rg + rstep * i;
@@ -1175,10 +1175,12 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(
     for (int e = 0; e < 4; ++e) {
       const float kv = k * v[e], was = x[e];
       x[e] = fmaf(a, was, kv);
-      o[e] = fmaf(BONUS ? fmaf(u, kv, was) : x[e], q, o[e]);
+      pair[i / 2][e] = fmaf(BONUS ? fmaf(u, kv, was) : x[e], q, pair[i / 2][e]);
     }
     *reinterpret_cast<float4*>(st + (size_t)r * dv) = float4{x[0], x[1], x[2], x[3]};
   }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = pair[0][e] + pair[1][e];
   for (int d = groups; d < TA_WAVE; d <<= 1) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], d, TA_WAVE);
@@ -1187,8 +1189,18 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(
   __syncthreads();
   float y = 0.f;
   const int waves = threads / TA_WAVE;
-  if (tid < dv)
-    for (int i = 0; i < waves; ++i) y += s_o[i][tid];
+  if (tid < dv) {                              // (four sums side by side: one chain over 16 waves is further off)
+    float r[16], part[4];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r[i] = s_o[i][tid];           // (all at once; what no wave has written is not used)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      part[e] = e < waves ? r[e] : 0.f;
+#pragma unroll
+      for (int i = 4; i < 16; i += 4) part[e] += i + e < waves ? r[i + e] : 0.f;
+    }
+    y = (part[0] + part[1]) + (part[2] + part[3]);
+  }
   const float ss = wave_sum(y * y);
   if (tid % TA_WAVE == 0 && tid < dv) s_ss[tid / TA_WAVE] = ss;
   __syncthreads();
