@@ -295,7 +295,8 @@ extern "C" int ta_memory_recurrent(hipStream_t stream, int dtype, const void* pr
   // From a million numbers of state on the walk fills the CUs and is bound by its vector instructions; below, both are
   // chains of latencies, of which the walk's is the shorter (walk / chunks: 1 x 1,000 tokens of 8 heads of 256 x 512
   // 261 / 236 us, 4 x 300 236 / 116, 32 x 100 of 8 of 64 x 64 39 / 35, but 8 x 300 of those 47 / 59).
-  if (lanes == 0 && (long long)batch * H * dk * dv >= 1 << 20 && ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
+  // Float32 rows are walked, as everywhere (recurrent.hip).
+  if (lanes == 0 && dtype == TA_BF16 && (long long)batch * H * dk * dv >= 1 << 20 && ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
     const TaChunked c = {proj, stride, qoff, koff, voff, 1, qscale, nullptr, keep, nullptr, write, nullptr, state, cu_q, slots,
                          H, dk, dv, (size_t)nt * H * dv, 1, o_out, n_state, den_out, false};
     return ta_chunked_launch(stream, dtype, c, batch, "ta_memory_recurrent");

@@ -24,8 +24,9 @@
 //   attention variant that convolves its q, k and v.
 //
 // All state, decays, gates and sums are float32. Tokens are walked in order, except in long steps: `rglru_scan` scans
-// segments side by side and the matrix states go 16 tokens at a time (chunked.hip), counted from the step's first token, so
-// that a cut of the sequence into steps changes the order of 32-bit sums.
+// segments side by side, and the matrix states of bfloat16 rows go 16 tokens at a time (chunked.hip), counted from the step's
+// first token. There a cut of the sequence into steps, and who shares a step, change the order of 32-bit sums, as they change the
+// kernels of a bfloat16 engine's products; the matrix states and the gates of float32 rows keep their bits.
 #include "chunked.h"
 
 __device__ __forceinline__ int seq_of_token_r(const int* __restrict__ cu_q, int batch, int t) {
@@ -245,7 +246,8 @@ __global__ __launch_bounds__(256) void rglru_gates_tiled_kernel(
   }
 }
 
-// Few tokens: a workgroup owns 16 channels of a block (32 rows of the two gates) and TT tokens. Eight lanes share a row and
+// Few bfloat16 tokens (float32 ones keep to the tiles above, whose sums are the same for any number of tokens): a workgroup
+// owns 16 channels of a block (32 rows of the two gates) and TT tokens. Eight lanes share a row and
 // ask for its first 256 weights before anything else, so that the trip to memory runs beside the convolution of the block's
 // inputs, which every workgroup of the block forms for itself; sums over the lanes at the end. Bound by the latency of those
 // two: 8 single tokens of 16 blocks of 256 in bfloat16 (4 MB) 13.4 us, where the kernel above walks the block's inputs in
@@ -461,7 +463,7 @@ extern "C" int ta_rglru_gates(hipStream_t stream, int dtype, int wdtype, const v
   const int bsp = (bs + RGT_KC - 1) / RGT_KC * RGT_KC;
   const int few_tt = nt <= 4 ? 4 : nt <= 8 ? 8 : 16;
   const size_t lds_few = (size_t)few_tt * bs * sizeof(float);
-  if (nt <= RGF_MOST && bs % 64 == 0 && lds_few <= 60000 && (long long)nb * (bs / RGF_OC) <= 65535 && (uintptr_t)gates_w % 32 == 0) {
+  if (dtype == TA_BF16 && nt <= RGF_MOST && bs % 64 == 0 && lds_few <= 60000 && (long long)nb * (bs / RGF_OC) <= 65535 && (uintptr_t)gates_w % 32 == 0) {
     dim3 gf((nt + few_tt - 1) / few_tt, nb * (bs / RGF_OC));
 #define RGF_LAUNCH_K(T, TW, TT, TAPS)                                                                  \
   rglru_gates_few_kernel<T, TW, TT, TAPS><<<gf, 256, lds_few, stream>>>((const T*)yx, stride, xoff, xbias, taps, conv_bias, K, \
@@ -470,9 +472,8 @@ extern "C" int ta_rglru_gates(hipStream_t stream, int dtype, int wdtype, const v
   if (K == 4) RGF_LAUNCH_K(T, TW, TT, 4); else RGF_LAUNCH_K(T, TW, TT, 0)
 #define RGF_BY_TT(T, TW) \
   if (few_tt == 4) { RGF_LAUNCH(T, TW, 4); } else if (few_tt == 8) { RGF_LAUNCH(T, TW, 8); } else { RGF_LAUNCH(T, TW, 16); }
-    if (dtype == TA_F32 && wdtype == TA_F32) { RGF_BY_TT(float, float); }
-    else if (dtype == TA_BF16 && wdtype == TA_BF16) { RGF_BY_TT(bf16_t, bf16_t); }
-    else if (dtype == TA_BF16 && wdtype == TA_F32) { RGF_BY_TT(bf16_t, float); }
+    if (wdtype == TA_BF16) { RGF_BY_TT(bf16_t, bf16_t); }
+    else if (wdtype == TA_F32) { RGF_BY_TT(bf16_t, float); }
     else return ta_fail("ta_rglru_gates: unsupported dtypes %d / %d", dtype, wdtype);
 #undef RGF_BY_TT
 #undef RGF_LAUNCH
@@ -915,8 +916,9 @@ static int gla_recurrent_launch(hipStream_t stream, int dtype, int wdtype, const
   const bool few = nt <= 8 * batch;         // at most 8 tokens a sequence on average: the walk in short turns
   TA_REQUIRE(planes == parts || planes == recurrence_planes(head_decay || tok_decay, bonus, dk, nt, batch),
              "ta_gla_recurrent: a readout of %d planes", planes);
-  if (ta_chunked_long(nt, batch) && ta_chunked_takes(head_decay || tok_decay, bonus, dk)) {
-    const bool scalar = head_decay || tok_decay;
+  // float32 rows are walked unless the caller has no room for the walk's planes: their bits follow from their own sequence alone
+  const bool scalar = head_decay || tok_decay, walks = dtype == TA_F32 && planes == parts;
+  if (!walks && ta_chunked_long(nt, batch) && ta_chunked_takes(scalar, bonus, dk)) {
     const TaChunked c = {proj, stride, qoff, koff, voff, qk_share, qscale, scalar ? nullptr : alpha, tok_decay, head_decay,
                          tok_kscale, bonus, state, cu_q, slots, H, dk, dv, plane, planes, o_out, nullptr, nullptr, false};
     return ta_chunked_launch(stream, dtype, c, batch, "ta_gla_recurrent");

@@ -1361,9 +1361,13 @@ def gla_row_parts(key_dim: int) -> int:
     return int(library().ta_gla_row_parts(c_int(key_dim)))
 
 
-def recurrence_planes(key_dim: int, nt: int, batch: int, scalar_decay: bool = False, bonus: bool = False) -> int:
+def recurrence_planes(key_dim: int, nt: int, batch: int, scalar_decay: bool = False, bonus: bool = False,
+                      dtype: Optional[torch.dtype] = None) -> int:
     """Planes of a readout that the recurrences are given at least for a step of nt tokens: one where they go in chunks,
-    else ``gla_row_parts``."""
+    else ``gla_row_parts``. dtype: of the rows, when a layer asks what to take. Float32 rows are walked token by token in the
+    walk's planes, so that their bits do not depend on the step; in fewer they go in chunks too."""
+    if dtype == torch.float32:
+        return gla_row_parts(key_dim)
     return int(library().ta_recurrence_planes(c_int(int(scalar_decay)), c_int(int(bonus)), c_int(key_dim), c_int(nt),
                                               c_int(batch)))
 

@@ -4,9 +4,10 @@
 convolution (the recurrent block of De et al., "Griffin: Mixing Gated Linear Recurrences with
 Local Attention for Efficient Language Models"). ``GatedLinearAttention``: a matrix state per
 head with a decay per key channel. Both pass a sequence's state on from token to token (in long
-steps from segment to segment) in float32, so a cut of the sequence into steps changes the result by
-rounding alone; a step's products (the input
-and output projections) are the framework's usual ones.
+steps from segment to segment: of the diagonal recurrence always, of matrix states in a bfloat16 engine)
+in float32, so a cut of the sequence into steps changes the result by rounding at most, and a float32
+engine's matrix states by nothing; a step's products (the input and output projections) are the
+framework's usual ones.
 """
 from __future__ import annotations
 
@@ -97,7 +98,7 @@ class GatedLinearAttention(Part):
         s, nt = self.spec, h.shape[0]
         H, dk, dv = s.num_heads, s.key_dim, s.value_dim
         proj = linear(h, self.w["in.weight"], ctx.ws.take("gla.in", (nt, self.width), self.dtype))
-        if ctx.all_single and kernels.gla_step_fits(dk, dv):
+        if ctx.all_single and self.dtype == torch.bfloat16 and kernels.gla_step_fits(dk, dv):
             gates = 2 * H * dk + H * dv
             g = kernels.gla_step(proj, 0, H * dk, 2 * H * dk, proj[:, gates + H * dv:], self.w["decay.weight"],
                                  self.w["decay.bias"], float(s.tau), float(dk) ** -0.5, None, cache.layer_state(layer),
@@ -106,7 +107,8 @@ class GatedLinearAttention(Part):
             return linear_delta(g, self.w["out.weight"], ctx.ws, "gla.delta"), None
         o = kernels.gla_recurrent(proj, H, dk, dv, s.rank, self.w["decay.weight"], self.w["decay.bias"],
                                   float(s.tau), cache.layer_state(layer), ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("gla.o", (kernels.recurrence_planes(dk, nt, ctx.batch), nt, H, dv), torch.float32),
+                                  ctx.ws.take("gla.o", (kernels.recurrence_planes(dk, nt, ctx.batch, dtype=self.dtype), nt, H, dv),
+                                              torch.float32),
                                   ctx.ws.take("gla.alpha", (nt, H * dk), torch.float32))
         g = kernels.gla_out(o, proj, H, dk, dv, self.w["norm.weight"], float(s.eps),
                             ctx.ws.take("gla.gated", (nt, H * dv), self.dtype))
@@ -160,15 +162,15 @@ class BonusRecurrence(Part):
             for i in range(4):
                 linear(mixed[i], w[i], rkvg[i])
         low = linear(mixed[4], self.w["w1.weight"], ctx.ws.take("bonus.low", (nt, s.decay_rank), self.dtype))
-        if ctx.all_single and kernels.gla_step_fits(dk, dk):
+        if ctx.all_single and self.dtype == torch.bfloat16 and kernels.gla_step_fits(dk, dk):
             g = kernels.gla_step(rkvg[0], 0, nt * n, 2 * nt * n, low, self.w["w2.weight"], self.w["w0"], 1.0, 1.0,
                                  self.w["bonus"], state, ctx.slots, rkvg[3], self.w["norm.weight"], float(s.eps),
                                  ctx.ws.take("bonus.gated", (nt, n), self.dtype))
             return linear_delta(g, self.w["out.weight"], ctx.ws, "bonus.delta"), None
         o = kernels.wkv_recurrent(rkvg, low, H, dk, dk, self.w["w2.weight"], self.w["w0"], self.w["bonus"], state,
                                   ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("bonus.o", (kernels.recurrence_planes(dk, nt, ctx.batch, bonus=True), nt, H, dk),
-                                              torch.float32),
+                                  ctx.ws.take("bonus.o", (kernels.recurrence_planes(dk, nt, ctx.batch, bonus=True, dtype=self.dtype),
+                                                          nt, H, dk), torch.float32),
                                   ctx.ws.take("bonus.decay", (nt, n), torch.float32))
         g = kernels.head_norm_gate(o, rkvg[3], H, dk, self.w["norm.weight"], float(s.eps),
                                    ctx.ws.take("bonus.gated", (nt, n), self.dtype))
@@ -186,7 +188,7 @@ class DecayLinearAttention(Part):
     over all heads at once, with or without a weight; the gate's activation. The recurrence is
     the kernel of ``GatedLinearAttention`` with the head's constant in place of a decay per
     key channel and token: state, decays and readout stay float32, a cut
-    of the sequence changes the order of sums alone."""
+    of the sequence changes the order of sums at most (in a bfloat16 engine)."""
     graph_safe = True
 
     def __init__(self, spec, dtype, device):
@@ -240,8 +242,8 @@ class DecayLinearAttention(Part):
         o = kernels.decay_recurrent(proj, 0, self.nk, 2 * self.nk, H, dk, dv, self.decays, float(s.key_scale),
                                     cache.layer_state(layer), ctx.cu_q, ctx.slots,
                                     ctx.ws.take("decay_attention.o",
-                                                (kernels.recurrence_planes(dk, nt, ctx.batch, scalar_decay=True), nt, H, dv),
-                                                torch.float32))
+                                                (kernels.recurrence_planes(dk, nt, ctx.batch, scalar_decay=True, dtype=self.dtype),
+                                                 nt, H, dv), torch.float32))
         gate = proj[:, 2 * self.nk + self.nv:]
         gated = ctx.ws.take("decay_attention.gated", (nt, self.nv), self.dtype)
         if s.head_norm == "all_heads":
@@ -313,8 +315,8 @@ class StateSpace(Part):
         o = kernels.ssm_recurrent(xbc, 0, self.inner, self.inner + self.gn, H, s.groups, N, P, decay, dt,
                                   cache.layer_state(layer[0]), ctx.cu_q, ctx.slots,
                                   ctx.ws.take("state_space.o",
-                                              (kernels.recurrence_planes(N, nt, ctx.batch, scalar_decay=True), nt, H, P),
-                                              torch.float32))
+                                              (kernels.recurrence_planes(N, nt, ctx.batch, scalar_decay=True, dtype=self.dtype),
+                                               nt, H, P), torch.float32))
         y = kernels.gated_group_norm(o.view(o.shape[0], nt, self.inner), proj, 0, self.w["norm.weight"], float(s.eps),
                                      s.norm_groups, ctx.ws.take("state_space.y", (nt, self.inner), self.dtype),
                                      x=xbc, x_off=0, skip=self.w["D"], head_dim=P)
