@@ -229,3 +229,28 @@ def test_an_infinite_number_stays_infinite(column):
     inf[at, 0] = True
     got = o.sum(0)
     assert (got[inf] == float("inf")).all() and torch.isfinite(got[~inf]).all()
+
+
+@pytest.mark.parametrize("geom,lens,chunks", [((2, 64, 32), [23, 23, 24], False), ((2, 64, 32), [24, 24, 24], True), ((3, 128, 64), [190, 193], False),
+                                              ((3, 128, 64), [191, 193], True), ((3, 192, 64), [300], False), ((64, 192, 64), [40, 35], True),
+                                              ((95, 128, 64), [30, 29], False), ((96, 128, 64), [30, 29], True)])
+def test_both_sides_of_the_line_between_walk_and_chunks(geom, lens, chunks):
+    """Few long sequences and many heads: the planes say which it is; readouts and states against 64 bits either way."""
+    from transformer_amd import kernels as K
+    H, dk, dv = geom
+    nt, B = sum(lens), len(lens)
+    ask = dict(scalar_decay=True, dtype=torch.bfloat16, heads=H, value_dim=dv)
+    planes = K.recurrence_planes(dk, nt, B, **ask)
+    assert planes == (1 if chunks else K.gla_row_parts(dk)) and K.gla_row_parts(dk) > 1
+    assert K.recurrence_planes(dk, nt, B, **{**ask, "dtype": torch.float32}) == K.gla_row_parts(dk)
+    g = torch.Generator(device=DEV).manual_seed(H + dk)
+    rows = torch.randn(nt, 2 * H * dk + H * dv, generator=g, device=DEV).bfloat16()
+    first, d = torch.randn(B, H, dk, dv, generator=g, device=DEV), torch.rand(H, generator=g, device=DEV)
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    args, state, o = (_t(cu, torch.int32), _t(np.arange(B), torch.int32)), first.clone(), torch.full((planes, nt, H, dv), float("nan"), device=DEV)
+    K.decay_recurrent(rows, 0, H * dk, 2 * H * dk, H, dk, dv, d, 0.5, state, *args, o)
+    q, k, v = (x.double().cpu().numpy().reshape(nt, H, -1) for x in rows.split([H * dk, H * dk, H * dv], 1))
+    a = np.broadcast_to(d.double().cpu().numpy()[None, :, None], (nt, H, dk))
+    want = [_walk(*(x[cu[i]:cu[i + 1]] for x in (0.5 * q, k, v, a)), first[i].double().cpu().numpy()) for i in range(B)]
+    assert _off(o.sum(0), _t(np.concatenate([w[0] for w in want]), torch.float64)) <= 2e-6
+    assert _off(state, _t(np.array([w[1] for w in want]), torch.float64)) <= 2e-6

@@ -23,8 +23,7 @@ struct TaChunked {
 };
 
 #define TA_CHUNK 16
-// Steps that go in chunks: a chunk costs all of its 16 tokens, and the first one a start that a few tokens do not earn back
-// (32 heads of 128 x 128 with their decays: 1 x 40 tokens 33.2 us against 31.6 by the walk, 1 x 100 43 / 47, 8 x 12 28 / 54).
+// Steps that may go in chunks: a chunk costs all of its 16 tokens.
 static inline bool ta_chunked_long(int nt, int batch) { return nt > 48 && nt > 8 * batch; }
 
 bool ta_chunked_takes(bool scalar_decay, bool bonus, int dk);

@@ -873,11 +873,28 @@ __global__ __launch_bounds__(256) void gla_recurrent_kernel(
 
 extern "C" int ta_gla_row_parts(int dk) { return (dk + GLA_RT - 1) / GLA_RT; }
 
+// Whether a long step of bfloat16 rows is taken 16 tokens at a time. The walk's workgroups (32 key channels x 64 value columns)
+// are short chains that run side by side until they fill the CUs, from about 768 of them on every chunk gains: 4 x 20 tokens of 32 heads of
+// 128 x 128 26.4 us walked, 21.0 in chunks, of 16 heads 15.8 / 19.4; 8 x 60 of 16 heads 45.8 / 31.1, of 4 heads 21.7 / 25.4;
+// 32 x 20 of 4 heads of 200 x 64 20.5 / 18.2. With fewer it is one chain against the other: a chunk takes longer to start, and
+// less than 16 walked tokens with narrow keys (1 x 60 of 4 heads of 64 x 64 19.6 / 16.7, 4 x 20 with a decay per token 9.8 / 10.7), as long
+// with up to 128 channels (4 heads of 128 x 128, 1 x 100 32.1 / 33.0, 1 x 200 52.2 / 51.5, 4 x 150 41.8 / 44.3), longer with more (8
+// heads of 256 x 256 with a decay per token 1 x 200 47 / 51, 1 x 1,000 196 / 207).
+static bool chunks_pay(int nt, int batch, int H, int dk, int dv) {
+  const long long walks = (long long)batch * H * ((dk + GLA_RT - 1) / GLA_RT) * ((dv + GLA_CT - 1) / GLA_CT);
+  return walks >= 768 || (dk <= 128 && nt >= (long long)batch * (dk <= 64 ? 24 : 192));
+}
+
 // Planes that the recurrence's readout takes at least: chunks leave it whole.
 static int recurrence_planes(bool scalar_decay, bool bonus, int dk, int nt, int batch) {
   return ta_chunked_long(nt, batch) && ta_chunked_takes(scalar_decay, bonus, dk) ? 1 : ta_gla_row_parts(dk);
 }
 extern "C" int ta_recurrence_planes(int scalar_decay, int bonus, int dk, int nt, int batch) {
+  return recurrence_planes(scalar_decay != 0, bonus != 0, dk, nt, batch);
+}
+// Planes that it is best given.
+extern "C" int ta_recurrence_planes_of(int dtype, int scalar_decay, int bonus, int H, int dk, int dv, int nt, int batch) {
+  if (dtype == TA_F32 || !chunks_pay(nt, batch, H, dk, dv)) return ta_gla_row_parts(dk);
   return recurrence_planes(scalar_decay != 0, bonus != 0, dk, nt, batch);
 }
 
@@ -916,8 +933,8 @@ static int gla_recurrent_launch(hipStream_t stream, int dtype, int wdtype, const
   const bool few = nt <= 8 * batch;         // at most 8 tokens a sequence on average: the walk in short turns
   TA_REQUIRE(planes == parts || planes == recurrence_planes(head_decay || tok_decay, bonus, dk, nt, batch),
              "ta_gla_recurrent: a readout of %d planes", planes);
-  // float32 rows are walked unless the caller has no room for the walk's planes: their bits follow from their own sequence alone
-  const bool scalar = head_decay || tok_decay, walks = dtype == TA_F32 && planes == parts;
+  // with room for the walk's planes: float32 rows are walked, so that their bits follow from their own sequence alone
+  const bool scalar = head_decay || tok_decay, walks = planes == parts && (dtype == TA_F32 || !chunks_pay(nt, batch, H, dk, dv));
   if (!walks && ta_chunked_long(nt, batch) && ta_chunked_takes(scalar, bonus, dk)) {
     const TaChunked c = {proj, stride, qoff, koff, voff, qk_share, qscale, scalar ? nullptr : alpha, tok_decay, head_decay,
                          tok_kscale, bonus, state, cu_q, slots, H, dk, dv, plane, planes, o_out, nullptr, nullptr, false};

@@ -1362,12 +1362,14 @@ def gla_row_parts(key_dim: int) -> int:
 
 
 def recurrence_planes(key_dim: int, nt: int, batch: int, scalar_decay: bool = False, bonus: bool = False,
-                      dtype: Optional[torch.dtype] = None) -> int:
+                      dtype: Optional[torch.dtype] = None, heads: Optional[int] = None, value_dim: Optional[int] = None) -> int:
     """Planes of a readout that the recurrences are given at least for a step of nt tokens: one where they go in chunks,
-    else ``gla_row_parts``. dtype: of the rows, when a layer asks what to take. Float32 rows are walked token by token in the
-    walk's planes, so that their bits do not depend on the step; in fewer they go in chunks too."""
-    if dtype == torch.float32:
-        return gla_row_parts(key_dim)
+    else ``gla_row_parts``. With the rows' dtype, the heads and their value width: what a layer does best to give. Float32
+    rows are walked token by token, so that their bits do not depend on the step, and so are steps that chunks would not
+    make shorter; in fewer planes than the walk's they go in chunks all the same."""
+    if heads is not None:
+        return int(library().ta_recurrence_planes_of(c_int(_code(dtype)), c_int(int(scalar_decay)), c_int(int(bonus)), c_int(heads),
+                                                     c_int(key_dim), c_int(value_dim), c_int(nt), c_int(batch)))
     return int(library().ta_recurrence_planes(c_int(int(scalar_decay)), c_int(int(bonus)), c_int(key_dim), c_int(nt),
                                               c_int(batch)))
 

@@ -20,6 +20,12 @@ from .base import Part, PartError, register_part
 from .linear import adds_in_place, aligned_rows, finish, linear, linear_delta
 
 
+def _readout(ctx, name, dtype, nt, heads, key_dim, value_dim, **kind):
+    """The step's buffer [planes, nt, heads, value_dim] for a matrix recurrence's readout."""
+    planes = kernels.recurrence_planes(key_dim, nt, ctx.batch, dtype=dtype, heads=heads, value_dim=value_dim, **kind)
+    return ctx.ws.take(name, (planes, nt, heads, value_dim), torch.float32)
+
+
 class DiagonalRecurrence(Part):
     graph_safe = True
 
@@ -107,8 +113,7 @@ class GatedLinearAttention(Part):
             return linear_delta(g, self.w["out.weight"], ctx.ws, "gla.delta"), None
         o = kernels.gla_recurrent(proj, H, dk, dv, s.rank, self.w["decay.weight"], self.w["decay.bias"],
                                   float(s.tau), cache.layer_state(layer), ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("gla.o", (kernels.recurrence_planes(dk, nt, ctx.batch, dtype=self.dtype), nt, H, dv),
-                                              torch.float32),
+                                  _readout(ctx, "gla.o", self.dtype, nt, H, dk, dv),
                                   ctx.ws.take("gla.alpha", (nt, H * dk), torch.float32))
         g = kernels.gla_out(o, proj, H, dk, dv, self.w["norm.weight"], float(s.eps),
                             ctx.ws.take("gla.gated", (nt, H * dv), self.dtype))
@@ -169,8 +174,7 @@ class BonusRecurrence(Part):
             return linear_delta(g, self.w["out.weight"], ctx.ws, "bonus.delta"), None
         o = kernels.wkv_recurrent(rkvg, low, H, dk, dk, self.w["w2.weight"], self.w["w0"], self.w["bonus"], state,
                                   ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("bonus.o", (kernels.recurrence_planes(dk, nt, ctx.batch, bonus=True, dtype=self.dtype),
-                                                          nt, H, dk), torch.float32),
+                                  _readout(ctx, "bonus.o", self.dtype, nt, H, dk, dk, bonus=True),
                                   ctx.ws.take("bonus.decay", (nt, n), torch.float32))
         g = kernels.head_norm_gate(o, rkvg[3], H, dk, self.w["norm.weight"], float(s.eps),
                                    ctx.ws.take("bonus.gated", (nt, n), self.dtype))
@@ -241,9 +245,7 @@ class DecayLinearAttention(Part):
                                k_inplace=True)
         o = kernels.decay_recurrent(proj, 0, self.nk, 2 * self.nk, H, dk, dv, self.decays, float(s.key_scale),
                                     cache.layer_state(layer), ctx.cu_q, ctx.slots,
-                                    ctx.ws.take("decay_attention.o",
-                                                (kernels.recurrence_planes(dk, nt, ctx.batch, scalar_decay=True, dtype=self.dtype),
-                                                 nt, H, dv), torch.float32))
+                                    _readout(ctx, "decay_attention.o", self.dtype, nt, H, dk, dv, scalar_decay=True))
         gate = proj[:, 2 * self.nk + self.nv:]
         gated = ctx.ws.take("decay_attention.gated", (nt, self.nv), self.dtype)
         if s.head_norm == "all_heads":
@@ -314,9 +316,7 @@ class StateSpace(Part):
         kernels.ssm_steps(proj, self.inner + self.conv_width, H, self.w["dt_bias"], self.w["A_log"], dt, decay)
         o = kernels.ssm_recurrent(xbc, 0, self.inner, self.inner + self.gn, H, s.groups, N, P, decay, dt,
                                   cache.layer_state(layer[0]), ctx.cu_q, ctx.slots,
-                                  ctx.ws.take("state_space.o",
-                                              (kernels.recurrence_planes(N, nt, ctx.batch, scalar_decay=True, dtype=self.dtype),
-                                               nt, H, P), torch.float32))
+                                  _readout(ctx, "state_space.o", self.dtype, nt, H, N, P, scalar_decay=True))
         y = kernels.gated_group_norm(o.view(o.shape[0], nt, self.inner), proj, 0, self.w["norm.weight"], float(s.eps),
                                      s.norm_groups, ctx.ws.take("state_space.y", (nt, self.inner), self.dtype),
                                      x=xbc, x_off=0, skip=self.w["D"], head_dim=P)
