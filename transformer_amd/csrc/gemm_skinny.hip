@@ -76,16 +76,21 @@ union Frag16 {
 
 
 // COLS: columns of a workgroup, a multiple of 4 (a load brings four rows of W): 16, or what gives every CU one workgroup of
-// a weight that in tiles of 16 would leave some CUs with two (see skinny_cols).
-template <int WAVES, bool SWIGLU, bool TAIL, typename TC, bool SCALE, bool FOLD, int COLS = 16>
+// a weight that in tiles of 16 would leave some CUs with two (see skinny_cols). EXTRA: an activation behind the product, or
+// several products; the others do not carry the code (2,048 columns over k = 2,048 at 1 / 8 / 16 rows 4.46 / 4.88 / 5.30 us without,
+// 4.58 / 5.00 / 5.43 with it behind a flag).
+template <int WAVES, bool SWIGLU, bool TAIL, typename TC, bool SCALE, bool FOLD, int COLS = 16, bool EXTRA = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ A, int lda,
                                                                  const bf16_t* __restrict__ W, int ldw,
                                                                  const float* __restrict__ bias,
                                                                  TC* __restrict__ C, int ldc, int M,
                                                                  int n_out, int K, SkinnyNorm nm) {
-  A += blockIdx.y * nm.a_step;
-  W += blockIdx.y * nm.w_step;
-  C += blockIdx.y * nm.c_step;
+  if (EXTRA) {
+    A += blockIdx.y * nm.a_step;
+    W += blockIdx.y * nm.w_step;
+    C += blockIdx.y * nm.c_step;
+  }
+  static_assert(!EXTRA || !(SWIGLU || SCALE || FOLD), "not beside gates, a norm's factor or a fold");
   static_assert(COLS % 4 == 0 && COLS >= 16 && (COLS == 16 || (!SWIGLU && !FOLD)), "gates and folds go by tiles of 16");
   constexpr int NT = SWIGLU ? 2 : (COLS + 15) / 16;
   constexpr int SP = 16;       // partial sums of squares a thread asks for ahead of the product
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     for (int nt = 1; nt < NT; ++nt) {
       const int col = n + 16 * nt;
       if (16 * nt + (int)threadIdx.x % 16 < COLS && col < n_out) {
-        if (nm.act) v[nt] = skinny_act<TC>(nm, v[nt], m, col);
+        if (EXTRA && nm.act) v[nt] = skinny_act<TC>(nm, v[nt], m, col);
         C[(size_t)m * ldc + col] = from_f32<TC>(v[nt]);
       }
     }
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
     if (threadIdx.x % 16 == 0) nm.out_parts[(size_t)blockIdx.x * 16 + m] = sq;
     return;
   }
-  if (!SWIGLU && nm.act && col_ok) o = skinny_act<TC>(nm, o, m, n);
+  if (EXTRA && nm.act && col_ok) o = skinny_act<TC>(nm, o, m, n);
   if (col_ok) C[(size_t)m * ldc + n] = from_f32<TC>(o);
 }
 
@@ -291,7 +296,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
 // one barrier per tile is enough. SWIGLU: the walk alternates between the gate rows and the
 // up rows of a tile's columns, and the threads that sum a tile keep the gate value until
 // the up value arrives.
-template <int CPW, bool TAIL, bool SWIGLU, typename TC>
+template <int CPW, bool TAIL, bool SWIGLU, typename TC, bool ACT = false>
 __global__ __launch_bounds__(1024) void gemm_skinny_hold_kernel(const bf16_t* __restrict__ A, int lda,
                                                                 const bf16_t* __restrict__ W, int ldw,
                                                                 const float* __restrict__ bias,
@@ -409,7 +414,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_hold_kernel(const bf16_t* __
             gate = sum;
         } else {
           if (bias) sum += bias[n];
-          if (nm.act) sum = skinny_act<TC>(nm, sum, m, n);
+          if (ACT && nm.act) sum = skinny_act<TC>(nm, sum, m, n);
           C[(size_t)m * ldc + n] = from_f32<TC>(sum);
         }
       }
@@ -521,7 +526,9 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
   TA_REQUIRE(out_dtype == TA_BF16 || out_dtype == TA_F32, "ta_gemm_skinny_bf16: unknown output dtype %d", out_dtype);
   if (M == 0) return 0;
   const int tiles = (n_out + 15) / 16, chunks = (K + 127) / 128;
-  if (waves == 0 && !nm.X && count == 1 && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32) {
+  const bool hold = waves == 0 && !nm.X && count == 1 && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32;
+  const bool extra = nm.act != 0 || count > 1;
+  if (hold) {
     // about one workgroup per CU and round, at most eight tiles each
     const int steps = (swiglu ? 2 : 1) * tiles;
     const int rounds = (steps + 2047) / 2048;
@@ -530,11 +537,12 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
     const int cpw = chunks <= 16 ? 1 : 2;
     const bool tail = K % 128 != 0 || chunks != 16 * cpw;
     dim3 g((tiles + per - 1) / per), b(1024);
-#define HOLD_SW(CPW, TL, SW, TC)                                                                    \
-  gemm_skinny_hold_kernel<CPW, TL, SW, TC><<<g, b, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, \
+#define HOLD_SW(CPW, TL, SW, TC, AC)                                                                \
+  gemm_skinny_hold_kernel<CPW, TL, SW, TC, AC><<<g, b, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, \
                                                                 ldw, bias, (TC*)C, ldc, M, n_out, K, per, nm)
 #define HOLD(CPW, TL, TC) \
-  if (swiglu) HOLD_SW(CPW, TL, true, TC); else HOLD_SW(CPW, TL, false, TC)
+  if (swiglu) HOLD_SW(CPW, TL, true, TC, false); else if (extra) HOLD_SW(CPW, TL, false, TC, true); \
+  else HOLD_SW(CPW, TL, false, TC, false)
 #define HOLD_BY(TC)                                                  \
   if (cpw == 1) { if (tail) { HOLD(1, true, TC); } else { HOLD(1, false, TC); } } \
   else { if (tail) { HOLD(2, true, TC); } else { HOLD(2, false, TC); } }
@@ -548,12 +556,15 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
     const int cols = skinny_cols(n_out);
     if (cols != 16) {
       const dim3 gc((n_out + cols - 1) / cols);
-#define COLS_RUN(WV, TL, TC, SC, CO)                                                                                \
-  gemm_skinny_kernel<WV, false, TL, TC, SC, false, CO><<<gc, WV * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, \
+#define COLS_RUN(WV, TL, TC, SC, CO, EX)                                                                            \
+  gemm_skinny_kernel<WV, false, TL, TC, SC, false, CO, EX><<<gc, WV * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, \
                                                                                   bias, (TC*)C, ldc, M, n_out, K, nm)
-#define COLS_BY(TC, CO)                                                                                                \
-  if (K % 128 == 0) { if (nm.scale_parts) COLS_RUN(4, false, TC, true, CO); else COLS_RUN(4, false, TC, false, CO); } \
-  else { if (nm.scale_parts) COLS_RUN(4, true, TC, true, CO); else COLS_RUN(4, true, TC, false, CO); }
+#define COLS_TAIL(TL, TC, CO)                                             \
+  if (nm.scale_parts) COLS_RUN(4, TL, TC, true, CO, false);             \
+  else if (extra) COLS_RUN(4, TL, TC, false, CO, true);                 \
+  else COLS_RUN(4, TL, TC, false, CO, false)
+#define COLS_BY(TC, CO) \
+  if (K % 128 == 0) { COLS_TAIL(false, TC, CO); } else { COLS_TAIL(true, TC, CO); }
 #define COLS_TYPE(CO) \
   if (out_dtype == TA_BF16) { COLS_BY(bf16_t, CO) } else { COLS_BY(float, CO) }
       switch (cols) {
@@ -563,6 +574,7 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
       }
 #undef COLS_TYPE
 #undef COLS_BY
+#undef COLS_TAIL
 #undef COLS_RUN
       return ta_check_launch("ta_gemm_skinny_bf16 (a workgroup a CU)");
     }
@@ -590,17 +602,34 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
     case 8: LAUNCH(8, SW, TC); break;    \
     default: LAUNCH(16, SW, TC); break;  \
   }
+#define LAUNCH_X(WV, TL, TC)                                                                                        \
+  gemm_skinny_kernel<WV, false, TL, TC, false, false, 16, true><<<g, b, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, \
+                                                                                     bias, (TC*)C, ldc, M, n_out, K, nm)
+#define EXTRA_BY(WV, TC) \
+  if (K % 128 == 0) LAUNCH_X(WV, false, TC); else LAUNCH_X(WV, true, TC)
+#define EXTRA(TC)                           \
+  switch (waves) {                          \
+    case 4: EXTRA_BY(4, TC); break;         \
+    case 8: EXTRA_BY(8, TC); break;         \
+    default: EXTRA_BY(16, TC); break;       \
+  }
+  TA_REQUIRE(!extra || !(swiglu || nm.X || nm.scale_parts), "ta_gemm_skinny_bf16: an activation or several products beside gates, a fold or a scale");
   if (nm.X) {
     switch (waves) {
       case 4: LAUNCH_FOLD(4); break;
       case 8: LAUNCH_FOLD(8); break;
       default: LAUNCH_FOLD(16); break;
     }
+  } else if (extra) {
+    if (out_dtype == TA_BF16) { EXTRA(bf16_t) } else { EXTRA(float) }
   } else if (swiglu) {
     if (out_dtype == TA_BF16) { BY_WAVES(true, bf16_t) } else { BY_WAVES(true, float) }
   } else {
     if (out_dtype == TA_BF16) { BY_WAVES(false, bf16_t) } else { BY_WAVES(false, float) }
   }
+#undef EXTRA
+#undef EXTRA_BY
+#undef LAUNCH_X
 #undef BY_WAVES
 #undef LAUNCH_FOLD
 #undef LAUNCH
