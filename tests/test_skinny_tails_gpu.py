@@ -80,3 +80,15 @@ def test_a_workgroup_a_cu_has_the_bits_of_tiles_of_16(m, k, n, dtype):
         assert torch.equal(got[:, :n], want) and (got[:, n:] == 7).all()
     want = K.activation(K.gemm_skinny(a, w, torch.empty(m, n, dtype=dtype, device=DEV), waves=4), want, "relu2")
     assert torch.equal(K.gemm_skinny_act(a, w, torch.empty(m, n, dtype=dtype, device=DEV), "relu2"), want)
+
+
+@pytest.mark.parametrize("count,m,n,k", [(2, 16, 10240, 256), (3, 4, 10250, 2048), (2, 1, 10233, 4096), (2, 9, 10240, 4104)])
+def test_wide_products_in_one_call_have_the_bits_of_their_own(count, m, n, k):
+    """640 tiles of columns and more: each goes to the kernel that holds its rows, as it would alone; a k that it does not hold."""
+    from transformer_amd import kernels as K
+    a, w = _randn(14, count + 1, m, k)[:count], _randn(15, count, n, k)
+    out = torch.full((count, m, n + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    K.gemm_skinny_many(a, w, out[:, :, :n])
+    for i in range(count):
+        assert torch.equal(out[i, :, :n], K.gemm_skinny(a[i], w[i], torch.empty(m, n, dtype=torch.bfloat16, device=DEV)))
+    assert (out[:, :, n:] == 7).all()

@@ -526,7 +526,17 @@ static int skinny_launch(hipStream_t stream, int out_dtype, int swiglu, const vo
   TA_REQUIRE(out_dtype == TA_BF16 || out_dtype == TA_F32, "ta_gemm_skinny_bf16: unknown output dtype %d", out_dtype);
   if (M == 0) return 0;
   const int tiles = (n_out + 15) / 16, chunks = (K + 127) / 128;
-  const bool hold = waves == 0 && !nm.X && count == 1 && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32;
+  const bool hold = waves == 0 && !nm.X && (swiglu ? 2 : 1) * tiles >= 640 && chunks <= 32;
+  if (hold && count > 1) {
+    // so many columns fill the chip by themselves, and A is not read again with every tile: four products of 16,384 over
+    // k = 2,048 at 1 / 8 / 16 rows 50.8 / 51.2 / 53.2 us one after the other, 57.9 / 63.7 / 72.4 in one launch (10,240 over 4,096
+    // 64 / 67 / 72 and 58 / 63 / 78; 8,192 over 4,096, which is not held, 55 / 59 / 71 and 48 / 51 / 63)
+    for (int i = 0; i < count; ++i)
+      if (int rc = skinny_launch(stream, out_dtype, swiglu, (const bf16_t*)A + i * nm.a_step, lda, (const bf16_t*)W + i * nm.w_step, ldw,
+                                 bias, (char*)C + i * nm.c_step * (out_dtype == TA_BF16 ? 2 : 4), ldc, M, n_out, K, waves, nm))
+        return rc;
+    return 0;
+  }
   const bool extra = nm.act != 0 || count > 1;
   if (hold) {
     // about one workgroup per CU and round, at most eight tiles each
