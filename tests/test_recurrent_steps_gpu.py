@@ -86,11 +86,11 @@ def test_heads_that_a_step_takes_and_refuses():
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("geom", [(2, 64, 4), (3, 128, 1), (1, 256, 4), (2, 320, 2)])
+@pytest.mark.parametrize("geom", [(2, 64, 4), (3, 128, 1), (1, 256, 4), (2, 320, 2), (4, 640, 2)])
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1, 1, 1], [2, 1, 5], [1] * 17, [3, 250], [2, 0], [0, 2, 1], [1] * 16 + [0, 2]])
 def test_gates_of_few_tokens(lens, geom, dtype):
     """Blocks of whole 64 inputs, against the formulas in 64 bits: sums of ``size`` products of order 1 / sqrt(size). As many
-    tokens as sequences, too, where a sequence brings none and another two."""
+    tokens as sequences, too, where a sequence brings none and another two, and blocks so wide that 253 tokens go by the tiles."""
     from transformer_amd import kernels as K
     nb, size, taps = geom
     C, nt, B = nb * size, sum(lens), len(lens)

@@ -253,7 +253,16 @@ __global__ __launch_bounds__(256) void rglru_gates_tiled_kernel(
 // two: 8 single tokens of 16 blocks of 256 in bfloat16 (4 MB) 13.4 us, where the kernel above walks the block's inputs in
 // turns behind barriers on a quarter of the workgroups (49).
 #define RGF_OC 16
-#define RGF_MOST 256          // tokens of a step, from there on the tiles above (or the library, in bfloat16)
+// Up to 256 tokens (from there on the tiles, or the library). Every workgroup forms its block's inputs again, which wide blocks pay
+// for once the chip is full; lines by workgroups times block. us by the tiles / here, bfloat16: 16 blocks of 256 at 64 / 128 / 255 tokens
+// 44 / 59 / 95 and 26 / 52 / 82; 8 of 512 at 255 221 and 188; 4 of 640 at 128 / 160 / 192 123 / 129 / 125 and 103 / 144 / 150; 10 of 640 at
+// 64 125 and 143. Blocks that the tiles' LDS does not hold, by the kernel in front of those: 4 of 768 at 255 259 and 247, 4 of 896 at
+// 160 / 224 372 / 383 and 342 / 455.
+#define RGF_MOST 256
+static bool rglru_few_pays(int nt, int few_tt, int nb, int bs, bool tiled) {
+  if (nt > RGF_MOST) return false;
+  return bs <= 512 || (long long)((nt + few_tt - 1) / few_tt) * nb * (bs / RGF_OC) * bs <= (tiled ? 900000 : 2400000);
+}
 
 template <typename TW> struct alignas(8 * sizeof(TW)) RgRun { TW x[8]; };
 
@@ -266,7 +275,8 @@ __global__ __launch_bounds__(256) void rglru_gates_few_kernel(
     const float* __restrict__ gates_b, const float* __restrict__ lam, float c0,
     const int* __restrict__ cu_q, const int* __restrict__ slots, int batch, int nt, int C, int nb,
     float* __restrict__ a_out, float* __restrict__ b_out) {
-  extern __shared__ __attribute__((aligned(16))) float u[];      // [TT][bs], read four at a time
+  extern __shared__ __attribute__((aligned(16))) float few_u[];
+  float* u = few_u;                            // [TT][bs], read four at a time
   const int K = TAPS ? TAPS : K_;
   __shared__ int s_start[TT], s_slot[TT], s_single;
   __shared__ float s_sum[2 * RGF_OC][TT];
@@ -463,7 +473,10 @@ extern "C" int ta_rglru_gates(hipStream_t stream, int dtype, int wdtype, const v
   const int bsp = (bs + RGT_KC - 1) / RGT_KC * RGT_KC;
   const int few_tt = nt <= 4 ? 4 : nt <= 8 ? 8 : 16;
   const size_t lds_few = (size_t)few_tt * bs * sizeof(float);
-  if (dtype == TA_BF16 && nt <= RGF_MOST && bs % 64 == 0 && lds_few <= 60000 && (long long)nb * (bs / RGF_OC) <= 65535 && (uintptr_t)gates_w % 32 == 0) {
+  const size_t lds_tiled = ((size_t)RGT_TT * bsp + 2 * RGT_KC * RGT_OC) * sizeof(float);
+  const int tiles = (bs + RGT_OC - 1) / RGT_OC;
+  const bool tiled = lds_tiled <= 64000 && (long long)nb * tiles <= 65535;
+  if (dtype == TA_BF16 && rglru_few_pays(nt, few_tt, nb, bs, tiled) && bs % 64 == 0 && lds_few <= 60000 && (long long)nb * (bs / RGF_OC) <= 65535 && (uintptr_t)gates_w % 32 == 0) {
     dim3 gf((nt + few_tt - 1) / few_tt, nb * (bs / RGF_OC));
 #define RGF_LAUNCH_K(T, TW, TT, TAPS)                                                                  \
   rglru_gates_few_kernel<T, TW, TT, TAPS><<<gf, 256, lds_few, stream>>>((const T*)yx, stride, xoff, xbias, taps, conv_bias, K, \
@@ -480,9 +493,7 @@ extern "C" int ta_rglru_gates(hipStream_t stream, int dtype, int wdtype, const v
 #undef RGF_LAUNCH_K
     return ta_check_launch("ta_rglru_gates");
   }
-  const size_t lds_tiled = ((size_t)RGT_TT * bsp + 2 * RGT_KC * RGT_OC) * sizeof(float);
-  const int tiles = (bs + RGT_OC - 1) / RGT_OC;
-  if (lds_tiled <= 64000 && (long long)nb * tiles <= 65535) {
+  if (tiled) {
     dim3 gt((nt + RGT_TT - 1) / RGT_TT, nb * tiles);
 #define RGT_LAUNCH(T, TW)                                                                              \
   rglru_gates_tiled_kernel<T, TW><<<gt, 256, lds_tiled, stream>>>((const T*)yx, stride, xoff, xbias, taps, conv_bias, K, \
