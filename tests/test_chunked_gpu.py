@@ -254,3 +254,22 @@ def test_both_sides_of_the_line_between_walk_and_chunks(geom, lens, chunks):
     want = [_walk(*(x[cu[i]:cu[i + 1]] for x in (0.5 * q, k, v, a)), first[i].double().cpu().numpy()) for i in range(B)]
     assert _off(o.sum(0), _t(np.concatenate([w[0] for w in want]), torch.float64)) <= 2e-6
     assert _off(state, _t(np.array([w[1] for w in want]), torch.float64)) <= 2e-6
+
+
+def test_the_entry_without_planes_keeps_its_arguments():
+    """``ta_decay_recurrent`` takes the walk's planes and no number of them."""
+    from ctypes import c_float, c_int, c_void_p
+    from transformer_amd import kernels as K
+    H, d, n = 3, 64, 50
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rows, decays = torch.randn(n, 3 * H * d, generator=g, device=DEV).bfloat16(), torch.rand(H, generator=g, device=DEV)
+    cu, slots = _t([0, n], torch.int32), _t([0], torch.int32)
+    state, other = torch.zeros(1, H, d, d, device=DEV), torch.zeros(1, H, d, d, device=DEV)
+    o, want = torch.empty(2, n, H, d, device=DEV), torch.empty(2, n, H, d, device=DEV)
+    K.decay_recurrent(rows, 0, H * d, 2 * H * d, H, d, d, decays, 0.5, state, cu, slots, want)
+    p = lambda t: c_void_p(t.data_ptr())
+    rc = K.library().ta_decay_recurrent(K._stream(), c_int(K._code(rows.dtype)), p(rows), c_int(3 * H * d), c_int(0), c_int(H * d),
+                                        c_int(2 * H * d), p(decays), c_float(0.5), p(other), p(cu), p(slots), c_int(1), c_int(n),
+                                        c_int(H), c_int(d), c_int(d), p(o))
+    torch.cuda.synchronize()
+    assert rc == 0 and torch.equal(o, want) and torch.equal(state, other)

@@ -970,40 +970,65 @@ static int gla_recurrent_launch(hipStream_t stream, int dtype, int wdtype, const
   return ta_check_launch("ta_gla_recurrent");
 }
 
+extern "C" int ta_gla_recurrent_planes(hipStream_t stream, int dtype, int wdtype, const void* proj, int stride,
+                                       int qoff, int koff, int voff, int aoff, int rank, const void* a2,
+                                       const float* a2b, float inv_tau, float qscale, float* alpha, float* state,
+                                       const int* cu_q, const int* slots, int batch, int nt, int H, int dk, int dv,
+                                       int planes, float* o_out) {
+  return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, proj, stride, aoff, rank, a2,
+                              a2b, inv_tau, qscale, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 0,
+                              nullptr);
+}
+// With the walk's planes.
 extern "C" int ta_gla_recurrent(hipStream_t stream, int dtype, int wdtype, const void* proj, int stride,
                                 int qoff, int koff, int voff, int aoff, int rank, const void* a2,
                                 const float* a2b, float inv_tau, float qscale, float* alpha, float* state,
                                 const int* cu_q, const int* slots, int batch, int nt, int H, int dk, int dv,
-                                int planes, float* o_out) {
-  return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, proj, stride, aoff, rank, a2,
-                              a2b, inv_tau, qscale, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 0,
-                              nullptr);
+                                float* o_out) {
+  return ta_gla_recurrent_planes(stream, dtype, wdtype, proj, stride, qoff, koff, voff, aoff, rank, a2, a2b, inv_tau,
+                                 qscale, alpha, state, cu_q, slots, batch, nt, H, dk, dv, ta_gla_row_parts(dk), o_out);
 }
 
 // The recurrence with the readout before the update and a bonus for the current token (see
 // BONUS above) and the decay exp(-exp(a2 tanh(low) + a2b)) per key channel. q, k, v sit at
 // element offsets qoff, koff, voff of ``proj`` with ``stride`` elements between tokens (three
 // planes of one buffer, or three column ranges of its rows); low: [nt, rank] rows of their own.
+extern "C" int ta_wkv_recurrent_planes(hipStream_t stream, int dtype, int wdtype, const void* proj, int stride,
+                                       int qoff, int koff, int voff, const void* low, int low_stride, int rank,
+                                       const void* a2, const float* a2b, const float* bonus, float* alpha,
+                                       float* state, const int* cu_q, const int* slots, int batch, int nt, int H,
+                                       int dk, int dv, int planes, float* o_out) {
+  TA_REQUIRE(bonus != nullptr, "ta_wkv_recurrent: the bonus is required");
+  return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, low, low_stride, 0, rank, a2,
+                              a2b, 1.0f, 1.0f, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 1, bonus);
+}
+// With the walk's planes.
 extern "C" int ta_wkv_recurrent(hipStream_t stream, int dtype, int wdtype, const void* proj, int stride,
                                 int qoff, int koff, int voff, const void* low, int low_stride, int rank,
                                 const void* a2, const float* a2b, const float* bonus, float* alpha,
                                 float* state, const int* cu_q, const int* slots, int batch, int nt, int H,
-                                int dk, int dv, int planes, float* o_out) {
-  TA_REQUIRE(bonus != nullptr, "ta_wkv_recurrent: the bonus is required");
-  return gla_recurrent_launch(stream, dtype, wdtype, proj, stride, qoff, koff, voff, low, low_stride, 0, rank, a2,
-                              a2b, 1.0f, 1.0f, alpha, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 1, bonus);
+                                int dk, int dv, float* o_out) {
+  return ta_wkv_recurrent_planes(stream, dtype, wdtype, proj, stride, qoff, koff, voff, low, low_stride, rank, a2, a2b,
+                                 bonus, alpha, state, cu_q, slots, batch, nt, H, dk, dv, ta_gla_row_parts(dk), o_out);
 }
 
 // The recurrence with ONE fixed decay per head, S_t = decay_h S_{t-1} + k_t v_t^T, o_t = S_t^T
 // (qscale q_t): head_decay [H] float32 on the device; q, k, v at element offsets of the rows of
 // ``proj`` as above. No decay input, no scratch for decays.
-extern "C" int ta_decay_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int qoff, int koff,
-                                  int voff, const float* head_decay, float qscale, float* state, const int* cu_q,
-                                  const int* slots, int batch, int nt, int H, int dk, int dv, int planes, float* o_out) {
+extern "C" int ta_decay_recurrent_planes(hipStream_t stream, int dtype, const void* proj, int stride, int qoff, int koff,
+                                         int voff, const float* head_decay, float qscale, float* state, const int* cu_q,
+                                         const int* slots, int batch, int nt, int H, int dk, int dv, int planes, float* o_out) {
   TA_REQUIRE(head_decay != nullptr, "ta_decay_recurrent: the heads' decays are required");
   return gla_recurrent_launch(stream, dtype, dtype, proj, stride, qoff, koff, voff, nullptr, 0, 0, 0, nullptr,
                               nullptr, 1.0f, qscale, nullptr, state, cu_q, slots, batch, nt, H, dk, dv, planes, o_out, 0,
                               nullptr, head_decay);
+}
+// With the walk's planes.
+extern "C" int ta_decay_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int qoff, int koff,
+                                  int voff, const float* head_decay, float qscale, float* state, const int* cu_q,
+                                  const int* slots, int batch, int nt, int H, int dk, int dv, float* o_out) {
+  return ta_decay_recurrent_planes(stream, dtype, proj, stride, qoff, koff, voff, head_decay, qscale, state, cu_q, slots,
+                                   batch, nt, H, dk, dv, ta_gla_row_parts(dk), o_out);
 }
 
 // ------------------------------------------------------------------ gla: head norm and output gate
@@ -1587,14 +1612,22 @@ extern "C" int ta_ssm_steps(hipStream_t stream, int dtype, const void* proj, int
 // The recurrence S_t = decay_t S_{t-1} + dt_t B_t x_t^T, o_t = S_t^T C_t per head, with B and C shared
 // by the ``share`` heads of a group: the kernel of gated linear attention with q = C, k = B, v = x,
 // one decay per (token, head) and the step size as a factor on the key. decay, dt: [nt, H] float32.
-extern "C" int ta_ssm_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int coff, int boff,
-                                int xoff, int share, const float* decay, const float* dt, float* state,
-                                const int* cu_q, const int* slots, int batch, int nt, int H, int N, int P,
-                                int planes, float* o_out) {
+extern "C" int ta_ssm_recurrent_planes(hipStream_t stream, int dtype, const void* proj, int stride, int coff, int boff,
+                                       int xoff, int share, const float* decay, const float* dt, float* state,
+                                       const int* cu_q, const int* slots, int batch, int nt, int H, int N, int P,
+                                       int planes, float* o_out) {
   TA_REQUIRE(decay != nullptr && dt != nullptr, "ta_ssm_recurrent: decays and step sizes are required");
   return gla_recurrent_launch(stream, dtype, dtype, proj, stride, coff, boff, xoff, nullptr, 0, 0, 0, nullptr,
                               nullptr, 1.0f, 1.0f, nullptr, state, cu_q, slots, batch, nt, H, N, P, planes, o_out, 0,
                               nullptr, nullptr, share, decay, dt);
+}
+// With the walk's planes.
+extern "C" int ta_ssm_recurrent(hipStream_t stream, int dtype, const void* proj, int stride, int coff, int boff,
+                                int xoff, int share, const float* decay, const float* dt, float* state,
+                                const int* cu_q, const int* slots, int batch, int nt, int H, int N, int P,
+                                float* o_out) {
+  return ta_ssm_recurrent_planes(stream, dtype, proj, stride, coff, boff, xoff, share, decay, dt, state, cu_q, slots,
+                                 batch, nt, H, N, P, ta_gla_row_parts(N), o_out);
 }
 
 // y = (sum of the readout's planes + skip[h] * x) * silu(z), cut into ``groups`` equal parts of the row,

@@ -1400,7 +1400,7 @@ def gla_recurrent(proj: torch.Tensor, heads: int, key_dim: int, value_dim: int, 
         raise KernelError(f"gla_recurrent: shapes do not fit {H} heads of {dk} / {dv}, rank {rank}: "
                           f"proj {tuple(proj.shape)} a2 {tuple(a2.shape)} state {tuple(state.shape)} "
                           f"o_out {tuple(o_out.shape)} alpha {tuple(alpha.shape)}")
-    _check(library().ta_gla_recurrent(
+    _check(library().ta_gla_recurrent_planes(
         _stream(), c_int(_code(proj.dtype)), c_int(_wcode(a2, proj.dtype, "gla_recurrent")), _ptr(proj),
         c_int(stride), c_int(0), c_int(H * dk), c_int(2 * H * dk), c_int(2 * H * dk + 2 * H * dv),
         c_int(rank), _ptr(a2), _ptr(a2_bias), c_float(1.0 / tau), c_float(float(dk) ** -0.5), _ptr(alpha),
@@ -1608,7 +1608,7 @@ def wkv_recurrent(rkvg: torch.Tensor, low: torch.Tensor, heads: int, key_dim: in
             or decay.shape != (nt, n) or 3 * nt * n >= 2 ** 31:
         raise KernelError(f"wkv_recurrent: shapes do not fit {H} heads of {dk}: low {tuple(low.shape)} w2 "
                           f"{tuple(w2.shape)} state {tuple(state.shape)} o_out {tuple(o_out.shape)}")
-    _check(library().ta_wkv_recurrent(
+    _check(library().ta_wkv_recurrent_planes(
         _stream(), c_int(_code(rkvg.dtype)), c_int(_wcode(w2, rkvg.dtype, "wkv_recurrent")), _ptr(rkvg), c_int(n),
         c_int(0), c_int(nt * n), c_int(2 * nt * n), _ptr(low), c_int(ls), c_int(rank), _ptr(w2), _ptr(w0),
         _ptr(bonus), _ptr(decay), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt), c_int(H),
@@ -1672,7 +1672,7 @@ def decay_recurrent(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, head
         raise KernelError(f"decay_recurrent: shapes do not fit {H} heads of {dk} / {dv}: proj {tuple(proj.shape)} "
                           f"offsets {(q_off, k_off, v_off)} decays {tuple(decays.shape)} state {tuple(state.shape)} "
                           f"o_out {tuple(o_out.shape)}")
-    _check(library().ta_decay_recurrent(
+    _check(library().ta_decay_recurrent_planes(
         _stream(), c_int(_code(proj.dtype)), _ptr(proj), c_int(stride), c_int(q_off), c_int(k_off), c_int(v_off),
         _ptr(decays), c_float(q_scale), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt), c_int(H),
         c_int(dk), c_int(dv), c_int(o_out.shape[0]), _ptr(o_out)))
@@ -2324,7 +2324,7 @@ def ssm_recurrent(xbc: torch.Tensor, x_off: int, b_off: int, c_off: int, heads: 
     batch = _step_tables(cu_q, slots, nt, "ssm_recurrent")
     if not _planes_fit(o_out, (nt, heads, head_dim), state_dim, batch, scalar_decay=True):
         raise KernelError(f"ssm_recurrent: o_out is {tuple(o_out.shape)}")
-    _check(library().ta_ssm_recurrent(
+    _check(library().ta_ssm_recurrent_planes(
         _stream(), c_int(_code(xbc.dtype)), _ptr(xbc), c_int(stride), c_int(c_off), c_int(b_off), c_int(x_off),
         c_int(heads // groups), _ptr(decay), _ptr(dt), _ptr(state), _ptr(cu_q), _ptr(slots), c_int(batch), c_int(nt),
         c_int(heads), c_int(state_dim), c_int(head_dim), c_int(o_out.shape[0]), _ptr(o_out)))
