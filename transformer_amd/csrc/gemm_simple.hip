@@ -463,7 +463,8 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
   const int n0 = blockIdx.x * 32 * WN, m0 = blockIdx.y * 32 * WM;
   const int group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
   const int segs = (K + SEG - 1) / SEG, rounds = (segs + 1) / 2, steps = rounds * (SEG / 32);
-  // the chunks this wave brings (the last ones of WM = 3 are brought twice, by two waves)
+  // the chunks this wave brings (WM = 3: four loads a wave for 40 chunks, so that every wave waits for as many; the last chunk
+  // is brought by nine of the twelve waves, the same bytes each time)
   const float* src[PER];
   int to[PER], from_k[PER];
 #pragma unroll
