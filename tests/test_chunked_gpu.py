@@ -192,9 +192,12 @@ def test_chunks_are_no_further_off_than_a_walk_in_32_bits(kind, fade):
         assert _off(got, exact) <= 1.1 * (_off(walk, exact) ** 2 + 2.5e-8 ** 2) ** 0.5
 
 
-def test_matrix_memory_in_chunks_is_no_further_off_than_its_walk():
+@pytest.mark.parametrize("geom", [(8, 256, 512), (128, 64, 130), (256, 30, 140), (20, 250, 212)])
+def test_matrix_memory_in_chunks_is_no_further_off_than_its_walk(geom):
+    """A million numbers of state and more, 400 tokens: readouts, denominators, states and normalisers against 64 bits. What a
+    chunk adds is one rounding of every decayed key, as above."""
     from transformer_amd import kernels as K
-    H, dk, dv, n = 8, 256, 512, 400
+    (H, dk, dv), n = geom, 400
     g = torch.Generator(device=DEV).manual_seed(7)
     rows = torch.randn(n, 2 * H * dk + H * dv, generator=g, device=DEV).bfloat16()
     keep, write = 1 - 0.1 * torch.rand(n, H, generator=g, device=DEV), torch.rand(n, H, generator=g, device=DEV)
@@ -210,7 +213,7 @@ def test_matrix_memory_in_chunks_is_no_further_off_than_its_walk():
         K.memory_recurrent(rows, 0, H * dk, 2 * H * dk, dk ** -0.5, keep, write, state, norm, _t([0, n], torch.int32),
                            _t([0], torch.int32), o, den, lanes=lanes)
         off.append([_off(o, want[..., :dv]), _off(den, want[..., dv]), _off(state[0], end[..., :dv]), _off(norm[0], end[..., dv])])
-    assert all(a <= 1.1 * b for a, b in zip(*off)), off
+    assert all(a <= 1.1 * (b ** 2 + 2.5e-8 ** 2) ** 0.5 for a, b in zip(*off)), off
 
 
 @pytest.mark.parametrize("column", ["key", "query"])

@@ -292,11 +292,14 @@ extern "C" int ta_memory_recurrent(hipStream_t stream, int dtype, const void* pr
              stride >= voff + H * dv, "ta_memory_recurrent: rows of %d are too short", stride);
   TA_REQUIRE(lanes == 0 || lanes == 16 || lanes == 32, "ta_memory_recurrent: %d lanes", lanes);
   TA_REQUIRE(dtype == TA_F32 || dtype == TA_BF16, "ta_memory_recurrent: unknown dtype %d", dtype);
-  // From a million numbers of state on the walk fills the CUs and is bound by its vector instructions; below, both are
-  // chains of latencies, of which the walk's is the shorter (walk / chunks: 1 x 1,000 tokens of 8 heads of 256 x 512
-  // 261 / 236 us, 4 x 300 236 / 116, 32 x 100 of 8 of 64 x 64 39 / 35, but 8 x 300 of those 47 / 59).
-  // Float32 rows are walked, as everywhere (recurrent.hip).
-  if (lanes == 0 && dtype == TA_BF16 && (long long)batch * H * dk * dv >= 1 << 20 && ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
+  // From two million numbers of state on the walk fills the CUs and is bound by its vector instructions, from one million on in
+  // steps of a hundred tokens a sequence; below, both are chains of latencies, of which the walk's is the shorter (walk / chunks:
+  // 4 x 20 tokens of 8 heads of 256 x 512 33.3 / 29.3 us, 4 x 300 214 / 104, 1 x 1,000 240 / 229; 2 x 60 of 32 of 128 x 128 19.6 /
+  // 21.0, 2 x 200 46.5 / 45.6; 32 x 20 of 8 of 64 x 64 11.1 / 11.5, 32 x 100 26.5 / 23.3). Float32 rows are walked, as everywhere
+  // (recurrent.hip).
+  const long long numbers = (long long)batch * H * dk * dv;
+  if (lanes == 0 && dtype == TA_BF16 && (numbers >= 1 << 21 || (numbers >= 1 << 20 && nt >= 96 * (long long)batch)) &&
+      ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
     const TaChunked c = {proj, stride, qoff, koff, voff, 1, qscale, nullptr, keep, nullptr, write, nullptr, state, cu_q, slots,
                          H, dk, dv, (size_t)nt * H * dv, 1, o_out, n_state, den_out, false};
     return ta_chunked_launch(stream, dtype, c, batch, "ta_memory_recurrent");
