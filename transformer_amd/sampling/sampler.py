@@ -45,8 +45,7 @@ class _Buffers:
 
     def used(self):
         """Marks the work that the current stream has been given so far as the last to touch these buffers."""
-        stream = torch.cuda.current_stream()
-        event = torch.cuda.Event()
+        stream, event = torch.cuda.current_stream(), torch.cuda.Event()
         event.record(stream)
         self._last[stream.cuda_stream] = event
         return event
@@ -60,9 +59,8 @@ class Chosen:
     """Tokens that the GPU has been asked to choose: ``device`` holds them (int32) as soon as
     the stream gets there; ``result()`` waits for their copy to the host."""
 
-    def __init__(self, buffers: _Buffers, rows: int):
-        self.device, self._host = buffers.device[:rows], buffers.host[:rows]
-        self._buffers, self._event = buffers, buffers.used()
+    def __init__(self, device: torch.Tensor, host: torch.Tensor, buffers: _Buffers):
+        self.device, self._host, self._buffers, self._event = device, host, buffers, buffers.used()
 
     def result(self):
         self._event.synchronize()
@@ -113,7 +111,7 @@ class Sampler:
                 kernels.sample(logits, u_dev, out, float(self.args.temperature), int(k),
                                float(self.args.top_p), b.scratch if need else None)
                 out_host.copy_(out, non_blocking=True)
-        return Chosen(b, n)
+        return Chosen(out, out_host, b)
 
     def choose(self, logits: torch.Tensor, sequences: Sequence[int], drawn: Sequence[int]):
         """As ``choose_async``, returning the chosen tokens as a list of ints."""
