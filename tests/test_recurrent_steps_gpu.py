@@ -144,3 +144,30 @@ def test_convolution_of_four_channels_a_thread_has_the_bits_of_one(channels, tap
     assert torch.equal(got[0][0], got[1][0]) and torch.isfinite(got[0][0]).all()
     if taps > 1:
         assert torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("dtype,last", [("bfloat16", 640), ("float32", 1340)])
+@pytest.mark.parametrize("taps", [1, 2, 4, 8])
+def test_large_convolutions_have_the_bits_of_one_channel_a_thread(taps, dtype, last):
+    """As above with as many numbers as it takes four channels a thread (8 million, 16 million in float32), the last workgroup of
+    a row part of one."""
+    from transformer_amd import kernels as K
+    td, lens, C = getattr(torch, dtype), [1, 2, 30, 16, last, 5], 12292
+    nt, most = sum(lens), (16 if dtype == "float32" else 8) << 20
+    assert nt * C >= most
+    g = torch.Generator(device=DEV).manual_seed(taps)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    x, w, bi, bo, mem = r(nt, C).to(td), r(C, taps), r(C), r(C), r(8, taps - 1, C)
+    cu, slots = _t(np.concatenate([[0], np.cumsum(lens)]), torch.int32), _t([7, 0, 3, 2, 5, 6], torch.int32)
+    got = []
+    for off in (4, 5):
+        rows = torch.zeros(nt, C + 8, dtype=td, device=DEV)
+        rows[:, off:off + C] = x
+        state = mem.clone() if taps > 1 else None
+        out = torch.full((nt, C + 4), 7.0, dtype=td, device=DEV)
+        K.causal_conv(rows, off, C, w, out[:, :C], state, cu, slots, max(lens), bias_in=bi, bias_out=bo, activation="silu")
+        assert (out[:, C:] == 7).all()
+        got.append((out[:, :C], state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.isfinite(got[0][0]).all()
+    if taps > 1:
+        assert torch.equal(got[0][1], got[1][1])

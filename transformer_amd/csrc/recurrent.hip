@@ -1367,10 +1367,11 @@ __global__ __launch_bounds__(256) void causal_conv_run_kernel(
 
 // The same with four neighbouring channels a thread, read and written at once, and all CONV_RUN tokens' inputs asked for in
 // front of the walk: rows, columns and pointers on whole pieces. One channel at a time is 2-byte accesses, a trip to memory a
-// token behind the branch for the next sequence. Bound by memory and by the activation's arithmetic: 2,943 tokens of 12,288
-// and of 6,144 channels in bfloat16 (145 and 72 MB) with silu 54-65 and 20-22 us; the call with the memory's update 64 and
-// 41 us, with one channel a thread 107 and 61, and 18 against 23 at 1,013 x 2,560, 16 against 19 at 200 x 512: wide wherever
-// it may run. Blocks go along the rows first: down the columns first it is 59-73 and 20-23.
+// token behind the branch for the next sequence, which many waves hide; four a thread are a quarter of the waves, each with four
+// times the activations in a row. So it is the larger calls that gain (CONV_WIDE_BF16, CONV_WIDE_F32). Bound by memory and by the activation's
+// arithmetic: 2,943 tokens of 12,288 and of 6,144 channels in bfloat16 (145 and 72 MB) with silu 54-65 and 20-22 us; the call
+// with the memory's update 64 and 41 us, with one channel a thread 107 and 61. Blocks go along the rows first: down the columns first it
+// is 59-73 and 20-23.
 template <typename T, int K>
 __global__ __launch_bounds__(256) void causal_conv_wide_kernel(
     const T* __restrict__ in, int stride, int off, const float* __restrict__ bias_in,
@@ -1506,6 +1507,12 @@ __global__ __launch_bounds__(256) void causal_conv_step_kernel(
   }
 }
 
+// Numbers of a call from which on four channels a thread are faster, with the rows in the caches and the rest in memory (us by one / by
+// four): bfloat16 1,000 x 2,560 10.1 / 13.7, 1,000 x 6,144 17.6 / 18.1, 3,000 x 2,560 18.8 / 21.1, 1,500 x 6,144 26.6 / 22.6, 6,000 x 2,560
+// 31.5 / 31.8, 6,000 x 12,288 162 / 90; float32 1,500 x 6,144 28.7 / 27.5, 6,000 x 2,560 33.3 / 37.7, 3,000 x 6,144 41.9 / 40.1, 3,000 x 12,288
+// 112 / 70; 64 x 512 9.0 / 12.4 in either.
+#define CONV_WIDE_BF16 (8ll << 20)
+#define CONV_WIDE_F32 (16ll << 20)
 // in: [nt, stride] rows, the convolution reads columns off .. off + C; out: [nt, out_stride] rows,
 // columns 0 .. C. taps [C, K] float32; bias_in, bias_out [C] float32 or null; conv_state [slots, K-1, C]
 // float32 (null with K == 1: no memory). update 0: the state is left as it is. max_qlen: the most
@@ -1549,7 +1556,7 @@ extern "C" int ta_causal_conv(hipStream_t stream, int dtype, const void* in, int
   causal_conv_wide_kernel<T, KK><<<(nt + CONV_RUN - 1) / CONV_RUN * ((C / 4 + 255) / 256), 256, 0, stream>>>(              \
       (const T*)in, stride, off, bias_in, taps, bias_out, conv_state, cu_q, slots, batch, nt, C, act, (T*)out, out_stride)
   const int piece = dtype == TA_F32 ? 16 : 8;
-  const bool wide = C % 4 == 0 && off % 4 == 0 && stride % 4 == 0 && out_stride % 4 == 0 && (uintptr_t)in % piece == 0 &&
+  const bool wide = (long long)nt * C >= (dtype == TA_F32 ? CONV_WIDE_F32 : CONV_WIDE_BF16) && C % 4 == 0 && off % 4 == 0 && stride % 4 == 0 && out_stride % 4 == 0 && (uintptr_t)in % piece == 0 &&
                     (uintptr_t)out % piece == 0;
   if (K <= CONV_MAX_TAPS && wide) {
     if (dtype == TA_F32) { CONV_BY_TAPS(CONV_WIDE, float) } else { CONV_BY_TAPS(CONV_WIDE, bf16_t) }
