@@ -819,7 +819,8 @@ def test_gemm_simple_at_the_edges_of_its_tiles(mnk, types):
 # float32, two groups of waves: each height of the tiles with rows and columns that end inside a tile, an odd and an even number of
 # segments, k that ends inside a block, a segment of the first and of the second group, right behind the first two
 @pytest.mark.parametrize("mnk", [(65, 16400, 516), (67, 16384, 1024), (743, 2048, 1292), (739, 2020, 1536), (1021, 2048, 772),
-                                 (1000, 2000, 2052), (300, 2100, 1028), (130, 4100, 2000)])
+                                 (1000, 2000, 2052), (300, 2100, 1028), (130, 4100, 2000), (200, 2900, 516), (190, 2930, 772),
+                                 (170, 3000, 1292), (180, 2990, 540), (743, 2048, 2052), (739, 2020, 3076)])
 def test_gemm_groups_of_waves_in_turn(mnk):
     from transformer_amd import kernels
     M, N, K = mnk

@@ -256,6 +256,12 @@ static bool walk_takes(int M, int N, int K) {
   const int side = M <= 8 ? 8 : 16;
   return M >= 1 && M <= 16 && K > 512 && K <= 4096 && (N + side - 1) / side >= walk_groups(M, K) * 5 / 4;
 }
+// Without an activation to save a launch: two tiles a workgroup where most of the last waves' k is past the end (6,000 x 520 at 1 /
+// 8 rows 6.4 / 6.7 us by few rows, 7.0 / 7.2 here, but 16,384 x 520 15.5 and 12.9; 3,000 x 1,032 at one row 6 % more here).
+static bool walk_pays(int M, int N, int K) {
+  const bool thin = M <= 8 && (K <= 640 || (M == 1 && K > 1024 && K <= 1280));
+  return walk_takes(M, N, K) && (!thin || (N + 7) / 8 >= 2 * walk_groups(M, K));
+}
 template <bool GLU>
 static void walk(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc,
                  int M, int N, int K) {
@@ -444,7 +450,15 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
 // or on two (an older workgroup's waves go first and the younger one is left with a CU to itself), so that the host picks
 // the height whose tiles leave the CUs evenly filled. 2,048 columns over k = 8,192: 1,021 rows 292 us (309 to 331 by 64 x 64),
 // 743 rows 233 (305), 300 rows 160 (247 by few rows). The matrix instructions alone take 232 of the 292, LDS reads 20 more; the
-// rest goes with the loads (four further waves that do nothing but load, 64 x 64 and one group: 294).
+// rest goes with the loads (four further waves that do nothing but load, 64 x 64 and one group: 294). A k that ends inside a round
+// of 512 ends the round (300 rows of 6,000 columns over k = 520 / 1,544 29.8 / 67.7 us, in whole rounds 45.5 / 81.3).
+// Its steps of 32 k of either group: the last round ends where its first segment does (the second is no longer, and there is none
+// where there is an odd number).
+__host__ __device__ __forceinline__ int groups_steps(int K) {
+  const int full = ((K + SEG - 1) / SEG - 1) / 2, rest = K - full * (2 * SEG);
+  return full * (SEG / 32) + (rest < SEG ? (rest + 31) / 32 : SEG / 32);
+}
+
 template <int WM>
 __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __restrict__ A, int lda,
                                                                const float* __restrict__ W, int ldw,
@@ -462,7 +476,7 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
   const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
   const int n0 = blockIdx.x * 32 * WN, m0 = blockIdx.y * 32 * WM;
   const int group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const int segs = (K + SEG - 1) / SEG, rounds = (segs + 1) / 2, steps = rounds * (SEG / 32);
+  const int segs = (K + SEG - 1) / SEG, steps = groups_steps(K);
   // the chunks this wave brings (WM = 3: four loads a wave for 40 chunks, so that every wave waits for as many; the last chunk
   // is brought by nine of the twelve waves, the same bytes each time)
   const float* src[PER];
@@ -526,11 +540,11 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
     read(0, (s + 1) % ST);
 #pragma unroll
     for (int j = 0; j < 4; ++j) multiply(1, j);
-    if (s % (SEG / 32) == SEG / 32 - 1) {
+    if (s % (SEG / 32) == SEG / 32 - 1 || s == steps - 1) {
       if (group == 0) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) total[e] += acc[e];
-      } else {
+      } else if (s / (SEG / 32) * 2 + 1 < segs) {        // (a round of one segment may end before the sums in front of it are read)
 #pragma unroll
         for (int e = 0; e < 16; ++e) handed[wave - WM * WN][e][lane] = acc[e];
       }
@@ -558,10 +572,13 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
 // and 12 % less in gemm_tiles' 128 x 128 once there are enough of those to fill it (1,021 x 16,384 x 2,048: 534 us there, 614 here;
 // 300 rows 265 and 205). Below 129 tiles of 64 x 64 the few-rows kernel's finer workgroups are as fast (2,048 columns over k =
 // 8,192: 256 rows 168 and 161 us, 128 rows 79 and 158), and two segments or fewer give the groups too little (2,048 x 512 x 300
-// 13 us by 64 x 64, 17 here).
+// 13 us by 64 x 64, 17 here). Nor do they gain where a round is half empty and the tiles of 64 x 64 would fill the CUs: time follows the
+// steps (300 rows of 6,000 columns over k = 768 / 900 / 1,280 / 2,300 22, 9, 13 and 8 % more than by 64 x 64, 1,024 / 2,048 / 2,056 level, 3,000
+// columns 2 to 6 % less).
 static int groups_height(int M, int N, int K, int batch) {
   auto tiles = [&](int rows, int cols) { return (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * batch; };
   if (M <= 64 || K <= 2 * SEG || tiles(64, 64) <= 128) return 0;
+  if (tiles(64, 64) >= 192 && tiles(128, 128) < 384 && groups_steps(K) * 6400ll > K * 103ll) return 0;
   auto cost = [&](int wm, int each) { return (tiles(32 * wm, 64) + CUS - 1) / CUS * wm * each; };
   const long long c2 = cost(2, 100), c3 = cost(3, 103), c4 = cost(4, 98);
   const long long least = c2 < c3 ? (c2 < c4 ? c2 : c4) : (c3 < c4 ? c3 : c4);
@@ -601,7 +618,7 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
     return;
   }
   if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
-    if (batch == 1 && walk_takes(M, N, K)) {
+    if (batch == 1 && walk_pays(M, N, K)) {
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
     }
