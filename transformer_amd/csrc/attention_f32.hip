@@ -257,7 +257,9 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
 // that a recorded launch fits every length; the pages are its slowest index, since workgroups that find no page are then handed out
 // last (with the pages fastest 4 x 200 keys, 16 heads over 4 kv heads, 14.0 us for both kernels where it now takes 9.1).
 // Both kernels, those heads, 4 x 200 / 16 x 300 / 16 x 2,000 keys: 9.1 / 12.3 / 36 us; with a wave a page, which brings 64 KB by
-// itself, 20.6 / 58 / 65; by one workgroup per sequence and kv head 279 (4 of 50 to 300).
+// itself, 20.6 / 58 / 65; by one workgroup per sequence and kv head 279 (4 of 50 to 300). Heads of 64, whose pages are half as long: 8 x
+// 1,000 keys, 16 heads over 4, 12.8 us where a wave a page took 15.2, but with every CU full the four waves' barrier shows (32 x
+// 2,000 39.1 and 37.0; 64 x 1,000, 16 heads with keys of their own, 120 and 105); of 128, 64 x 1,000 214 and 278.
 template <int NB, bool EXACT>
 __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
   __shared__ f32x4 scores[2][4][TA_WAVE];

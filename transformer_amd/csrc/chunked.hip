@@ -21,11 +21,11 @@
 // operands' layout of the readout, so S never leaves its registers.
 //
 // A chunk takes 4 to 8 us (1 to 8 sequences of 32 heads of 128 x 128), of which the matrix instructions need 1.8 at the
-// most: bound by the preparation's chain of reads from LDS, products and sums over
-// lanes. 8 x 656 tokens of 32 heads of 128 x 128, decays included: 829 us token by token, 336 in chunks (287 with products of
-// decays in one number), and the norm reads one plane of readouts instead of four; the matrix memory of 2 x 1,536 tokens, 8 heads of
-// 256 x 512: 730 -> 390. Half as many preparing waves cost 1.5 times as much; reading a group of tokens ahead of the branches, for
-// every wave, 10 to 30 % more.
+// most: bound by the preparation's chain of reads from LDS, products and sums over lanes. 8 x 656 tokens of 32 heads of
+// 128 x 128, decays included: 829 us token by token, 336 in chunks (287 with products of decays in one number), and the norm
+// reads one plane of readouts instead of four; the matrix memory of 2 x 1,536 tokens, 8 heads of 256 x 512: 730 -> 390. Half
+// as many preparing waves cost 1.5 times as much; reading a group of tokens ahead of the branches, for every wave, 10 to 30 %
+// more.
 #include "chunked.h"
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
