@@ -459,7 +459,8 @@ __host__ __device__ __forceinline__ int groups_steps(int K) {
   return full * (SEG / 32) + (rest < SEG ? (rest + 31) / 32 : SEG / 32);
 }
 
-template <int WM>
+// WHOLE: of whole rounds (asking every step whether it is the last costs a hundredth of the time).
+template <int WM, bool WHOLE>
 __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __restrict__ A, int lda,
                                                                const float* __restrict__ W, int ldw,
                                                                const float* __restrict__ bias, float* __restrict__ C,
@@ -476,7 +477,7 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
   const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
   const int n0 = blockIdx.x * 32 * WN, m0 = blockIdx.y * 32 * WM;
   const int group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const int segs = (K + SEG - 1) / SEG, steps = groups_steps(K);
+  const int segs = (K + SEG - 1) / SEG, steps = WHOLE ? (segs + 1) / 2 * (SEG / 32) : groups_steps(K);
   // the chunks this wave brings (WM = 3: four loads a wave for 40 chunks, so that every wave waits for as many; the last chunk
   // is brought by nine of the twelve waves, the same bytes each time)
   const float* src[PER];
@@ -540,11 +541,11 @@ __global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __re
     read(0, (s + 1) % ST);
 #pragma unroll
     for (int j = 0; j < 4; ++j) multiply(1, j);
-    if (s % (SEG / 32) == SEG / 32 - 1 || s == steps - 1) {
+    if (s % (SEG / 32) == SEG / 32 - 1 || (!WHOLE && s == steps - 1)) {
       if (group == 0) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) total[e] += acc[e];
-      } else if (s / (SEG / 32) * 2 + 1 < segs) {        // (a round of one segment may end before the sums in front of it are read)
+      } else if (WHOLE || s / (SEG / 32) * 2 + 1 < segs) {       // (a round of one segment may end before the sums in front of it are read)
 #pragma unroll
         for (int e = 0; e < 16; ++e) handed[wave - WM * WN][e][lane] = acc[e];
       }
@@ -601,11 +602,13 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
     if (const int wm = groups_height(M, N, K, batch)) {
       const dim3 grid((N + 63) / 64, (M + 32 * wm - 1) / (32 * wm), batch);
-#define GROUPS(WM) gemm_groups_kernel<WM><<<grid, WM * 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
-      if (wm == 2) GROUPS(2);
-      else if (wm == 3) GROUPS(3);
-      else GROUPS(4);
+#define GROUPS_(WM, WHOLE) \
+  gemm_groups_kernel<WM, WHOLE><<<grid, WM * 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
+#define GROUPS(WM) \
+  if (groups_steps(K) % (SEG / 32) == 0) GROUPS_(WM, true); else GROUPS_(WM, false)
+      if (wm == 2) { GROUPS(2); } else if (wm == 3) { GROUPS(3); } else { GROUPS(4); }
 #undef GROUPS
+#undef GROUPS_
       return;
     }
   if (tiles(64) >= 192 && (M > 64 || brief)) {
