@@ -295,11 +295,13 @@ extern "C" int ta_memory_recurrent(hipStream_t stream, int dtype, const void* pr
   // From two million numbers of state on the walk fills the CUs and is bound by its vector instructions, from one million on in
   // steps of a hundred tokens a sequence; below, both are chains of latencies, of which the walk's is the shorter (walk / chunks:
   // 4 x 20 tokens of 8 heads of 256 x 512 33.3 / 29.3 us, 4 x 300 214 / 104, 1 x 1,000 240 / 229; 2 x 60 of 32 of 128 x 128 19.6 /
-  // 21.0, 2 x 200 46.5 / 45.6; 32 x 20 of 8 of 64 x 64 11.1 / 11.5, 32 x 100 26.5 / 23.3). Float32 rows are walked, as everywhere
-  // (recurrent.hip).
+  // 21.0, 2 x 200 46.5 / 45.6; 32 x 20 of 8 of 64 x 64 11.1 / 11.5, 32 x 100 26.5 / 23.3). From sixteen million on it is the states'
+  // way from memory and back that counts, and the walk's many small workgroups hide it better until there are tokens enough (8
+  // heads of 256 x 512, 16 x 20 108 / 108, 33 x 12 183 / 203, 33 x 20 213 / 241, 64 x 20 405 / 455, 33 x 40 277 / 277). Float32 rows
+  // are walked, as everywhere (recurrent.hip).
   const long long numbers = (long long)batch * H * dk * dv;
-  if (lanes == 0 && dtype == TA_BF16 && (numbers >= 1 << 21 || (numbers >= 1 << 20 && nt >= 96 * (long long)batch)) &&
-      ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
+  const int least = numbers >= 1 << 24 ? 40 : numbers >= 1 << 21 ? 0 : 96;       // tokens a sequence
+  if (lanes == 0 && dtype == TA_BF16 && numbers >= 1 << 20 && nt >= (long long)least * batch && ta_chunked_long(nt, batch) && ta_chunked_takes(true, false, dk)) {
     const TaChunked c = {proj, stride, qoff, koff, voff, 1, qscale, nullptr, keep, nullptr, write, nullptr, state, cu_q, slots,
                          H, dk, dv, (size_t)nt * H * dv, 1, o_out, n_state, den_out, false};
     return ta_chunked_launch(stream, dtype, c, batch, "ta_memory_recurrent");
