@@ -17,6 +17,7 @@
 // gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS; gemm_groups: 64, 96 or 128 x 64, two groups
 // of waves that take the segments in turn.
 #include "common.h"
+#include "gemm_stream.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -621,6 +622,11 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
     return;
   }
   if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
+    if (batch == 1 && ta_gemm_stream_pays(M, N, K, 0)) {
+      ta_gemm_stream(stream, A, lda, W, ldw, bias, C, ldc, M, N, K, 0, 0, nullptr, 0.f);
+      return;
+    }
+  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
     if (batch == 1 && walk_pays(M, N, K)) {
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
@@ -696,6 +702,8 @@ extern "C" int ta_gemm_simple_glu(hipStream_t stream, const float* A, int lda, c
   TA_REQUIRE(ta_gemm_simple_glu_takes(M, di, K), "ta_gemm_simple_glu: M=%d di=%d K=%d", M, di, K);
   TA_REQUIRE(lda >= K && ldw >= K && ldc >= di && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
              "ta_gemm_simple_glu: rows of %d, %d, %d floats or their start", lda, ldw, ldc);
+  if (ta_gemm_stream_pays(M, 2 * di, K, 1))
+    return ta_gemm_stream(stream, A, lda, W, ldw, bias, C, ldc, M, 2 * di, K, 1, 0, nullptr, 0.f);
   walk<true>(stream, A, lda, W, ldw, bias, C, ldc, M, 2 * di, K);
   return ta_check_launch("ta_gemm_simple_glu");
 }

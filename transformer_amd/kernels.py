@@ -642,6 +642,63 @@ def gemm_simple_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: O
     return out
 
 
+class RowNorm:
+    """Rows of the float32 residual stream ``x`` that an RMS norm (its gain and eps) has not gone over yet: the product that
+    reads them does it first."""
+
+    def __init__(self, x: torch.Tensor, weight: torch.Tensor, eps: float):
+        self.x, self.weight, self.eps = x, weight, float(eps)
+
+
+def _f32_rows_fit(w: torch.Tensor) -> bool:
+    return w.dtype == torch.float32 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0
+
+
+def normed_takes(rows: int, w: torch.Tensor, glu: bool = False) -> bool:
+    """Whether ``gemm_normed`` should take a float32 norm in front of this weight over."""
+    return _f32_rows_fit(w) and not (glu and w.shape[0] % 2) \
+        and bool(library().ta_gemm_stream_normed_pays(c_int(rows), c_int(w.shape[0]), c_int(w.shape[1])))
+
+
+def add_takes(rows: int, w: torch.Tensor) -> bool:
+    """Whether ``gemm_add`` takes a float32 product of this weight."""
+    return _f32_rows_fit(w) and bool(library().ta_gemm_stream_pays(c_int(rows), c_int(w.shape[0]), c_int(w.shape[1]), c_int(0)))
+
+
+def _gemm_stream(what, a, w, out, bias=None, glu=False, add=False, norm=None):
+    _dev(a, "a", torch.float32, contiguous=False); _dev(w, "w", torch.float32, contiguous=False)
+    _dev(out, "out", torch.float32, contiguous=False)
+    M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
+    if w.shape[1] != a.shape[1] or Mo != M or out.shape[1] * (2 if glu else 1) != N:
+        raise KernelError(f"{what}: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    if bias is not None:
+        _dev(bias, "bias", torch.float32)
+        if bias.numel() != N:
+            raise KernelError(f"{what}: bias must hold one entry per row of w")
+    gain, eps = None, 0.0
+    if norm is not None:
+        gain, eps = norm.weight, norm.eps
+        _dev(gain, "norm weight", torch.float32)
+        if gain.numel() != a.shape[1]:
+            raise KernelError(f"{what}: a norm over {gain.numel()} for rows of {a.shape[1]}")
+    _check(library().ta_gemm_stream(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(bias), _ptr(out), c_int(ldc),
+                                    c_int(M), c_int(N), c_int(a.shape[1]), c_int(int(glu)), c_int(int(add)), _ptr(gain), c_float(eps)))
+    return out
+
+
+def gemm_normed(norm: RowNorm, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                glu: bool = False) -> torch.Tensor:
+    """``add_rmsnorm`` of the rows of norm.x and then ``gemm_simple``, with ``glu`` ``gemm_simple_glu``, in one kernel with the
+    same bits: at most 8 float32 rows (``normed_takes``)."""
+    return _gemm_stream("gemm_normed", norm.x, w, out, bias, glu, norm=norm)
+
+
+def gemm_add(a: torch.Tensor, w: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """x += a @ w.T in float32: ``gemm_simple`` whose result is added to the residual stream where it is stored, with the bits
+    that the next norm's add would give (``add_takes``)."""
+    return _gemm_stream("gemm_add", a, w, x, add=True)
+
+
 class RowScale:
     """Rows of activations that an RMS norm has not scaled yet: ``parts`` [tiles, 16] float32
     holds sums of squares per row (16 columns each), and the product that reads the rows

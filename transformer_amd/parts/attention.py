@@ -86,9 +86,13 @@ class CachedAttention(Part):
     def can_fold(self, nt: int) -> bool:
         return kernels.skinny_folds(nt, self.w["out.weight"])
 
-    # with many rows the last product can add itself to the residual stream (``into``)
+    # the same of a float32 engine: the first product goes over the norm itself (``norm``)
+    def takes_normed(self, nt: int) -> bool:
+        return kernels.normed_takes(nt, self.w["qkv.weight"])
+
+    # with many rows (or a few of float32) the last product can add itself to the residual stream (``into``)
     def can_add(self, nt: int) -> bool:
-        return adds_in_place(nt, self.w["out.weight"])
+        return adds_in_place(nt, self.w["out.weight"], self.dtype)
 
     def _out(self, o, ctx, fold, into):
         if fold is not None:
@@ -97,14 +101,14 @@ class CachedAttention(Part):
         return (linear_delta(o, self.w["out.weight"], ctx.ws, "attention.delta", into=into),
                 self.w.get("out.bias"))
 
-    def run(self, h, ctx, cache, layer, writes_cache=True, scale=None, fold=None, into=None):
+    def run(self, h, ctx, cache, layer, writes_cache=True, scale=None, fold=None, into=None, norm=None):
         """h: [nt, hidden] engine dtype -> (delta float32 [nt, hidden], bias row or None);
         None with ``fold``, which has then taken the result; (None, bias) with ``into``, the
-        residual stream that the output projection has then added itself to."""
+        residual stream that the output projection has then added itself to. ``norm`` stands for h."""
         nt = h.shape[0]
         width = (self.nq + 2 * self.nkv) * self.dh
         qkv = linear(h, self.w["qkv.weight"], ctx.ws.take("attention.qkv", (nt, width), self.dtype),
-                     scale=scale)
+                     scale=scale, norm=norm)
         kc, vc, group = cache.layer_kv(layer)
         meta = ctx.kv[group]
         o = ctx.ws.take("attention.o", (nt, self.nq * self.dh), self.dtype)
@@ -374,7 +378,7 @@ class SinkAttention(Part):
     # with many rows the output projection can add itself to the residual stream (``into``)
     def can_add(self, nt: int) -> bool:
         w = self.out_wide if getattr(self, "out_wide", None) is not None else self.w["out.weight"]
-        return adds_in_place(nt, w)
+        return adds_in_place(nt, w, self.dtype)
 
     # single-token steps: the norm in front and the norm behind ride on the products (``PreNormBlock``)
     def takes_scaled(self, nt: int) -> bool:

@@ -62,6 +62,13 @@ class PreNormBlock(Part):
         f = getattr(part, what, None)
         return f is not None and bool(f(nt))
 
+    def _normed(self, norm, part, pending, x):
+        """The norm for a float32 part whose first product goes over it itself; None where its own kernel runs."""
+        if self.dtype == torch.float32 and isinstance(pending, tuple) and pending[0] is None and pending[1] is None \
+                and hasattr(norm, "gain") and self._offers(part, "takes_normed", x.shape[0]):
+            return kernels.RowNorm(x, norm.gain(), norm.eps)
+        return None
+
     def entry_fold(self, x, ctx):
         """What the last product of the block in front needs to take over norm1, or None."""
         if not (self._fusable(x.shape[0]) and self._offers(self.mixer, "takes_scaled", x.shape[0])
@@ -100,8 +107,11 @@ class PreNormBlock(Part):
         if isinstance(pending, kernels.RowScale):
             kw["scale"] = pending                  # h already holds the rows, not yet scaled
         elif not (isinstance(pending, str) and pending == "normed"):
-            with span(ctx, "norm"):
-                self.norm1.run(x, h, pending[0], pending[1])
+            kw["norm"] = self._normed(self.norm1, self.mixer, pending, x)
+            if kw["norm"] is None:
+                del kw["norm"]
+                with span(ctx, "norm"):
+                    self.norm1.run(x, h, pending[0], pending[1])
         # the rows that the side part reads: the stream itself where the engine computes in float32
         xcast = None
         if self.side is not None:
@@ -128,8 +138,11 @@ class PreNormBlock(Part):
         if "fold" in kw:
             kw2["scale"] = kw["fold"].scale()
         else:
-            with span(ctx, "norm"):
-                self.norm2.run(x, h, pending[0], pending[1])
+            kw2["norm"] = self._normed(self.norm2, self.ffn, pending, x)
+            if kw2["norm"] is None:
+                del kw2["norm"]
+                with span(ctx, "norm"):
+                    self.norm2.run(x, h, pending[0], pending[1])
         if self.side is not None:
             if fusable and self._offers(self.ffn, "can_fold", nt):
                 with span(ctx, "ffn"):

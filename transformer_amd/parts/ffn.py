@@ -37,17 +37,22 @@ class SwiGLU(Part):
     def can_fold(self, nt: int) -> bool:
         return kernels.skinny_folds(nt, self.w["down.weight"])
 
-    def can_add(self, nt: int) -> bool:
-        return adds_in_place(nt, self.w["down.weight"])
+    def takes_normed(self, nt: int) -> bool:
+        return self.limits is None and kernels.normed_takes(nt, self.w["gate_up.weight"], glu=True)
 
-    def run(self, h, ctx, scale=None, fold=None, into=None):
+    def can_add(self, nt: int) -> bool:
+        return adds_in_place(nt, self.w["down.weight"], self.dtype)
+
+    def run(self, h, ctx, scale=None, fold=None, into=None, norm=None):
         """h: [nt, hidden] engine dtype -> (delta float32 [nt, hidden], bias row or None);
         None with ``fold``, which has then taken the result; (None, bias) with ``into``, the
         residual stream that the down projection has then added itself to. ``scale``: the rows
-        of h still lack their norm's factor."""
+        of h still lack their norm's factor; ``norm`` (float32) stands for h."""
         s, nt = self.spec, h.shape[0]
         act = ctx.ws.take("swiglu.act", (nt, s.intermediate), self.dtype)
-        if scale is not None or kernels.skinny_wins(h, self.w["gate_up.weight"]):
+        if norm is not None:
+            kernels.gemm_normed(norm, self.w["gate_up.weight"], act, self.w.get("gate_up.bias"), glu=True)
+        elif scale is not None or kernels.skinny_wins(h, self.w["gate_up.weight"]):
             # few rows: the product applies the activation itself and [nt, 2*di] is never stored
             kernels.gemm_skinny(h, self.w["gate_up.weight"], act, swiglu=True,
                                 bias=self.w.get("gate_up.bias"), scale=scale, limits=self.limits)
@@ -93,9 +98,12 @@ class GLU(SwiGLU):
     def takes_scaled(self, nt: int) -> bool:
         return self.activation in ("silu", "limited") and super().takes_scaled(nt)
 
-    def run(self, h, ctx, scale=None, fold=None, into=None):
+    def takes_normed(self, nt: int) -> bool:
+        return self.activation == "silu" and super().takes_normed(nt)
+
+    def run(self, h, ctx, scale=None, fold=None, into=None, norm=None):
         if self.activation in ("silu", "limited"):
-            return super().run(h, ctx, scale=scale, fold=fold, into=into)
+            return super().run(h, ctx, scale=scale, fold=fold, into=into, norm=norm)
         s, nt = self.spec, h.shape[0]
         act = ctx.ws.take("swiglu.act", (nt, s.intermediate), self.dtype)
         if not s.bias and kernels.skinny_wins(h, self.w["gate_up.weight"]):

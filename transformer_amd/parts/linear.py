@@ -46,14 +46,17 @@ class Workspace:
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor], scale=None,
-           fold=None) -> torch.Tensor:
+           fold=None, norm=None) -> torch.Tensor:
     """out[nt, n] = x[nt, k] @ weight[n, k]^T. x and weight share a dtype, or the weight is
     a float32 matrix of a bfloat16 engine (its file stores it in 32 bits and it stays so).
 
     scale (``kernels.RowScale``): the rows of x still lack their norm's factor, which the
     product applies. fold (``kernels.NormFold``): the product is added to the residual stream
     and prepares the next norm instead of writing ``out``. Only the few-rows product can do
-    either, so a caller asks ``kernels.skinny_takes`` before it hands them over."""
+    either, so a caller asks ``kernels.skinny_takes`` before it hands them over. norm (``kernels.RowNorm``): the
+    norm of the residual stream, which stands for x; a caller asks ``kernels.normed_takes``."""
+    if norm is not None:
+        return kernels.gemm_normed(norm, weight, out)
     if scale is not None or fold is not None:
         return kernels.gemm_skinny(x, weight, out, scale=scale, fold=fold)
     mixed = x.dtype == torch.bfloat16 and weight.dtype == torch.float32
@@ -135,9 +138,11 @@ def library_rows(rows: int, n: int, k: int) -> list:
     return calls
 
 
-def adds_in_place(rows: int, weight: torch.Tensor) -> bool:
-    """Whether ``linear_delta`` can add this product to the residual stream by itself: the
-    vendor library's product in one plane, which takes what it adds to as its third operand."""
+def adds_in_place(rows: int, weight: torch.Tensor, dtype: torch.dtype = torch.bfloat16) -> bool:
+    """Whether ``linear_delta`` can add this product of ``dtype`` activations to the residual stream by itself: the
+    vendor library's product in one plane, which takes what it adds to as its third operand, or a few float32 rows."""
+    if dtype == torch.float32:
+        return kernels.add_takes(rows, weight)
     return weight.dtype == torch.bfloat16 and rows > kernels.MID_MAX_ROWS and \
         library_planes(rows, weight) == 1
 
@@ -156,10 +161,12 @@ def linear_delta(x: torch.Tensor, weight: torch.Tensor, ws: Workspace, name: str
     stream and delta and writing the stream back (2,048 tokens of the 8B shape: 21 to 10 us)."""
     nt, n = x.shape[0], weight.shape[0]
     if into is not None:
-        if not (x.dtype == torch.bfloat16 and adds_in_place(nt, weight)) or into.shape != (nt, n) \
-                or into.dtype != torch.float32:
+        if not adds_in_place(nt, weight, x.dtype) or into.shape != (nt, n) or into.dtype != torch.float32:
             raise kernels.KernelError(f"linear_delta: cannot add {tuple(x.shape)} x {tuple(weight.shape)} "
                                       f"in place into {tuple(into.shape)} {into.dtype}")
+        if x.dtype == torch.float32:
+            kernels.gemm_add(x, weight, into)
+            return None
         at = 0
         for rows in library_rows(nt, n, x.shape[1]):
             part = into[at:at + rows]

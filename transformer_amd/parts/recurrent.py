@@ -385,7 +385,7 @@ class GatedDelta(Part):
     # with many rows the output projection can add itself to the residual stream (``into``); in
     # single-token steps the norms around the mixer ride on its products (``PreNormBlock``)
     def can_add(self, nt: int) -> bool:
-        return adds_in_place(nt, self.w["out.weight"])
+        return adds_in_place(nt, self.w["out.weight"], self.dtype)
 
     def takes_scaled(self, nt: int) -> bool:
         return kernels.skinny_takes(nt, self.w["in.weight"])
@@ -470,7 +470,7 @@ class MatrixMemory(Part):
 
     # as in ``GatedDelta``
     def can_add(self, nt: int) -> bool:
-        return adds_in_place(nt, self.w["out.weight"])
+        return adds_in_place(nt, self.w["out.weight"], self.dtype)
 
     def takes_scaled(self, nt: int) -> bool:
         return kernels.skinny_takes(nt, self.w["in.weight"])
