@@ -990,8 +990,9 @@ __device__ void sample_whole_row(const float* __restrict__ row, int vocab, float
 //   draw    one workgroup a row: the threshold among the gathered tokens by the digits of their keys, the part that
 //           holds the drawn mass, the token in it.
 // 8 rows of 128,256 tokens, top-k 40 and top-p 0.95: 125 us by one workgroup a row (which gathered whole kept sets of a
-// few thousand tokens), 29 us in parts
-// (5 + 10 + 15; the draw 12 since it asks for all it needs of the records at once and a wave adds up over the parts); 64 rows 51 us, 256 rows 125, one row without a cut 16.
+// few thousand tokens), 27 us in parts
+// (5 + 10 + 12, the draw asking for all it needs of the records at once); 64 rows 50 us, 256 rows 125, one row without a cut 16. Cuts at
+// few tokens go by the two kernels below.
 struct PartRecord {
   float2 mass[STEPS / 2];    // of two steps each, relative to the part's maximum
   uint32_t cnt[STEPS / 2];   // tokens of two steps each, 16 bits of them (a part has 4,096)
@@ -1550,6 +1551,418 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
   }
 }
 
+// ------------------------------------------------------------------ few tokens kept at most
+// A cut at top_k <= TOP_MOST_K in two kernels. A row keeps no token that top_k others of its own part go before, so
+//   top     a part hands on its tokens down to the step (1/16 of a unit of logit / T, counted from its largest) with which
+//           it has top_k of them, and the mass of all its tokens relative to its own largest;
+//   draw    one workgroup a row: of these some 40 to 100 tokens a part the step that holds the threshold, the order of the
+//           few tokens in it one against the other, and the token drawn, all from LDS.
+// The cut by mass wants a share of the row's exact mass, which no part knows; the sum of the parts' is within MASS_ERROR of it,
+// and where the two ends of that interval keep different tokens, the row is added up exactly. A row whose threshold lies
+// below what some part has handed on (its largest tokens 16 units and more above the threshold), or with more equal tokens than
+// there is room for, is one workgroup's from the start. 8 rows of 128,256, top-k 40 and top-p 0.95: 27 us in the three
+// kernels above, 15 in these two; 64 rows 50 and 24, 128 rows 75 and 34, 8 rows of 32,000 with top-k 50 24 and 13. Bound by the two kernels' chains:
+// a trip to memory and a histogram each, then one scan, the order in the step and a scan for the token.
+#define TOP_MOST_K 128
+#define TOP_STEPS 256
+#define TOP_PER_UNIT 16.0f
+#define TOP_CAND 384       // handed on by a part
+#define TOP_TIES 1024      // in the step that holds the threshold
+#define MASS_ERROR 2e-5    // three roundings of at most 40 in the exponent on either way: 1e-5
+#define NO_STEP (-2000000000)
+struct TopRecord {
+  double rest;             // mass of all its tokens, relative to its largest
+  float max;
+  int floor;               // all tokens from this step on are handed on; NO_STEP: all there are
+  int n, unused;
+  float l[TOP_CAND];       // in index order
+  uint16_t i[TOP_CAND];
+};
+static_assert(sizeof(TopRecord) <= sizeof(PartRecord), "either records fit the scratch");
+
+__device__ __forceinline__ int top_step(float l, float inv_t) {
+  return (int)floorf(fminf(fmaxf(l * inv_t * TOP_PER_UNIT, -1e9f), 1e9f));
+}
+
+__global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                  float inv_t, int top_k, int by_mass,
+                                                                  TopRecord* __restrict__ records) {
+  constexpr int WAVES = PART_THREADS / TA_WAVE;
+  const float* row = logits + (size_t)blockIdx.y * ld;
+  TopRecord& rec = records[(size_t)blockIdx.y * gridDim.x + blockIdx.x];
+  const int groups = (vocab + 3) / 4, wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  const int live = vocab - (int)blockIdx.x * PART < PART ? vocab - (int)blockIdx.x * PART : PART;
+  __shared__ float s_f[WAVES];
+  __shared__ uint32_t cnt[TOP_STEPS];
+  __shared__ u64 s_rest[WAVES];
+  __shared__ int s_low, s_n[4][WAVES];
+  static_assert(TOP_STEPS == PART_THREADS, "a thread a step");
+  cnt[threadIdx.x] = 0;
+  Four f[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) f[u] = load_four_if(row, part_group(blockIdx.x, u), groups, vocab);
+  float m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) m = fmaxf(m, f[u].v[e]);
+  m = wave_max(m);
+  if (lane == 0) s_f[wave] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) m = fmaxf(m, s_f[w]);
+  if (m == -INFINITY) {                            // nothing here to be kept before anything of another part
+    if (threadIdx.x == 0) {
+      rec.rest = 0.0;
+      rec.max = m;
+      rec.floor = 1 - 1000000000;
+      rec.n = 0;
+    }
+    return;
+  }
+  const int top = top_step(m, inv_t);
+  int at[4][4];
+  u64 all = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      at[u][e] = f[u].ok[e] ? top - top_step(f[u].v[e], inv_t) : TOP_STEPS;
+      if (at[u][e] < TOP_STEPS) atomicAdd(&cnt[at[u][e]], 1u);
+      if (by_mass && f[u].ok[e]) all += fixed_mass(f[u].v[e], m, inv_t);
+    }
+  if (by_mass) {
+    all = wave_sum_u64(all);
+    if (lane == 0) s_rest[wave] = all;
+  }
+  __syncthreads();
+  if (wave == 0) {                                 // a lane four steps
+    const uint4 c = *reinterpret_cast<const uint4*>(&cnt[4 * lane]);
+    const uint32_t mine = c.x + c.y + c.z + c.w;
+    uint32_t inc = mine;
+#pragma unroll
+    for (int o = 1; o < TA_WAVE; o <<= 1) {
+      const uint32_t up = __shfl_up(inc, o, TA_WAVE);
+      if (lane >= o) inc += up;
+    }
+    const u64 found = __ballot(inc >= (uint32_t)top_k);
+    const int who = found ? __ffsll((unsigned long long)found) - 1 : TA_WAVE - 1;
+    if (lane == who) {
+      uint32_t run = inc - mine;
+      int step = 4 * lane + 3;
+      uint32_t n = inc;
+      if (found) {
+        const uint32_t k = (uint32_t)top_k;
+        if (run + c.x >= k) { step = 4 * lane; n = run + c.x; }
+        else if (run + c.x + c.y >= k) { step = 4 * lane + 1; n = run + c.x + c.y; }
+        else if (run + c.x + c.y + c.z >= k) { step = 4 * lane + 2; n = run + c.x + c.y + c.z; }
+      }
+      s_low = step;
+      u64 rest = 0;
+      if (by_mass)
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) rest += s_rest[w];
+      rec.rest = (double)rest;
+      rec.max = m;
+      rec.floor = (int)n < live ? top - step : NO_STEP;
+      rec.n = (int)n;
+    }
+  }
+  __syncthreads();
+  const int low = s_low;
+  int before[4];
+  u64 take[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    int sum = 0;
+    before[u] = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      take[u][e] = __ballot(at[u][e] <= low);
+      before[u] += __popcll(take[u][e] & (((u64)1 << lane) - 1));
+      sum += __popcll(take[u][e]);
+    }
+    if (lane == 0) s_n[u][wave] = sum;
+  }
+  __syncthreads();
+  int base = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (w == wave) {
+        int to = base + before[u];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if ((take[u][e] >> lane) & 1) {
+            if (to < TOP_CAND) {
+              rec.l[to] = f[u].v[e];
+              rec.i[to] = (uint16_t)(4 * (u * PART_THREADS + (int)threadIdx.x) + e);
+            }
+            ++to;
+          }
+      }
+      base += s_n[u][w];
+    }
+}
+
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const float* __restrict__ logits, size_t ld, int vocab,
+                                                                         float inv_t, int top_k, float top_p, int parts,
+                                                                         const TopRecord* __restrict__ records,
+                                                                         const float* __restrict__ uniform, SampleUniforms given,
+                                                                         int row0, int* __restrict__ out, int* __restrict__ out_host) {
+  const float* row = logits + (size_t)blockIdx.x * ld;
+  const TopRecord* all = records + (size_t)blockIdx.x * parts;
+  const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  __shared__ float cand_l[ROW_CAND];
+  __shared__ uint32_t cand_i[ROW_CAND];
+  __shared__ uint8_t keep[ROW_CAND];
+  __shared__ uint32_t h_cnt[TOP_STEPS], tie_key[TOP_TIES], tie_at[TOP_TIES];
+  __shared__ u64 h_mass[TOP_STEPS], tie_q[TOP_TIES], s_wave[SAMPLE_WAVES];
+  __shared__ int s_first[MAX_PARTS], s_n[MAX_PARTS];
+  __shared__ int s_ok, s_cands, s_floor, s_bin, s_ties, s_unsure, s_pick;
+  __shared__ uint32_t s_count;
+  __shared__ u64 s_mass, s_p[2];
+  __shared__ float s_max;
+  const bool by_mass = top_p < 1.0f;
+  const float uni = uniform ? uniform[blockIdx.x] : given.u[row0 + blockIdx.x];
+  // the first 64 tokens of a wave's parts are on their way before it is known how many there are
+  constexpr int AHEAD = 2;
+  float ahead_l[AHEAD];
+  uint32_t ahead_i[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) {
+    const int p = wave + i * SAMPLE_WAVES;
+    ahead_l[i] = all[p < parts ? p : 0].l[lane];
+    ahead_i[i] = all[p < parts ? p : 0].i[lane];
+  }
+  if (threadIdx.x < TOP_STEPS) {
+    h_cnt[threadIdx.x] = 0;
+    h_mass[threadIdx.x] = 0;
+  }
+  if (wave == 0) {
+    float m = -INFINITY;
+    for (int p = lane; p < parts; p += TA_WAVE) m = fmaxf(m, all[p].max);
+    m = wave_max(m);
+    int run = 0, floor = NO_STEP;
+    bool ok = true;
+    double t = 0.0;
+    for (int p0 = 0; p0 < parts; p0 += TA_WAVE) {
+      const int p = p0 + lane;
+      const bool in = p < parts;
+      const TopRecord& r = all[in ? p : 0];
+      const int n = in ? r.n : 0;
+      ok = ok && n <= TOP_CAND;
+      if (in) floor = r.floor > floor ? r.floor : floor;
+      if (in && by_mass) t += r.rest * (double)__builtin_amdgcn_exp2f((r.max - m) * inv_t * 1.44269504088896341f);
+      int inc = n;
+#pragma unroll
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const int up = __shfl_up(inc, o, TA_WAVE);
+        if (lane >= o) inc += up;
+      }
+      if (in) {
+        s_first[p] = run + inc - n;
+        s_n[p] = n;
+      }
+      run += __shfl(inc, TA_WAVE - 1, TA_WAVE);
+    }
+#pragma unroll
+    for (int o = 1; o < TA_WAVE; o <<= 1) {
+      t += __shfl_xor(t, o, TA_WAVE);
+      const int other = __shfl_xor(floor, o, TA_WAVE);
+      floor = other > floor ? other : floor;
+    }
+    ok = __ballot(!ok) == 0;
+    if (lane == 0) {
+      s_max = m;
+      s_floor = floor;
+      s_cands = run;
+      s_ok = ok && run <= ROW_CAND && m > -INFINITY && m < INFINITY;
+      s_ties = 0;
+      s_unsure = 0;
+      s_pick = 0;
+      // the mass with which the cut is reached lies between these
+      const double want = (double)top_p * t;
+      s_p[0] = by_mass ? (u64)fmax(ceil(want * (1.0 - MASS_ERROR)), 1.0) : NO_MASS_LIMIT;
+      s_p[1] = by_mass ? (u64)fmax(ceil(want * (1.0 + MASS_ERROR)), 1.0) : NO_MASS_LIMIT;
+    }
+  }
+  __syncthreads();
+  auto whole = [&]() {
+    sample_whole_row<false>(row, vocab, inv_t, top_k, top_p, uni, out + blockIdx.x);
+    __syncthreads();
+    if (threadIdx.x == 0 && out_host) out_host[blockIdx.x] = out[blockIdx.x];
+  };
+  if (!s_ok) return whole();
+  const float m = s_max;
+  const int cands = s_cands, top = top_step(m, inv_t);
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) {
+    const int p = wave + i * SAMPLE_WAVES;
+    if (p < parts && lane < s_n[p]) {
+      cand_l[s_first[p] + lane] = ahead_l[i];
+      cand_i[s_first[p] + lane] = p * PART + ahead_i[i];
+    }
+  }
+  for (int p = wave; p < parts; p += SAMPLE_WAVES)
+    for (int c = lane + (p < AHEAD * SAMPLE_WAVES ? TA_WAVE : 0); c < s_n[p]; c += TA_WAVE) {
+      cand_l[s_first[p] + c] = all[p].l[c];
+      cand_i[s_first[p] + c] = p * PART + all[p].i[c];
+    }
+  __syncthreads();
+  auto step = [&](float l) {
+    const int at = top - top_step(l, inv_t);
+    return at < TOP_STEPS - 1 ? at : TOP_STEPS - 1;
+  };
+  for (int c = threadIdx.x; c < cands; c += SAMPLE_THREADS) {
+    const float l = cand_l[c];
+    const int at = step(l);
+    atomicAdd(&h_cnt[at], 1u);
+    atomicAdd(&h_mass[at], fixed_mass(l, m, inv_t));
+  }
+  __syncthreads();
+  const uint32_t k_lim = (uint32_t)(top_k < vocab ? top_k : vocab);
+  for (int exact = 0;; exact = 1) {
+    // ---- the step that holds the threshold: with it the count reaches k_lim or the mass its share
+    if (wave == 0) {
+      uint32_t c[4], cs = 0;
+      u64 q[4], qs = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        cs += c[i] = h_cnt[4 * lane + i];
+        qs += q[i] = h_mass[4 * lane + i];
+      }
+      uint32_t ci = cs;
+      u64 qi = qs;
+#pragma unroll
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const uint32_t cu = __shfl_up(ci, o, TA_WAVE);
+        const u64 qu = shfl_up_u64(qi, o);
+        if (lane >= o) {
+          ci += cu;
+          qi += qu;
+        }
+      }
+      const u64 p0 = s_p[0], p1 = s_p[1];
+      const u64 at_least = __ballot(ci >= k_lim || qi >= p0), surely = __ballot(ci >= k_lim || qi >= p1);
+      if (!surely) {
+        if (lane == 0) s_bin = at_least && !exact ? -2 : -1;
+      } else if (lane == __ffsll((unsigned long long)surely) - 1) {
+        uint32_t ca = ci - cs;
+        u64 ma = qi - qs;
+        int hit = 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          if (hit == i && !(ca + c[i] >= k_lim || ma + q[i] >= p1)) {
+            ca += c[i];
+            ma += q[i];
+            hit = i + 1;
+          }
+        // reached before at the lower end of the interval: it matters which it is
+        s_bin = ma >= p0 ? -2 : 4 * lane + hit;
+        s_count = ca;
+        s_mass = ma;
+      }
+    }
+    __syncthreads();
+    const int bin = s_bin;
+    if (bin == -1 || bin == TOP_STEPS - 1 || (bin >= 0 && top - bin < s_floor)) return whole();
+    if (bin >= 0) {
+      for (int c = threadIdx.x; c < cands; c += SAMPLE_THREADS) {
+        const float l = cand_l[c];
+        const int at = step(l);
+        keep[c] = at < bin;
+        if (at == bin) {
+          const int to = atomicAdd(&s_ties, 1);
+          if (to < TOP_TIES) {
+            tie_key[to] = order_key(l);
+            tie_at[to] = c;
+            tie_q[to] = fixed_mass(l, m, inv_t);
+          }
+        }
+      }
+      __syncthreads();
+      const int ties = s_ties;
+      if (ties > TOP_TIES) return whole();
+      // ---- what goes before each of them: higher logits, lower indices among equals
+      if ((int)threadIdx.x < ties) {
+        const uint32_t key = tie_key[threadIdx.x], place = tie_at[threadIdx.x];
+        uint32_t n = s_count;
+        u64 q = s_mass;
+        for (int j = 0; j < ties; ++j) {
+          const bool first = tie_key[j] > key || (tie_key[j] == key && tie_at[j] < place);
+          n += first;
+          q += first ? tie_q[j] : 0;
+        }
+        const bool low = n < k_lim && q < s_p[0], high = n < k_lim && q < s_p[1];
+        keep[place] = low;
+        if (low != high) s_unsure = 1;
+      }
+      __syncthreads();
+      if (!s_unsure) break;
+    }
+    // ---- the row's mass itself
+    u64 sum = 0;
+    const int groups = (vocab + 3) / 4;
+    for (int j = threadIdx.x; j < groups; j += SAMPLE_THREADS) {
+      const Four f = load_four(row, j, vocab);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum += f.ok[e] ? fixed_mass(f.v[e], m, inv_t) : 0;
+    }
+    sum = wave_sum_u64(sum);
+    if (lane == 0) s_wave[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      u64 total = 0;
+      for (int w = 0; w < SAMPLE_WAVES; ++w) total += s_wave[w];
+      u64 p_lim = (u64)ceil((double)top_p * (double)total);
+      if (p_lim < 1) p_lim = 1;
+      if (p_lim > total) p_lim = total;
+      s_p[0] = s_p[1] = p_lim;
+      s_ties = 0;
+      s_unsure = 0;
+    }
+    __syncthreads();
+  }
+  // ---- the token: the running sum of the kept ones in index order, four neighbours a thread
+  u64 q[ROW_CAND / SAMPLE_THREADS], mine = 0;
+  constexpr int EACH = ROW_CAND / SAMPLE_THREADS;
+#pragma unroll
+  for (int i = 0; i < EACH; ++i) {
+    const int c = EACH * (int)threadIdx.x + i;
+    q[i] = c < cands && keep[c < cands ? c : 0] ? fixed_mass(cand_l[c], m, inv_t) : 0;
+    mine += q[i];
+  }
+  u64 inc = mine;
+#pragma unroll
+  for (int o = 1; o < TA_WAVE; o <<= 1) {
+    const u64 up = shfl_up_u64(inc, o);
+    if (lane >= o) inc += up;
+  }
+  if (lane == TA_WAVE - 1) s_wave[wave] = inc;
+  __syncthreads();
+  u64 sum = 0, run = 0;
+#pragma unroll
+  for (int w = 0; w < SAMPLE_WAVES; ++w) {
+    if (w == wave) run = sum;
+    sum += s_wave[w];
+  }
+  u64 target = (u64)((double)uni * (double)sum);
+  if (sum > 0 && target >= sum) target = sum - 1;
+  if (mine > 0 && run + inc > target && run + inc - mine <= target) {
+    u64 at = run + inc - mine;
+    int pick = 0;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+      if (q[i] > 0 && at + q[i] > target && at <= target) pick = (int)cand_i[EACH * (int)threadIdx.x + i];
+      at += q[i];
+    }
+    out[blockIdx.x] = pick;
+    if (out_host) out_host[blockIdx.x] = pick;
+  }
+}
+
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(const float* __restrict__ logits, size_t ld, int vocab,
                                                                      float inv_t, int top_k, float top_p,
                                                                      const float* __restrict__ uniform, int* __restrict__ out) {
@@ -1616,6 +2029,8 @@ static int sample_launch(hipStream_t stream, const float* logits, long long ld, 
     TA_REQUIRE(scratch_bytes >= ta_sample_scratch(n, vocab), "ta_sample: %lld bytes of scratch, %lld are needed", scratch_bytes,
                ta_sample_scratch(n, vocab));
     const int parts = sample_parts(vocab), cut = top_k < vocab || top_p < 1.0f;
+    // half as many again as top_k, with room to spare, are what a part hands on
+    const bool few = top_k < vocab && top_k <= TOP_MOST_K && parts * top_k <= ROW_CAND / 2;
     PartRecord* rec = (PartRecord*)scratch;
     const int turn = rows_at_a_time(vocab);
     SampleUniforms args = {};
@@ -1625,6 +2040,14 @@ static int sample_launch(hipStream_t stream, const float* logits, long long ld, 
       const int rows = n - r0 < turn ? n - r0 : turn;
       const float* from = logits + (size_t)r0 * ld;
       const dim3 g(parts, rows);
+      if (few) {
+        TopRecord* tops = (TopRecord*)scratch;
+        sample_top_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p < 1.0f, tops);
+        sample_top_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, parts, tops,
+                                                                    given ? nullptr : uniform + r0, args, r0, out + r0,
+                                                                    out_host ? out_host + r0 : nullptr);
+        continue;
+      }
       sample_parts_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, cut, top_p < 1.0f, rec, args,
                                                       given && r0 == 0 ? n : 0, uniform);
       sample_gather_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, cut, rec);
