@@ -433,7 +433,12 @@ __device__ __forceinline__ void la_chunk(const bf16_t* __restrict__ Ks, int RS, 
     }
   }
 
-template <int KS, int CT, int RT>
+// TEAM: the four waves of a workgroup take ONE tile and share its chunks, which all threads bring into one of two
+// buffers behind a barrier a chunk; each forms the tile's scores and sums a quarter of the coordinates. A step of single
+// tokens has one tile a sequence where 16 heads share a row, and by a wave for itself the other three of its workgroup are gone: attention
+// and merge, 16 heads, rank 256, 900 keys, 1 / 4 / 64 sequences 26.2 / 26.9 / 103 us that way, 16.7 / 17.3 / 48 by four (30 with
+// the fewer shares that four waves want); 128 heads, rank 512, 4 x 2,000 keys 199 and 62.
+template <int KS, int CT, int RT, bool TEAM = false>
 __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qa, bf16_t* __restrict__ out, const bf16_t* __restrict__ kcache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ cu_q,
@@ -444,17 +449,18 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int c = lane % 16, g = lane / 16;
   const int RS = dc + 8;                                  // elements between rows of the LDS copy
-  bf16_t* Ks = reinterpret_cast<bf16_t*>(la_lds) + (size_t)wave * 32 * RS;
+  bf16_t* Ks = reinterpret_cast<bf16_t*>(la_lds) + (TEAM ? 0 : (size_t)wave * 32 * RS);
   const int b = blockIdx.y, split = blockIdx.z;
   const int q0 = cu_q[b], qlen = cu_q[b + 1] - q0;
   const int nrows = qlen * H;
   // HALVES: rows too wide for one wave's registers (128 accumulators and 72 query registers): two
   // waves take the same tile, form the same scores, and each sums one half of the coordinates.
-  constexpr bool HALVES = KS > 10;
+  constexpr bool HALVES = KS > 10 && !TEAM;
+  static_assert(!TEAM || (RT == 1 && CT % 16 == 0), "a quarter of the coordinates is whole blocks of 64");
   const int wid = blockIdx.x * 4 + wave;
-  const int tile = HALVES ? wid / 2 : wid, half = HALVES ? wid % 2 : 0;
+  const int tile = TEAM ? blockIdx.x : HALVES ? wid / 2 : wid, half = TEAM ? wave : HALVES ? wid % 2 : 0;
   const int row0 = tile * 16 * RT;
-  if (row0 >= nrows) return;                              // a wave leaves alone: nothing below waits for others
+  if (row0 >= nrows) return;                              // a wave (TEAM: a workgroup) leaves: nothing below waits for others
   const int p0 = pos0[b];
   int my_start[RT], my_end[RT];
   bool ok[RT];
@@ -483,7 +489,7 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   const int c0 = tile_start / 32, c1 = (tile_end + 31) / 32;
   const int n = c1 - c0;
   const int ca = c0 + (int)((long long)n * split / splits), cb = c0 + (int)((long long)n * (split + 1) / splits);
-  constexpr int CTP = HALVES ? CT / 2 : CT;               // coordinate tiles this wave sums
+  constexpr int CTP = TEAM ? CT / 4 : HALVES ? CT / 2 : CT;     // coordinate tiles this wave sums
   const int qb0 = half * (CTP / 4);                       // its first block of 64 coordinates
   la_floatx4 O[RT][CTP];
 #pragma unroll
@@ -497,8 +503,10 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   const int pieces = dc / 8;                              // 16-byte pieces of a row
   // A chunk is 32 * pieces pieces, NL = 2 KS of them a lane at most. With PRE they are asked for
   // one chunk ahead and wait in registers while the chunk before is multiplied.
-  constexpr int NL = 2 * KS;
-  constexpr bool PRE = KS <= 10;
+  constexpr int NL = TEAM ? (KS + 1) / 2 : 2 * KS;
+  constexpr int BRING = TEAM ? 256 : 64;                  // lanes that bring a chunk
+  const int bring = TEAM ? (int)threadIdx.x : lane;
+  constexpr bool PRE = KS <= 10 || TEAM;
   uint4 pre[PRE ? NL : 1];
   auto fetch = [&](int ch, uint4* buf, auto I0, auto I1) {
     constexpr int i0 = decltype(I0)::value, i1 = decltype(I1)::value;
@@ -507,7 +515,7 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
     const bf16_t* src = kcache + (page * TA_PAGE + key0 % TA_PAGE) * (size_t)dc;
 #pragma unroll
     for (int i = i0; i < i1; ++i) {
-      const int idx = lane + 64 * i;
+      const int idx = bring + BRING * i;
       const int k = idx / pieces, pc = idx - k * pieces;
       const bool live = idx < 32 * pieces && key0 + k < tile_end;       // keys not written yet read as zero
       const uint4 v = *reinterpret_cast<const uint4*>(live ? src + (size_t)k * dc + pc * 8 : kcache);
@@ -518,7 +526,7 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
     constexpr int i0 = decltype(I0)::value, i1 = decltype(I1)::value;
 #pragma unroll
     for (int i = i0; i < i1; ++i) {
-      const int idx = lane + 64 * i;
+      const int idx = bring + BRING * i;
       const int k = idx / pieces, pc = idx - k * pieces;
       if (idx < 32 * pieces) *reinterpret_cast<uint4*>(Ks + k * RS + pc * 8) = buf[i - i0];
     }
@@ -529,6 +537,15 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   if (PRE && ca < cb) fetch(ca, pre, la_i0{}, la_nl{});
   for (int ch = ca; ch < cb; ++ch) {
     const int key0 = ch * 32;
+    if (TEAM) {
+      // who comes to this buffer again has passed the other one's barrier, behind which all have read this one
+      Ks = reinterpret_cast<bf16_t*>(la_lds) + (size_t)((ch - ca) & 1) * 32 * RS;
+      stash(pre, la_i0{}, la_nl{});
+      if (ch + 1 < cb) fetch(ch + 1, pre, la_i0{}, la_nl{});
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      la_chunk<KS, CTP, RT>(Ks, RS, dc, rank, key0, c, g, qf, ok, my_start, my_end, scale_log2, m, l, O, qb0);
+      continue;
+    }
     __builtin_amdgcn_wave_barrier();                      // the chunk before has been read
     if (PRE) {
       stash(pre, la_i0{}, la_nl{});
@@ -743,8 +760,9 @@ static int latent_mfma_wg_run(hipStream_t stream, dim3 g, size_t lds, const void
   return 0;
 }
 
-// One wave per row: the shares of a row's keys are put together.
-__global__ __launch_bounds__(64) void latent_merge_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
+// The shares of a row's keys are put together by four waves, a thread a coordinate (each wave forms the weights for itself):
+// attention and merge of 4 x 900 keys in 17 shares 17.3 us with one wave a row, 14.3 with four; 4 x 3,000, rank 512, 65 shares 58 and 41.
+__global__ __launch_bounds__(256) void latent_merge_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
                                                           const int* __restrict__ cu_q, int H, int rank, int splits,
                                                           int tiles_max, int rows_per_tile,
                                                           const bf16_t* __restrict__ gate, int gate_stride,
@@ -756,14 +774,15 @@ __global__ __launch_bounds__(64) void latent_merge_kernel(const float* __restric
   const float* base = partial + (((size_t)b * tiles_max + tile) * splits * rows_per_tile + rl) * (rank + 2);
   const size_t step = (size_t)rows_per_tile * (rank + 2);
   extern __shared__ float wts[];          // [splits] weight of every share
+  const int lane = threadIdx.x % TA_WAVE;
   float M = -INFINITY;
-  for (int s = threadIdx.x; s < splits; s += 64) M = fmaxf(M, base[s * step + rank]);
+  for (int s = lane; s < splits; s += 64) M = fmaxf(M, base[s * step + rank]);
   M = wave_max(M);
   float L = 0.f;
-  for (int s = threadIdx.x; s < splits; s += 64) {
+  for (int s = lane; s < splits; s += 64) {
     const float ms = base[s * step + rank];
     const float w = ms != -INFINITY ? exp2f(ms - M) : 0.f;
-    wts[s] = w;
+    if (threadIdx.x < TA_WAVE) wts[s] = w;
     L += w * base[s * step + rank + 1];
   }
   L = wave_sum(L);
@@ -774,7 +793,7 @@ __global__ __launch_bounds__(64) void latent_merge_kernel(const float* __restric
     f *= 1.0f / (1.0f + expf(-gv));
   }
   bf16_t* o = out + ((size_t)q0 * H + row) * rank;
-  for (int cdx = threadIdx.x; cdx < rank; cdx += 64) {
+  for (int cdx = threadIdx.x; cdx < rank; cdx += 256) {
     float acc = 0.f;
 #pragma unroll 8
     for (int s = 0; s < splits; ++s) acc = fmaf(wts[s], base[s * step + cdx], acc);     // shares in order
@@ -782,12 +801,12 @@ __global__ __launch_bounds__(64) void latent_merge_kernel(const float* __restric
   }
 }
 
-template <int KS, int CT, int RT>
+template <int KS, int CT, int RT, bool TEAM = false>
 static int latent_mfma_run(hipStream_t stream, dim3 g, size_t lds, const void* qa, void* out, const void* kcache,
                            const int* block_table, int max_blocks, const int* cu_q, const int* pos0, int H,
                            int rank, int dc, float scale_log2, int window, const void* gate, int gate_stride,
                            int splits, int tiles_max, float* partial, const float* sink) {
-  auto kern = latent_attention_mfma_kernel<KS, CT, RT>;
+  auto kern = latent_attention_mfma_kernel<KS, CT, RT, TEAM>;
   static size_t allowed = 64 * 1024;                    // per instantiation: asked for once, not at every launch
   if (lds > allowed) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -801,6 +820,210 @@ static int latent_mfma_run(hipStream_t stream, dim3 g, size_t lds, const void* q
   return 0;
 }
 
+// ------------------------------------------------------------------ the heads' maps in steps of few single tokens
+// The maps on either side of the attention are a product per head, [tokens] x 128 x 256 and the like: 64 KB a head, launches that wait
+// for one trip to memory. Up to 16 tokens they ride on their neighbours: the queries' on the rotation, the results' on the merge. A
+// workgroup takes 64 columns of a head for 4 tokens (attention, merge and map of 8 tokens 30.6 us by workgroups of 8, 23.6 of 4); a thread 8 of them and every 32nd k, all asked for at once, and the 32 sums of a column
+// are put together in LDS. (4 tokens, 16 heads of 128, rank 256, the products by the library: rotation and product 7.7 us, 4.5 here; attention, merge and
+// product 21.8, 19.7 here; 16 tokens 7.7 and 5.1, 26.0 and 26.0.)
+#define LA_FEW 16
+#define LA_ROWS_MAP 4
+struct LaMap {
+  static constexpr int R = LA_ROWS_MAP, KI = 8;
+  // w: [k][n] of one head; xs: [R][ld] rows in LDS; sums of columns n0 + 8 (t % 8) .. + 7 over k = t / 8 + 32 i
+  uint4 w[KI];
+  __device__ __forceinline__ void ask(const bf16_t* wp, int K, int N, int n0) {
+    const int col = n0 + 8 * ((int)threadIdx.x % 8);
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const int k = (int)threadIdx.x / 8 + 32 * i;
+      w[i] = *reinterpret_cast<const uint4*>(wp + (k < K && col < N ? (size_t)k * N + col : 0));
+    }
+  }
+  // red: [16][R][64] floats; thread t's result: row t / 64, column n0 + t % 64
+  __device__ __forceinline__ float multiply(const float* xs, int ld, int K, float* red) {
+    float acc[R][8];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const int k = (int)threadIdx.x / 8 + 32 * i;
+      if (k < K) {
+        float f[8];
+        const uint32_t u[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f[2 * e] = __uint_as_float(u[e] << 16);
+          f[2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const float x = xs[r * ld + k];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[r][e] = fmaf(f[e], x, acc[r][e]);
+        }
+      }
+    }
+    const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[r][e] += __shfl_xor(acc[r][e], 32, TA_WAVE);
+    if (lane < 32) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float* to = red + ((wave * 4 + lane / 8) * R + r) * 64 + 8 * (lane % 8);
+        *reinterpret_cast<float4*>(to) = make_float4(acc[r][0], acc[r][1], acc[r][2], acc[r][3]);
+        *reinterpret_cast<float4*>(to + 4) = make_float4(acc[r][4], acc[r][5], acc[r][6], acc[r][7]);
+      }
+    }
+    __syncthreads();
+    float sum = 0.f;
+#pragma unroll
+    for (int p = 0; p < 16; ++p) sum += red[(p * R + (int)threadIdx.x / 64) * 64 + threadIdx.x % 64];
+    return sum;
+  }
+};
+
+__global__ __launch_bounds__(256) void latent_query_map_kernel(const bf16_t* __restrict__ q, int q_stride, int H, int dn, int rot,
+                                                               int rot_dims, const float* __restrict__ angles,
+                                                               const bf16_t* __restrict__ uk, bf16_t* __restrict__ qa, int rank,
+                                                               int dc, int nt) {
+  constexpr int R = LA_ROWS_MAP;
+  const int h = blockIdx.y, n0 = blockIdx.x * 64, t0 = blockIdx.z * R;
+  q += (size_t)t0 * q_stride;
+  qa += (size_t)t0 * H * dc;
+  if (angles) angles += (size_t)t0 * rot_dims;
+  nt = nt - t0 < R ? nt - t0 : R;
+  if (n0 >= rank) {                                       // the last workgroup of a head: its rotated parts and the padding
+    const int pad = dc - rank - rot, pairs = (rot + 1) / 2;
+    for (int idx = threadIdx.x; idx < nt * pad; idx += 256)
+      qa[((size_t)(idx / pad) * H + h) * dc + rank + rot + idx % pad] = from_f32<bf16_t>(0.f);
+    for (int idx = threadIdx.x; idx < nt * pairs; idx += 256) {
+      const int t = idx / pairs, i = idx % pairs;
+      const float* ang = angles + (size_t)t * rot_dims;
+      const bf16_t* src = q + (size_t)t * q_stride + h * (dn + rot) + dn;
+      bf16_t* dst = qa + ((size_t)t * H + h) * dc + rank;
+      const float u = to_f32(src[2 * i]);
+      if (2 * i + 1 >= rot) { dst[2 * i] = from_f32<bf16_t>(u); continue; }
+      const float v = to_f32(src[2 * i + 1]);
+      if (2 * i + 1 < rot_dims) {
+        const float c = ang[2 * i], s = ang[2 * i + 1];
+        dst[2 * i] = from_f32<bf16_t>(u * c - v * s);
+        dst[2 * i + 1] = from_f32<bf16_t>(v * c + u * s);
+      } else {
+        dst[2 * i] = from_f32<bf16_t>(u);
+        dst[2 * i + 1] = from_f32<bf16_t>(v);
+      }
+    }
+    return;
+  }
+  __shared__ float xs[R][256];
+  __shared__ __attribute__((aligned(16))) float red[16 * R * 64];
+  LaMap map;
+  map.ask(uk + (size_t)h * dn * rank, dn, rank, n0);
+  for (int idx = threadIdx.x; idx < R * dn; idx += 256) {
+    const int t = idx / dn, k = idx % dn;
+    xs[t][k] = t < nt ? to_f32(q[(size_t)t * q_stride + h * (dn + rot) + k]) : 0.f;
+  }
+  __syncthreads();
+  const float sum = map.multiply(&xs[0][0], 256, dn, red);
+  const int t = (int)threadIdx.x / 64, n = n0 + (int)threadIdx.x % 64;
+  if (t < nt && n < rank) qa[((size_t)t * H + h) * dc + n] = from_f32<bf16_t>(sum);
+}
+
+// Token t is sequence t's only one (or, where it brings none, missing). The merged row is rounded once, as latent_merge_kernel stores it.
+__global__ __launch_bounds__(256) void latent_merge_map_kernel(const float* __restrict__ partial, const bf16_t* __restrict__ uv,
+                                                               bf16_t* __restrict__ o, const int* __restrict__ cu_q, int H, int rank,
+                                                               int dv, int splits, int tiles_max, int rows_per_tile,
+                                                               const bf16_t* __restrict__ gate, int gate_stride,
+                                                               const float* __restrict__ sink, int nt) {
+  constexpr int R = LA_ROWS_MAP;
+  const int h = blockIdx.y, n0 = blockIdx.x * 64, t0 = blockIdx.z * R, wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
+  cu_q += t0;
+  nt = nt - t0 < R ? nt - t0 : R;
+  __shared__ float xs[R][256];
+  __shared__ __attribute__((aligned(16))) float red[16 * R * 64];     // first the shares' weights, [R][splits], splits <= 1,024
+  __shared__ float factor[R];
+  LaMap map;
+  map.ask(uv + (size_t)h * rank * dv, rank, dv, n0);
+  const int tile = h / rows_per_tile, rl = h % rows_per_tile;
+  const size_t step = (size_t)rows_per_tile * (rank + 2);
+  auto base = [&](int t) { return partial + (((size_t)(t0 + t) * tiles_max + tile) * splits * rows_per_tile + rl) * (rank + 2); };
+  // the first shares' sums are asked for before their weights are known: in steps of four shares 21.6 us, here 19.7
+  constexpr int AHEAD = 20;
+  const int d = (int)threadIdx.x < rank ? threadIdx.x : 0;
+  float v[R][AHEAD];
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) v[t][i] = base(t < nt ? t : 0)[(i < splits ? i : 0) * step + d];
+  static_assert(R == 4, "a wave a token");
+  if (wave < nt && cu_q[wave + 1] != cu_q[wave]) {
+    const float* from = base(wave);
+    float M = -INFINITY;
+    for (int s = lane; s < splits; s += 64) M = fmaxf(M, from[s * step + rank]);
+    M = wave_max(M);
+    float L = 0.f;
+    for (int s = lane; s < splits; s += 64) {
+      const float ms = from[s * step + rank];
+      const float w = ms != -INFINITY ? exp2f(ms - M) : 0.f;
+      red[wave * splits + s] = w;
+      L += w * from[s * step + rank + 1];
+    }
+    L = wave_sum(L);
+    float f = la_inverse(L, M, sink, h);
+    if (gate) {
+      const float gv = to_f32(gate[(size_t)cu_q[wave] * gate_stride + h]);
+      f *= 1.0f / (1.0f + expf(-gv));
+    }
+    if (lane == 0) factor[wave] = f;
+  }
+  __syncthreads();
+  float acc[R];
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    acc[t] = 0.f;
+    if (t >= nt) continue;
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      if (i < splits) acc[t] = fmaf(red[t * splits + i], v[t][i], acc[t]);               // shares in order
+    const float* from = base(t) + d;
+#pragma unroll 8
+    for (int s = AHEAD; s < splits; ++s) acc[t] = fmaf(red[t * splits + s], from[s * step], acc[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < R; ++t)
+    if ((int)threadIdx.x < rank) xs[t][d] = t < nt && cu_q[t + 1] != cu_q[t] ? to_f32(from_f32<bf16_t>(acc[t] * factor[t])) : 0.f;
+  __syncthreads();                                        // the weights have been read
+  const float sum = map.multiply(&xs[0][0], 256, rank, red);
+  const int t = (int)threadIdx.x / 64, n = n0 + (int)threadIdx.x % 64;
+  if (t < nt && n < dv && cu_q[t + 1] != cu_q[t]) o[((size_t)cu_q[t] * H + h) * dv + n] = from_f32<bf16_t>(sum);
+}
+
+// Whether ta_latent_query_map and ta_latent_attention_map take a step of `nt` single tokens.
+extern "C" int ta_latent_maps_take(int nt, int H, int dn, int rank, int dv, int splits) {
+  return nt >= 1 && nt <= LA_FEW && H >= 1 && H <= 65535 && dn >= 1 && dn <= 256 && rank >= 8 && rank <= 256 && rank % 8 == 0 &&
+         dv >= 8 && dv % 8 == 0 && splits > 1 && splits <= 1024;
+}
+
+// ta_latent_query_rot, and the unrotated parts times uk [H][dn][rank] (bfloat16, on 16 bytes) into the first ``rank`` coordinates:
+// bfloat16 rows.
+extern "C" int ta_latent_query_map(hipStream_t stream, const void* q, int q_stride, int H, int dn, int rot, int rot_dims,
+                                   const float* angles, const void* uk, void* qa, int rank, int dc, int nt) {
+  TA_REQUIRE(nt >= 0 && ta_latent_maps_take(nt > 0 ? nt : 1, H, dn, rank, 8, 2), "ta_latent_query_map: %d tokens of %d heads, %d -> %d", nt, H, dn, rank);
+  TA_REQUIRE(rot >= 0 && rot_dims >= 0 && rot_dims <= rot && rot_dims % 2 == 0 && dc >= rank + rot && q_stride >= H * (dn + rot),
+             "ta_latent_query_map: rotated part of %d (%d), rows of %d / %d", rot, rot_dims, q_stride, dc);
+  TA_REQUIRE((uintptr_t)uk % 16 == 0 && (rot_dims == 0 || angles != nullptr), "ta_latent_query_map: matrices must start on 16 bytes, angles are required");
+  if (nt == 0) return 0;
+  const dim3 g((rank + 63) / 64 + 1, H, (nt + LA_ROWS_MAP - 1) / LA_ROWS_MAP);
+  latent_query_map_kernel<<<g, 256, 0, stream>>>((const bf16_t*)q, q_stride, H, dn, rot, rot_dims, rot_dims ? angles : nullptr,
+                                                 (const bf16_t*)uk, (bf16_t*)qa, rank, dc, nt);
+  return ta_check_launch("ta_latent_query_map");
+}
+
 // Rows per tile that the matrix-core kernel gives a wave for this geometry (0: it does not take
 // it), and the float32 values of scratch that `splits` shares of the keys need.
 extern "C" int ta_latent_mfma_rows(int rank, int dc, int max_qlen, int H) {
@@ -808,6 +1031,8 @@ extern "C" int ta_latent_mfma_rows(int rank, int dc, int max_qlen, int H) {
   if (dc <= 192 && rank <= 128) return (long long)max_qlen * H >= 64 ? 32 : 16;
   return 16;
 }
+// Waves that a share of a tile's keys gets: the four of a workgroup where a quarter of the coordinates is whole blocks of 64.
+extern "C" int ta_latent_share_waves(int rank, int dc) { return dc <= 192 && rank <= 128 ? 1 : 4; }
 extern "C" long long ta_latent_mfma_scratch(int batch, int max_qlen, int H, int rank, int dc, int splits) {
   const int rows = ta_latent_mfma_rows(rank, dc, max_qlen, H);
   if (rows == 0 || splits <= 1) return 0;
@@ -854,20 +1079,21 @@ extern "C" int ta_latent_attention(hipStream_t stream, int dtype, const void* qa
     }
     const long long tiles = ((long long)max_qlen * H + rows - 1) / rows;
     TA_REQUIRE(tiles <= 2147483647ll, "ta_latent_attention: too many rows");
+    const bool narrow = dc <= 192 && rank <= 128, team = splits > 1 && ta_latent_share_waves(rank, dc) == 4;
     const bool halves = !(dc <= 320 && rank <= 256);      // two waves a tile: see the kernel
-    dim3 g((unsigned)(((halves ? 2 : 1) * tiles + 3) / 4), batch, splits);
-    const size_t lds = (size_t)4 * 32 * (dc + 8) * sizeof(bf16_t);
+    dim3 g((unsigned)(team ? tiles : ((halves ? 2 : 1) * tiles + 3) / 4), batch, splits);
+    const size_t lds = (size_t)(team ? 2 : 4) * 32 * (dc + 8) * sizeof(bf16_t);
     const float sl2 = scale * 1.4426950408889634f;
     int rc;
-#define LA_MFMA(KS, CT, RT) latent_mfma_run<KS, CT, RT>(stream, g, lds, qa, out, kcache, block_table, max_blocks, cu_q, pos0, H, rank, dc, sl2, window, gate, gate_stride, splits, (int)tiles, scratch, sink)
-    if (dc <= 192 && rank <= 128) rc = rows == 32 ? LA_MFMA(6, 8, 2) : LA_MFMA(6, 8, 1);
-    else if (dc <= 320 && rank <= 256) rc = LA_MFMA(10, 16, 1);
-    else rc = LA_MFMA(18, 32, 1);
+#define LA_MFMA(KS, CT, RT, ...) latent_mfma_run<KS, CT, RT, ##__VA_ARGS__>(stream, g, lds, qa, out, kcache, block_table, max_blocks, cu_q, pos0, H, rank, dc, sl2, window, gate, gate_stride, splits, (int)tiles, scratch, sink)
+    if (narrow) rc = rows == 32 ? LA_MFMA(6, 8, 2) : LA_MFMA(6, 8, 1);
+    else if (!halves) rc = team ? LA_MFMA(10, 16, 1, true) : LA_MFMA(10, 16, 1);
+    else rc = team ? LA_MFMA(18, 32, 1, true) : LA_MFMA(18, 32, 1);
 #undef LA_MFMA
     if (rc) return rc;
-    if (splits > 1) {
+    if (splits > 1 && out != nullptr) {
       dim3 gm((unsigned)(max_qlen * H), batch);
-      latent_merge_kernel<<<gm, 64, (size_t)splits * sizeof(float), stream>>>(scratch, (bf16_t*)out, cu_q, H, rank, splits, (int)tiles, rows,
+      latent_merge_kernel<<<gm, 256, (size_t)splits * sizeof(float), stream>>>(scratch, (bf16_t*)out, cu_q, H, rank, splits, (int)tiles, rows,
                                                  (const bf16_t*)gate, gate_stride, sink);
     }
     return ta_check_launch("ta_latent_attention");
@@ -889,4 +1115,25 @@ extern "C" int ta_latent_attention(hipStream_t stream, int dtype, const void* qa
 #undef LA_RUN
   if (rc) return rc;
   return ta_check_launch("ta_latent_attention");
+}
+
+// ta_latent_attention of a step in which every sequence brings one token (or none), ``splits`` > 1 shares, followed by the heads'
+// maps: o [nt, H, dv] = the merged rows times uv [H][rank][dv] (bfloat16, on 16 bytes).
+extern "C" int ta_latent_attention_map(hipStream_t stream, const void* qa, void* o, const void* kcache, const int* block_table,
+                                       int max_blocks, const int* cu_q, const int* pos0, int batch, int H, int rank, int rot, int dc,
+                                       float scale, int window, const void* gate, int gate_stride, int splits, float* scratch,
+                                       const float* sink, const void* uv, int dv) {
+  TA_REQUIRE(batch >= 0 && ta_latent_maps_take(batch > 0 ? batch : 1, H, 8, rank, dv, splits), "ta_latent_attention_map: %d sequences, %d heads, %d -> %d, %d shares",
+             batch, H, rank, dv, splits);
+  TA_REQUIRE(ta_latent_mfma_rows(rank, dc, 1, H) > 0 && (uintptr_t)uv % 16 == 0 && o != nullptr && scratch != nullptr,
+             "ta_latent_attention_map: rows of %d or the matrices' start", dc);
+  if (batch == 0) return 0;
+  if (int rc = ta_latent_attention(stream, TA_BF16, qa, nullptr, kcache, block_table, max_blocks, cu_q, pos0, batch, 1, H, rank, rot, dc, scale,
+                                   window, gate, gate_stride, splits, scratch, sink))
+    return rc;
+  const int rows = ta_latent_mfma_rows(rank, dc, 1, H), tiles = (H + rows - 1) / rows;
+  const dim3 g((dv + 63) / 64, H, (batch + LA_ROWS_MAP - 1) / LA_ROWS_MAP);
+  latent_merge_map_kernel<<<g, 256, 0, stream>>>(scratch, (const bf16_t*)uv, (bf16_t*)o, cu_q, H, rank, dv, splits, tiles, rows,
+                                                 (const bf16_t*)gate, gate_stride, sink, batch);
+  return ta_check_launch("ta_latent_attention_map");
 }

@@ -1846,7 +1846,7 @@ def latent_key_shares(batch: int, max_qlen: int, heads: int, rank: int, width: i
         return 1
     if max_qlen * heads >= 64 and batch * -(-max_qlen * heads // 64) >= 128:
         return 1        # enough workgroups of four tiles that share their chunks (the kernel for many rows)
-    waves = batch * -(-max_qlen * heads // rows)
+    waves = batch * -(-max_qlen * heads // rows) * int(library().ta_latent_share_waves(c_int(rank), c_int(width)))
     keys = max_kv_len if not window else min(max_kv_len, window + max_qlen)
     chunks = keys // 32 + 2
     return max(1, min(chunks // 2, 2048 // max(waves, 1)))
@@ -1894,6 +1894,70 @@ def latent_attention(qa: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor, 
         c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0), c_int(B), c_int(max_qlen), c_int(H), c_int(rank),
         c_int(rot), c_int(width), c_float(scale), c_int(window or 0), _ptr(gate), c_int(gs), c_int(shares),
         _ptr(scratch), _ptr(sink)))
+    return out
+
+
+def latent_maps_take(rows: int, heads: int, nope: int, rank: int, value_dim: int, shares: int) -> bool:
+    """Whether a bfloat16 step of that many single tokens has its heads' maps done by ``latent_query_map`` and
+    ``latent_attention_map``."""
+    return bool(library().ta_latent_maps_take(c_int(rows), c_int(heads), c_int(nope), c_int(rank), c_int(value_dim), c_int(shares)))
+
+
+def latent_query_map(q: torch.Tensor, heads: int, nope: int, rot: int, rot_dims: int, angles, uk: torch.Tensor,
+                     qa: torch.Tensor, rank: int) -> torch.Tensor:
+    """``latent_query_rot`` and qa[:, h, :rank] = the head's unrotated part @ uk[h], uk [heads, nope, rank], in one kernel:
+    at most 16 bfloat16 rows (``latent_maps_take``)."""
+    _dev(q, "q", torch.bfloat16, contiguous=False); _dev(qa, "qa", torch.bfloat16); _dev(uk, "uk", torch.bfloat16)
+    nt, qs = _rows2d(q, "q")
+    if q.shape[1] < heads * (nope + rot) or qa.dim() != 3 or tuple(qa.shape[:2]) != (nt, heads) or qa.shape[2] < rank + rot \
+            or tuple(uk.shape) != (heads, nope, rank):
+        raise KernelError(f"latent_query_map: q {tuple(q.shape)} uk {tuple(uk.shape)} qa {tuple(qa.shape)}")
+    if rot_dims:
+        _dev(angles, "angles", torch.float32)
+        if tuple(angles.shape) != (nt, rot_dims // 2, 2):
+            raise KernelError(f"latent_query_map: angles are {tuple(angles.shape)}")
+    _check(library().ta_latent_query_map(_stream(), _ptr(q), c_int(qs), c_int(heads), c_int(nope), c_int(rot), c_int(rot_dims),
+                                         _ptr(angles if rot_dims else None), _ptr(uk), _ptr(qa), c_int(rank),
+                                         c_int(qa.shape[2]), c_int(nt)))
+    return qa
+
+
+def latent_attention_map(qa: torch.Tensor, uv: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor, block_table, cu_q, pos0,
+                         rank: int, rot: int, scale: float, window, gate, shares: int, sink) -> torch.Tensor:
+    """``latent_attention`` of a step in which every sequence brings one token, followed by out[t, h] = its row @ uv[h], uv [heads,
+    rank, value width], without storing the rows in between (``latent_maps_take``; the rows are rounded as there)."""
+    _dev(qa, "qa", torch.bfloat16); _dev(out, "out", torch.bfloat16); _dev(kcache, "kcache", torch.bfloat16)
+    _dev(uv, "uv", torch.bfloat16)
+    nt, H = qa.shape[0], qa.shape[1]
+    width = qa.shape[2] if qa.dim() == 3 else -1
+    if qa.dim() != 3 or width < rank + rot or uv.dim() != 3 or tuple(uv.shape[:2]) != (H, rank) or kcache.dim() != 4 \
+            or tuple(out.shape) != (nt, H, uv.shape[2]) or tuple(kcache.shape[1:]) != (1, PAGE, width):
+        raise KernelError(f"latent_attention_map: qa {tuple(qa.shape)} uv {tuple(uv.shape)} out {tuple(out.shape)} "
+                          f"cache {tuple(kcache.shape)}")
+    _dev(block_table, "block_table", torch.int32); _dev(cu_q, "cu_q", torch.int32); _dev(pos0, "pos0", torch.int32)
+    B = pos0.numel()
+    if nt != B or cu_q.numel() != B + 1 or block_table.dim() != 2 or block_table.shape[0] != B:
+        raise KernelError("latent_attention_map: cu_q / pos0 / block_table disagree about the batch size")
+    gs = 0
+    if gate is not None:
+        _dev(gate, "gate", torch.bfloat16, contiguous=False)
+        ng, gs = _rows2d(gate, "gate")
+        if ng != nt or gate.shape[1] < H:
+            raise KernelError(f"latent_attention_map: gate is {tuple(gate.shape)}")
+    if sink is not None:
+        _dev(sink, "sink", torch.float32)
+        if sink.shape != (H,):
+            raise KernelError(f"latent_attention_map: sink is {tuple(sink.shape)}, expected {(H,)}")
+    need = library().ta_latent_mfma_scratch
+    need.restype = c_longlong
+    floats = need(c_int(B), c_int(1), c_int(H), c_int(rank), c_int(width), c_int(shares))
+    if floats <= 0:
+        raise KernelError(f"latent_attention_map: rows of {width} in {shares} shares")
+    scratch = _scratch_floats(qa.device, floats)
+    _check(library().ta_latent_attention_map(
+        _stream(), _ptr(qa), _ptr(out), _ptr(kcache), _ptr(block_table), c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0),
+        c_int(B), c_int(H), c_int(rank), c_int(rot), c_int(width), c_float(scale), c_int(window or 0), _ptr(gate), c_int(gs),
+        c_int(shares), _ptr(scratch), _ptr(sink), _ptr(uv), c_int(uv.shape[2])))
     return out
 
 

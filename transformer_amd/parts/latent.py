@@ -98,6 +98,11 @@ class LatentAttention(Part):
         torch.bmm(a.transpose(0, 1), w, out=out.transpose(0, 1))
         return out
 
+    # a few single tokens of a bfloat16 engine: the heads' maps ride on the rotation and on the merge of the keys' shares
+    def _maps_fit(self, nt: int, shares: int) -> bool:
+        return self.dn > 0 and self._by_library(self.uk_op) and self._by_library(self.uv_op) and self.row % 8 == 0 \
+            and kernels.latent_maps_take(nt, self.H, self.dn, self.spec.kv_rank, self.dv, shares)
+
     # with many rows the output projection can add itself to the residual stream (``into``); in
     # single-token steps the norms around the mixer ride on its products (``PreNormBlock``)
     def can_add(self, nt: int) -> bool:
@@ -129,18 +134,22 @@ class LatentAttention(Part):
         else:
             q = proj[:, :self.kv_off]
         qa = ctx.ws.take("latent.qa", (nt, H, self.row), self.dtype)
+        shares = kernels.latent_key_shares(ctx.batch, ctx.max_qlen, H, r, self.row, ctx.max_kv_len, s.window)
+        gate = proj[:, self.gate_off:] if s.gated else None
+        o = ctx.ws.take("latent.o", (nt, H, self.dv), self.dtype)
+        if ctx.all_single and self._maps_fit(nt, shares):
+            kernels.latent_query_map(q, H, self.dn, dr, s.rot_dims, angles, self.uk_op, qa, r)
+            kernels.latent_attention_map(qa, self.uv_op, o, kc, meta.block_table, ctx.cu_q, ctx.pos0, r, dr, float(s.scale),
+                                         s.window, gate, shares, self.w.get("sink"))
+            return finish(o.view(nt, H * self.dv), self.w["out.weight"], ctx.ws, "latent.delta", fold, into)
         kernels.latent_query_rot(q, H, self.dn, dr, s.rot_dims, angles, qa, r)
         if self.dn:
             self._per_head(q.unflatten(1, (H, self.dn + dr))[:, :, :self.dn], self.uk_op, qa[:, :, :r])
         else:
             qa[:, :, :r].zero_()
         ol = ctx.ws.take("latent.ol", (nt, H, r), self.dtype)
-        shares = kernels.latent_key_shares(ctx.batch, ctx.max_qlen, H, r, self.row, ctx.max_kv_len, s.window)
         kernels.latent_attention(qa, ol, kc, meta.block_table, ctx.cu_q, ctx.pos0, ctx.max_qlen, r, dr,
-                                 float(s.scale), s.window,
-                                 gate=proj[:, self.gate_off:] if s.gated else None, shares=shares,
-                                 sink=self.w.get("sink"))
-        o = ctx.ws.take("latent.o", (nt, H, self.dv), self.dtype)
+                                 float(s.scale), s.window, gate=gate, shares=shares, sink=self.w.get("sink"))
         self._per_head(ol, self.uv_op, o)
         return finish(o.view(nt, H * self.dv), self.w["out.weight"], ctx.ws, "latent.delta", fold, into)
 
