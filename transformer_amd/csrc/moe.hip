@@ -4,7 +4,7 @@
 //                 the `top` largest (lowest index among equals), optionally renormalised
 //   moe_plan    : the (token, choice) pairs ordered by expert: each expert's pairs take a run
 //                 of rows that starts on a multiple of 16, so a tile of 16 rows belongs to one
-//                 expert; the row count is bounded by pairs + 15 * E whatever the routing is,
+//                 expert; the row count is bounded by pairs + 15 * min(pairs, E) whatever the routing is,
 //                 so a step's launches do not depend on the data
 //   moe_gather  : the ordered rows of activations, each times its pair's weight when the weight
 //                 acts on the expert's input
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
 }
 
 extern "C" int ta_moe_max_rows(int pairs, int E) {
-  const long long n = (long long)pairs + (long long)(MOE_TILE - 1) * E;
+  const long long n = (long long)pairs + (long long)(MOE_TILE - 1) * (pairs < E ? pairs : E);
   const long long r = (n + MOE_TILE - 1) / MOE_TILE * MOE_TILE;
   return r > 2147483647ll ? -1 : (int)r;
 }
@@ -509,33 +509,35 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16_t* __rest
 __device__ uint4 moe_zeros;             // where a piece past K is read from (never written: zero)
 
 // Few tiles (a step of few tokens), bound by reading the chosen experts' matrices: a workgroup owns ONE tile of 16
-// rows and 64 rows of the matrix and its four waves divide K; the partial tiles are added in wave order through
+// rows and 16 NT rows of the matrix and its four waves divide K; the partial tiles are added in wave order through
 // LDS. While 128 k are multiplied the next are on their way (16 KB a wave). The matrix comes in whole lines, sixteen lanes a
 // row's 256 bytes, and takes the operands' layout in the wave's own LDS: read in that layout straight from memory, 16 bytes of
 // sixteen rows at a time, it is the lines a CU touches that bind. 2 tokens of six of 64 experts of 1,408 x 4,096 (gate and up,
 // then down) 49.8 -> 35 and 29.9 -> 22.4 us; 4 of four of 32 of 1,024 x 2,048 16.3 -> 14.0 and 16.2 -> 12.2.
 // row_pair (or null: A holds the ordered rows): the tile's rows are read from the tokens' rows h, each times its
 // pair's weight, rounded as moe_gather rounds it: a step of few tokens needs no ordered copy.
-// GLU: the matrix holds gate rows, then up rows; the workgroup takes 32 of each and joins them.
+// GLU: the matrix holds gate rows, then up rows; the workgroup takes 8 NT of each and joins them.
 struct MoeRows {
   const bf16_t* A;
   const int* row_pair;
   const float* weight;
   int top;
 };
-template <typename TC, bool GLU>
+template <typename TC, bool GLU, int NT>
 __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows, const bf16_t* __restrict__ W,
                                                                    const int* __restrict__ tile_expert,
                                                                    TC* __restrict__ C, int N, int K, int act, TaGlu glu) {
-  // a wave's 64 rows x 128 k of the matrix on their way from whole lines to the operands' layout, then its sums
-  __shared__ __attribute__((aligned(16))) uint32_t stage[4][4][1024];
-  typedef float Sums[16][65];
+  static_assert(NT == 1 || NT == 2 || NT == 4, "tiles of 16 rows of the matrix");
+  static_assert(!GLU || NT > 1, "gates and ups");
+  // a wave's 16 NT rows x 128 k of the matrix on their way from whole lines to the operands' layout, then its sums
+  __shared__ __attribute__((aligned(16))) uint32_t stage[4][NT][1024];
+  typedef float Sums[16][16 * NT + 1];
   Sums* red = reinterpret_cast<Sums*>(&stage[0][0][0]);
   const int e = tile_expert[blockIdx.y];
   if (e < 0) return;                                    // the whole workgroup: tiles past the last expert's rows
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int r = lane % 16, kb = lane / 16;
-  constexpr int COLS = GLU ? 32 : 64;                   // of C
+  constexpr int COLS = GLU ? 8 * NT : 16 * NT, HALF = NT / 2;     // of C
   const int n0 = blockIdx.x * COLS;
   const size_t r0 = (size_t)blockIdx.y * MOE_TILE;
   const bf16_t* We = W + (size_t)e * (GLU ? 2 : 1) * N * K;
@@ -547,28 +549,28 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   // row's number so that the operands' reads meet no bank twice
   const int lrow = lane / 16, lpiece = lane % 16;
   const bf16_t* wbase[2] = {We + (size_t)n0 * K, We + (size_t)(GLU ? N + n0 : n0) * K};
-  uint32_t woff[4][4];                                  // rows past N: another row, whose products are not stored
+  uint32_t woff[NT][4];                                  // rows past N: another row, whose products are not stored
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int n = (GLU ? 16 * (t % 2) : 16 * t) + 4 * i + lrow;
+      const int n = (GLU ? 16 * (t % HALF) : 16 * t) + 4 * i + lrow;
       woff[t][i] = (uint32_t)(n0 + n < N ? n : N - 1 - n0) * (uint32_t)K + (uint32_t)((lpiece ^ (4 * i + lrow)) * 8);
     }
-  moe_floatx4 acc[4];
+  moe_floatx4 acc[NT];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) acc[t] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
   constexpr int DEPTH = 4;                              // steps of 32 k asked for together
-  MoeFrag af[2][DEPTH], wf[2][4][4];
+  MoeFrag af[2][DEPTH], wf[2][NT][4];
   auto load_matrix = [&](int set, int k0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int k = k0 + (lpiece ^ (4 * i + lrow)) * 8;
       const bool kok = k < kend && k < K;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < NT; ++t)
         wf[set][t][i].q = __builtin_nontemporal_load(
-            reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(wbase[GLU && t >= 2] + k0 + woff[t][i]) : (const void*)&moe_zeros));
+            reinterpret_cast<const moe_u32x4*>(kok ? (const void*)(wbase[GLU && t >= HALF] + k0 + woff[t][i]) : (const void*)&moe_zeros));
     }
   };
   load_matrix(0, kbeg);
@@ -590,7 +592,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   };
   auto multiply = [&](int set) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         *reinterpret_cast<moe_u32x4*>(&stage[wave][t][(4 * i + lrow) * 64 + lpiece * 4]) = wf[set][t][i].q;
@@ -606,7 +608,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
         }
       }
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < NT; ++t) {
         MoeFrag w;
         w.q = *reinterpret_cast<const moe_u32x4*>(&stage[wave][t][r * 64 + ((4 * u + kb) ^ r) * 4]);
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.v, af[set][u].v, acc[t], 0, 0, 0);
@@ -634,16 +636,17 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
   }
   __syncthreads();                                      // (the waves' sums lie where the others' rows were)
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int j = 0; j < 4; ++j) red[wave][r][16 * t + 4 * kb + j] = acc[t][j];
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < COLS / 16; ++i) {
+  for (int i = 0; i < (COLS + 15) / 16; ++i) {
     const int idx = threadIdx.x + 256 * i, row = idx / COLS, col = idx % COLS;
+    if (idx >= 16 * COLS) break;
     float v = (red[0][row][col] + red[1][row][col]) + (red[2][row][col] + red[3][row][col]);
     if (GLU) {
-      const int up = col + 32;
+      const int up = col + 16 * HALF;
       const float u = (red[0][row][up] + red[1][row][up]) + (red[2][row][up] + red[3][row][up]);
       // the product of its own stores gate and up in the engine's type
       v = ta_glu(glu, to_f32(from_f32<bf16_t>(v)), to_f32(from_f32<bf16_t>(u)));
@@ -652,6 +655,27 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_splitk_kernel(MoeRows rows,
     }
     if (n0 + col < N) C[(r0 + row) * N + n0 + col] = from_f32<TC>(v);
   }
+}
+
+// 16 NT rows of the matrix a workgroup: fewer where the tiles of 64 would leave CUs with one workgroup or none. us with 64 / 32 / 16
+// rows, by tiles times blocks of 64: 4 tokens of four of 32 experts 1,024 x 2,048 (256) 13.8 / 12.6 / 10.5, 2,048 x 1,024 (512) 12.9 / 11.9 /
+// 13.0, one token (64, 128) 12.2 / 8.9 / 6.7 and 8.9 / 7.6 / 7.1, 8 tokens (512, 1,024) 22.4 / 19.1 / 18.4 and 21.9 / 21.6 / 23.5; of six
+// of 64 experts of 1,408 x 4,096, gated, and 4,096 x 1,408 one token (264, 384) 34.8 / 30.1 and 20.0 / 18.2 / 21.7, two (528, 768)
+// 43.8 / 44.8 and 30.5 / 31.8 / 35.8.
+template <typename TC, bool GLU>
+static void moe_splitk(hipStream_t stream, const MoeRows& rows, const void* W, const int* tile_expert, void* C, int tiles, int N, int K,
+                       int act, const TaGlu& glu) {
+  const long long blocks = (long long)tiles * ((N + (GLU ? 31 : 63)) / (GLU ? 32 : 64));
+#define SPLITK(NT)                                                                                                            \
+  moe_gemm_mfma_splitk_kernel<TC, GLU, NT><<<dim3((N + (GLU ? 8 : 16) * NT - 1) / ((GLU ? 8 : 16) * NT), tiles), 256, 0, stream>>>( \
+      rows, (const bf16_t*)W, tile_expert, (TC*)C, N, K, act, glu)
+  if constexpr (!GLU)
+    if (blocks <= 256) {
+      SPLITK(1);
+      return;
+    }
+  if (blocks <= 512) SPLITK(2); else SPLITK(4);
+#undef SPLITK
 }
 
 // Many tiles (a prompt): operands through LDS. An expert's tiles of 16 rows are cut, from its first one on, into
@@ -974,12 +998,8 @@ extern "C" int ta_moe_gemm_tokens(hipStream_t stream, const void* h, int nt, con
   const MoeRows rows = {(const bf16_t*)h, row_pair, weight, top};
   const TaGlu g = {limit, slope, shift};
   const int tiles = max_rows / MOE_TILE;
-  if (glu)
-    moe_gemm_mfma_splitk_kernel<bf16_t, true><<<dim3((N + 31) / 32, tiles), 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert,
-                                                                                            (bf16_t*)C, N, K, 0, g);
-  else
-    moe_gemm_mfma_splitk_kernel<bf16_t, false><<<dim3((N + 63) / 64, tiles), 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert,
-                                                                                             (bf16_t*)C, N, K, act, g);
+  if (glu) moe_splitk<bf16_t, true>(stream, rows, W, tile_expert, C, tiles, N, K, 0, g);
+  else moe_splitk<bf16_t, false>(stream, rows, W, tile_expert, C, tiles, N, K, act, g);
   return ta_check_launch("ta_moe_gemm_tokens");
 }
 
@@ -1000,13 +1020,10 @@ extern "C" int ta_moe_gemm_form(hipStream_t stream, int dtype, int out_dtype, co
     if ((form == 3 || (form == 0 && !few)) && aligned)
       return moe_gemm_lds_launch(stream, out_dtype, A, W, tile_expert, C, tiles, N, K, act);
     if (form == 1 || (form == 0 && few)) {   // too few workgroups to fill the CUs: the waves divide K
-      dim3 gk((N + 63) / 64, tiles);
       const MoeRows rows = {(const bf16_t*)A, nullptr, nullptr, 1};
       const TaGlu none = {0.f, 1.f, 0.f};
-      if (out_dtype == TA_BF16)
-        moe_gemm_mfma_splitk_kernel<bf16_t, false><<<gk, 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert, (bf16_t*)C, N, K, act, none);
-      else
-        moe_gemm_mfma_splitk_kernel<float, false><<<gk, 256, 0, stream>>>(rows, (const bf16_t*)W, tile_expert, (float*)C, N, K, act, none);
+      if (out_dtype == TA_BF16) moe_splitk<bf16_t, false>(stream, rows, W, tile_expert, C, tiles, N, K, act, none);
+      else moe_splitk<float, false>(stream, rows, W, tile_expert, C, tiles, N, K, act, none);
       return ta_check_launch("ta_moe_gemm");
     }
     dim3 g((N + 255) / 256, (tiles + 3) / 4);
