@@ -681,43 +681,48 @@ static void moe_splitk(hipStream_t stream, const MoeRows& rows, const void* W, c
 // Many tiles (a prompt): operands through LDS. An expert's tiles of 16 rows are cut, from its first one on, into
 // blocks of up to 16, so that its matrix is read once for every 256 rows. A workgroup of eight waves owns 256 columns
 // of the blocks that begin at four neighbouring tiles (one block where the experts have four tiles or more), and what is
-// sent for runs on from one block into the next. The operands go from
-// memory to LDS without passing through registers, 32 k at a time, four steps ahead into five buffers (160 KB). A
-// row's four pieces of 16 bytes are permuted by half the row number, so that eight rows' reads meet no bank twice. The
-// waves stand in 2 x 4; each multiplies half of the block's tiles by 64 columns. What bounds it: few rows an expert, the
-// experts' matrices from memory (3.9 TB/s); many, the loads and the reads of LDS around the products (0.67 PFLOP/s).
+// sent for runs on from one block into the next. The operands go from memory to LDS without passing through registers, 64 k of
+// a step at a time and so whole lines of 128 bytes: with 32 k a CU takes in 27 bytes a clock, with 64 36, and alone the loads of
+// 64 experts of 2,816 x 4,096 with 256 rows each take 433 us and 368 (the load of half lines was what bounded this
+// kernel). The columns, from HBM, go two steps ahead into three buffers, the rows, which other workgroups read too, one step
+// into two (160 KB). A row's eight pieces of 16 bytes are permuted by the row number, so that eight rows' reads meet no bank
+// twice. The waves stand in 2 x 4; each multiplies half of the block's tiles by 64 columns, and reads the operands of the
+// next 32 k meanwhile, which also frees a step's buffers before its last products: one barrier every 64 k. What bounds it: few
+// rows an expert, the experts' matrices from memory (4.1 TB/s); many, the loads into LDS (0.78 to 0.98 PFLOP/s).
+// us with steps of 32 k, operands read when they are due / so: 64 experts of 2,816 x 4,096 at 2,943 tokens of six, unevenly routed
+// 622 / 558, evenly 774 / 673, at 1,200 402 / 364; of 4,096 x 1,408 366 / 328 and 237 / 209; 32 experts of 2,048 x 1,408 at 8,000 of
+// four 309 / 272, of 1,024 x 4,096 404 / 345, at 2,000 of 1,024 x 2,048 99 / 91; 8 of 28,672 x 4,096 at 4,096 of two 2,116 / 1,968;
+// 8 of 1,024 x 4,096 174 / 147 and 64 of 384 x 2,048 at 6,000 of six 142 / 134. Loads for the rows of a block only, by the
+// exec mask, cost more than they saved (592 against 558); an XCD's workgroups on neighbouring blocks gained where experts are
+// evenly used (629) and lost where not (571, 2,210).
 // Workgroups are numbered by the blocks there are: with one for every four tiles, most of them empty, the blocks of long
-// runs fell on every fourth workgroup and so on a part of the XCDs and shader engines: 32 experts of 2,048 x 1,408 at
-// 8,000 tokens of four 612 us, 292 now (412 by the kernel before blocks); of 1,024 x 4,096 547 and 415 (488); 64 experts
-// of 2,816 x 4,096 at 2,943 tokens of six, unevenly routed, 726 and 652 (978), evenly 764 and 777 (949). Finding its
-// number costs a workgroup some 2 us. Some shapes stay slower than by that kernel (128 rows by 128 columns through
-// registers), whose smaller pieces suit narrow matrices of long k: 8 experts of 1,024 x 4,096 at 4,096 tokens of two 171
-// against 151, 64 of 384 x 2,048 at 6,000 of six 176 against 149.
+// runs fell on every fourth workgroup and so on a part of the XCDs and shader engines (32 experts of 2,048 x 1,408 at
+// 8,000 tokens of four twice the time). Finding its number costs a workgroup some 2 us.
 #define ML_BM 256
 #define ML_BN 256
-#define ML_BK 32
-#define ML_ST 5
+#define ML_BK 64
 #define ML_TILES (ML_BM / MOE_TILE)
 #define ML_OWN 4
 
 static __device__ const moe_u32x4 ml_zeros = {0, 0, 0, 0};
 
-// 32 k of a block: UU tiles of rows from `rows` on by 64 columns from `cols` on
+// Multiplies 32 k of a block, UU tiles of rows from As on by 64 columns from Ws on, and while it does reads the next 32 k's: the
+// columns' into the other set, a tile's rows into the registers that its last product has just left. `at`: the lane's piece.
 template <int UU>
-static __device__ __forceinline__ void ml_multiply(moe_floatx4 (&acc)[UU][4], const moe_u32x4* As, const moe_u32x4* Ws, int rows, int cols,
-                                                   int r, int kb) {
-  MoeFrag af[UU], wf[4];
+static __device__ __forceinline__ void ml_multiply(moe_floatx4 (&acc)[UU][4], MoeFrag (&af)[UU], const MoeFrag (&wf)[4], MoeFrag (&wn)[4],
+                                                   const moe_u32x4* As, const moe_u32x4* Ws, int at) {
 #pragma unroll
-  for (int v = 0; v < 4; ++v) wf[v].q = Ws[(cols + 16 * v + r) * 4 + (kb ^ ((r >> 1) & 3))];
+  for (int v = 0; v < 4; ++v) wn[v].q = Ws[16 * 8 * v + at];
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int u = 0; u < UU; ++u) af[u].q = As[(rows + 16 * u + r) * 4 + (kb ^ ((r >> 1) & 3))];
-  __builtin_amdgcn_sched_barrier(0);                    // every read goes out before the first product waits for one
-#pragma unroll
-  for (int u = 0; u < UU; ++u)
+  for (int u = 0; u < UU; ++u) {
 #pragma unroll
     for (int v = 0; v < 4; ++v)
       // register j of a lane: column 4 * (lane / 16) + j of the tile, row lane % 16
       acc[u][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[v].v, af[u].v, acc[u][v], 0, 0, 0);
+    af[u].q = As[16 * 8 * u + at];
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // Of the windows of ML_OWN tiles in which a block begins, number `want`: its first tile, or -1 if there are fewer, and in
@@ -792,13 +797,16 @@ static __device__ __forceinline__ int ml_find(const int* __restrict__ tile_exper
   return -1;
 }
 
+// a barrier for LDS alone: what is on its way from memory stays on its way
+static __device__ __forceinline__ void ml_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 template <typename TC, bool ACT>
 __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                            const int* __restrict__ tile_expert, int tiles, int most,
                                                            TC* __restrict__ C, int N, int K, int act) {
   extern __shared__ __attribute__((aligned(16))) unsigned char ml_lds[];
-  moe_u32x4* As = reinterpret_cast<moe_u32x4*>(ml_lds);                 // [ML_ST][ML_BM * 4]
-  moe_u32x4* Ws = As + ML_ST * ML_BM * 4;                               // [ML_ST][ML_BN * 4]
+  moe_u32x4* As = reinterpret_cast<moe_u32x4*>(ml_lds);                 // [2][ML_BM * 8]
+  moe_u32x4* Ws = As + 2 * ML_BM * 8;                                   // [3][ML_BN * 8]
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = threadIdx.x % 64;
   const int r = lane % 16, kb = lane / 16, wr = wave / 4, wc = wave % 4;
   const int ncol = (N + ML_BN - 1) / ML_BN;
@@ -831,56 +839,72 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
   auto run_of = [&](int i) { return (int)(blocks >> (5 * i) & 31u); };
   const int nk = (K + ML_BK - 1) / ML_BK;
 
-  // The sender: block `sent`, step `ks` of it. A wave brings 16 rows at a time: rows 16 (wave + 8 i).
-  const int srow = lane / 4, piece = lane % 4 ^ ((srow >> 1) & 3);
-  const bf16_t *abase, *wbase;                          // of the block, at step ks
-  uint32_t aoff[2], woff[2];                            // bytes from there on
+  // The senders, of rows and of columns: a block and a step of it each. A wave brings 8 rows at a time, 128 bytes of each: rows
+  // 8 (wave + 8 i).
+  const int srow = lane / 8, piece = lane % 8 ^ srow;
+  const bf16_t *abase, *wbase;                          // of the block, at the step
+  uint32_t aoff[4], woff[4];                            // bytes from there on
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = 16 * (wave + 8 * i) + srow;
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * (wave + 8 * i) + srow;
     woff[i] = ((uint32_t)(n0 + row < N ? row : N - 1 - n0) * K + piece * 8) * 2;   // columns past N: read again, never stored
   }
-  int sent = next_block(0), ks = 0;
-  auto aim = [&]() {
-    const int R = run_of(sent) * MOE_TILE;
-    abase = A + (size_t)(t0 + sent) * MOE_TILE * K;
-    wbase = W + ((size_t)__builtin_amdgcn_readfirstlane(tile_expert[t0 + sent]) * N + n0) * K;
+  int asent = next_block(0), wsent = asent, aks = 0, wks = 0;
+  auto aim_rows = [&]() {
+    const int R = run_of(asent) * MOE_TILE;
+    abase = A + (size_t)(t0 + asent) * MOE_TILE * K;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = 16 * (wave + 8 * i) + srow;
+    for (int i = 0; i < 4; ++i) {
+      const int row = 8 * (wave + 8 * i) + srow;
       aoff[i] = ((uint32_t)(row < R ? row : R - 1) * K + piece * 8) * 2;           // rows past the block likewise
     }
   };
-  auto send = [&](int buf) {
+  auto aim_columns = [&]() { wbase = W + ((size_t)__builtin_amdgcn_readfirstlane(tile_expert[t0 + wsent]) * N + n0) * K; };
+  auto bring = [&](const bf16_t* base, const uint32_t (&off)[4], int ks, moe_u32x4* to) {
     if (ks + 1 < nk || K % ML_BK == 0) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ta_load_to_lds16(abase, aoff[i], &As[buf * ML_BM * 4 + 64 * (wave + 8 * i)]);
-        ta_load_to_lds16(wbase, woff[i], &Ws[buf * ML_BN * 4 + 64 * (wave + 8 * i)]);
-      }
+      for (int i = 0; i < 4; ++i) ta_load_to_lds16(base, off[i], &to[64 * (wave + 8 * i)]);
     } else {                                                            // the last, partial step: past K zeros
       const bool in = ks * ML_BK + piece * 8 < K;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ta_load_to_lds16(in ? (const char*)abase + aoff[i] : (const char*)&ml_zeros, &As[buf * ML_BM * 4 + 64 * (wave + 8 * i)]);
-        ta_load_to_lds16(in ? (const char*)wbase + woff[i] : (const char*)&ml_zeros, &Ws[buf * ML_BN * 4 + 64 * (wave + 8 * i)]);
-      }
+      for (int i = 0; i < 4; ++i) ta_load_to_lds16(in ? (const char*)base + off[i] : (const char*)&ml_zeros, &to[64 * (wave + 8 * i)]);
     }
-    if (ks + 1 < nk) {
-      ++ks;
-      abase += ML_BK;
-      wbase += ML_BK;
-    } else if (next_block(sent + 1) < ML_OWN) {                         // on into the next block
-      sent = next_block(sent + 1);
-      ks = 0;
-      aim();
-    }                                                                   // else the last step again, unused
   };
-  aim();
-#pragma unroll
-  for (int s = 0; s < ML_ST - 1; ++s) send(s);
+  // the next step, on into the next block; after the last one the last step again, unused
+  auto send_rows = [&](int buf) {
+    bring(abase, aoff, aks, As + buf * ML_BM * 8);
+    if (aks + 1 < nk) {
+      ++aks;
+      abase += ML_BK;
+    } else if (next_block(asent + 1) < ML_OWN) {
+      asent = next_block(asent + 1);
+      aks = 0;
+      aim_rows();
+    }
+  };
+  auto send_columns = [&](int buf) {
+    bring(wbase, woff, wks, Ws + buf * ML_BN * 8);
+    if (wks + 1 < nk) {
+      ++wks;
+      wbase += ML_BK;
+    } else if (next_block(wsent + 1) < ML_OWN) {
+      wsent = next_block(wsent + 1);
+      wks = 0;
+      aim_columns();
+    }
+  };
+  aim_rows();
+  aim_columns();
+  send_rows(0);
+  send_columns(0);
+  send_columns(1);
+  send_rows(1);
+  send_columns(2);
+  ta_wait_loads<12>();                                  // the first step
+  ml_barrier();
 
-  int buf = 0;
+  const int at = r * 8 + (kb ^ (r & 7));                // a lane's piece of a step's first 32 k; the others': ^ 4
+  int abuf = 0, wbuf = 0;
   for (int i = next_block(0); i < ML_OWN; i = next_block(i + 1)) {
     const int run = run_of(i), half = (run + 1) / 2;
     auto block = [&](auto width) {
@@ -890,9 +914,12 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
         const uint32_t high = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32)), low = __builtin_amdgcn_readfirstlane((uint32_t)x);
         return (uint64_t)high << 32 | low;
       };
-      sent = __builtin_amdgcn_readfirstlane(sent);
-      ks = __builtin_amdgcn_readfirstlane(ks);
-      buf = __builtin_amdgcn_readfirstlane(buf);
+      asent = __builtin_amdgcn_readfirstlane(asent);
+      wsent = __builtin_amdgcn_readfirstlane(wsent);
+      aks = __builtin_amdgcn_readfirstlane(aks);
+      wks = __builtin_amdgcn_readfirstlane(wks);
+      abuf = __builtin_amdgcn_readfirstlane(abuf);
+      wbuf = __builtin_amdgcn_readfirstlane(wbuf);
       abase = reinterpret_cast<const bf16_t*>(same((uint64_t)abase));
       wbase = reinterpret_cast<const bf16_t*>(same((uint64_t)wbase));
       moe_floatx4 acc[U][4];
@@ -900,12 +927,22 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int v = 0; v < 4; ++v) acc[u][v] = moe_floatx4{0.f, 0.f, 0.f, 0.f};
+      // 32 k's operands are read while the 32 before are multiplied, so that a step's buffers are free when its second half is.
+      const moe_u32x4 *ar = As + 16 * U * wr * 8, *wr_ = Ws + 64 * wc * 8;
+      MoeFrag af[U], wf[2][4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) wf[0][v].q = wr_[wbuf * ML_BN * 8 + 16 * 8 * v + at];
+#pragma unroll
+      for (int u = 0; u < U; ++u) af[u].q = ar[abuf * ML_BM * 8 + 16 * 8 * u + at];
       for (int step = 0; step < nk; ++step) {
-        ta_wait_loads<4 * (ML_ST - 2)>();                 // this step's pieces; C's stores, if any, only make it wait longer
-        __syncthreads();                                  // everyone's; and all have read the buffer that is sent for now
-        send(buf == 0 ? ML_ST - 1 : buf - 1);
-        if (n0 + 64 * wc < N) ml_multiply<U>(acc, As + buf * ML_BM * 4, Ws + buf * ML_BN * 4, 16 * U * wr, 64 * wc, r, kb);
-        buf = buf + 1 == ML_ST ? 0 : buf + 1;
+        ml_multiply<U>(acc, af, wf[0], wf[1], ar + abuf * ML_BM * 8, wr_ + wbuf * ML_BN * 8, at ^ 4);
+        ta_wait_loads<4>();                             // the next step's rows and columns; C's stores, if any, only make it wait longer
+        ml_barrier();                                   // everyone's; and everyone has this step's operands in registers
+        send_rows(abuf);
+        send_columns(wbuf);
+        abuf ^= 1;
+        wbuf = wbuf == 2 ? 0 : wbuf + 1;
+        ml_multiply<U>(acc, af, wf[1], wf[0], ar + abuf * ML_BM * 8, wr_ + wbuf * ML_BN * 8, at);   // a last step's: the next block's, read again
       }
       TC* out = C + ((size_t)(t0 + i) * MOE_TILE + r) * N;
       const bool whole = N % 4 == 0 && (uintptr_t)C % (4 * sizeof(TC)) == 0;   // a lane's four columns are stored at once
@@ -949,7 +986,7 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_lds_kernel(const bf16_t* __re
 // rows are skipped and their rows of C keep what they held.
 static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A, const void* W, const int* tile_expert,
                                void* C, int tiles, int N, int K, int act) {
-  const size_t lds = (size_t)ML_ST * (ML_BM + ML_BN) * ML_BK * sizeof(bf16_t);
+  const size_t lds = (size_t)(2 * ML_BM + 3 * ML_BN) * ML_BK * sizeof(bf16_t);
   const int ncol = (N + ML_BN - 1) / ML_BN;
   const unsigned g = (unsigned)ncol * (unsigned)((tiles + ML_OWN - 1) / ML_OWN);
   // Blocks of 8 where they give every CU one at most (8 experts, tiles x columns x k: 133 x 2,048 x 1,408 71 us by 16 and
