@@ -1112,11 +1112,14 @@ static int moe_gemm_lds_launch(hipStream_t stream, int out_dtype, const void* A,
 }
 
 // Whether the experts' product of this many ordered rows takes the form for few tiles (bfloat16). Below the line the
-// blocks of the other form leave CUs idle, above it this one reads an expert's matrix once for every tile. Few against
-// LDS, us (tiles, in brackets those with rows): 66 (51) of 4,096 x 1,408 139 and 139, 83 (72) 200 and 246; 81 (64) of 2,816
-// x 4,096 308 and 310, 105 (72) 368 and 333; 80 (66) of 2,048 x 1,024 52 and 40, 255 (239) 151 and 59.
+// blocks of the other form leave CUs idle, above it this one reads an expert's matrix once for every tile; the larger the matrices,
+// the longer the other's few workgroups walk. Tiles by blocks of 256 columns, us few / LDS: 4,096 x 2,048 1,120 126 / 128,
+// 1,280 143 / 157, 1,600 178 / 152; 4,096 x 1,408 1,328 150 / 175, 1,760 188 / 180; 2,816 x 4,096 1,210 330 / 416, 1,430 379 / 407, 1,650
+// 423 / 353; 28,672 x 4,096 1,344 384 / 444; smaller ones 4,096 x 1,024 960 55 / 67, 1,120 61 / 50; 2,048 x 2,048 560 60 / 65, 800 77 / 68;
+// 2,048 x 1,024 480 31 / 51, 800 43 / 38 (and a first product through LDS wants its rows ordered, some 5 us).
 extern "C" int ta_moe_few_rows(int max_rows, int N, int K) {
-  return K % 8 == 0 && (long long)(max_rows / MOE_TILE) * ((N + 255) / 256) < 1024;
+  const long long size = (long long)N * K, line = size < 5 << 20 ? 1024 : 1400;
+  return K % 8 == 0 && (long long)(max_rows / MOE_TILE) * ((N + 255) / 256) < line;
 }
 
 // The first product of the experts of a step of few tokens, from the tokens' rows h [nt, K]: C [max_rows, N] in
