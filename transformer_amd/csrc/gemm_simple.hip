@@ -15,7 +15,7 @@
 // Four kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk: the same for
 // wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns.
 // gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS; gemm_groups: 64, 96 or 128 x 64, two groups
-// of waves that take the segments in turn.
+// of waves that take the segments in turn. Up to 8 rows of a long enough matrix are gemm_stream.hip's, with the same bits.
 #include "common.h"
 #include "gemm_stream.h"
 
