@@ -163,7 +163,9 @@ class PreNormBlock(Part):
             with span(ctx, "ffn"):
                 self.ffn.run(h, ctx, fold=handover, **kw2)
             return handover.scale()
-        if self._offers(self.ffn, "can_add", nt):
+        # Where rows of the model's own may join the stream before anything reads it (no ``after``), float32 leaves the
+        # add to the norm behind them: how many rows a step has would otherwise decide which of the two comes first
+        if (after is not None or self.dtype != torch.float32) and self._offers(self.ffn, "can_add", nt):
             kw2["into"] = x
         with span(ctx, "ffn"):
             return self.ffn.run(h, ctx, **kw2)
