@@ -94,3 +94,48 @@ def test_what_the_maps_refuse():
     assert not kernels.latent_maps_take(4, 2, 257, 64, 16, 4) and not kernels.latent_maps_take(4, 2, 16, 60, 16, 4)
     with pytest.raises(kernels.KernelError):
         kernels.latent_query_map(s["q"], 2, 16, 16, 16, s["ang"], s["uk"], qa, 64)
+
+
+@pytest.mark.parametrize("H,rank,rot,window", [(40, 256, 64, None), (5, 512, 64, 70), (3, 264, 120, None), (2, 130, 60, 1), (63, 200, 0, 600)])
+def test_one_share_of_wide_rows_against_64_bits(H, rank, rot, window):
+    """Four waves a tile without a merge: the gate and the sink in their own epilogue."""
+    lens = [0, 100, 1500, 63, 31, 32]
+    s = _step(lens, H, rank, rot, 8, 8, H)
+    qa = torch.zeros(len(lens), H, s["W"], device="cuda", dtype=BF)
+    qa[..., :rank + rot] = torch.randn(len(lens), H, rank + rot, generator=torch.Generator(device="cuda").manual_seed(H), device="cuda").to(BF)
+    for gate, sink in ((False, False), (True, True)):
+        ol = torch.empty(len(lens), H, rank, device="cuda", dtype=BF)
+        kernels.latent_attention(qa, ol, s["kc"], s["table"], s["cu"], s["pos"], 1, rank, rot, 0.05, window,
+                                 gate=s["gate"] if gate else None, shares=1, sink=s["sink"] if sink else None)
+        rows = _rows(s, qa, lens, rank, rot, window, gate, sink, 0.05)
+        assert bool(((ol.double() - rows).abs() <= 2.0 ** -8 * rows.abs() + 2e-5).all())
+
+
+@pytest.mark.parametrize("B,H", [(257, 16), (129, 32), (86, 40)])
+def test_one_more_sequence_does_not_leave_the_keys_to_one_wave(B, H):
+    """Where the rule goes from two shares to one, one takes about as long as two: a wave that walks a tile's keys by itself
+    took five times as long."""
+    rank, rot, n = 256, 64, 900
+    g = torch.Generator(device="cuda").manual_seed(B)
+    W, pages = rank + rot, n // 64 + 1
+    table = torch.arange(B * pages, dtype=torch.int32, device="cuda").view(B, pages)
+    kc = torch.randn(B * pages, 1, 64, W, generator=g, device="cuda", dtype=BF)
+    qa = torch.randn(B, H, W, generator=g, device="cuda", dtype=BF)
+    out = torch.empty(B, H, rank, device="cuda", dtype=BF)
+    cu, pos = torch.arange(B + 1, dtype=torch.int32, device="cuda"), torch.full((B,), n, dtype=torch.int32, device="cuda")
+    assert kernels.latent_key_shares(B, 1, H, rank, W, n + 1, None) == 1 and kernels.latent_key_shares(B - 1, 1, H, rank, W, n + 1, None) == 2
+
+    def us(shares):
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                kernels.latent_attention(qa, out, kc, table, cu, pos, 1, rank, rot, 0.05, None, shares=shares)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    us(2)
+    assert us(1) < 2 * us(2)

@@ -309,15 +309,16 @@ static int latent_attention_run(hipStream_t stream, dim3 g, size_t lds, const vo
 }
 
 // ------------------------------------------------------------------ the same on the matrix cores (bfloat16)
-// Steps of few rows: a wave owns RT tiles of 16 rows and a share of their keys; a workgroup is four
-// such waves that share nothing (no barrier between them). Keys come in chunks of 32 aligned to absolute
-// positions: the wave copies a chunk's rows into its own piece of LDS, forms S^T = K Q^T on
+// Steps of few rows: a wave owns RT tiles of 16 rows and a share of their keys, and a workgroup is four
+// such waves that share nothing (no barrier between them); of wide rows the four take one tile and share its
+// chunks (TEAM below). Keys come in chunks of 32 aligned to absolute positions: the rows of a chunk are copied
+// into LDS, the wave forms S^T = K Q^T on
 // v_mfma_f32_16x16x32_bf16 (a lane then holds 4 keys x 2 tiles of ONE row: the softmax stays in
 // the lane but for two shuffles), and O^T += C^T P^T with the latent's coordinates gathered
 // from the same LDS rows. Scores, maxima, sums and weights are float32; a weight enters the
 // second product as THREE bfloat16 pieces (p = p0 + p1 + p2 exactly: 3 x 8 bits of mantissa), so
 // the product sees all of its 24 bits and only the cached rows are bfloat16.
-// With `splits` > 1 a tile's chunks are dealt to that many waves, which leave (sums, maximum,
+// With `splits` > 1 a tile's chunks are dealt to that many waves (TEAM: workgroups), which leave (sums, maximum,
 // sum of weights) in `partial` for `latent_merge_kernel`: steps of single tokens have few rows
 // and long key ranges.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 la_bf16x8;
@@ -433,12 +434,14 @@ __device__ __forceinline__ void la_chunk(const bf16_t* __restrict__ Ks, int RS, 
     }
   }
 
-// TEAM: the four waves of a workgroup take ONE tile and share its chunks, which all threads bring into one of two
-// buffers behind a barrier a chunk; each forms the tile's scores and sums a quarter of the coordinates. A step of single
-// tokens has one tile a sequence where 16 heads share a row, and by a wave for itself the other three of its workgroup are gone: attention
-// and merge, 16 heads, rank 256, 900 keys, 1 / 4 / 64 sequences 26.2 / 26.9 / 103 us that way, 16.7 / 17.3 / 48 by four (30 with
-// the fewer shares that four waves want); 128 heads, rank 512, 4 x 2,000 keys 199 and 62.
-template <int KS, int CT, int RT, bool TEAM = false>
+// Narrow rows: a wave a tile. TEAM (the others): the four waves of a workgroup take ONE tile and share its chunks, which all threads
+// bring into one of two buffers behind a barrier a chunk; each forms the tile's scores and sums a quarter of the coordinates. A step of
+// single tokens has one tile a sequence where 16 heads share a row, and by a wave for itself the other three of its workgroup are gone:
+// attention and merge, 16 heads, rank 256, 900 keys, 1 / 4 / 64 sequences 26.2 / 26.9 / 103 us that way, 16.7 / 17.3 / 48 by four (30
+// with the fewer shares that four waves want); 128 heads, rank 512, 4 x 2,000 keys 199 and 62. With one share too: 257 / 512 / 1,000
+// sequences of 900 keys 554 / 577 / 1,145 us by a wave each (357 / 616 / 1,180 in seven, four, two shares), 88 / 94 / 186 by four;
+// 300 of 2,000, rank 512, 1,519 and 510; 300 of 60 43 and 13.
+template <int KS, int CT, int RT>
 __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qa, bf16_t* __restrict__ out, const bf16_t* __restrict__ kcache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ cu_q,
@@ -446,6 +449,7 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
     const bf16_t* __restrict__ gate, int gate_stride, int splits, int tiles_max, float* __restrict__ partial,
     const float* __restrict__ sink) {
   extern __shared__ __attribute__((aligned(16))) unsigned char la_lds[];
+  constexpr bool TEAM = KS > 6;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int c = lane % 16, g = lane / 16;
   const int RS = dc + 8;                                  // elements between rows of the LDS copy
@@ -453,12 +457,8 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   const int b = blockIdx.y, split = blockIdx.z;
   const int q0 = cu_q[b], qlen = cu_q[b + 1] - q0;
   const int nrows = qlen * H;
-  // HALVES: rows too wide for one wave's registers (128 accumulators and 72 query registers): two
-  // waves take the same tile, form the same scores, and each sums one half of the coordinates.
-  constexpr bool HALVES = KS > 10 && !TEAM;
   static_assert(!TEAM || (RT == 1 && CT % 16 == 0), "a quarter of the coordinates is whole blocks of 64");
-  const int wid = blockIdx.x * 4 + wave;
-  const int tile = TEAM ? blockIdx.x : HALVES ? wid / 2 : wid, half = TEAM ? wave : HALVES ? wid % 2 : 0;
+  const int tile = TEAM ? blockIdx.x : blockIdx.x * 4 + wave, quarter = TEAM ? wave : 0;
   const int row0 = tile * 16 * RT;
   if (row0 >= nrows) return;                              // a wave (TEAM: a workgroup) leaves: nothing below waits for others
   const int p0 = pos0[b];
@@ -489,8 +489,8 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   const int c0 = tile_start / 32, c1 = (tile_end + 31) / 32;
   const int n = c1 - c0;
   const int ca = c0 + (int)((long long)n * split / splits), cb = c0 + (int)((long long)n * (split + 1) / splits);
-  constexpr int CTP = TEAM ? CT / 4 : HALVES ? CT / 2 : CT;     // coordinate tiles this wave sums
-  const int qb0 = half * (CTP / 4);                       // its first block of 64 coordinates
+  constexpr int CTP = TEAM ? CT / 4 : CT;                 // coordinate tiles this wave sums
+  const int qb0 = quarter * (CTP / 4);                    // its first block of 64 coordinates
   la_floatx4 O[RT][CTP];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
@@ -501,74 +501,43 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
   for (int rt = 0; rt < RT; ++rt) { m[rt] = -INFINITY; l[rt] = 0.f; }
   const int* table = block_table + (size_t)b * max_blocks;
   const int pieces = dc / 8;                              // 16-byte pieces of a row
-  // A chunk is 32 * pieces pieces, NL = 2 KS of them a lane at most. With PRE they are asked for
-  // one chunk ahead and wait in registers while the chunk before is multiplied.
+  // A chunk is 32 * pieces pieces, NL of them a lane at most, which are asked for one chunk ahead and wait in registers while the
+  // chunk before is multiplied.
   constexpr int NL = TEAM ? (KS + 1) / 2 : 2 * KS;
   constexpr int BRING = TEAM ? 256 : 64;                  // lanes that bring a chunk
   const int bring = TEAM ? (int)threadIdx.x : lane;
-  constexpr bool PRE = KS <= 10 || TEAM;
-  uint4 pre[PRE ? NL : 1];
-  auto fetch = [&](int ch, uint4* buf, auto I0, auto I1) {
-    constexpr int i0 = decltype(I0)::value, i1 = decltype(I1)::value;
+  uint4 pre[NL];
+  auto fetch = [&](int ch) {
     const int key0 = ch * 32;
     const size_t page = (size_t)table[key0 / TA_PAGE];
     const bf16_t* src = kcache + (page * TA_PAGE + key0 % TA_PAGE) * (size_t)dc;
 #pragma unroll
-    for (int i = i0; i < i1; ++i) {
+    for (int i = 0; i < NL; ++i) {
       const int idx = bring + BRING * i;
       const int k = idx / pieces, pc = idx - k * pieces;
       const bool live = idx < 32 * pieces && key0 + k < tile_end;       // keys not written yet read as zero
       const uint4 v = *reinterpret_cast<const uint4*>(live ? src + (size_t)k * dc + pc * 8 : kcache);
-      buf[i - i0] = live ? v : uint4{0, 0, 0, 0};
+      pre[i] = live ? v : uint4{0, 0, 0, 0};
     }
   };
-  auto stash = [&](const uint4* buf, auto I0, auto I1) {
-    constexpr int i0 = decltype(I0)::value, i1 = decltype(I1)::value;
+  auto stash = [&]() {
 #pragma unroll
-    for (int i = i0; i < i1; ++i) {
+    for (int i = 0; i < NL; ++i) {
       const int idx = bring + BRING * i;
       const int k = idx / pieces, pc = idx - k * pieces;
-      if (idx < 32 * pieces) *reinterpret_cast<uint4*>(Ks + k * RS + pc * 8) = buf[i - i0];
+      if (idx < 32 * pieces) *reinterpret_cast<uint4*>(Ks + k * RS + pc * 8) = pre[i];
     }
   };
-  using la_i0 = std::integral_constant<int, 0>;
-  using la_nl = std::integral_constant<int, NL>;
-  constexpr int NB = 12;                                  // pieces a lane brings in together without PRE
-  if (PRE && ca < cb) fetch(ca, pre, la_i0{}, la_nl{});
+  if (ca < cb) fetch(ca);
   for (int ch = ca; ch < cb; ++ch) {
-    const int key0 = ch * 32;
-    if (TEAM) {
-      // who comes to this buffer again has passed the other one's barrier, behind which all have read this one
-      Ks = reinterpret_cast<bf16_t*>(la_lds) + (size_t)((ch - ca) & 1) * 32 * RS;
-      stash(pre, la_i0{}, la_nl{});
-      if (ch + 1 < cb) fetch(ch + 1, pre, la_i0{}, la_nl{});
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      la_chunk<KS, CTP, RT>(Ks, RS, dc, rank, key0, c, g, qf, ok, my_start, my_end, scale_log2, m, l, O, qb0);
-      continue;
-    }
-    __builtin_amdgcn_wave_barrier();                      // the chunk before has been read
-    if (PRE) {
-      stash(pre, la_i0{}, la_nl{});
-      if (ch + 1 < cb) fetch(ch + 1, pre, la_i0{}, la_nl{});
-    } else {
-      uint4 buf[NB];
-      using b0 = std::integral_constant<int, 0>;
-      using b1 = std::integral_constant<int, (NB < NL ? NB : NL)>;
-      using b2 = std::integral_constant<int, (2 * NB < NL ? 2 * NB : NL)>;
-      using b3 = std::integral_constant<int, (3 * NB < NL ? 3 * NB : NL)>;
-      static_assert(3 * NB >= NL, "three batches cover a chunk");
-      fetch(ch, buf, b0{}, b1{});
-      stash(buf, b0{}, b1{});
-      __builtin_amdgcn_sched_barrier(0);
-      fetch(ch, buf, b1{}, b2{});
-      stash(buf, b1{}, b2{});
-      __builtin_amdgcn_sched_barrier(0);
-      fetch(ch, buf, b2{}, b3{});
-      stash(buf, b2{}, b3{});
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    __builtin_amdgcn_wave_barrier();
-    la_chunk<KS, CTP, RT>(Ks, RS, dc, rank, key0, c, g, qf, ok, my_start, my_end, scale_log2, m, l, O, qb0);
+    // TEAM: who comes to this buffer again has passed the other one's barrier, behind which all have read this one
+    if (TEAM) Ks = reinterpret_cast<bf16_t*>(la_lds) + (size_t)((ch - ca) & 1) * 32 * RS;
+    else __builtin_amdgcn_wave_barrier();                 // the chunk before has been read
+    stash();
+    if (ch + 1 < cb) fetch(ch + 1);
+    if (TEAM) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else __builtin_amdgcn_wave_barrier();
+    la_chunk<KS, CTP, RT>(Ks, RS, dc, rank, ch * 32, c, g, qf, ok, my_start, my_end, scale_log2, m, l, O, qb0);
   }
   // ---- results: register j of O[4 qi + q] is coordinate 64 (qb0 + qi) + 16 g + 4 j + q of the lane's row c
 #pragma unroll
@@ -584,7 +553,7 @@ __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_at
           const int coord = 64 * (qb0 + ct / 4) + 16 * g + 4 * j + (ct % 4);
           if (coord < rank) dst[coord] = O[rt][ct][j];
         }
-      if (g == 0 && half == 0) { dst[rank] = m[rt]; dst[rank + 1] = l[rt]; }
+      if (g == 0 && quarter == 0) { dst[rank] = m[rt]; dst[rank + 1] = l[rt]; }
       continue;
     }
     float f = la_inverse(l[rt], m[rt], sink, row % H);
@@ -801,12 +770,12 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* __restri
   }
 }
 
-template <int KS, int CT, int RT, bool TEAM = false>
+template <int KS, int CT, int RT>
 static int latent_mfma_run(hipStream_t stream, dim3 g, size_t lds, const void* qa, void* out, const void* kcache,
                            const int* block_table, int max_blocks, const int* cu_q, const int* pos0, int H,
                            int rank, int dc, float scale_log2, int window, const void* gate, int gate_stride,
                            int splits, int tiles_max, float* partial, const float* sink) {
-  auto kern = latent_attention_mfma_kernel<KS, CT, RT, TEAM>;
+  auto kern = latent_attention_mfma_kernel<KS, CT, RT>;
   static size_t allowed = 64 * 1024;                    // per instantiation: asked for once, not at every launch
   if (lds > allowed) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -1044,8 +1013,8 @@ extern "C" long long ta_latent_mfma_scratch(int batch, int max_qlen, int H, int 
 // layer, [pages][1][TA_PAGE][dc]. gate (or null): pre-activation of a sigmoid gate per
 // (token, head), element h of a row of gate_stride elements. sink (or null): [H] float32, a row's
 // denominator also holds exp(sink[head]). window <= 0: all earlier keys.
-// bfloat16 with rows of whole 16-byte pieces runs on the matrix cores; `splits` > 1 deals a
-// row's keys to that many waves (scratch: ta_latent_mfma_scratch floats). float32, and rows
+// bfloat16 with rows of whole 16-byte pieces runs on the matrix cores; `splits` > 1 cuts a
+// row's keys into that many shares (scratch: ta_latent_mfma_scratch floats). float32, and rows
 // that are no multiple of 8 wide, run on the vector ALU (splits is ignored).
 extern "C" int ta_latent_attention(hipStream_t stream, int dtype, const void* qa, void* out, const void* kcache,
                                    const int* block_table, int max_blocks, const int* cu_q, const int* pos0,
@@ -1079,16 +1048,14 @@ extern "C" int ta_latent_attention(hipStream_t stream, int dtype, const void* qa
     }
     const long long tiles = ((long long)max_qlen * H + rows - 1) / rows;
     TA_REQUIRE(tiles <= 2147483647ll, "ta_latent_attention: too many rows");
-    const bool narrow = dc <= 192 && rank <= 128, team = splits > 1 && ta_latent_share_waves(rank, dc) == 4;
-    const bool halves = !(dc <= 320 && rank <= 256);      // two waves a tile: see the kernel
-    dim3 g((unsigned)(team ? tiles : ((halves ? 2 : 1) * tiles + 3) / 4), batch, splits);
+    const bool team = ta_latent_share_waves(rank, dc) == 4;
+    dim3 g((unsigned)(team ? tiles : (tiles + 3) / 4), batch, splits);
     const size_t lds = (size_t)(team ? 2 : 4) * 32 * (dc + 8) * sizeof(bf16_t);
     const float sl2 = scale * 1.4426950408889634f;
     int rc;
-#define LA_MFMA(KS, CT, RT, ...) latent_mfma_run<KS, CT, RT, ##__VA_ARGS__>(stream, g, lds, qa, out, kcache, block_table, max_blocks, cu_q, pos0, H, rank, dc, sl2, window, gate, gate_stride, splits, (int)tiles, scratch, sink)
-    if (narrow) rc = rows == 32 ? LA_MFMA(6, 8, 2) : LA_MFMA(6, 8, 1);
-    else if (!halves) rc = team ? LA_MFMA(10, 16, 1, true) : LA_MFMA(10, 16, 1);
-    else rc = team ? LA_MFMA(18, 32, 1, true) : LA_MFMA(18, 32, 1);
+#define LA_MFMA(KS, CT, RT) latent_mfma_run<KS, CT, RT>(stream, g, lds, qa, out, kcache, block_table, max_blocks, cu_q, pos0, H, rank, dc, sl2, window, gate, gate_stride, splits, (int)tiles, scratch, sink)
+    if (!team) rc = rows == 32 ? LA_MFMA(6, 8, 2) : LA_MFMA(6, 8, 1);
+    else rc = dc <= 320 && rank <= 256 ? LA_MFMA(10, 16, 1) : LA_MFMA(18, 32, 1);
 #undef LA_MFMA
     if (rc) return rc;
     if (splits > 1 && out != nullptr) {

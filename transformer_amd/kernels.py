@@ -1837,10 +1837,12 @@ def latent_row_width(rank: int, rot: int, dtype: torch.dtype) -> int:
 
 def latent_key_shares(batch: int, max_qlen: int, heads: int, rank: int, width: int, max_kv_len: int,
                       window: Optional[int]) -> int:
-    """Waves that share a row's keys in ``latent_attention`` on the matrix cores: one when the
-    step's rows alone give the CUs enough work (then the kernel whose workgroups share their
-    chunks runs), else enough to reach about two waves per SIMD while a share keeps at least
-    two chunks of 32 keys. A function of the step's shape only."""
+    """Shares of a row's keys in ``latent_attention`` on the matrix cores: one when the step's rows
+    alone give the CUs enough work (where they are many, the kernel whose workgroups share their
+    chunks runs then), else enough to reach about two waves per SIMD while a share keeps at least
+    two chunks of 32 keys. A share of wide rows is four waves' work, so from 257 tiles of 16 rows
+    on it is one (16 heads, 900 keys, one / two / three shares: 256 sequences 81 / 68 / 81 us, 257
+    88 / 101 / 85, 512 94 / 125 / 136). A function of the step's shape only."""
     rows = int(library().ta_latent_mfma_rows(c_int(rank), c_int(width), c_int(max_qlen), c_int(heads)))
     if rows == 0:
         return 1
@@ -1859,7 +1861,7 @@ def latent_attention(qa: torch.Tensor, out: torch.Tensor, kcache: torch.Tensor, 
     [pages, 1, PAGE, width] (width >= rank + rot, the rest zero); out [nt, H, rank] = weighted
     sums of the rows' first ``rank`` coordinates, times sigmoid(gate[t, h]) (gate [nt, >= H],
     contiguous rows). sink (float32 [H]): a row's denominator also holds exp(sink[h]). bfloat16 rows of whole 16-byte pieces run on the matrix cores, where
-    ``shares`` waves divide a row's keys (``latent_key_shares``); all else on the vector ALU."""
+    a row's keys are cut into ``shares`` (``latent_key_shares``); all else on the vector ALU."""
     _dev(qa, "qa"); _dev(out, "out", qa.dtype); _dev(kcache, "kcache", qa.dtype)
     nt, H = qa.shape[0], qa.shape[1]
     width = qa.shape[2] if qa.dim() == 3 else -1
