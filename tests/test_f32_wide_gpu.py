@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import plain_linonex
+import plain_llama
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,29 @@ def test_loops_with_wide_feed_forwards(tmp_path, stop):
     want = _logits(engine, tokens, [1] * 12)
     for beside in (3, 7, 8, 11):
         assert np.array_equal(_logits(engine, tokens, [1] * 12, beside), want), beside
+
+
+# hidden sizes whose products go over the norm by four waves' rows and by eight
+def _llama(hidden, layers=2):
+    return {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "num_hidden_layers": layers, "hidden_size": hidden,
+            "num_attention_heads": 12, "num_key_value_heads": 2, "head_dim": 128, "intermediate_size": 1600, "vocab_size": 300,
+            "rope_theta": 5e5, "rms_norm_eps": 1e-5, "tie_word_embeddings": False, "max_position_embeddings": 256}
+
+
+def test_norm_weights_that_start_off_16_bytes(tmp_path):
+    """A product does not go over such a norm; the norm's own kernel takes it, in steps of any size."""
+    import torch
+    engine = _engine(plain_llama, _llama(1536), 3, tmp_path)
+    tokens = _tokens(300, 12)
+    want = _logits(engine, tokens, [12])
+    tensors = dict(engine.tensors)
+    for n, t in tensors.items():
+        if "norm" in n:
+            tensors[n] = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].copy_(t)
+            assert tensors[n].data_ptr() % 16 == 4
+    engine.bind(tensors)
+    got = _logits(engine, tokens, [12])
+    # the same formulas with the squares of a row added in another order
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+    for cuts, beside in (([1] * 12, 0), ([8, 4], 0), ([9, 1, 1, 1], 7)):
+        assert np.array_equal(_logits(engine, tokens, cuts, beside), got), cuts

@@ -650,6 +650,11 @@ class RowNorm:
     def __init__(self, x: torch.Tensor, weight: torch.Tensor, eps: float):
         self.x, self.weight, self.eps = x, weight, float(eps)
 
+    @property
+    def on_pieces(self) -> bool:
+        """Whether both start on the 16 bytes that the product reads at once (``add_rmsnorm`` takes them anywhere)."""
+        return self.x.data_ptr() % 16 == 0 and self.weight.data_ptr() % 16 == 0
+
 
 def _f32_rows_fit(w: torch.Tensor) -> bool:
     return w.dtype == torch.float32 and w.dim() == 2 and w.stride(1) == 1 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0

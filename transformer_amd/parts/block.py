@@ -66,7 +66,8 @@ class PreNormBlock(Part):
         """The norm for a float32 part whose first product goes over it itself; None where its own kernel runs."""
         if self.dtype == torch.float32 and isinstance(pending, tuple) and pending[0] is None and pending[1] is None \
                 and hasattr(norm, "gain") and self._offers(part, "takes_normed", x.shape[0]):
-            return kernels.RowNorm(x, norm.gain(), norm.eps)
+            rows = kernels.RowNorm(x, norm.gain(), norm.eps)
+            return rows if rows.on_pieces else None
         return None
 
     def entry_fold(self, x, ctx):
