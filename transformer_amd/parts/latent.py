@@ -85,7 +85,9 @@ class LatentAttention(Part):
 
         uk = tensors["uk.weight"].view(self.H, self.dn, s.kv_rank) if self.dn else None     # [K, N] of Uk^T
         uv = tensors["uv.weight"].view(self.H, self.dv, s.kv_rank)                          # [N, K]
-        self.uk_op = None if uk is None else uk if self._by_library(uk) else packed(uk.transpose(1, 2))
+        # (where the tensor given does not hold them in whole pieces of 16 bytes, which the kernels that apply them read, a copy)
+        whole = uk is not None and uk.is_contiguous() and uk.data_ptr() % 16 == 0
+        self.uk_op = None if uk is None else (uk if whole else packed(uk)) if self._by_library(uk) else packed(uk.transpose(1, 2))
         self.uv_op = packed(uv.transpose(1, 2)) if self._by_library(uv) else uv
 
     def _by_library(self, w) -> bool:
