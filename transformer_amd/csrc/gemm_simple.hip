@@ -622,11 +622,6 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
     return;
   }
   if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
-    if (batch == 1 && ta_gemm_stream_pays(M, N, K, 0)) {
-      ta_gemm_stream(stream, A, lda, W, ldw, bias, C, ldc, M, N, K, 0, 0, nullptr, 0.f);
-      return;
-    }
-  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
     if (batch == 1 && walk_pays(M, N, K)) {
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
@@ -668,6 +663,8 @@ extern "C" int ta_gemm_simple_batched(hipStream_t stream, int in_dtype, int w_dt
     return (uintptr_t)p % (dtype == TA_F32 ? 16 : 8) == 0 && ld % 4 == 0 && stride % 4 == 0;
   };
   const bool vec = K % 4 == 0 && aligned(A, in_dtype, lda, sa) && aligned(W, w_dtype, ldw, sw);
+  if (vec && in_dtype == TA_F32 && w_dtype == TA_F32 && out_dtype == TA_F32 && batch == 1 && ta_gemm_stream_pays(M, N, K, 0))
+    return ta_gemm_stream(stream, (const float*)A, lda, (const float*)W, ldw, bias, (float*)C, ldc, M, N, K, 0, 0, nullptr, 0.f);
 #define LAUNCH(T, TW, TC)                                                                                   \
   do {                                                                                                      \
     if (vec) launch<T, TW, TC, true>(stream, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch);     \
