@@ -1554,13 +1554,17 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
 // ------------------------------------------------------------------ few tokens kept at most
 // A cut at top_k <= TOP_MOST_K in two kernels. A row keeps no token that top_k others of its own part go before, so
 //   top     a part hands on its tokens down to the step (1/16 of a unit of logit / T, counted from its largest) with which
-//           it has top_k of them, and the mass of all its tokens relative to its own largest;
-//   draw    one workgroup a row: of these some 40 to 100 tokens a part the step that holds the threshold, the order of the
-//           few tokens in it one against the other, and the token drawn, all from LDS.
+//           it has top_k of them (of the last one, where it holds too many, those down to one of its 256 equal pieces), and
+//           the mass of all its tokens relative to its own largest;
+//   draw    one workgroup a row: of these some 40 to 100 tokens a part the step that holds the threshold (the steps cut into as
+//           many as there is room for), the order of the few tokens in it one against the other, and the token drawn, all from LDS.
+// What is not handed on has top_k tokens of its own part in front of it, all of them handed on, so that neither counts nor sums
+// down to the threshold miss anything.
 // The cut by mass wants a share of the row's exact mass, which no part knows; the sum of the parts' is within MASS_ERROR of it,
 // and where the two ends of that interval keep different tokens, the row is added up exactly. A row whose threshold lies
-// below what some part has handed on (its largest tokens 16 units and more above the threshold), or with more equal tokens than
-// there is room for, is one workgroup's from the start. 8 rows of 128,256, top-k 40 and top-p 0.95: 27 us in the three
+// below what some part has handed on (its largest tokens 16 units and more above the threshold), or with more tokens within
+// 1/4,096 of a unit than there is room for, is one workgroup's from the start. (Whole steps alone left flat rows to it: 8 rows of
+// 128,256 of deviation 0.05 206 us, by the three kernels above 30, in pieces 17; of 0.003 204, 208 and 21.) 8 rows of 128,256, top-k 40 and top-p 0.95: 27 us in the three
 // kernels above, 15 in these two; 64 rows 50 and 24, 128 rows 75 and 34, 8 rows of 32,000 with top-k 50 24 and 13. Bound by the two kernels' chains:
 // a trip to memory and a histogram each, then one scan, the order in the step and a scan for the token.
 #define TOP_MOST_K 128
@@ -1585,7 +1589,7 @@ __device__ __forceinline__ int top_step(float l, float inv_t) {
 }
 
 __global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* __restrict__ logits, size_t ld, int vocab,
-                                                                  float inv_t, int top_k, int by_mass,
+                                                                  float inv_t, int top_k, int by_mass, int most,
                                                                   TopRecord* __restrict__ records) {
   constexpr int WAVES = PART_THREADS / TA_WAVE;
   const float* row = logits + (size_t)blockIdx.y * ld;
@@ -1595,7 +1599,7 @@ __global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* _
   __shared__ float s_f[WAVES];
   __shared__ uint32_t cnt[TOP_STEPS];
   __shared__ u64 s_rest[WAVES];
-  __shared__ int s_low, s_n[4][WAVES];
+  __shared__ int s_low, s_got, s_before, s_n[4][WAVES];
   static_assert(TOP_STEPS == PART_THREADS, "a thread a step");
   cnt[threadIdx.x] = 0;
   Four f[4];
@@ -1636,40 +1640,71 @@ __global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* _
     if (lane == 0) s_rest[wave] = all;
   }
   __syncthreads();
-  if (wave == 0) {                                 // a lane four steps
-    const uint4 c = *reinterpret_cast<const uint4*>(&cnt[4 * lane]);
-    const uint32_t mine = c.x + c.y + c.z + c.w;
-    uint32_t inc = mine;
+  // the step with which there are k tokens (the last one if there are not): how many with it, and how many in front of it
+  auto reach = [&](uint32_t k) {
+    if (wave == 0) {                               // a lane four steps
+      const uint4 c = *reinterpret_cast<const uint4*>(&cnt[4 * lane]);
+      const uint32_t mine = c.x + c.y + c.z + c.w;
+      uint32_t inc = mine;
 #pragma unroll
-    for (int o = 1; o < TA_WAVE; o <<= 1) {
-      const uint32_t up = __shfl_up(inc, o, TA_WAVE);
-      if (lane >= o) inc += up;
-    }
-    const u64 found = __ballot(inc >= (uint32_t)top_k);
-    const int who = found ? __ffsll((unsigned long long)found) - 1 : TA_WAVE - 1;
-    if (lane == who) {
-      uint32_t run = inc - mine;
-      int step = 4 * lane + 3;
-      uint32_t n = inc;
-      if (found) {
-        const uint32_t k = (uint32_t)top_k;
-        if (run + c.x >= k) { step = 4 * lane; n = run + c.x; }
-        else if (run + c.x + c.y >= k) { step = 4 * lane + 1; n = run + c.x + c.y; }
-        else if (run + c.x + c.y + c.z >= k) { step = 4 * lane + 2; n = run + c.x + c.y + c.z; }
+      for (int o = 1; o < TA_WAVE; o <<= 1) {
+        const uint32_t up = __shfl_up(inc, o, TA_WAVE);
+        if (lane >= o) inc += up;
       }
-      s_low = step;
-      u64 rest = 0;
-      if (by_mass)
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) rest += s_rest[w];
-      rec.rest = (double)rest;
-      rec.max = m;
-      rec.floor = (int)n < live ? top - step : NO_STEP;
-      rec.n = (int)n;
+      const u64 found = __ballot(inc >= k);
+      const int who = found ? __ffsll((unsigned long long)found) - 1 : TA_WAVE - 1;
+      if (lane == who) {
+        const uint32_t run = inc - mine;
+        int step = 4 * lane + 3;
+        uint32_t n = inc, last = c.w;
+        if (found) {
+          if (run + c.x >= k) { step = 4 * lane; n = run + c.x; last = c.x; }
+          else if (run + c.x + c.y >= k) { step = 4 * lane + 1; n = run + c.x + c.y; last = c.y; }
+          else if (run + c.x + c.y + c.z >= k) { step = 4 * lane + 2; n = run + c.x + c.y + c.z; last = c.z; }
+        }
+        s_low = step;
+        s_got = (int)n;
+        s_before = (int)(n - last);
+      }
     }
-  }
-  __syncthreads();
+    __syncthreads();
+  };
+  reach((uint32_t)top_k);
   const int low = s_low;
+  int n = s_got;
+  if (n > most) {                                  // more than top_k, then: of the last step the pieces that it takes from above
+    const int in_front = s_before;
+    auto piece = [&](float l) {                    // the fraction is exact
+      const float x = fminf(fmaxf(l * inv_t * TOP_PER_UNIT, -1e9f), 1e9f);
+      return TOP_STEPS - 1 - (int)((x - floorf(x)) * (float)TOP_STEPS);
+    };
+    cnt[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (at[u][e] == low) atomicAdd(&cnt[piece(f[u].v[e])], 1u);
+    __syncthreads();
+    reach((uint32_t)(top_k - in_front));
+    const int fine = s_low;
+    n = in_front + s_got;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (at[u][e] == low && piece(f[u].v[e]) > fine) at[u][e] = TOP_STEPS;
+  }
+  if (threadIdx.x == 0) {
+    u64 rest = 0;
+    if (by_mass)
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) rest += s_rest[w];
+    rec.rest = (double)rest;
+    rec.max = m;
+    rec.floor = n < live ? top - low : NO_STEP;
+    rec.n = n;
+  }
   int before[4];
   u64 take[4][4];
 #pragma unroll
@@ -1796,7 +1831,15 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const f
   };
   if (!s_ok) return whole();
   const float m = s_max;
-  const int cands = s_cands, top = top_step(m, inv_t);
+  const int cands = s_cands;
+  // the threshold lies in the steps from s_floor on: each is cut into as many as all 256 allow
+  int finer = 0;
+  const int span = s_floor > NO_STEP ? top_step(m, inv_t) - s_floor + 1 : TOP_STEPS;
+  if (fabsf(m * inv_t * TOP_PER_UNIT) < (float)(1 << 21))
+    while (finer < 7 && span <= (TOP_STEPS - 1) >> (finer + 1)) ++finer;
+  const float per_unit = TOP_PER_UNIT * (float)(1 << finer);
+  auto fine_step = [&](float l) { return (int)floorf(fminf(fmaxf(l * inv_t * per_unit, -1e9f), 1e9f)); };
+  const int top = fine_step(m);
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i) {
     const int p = wave + i * SAMPLE_WAVES;
@@ -1812,7 +1855,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const f
     }
   __syncthreads();
   auto step = [&](float l) {
-    const int at = top - top_step(l, inv_t);
+    const int at = top - fine_step(l);
     return at < TOP_STEPS - 1 ? at : TOP_STEPS - 1;
   };
   for (int c = threadIdx.x; c < cands; c += SAMPLE_THREADS) {
@@ -1867,7 +1910,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const f
     }
     __syncthreads();
     const int bin = s_bin;
-    if (bin == -1 || bin == TOP_STEPS - 1 || (bin >= 0 && top - bin < s_floor)) return whole();
+    if (bin == -1 || bin == TOP_STEPS - 1 || (bin >= 0 && (top - bin) >> finer < s_floor)) return whole();
     if (bin >= 0) {
       for (int c = threadIdx.x; c < cands; c += SAMPLE_THREADS) {
         const float l = cand_l[c];
@@ -2042,7 +2085,8 @@ static int sample_launch(hipStream_t stream, const float* logits, long long ld, 
       const dim3 g(parts, rows);
       if (few) {
         TopRecord* tops = (TopRecord*)scratch;
-        sample_top_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p < 1.0f, tops);
+        sample_top_kernel<<<g, PART_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p < 1.0f,
+                                                          ROW_CAND / parts < TOP_CAND ? ROW_CAND / parts : TOP_CAND, tops);
         sample_top_draw_kernel<<<rows, SAMPLE_THREADS, 0, stream>>>(from, (size_t)ld, vocab, inv_t, top_k, top_p, parts, tops,
                                                                     given ? nullptr : uniform + r0, args, r0, out + r0,
                                                                     out_host ? out_host + r0 : nullptr);
