@@ -258,8 +258,10 @@ static bool walk_takes(int M, int N, int K) {
   return M >= 1 && M <= 16 && K > 512 && K <= 4096 && (N + side - 1) / side >= walk_groups(M, K) * 5 / 4;
 }
 // Without an activation to save a launch: two tiles a workgroup where most of the last waves' k is past the end (6,000 x 520 at 1 /
-// 8 rows 6.4 / 6.7 us by few rows, 7.0 / 7.2 here, but 16,384 x 520 15.5 and 12.9; 3,000 x 1,032 at one row 6 % more here).
+// 8 rows 6.4 / 6.7 us by few rows, 7.0 / 7.2 here, but 16,384 x 520 15.5 and 12.9; 3,000 x 1,032 at one row 6 % more here). Up to 8
+// rows of a k above 2,048 are gemm_stream's (28,672 x 4,096 at 4 rows, gated, 88 us here and 80 there).
 static bool walk_pays(int M, int N, int K) {
+  if (M <= 8 && K > 2048) return false;
   const bool thin = M <= 8 && (K <= 640 || (M == 1 && K > 1024 && K <= 1280));
   return walk_takes(M, N, K) && (!thin || (N + 7) / 8 >= 2 * walk_groups(M, K));
 }
@@ -272,7 +274,7 @@ static void walk(hipStream_t stream, const float* A, int lda, const float* W, in
   if (M <= 8) {
     if (K <= 1024) WALK(2, true);
     else if (K <= 2048) WALK(4, true);
-    else WALK(8, true);
+    else if constexpr (GLU) WALK(8, true);
   } else {
     if (K <= 1024) WALK(4, false);
     else if (K <= 2048) WALK(8, false);
