@@ -1577,7 +1577,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
 struct TopRecord {
   double rest;             // mass of all its tokens, relative to its largest
   float max;
-  int floor;               // all tokens from this step on are handed on; NO_STEP: all there are
+  int floor;               // what is left out lies in this step, behind top_k others, or below; NO_STEP: nothing is left out
   int n, unused;
   float l[TOP_CAND];       // in index order
   uint16_t i[TOP_CAND];
@@ -1755,7 +1755,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const f
   __shared__ uint32_t h_cnt[TOP_STEPS], tie_key[TOP_TIES], tie_at[TOP_TIES];
   __shared__ u64 h_mass[TOP_STEPS], tie_q[TOP_TIES], s_wave[SAMPLE_WAVES];
   __shared__ int s_first[MAX_PARTS], s_n[MAX_PARTS];
-  __shared__ int s_ok, s_cands, s_floor, s_bin, s_ties, s_unsure, s_pick;
+  __shared__ int s_ok, s_cands, s_floor, s_bin, s_ties, s_unsure;
   __shared__ uint32_t s_count;
   __shared__ u64 s_mass, s_p[2];
   __shared__ float s_max;
@@ -1816,7 +1816,6 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_top_draw_kernel(const f
       s_ok = ok && run <= ROW_CAND && m > -INFINITY && m < INFINITY;
       s_ties = 0;
       s_unsure = 0;
-      s_pick = 0;
       // the mass with which the cut is reached lies between these
       const double want = (double)top_p * t;
       s_p[0] = by_mass ? (u64)fmax(ceil(want * (1.0 - MASS_ERROR)), 1.0) : NO_MASS_LIMIT;
@@ -2026,11 +2025,12 @@ static int rows_at_a_time(int vocab) {
 //   32,000 14.5 against 14.5; 8 x 128,256 16 against 44; 64 x 128,256 29 against 48; 512 x 128,256 148 against 104. A row
 //   alone costs 5 + 3e-4 a token, parts 12 + 2.1e-6 a token of all rows.
 // - else a workgroup gathers the kept tokens where they are few, and with every CU busy its three passes are cheaper than
-//   the parts' two with the exponential in both. k 40, p 0.95: 100 x 128,256 68 against 110 or so; 188: 101 against 80;
-//   512: 240 against 146; 2,500: 1,164 against 599; 740 x 32,000 108 against 130; 760: 119 against 72; 1,024 x 8,192 61
-//   against 121. Kept tokens that don't fit (a cut by mass alone can keep thousands) are walked nine times: 188 x 128,256,
+//   the parts' two with the exponential in both. k 200, p 0.95: 100 x 128,256 70 against 74, 187 105 against 81, 512 263 against 144;
+//   k 300: 750 x 32,000 122 against 74.
+//   Kept tokens that don't fit (a cut by mass alone can keep thousands) are walked nine times: 188 x 128,256,
 //   p 0.9, 109 against 286, 512 257 against 451, but 235 against 129 where dozens are kept: such cuts stay in parts a little
-//   longer.
+//   longer. Cuts at few tokens share the line, although their two kernels stay ahead beyond it: k 40, 187 x 128,256 43 against
+//   80, 512 110 against 142, 2,048 448 against 489, 750 x 32,000 54 against 71; with k 128 1,500 x 32,000 125 against 124.
 static bool in_parts(int n, int vocab, int top_k, float top_p) {
   if (sample_parts(vocab) > MAX_PARTS) return false;
   const long long all = (long long)n * vocab;
