@@ -437,10 +437,10 @@ __device__ __forceinline__ void la_chunk(const bf16_t* __restrict__ Ks, int RS, 
 // Narrow rows: a wave a tile. TEAM (the others): the four waves of a workgroup take ONE tile and share its chunks, which all threads
 // bring into one of two buffers behind a barrier a chunk; each forms the tile's scores and sums a quarter of the coordinates. A step of
 // single tokens has one tile a sequence where 16 heads share a row, and by a wave for itself the other three of its workgroup are gone:
-// attention and merge, 16 heads, rank 256, 900 keys, 1 / 4 / 64 sequences 26.2 / 26.9 / 103 us that way, 16.7 / 17.3 / 48 by four (30
-// with the fewer shares that four waves want); 128 heads, rank 512, 4 x 2,000 keys 199 and 62. With one share too: 257 / 512 / 1,000
-// sequences of 900 keys 554 / 577 / 1,145 us by a wave each (357 / 616 / 1,180 in seven, four, two shares), 88 / 94 / 186 by four;
-// 300 of 2,000, rank 512, 1,519 and 510; 300 of 60 43 and 13.
+// attention and merge, 16 heads, rank 256, 900 keys, 1 / 4 / 64 sequences 26.2 / 26.9 / 103 us that way, 16.7 / 17.3 / 48 by four, and
+// 14.5 / 15.5 / 29 with the fewer shares that four waves want and a merge by four; 128 heads, rank 512, 4 x 2,000 keys 199 and 62. With
+// one share too: 257 / 512 / 1,000 sequences of 900 keys 554 / 577 / 1,145 us by a wave each (357 / 616 / 1,180 in seven, four, two
+// shares), 88 / 94 / 186 by four; 300 of 2,000, rank 512, 1,519 and 510; 300 of 60 43 and 13.
 template <int KS, int CT, int RT>
 __global__ __launch_bounds__(256, ((KS <= 6 && RT == 1) ? 2 : 1)) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qa, bf16_t* __restrict__ out, const bf16_t* __restrict__ kcache,

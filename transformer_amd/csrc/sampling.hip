@@ -1564,9 +1564,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_draw_kernel(const float
 // and where the two ends of that interval keep different tokens, the row is added up exactly. A row whose threshold lies
 // below what some part has handed on (its largest tokens 16 units and more above the threshold), or with more tokens within
 // 1/4,096 of a unit than there is room for, is one workgroup's from the start. (Whole steps alone left flat rows to it: 8 rows of
-// 128,256 of deviation 0.05 206 us, by the three kernels above 30, in pieces 17; of 0.003 204, 208 and 21.) 8 rows of 128,256, top-k 40 and top-p 0.95: 27 us in the three
-// kernels above, 15 in these two; 64 rows 50 and 24, 128 rows 75 and 34, 8 rows of 32,000 with top-k 50 24 and 13. Bound by the two kernels' chains:
-// a trip to memory and a histogram each, then one scan, the order in the step and a scan for the token.
+// 128,256 of deviation 0.05 206 us, by the three kernels above 30, in pieces 17; of 0.003 204, 208 and 21.) 8 rows of 128,256,
+// top-k 40 and top-p 0.95: 27 us in the three kernels above, 15 in these two; 64 rows 50 and 24, 128 rows 75 and 34, 8 rows of
+// 32,000 with top-k 50 24 and 13. Bound by the two kernels' chains: a trip to memory and a histogram each, then one scan, the order
+// in the step and a scan for the token.
 #define TOP_MOST_K 128
 #define TOP_STEPS 256
 #define TOP_PER_UNIT 16.0f
