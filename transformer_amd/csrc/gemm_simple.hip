@@ -1,30 +1,25 @@
 // C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits on the matrix cores: the product of the true
 // 32-bit path, and the fallback for storage types and shapes that no faster kernel takes.
 //
-// The float32 matrix instructions are chains of fused multiply-adds: v_mfma_f32_16x16x4_f32 and
-// v_mfma_f32_32x32x2_f32 give the bits of fmaf over their 4 (2) k-slots in ascending order, denormals
-// included. Every output element is therefore summed in one order that depends on K alone, whatever
-// M, N, the kernel or the tile:
+// Every output element is summed in one order that depends on K and the types alone, whatever M, N, the kernel or the tile, so
+// a row of A gives the same bits alone or inside any batch. float32 by float32: split.h's. With a bfloat16 operand the products go to
+// the float32 matrix instructions, which are chains of fused multiply-adds: v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 give the
+// bits of fmaf over their 4 (2) k-slots in ascending order, denormals included. Then
 //   k is cut into segments of 256 and these into blocks of 16; a segment's chain starts at zero and takes
 //   its blocks in ascending order, and of a block k = 0 4 8 12, 1 5 9 13, 2 6 10 14, 3 7 11 15; the
 //   segments' sums are added in ascending order.
-// So a row of A gives the same bits alone or inside any batch. The order inside a block is the one in
-// which a lane that has read 4 consecutive k holds them: no operand is turned round.
-// Segments (instead of one chain over K) let few rows be split over waves; they also round less.
+// The order inside a block is the one in which a lane that has read 4 consecutive k holds them: no operand is turned round.
 //
-// Four kernels. gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk: the same for
-// wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns.
-// gemm_tiles: a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS; gemm_groups: 64, 96 or 128 x 64, two groups
-// of waves that take the segments in turn. Up to 8 rows of a long enough matrix are gemm_stream.hip's, with the same bits.
-#include "common.h"
+// gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk (float32): the same for
+// wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns. gemm_tiles (a bfloat16
+// operand): a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS. Many rows of float32 are gemm_split.hip's, up to 8 of a long
+// enough matrix gemm_stream.hip's, with the same bits.
+#include "gemm_split.h"
 #include "gemm_stream.h"
+#include "split.h"
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-#define SEG 256      // k per segment
-#define BLK 16       // k per block
 
 __device__ float4 gemm_zeros;      // where a piece past K is read from (never written: zero)
 
@@ -49,17 +44,18 @@ __device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
 }
 
 // Few rows (up to 16 * RT of them a workgroup), bound by reading W. A lane reads 4 consecutive k of a row of W and
-// of RT rows of A, which are the operands of 4 matrix instructions as they are (a row's four lanes cover 64
+// of RT rows of A, which are operands as they are (a row's four lanes cover 64
 // bytes); while one chunk of BC blocks is multiplied the next is on its way. The waves take the segments in
 // turn and leave the partial tiles in LDS, where they are added in ascending order after every round.
-// 16,384 x 2,048 at 1 / 4 / 16 rows: 30 / 33 / 38 us (4.5 TB/s of W at one row; 220 us by one thread an output on
-// the vector ALU), 2,048 x 8,192: 14.4 / 16.7 / 34.7 us (530).
+// float32, 2,048 columns over k = 8,192 at 9 / 16 / 32 / 64 rows 31 / 37 / 54 / 84 us (30 / 35 / 51 / 84 on the float32 matrix instructions:
+// from 32 rows on it is the splitting of A, once more for every 16 columns, that binds), 3,072 x 2,048 at 32 / 64 rows 15.2 / 21.8.
 // PAIR (up to 8 rows): a matrix instruction multiplies two segments side by side, 8 columns of W each, of
 // whose 16 x 16 products the two squares on the diagonal are used. A workgroup then owns 8 columns: a matrix of
 // 2,048 rows keeps 256 CUs reading instead of 128.
 // SHORT: k does not fill a round of segments. A wave then ends where k does instead of multiplying zeros to the end of
 // its segment: 40 x 5,000 x 64 6.3 us (21 without), 1 x 5,000 x 768 6.9 (10.6). The test between the chunks costs
 // long k 2 to 4 % (8 x 16,384 x 4,096 74.6 us without it, 77.3 with).
+// Eight waves take float32 products of 9 to 32 rows over a k of 4,096 and more whose workgroups leave the CUs half empty.
 template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool SHORT, bool VEC>
 __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __restrict__ A, int lda,
                                                                    const TW* __restrict__ W, int ldw,
@@ -67,6 +63,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
                                                                    TC* __restrict__ C, int ldc, int M, int N, int K,
                                                                    long long sa, long long sw, long long sc) {
   static_assert(!PAIR || RT == 1, "two segments in one tile");
+  static_assert(BC % 2 == 0, "blocks of split.h in pairs of 16 k");
+  constexpr bool SPLIT = sizeof(T) == 4 && sizeof(TW) == 4;
   A += (size_t)blockIdx.z * sa;
   W += (size_t)blockIdx.z * sw;
   C += (size_t)blockIdx.z * sc;
@@ -102,13 +100,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
   };
   f32x4 acc[RT];
   auto multiply = [&](int set) {
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int i = 0; i < BC; ++i)
+      for (int i = 0; i < BC; i += 2) {
+        const Split8 w = split8<false>(wreg[set][i], wreg[set][i + 1]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+        for (int t = 0; t < RT; ++t) acc[t] += split_block(w, split8<true>(areg[set][t][i], areg[set][t][i + 1]));
+      }
+    } else {
 #pragma unroll
-        for (int t = 0; t < RT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wreg[set][i][j], areg[set][t][i][j], acc[t], 0, 0, 0);
+      for (int i = 0; i < BC; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int t = 0; t < RT; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wreg[set][i][j], areg[set][t][i][j], acc[t], 0, 0, 0);
+    }
   };
   float total[OUT];
 #pragma unroll
@@ -153,8 +160,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
   for (int e = 0; e < OUT; ++e) {
     const int at = (int)threadIdx.x + WAVES * 64 * e;
     const int m = m0 + at / COLS, n = n0 + at % COLS;
-    if (at < ROWS * COLS && m < M && n < N)
-      C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
+    if (at >= ROWS * COLS || m >= M || n >= N) continue;
+    if (SPLIT && split_bad(total[e]))
+      total[e] = split_again([&](int k) { return to_f32(A[(size_t)m * lda + k]); }, reinterpret_cast<const float*>(W + (size_t)n * ldw), K);
+    C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
   }
 }
 
@@ -162,19 +171,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
 // segments of A in registers, the workgroup walks over tiles of 8 (16) columns, and the next tile's k are on their way
 // while the last ones of this are multiplied and added up. Bound by reading W. gemm_few_rows reads A again with every
 // tile, as many bytes as W at 8 rows, and its workgroups, which live for four chunks, start and end all the time:
-// 16,384 x 2,048 at 1 / 4 / 8 / 16 rows 31.6 / 33.5 / 40.2 / 39.0 us there, 25.4 / 25.7 / 26.6 / 28.9 here (5.2 TB/s
-// at 4 rows); 32,000 x 2,048 at 4 rows 67 and 48, 28,672 x 4,096 at 4 rows 116 and 85, 5,000 x 3,000 at 8 rows 27 and 20. One workgroup a CU with 8 KB of W a wave on their way is enough;
+// 16,384 x 2,048 at 16 rows 39 us there, 29.9 here (29.3 on the float32 matrix instructions), 32,000 x 2,048 52, 8,192 x 4,096 at 9 rows 35.7
+// (k above 2,048: eight waves with two segments each). One workgroup a CU with 8 KB of W a wave on their way is enough;
 // two or three a CU are up to 4 % slower. W passes the caches like any other read here: past them 3 % slower.
 // GLU: W holds gate rows, then up rows; a tile has half its columns of either and stores silu(gate) * up, with the bits
 // that the product and the activation's kernel give one after the other (a launch and two passes over its rows less).
-template <int WAVES, bool PAIR, bool GLU>
+template <int WAVES, int OWN, bool PAIR, bool GLU>
 __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __restrict__ A, int lda,
                                                                const float* __restrict__ W, int ldw,
                                                                const float* __restrict__ bias, float* __restrict__ C,
                                                                int ldc, int M, int N, int K, int tiles) {
   constexpr int SIDE = PAIR ? 8 : 16;            // rows and columns of a tile
-  constexpr int TURN = PAIR ? 2 * WAVES : WAVES; // segments
-  constexpr int BC = WAVES > 8 ? 4 : 8;          // blocks per chunk: sixteen waves have 128 registers each
+  static_assert(!PAIR || OWN == 1, "a wave's segments side by side or one after the other");
+  constexpr int TURN = PAIR ? 2 * WAVES : WAVES * OWN;   // segments
+  constexpr int BC = OWN == 1 ? 8 : 4;           // pieces per chunk: more registers for A, fewer for W
   constexpr int CH = SEG / (BC * BLK);           // chunks per segment
   constexpr int HALF = SIDE / 2;
   static_assert(WAVES * 64 >= SIDE * SIDE, "a thread an output");
@@ -188,32 +198,49 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
     const int n = GLU ? HALF * tile + col % HALF : SIDE * tile + col;
     return W + (size_t)((n < n_out ? n : n_out - 1) + (GLU && col >= HALF ? n_out : 0)) * ldw;
   };
-  f32x4 a[CH][BC], w[2][BC];
+  // the first k of a piece of chunk c: the wave's segments lie WAVES apart
+  auto k_of = [&](int c, int i) { return k0 + c / CH * WAVES * SEG + (c % CH * BC + i) * BLK; };
+  constexpr bool KEEP = OWN == 1;                // A split once; two segments of it take too many registers and are split every time
+  f32x4 a[KEEP ? 1 : CH * OWN][BC], w[2][BC];
+  Split8 as[KEEP ? CH : 1][BC / 2];
   auto load = [&](int c, const float* row) {
 #pragma unroll
-    for (int i = 0; i < BC; ++i) w[c % 2][i] = load_piece<float, true, false>(row, k0 + (c * BC + i) * BLK, K);
+    for (int i = 0; i < BC; ++i) w[c % 2][i] = load_piece<float, true, false>(row, k_of(c, i), K);
   };
   int tile = blockIdx.x;
   const float* row = rows_of(tile);
   load(0, row);
   const float* arow = A + (size_t)(col < M ? col : 0) * lda;
 #pragma unroll
-  for (int c = 0; c < CH; ++c)
+  for (int c = 0; c < CH * OWN; ++c) {
+    f32x4* to = a[KEEP ? 0 : c];
 #pragma unroll
-    for (int i = 0; i < BC; ++i) a[c][i] = load_piece<float, true, false>(arow, k0 + (c * BC + i) * BLK, K);
+    for (int i = 0; i < BC; ++i) to[i] = load_piece<float, true, false>(arow, k_of(c, i), K);
+    if (KEEP)
+#pragma unroll
+      for (int i = 0; i < BC; i += 2) as[KEEP ? c : 0][i / 2] = split8<true>(to[i], to[i + 1]);
+  }
   const int m = threadIdx.x / SIDE, nn = threadIdx.x % SIDE;
   for (int turn = 0; tile < tiles; tile += gridDim.x, turn ^= 1) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](int c) {
 #pragma unroll
-      for (int i = 0; i < BC; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[c % 2][i][j], a[c][i][j], acc, 0, 0, 0);
+      for (int i = 0; i < BC; i += 2) {
+        const Split8 wi = split8<false>(w[c % 2][i], w[c % 2][i + 1]);
+        if (KEEP) {
+          acc += split_block(wi, as[KEEP ? c : 0][i / 2]);
+        } else {
+          f32x4 x = a[KEEP ? 0 : c][i], y = a[KEEP ? 0 : c][i + 1];
+          asm volatile("" : "+v"(x), "+v"(y));   // or the compiler splits all of A in front of the loop and has no registers for it
+          acc += split_block(wi, split8<true>(x, y));
+        }
+      }
     };
     static_assert(CH % 2 == 0, "a segment's chunks in two sets of registers in turn");
+    auto* to = part[turn];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      if (c + 1 < CH) {
+    for (int c = 0; c < CH * OWN; ++c) {
+      if (c + 1 < CH * OWN) {
         load(c + 1, row);
       } else {                                   // the next tile's first
         row = rows_of(tile + (int)gridDim.x < tiles ? tile + (int)gridDim.x : tile);
@@ -222,13 +249,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
       __builtin_amdgcn_sched_barrier(0);
       multiply(c);
       __builtin_amdgcn_sched_barrier(0);
-    }
-    // a lane holds columns 4 kb .. + 3 of row r
-    auto* to = part[turn];
-    if (PAIR) {
-      if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[seg][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
-    } else {
-      *reinterpret_cast<f32x4*>(&to[seg][r * 16 + 4 * kb]) = acc;
+      if (c % CH != CH - 1) continue;
+      // a segment's end: a lane holds columns 4 kb .. + 3 of row r
+      if (PAIR) {
+        if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[seg][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
+      } else {
+        *reinterpret_cast<f32x4*>(&to[seg + c / CH * WAVES][r * 16 + 4 * kb]) = acc;
+      }
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     // one barrier a tile: who comes to this half again has passed the other half's, behind which all have read this one
     __syncthreads();
@@ -236,6 +264,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
       float total = 0.f;
       for (int s = 0; s < segs; ++s) total += to[s][threadIdx.x];
       const int n = (GLU ? HALF * tile + nn % HALF : SIDE * tile + nn);
+      if (split_bad(total) && m < M && n < n_out)
+        total = split_again([&](int k) { return A[(size_t)m * lda + k]; }, W + (size_t)(n + (GLU && nn >= HALF ? n_out : 0)) * ldw, K);
       if (bias && n < n_out) total += bias[n + (GLU && nn >= HALF ? n_out : 0)];
       if (GLU) {
         const float up = __shfl_xor(total, HALF, TA_WAVE);
@@ -269,29 +299,25 @@ template <bool GLU>
 static void walk(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc,
                  int M, int N, int K) {
   const int side = M <= 8 ? 8 : 16, tiles = (N + side - 1) / side, grid = walk_groups(M, K);
-#define WALK(WAVES, PAIR) \
-  gemm_walk_kernel<WAVES, PAIR, GLU><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles)
+#define WALK(WAVES, OWN, PAIR) \
+  gemm_walk_kernel<WAVES, OWN, PAIR, GLU><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles)
   if (M <= 8) {
-    if (K <= 1024) WALK(2, true);
-    else if (K <= 2048) WALK(4, true);
-    else if constexpr (GLU) WALK(8, true);
+    if (K <= 1024) WALK(2, 1, true);
+    else if (K <= 2048) WALK(4, 1, true);
+    else if constexpr (GLU) WALK(8, 1, true);
   } else {
-    if (K <= 1024) WALK(4, false);
-    else if (K <= 2048) WALK(8, false);
-    else WALK(16, false);
+    if (K <= 1024) WALK(4, 1, false);
+    else if (K <= 2048) WALK(8, 1, false);
+    else WALK(8, 2, false);
   }
 #undef WALK
 }
 
-// Many rows, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
+// Many rows with a bfloat16 operand, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
 // bytes of operands). 4 waves in 2 x 2 share a tile of 64 TT x 64 TT; each owns TT x TT tiles of 32 x 32. 32 k at a
-// time go through LDS, double buffered: row by row in 8 pieces of 16 bytes, permuted by the row number so that the
-// eight lanes that are served together meet no bank twice. float32 operands go from memory to LDS without passing
-// through registers (a wave's 64 pieces land side by side, so the permutation is in the addresses they are read
-// from); other types are converted on the way. Half h of a wave multiplies pieces h and h + 2 of a block's four,
-// element by element: the order above. 1,021 x 16,384 x 2,048: 535 us back to back (128 TFLOP/s; 566 in a prompt's
-// trace; 630 through registers, 1,880 on the vector ALU); the instruction alone reaches 154. With the barrier at a step's end instead of in its
-// middle 553, and 1,021 x 3,072 x 2,048 141 where it now takes 130.
+// time go through registers, where they become float32, and LDS, double buffered: row by row in 8 pieces of 16 bytes, permuted by the row
+// number so that the eight lanes that are served together meet no bank twice. Half h of a wave multiplies pieces h and h + 2 of a block's
+// four, element by element: the order above.
 template <typename T, typename TW, typename TC, int TT, bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict__ A, int lda,
                                                             const TW* __restrict__ W, int ldw,
@@ -301,60 +327,37 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
   A += (size_t)blockIdx.z * sa;
   W += (size_t)blockIdx.z * sw;
   C += (size_t)blockIdx.z * sc;
-  constexpr bool DIRECT = VEC && sizeof(T) == 4 && sizeof(TW) == 4;
   constexpr int BT = 64 * TT;                    // rows and columns of the tile
   constexpr int PER = BT * 8 / 256;              // pieces of an operand that a thread brings
-  constexpr int ST = DIRECT && TT == 1 ? 4 : 2;  // LDS buffers: ST - 1 steps are on their way
-  __shared__ f32x4 As[ST][BT * 8], Ws[ST][BT * 8];
+  __shared__ f32x4 As[2][BT * 8], Ws[2][BT * 8];
   const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
   const int n0 = blockIdx.x * BT, m0 = blockIdx.y * BT;
   const int lrow = threadIdx.x / 8;              // 32 rows of 128 bytes at a time
-  const int place = threadIdx.x % 8;             // piece of the row in LDS (DIRECT) or in memory
-  const int piece = DIRECT ? place ^ (lrow & 7) : place;
+  const int place = threadIdx.x % 8;             // piece of the row
   const T* asrc[PER];
   const TW* wsrc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int row = lrow + 32 * i;
-    asrc[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda + piece * 4;
-    wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw + piece * 4;
+    asrc[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda;
+    wsrc[i] = W + (size_t)(n0 + row < N ? n0 + row : N - 1) * ldw;
   }
-  f32x4 ain[DIRECT ? 1 : PER], win[DIRECT ? 1 : PER];
-  // step s's 32 k: into LDS buffer `buf` (DIRECT, piece i of each operand; the pointers walk along) or the registers
-  const int steps = (K + 31) / 32;
-  auto send = [&](int i, int buf, int s) {
-    if constexpr (DIRECT) {
-      const void *a = asrc[i], *w = wsrc[i];
-      if (s + 1 >= steps && K % 32 != 0) {       // past K: zeros from one address
-        const bool in = (steps - 1) * 32 + piece * 4 < K;
-        a = in ? a : (const void*)&gemm_zeros;
-        w = in ? w : (const void*)&gemm_zeros;
-      }
-      ta_load_to_lds16(a, &As[buf][(32 * i + 8 * wave) * 8]);
-      ta_load_to_lds16(w, &Ws[buf][(32 * i + 8 * wave) * 8]);
-      const int on = s + 1 < steps ? 32 : 0;     // behind the last step: the same once more, unused
-      asrc[i] += on;
-      wsrc[i] += on;
-    }
-  };
+  f32x4 ain[PER], win[PER];
+  const int steps = (K + 31) / 32;               // of 32 k
   auto fetch = [&](int s) {
-    if constexpr (!DIRECT) {
-      const int k0 = (s < steps ? s : steps - 1) * 32;
+    const int k0 = (s < steps ? s : steps - 1) * 32;
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        ain[i] = load_piece<T, VEC, false>(asrc[i] - piece * 4, k0 + piece * 4, K);
-        win[i] = load_piece<TW, VEC, false>(wsrc[i] - piece * 4, k0 + piece * 4, K);
-      }
+    for (int i = 0; i < PER; ++i) {
+      ain[i] = load_piece<T, VEC, false>(asrc[i], k0 + place * 4, K);
+      win[i] = load_piece<TW, VEC, false>(wsrc[i], k0 + place * 4, K);
     }
   };
   auto stash = [&](int buf) {
-    if constexpr (!DIRECT) {
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        const int row = lrow + 32 * i, at = row * 8 + (place ^ (row & 7));
-        As[buf][at] = ain[i];
-        Ws[buf][at] = win[i];
-      }
+    for (int i = 0; i < PER; ++i) {
+      const int row = lrow + 32 * i, at = row * 8 + (place ^ (row & 7));
+      As[buf][at] = ain[i];
+      Ws[buf][at] = win[i];
     }
   };
   const int half = lane / 32, r = lane % 32;
@@ -389,31 +392,24 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
   };
 
 #pragma unroll
-  for (int s = 0; s < ST; ++s) {
+  for (int s = 0; s < 2; ++s) {
     fetch(s);
-#pragma unroll
-    for (int i = 0; i < PER; ++i) send(i, s, s);
     stash(s);
   }
-  if constexpr (DIRECT) ta_wait_loads<2 * PER * (ST - 1)>();
   __syncthreads();
   read(0, 0);
   // The barrier stands in the middle of a step: in front of it a step's second block is read, behind it the
-  // step's buffer is free for the step ST further on, and the next step's first block is read while the second
-  // is multiplied, so that no wave waits for LDS right behind a barrier. What is sent for goes out between the
-  // products.
+  // step's buffer is free for the step after the next, and the next step's first block is read while the second
+  // is multiplied, so that no wave waits for LDS right behind a barrier.
   for (int s = 0; s < steps; ++s) {
-    const int buf = s % ST;
-    fetch(s + ST);
+    const int buf = s % 2;
+    fetch(s + 2);
     read(1, buf);
 #pragma unroll
     for (int j = 0; j < 4; ++j) multiply(0, j);
-    if constexpr (DIRECT) ta_wait_loads<2 * PER * (ST - 2)>();                // the next step's k have come
     __syncthreads();
     stash(buf);
-#pragma unroll
-    for (int i = 0; i < PER; ++i) send(i, buf, s + ST);
-    read(0, (s + 1) % ST);
+    read(0, (s + 1) % 2);
 #pragma unroll
     for (int j = 0; j < 4; ++j) multiply(1, j);
     if ((s + 1) % (SEG / 32) == 0 || s + 1 == steps) {
@@ -428,7 +424,6 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
           }
     }
   }
-  if constexpr (DIRECT) ta_wait_loads<0>();      // nothing may land in LDS that is another's
   // accumulator: register e of a lane is row 8 (e / 4) + 4 half + e % 4 of the tile, column r
 #pragma unroll
   for (int y = 0; y < TT; ++y) {
@@ -445,185 +440,35 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
   }
 }
 
-// Tiles of 32 WM x 64 over k of more than a segment, float32: two groups of 2 WM waves take the segments in turn, each
-// wave one 32 x 32 of the tile, and the second group hands its segment's sums to the first through LDS, which adds them in
-// ascending order. Operands go to LDS as in gemm_tiles, for both groups' 32 k at a time, the barrier in the middle of a step.
-// What it gains over gemm_tiles with 64 x 64 (one group): four waves a SIMD instead of two, whose waits for LDS, loads and
-// barriers fill each other, and a tile's height that fits the CUs: a CU's time follows the rows it is given, on one workgroup
-// or on two (an older workgroup's waves go first and the younger one is left with a CU to itself), so that the host picks
-// the height whose tiles leave the CUs evenly filled. 2,048 columns over k = 8,192: 1,021 rows 292 us (309 to 331 by 64 x 64),
-// 743 rows 233 (305), 300 rows 160 (247 by few rows). The matrix instructions alone take 232 of the 292, LDS reads 20 more; the
-// rest goes with the loads (four further waves that do nothing but load, 64 x 64 and one group: 294). A k that ends inside a round
-// of 512 ends the round (300 rows of 6,000 columns over k = 520 / 1,544 29.8 / 67.7 us, in whole rounds 45.5 / 81.3).
-// Its steps of 32 k of either group: the last round ends where its first segment does (the second is no longer, and there is none
-// where there is an odd number).
-__host__ __device__ __forceinline__ int groups_steps(int K) {
-  const int full = ((K + SEG - 1) / SEG - 1) / 2, rest = K - full * (2 * SEG);
-  return full * (SEG / 32) + (rest < SEG ? (rest + 31) / 32 : SEG / 32);
-}
-
-// WHOLE: of whole rounds (asking every step whether it is the last costs a hundredth of the time).
-template <int WM, bool WHOLE>
-__global__ __launch_bounds__(WM * 256) void gemm_groups_kernel(const float* __restrict__ A, int lda,
-                                                               const float* __restrict__ W, int ldw,
-                                                               const float* __restrict__ bias, float* __restrict__ C,
-                                                               int ldc, int M, int N, int K, long long sa, long long sw,
-                                                               long long sc) {
-  constexpr int WN = 2, WK = 2, ST = 2;          // waves along the columns, groups, LDS buffers
-  constexpr int WAVES = WM * WN * WK, ROWS = 32 * (WM + WN);
-  constexpr int CHUNKS = WK * ROWS / 8, PER = (CHUNKS + WAVES - 1) / WAVES;     // 8 rows of 128 bytes a load
-  A += (size_t)blockIdx.z * sa;
-  W += (size_t)blockIdx.z * sw;
-  C += (size_t)blockIdx.z * sc;
-  __shared__ f32x4 S[ST][WK][ROWS * 8];          // rows of A, then rows of W
-  __shared__ float handed[WM * WN][16][TA_WAVE];
-  const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE;
-  const int n0 = blockIdx.x * 32 * WN, m0 = blockIdx.y * 32 * WM;
-  const int group = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const int segs = (K + SEG - 1) / SEG, steps = WHOLE ? (segs + 1) / 2 * (SEG / 32) : groups_steps(K);
-  // the chunks this wave brings (WM = 3: four loads a wave for 40 chunks, so that every wave waits for as many; the last chunk
-  // is brought by nine of the twelve waves, the same bytes each time)
-  const float* src[PER];
-  int to[PER], from_k[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int c = wave + WAVES * i < CHUNKS ? wave + WAVES * i : CHUNKS - 1;
-    const int of = c / (ROWS / 8), rows8 = c % (ROWS / 8) * 8, row = rows8 + lane / 8;
-    from_k[i] = of * SEG + ((lane % 8) ^ (row & 7)) * 4;
-    if (row < 32 * WM) src[i] = A + (size_t)(m0 + row < M ? m0 + row : M - 1) * lda + from_k[i];
-    else src[i] = W + (size_t)(n0 + row - 32 * WM < N ? n0 + row - 32 * WM : N - 1) * ldw + from_k[i];
-    to[i] = (of * ROWS + rows8) * 8;
-  }
-  const int inside = K / (WK * SEG) * (SEG / 32);      // steps that lie inside K in both groups
-  auto send = [&](int buf, int s) {
-    if (s >= steps) s = steps - 1;                     // behind the last step: the same once more, unused
-    const int k = s / (SEG / 32) * (WK * SEG) + s % (SEG / 32) * 32;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const void* p = src[i] + k;
-      if (s >= inside) p = from_k[i] + k < K ? p : (const void*)&gemm_zeros;    // past K: zeros from one address
-      ta_load_to_lds16(p, &S[buf][0][to[i]]);
-    }
-  };
-  const int half = lane / 32, r = lane % 32;
-  f32x16 total, acc;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) total[e] = acc[e] = 0.f;
-  f32x4 a[2][2], w[2][2];
-  auto read = [&](int set, int buf) {
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int at = (4 * set + 2 * p + half) ^ (r & 7);
-      a[set][p] = S[buf][group][(32 * wm + r) * 8 + at];
-      w[set][p] = S[buf][group][(32 * (WM + wn) + r) * 8 + at];
-    }
-  };
-  auto multiply = [&](int set, int j) {
-#pragma unroll
-    for (int p = 0; p < 2; ++p) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][p][j], w[set][p][j], acc, 0, 0, 0);
-  };
-  auto take_over = [&]() {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) total[e] += handed[wave][e][lane];
-  };
-#pragma unroll
-  for (int s = 0; s < ST; ++s) send(s, s);
-  ta_wait_loads<PER * (ST - 1)>();
-  __syncthreads();
-  read(0, 0);
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s % ST;
-    read(1, buf);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) multiply(0, j);
-    ta_wait_loads<PER * (ST - 2)>();                   // the next step's k have come
-    __syncthreads();
-    // the first step's barrier of a round: the other group's sums of the round before lie in LDS
-    if (group == 0 && s % (SEG / 32) == 0 && s > 0) take_over();
-    send(buf, s + ST);
-    read(0, (s + 1) % ST);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) multiply(1, j);
-    if (s % (SEG / 32) == SEG / 32 - 1 || (!WHOLE && s == steps - 1)) {
-      if (group == 0) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) total[e] += acc[e];
-      } else if (WHOLE || s / (SEG / 32) * 2 + 1 < segs) {       // (a round of one segment may end before the sums in front of it are read)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) handed[wave - WM * WN][e][lane] = acc[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    }
-  }
-  ta_wait_loads<0>();                                  // nothing may land in LDS that is another's
-  __syncthreads();
-  if (group != 0) return;
-  if (segs % 2 == 0) take_over();                      // an odd number of segments ends with the first group's
-  // accumulator: register e of a lane is row 8 (e / 4) + 4 half + e % 4 of the tile, column r
-  const int n = n0 + 32 * wn + r;
-  if (n >= N) return;
-  const float add = bias ? bias[n] : 0.f;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int m = m0 + 32 * wm + 8 * (e / 4) + 4 * half + e % 4;
-    if (m < M) C[(size_t)m * ldc + n] = bias ? total[e] + add : total[e];
-  }
-}
-
-// The height WM of gemm_groups' tiles for a product, or 0 where another kernel takes it. A CU's time is that of the tiles it is
-// given, 36.5 us for 32 rows of 64 columns over k = 8,192 in tiles of 64 rows, 3 % more in tiles of 96, 2 % less in tiles of 128,
-// and 12 % less in gemm_tiles' 128 x 128 once there are enough of those to fill it (1,021 x 16,384 x 2,048: 534 us there, 614 here;
-// 300 rows 265 and 205). Below 129 tiles of 64 x 64 the few-rows kernel's finer workgroups are as fast (2,048 columns over k =
-// 8,192: 256 rows 168 and 161 us, 128 rows 79 and 158), and two segments or fewer give the groups too little (2,048 x 512 x 300
-// 13 us by 64 x 64, 17 here). Nor do they gain where a round is half empty and the tiles of 64 x 64 would fill the CUs: time follows the
-// steps (300 rows of 6,000 columns over k = 768 / 900 / 1,280 / 2,300 22, 9, 13 and 8 % more than by 64 x 64, 1,024 / 2,048 / 2,056 level, 3,000
-// columns 2 to 6 % less).
-static int groups_height(int M, int N, int K, int batch) {
-  auto tiles = [&](int rows, int cols) { return (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * batch; };
-  if (M <= 64 || K <= 2 * SEG || tiles(64, 64) <= 128) return 0;
-  if (tiles(64, 64) >= 192 && tiles(128, 128) < 384 && groups_steps(K) * 6400ll > K * 103ll) return 0;
-  auto cost = [&](int wm, int each) { return (tiles(32 * wm, 64) + CUS - 1) / CUS * wm * each; };
-  const long long c2 = cost(2, 100), c3 = cost(3, 103), c4 = cost(4, 98);
-  const long long least = c2 < c3 ? (c2 < c4 ? c2 : c4) : (c3 < c4 ? c3 : c4);
-  if (tiles(128, 128) >= 384 && (tiles(128, 128) + CUS - 1) / CUS * 8 * 88 <= least) return 0;
-  return least == c4 ? 4 : least == c2 ? 2 : 3;
-}
-
 template <typename T, typename TW, typename TC, bool VEC>
 static void launch(hipStream_t stream, const void* A_, int lda, long long sa, const void* W_, int ldw, long long sw,
                    const float* bias, void* C_, int ldc, long long sc, int M, int N, int K, int batch) {
   const T* A = (const T*)A_;
   const TW* W = (const TW*)W_;
   TC* C = (TC*)C_;
-  auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
-  // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
-  // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
-  // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
-  // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
-  const bool brief = K <= 128;
-  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
-    if (const int wm = groups_height(M, N, K, batch)) {
-      const dim3 grid((N + 63) / 64, (M + 32 * wm - 1) / (32 * wm), batch);
-#define GROUPS_(WM, WHOLE) \
-  gemm_groups_kernel<WM, WHOLE><<<grid, WM * 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
-#define GROUPS(WM) \
-  if (groups_steps(K) % (SEG / 32) == 0) GROUPS_(WM, true); else GROUPS_(WM, false)
-      if (wm == 2) { GROUPS(2); } else if (wm == 3) { GROUPS(3); } else { GROUPS(4); }
-#undef GROUPS
-#undef GROUPS_
+  constexpr bool F32 = sizeof(T) == 4 && sizeof(TW) == 4;
+  if constexpr (F32) {
+    if (const int form = ta_gemm_split_form(M, N, K, lda, ldw, batch, VEC)) {
+      ta_gemm_split(stream, form, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch, VEC);
       return;
     }
-  if (tiles(64) >= 192 && (M > 64 || brief)) {
-    if (tiles(128) >= 384)
-      gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
-          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
-    else
-      gemm_tiles_kernel<T, TW, TC, 1, VEC><<<dim3((N + 63) / 64, (M + 63) / 64, batch), 256, 0, stream>>>(
-          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
-    return;
+  } else {
+    // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
+    // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
+    // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
+    // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
+    auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
+    if (tiles(64) >= 192 && (M > 64 || K <= 128)) {
+      if (tiles(128) >= 384)
+        gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
+            A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+      else
+        gemm_tiles_kernel<T, TW, TC, 1, VEC><<<dim3((N + 63) / 64, (M + 63) / 64, batch), 256, 0, stream>>>(
+            A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+      return;
+    }
   }
-  if constexpr (VEC && sizeof(T) == 4 && sizeof(TW) == 4 && sizeof(TC) == 4)
+  if constexpr (VEC && F32)
     if (batch == 1 && walk_pays(M, N, K)) {
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
@@ -640,8 +485,8 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   // four waves a workgroup and 16 KB on their way in each: several workgroups share a CU and fill each other's
   // starts and ends (16,384 x 2,048 at 16 rows: 38 us; 44 with eight waves and twice the loads)
   if (M <= 8) FEW(4, 1, 4, true);
-  else if (M <= 16) FEW(4, 1, 4, false);
-  else if (M <= 32) FEW(4, 2, 2, false);
+  else if (M <= 16) { if (F32 && K >= 4096 && (N + 15) / 16 <= 256) FEW(8, 1, 4, false); else FEW(4, 1, 4, false); }
+  else if (M <= 32) { if (F32 && K >= 4096 && (N + 15) / 16 <= 256) FEW(8, 2, 2, false); else FEW(4, 2, 2, false); }
   else FEW(4, 4, 2, false);
 #undef FEW_
 #undef FEW

@@ -1,0 +1,284 @@
+// C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits for many rows, on the 16-bit matrix instructions (split.h, which also states the
+// order of the sums: a row has the bits here that it has in the kernels for few rows).
+#include "split.h"
+#include "gemm_split.h"
+
+__device__ f32x4 split_zeros;      // where a piece past K is read from (never written: zero)
+
+// A workgroup owns 32 WAVES x 16 NT of C. A wave owns 32 of the rows: it reads them from memory in operand layout and splits them,
+// which no other wave needs; the columns' k are split once per workgroup, by all its waves, and go through LDS in operand layout,
+// 32 k at a time in two buffers, one barrier a step. The next step's operands are split between this step's products and what comes after them is
+// asked for right there. Bound by issue: 96 matrix instructions of 16 cycles, some 230 vector instructions and 30 of LDS a step of 32 k and wave. 1,021 x
+// 16,384 x 2,048 352 us (195 TFLOP/s, 1.17 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 80
+// (122), x 2,048 x 2,048 59 (79), x 2,048 x 8,192 211 (292). A split once by a kernel in front: the same (386 us and 384). Four waves of 64 rows: 455 for 370. G groups of WAVES waves take the segments of k in turn and the first adds up what the others hand it through LDS,
+// in ascending order.
+template <int WAVES, int NT, int G, bool VEC, bool WHOLE>
+__global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
+                                                                    int ldw, const float* __restrict__ bias, float* __restrict__ C,
+                                                                    int ldc, int M, int N, int K, long long sa, long long sw,
+                                                                    long long sc, int tiles_m, int tiles) {
+  static_assert(NT >= 4 && NT % 2 == 0, "columns in pairs of tiles, the rows' splits between them");
+  constexpr int MT = 2, COLS = 16 * NT, ROWS = 16 * MT * WAVES;
+  constexpr int BRING = (NT + WAVES - 1) / WAVES;      // tiles of 16 columns that a wave brings
+  __shared__ bf16x8 S[G][2][3][NT][TA_WAVE];
+  __shared__ f32x4 handed[G > 1 ? G - 1 : 1][G > 1 ? WAVES : 1][G > 1 ? MT * NT : 1][G > 1 ? TA_WAVE : 1];
+  const int lane = threadIdx.x % TA_WAVE, at = __builtin_amdgcn_readfirstlane(threadIdx.x / TA_WAVE), wave = at % WAVES, group = at / WAVES;
+  const int r = lane % 16, kb = lane / 16;
+  // an XCD's workgroups (every eighth) walk neighbouring tiles, rows first
+  const int share = (tiles + 7) / 8, tile = blockIdx.x % 8 * share + blockIdx.x / 8;
+  if (tile >= tiles) return;
+  A += (size_t)blockIdx.y * sa;
+  W += (size_t)blockIdx.y * sw;
+  C += (size_t)blockIdx.y * sc;
+  const int m0 = tile % tiles_m * ROWS, n0 = tile / tiles_m * COLS;
+  const int blocks = (K + 31) / 32, segs = (K + SEG - 1) / SEG, rounds = (segs + G - 1) / G;
+  // steps of this group: 8 to a segment, and no further than the longest group's k
+  const int last = segs - (rounds - 1) * G > 1 ? SEG / 32 : blocks - (segs - 1) * (SEG / 32);
+  const int steps = (rounds - 1) * (SEG / 32) + last;
+  const char* abase = reinterpret_cast<const char*>(A + (size_t)m0 * lda);
+  const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw);
+  uint32_t aoff[MT], woff[BRING];                      // rows past M or N read another row and feed what is never stored
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = wave * 16 * MT + 16 * i + r;
+    aoff[i] = ((uint32_t)(m0 + m < M ? m : M - 1 - m0) * lda + 4 * kb) * 4;
+  }
+#pragma unroll
+  for (int i = 0; i < BRING; ++i) {
+    const int f = wave + WAVES * i < NT ? wave + WAVES * i : NT - 1, n = 16 * f + r;
+    woff[i] = ((uint32_t)(n0 + n < N ? n : N - 1 - n0) * ldw + 4 * kb) * 4;
+  }
+  auto piece = [&](const char* base, uint32_t off, int b, int h) {
+    const char* p = base + (size_t)b * 128 + off + 64 * h;
+    if (VEC) {
+      if (!WHOLE) p = b * 32 + 16 * h + 4 * kb < K ? p : reinterpret_cast<const char*>(&split_zeros);
+      return *reinterpret_cast<const f32x4*>(p);
+    }
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const char* q = b * 32 + 16 * h + 4 * kb + e < K ? p + 4 * e : reinterpret_cast<const char*>(&split_zeros);
+      v[e] = *reinterpret_cast<const float*>(q);
+    }
+    return v;
+  };
+  f32x4 win[BRING][2], ain[MT][2];
+  Split8 a[2][MT];
+  // WHOLE (K of whole segments): behind the last block the same once more, unused; else zeros
+  auto block_of = [&](int s) {
+    const int b = (s / (SEG / 32) * G + group) * (SEG / 32) + s % (SEG / 32);
+    return !WHOLE || b < blocks ? b : blocks - 1;
+  };
+  auto load_w = [&](int s) {
+    const int b = block_of(s);
+#pragma unroll
+    for (int i = 0; i < BRING; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) win[i][h] = piece(wbase, woff[i], b, h);
+  };
+  auto load_a = [&](int i, int s) {
+    const int b = block_of(s);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) ain[i][h] = piece(abase, aoff[i], b, h);
+  };
+  auto stash = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < BRING; ++i) {
+      const int f = wave + WAVES * i;
+      if (NT % WAVES == 0 || f < NT) {
+        const Split8 w = split8<false>(win[i][0], win[i][1]);
+        S[group][buf][0][f][lane] = w.h;
+        S[group][buf][1][f][lane] = w.m;
+        S[group][buf][2][f][lane] = w.l;
+      }
+    }
+  };
+  f32x4 acc[MT][NT], total[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  load_w(0);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) load_a(i, 0);
+  stash(0);
+  load_w(1);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    a[0][i] = split8<true>(ain[i][0], ain[i][1]);
+    load_a(i, 1);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  auto step = [&](int s, int buf) {
+#pragma unroll
+    for (int j = 0; j < NT; j += 2) {
+      Split8 w[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        w[x].h = S[group][buf][0][j + x][lane];
+        w[x].m = S[group][buf][1][j + x][lane];
+        w[x].l = S[group][buf][2][j + x][lane];
+      }
+      f32x4 t[MT][2];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) t[i][0] = t[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) t[i][x] = split_mul(q, w[x], a[buf][i], t[i][x]);
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[i][j + x] += t[i][x];
+      if (j == 0) {
+        stash(buf ^ 1);
+        load_w(s + 2);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        if (j == (NT > 4 ? 2 + 2 * i : 2 * i)) {
+          a[buf ^ 1][i] = split8<true>(ain[i][0], ain[i][1]);
+          load_a(i, s + 2);
+        }
+      // two products, then up to five of the vector instructions between them
+#pragma unroll
+      for (int z = 0; z < 12; ++z) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  for (int s0 = 0, round = 0; round < rounds; ++round) {
+    const int end = s0 + SEG / 32 < steps ? s0 + SEG / 32 : steps;
+    for (; s0 < end; s0 += 2) {
+      step(s0, 0);
+      if (s0 + 1 < end) step(s0 + 1, 1);
+    }
+    if (G > 1 && group > 0) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) handed[group - 1][wave][i * NT + j][lane] = acc[i][j];
+    }
+    if (G > 1) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // (the next round's first barrier lies behind these reads and in front of its sums)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if (group == 0) {
+          total[i][j] += acc[i][j];
+#pragma unroll
+          for (int g = 1; g < G; ++g)
+            if (round * G + g < segs) total[i][j] += handed[g - 1][wave][i * NT + j][lane];
+        }
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  if (group > 0) return;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int m = m0 + wave * 16 * MT + 16 * i + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int n = n0 + 16 * j + 4 * kb + e;
+        if (n >= N) continue;
+        const float v = total[i][j][e];
+        bad |= split_bad(v);
+        C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
+      }
+  }
+  if (!bad) return;
+#pragma unroll 1
+  for (int x = 0; x < MT * NT * 4; ++x) {              // what this lane has stored that is not finite
+    const int m = m0 + wave * 16 * MT + 16 * (x / (NT * 4)) + r, n = n0 + 16 * (x / 4 % NT) + 4 * kb + x % 4;
+    if (m >= M || n >= N) continue;
+    float* c = C + (size_t)m * ldc + n;
+    if (!split_bad(*c)) continue;
+    const float* row = A + (size_t)m * lda;
+    const float v = split_again([&](int k) { return row[k]; }, W + (size_t)n * ldw, K);
+    *c = bias ? v + bias[n] : v;
+  }
+}
+
+// us a step of 32 k (of all groups) when every CU has its workgroups: measured at 130 to 3,000 rows of 2,048 to 16,384 columns, k = 2,048
+// and 8,192. 256 x 128 reads and splits least per product but leaves CUs idle where there are few tiles: 1,021 x 16,384 x 2,048 330 to 380 us there,
+// 427 by 128 x 64, 483 by 128 x 96; 1,021 x 3,072 x 2,048 149, 107 and 82. Groups fill a CU that has a tile to itself: 1,021 x 2,048 x 8,192 268
+// by one group, 214 by two; 300 x 2,048 x 8,192 264, 187 and by four groups on 64 x 64 127. Two workgroups of 128 x 64 with one group share a CU.
+struct SplitForm {
+  int waves, nt, groups;
+  float us;
+};
+constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f}, {8, 8, 1, 2.5f}, {4, 6, 2, 2.45f}, {4, 4, 2, 1.7f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}, {2, 4, 1, 0.f}};
+enum { SPLIT_PAIRED = 5, SPLIT_SMALL = 6, SPLIT_CUS = 256 };
+
+static long long split_tiles(int form, int M, int N) {
+  const SplitForm& f = SPLIT_FORMS[form];
+  return (long long)((M + 32 * f.waves - 1) / (32 * f.waves)) * ((N + 16 * f.nt - 1) / (16 * f.nt));
+}
+static double split_cost(int form, int M, int N, int K, int batch) {
+  const SplitForm& f = SPLIT_FORMS[form];
+  const long long tiles = split_tiles(form, M, N) * batch;
+  const int segs = (K + SEG - 1) / SEG, steps = f.groups == 1 ? (K + 31) / 32 : (segs + f.groups - 1) / f.groups * (SEG / 32);
+  if (form != SPLIT_PAIRED) return (double)((tiles + SPLIT_CUS - 1) / SPLIT_CUS) * steps * f.us;
+  const long long rest = tiles % (2 * SPLIT_CUS);      // alone on its CU a workgroup takes 1.05 us a step
+  return (tiles / (2 * SPLIT_CUS) * f.us + (rest > SPLIT_CUS ? f.us : rest > 0 ? 1.05f : 0.f)) * steps;
+}
+
+// the few-rows kernel's: a workgroup of 16 columns and 32 or 64 rows, four segments at a time
+static double split_few_cost(int M, int N, int K, int batch) {
+  const int rows = M <= 32 ? 32 : 64;
+  const long long groups = (long long)((N + 15) / 16) * ((M + rows - 1) / rows) * batch;
+  const int rounds = (K + 4 * SEG - 1) / (4 * SEG);
+  return (double)((groups + SPLIT_CUS - 1) / SPLIT_CUS) * rounds * (M <= 32 ? 7.0 : rounds > 1 ? 10.5 : 7.5);
+}
+
+int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool vec) {
+  if (lda > 4194303 || ldw > 4194303) return 0;        // rows of a tile by 32-bit offsets
+  const long long tiles = split_tiles(SPLIT_SMALL, M, N) * batch;
+  const bool brief = K <= 128;
+  if (tiles > 2147483640ll || (M <= 16 && !brief)) return 0;
+  // over a short k it is the start and the end that count (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2)
+  if (brief) return tiles < 192 ? 0 : tiles < 2 * SPLIT_CUS ? SPLIT_SMALL : SPLIT_PAIRED;
+  int best = 0;
+  double least = split_few_cost(M, N, K, batch);
+  for (int f = vec ? 1 : SPLIT_PAIRED; f <= SPLIT_PAIRED; ++f) {
+    const double cost = split_cost(f, M, N, K, batch) + 4.0;
+    if (cost < least) best = f, least = cost;
+  }
+  return best;
+}
+
+void ta_gemm_split(hipStream_t stream, int form, const float* A, int lda, long long sa, const float* W, int ldw, long long sw,
+                   const float* bias, float* C, int ldc, long long sc, int M, int N, int K, int batch, bool vec) {
+  const int tiles = (int)split_tiles(form, M, N), tiles_m = (M + 32 * SPLIT_FORMS[form].waves - 1) / (32 * SPLIT_FORMS[form].waves);
+#define RUN_(WAVES, NT, G, VEC, WHOLE)                                                                        \
+  gemm_split_kernel<WAVES, NT, G, VEC, WHOLE><<<dim3((tiles + 7) / 8 * 8, batch), WAVES * G * 64, 0, stream>>>( \
+      A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc, tiles_m, tiles)
+#define RUN(WAVES, NT, G)                              \
+  if (K % SEG == 0) RUN_(WAVES, NT, G, true, true);    \
+  else RUN_(WAVES, NT, G, true, false)
+#define RUN_ANY(WAVES, NT, G)                          \
+  if (!vec) RUN_(WAVES, NT, G, false, false);          \
+  else RUN(WAVES, NT, G)
+  switch (form) {
+    case 1: RUN(8, 8, 1); break;
+    case 2: RUN(4, 6, 2); break;
+    case 3: RUN(4, 4, 2); break;
+    case 4: RUN(2, 4, 4); break;
+    case 5: RUN_ANY(4, 4, 1); break;
+    default: RUN_ANY(2, 4, 1); break;
+  }
+#undef RUN_ANY
+#undef RUN
+#undef RUN_
+}

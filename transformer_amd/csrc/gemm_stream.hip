@@ -1,22 +1,18 @@
 // C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits for up to 8 rows: the products of a float32 decode step, bound by
-// reading W once. The sums are gemm_simple.hip's (segments of 256 k, blocks of 16, chains of fused multiply-adds in its
-// order; a matrix instruction multiplies two segments side by side, 8 columns of W each), so a row has the same bits here and there.
+// reading W once. The sums are split.h's (a matrix instruction multiplies two segments side by side, 8 columns of W each), so a row
+// has the same bits here and in the kernels for more rows.
 //
 // W goes from memory to LDS without passing through registers, whole lines at a time: 64 k of 8 columns of two segments are
 // 16 runs of 256 bytes, 4 KB, and every wave has a ring of its own of such chunks, up to 128 KB a CU on their way, that is
 // asked for across the ends of tiles. Operand layout straight from memory (gemm_walk, gemm_few_rows) touches half a line per row and
 // instruction: at 4 rows 16,384 x 2,048 gated 28.2 us there and 24.9 here (5.4 TB/s), 28,672 x 4,096 gated 88 and 80, 2,048 x 8,192 19.2 and 15.4,
-// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55.
+// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55 (on the float32 matrix instructions; splitting the operands costs a kernel 0.2 to 0.5
+// us more at its start and end: the four products of a layer of width 2,048 and 8,192, 1 / 4 / 8 rows, 57.6 / 60.2 / 64.3 us and 59.7 / 61.3 / 64.6).
 //
 // A product may take the RMS norm in front of it (its workgroups form the rows' factors once more each, which costs 1 to 3 us
 // where the norm's own launch costs 4 to 5), and add its result to the residual stream where it stores it.
-#include "common.h"
 #include "gemm_stream.h"
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-#define SEG 256      // k per segment
-#define BLK 16       // k per block
+#include "split.h"
 
 __device__ float4 stream_zeros;    // where a piece past K is read from (never written: zero)
 
@@ -37,7 +33,7 @@ struct StreamNorm {
 // others: behind all of them they would be there only when those are, in front of all of them memory would wait for them (the norm's
 // rows by waves of their own: 16,384 x 2,048 33 us instead of 27).
 template <int WAVES, int PF, bool GLU, bool NORM, bool TAIL>
-__global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const float* __restrict__ A, int lda,
+__global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float* __restrict__ A, int lda,
                                                                  const float* __restrict__ W, int ldw,
                                                                  const float* __restrict__ bias, float* __restrict__ C, int ldc,
                                                                  int M, int N, int K, int tiles, int add, StreamNorm nm) {
@@ -143,8 +139,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const float* __
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[i][e] = a[i][e] * rstd * g[i][e];
   }
+  Split8 as[CH * 2];                             // A, split where the first tile needs it
   int slot = 0, turn = 0;
-  for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x, turn ^= 1) {
+  auto multiply = [&](int tile, bool first) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
@@ -157,9 +154,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const float* __
       request(slot);
       slot = slot + 1 == PF ? 0 : slot + 1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][j], a[4 * c + i][j], acc, 0, 0, 0);
+      for (int i = 0; i < 2; ++i) {
+        if (first) as[2 * c + i] = split8<true>(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
+        acc += split_block(split8<false>(w[2 * i], w[2 * i + 1]), as[2 * c + i]);
+      }
     }
     // a lane holds columns 4 kb .. + 3 of row r: of the products, the two squares on the diagonal are used
     auto* to = part[turn];
@@ -170,6 +168,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const float* __
       const int m = lane / 8, nn = lane % 8, n = GLU ? 4 * tile + nn % 4 : 8 * tile + nn;
       float total = 0.f;
       for (int s = 0; s < segs; ++s) total += to[s][lane];
+      if (split_bad(total) && m < M && n < n_out) {
+        float rstd = 1.f;
+        if (NORM) {
+          float all = 0.f;
+#pragma unroll
+          for (int i = 0; i < WAVES / 2; ++i) all += sq[m][i];
+          rstd = 1.0f / sqrtf(all / (float)K + nm.eps);
+        }
+        const float* row = A + (size_t)m * lda;
+        total = split_again([&](int k) { return NORM ? row[k] * rstd * nm.w[k] : row[k]; },
+                            W + (size_t)(n + (GLU && nn >= 4 ? n_out : 0)) * ldw, K);
+      }
       if (bias && n < n_out) total += bias[n + (GLU && nn >= 4 ? n_out : 0)];
       if (GLU) {
         const float up = __shfl_xor(total, 4, TA_WAVE);
@@ -179,7 +189,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_kernel(const float* __
         *c = add ? *c + total : total;
       }
     }
-  }
+    turn ^= 1;
+  };
+  multiply(blockIdx.x, true);                    // (no more workgroups than tiles)
+  for (int tile = blockIdx.x + gridDim.x; tile < tiles; tile += gridDim.x) multiply(tile, false);
   ta_wait_loads<0>();                            // no wave ends with a load to LDS on its way
 }
 
@@ -256,9 +269,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
       request(slot);
       slot = slot + 1 == PF ? 0 : slot + 1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][j], a[i][j], acc, 0, 0, 0);
+      for (int i = 0; i < 4; i += 2) acc += split_block(split8<false>(w[i], w[i + 1]), split8<true>(a[i], a[i + 1]));
     }
     auto* to = part[round & 1];
     if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[2 * wave + r / 8][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
@@ -269,6 +280,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
     }
   }
   if (wave == 0 && m < M && n < N) {
+    if (split_bad(total)) total = split_again([&](int k) { return A[(size_t)m * lda + k]; }, W + (size_t)n * ldw, K);
     if (bias) total += bias[n];
     float* c = C + (size_t)m * ldc + n;
     *c = add ? *c + total : total;

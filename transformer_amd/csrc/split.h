@@ -1,0 +1,78 @@
+// Products of 32-bit numbers on the 16-bit matrix instructions. A float32 x is the sum of three bfloat16, x = h + m + l, exactly
+// (24 bits in three times 8), and of the nine products of two such sums the six that matter are multiplied:
+// h h, h m, m h, m m, h l, l h; what is left out is 2^-24 of a product at the most, of either sign, and 2^-28 in the mean. v_mfma_f32_16x16x32_bf16 multiplies exactly and
+// takes denormals: 32 k of all six occupy a SIMD for 96 cycles where the float32 instructions need 256.
+//
+// The order of the sums, the same in every kernel that uses this, whatever M, N, the kernel or the tile:
+//   k is cut into segments of 256 and these into blocks of 32; a block's six products are a chain of instructions from zero, the
+//   small ones first; the blocks' results are added in float32 in ascending order, and so are the segments'. Inside an
+//   instruction lane (r, kb) holds k = 4 kb .. + 3 and 16 + 4 kb .. + 3 of the block: what a lane has that reads 16 bytes at a time.
+// So a row of A gives the same bits alone or inside any batch. Segments let few rows be split over waves; they also round less.
+// Against 64 bits (rms of the difference over rms of the result; normal entries, k = 2,048 / 8,192) 1.0e-7 / 1.6e-7, where chains of
+// fused multiply-adds over segments of 256 give 2.9e-7 / 3.1e-7; positive entries 4.9e-8 / 7.8e-8 and 9.0e-8 / 8.7e-8; entries
+// spread over e^(2 normal) 1.0e-7 / 1.5e-7 and 2.9e-7 / 3.3e-7.
+//
+// An operand that is infinite, undefined or rounds to an infinite bfloat16, and a sum that overflows on the way, give a result that
+// is not finite here, never a wrong finite one; such a result is formed once more by split_again, in fused multiply-adds.
+#pragma once
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+#define SEG 256      // k per segment
+#define BLK 16       // k that a row's four lanes read at once; two of them are a block
+
+struct Split8 {
+  bf16x8 h, m, l;
+};
+
+// A lane's 8 numbers of a block: x its k = 4 kb .. + 3, y its 16 + 4 kb .. + 3. h is a row's (ROUND) number to the nearest (half away from
+// zero) or a column's cut off after 8 bits, m what is left cut off again, l the rest, which fits. One operand is enough to round: what is
+// left out of a product is then of either sign. Plain instructions, 5.5 a number: v_cvt_pk_bf16_f32 takes as long as three of them, and
+// v_dot2_f32_bf16, which takes h away in one, holds up the matrix instructions (a tile of 256 x 128 over k = 8,192 590 us with it, 500 so).
+template <bool ROUND>
+__device__ __forceinline__ Split8 split8(const f32x4& x, const f32x4& y) {
+#pragma clang fp contract(off)   // x and y may be products, which are rounded before they are split
+  Split8 s;
+  uint32_t *h = reinterpret_cast<uint32_t*>(&s.h), *m = reinterpret_cast<uint32_t*>(&s.m), *l = reinterpret_cast<uint32_t*>(&s.l);
+  auto rest = [](float v, uint32_t near) { return v - __uint_as_float(near & 0xffff0000u); };
+  auto tops = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = i < 2 ? x[2 * i] : y[2 * i - 4], b = i < 2 ? x[2 * i + 1] : y[2 * i - 3];
+    const uint32_t na = __float_as_uint(a) + (ROUND ? 0x8000u : 0u), nb = __float_as_uint(b) + (ROUND ? 0x8000u : 0u);
+    const float ra = rest(a, na), rb = rest(b, nb);
+    const uint32_t ma = __float_as_uint(ra), mb = __float_as_uint(rb);
+    h[i] = tops(na, nb);
+    m[i] = tops(ma, mb);
+    l[i] = tops(__float_as_uint(rest(ra, ma)), __float_as_uint(rest(rb, mb)));
+  }
+  return s;
+}
+
+// step i (0 .. 5) of a block's chain
+__device__ __forceinline__ f32x4 split_mul(int i, const Split8& w, const Split8& a, const f32x4& c) {
+  const bf16x8& x = i == 0 ? w.l : i == 2 || i == 3 ? w.m : w.h;
+  const bf16x8& y = i == 1 ? a.l : i == 2 || i == 4 ? a.m : a.h;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+}
+
+// a block's product: element e of lane (r, kb) is column 4 kb + e (w's row) of row r (a's)
+__device__ __forceinline__ f32x4 split_block(const Split8& w, const Split8& a) {
+  f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 6; ++i) c = split_mul(i, w, a, c);
+  return c;
+}
+
+__device__ __forceinline__ bool split_bad(float x) { return !(fabsf(x) <= 3.402823466e38f); }
+
+// the sum over k of a(k) w[k], k ascending
+template <typename F>
+__device__ __forceinline__ float split_again(F a, const float* w, int K) {
+  float s = 0.f;
+#pragma unroll 1
+  for (int k = 0; k < K; ++k) s = fmaf(a(k), w[k], s);
+  return s;
+}

@@ -1,9 +1,9 @@
 """y = x @ W^T, the matrix product every part uses.
 
-float32 engine: the hand-written product of csrc/gemm_simple.hip, whose every
-output element is summed by fused multiply-adds in one order that depends on k
-alone; no library and no reduced-precision matrix mode is involved anywhere in
-that path.
+float32 engine: the hand-written products of csrc/gemm_simple.hip, gemm_stream.hip
+and gemm_split.hip, whose every output element is summed in one order that depends
+on k alone. All 24 bits of both operands are multiplied (csrc/split.h); no library
+and no reduced-precision matrix mode is involved anywhere in that path.
 
 bfloat16 engine: the vendor library through ``torch.mm`` (the reference's
 engine also hands its products to a library: the external ``mat_mul`` operator,
