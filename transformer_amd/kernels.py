@@ -883,6 +883,35 @@ def gemm_mid(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, swiglu: bool =
     return out
 
 
+def gemm_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, activation: str = "silu", bias: Optional[torch.Tensor] = None,
+             limits: Optional[Sequence[float]] = None) -> torch.Tensor:
+    """out [m, n] = act(a @ w[:n].T + bias[:n]) * (a @ w[n:].T + bias[n:]) in bfloat16, any number of rows: the product and the
+    activation in one kernel, gates and ups joined in float32. activation "silu" or "gelu_tanh"; limits as in ``gemm_skinny``."""
+    _dev(a, "a", torch.bfloat16, contiguous=False); _dev(w, "w", torch.bfloat16, contiguous=False)
+    _dev(out, "out", torch.bfloat16, contiguous=False)
+    if activation not in _GLU_ACTS or (limits is not None and (activation != "silu" or not limits[0] > 0)):
+        raise KernelError(f"gemm_glu: activation {activation!r}, limits {limits}")
+    M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
+    if N % 2 or w.shape[1] != a.shape[1] or Mo != M or out.shape[1] != N // 2:
+        raise KernelError(f"gemm_glu: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    if bias is not None:
+        _dev(bias, "bias", torch.float32)
+        if bias.numel() != N:
+            raise KernelError("gemm_glu: bias must hold one entry per row of w")
+    _check(library().ta_gemm_glu(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(bias), _ptr(out), c_int(ldc), c_int(M),
+                                 c_int(N // 2), c_int(a.shape[1]), c_int(_GLU_ACTS[activation]),
+                                 *[c_float(v) for v in (limits or (0.0, 0.0, 0.0))]))
+    return out
+
+
+def glu_pays(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_glu`` is better than the vendor library's product and the activation's kernel: many rows against a wide weight."""
+    return a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and w.dim() == 2 and w.shape[0] % 2 == 0 \
+        and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 \
+        and max(a.stride(0), w.stride(0)) <= 4194304 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+        and bool(library().ta_gemm_glu_pays(c_int(a.shape[0]), c_int(w.shape[0] // 2), c_int(a.shape[1])))
+
+
 def mid_takes(rows: int, w: torch.Tensor) -> bool:
     """Shapes for which ``gemm_mid`` is used instead of the vendor library: more rows than the
     few-rows product takes (or a k too long for it), at most 64."""

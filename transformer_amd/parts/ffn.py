@@ -64,6 +64,9 @@ class SwiGLU(Part):
         elif self.limits is None and kernels.simple_glu_takes(h, self.w["gate_up.weight"]):
             # few float32 rows: the product applies the activation itself, with the same bits
             kernels.gemm_simple_glu(h, self.w["gate_up.weight"], act, self.w.get("gate_up.bias"))
+        elif kernels.glu_pays(h, self.w["gate_up.weight"]):
+            # many bfloat16 rows: likewise, gates and ups joined before they are rounded
+            kernels.gemm_glu(h, self.w["gate_up.weight"], act, bias=self.w.get("gate_up.bias"), limits=self.limits)
         else:
             gu = linear(h, self.w["gate_up.weight"],
                         ctx.ws.take("swiglu.gate_up", (nt, 2 * s.intermediate), self.dtype))
@@ -108,6 +111,8 @@ class GLU(SwiGLU):
         act = ctx.ws.take("swiglu.act", (nt, s.intermediate), self.dtype)
         if not s.bias and kernels.skinny_wins(h, self.w["gate_up.weight"]):
             kernels.gemm_skinny_act(h, self.w["gate_up.weight"], act, self.activation, glu=True)
+        elif kernels.glu_pays(h, self.w["gate_up.weight"]):
+            kernels.gemm_glu(h, self.w["gate_up.weight"], act, self.activation, self.w.get("gate_up.bias"))
         else:
             gu = linear(h, self.w["gate_up.weight"],
                         ctx.ws.take("swiglu.gate_up", (nt, 2 * s.intermediate), self.dtype))
