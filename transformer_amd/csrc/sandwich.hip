@@ -7,6 +7,8 @@
 //                      out = rms_norm(x) * w_next, so that a row is read and written once
 //   stream_add       : x += delta (+ a row), with a copy of the new rows in the engine's type: where
 //                      something reads the stream itself before its next norm
+//   side_step        : postnorm_add of a sublayer's result (or of routed experts' rows), then the token side input and its
+//                      postnorm_add, for a step of few tokens in one kernel
 //   activation       : out = act(in) (* rows of a float32 side table), act one of gelu (erf),
 //                      gelu (tanh), relu squared, silu
 //
@@ -420,4 +422,226 @@ extern "C" int ta_weighted_sum(hipStream_t stream, int n, const float* const* de
   const unsigned blocks = (unsigned)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
   weighted_sum_kernel<<<blocks, 256, 0, stream>>>(br, n, out, total);
   return ta_check_launch("ta_weighted_sum");
+}
+
+// The end of a block with a token side input, for a step of few tokens:
+//   x += rms_norm(delta) * w;  g = gelu_tanh(G x) * side;  x += rms_norm(P g) * v;  out = rms_norm(x) * w_next
+// delta: planes of rows, or what moe_combine would form of the experts' rows. One workgroup a token; what the kernels in turn round (x and g
+// for their products) is rounded here too. Five kernels of 3.0 to 4.6 us, most of which is their launch and their trips to memory (17.6 us in a
+// recorded chain at 4 tokens of width 2,048 with 64 side columns, 25 at 64 tokens), here 13.7 (13.0). Bound by what one CU takes in: 256 KB of G, asked
+// for at the start, and 256 KB of P, 5 us either (timestamps; eight workgroups an XCD that bring both into its L2 change nothing), sums over the
+// workgroup 1.5.
+struct SideStep {
+  float* x;
+  int d;
+  const float *delta, *w;        // [planes, nt, d]; [d]
+  int planes;
+  size_t plane;
+  float eps;
+  const float* rows;             // experts' rows [.., d] (delta null), a token's `top` of them and their weights or null
+  int top;
+  const int* pair_row;
+  const float *weight, *shared, *shared_gate;        // shared [planes, nt, d] or null, times sigmoid(shared_gate) or one
+  int gate_ld;
+  const bf16_t* G;               // [DIM, d]
+  const float* side;             // [nt, DIM], side_ld apart
+  int side_ld;
+  const bf16_t* P;               // [d, DIM]
+  const float* v;
+  float eps_side;
+  const float* w_next;
+  float eps_next;
+  bf16_t* out;
+};
+
+__device__ __forceinline__ float side_dot8(const uint4& a, const uint4& b, float c) {
+  typedef __bf16 pair __attribute__((ext_vector_type(2)));
+  c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair, a.x), __builtin_bit_cast(pair, b.x), c, false);
+  c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair, a.y), __builtin_bit_cast(pair, b.y), c, false);
+  c = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair, a.z), __builtin_bit_cast(pair, b.z), c, false);
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(pair, a.w), __builtin_bit_cast(pair, b.w), c, false);
+}
+
+// over 1,024 threads; `red` is not another sum's
+__device__ __forceinline__ float side_sum(float v, float* red) {
+  float none = 0.f;
+  ta_sums2<64>(v, none);
+  if (threadIdx.x % TA_WAVE == 0) red[threadIdx.x / TA_WAVE] = v;
+  __syncthreads();
+  return ta_sum16(red[threadIdx.x % 16]);
+}
+
+#define SIDE_MAX_D 4096
+template <int DIM>
+__global__ __launch_bounds__(1024) void side_step_kernel(SideStep p) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int OWN = DIM / 16, AHEAD = 16 / OWN;      // rows of G a wave; pieces of each that are on their way
+  constexpr int LANES = DIM / 8, ROWS = TA_WAVE / LANES, PASS = 16;   // lanes a row of P, rows a wave and load, loads on their way
+  constexpr int COLS = SIDE_MAX_D / 2048;              // pairs of columns a thread
+  __shared__ float red[3][16];
+  __shared__ __attribute__((aligned(16))) bf16_t xrow[SIDE_MAX_D];
+  __shared__ __attribute__((aligned(16))) bf16_t gate[DIM];
+  __shared__ __attribute__((aligned(16))) float y[SIDE_MAX_D];
+  const int tid = threadIdx.x, lane = tid % TA_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / TA_WAVE), d = p.d;
+  const size_t t = blockIdx.x, base = t * d;
+  const int pieces = d / 512;                          // of 8 numbers a lane in a row of G
+  u32x4 gw[OWN][AHEAD];
+  auto load_gate = [&](int i0) {
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i)
+        gw[o][i] = *reinterpret_cast<const u32x4*>(p.G + (size_t)(wave * OWN + o) * d + 8 * (lane + 64 * (i0 + i < pieces ? i0 + i : i0)));
+  };
+  load_gate(0);
+  // the sublayer's row, columns 2 (tid + 1024 i)
+  float2 s[COLS], xv[COLS];
+  float ss = 0.f;
+  const float sg = p.shared && p.shared_gate ? 1.0f / (1.0f + expf(-p.shared_gate[t * p.gate_ld])) : 1.f;
+#pragma unroll
+  for (int i = 0; i < COLS; ++i) {
+    const int c = 2 * (tid + 1024 * i);
+    s[i] = xv[i] = float2{0.f, 0.f};
+    if (c >= d) continue;
+    xv[i] = *reinterpret_cast<const float2*>(p.x + base + c);
+    if (p.rows) {
+      for (int j0 = 0; j0 < p.top; j0 += 4) {
+        float2 e[4];
+        float f[4];
+        int r[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const size_t pair = t * p.top + (j0 + j < p.top ? j0 + j : j0);
+          r[j] = p.pair_row[pair];
+          f[j] = p.weight ? p.weight[pair] : 1.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = *reinterpret_cast<const float2*>(p.rows + (size_t)(r[j] >= 0 ? r[j] : 0) * d + c);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j0 + j < p.top && r[j] >= 0) s[i] = float2{fmaf(e[j].x, f[j], s[i].x), fmaf(e[j].y, f[j], s[i].y)};
+      }
+    }
+    const float* from = p.rows ? p.shared : p.delta;
+    if (from) {
+      float2 a = *reinterpret_cast<const float2*>(from + base + c);
+      for (int q = 1; q < p.planes; ++q) {
+        const float2 b = *reinterpret_cast<const float2*>(from + base + c + q * p.plane);
+        a.x += b.x;
+        a.y += b.y;
+      }
+      s[i] = p.rows ? float2{fmaf(sg, a.x, s[i].x), fmaf(sg, a.y, s[i].y)} : a;
+    }
+    ss += s[i].x * s[i].x + s[i].y * s[i].y;
+  }
+  const float f = rsqrtf(side_sum(ss, red[0]) / (float)d + p.eps);
+#pragma unroll
+  for (int i = 0; i < COLS; ++i) {
+    const int c = 2 * (tid + 1024 * i);
+    if (c >= d) continue;
+    const float2 wv = *reinterpret_cast<const float2*>(p.w + c);
+    xv[i].x += s[i].x * f * wv.x;
+    xv[i].y += s[i].y * f * wv.y;
+    *reinterpret_cast<uint32_t*>(&xrow[c]) = f32x2_to_bf16x2_bits(xv[i].x, xv[i].y);
+  }
+  __syncthreads();
+  float sum[OWN];
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) sum[o] = 0.f;
+  for (int i0 = 0; i0 < pieces; i0 += AHEAD) {
+    if (i0 > 0) load_gate(i0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      if (i0 + i >= pieces) break;
+      const uint4 xp = *reinterpret_cast<const uint4*>(&xrow[8 * (lane + 64 * (i0 + i))]);
+#pragma unroll
+      for (int o = 0; o < OWN; ++o) sum[o] = side_dot8(__builtin_bit_cast(uint4, gw[o][i]), xp, sum[o]);
+    }
+  }
+  // rows of P: pass q brings 16 ROWS of them
+  const int passes = d / (16 * ROWS);
+  u32x4 pw[PASS];
+  auto load_proj = [&](int q0) {
+#pragma unroll
+    for (int q = 0; q < PASS; ++q)
+      pw[q] = *reinterpret_cast<const u32x4*>(p.P + (size_t)(((q0 + q < passes ? q0 + q : q0) * 16 + wave) * ROWS + lane / LANES) * DIM + 8 * (lane % LANES));
+  };
+  load_proj(0);
+#pragma unroll
+  for (int o = 0; o < OWN; o += 2) ta_sums2<64>(sum[o], sum[o + 1]);
+#pragma unroll
+  for (int o = 0; o < OWN; ++o)
+    if (lane == o) gate[wave * OWN + o] = from_f32<bf16_t>(ta_act(1, sum[o]) * p.side[t * p.side_ld + wave * OWN + o]);
+  __syncthreads();
+  const uint4 gp = *reinterpret_cast<const uint4*>(&gate[8 * (lane % LANES)]);
+  for (int q0 = 0; q0 < passes; q0 += PASS) {
+    if (q0 > 0) load_proj(q0);
+#pragma unroll
+    for (int q = 0; q < PASS; ++q) {
+      if (q0 + q >= passes) break;
+      float a = side_dot8(__builtin_bit_cast(uint4, pw[q]), gp, 0.f);
+      a += ta_dpp<0xB1>(a);
+      a += ta_dpp<0x4E>(a);
+      if (LANES >= 8) a += ta_dpp<0x141>(a);
+      if (LANES >= 16) a += ta_dpp<0x140>(a);
+      if (lane % LANES == 0) y[((q0 + q) * 16 + wave) * ROWS + lane / LANES] = a;
+    }
+  }
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < COLS; ++i) {
+    const int c = 2 * (tid + 1024 * i);
+    s[i] = c < d ? *reinterpret_cast<const float2*>(&y[c]) : float2{0.f, 0.f};
+    ss += s[i].x * s[i].x + s[i].y * s[i].y;
+  }
+  const float f1 = rsqrtf(side_sum(ss, red[1]) / (float)d + p.eps_side);
+  float s2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < COLS; ++i) {
+    const int c = 2 * (tid + 1024 * i);
+    if (c >= d) continue;
+    const float2 wv = *reinterpret_cast<const float2*>(p.v + c);
+    xv[i].x += s[i].x * f1 * wv.x;
+    xv[i].y += s[i].y * f1 * wv.y;
+    *reinterpret_cast<float2*>(p.x + base + c) = xv[i];
+    s2 += xv[i].x * xv[i].x + xv[i].y * xv[i].y;
+  }
+  if (!p.out) return;
+  const float f2 = rsqrtf(side_sum(s2, red[2]) / (float)d + p.eps_next);
+#pragma unroll
+  for (int i = 0; i < COLS; ++i) {
+    const int c = 2 * (tid + 1024 * i);
+    if (c >= d) continue;
+    const float2 wv = *reinterpret_cast<const float2*>(p.w_next + c);
+    *reinterpret_cast<uint32_t*>(p.out + base + c) = f32x2_to_bf16x2_bits(xv[i].x * f2 * wv.x, xv[i].y * f2 * wv.y);
+  }
+}
+
+// Whether ta_side_step takes a step: one by one and here 17.5 / 15.8 us at one token, 17.6 / 13.7 at 4, 18.4 / 13.6 at 16, 26.8 / 13.5 at 32, 25.3 / 13.0 at 64;
+// beyond, every token's workgroup reads both matrices again, and a prompt's products share them.
+extern "C" int ta_side_step_pays(int nt, int d, int dim) {
+  return nt >= 1 && nt <= 64 && d % 512 == 0 && d <= SIDE_MAX_D && (dim == 32 || dim == 64 || dim == 128);
+}
+
+// delta [planes, nt, d], or null and rows / top / pair_row / weight / shared [planes, nt, d] / shared_gate as in ta_moe_combine.
+extern "C" int ta_side_step(hipStream_t stream, float* x, const float* delta, int planes, long long plane, const float* w, float eps,
+                            const float* rows, int top, const int* pair_row, const float* weight, const float* shared,
+                            const float* shared_gate, int gate_ld, const void* G, const float* side, int side_ld, const void* P,
+                            int dim, const float* v, float eps_side, const float* w_next, float eps_next, void* out, int nt, int d) {
+  TA_REQUIRE(nt >= 0 && d > 0 && d % 512 == 0 && d <= SIDE_MAX_D && (dim == 32 || dim == 64 || dim == 128),
+             "ta_side_step: nt=%d d=%d, %d side columns", nt, d, dim);
+  TA_REQUIRE((delta == nullptr) != (rows == nullptr) && (!rows || (top >= 1 && pair_row)) && planes >= 1 && planes <= TA_MAX_PLANES &&
+                 plane % 2 == 0, "ta_side_step: a result or experts' rows, %d planes", planes);
+  TA_REQUIRE((out == nullptr) == (w_next == nullptr), "ta_side_step: w_next and out go together");
+  TA_REQUIRE(((uintptr_t)G | (uintptr_t)P) % 16 == 0 &&
+                 ((uintptr_t)x | (uintptr_t)delta | (uintptr_t)w | (uintptr_t)rows | (uintptr_t)shared | (uintptr_t)v | (uintptr_t)w_next) % 8 == 0 &&
+                 (uintptr_t)out % 4 == 0, "ta_side_step: operands off their pieces");
+  if (nt == 0) return 0;
+  const SideStep p = {x, d, delta, w, planes, (size_t)plane, eps, rows, top, pair_row, weight, shared, shared_gate, gate_ld, (const bf16_t*)G,
+                      side, side_ld, (const bf16_t*)P, v, eps_side, w_next, eps_next, (bf16_t*)out};
+  if (dim == 32) side_step_kernel<32><<<nt, 1024, 0, stream>>>(p);
+  else if (dim == 64) side_step_kernel<64><<<nt, 1024, 0, stream>>>(p);
+  else side_step_kernel<128><<<nt, 1024, 0, stream>>>(p);
+  return ta_check_launch("ta_side_step");
 }

@@ -2200,6 +2200,71 @@ def moe_combine(rows: torch.Tensor, top: int, pair_row: torch.Tensor, weight, sh
     return delta
 
 
+class RoutedRows:
+    """What ``moe_combine`` would make a sublayer's result of (its arguments); a kernel that reads the result may form it itself."""
+
+    def __init__(self, rows, top, pair_row, weight, shared, shared_gate):
+        self.rows, self.top, self.pair_row, self.weight, self.shared, self.shared_gate = rows, int(top), pair_row, weight, shared, shared_gate
+
+
+def side_step_takes(rows: int, d: int, gate: torch.Tensor, proj: torch.Tensor) -> bool:
+    """Whether ``side_step`` takes a step of ``rows`` tokens of width d with these matrices."""
+    return gate.dtype == torch.bfloat16 and proj.dtype == torch.bfloat16 and gate.is_contiguous() and proj.is_contiguous() \
+        and gate.data_ptr() % 16 == 0 and proj.data_ptr() % 16 == 0 \
+        and bool(library().ta_side_step_pays(c_int(rows), c_int(d), c_int(gate.shape[0])))
+
+
+def side_step(x: torch.Tensor, delta, weight: torch.Tensor, eps: float, gate: torch.Tensor, side: torch.Tensor, proj: torch.Tensor,
+              side_weight: torch.Tensor, side_eps: float, next_weight: Optional[torch.Tensor] = None, next_eps: float = 0.0,
+              out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``postnorm_add(x, delta, weight, eps)``, then x += rms_norm((gelu_tanh(x @ gate.T) * side) @ proj.T, side_eps) * side_weight and
+    ``out``, the stream's next norm, in one kernel: bfloat16 matrices, few tokens. delta as in ``postnorm_add``, or a ``RoutedRows``.
+    x and the gated side columns are rounded to bfloat16 in front of their products, as in the kernels one by one."""
+    _dev(x, "x", torch.float32); _dev(weight, "weight", torch.float32); _dev(side_weight, "side_weight", torch.float32)
+    _dev(gate, "gate", torch.bfloat16); _dev(proj, "proj", torch.bfloat16); _dev(side, "side", torch.float32, contiguous=False)
+    nt, d = x.shape
+    dim = gate.shape[0]
+    _, side_ld = _rows2d(side, "side")
+    if gate.shape != (dim, d) or proj.shape != (d, dim) or side.shape != (nt, dim) or weight.shape != (d,) or side_weight.shape != (d,):
+        raise KernelError(f"side_step: x {tuple(x.shape)} gate {tuple(gate.shape)} proj {tuple(proj.shape)} side {tuple(side.shape)}")
+    if (out is None) != (next_weight is None):
+        raise KernelError("side_step: next_weight and out go together")
+    if out is not None:
+        _dev(out, "out", torch.bfloat16); _dev(next_weight, "next_weight", torch.float32)
+        if out.shape != x.shape or next_weight.shape != (d,):
+            raise KernelError(f"side_step: out {tuple(out.shape)} next_weight {tuple(next_weight.shape)}")
+    routed = delta if isinstance(delta, RoutedRows) else None
+    planes, plane, gate_ld, rows, top, pair_row, pair_weight, shared, shared_gate = 1, 0, 0, None, 0, None, None, None, None
+    if routed is not None:
+        rows, top, pair_row, pair_weight, shared, shared_gate = (routed.rows, routed.top, routed.pair_row, routed.weight, routed.shared,
+                                                                 routed.shared_gate)
+        _dev(rows, "rows", torch.float32); _dev(pair_row, "pair_row", torch.int32)
+        if rows.shape[1] != d or pair_row.numel() != nt * top:
+            raise KernelError(f"side_step: rows {tuple(rows.shape)} for {nt} tokens x {top}")
+        if pair_weight is not None:
+            _dev(pair_weight, "weight", torch.float32)
+            if pair_weight.numel() != nt * top:
+                raise KernelError(f"side_step: {pair_weight.numel()} weights for {nt} tokens x {top}")
+        if shared_gate is not None:
+            _dev(shared_gate, "shared_gate", torch.float32, contiguous=False)
+            ng, gate_ld = _rows2d(shared_gate, "shared_gate")
+            if ng != nt:
+                raise KernelError(f"side_step: shared_gate is {tuple(shared_gate.shape)}")
+    added = delta if routed is None else shared
+    if added is not None:
+        _dev(added, "delta", torch.float32)
+        if added.dim() == 3 and added.shape[1:] == x.shape:
+            planes, plane = added.shape[0], nt * d
+        elif added.shape != x.shape:
+            raise KernelError(f"side_step: {tuple(added.shape)} for x {tuple(x.shape)}")
+    _check(library().ta_side_step(
+        _stream(), _ptr(x), _ptr(None if routed is not None else delta), c_int(planes), c_longlong(plane), _ptr(weight), c_float(eps),
+        _ptr(rows), c_int(top), _ptr(pair_row), _ptr(pair_weight), _ptr(shared), _ptr(shared_gate), c_int(gate_ld), _ptr(gate), _ptr(side),
+        c_int(side_ld), _ptr(proj), c_int(dim), _ptr(side_weight), c_float(side_eps), _ptr(next_weight), c_float(next_eps), _ptr(out),
+        c_int(nt), c_int(d)))
+    return x
+
+
 # ------------------------------------------------------------------ capped, sunk and gated softmax attention
 _ROT_STYLES = {"half": 0, "interleaved": 1}
 

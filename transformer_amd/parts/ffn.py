@@ -225,7 +225,9 @@ class RoutedMLP(Part):
         return kernels.glu_limit(pre, ws.take(name, (rows, n), self.dtype), float(act_limit),
                                  float(s.gate_slope), float(s.up_shift))
 
-    def run(self, h, ctx, extra=None):
+    def run(self, h, ctx, extra=None, combine=True):
+        """(delta, None); without ``combine``, where no expert is the input itself, the rows that make up the delta
+        (``kernels.RoutedRows``) in its place."""
         s, nt, d = self.spec, h.shape[0], self.spec.hidden
         E, top, ff = s.experts, s.top, s.intermediate
         ws = ctx.ws
@@ -262,6 +264,9 @@ class RoutedMLP(Part):
             u = self._first(h, self.w[f"shared.{first}.weight"], None, ws, "moe.shared_up", s.shared_intermediate,
                             getattr(s, "shared_limit", 0.0))
             shared = linear_delta(u, self.w["shared.down.weight"], ws, "moe.shared")
+        if not combine and extra is None and not self.identity:
+            return kernels.RoutedRows(out, top, pair_row, None if on_input else weight, shared,
+                                      logits[:, R:] if self.gated_shared else None), None
         delta = kernels.moe_combine(out, top, pair_row, None if on_input else weight, shared,
                                     logits[:, R:] if self.gated_shared else None,
                                     ws.take("moe.delta", (nt, d), torch.float32), extra=extra,

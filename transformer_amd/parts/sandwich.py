@@ -17,6 +17,7 @@ from .. import kernels
 from ..weights.loader import Param
 from .base import Part, PartError, build_part, register_part, span
 from .embedding import TokenSideTable
+from .ffn import RoutedMLP
 from .linear import activated, linear, linear_delta
 
 
@@ -34,16 +35,32 @@ class TokenSide(Part):
                 "proj.weight": Param((s.hidden, s.dim), "matrix"),
                 "norm.weight": Param((s.hidden,), "vector", init="around_one")}
 
-    def run(self, x, xcast, ctx, next_norm=None, out=None):
-        """x: the float32 stream, updated in place; xcast: the same rows in the engine's type.
-        next_norm / out: the norm that reads the stream next and where its rows go."""
-        s, nt = self.spec, x.shape[0]
+    def _columns(self, ctx):
+        """This block's own columns of the step's side-table rows."""
+        s = self.spec
         rows = ctx.shared.get(TokenSideTable.KEY)
         if rows is None or rows.shape[1] < s.offset + s.dim:
             raise PartError("the token side input needs the step's side-table rows "
                             f"(columns {s.offset}..{s.offset + s.dim})")
+        return rows[:, s.offset:s.offset + s.dim]
+
+    def takes_step(self, x) -> bool:
+        """Whether ``run_step`` takes this step: few bfloat16 tokens."""
+        return self.dtype == torch.bfloat16 and \
+            kernels.side_step_takes(x.shape[0], x.shape[1], self.w["gate.weight"], self.w["proj.weight"])
+
+    def run_step(self, x, delta, weight, eps, ctx, next_norm=None, out=None):
+        """The add in front (a sublayer's result normed with this weight and eps) and ``run`` in one kernel."""
+        kernels.side_step(x, delta, weight, eps, self.w["gate.weight"], self._columns(ctx), self.w["proj.weight"],
+                          self.w["norm.weight"], float(self.spec.eps), None if next_norm is None else next_norm.gain(),
+                          0.0 if next_norm is None else next_norm.eps, out)
+
+    def run(self, x, xcast, ctx, next_norm=None, out=None):
+        """x: the float32 stream, updated in place; xcast: the same rows in the engine's type.
+        next_norm / out: the norm that reads the stream next and where its rows go."""
+        s, nt = self.spec, x.shape[0]
         g = activated(xcast, self.w["gate.weight"], ctx.ws.take("side.gate", (nt, s.dim), self.dtype), "gelu_tanh",
-                      side=rows[:, s.offset:s.offset + s.dim])
+                      side=self._columns(ctx))
         y = linear(g, self.w["proj.weight"], ctx.ws.take("side.y", (nt, s.hidden), torch.float32))
         kernels.postnorm_add(x, y, self.w["norm.weight"], float(s.eps),
                              next_weight=None if next_norm is None else next_norm.gain(),
@@ -144,10 +161,17 @@ class SandwichBlock(Part):
             add("1", delta, follow if last == "mixer" else None, True)
         else:
             add("1", delta, self.norm2, False)
+            step = self.side is not None and self.side.takes_step(x)
             with span(ctx, "ffn"):
-                delta, bias = self.ffn.run(h, ctx)
+                kw = {"combine": False} if step and isinstance(self.ffn, RoutedMLP) else {}
+                delta, bias = self.ffn.run(h, ctx, **kw)
             if bias is not None:
                 raise PartError("a sandwich block's sublayers return no bias rows")
+            if step:                                  # the add, the side input and its own add in one kernel
+                with span(ctx, "side"):
+                    self.side.run_step(x, delta, self._post_weight("2"), float(self.norm2b.eps), ctx, next_norm=follow,
+                                       out=None if follow is None else h)
+                return "normed" if follow is not None else (None, None)
             add("2", delta, follow if last == "ffn" else None, True)
         if self.side is not None:
             with span(ctx, "side"):
