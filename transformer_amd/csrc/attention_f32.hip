@@ -14,6 +14,7 @@
 // kb < 4: scores K Q^T leave it row r's keys 16 t + 4 kb + i (t, i < 4), which is the layout in which the second
 // product V^T P^T wants the weights; both operands of either product are runs of 4 consecutive numbers of a key
 // or value row.
+#include <type_traits>
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -39,37 +40,57 @@ struct Span {
   __device__ __forceinline__ bool page(int p) const { return p * 64 < end && (p * 64 + 64 > start || p * 64 < keep); }
 };
 
-template <int NB, bool EXACT, typename KF>
+// Both products read the next operands from LDS while the present ones are multiplied (left to itself the compiler reads them right in
+// front of their use), where the widths are known (else the branches around the reads cost more registers than there are).
+template <int NB, bool EXACT, int T, typename KF>
 __device__ __forceinline__ void page_scores(const f32x4* qf, int nb, KF kfrag, f32x4* s) {
+  f32x4 k[2][T];
+  auto ask = [&](int d) __attribute__((always_inline)) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < T; ++t) k[d % 2][t] = kfrag(t, d);
+  };
+#pragma unroll
+  for (int t = 0; t < T; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (EXACT) ask(0);
 #pragma unroll
   for (int d = 0; d < NB; ++d)
     if (EXACT || d < nb) {
-      f32x4 k[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) k[t] = kfrag(t, d);
+      if (!EXACT) ask(d);
+      else if (d + 1 < NB) ask(d + 1);
+      if (EXACT) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[t][j], qf[d][j], s[t], 0, 0, 0);
+        for (int t = 0; t < T; ++t) s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[d % 2][t][j], qf[d][j], s[t], 0, 0, 0);
+      if (EXACT) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
-// scores -> weights relative to the page's maximum m, and their sum l
-__device__ __forceinline__ void page_softmax(const F32Attention& p, const Span& see, int key0, f32x4* s, float& m, float& l) {
+// scores -> weights relative to the page's maximum m, and their sum l. whole: every row of the wave sees the whole page.
+__device__ __forceinline__ void page_softmax(const F32Attention& p, const Span& see, int key0, bool whole, f32x4* s, float& m, float& l) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[t][i] *= p.scale;
+  if (p.softcap > 0.f)       // outside the loop above, or the compiler keeps a branch for every score
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[t][i] = p.softcap * tanhf(s[t][i] / p.softcap);
+  if (!whole)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[t][i] = see.key(key0 + 16 * t + i) ? s[t][i] : -INFINITY;
   m = -INFINITY;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float x = s[t][i] * p.scale;
-      if (p.softcap > 0.f) x = p.softcap * tanhf(x / p.softcap);
-      s[t][i] = see.key(key0 + 16 * t + i) ? x : -INFINITY;
-      m = fmaxf(m, s[t][i]);
-    }
-  m = fmaxf(m, __shfl_xor(m, 16, TA_WAVE));
-  m = fmaxf(m, __shfl_xor(m, 32, TA_WAVE));
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, s[t][i]);
+  const auto m16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);     // a lane's and its neighbour's
+  m = fmaxf(__uint_as_float(m16[0]), __uint_as_float(m16[1]));
+  const auto m32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = fmaxf(__uint_as_float(m32[0]), __uint_as_float(m32[1]));
   l = 0.f;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -78,29 +99,45 @@ __device__ __forceinline__ void page_softmax(const F32Attention& p, const Span& 
       s[t][i] = s[t][i] == -INFINITY ? 0.f : expf(s[t][i] - m);
       l += s[t][i];
     }
-  l += __shfl_xor(l, 16, TA_WAVE);
-  l += __shfl_xor(l, 32, TA_WAVE);
+  const auto l16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+  l = __uint_as_float(l16[0]) + __uint_as_float(l16[1]);
+  const auto l32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+  l = __uint_as_float(l32[0]) + __uint_as_float(l32[1]);
 }
 
 // o[d] = the page's sum of values, columns 16 d + 4 kb + i of row r. Keys from `live` on (of the page) were never
 // written and count as zero.
 template <int NB, bool EXACT, typename VF>
 __device__ __forceinline__ void page_values(const f32x4* e, int nb, int live, int kb, VF vfrag, f32x4* o) {
+  constexpr int G = !EXACT ? 1 : NB < 4 ? NB : 4, STEPS = 4 * NB / G;       // of G blocks of columns and 16 keys
+  auto sum = [&](auto all) __attribute__((always_inline)) {
+    f32x4 v[2][G];
+    auto ask = [&](int step) __attribute__((always_inline)) {
 #pragma unroll
-  for (int d = 0; d < NB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < G; ++i) v[step % 2][i] = vfrag(step / (NB / G), step % (NB / G) * G + i);
+    };
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+    for (int d = 0; d < NB; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (EXACT) ask(0);
 #pragma unroll
-    for (int d = 0; d < NB; ++d)
-      if (EXACT || d < nb) {
-        f32x4 v = vfrag(t, d);
-        if (live < 64) {
+    for (int step = 0; step < STEPS; ++step) {
+      const int t = step / (NB / G), d0 = step % (NB / G) * G;
+      if (!EXACT && d0 >= nb) continue;
+      if (!EXACT) ask(step);
+      else if (step + 1 < STEPS) ask(step + 1);
+      if (EXACT) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = 16 * t + 4 * kb + j < live ? v[j] : 0.f;
-        }
+      for (int j = 0; j < 4; ++j) {
+        const bool there = decltype(all)::value || 16 * t + 4 * kb + j < live;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j], e[t][j], o[d], 0, 0, 0);
+        for (int i = 0; i < G; ++i)
+          o[d0 + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(there ? v[step % 2][i][j] : 0.f, e[t][j], o[d0 + i], 0, 0, 0);
       }
+      if (EXACT) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (live >= 64) sum(std::true_type{});
+  else sum(std::false_type{});
 }
 
 // factors with which what was joined so far and a page's numbers enter the sums
@@ -129,62 +166,83 @@ __device__ __forceinline__ float gated(const F32Attention& p, float x, int head,
   return x;
 }
 
-// Prompts: 64 rows of one (sequence, kv head) a workgroup, 16 a wave; a page's keys and its values go through LDS
-// once for the four. The next page's keys are on their way during the softmax and the second product, its values
-// during the next scores; two workgroups share a CU. Bound by the matrix instructions: 256 of 32 cycles per
-// page and wave. 1,021 tokens, 16 heads of 128 over 4 kv heads: 102 us (807 on the vector ALU).
-template <int NB, bool EXACT>
+// Prompts: 64 / SPLIT rows of one (sequence, kv head) a workgroup of four waves, SPLIT waves for 16 rows: each forms the scores of its share of a page's
+// keys, takes the others' from LDS and sums its share of the columns, so every number comes about as with one wave. A page's keys and its
+// values go through LDS once for the four. The next page's keys are on their way during the softmax and the second product, its values
+// during the next scores; two workgroups share a CU. Bound by the chain of pages of the longest rows where they are few (a page is 256 matrix instructions of 32 cycles a
+// wave, and with SPLIT 1 a prompt of 1,021 tokens has one wave a SIMD, whose longest walks twice the mean), by the matrix instructions where they are many. 16 heads of 128 over 4 kv heads, us
+// before the split / with SPLIT 1, 2, 4: 256 tokens 30 / 28, 20, 16; 512 53 / 49, 35, 29; 1,021 102 / 95, 72, 88; 2,011 322 / 294, 231, 268; 3,000 535 / 487, 429, 548; 807 for 1,021 on the vector ALU.
+template <int NB, bool EXACT, int SPLIT>
 __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32Attention p) {
-  __shared__ f32x4 Ks[64 * 4 * NB], Vs[16 * NB * 16];
-  const int group = p.nh / p.nkv, b = blockIdx.z, kvh = blockIdx.y;
+  constexpr int ROWS = 64 / SPLIT, TILES = 4 / SPLIT, T = 4 / SPLIT, OWN = NB / SPLIT;
+  __shared__ f32x4 Ks[64 * 4 * NB], Vs[16 * NB * 16], scores[SPLIT > 1 ? TILES : 1][SPLIT > 1 ? 4 : 1][TA_WAVE];
+  const int group = p.nh / p.nkv, b = blockIdx.z, kvh = SPLIT > 1 ? blockIdx.x : blockIdx.y, nth = SPLIT > 1 ? blockIdx.y : blockIdx.x;
   const int q0 = p.cu_q[b], qlen = p.cu_q[b + 1] - q0, nrows = qlen * group;
-  const int blocks = (nrows + 63) / 64;
-  if ((int)blockIdx.x >= blocks) return;
-  const int row0 = (blocks - 1 - (int)blockIdx.x) * 64;            // the longest first
+  const int blocks = (nrows + ROWS - 1) / ROWS;
+  if (nth >= blocks) return;
+  // The longest first; with two workgroups a CU (SPLIT > 1) every other 256 the shortest first, so that a long and a short one meet
+  // (1,300 tokens of the shape above 156 us without, 119 so).
+  int row0 = (blocks - 1 - nth) * ROWS;
+  if (SPLIT > 1) {
+    const int turn = gridDim.x < 256 ? 256 / gridDim.x : 1, begin = b * gridDim.y;
+    auto odd = [&](int n) { return n / (2 * turn) * turn + (n % (2 * turn) > turn ? n % (2 * turn) - turn : 0); };
+    const int shorts = odd(begin + nth) - odd(begin);
+    row0 = ((begin + nth) / turn % 2 ? shorts : blocks - 1 - (nth - shorts)) * ROWS;
+  }
   const int pos0 = p.pos0[b];
   const int lane = threadIdx.x % TA_WAVE, wave = threadIdx.x / TA_WAVE, r = lane % 16, kb = lane / 16;
+  const int tile = wave / SPLIT, part = wave % SPLIT;
   const int nkb = EXACT ? NB : p.dh / 16, nvb = EXACT ? NB : p.dv / 16;
 
-  const int last = row0 + 63 < nrows - 1 ? row0 + 63 : nrows - 1;
+  const int last = row0 + ROWS - 1 < nrows - 1 ? row0 + ROWS - 1 : nrows - 1;
   const Span all = {ta_first_key(pos0 + row0 / group + 1, p.window, p.chunk), pos0 + last / group + 1, p.keep};
-  const int row = row0 + 16 * wave + r;
+  const int row = row0 + 16 * tile + r;
   const bool ok = row < nrows;
   const int qi = ok ? row / group : 0, head = kvh * group + (ok ? row % group : 0);
   Span see = {ta_first_key(pos0 + qi + 1, p.window, p.chunk), pos0 + qi + 1, p.keep};
   if (!ok) see = {0, 0, 0};
   // the wave's own rows
-  const int wfirst = row0 + 16 * wave, wlast = wfirst + 15 < nrows - 1 ? wfirst + 15 : nrows - 1;
+  const int wfirst = row0 + 16 * tile, wlast = wfirst + 15 < nrows - 1 ? wfirst + 15 : nrows - 1;
   const bool wlive = wfirst < nrows;
   const Span mine = {ta_first_key(pos0 + wfirst / group + 1, p.window, p.chunk), wlive ? pos0 + wlast / group + 1 : 0, p.keep};
+  // pages that all 16 of them see whole
+  const int whole0 = (ta_first_key(pos0 + wlast / group + 1, p.window, p.chunk) + 63) / 64;
+  const int whole1 = wfirst + 15 < nrows ? (pos0 + wfirst / group + 1) / 64 : 0;
 
-  f32x4 qf[NB], O[NB];
+  f32x4 qf[NB], O[OWN];
   const float* qrow = p.q + (size_t)(q0 + qi) * p.q_stride + (size_t)head * p.dh;
 #pragma unroll
   for (int d = 0; d < NB; ++d) {
     if (EXACT || d < nkb) qf[d] = *reinterpret_cast<const f32x4*>(qrow + 16 * d + 4 * kb);
-    O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (d < OWN) O[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   float M = -INFINITY, L = 0.f;
+  // here, or the compiler waits for them at their first use inside the loop, where that means all that is on its way
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+    if (EXACT || d < nkb) asm volatile("" : "+v"(qf[d]));
 
   // pieces of 16 bytes, permuted inside a row by the row's number
-  const int* table = p.table + (size_t)b * p.max_blocks;
+  // by the scalar unit: a load of a wave's own would be waited for together with all that the wave has asked for before it
+  const auto* table = (const __attribute__((address_space(4))) int*)(uintptr_t)(p.table + (size_t)b * p.max_blocks);
+  auto entry = [&](int page) { return (size_t)table[__builtin_amdgcn_readfirstlane(page)]; };
   const int kper = 4 * nkb, kmask = nkb % 4 == 0 ? 15 : nkb % 2 == 0 ? 7 : 3;
   auto bring_keys = [&](int page) {
-    const float* from = p.k + ((size_t)table[page] * p.nkv + kvh) * 64 * p.dh;
+    const float* from = p.k + (entry(page) * p.nkv + kvh) * 64 * p.dh;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
       if (EXACT || i < nkb) {
         const int at = i * 256 + (int)threadIdx.x, row_ = at / kper, piece = (at - row_ * kper) ^ (row_ & kmask);
-        ta_load_to_lds16(from + (size_t)row_ * p.dh + piece * 4, &Ks[i * 256 + wave * 64]);
+        ta_load_to_lds16(from, (uint32_t)(row_ * p.dh + piece * 4) * 4, &Ks[i * 256 + wave * 64]);
       }
   };
   auto bring_values = [&](int page) {
-    const float* from = p.v + ((size_t)table[page] * p.nkv + kvh) * 64 * p.dv;
+    const float* from = p.v + (entry(page) * p.nkv + kvh) * 64 * p.dv;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
       if (EXACT || i < nvb) {
         const int at = i * 256 + (int)threadIdx.x, row_ = at / 16, piece = (at % 16) ^ (row_ & 15);
-        ta_load_to_lds16(from + (size_t)row_ * 64 + piece * 4, &Vs[i * 256 + wave * 64]);
+        ta_load_to_lds16(from, (uint32_t)(row_ * 64 + piece * 4) * 4, &Vs[i * 256 + wave * 64]);
       }
   };
   auto next_page = [&](int page) {
@@ -204,21 +262,27 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
     __syncthreads();
     f32x4 s[4];
     if (use) {
-      page_scores<NB, EXACT>(qf, nkb, [&](int t, int d) {
-        return Ks[(16 * t + r) * kper + ((4 * d + kb) ^ (r & kmask))];
+      page_scores<NB, EXACT, T>(qf, nkb, [&](int t, int d) {
+        return Ks[(16 * (part * T + t) + r) * kper + ((4 * d + kb) ^ (r & kmask))];
       }, s);
+      if (SPLIT > 1)
+#pragma unroll
+        for (int t = 0; t < T; ++t) scores[tile][part * T + t][lane] = s[t];
     }
     __syncthreads();                               // everybody has done with the keys
     if (more) bring_keys(next);
+    if (SPLIT > 1 && use)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s[t] = scores[tile][t][lane];
     float m = -INFINITY, l = 0.f;
-    if (use) page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
+    if (use) page_softmax(p, see, page * 64 + 4 * kb, page >= whole0 && page < whole1, s, m, l);
     if (EXACT && more) ta_wait_loads<NB>(); else ta_wait_loads<0>();          // the values
     __syncthreads();
-    f32x4 o[NB];
+    f32x4 o[OWN];
     if (use) {
       const int live = all.end - page * 64;
-      page_values<NB, EXACT>(s, nvb, live, kb, [&](int t, int d) {
-        return Vs[(16 * d + r) * 16 + ((4 * t + kb) ^ r)];
+      page_values<OWN, EXACT>(s, (nvb - part + SPLIT - 1) / SPLIT, live, kb, [&](int t, int i) {
+        return Vs[(16 * (part + SPLIT * i) + r) * 16 + ((4 * t + kb) ^ r)];
       }, o);
     }
     __syncthreads();                               // everybody has done with the values
@@ -228,8 +292,8 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
       join(M, m, a, c);
       L = fmaf(l, c, L * a);
 #pragma unroll
-      for (int d = 0; d < NB; ++d)
-        if (EXACT || d < nvb)
+      for (int d = 0; d < OWN; ++d)
+        if (EXACT || part + SPLIT * d < nvb)
 #pragma unroll
           for (int i = 0; i < 4; ++i) O[d][i] = fmaf(o[d][i], c, O[d][i] * a);
     }
@@ -241,12 +305,13 @@ __global__ __launch_bounds__(256, EXACT ? 2 : 1) void attn_f32_rows_kernel(F32At
   const float inv = last_factor(p, M, L, head, token, rescale);
   float* orow = p.out + token * p.out_stride + (size_t)head * p.dv;
 #pragma unroll
-  for (int d = 0; d < NB; ++d)
-    if (EXACT || d < nvb) {
+  for (int d = 0; d < OWN; ++d)
+    if (EXACT || part + SPLIT * d < nvb) {
+      const int col = 16 * (part + SPLIT * d) + 4 * kb;
       f32x4 x;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = gated(p, O[d][i] * rescale * inv, head, token, 16 * d + 4 * kb + i);
-      *reinterpret_cast<f32x4*>(orow + 16 * d + 4 * kb) = x;
+      for (int i = 0; i < 4; ++i) x[i] = gated(p, O[d][i] * rescale * inv, head, token, col + i);
+      *reinterpret_cast<f32x4*>(orow + col) = x;
     }
 }
 
@@ -310,7 +375,7 @@ __global__ __launch_bounds__(256) void attn_f32_pages_kernel(F32Attention p) {
     for (int t = 0; t < 4; ++t) s[t] = scores[turn][t][lane];
     turn ^= 1;
     float m, l;
-    page_softmax(p, see, page * 64 + 4 * kb, s, m, l);
+    page_softmax(p, see, page * 64 + 4 * kb, false, s, m, l);
     page_values<OWN, EXACT>(s, (nvb - wave + 3) / 4, end - page * 64, kb, [&](int t, int i) { return vf[t][i]; }, o);
     if (!ok) continue;
     const size_t unit = ((size_t)blockIdx.y * p.heads + head - p.kv0 * group) * p.max_blocks + page;
@@ -392,13 +457,14 @@ extern "C" long long ta_attention_f32_scratch(int batch, int nh, int max_blocks,
 
 // As ta_attention_generic_sink, float32, dh and dv multiples of 16 up to 128, rows that start on 16 bytes. parts:
 // scratch of ta_attention_f32_turn_scratch floats for steps in which every sequence brings one token or none (max_qlen 1), or
-// null: the kernel for prompts then serves these too, with the same bits.
+// null: the kernel for prompts then serves these too, with the same bits. tokens: of all sequences, by which the prompts' kernel is split.
 extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride, void* out, int out_stride,
                                 const void* kcache, const void* vcache, const int* block_table, int max_blocks,
                                 const int* cu_q, const int* pos0, int batch, int max_qlen, int nh, int nkv, int dh,
                                 int dv, float scale, int window, float softcap, int sink_mode, const float* sink,
-                                const void* gate, int gate_stride, int gate_dv, int keep, int chunk, float* parts) {
-  TA_REQUIRE(batch >= 0 && max_qlen >= 0, "ta_attention_f32: bad batch=%d max_qlen=%d", batch, max_qlen);
+                                const void* gate, int gate_stride, int gate_dv, int keep, int chunk, float* parts,
+                                int tokens) {
+  TA_REQUIRE(batch >= 0 && max_qlen >= 0 && tokens >= 0, "ta_attention_f32: bad batch=%d max_qlen=%d tokens=%d", batch, max_qlen, tokens);
   TA_REQUIRE(sink_mode >= 0 && sink_mode <= 2 && (sink_mode != 2 || sink != nullptr) && softcap >= 0.f,
              "ta_attention_f32: sink mode %d, cap %f", sink_mode, softcap);
   TA_REQUIRE(gate == nullptr || (gate_dv >= 0 && gate_dv <= dv && gate_stride >= nh * (gate_dv > 0 ? gate_dv : 1)),
@@ -418,12 +484,12 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
                           sink, (const float*)gate, parts, q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window,
                           sink_mode, gate_stride, gate_dv, keep, chunk, scale, softcap, 0, 0, 0, 0};
   const int group = nh / nkv, most = dh > dv ? dh : dv;
-#define PICK(kernel, grid)                                                        \
-  do {                                                                            \
-    if (dh == 128 && dv == 128) kernel<8, true><<<grid, 256, 0, stream>>>(p);     \
-    else if (dh == 64 && dv == 64) kernel<4, true><<<grid, 256, 0, stream>>>(p);  \
-    else if (most <= 64) kernel<4, false><<<grid, 256, 0, stream>>>(p);           \
-    else kernel<8, false><<<grid, 256, 0, stream>>>(p);                           \
+#define PICK(kernel, grid, ...)                                                                \
+  do {                                                                                         \
+    if (dh == 128 && dv == 128) kernel<8, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);   \
+    else if (dh == 64 && dv == 64) kernel<4, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p); \
+    else if (most <= 64) kernel<4, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);         \
+    else kernel<8, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);                         \
   } while (0)
   if (max_qlen == 1 && parts != nullptr) {
     int kvs;
@@ -438,7 +504,16 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
         attn_f32_join_kernel<<<dim3(ks * group, bs), 128, 0, stream>>>(p);
       }
   } else {
-    PICK(attn_f32_rows_kernel, dim3((unsigned)(((long long)max_qlen * group + 63) / 64), nkv, batch));
+    // Waves for 16 rows by the blocks of 64 rows that the step has (half a block more a sequence), where SPLIT 4 keeps the CUs from idling and 2 the
+    // longest rows from walking alone. Many short sequences gain nothing: their pages are few and every workgroup brings them again. us of SPLIT 1, 2, 4, heads of 128
+    // over 4 kv heads: 2 + 34 blocks 22 / 16 / 14, 175 65 / 48 / 45, 4 x 50 to 300 tokens (190) 33 / 28 / 30, 4 x 400 (408) 63 / 58 / 67, 16 x 100 (432) 27 / 31 / 37, 8 x 300 (616) 63 / 67 / 78;
+    // 32 heads of 64 over 8: 200 29 / 23 / 26, 512 100 / 68 / 91, 1,005 265 / 242 / 300, 1,500 493 / 492 / 626.
+    const long long rows = (long long)max_qlen * group, blocks = ((long long)tokens * group + 63) / 64 * nkv + (long long)batch * nkv / 2;
+    const int most = max_qlen >= 1000 ? 1024 : max_qlen >= 256 ? 512 : 256;
+    const int split = rows > 65535 * 16 || blocks > most ? 1 : blocks <= 180 ? 4 : 2;
+    if (split == 4) PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 15) / 16), batch), 4);
+    else if (split == 2) PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 31) / 32), batch), 2);
+    else PICK(attn_f32_rows_kernel, dim3((unsigned)((rows + 63) / 64), nkv, batch), 1);
   }
 #undef PICK
   return ta_check_launch("ta_attention_f32");

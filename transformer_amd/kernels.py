@@ -270,7 +270,8 @@ def _attention_f32(q, qs, out, os_, kcache, vcache, block_table, cu_q, pos0, max
         _stream(), _ptr(q), c_int(qs), _ptr(out), c_int(os_), _ptr(kcache), _ptr(vcache), _ptr(block_table),
         c_int(block_table.shape[1]), _ptr(cu_q), _ptr(pos0), c_int(B), c_int(max_qlen), c_int(num_heads),
         c_int(num_kv_heads), c_int(key_dim), c_int(value_dim), c_float(scale), c_int(window or 0), c_float(cap),
-        c_int(mode), _ptr(sink), _ptr(gate), c_int(gs), c_int(gd), c_int(keep), c_int(chunk), _ptr(parts)))
+        c_int(mode), _ptr(sink), _ptr(gate), c_int(gs), c_int(gd), c_int(keep), c_int(chunk), _ptr(parts),
+        c_int(q.shape[0])))
     return out
 
 
