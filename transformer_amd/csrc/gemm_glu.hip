@@ -30,10 +30,12 @@ struct GluArgs {
   int lda, ldw, ldc, M, n, K;
   int tiles_m, whole, halves;    // rows of tiles; tiles of 256 rows; tiles of 128 rows behind them
   TaGlu glu;
+  float* X;                      // PLAIN: the result [M][ldc], to which the product is added where `add`
+  int add;
 };
 
-// 256 (SHORT: 128) rows from m0 on, 128 channels from n0 on
-template <bool SHORT>
+// 256 (SHORT: 128) rows from m0 on, 128 channels from n0 on. PLAIN: 256 columns, a product alone, in float32.
+template <bool SHORT, bool PLAIN>
 __device__ __forceinline__ void glu_tile(const GluArgs& p, uint16_t* S, int m0, int n0) {
   const int lane = threadIdx.x % TA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TA_WAVE), wm = wave / 4, wn = wave % 4;
   const int r = lane % 16, kb = lane / 16;
@@ -51,11 +53,11 @@ __device__ __forceinline__ void glu_tile(const GluArgs& p, uint16_t* S, int m0, 
         aoff[h < AH ? h : 0][i] = ((uint32_t)(m0 + m < p.M ? m : p.M - 1 - m0) * p.lda + piece * 8) * 2;
       }
     }
-    woff[i] = ((uint32_t)(n0 + row < p.n ? row : p.n - 1 - n0) * p.ldw + piece * 8) * 2;
+    woff[i] = ((uint32_t)(PLAIN || n0 + row < p.n ? row : p.n - 1 - n0) * p.ldw + piece * 8) * 2;
   }
   const char* abase = reinterpret_cast<const char*>(p.A + (size_t)m0 * p.lda);
-  const char* wbase[2] = {reinterpret_cast<const char*>(p.W + (size_t)n0 * p.ldw),      // gates, ups
-                          reinterpret_cast<const char*>(p.W + (size_t)(p.n + n0) * p.ldw)};
+  const char* wbase[2] = {reinterpret_cast<const char*>(p.W + (size_t)n0 * p.ldw),      // gates, ups; PLAIN: 128 columns and the next 128
+                          reinterpret_cast<const char*>(p.W + (size_t)((PLAIN ? 128 : p.n) + n0) * p.ldw)};
   const int steps = p.K / 64;
   const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)S) + wave * 2048;
   // half h of A (op 0), gates or ups (op 1) of step t into buffer `buf`; behind the last step that one once more, unused
@@ -177,6 +179,31 @@ __device__ __forceinline__ void glu_tile(const GluArgs& p, uint16_t* S, int m0, 
   }
   if (wm == 0) meet();
   ta_wait_loads<0>();                            // no wave ends with a load to LDS on its way
+  if constexpr (PLAIN) {
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float* to = p.X + n0 + y * 128 + wn * 32 + j * 16 + 4 * kb;
+        f32x4 old[AH][4];
+#pragma unroll
+        for (int x = 0; x < AH; ++x)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int m = m0 + wm * 64 * AH + x * 64 + i * 16 + r;
+            old[x][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (p.add) old[x][i] = *reinterpret_cast<const f32x4*>(to + (size_t)(m < p.M ? m : p.M - 1) * p.ldc);
+          }
+#pragma unroll
+        for (int x = 0; x < AH; ++x)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int m = m0 + wm * 64 * AH + x * 64 + i * 16 + r;
+            if (m < p.M) *reinterpret_cast<f32x4*>(to + (size_t)m * p.ldc) = old[x][i] + acc[x][y][i][j];
+          }
+      }
+    return;
+  }
   // a lane holds channels 4 kb .. + 3 of row r of each 16 x 16
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -201,18 +228,20 @@ __device__ __forceinline__ void glu_tile(const GluArgs& p, uint16_t* S, int m0, 
 }
 
 // Tiles in groups of 8 rows of tiles, column by column, so that the 32 workgroups of an XCD (every eighth) share 8 + 4 operands.
+template <bool PLAIN>
 __global__ __launch_bounds__(512, 2) void gemm_glu_kernel(GluArgs p) {
   __shared__ __attribute__((aligned(16))) uint16_t S[3 * 3 * HALF_TILE];         // 2 x 4 or 3 x 3 halves
-  const int tiles_n = (p.n + 127) / 128, grid_whole = (p.whole + 7) / 8 * 8;
+  constexpr int COLS = PLAIN ? 256 : 128;
+  const int tiles_n = (p.n + COLS - 1) / COLS, grid_whole = (p.whole + 7) / 8 * 8;
   const bool rest = (int)blockIdx.x >= grid_whole;
   const int id = rest ? blockIdx.x - grid_whole : blockIdx.x, all = rest ? p.halves : p.whole, share = (all + 7) / 8;
   const int at = id % 8 * share + id / 8;
   if (at >= all) return;
   const int tile = rest ? p.whole + at / 2 : at;
   const int group = tile / (8 * tiles_n), in = tile % (8 * tiles_n), high = p.tiles_m - group * 8 < 8 ? p.tiles_m - group * 8 : 8;
-  const int m0 = (group * 8 + in % high) * 256 + (rest ? at % 2 * 128 : 0), n0 = in / high * 128;
-  if (!rest && m0 + 128 < p.M) glu_tile<false>(p, S, m0, n0);
-  else if (m0 < p.M) glu_tile<true>(p, S, m0, n0);
+  const int m0 = (group * 8 + in % high) * 256 + (rest ? at % 2 * 128 : 0), n0 = in / high * COLS;
+  if (!rest && m0 + 128 < p.M) glu_tile<false, PLAIN>(p, S, m0, n0);
+  else if (m0 < p.M) glu_tile<true, PLAIN>(p, S, m0, n0);
 }
 
 enum { GLU_CUS = 256 };
@@ -237,11 +266,42 @@ extern "C" int ta_gemm_glu(hipStream_t stream, const void* A, int lda, const voi
   const long long tm = (M + 255) / 256, tiles = tm * ((n + 127) / 128), rest = tiles % GLU_CUS;
   TA_REQUIRE(tiles <= 1073741823, "ta_gemm_glu: M=%d n=%d too large for one launch", M, n);
   if (M == 0) return 0;
-  GluArgs p = {(const uint16_t*)A, (const uint16_t*)W, bias, (uint16_t*)C, lda, ldw, ldc, M, n, K, (int)tm, (int)tiles, 0, {limit, slope, shift, gelu}};
+  GluArgs p = {(const uint16_t*)A, (const uint16_t*)W, bias, (uint16_t*)C, lda, ldw, ldc, M, n, K, (int)tm, (int)tiles, 0, {limit, slope, shift, gelu}, nullptr, 0};
   if (rest <= GLU_CUS / 2) {
     p.whole = (int)(tiles - rest);
     p.halves = (int)(2 * rest);
   }
-  gemm_glu_kernel<<<(p.whole + 7) / 8 * 8 + (p.halves + 7) / 8 * 8, 512, 0, stream>>>(p);
+  gemm_glu_kernel<false><<<(p.whole + 7) / 8 * 8 + (p.halves + 7) / 8 * 8, 512, 0, stream>>>(p);
   return ta_check_launch("ta_gemm_glu");
+}
+
+// The same as a plain product with a float32 result. It is the library's equal while it multiplies (and sums in the same order except where that one cuts k);
+// it gains where its rounds are full, and where the library cuts its last round along k and falls to half. us there and here (the product added to the stream):
+// 4,096 columns over k = 14,336: 1,600 rows 333 / 182, 2,011 195 / 199, 2,502 0.83 times the library's rate, 3,164 501 / 289, 3,400 309 / 295, 4,000 335 / 322, 4,500 424 / 473, 5,640 753 / 494, 8,159 676 / 653; over 8,192 3,274 1.06, 3,853
+// 1.04; over 4,096 3,400 106 / 101, 4,000 112 / 110, but 8,159 216 / 224; 8,192 columns over 14,336: 1,573 328 / 303, 2,868 720 / 524; 5,120 over 14,336: 1,166 321 / 171,
+// 4,829 814 / 525; over 4,096 2,942 108 / 104. Rounds that end nearly half full gain for a long k alone, more than two rounds nowhere, results in bfloat16 lose 3 to 5 % (5,000 rows x 6,144 over
+// 4,096 182 / 194).
+extern "C" int ta_gemm_plain_pays(int M, int n, int K) {
+  if (M < 512 || n % 256 != 0 || K % 64 != 0 || K < 4096) return 0;
+  const long long tiles = (long long)(M + 255) / 256 * (n / 256), rest = tiles % GLU_CUS;
+  if (K < 8192) return tiles >= 208 && tiles <= GLU_CUS;
+  return tiles <= 2 * GLU_CUS && (rest == 0 || rest >= 208 || (rest >= 96 && rest <= (K <= 12288 ? 128 : 120)));
+}
+
+// C [M, n] = A W^T, or C += A W^T, float32.
+extern "C" int ta_gemm_plain(hipStream_t stream, const void* A, int lda, const void* W, int ldw, float* C, int ldc, int M, int n, int K, int add) {
+  TA_REQUIRE(M >= 0 && M <= 2147483392 && n > 0 && n % 256 == 0 && K > 0 && K % 64 == 0, "ta_gemm_plain: M=%d n=%d K=%d", M, n, K);
+  TA_REQUIRE(lda >= K && ldw >= K && ldc >= n && lda % 8 == 0 && ldw % 8 == 0 && ldc % 4 == 0 && lda <= 4194304 && ldw <= 4194304 &&
+                 ((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16 == 0,
+             "ta_gemm_plain: rows of %d, %d, %d or their start", lda, ldw, ldc);
+  const long long tm = ((long long)M + 255) / 256, tiles = tm * (n / 256), rest = tiles % GLU_CUS;
+  TA_REQUIRE(tiles <= 1073741823, "ta_gemm_plain: M=%d n=%d too large for one launch", M, n);
+  if (M == 0) return 0;
+  GluArgs p = {(const uint16_t*)A, (const uint16_t*)W, nullptr, nullptr, lda, ldw, ldc, M, n, K, (int)tm, (int)tiles, 0, {}, C, add};
+  if (rest <= GLU_CUS / 2) {
+    p.whole = (int)(tiles - rest);
+    p.halves = (int)(2 * rest);
+  }
+  gemm_glu_kernel<true><<<(p.whole + 7) / 8 * 8 + (p.halves + 7) / 8 * 8, 512, 0, stream>>>(p);
+  return ta_check_launch("ta_gemm_plain");
 }

@@ -905,12 +905,36 @@ def gemm_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, activation: st
     return out
 
 
+def _on_whole_pieces(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Operands whose rows the kernels for many bfloat16 rows can read: 16 bytes at a time."""
+    return a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and w.dim() == 2 \
+        and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 \
+        and max(a.stride(0), w.stride(0)) <= 4194304 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
 def glu_pays(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``gemm_glu`` is better than the vendor library's product and the activation's kernel: many rows against a wide weight."""
-    return a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and w.dim() == 2 and w.shape[0] % 2 == 0 \
-        and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 \
-        and max(a.stride(0), w.stride(0)) <= 4194304 and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+    return a.shape[0] > 384 and w.shape[0] % 2 == 0 and _on_whole_pieces(a, w) \
         and bool(library().ta_gemm_glu_pays(c_int(a.shape[0]), c_int(w.shape[0] // 2), c_int(a.shape[1])))
+
+
+def gemm_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, add: bool = False) -> torch.Tensor:
+    """out = a @ w.T, or out += a @ w.T, of many bfloat16 rows, out float32."""
+    _dev(a, "a", torch.bfloat16, contiguous=False); _dev(w, "w", torch.bfloat16, contiguous=False)
+    _dev(out, "out", torch.float32, contiguous=False)
+    M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
+    if w.shape[1] != a.shape[1] or tuple(out.shape) != (M, N):
+        raise KernelError(f"gemm_plain: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+    _check(library().ta_gemm_plain(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(out), c_int(ldc), c_int(M), c_int(N),
+                                   c_int(a.shape[1]), c_int(int(add))))
+    return out
+
+
+def plain_pays(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
+    """Whether ``gemm_plain`` is better than the vendor library's product: many rows whose tiles fill its rounds."""
+    return a.shape[0] >= 512 and out.dtype == torch.float32 and _on_whole_pieces(a, w) and out.dim() == 2 and out.stride(1) == 1 \
+        and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0 \
+        and bool(library().ta_gemm_plain_pays(c_int(a.shape[0]), c_int(w.shape[0]), c_int(a.shape[1])))
 
 
 def mid_takes(rows: int, w: torch.Tensor) -> bool:

@@ -71,6 +71,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor], s
     if kernels.mid_wins_plain(x.shape[0], weight) and x.stride(1) == 1 and x.stride(0) % 8 == 0 \
             and x.data_ptr() % 16 == 0:
         return kernels.gemm_mid(x, weight, out)
+    if kernels.plain_pays(x, weight, out):
+        return kernels.gemm_plain(x, weight, out)
     if out.dtype == x.dtype:
         torch.mm(x, weight.t(), out=out)
     else:
@@ -139,8 +141,8 @@ def library_rows(rows: int, n: int, k: int) -> list:
 
 
 def adds_in_place(rows: int, weight: torch.Tensor, dtype: torch.dtype = torch.bfloat16) -> bool:
-    """Whether ``linear_delta`` can add this product of ``dtype`` activations to the residual stream by itself: the
-    vendor library's product in one plane, which takes what it adds to as its third operand, or a few float32 rows."""
+    """Whether ``linear_delta`` can add this product of ``dtype`` activations to the residual stream by itself: a
+    product of many rows in one plane, which takes what it adds to as its third operand, or a few float32 rows."""
     if dtype == torch.float32:
         return kernels.add_takes(rows, weight)
     return weight.dtype == torch.bfloat16 and rows > kernels.MID_MAX_ROWS and \
@@ -166,6 +168,9 @@ def linear_delta(x: torch.Tensor, weight: torch.Tensor, ws: Workspace, name: str
                                       f"in place into {tuple(into.shape)} {into.dtype}")
         if x.dtype == torch.float32:
             kernels.gemm_add(x, weight, into)
+            return None
+        if kernels.plain_pays(x, weight, into):
+            kernels.gemm_plain(x, weight, into, add=True)
             return None
         at = 0
         for rows in library_rows(nt, n, x.shape[1]):
