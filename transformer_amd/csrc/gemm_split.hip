@@ -9,16 +9,20 @@ __device__ f32x4 split_zeros;      // where a piece past K is read from (never w
 // which no other wave needs; the columns' k are split once per workgroup, by all its waves, and go through LDS in operand layout,
 // 32 k at a time in two buffers, one barrier a step. The next step's operands are split between this step's products and what comes after them is
 // asked for right there. Bound by issue: 96 matrix instructions of 16 cycles, some 230 vector instructions and 30 of LDS a step of 32 k and wave. 1,021 x
-// 16,384 x 2,048 352 us (195 TFLOP/s, 1.17 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 80
+// 16,384 x 2,048 301 us (228 TFLOP/s, 1.37 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 80
 // (122), x 2,048 x 2,048 59 (79), x 2,048 x 8,192 211 (292). A split once by a kernel in front: the same (386 us and 384). Four waves of 64 rows: 455 for 370. G groups of WAVES waves take the segments of k in turn and the first adds up what the others hand it through LDS,
 // in ascending order.
-template <int WAVES, int NT, int G, bool VEC, bool WHOLE>
+//
+// GLU: W holds gate rows, then up rows (N in all); every other 16 of the workgroup's columns are the ups of the 16 before, and C = silu(gate) * up. 1,021 rows x 8,192
+// channels x 2,048 302 us, product and activation in turn 316; 2,000 rows 600 and 651; 3,000 x 14,336 x 4,096 3,400 and 3,477. Where the product goes by other
+// tiles (513 rows) it is their difference that would be lost.
+template <int WAVES, int NT, int G, bool VEC, bool WHOLE, bool GLU = false>
 __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
                                                                     int ldw, const float* __restrict__ bias, float* __restrict__ C,
                                                                     int ldc, int M, int N, int K, long long sa, long long sw,
                                                                     long long sc, int tiles_m, int tiles) {
   static_assert(NT >= 4 && NT % 2 == 0, "columns in pairs of tiles, the rows' splits between them");
-  constexpr int MT = 2, COLS = 16 * NT, ROWS = 16 * MT * WAVES;
+  constexpr int MT = 2, COLS = GLU ? 8 * NT : 16 * NT, ROWS = 16 * MT * WAVES;       // COLS: of C
   constexpr int BRING = (NT + WAVES - 1) / WAVES;      // tiles of 16 columns that a wave brings
   __shared__ bf16x8 S[G][2][3][NT][TA_WAVE];
   __shared__ f32x4 handed[G > 1 ? G - 1 : 1][G > 1 ? WAVES : 1][G > 1 ? MT * NT : 1][G > 1 ? TA_WAVE : 1];
@@ -31,6 +35,7 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
   W += (size_t)blockIdx.y * sw;
   C += (size_t)blockIdx.y * sc;
   const int m0 = tile % tiles_m * ROWS, n0 = tile / tiles_m * COLS;
+  const int n_out = GLU ? N / 2 : N;
   const int blocks = (K + 31) / 32, segs = (K + SEG - 1) / SEG, rounds = (segs + G - 1) / G;
   // steps of this group: 8 to a segment, and no further than the longest group's k
   const int last = segs - (rounds - 1) * G > 1 ? SEG / 32 : blocks - (segs - 1) * (SEG / 32);
@@ -45,8 +50,8 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
   }
 #pragma unroll
   for (int i = 0; i < BRING; ++i) {
-    const int f = wave + WAVES * i < NT ? wave + WAVES * i : NT - 1, n = 16 * f + r;
-    woff[i] = ((uint32_t)(n0 + n < N ? n : N - 1 - n0) * ldw + 4 * kb) * 4;
+    const int f = wave + WAVES * i < NT ? wave + WAVES * i : NT - 1, n = 16 * (GLU ? f / 2 : f) + r;
+    woff[i] = ((uint32_t)((n0 + n < n_out ? n : n_out - 1 - n0) + (GLU && f % 2 ? n_out : 0)) * ldw + 4 * kb) * 4;
   }
   auto piece = [&](const char* base, uint32_t off, int b, int h) {
     const char* p = base + (size_t)b * 128 + off + 64 * h;
@@ -181,21 +186,70 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
       }
   }
   if (group > 0) return;
+  // a lane's columns are four neighbours, stored at once where that is 16 bytes (1,021 x 16,384 x 2,048: 325 us one by one, 301 so)
+  const bool wide = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+  auto store = [&](int m, int n, const f32x4& v) __attribute__((always_inline)) {
+    float* c = C + (size_t)m * ldc + n;
+    if (wide && n + 3 < n_out) {
+      *reinterpret_cast<f32x4*>(c) = v;
+      return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < n_out) c[e] = v[e];
+  };
+  if constexpr (GLU) {
+    // Gates and ups that are not finite are formed again: C holds the other of the two meanwhile.
+    uint32_t bad[2] = {0, 0};
+    auto join = [&](float g, float u, int n) { return ta_glu(TaGlu{}, bias ? g + bias[n] : g, bias ? u + bias[n_out + n] : u); };
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int m = m0 + wave * 16 * MT + 16 * i + r;
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < NT / 2; ++j) {
+        const int n = n0 + 16 * j + 4 * kb;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = total[i][2 * j][e], u = total[i][2 * j + 1][e];
+          const bool bg = n + e < n_out && split_bad(g), bu = n + e < n_out && split_bad(u);
+          bad[0] |= (uint32_t)bg << (i * NT * 2 + j * 4 + e);
+          bad[1] |= (uint32_t)bu << (i * NT * 2 + j * 4 + e);
+          v[e] = bg ? u : bu ? g : n + e < n_out ? join(g, u, n + e) : 0.f;
+        }
+        store(m, n, v);
+      }
+    }
+#pragma unroll 1
+    for (uint32_t left = bad[0] | bad[1]; left; left &= left - 1) {
+      const int x = __ffs(left) - 1;
+      const int m = m0 + wave * 16 * MT + 16 * (x / (NT * 2)) + r, n = n0 + 16 * (x / 4 % (NT / 2)) + 4 * kb + x % 4;
+      float* c = C + (size_t)m * ldc + n;
+      const float* row = A + (size_t)m * lda;
+      float g = *c, u = *c;
+      if (bad[0] >> x & 1) g = split_again([&](int k) { return row[k]; }, W + (size_t)n * ldw, K);
+      if (bad[1] >> x & 1) u = split_again([&](int k) { return row[k]; }, W + (size_t)(n_out + n) * ldw, K);
+      *c = join(g, u, n);
+    }
+    return;
+  }
   bool bad = false;
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + wave * 16 * MT + 16 * i + r;
     if (m >= M) continue;
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; ++j) {
+      const int n = n0 + 16 * j + 4 * kb;
+      f32x4 v = total[i][j];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int n = n0 + 16 * j + 4 * kb + e;
-        if (n >= N) continue;
-        const float v = total[i][j][e];
-        bad |= split_bad(v);
-        C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
+        bad |= n + e < N && split_bad(v[e]);
+        if (bias && n + e < N) v[e] += bias[n + e];
       }
+      store(m, n, v);
+    }
   }
   if (!bad) return;
 #pragma unroll 1
@@ -281,4 +335,27 @@ void ta_gemm_split(hipStream_t stream, int form, const float* A, int lda, long l
 #undef RUN_ANY
 #undef RUN
 #undef RUN_
+}
+
+// Whether ta_gemm_split_glu takes the products of M rows with gates and ups (float32, rows on 16 bytes): where the product alone goes by
+// tiles of 256 x 128.
+extern "C" int ta_gemm_split_glu_takes(int M, int di, int K, int lda, int ldw) {
+  return M > 16 && di > 0 && di <= 1073741823 && K % 4 == 0 && ((long long)di + 64) * ldw < 1 << 30 &&
+         ta_gemm_split_form(M, 2 * di, K, lda, ldw, 1, true) == 1;
+}
+
+// C[M, di] = silu(A W[:di]^T + bias[:di]) * (A W[di:]^T + bias[di:]), W [2 di, K]: what the product and ta_swiglu give one after the other,
+// bit for bit.
+extern "C" int ta_gemm_split_glu(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc,
+                                 int M, int di, int K) {
+  TA_REQUIRE(ta_gemm_split_glu_takes(M, di, K, lda, ldw), "ta_gemm_split_glu: M=%d di=%d K=%d", M, di, K);
+  TA_REQUIRE(lda >= K && ldw >= K && ldc >= di && lda % 4 == 0 && ldw % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0,
+             "ta_gemm_split_glu: rows of %d, %d, %d floats or their start", lda, ldw, ldc);
+  const int tiles_m = (M + 255) / 256, tiles = tiles_m * ((di + 63) / 64);
+#define RUN(WHOLE) \
+  gemm_split_kernel<8, 8, 1, true, WHOLE, true><<<(tiles + 7) / 8 * 8, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, 2 * di, K, 0, 0, 0, tiles_m, tiles)
+  if (K % SEG == 0) RUN(true);
+  else RUN(false);
+#undef RUN
+  return ta_check_launch("ta_gemm_split_glu");
 }

@@ -630,18 +630,36 @@ def simple_glu_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_simple_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out [m, n] = silu(a @ w[:n].T) * (a @ w[n:].T) in float32, with the bits of ``gemm_simple`` and ``swiglu`` in turn."""
+    return _glu_rows(library().ta_gemm_simple_glu, "gemm_simple_glu", a, w, out, bias)
+
+
+def _glu_rows(run, what: str, a, w, out, bias) -> torch.Tensor:
     _dev(a, "a", torch.float32, contiguous=False); _dev(w, "w", torch.float32, contiguous=False)
     _dev(out, "out", torch.float32, contiguous=False)
     M, lda = _rows2d(a, "a"); N, ldw = _rows2d(w, "w"); Mo, ldc = _rows2d(out, "out")
     if N % 2 or w.shape[1] != a.shape[1] or Mo != M or out.shape[1] != N // 2:
-        raise KernelError(f"gemm_simple_glu: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
+        raise KernelError(f"{what}: a {tuple(a.shape)} w {tuple(w.shape)} out {tuple(out.shape)}")
     if bias is not None:
         _dev(bias, "bias", torch.float32)
         if bias.numel() != N:
-            raise KernelError("gemm_simple_glu: bias must hold one entry per row of w")
-    _check(library().ta_gemm_simple_glu(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(bias), _ptr(out), c_int(ldc),
-                                        c_int(M), c_int(N // 2), c_int(a.shape[1])))
+            raise KernelError(f"{what}: bias must hold one entry per row of w")
+    _check(run(_stream(), _ptr(a), c_int(lda), _ptr(w), c_int(ldw), _ptr(bias), _ptr(out), c_int(ldc), c_int(M), c_int(N // 2),
+               c_int(a.shape[1])))
     return out
+
+
+def split_glu_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``gemm_split_glu`` takes these operands: many float32 rows against a wide [gate rows | up rows]."""
+    return a.dtype == torch.float32 and w.dtype == torch.float32 and a.dim() == 2 and w.dim() == 2 and w.shape[0] % 2 == 0 \
+        and a.stride(1) == 1 and w.stride(1) == 1 and a.stride(0) % 4 == 0 and w.stride(0) % 4 == 0 \
+        and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+        and bool(library().ta_gemm_split_glu_takes(c_int(a.shape[0]), c_int(w.shape[0] // 2), c_int(a.shape[1]), c_int(a.stride(0)),
+                                                   c_int(w.stride(0))))
+
+
+def gemm_split_glu(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``gemm_simple_glu`` of many rows, with the bits of ``gemm_simple`` and ``swiglu`` in turn."""
+    return _glu_rows(library().ta_gemm_split_glu, "gemm_split_glu", a, w, out, bias)
 
 
 class RowNorm:

@@ -64,6 +64,9 @@ class SwiGLU(Part):
         elif self.limits is None and kernels.simple_glu_takes(h, self.w["gate_up.weight"]):
             # few float32 rows: the product applies the activation itself, with the same bits
             kernels.gemm_simple_glu(h, self.w["gate_up.weight"], act, self.w.get("gate_up.bias"))
+        elif self.limits is None and kernels.split_glu_takes(h, self.w["gate_up.weight"]):
+            # and many
+            kernels.gemm_split_glu(h, self.w["gate_up.weight"], act, self.w.get("gate_up.bias"))
         elif kernels.glu_pays(h, self.w["gate_up.weight"]):
             # many bfloat16 rows: likewise, gates and ups joined before they are rounded
             kernels.gemm_glu(h, self.w["gate_up.weight"], act, bias=self.w.get("gate_up.bias"), limits=self.limits)
