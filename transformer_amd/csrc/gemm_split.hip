@@ -9,8 +9,8 @@ __device__ f32x4 split_zeros;      // where a piece past K is read from (never w
 // which no other wave needs; the columns' k are split once per workgroup, by all its waves, and go through LDS in operand layout,
 // 32 k at a time in two buffers, one barrier a step. The next step's operands are split between this step's products and what comes after them is
 // asked for right there. Bound by issue: 96 matrix instructions of 16 cycles, some 230 vector instructions and 30 of LDS a step of 32 k and wave. 1,021 x
-// 16,384 x 2,048 301 us (228 TFLOP/s, 1.37 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 80
-// (122), x 2,048 x 2,048 59 (79), x 2,048 x 8,192 211 (292). A split once by a kernel in front: the same (386 us and 384). Four waves of 64 rows: 455 for 370. G groups of WAVES waves take the segments of k in turn and the first adds up what the others hand it through LDS,
+// 16,384 x 2,048 301 to 330 us by card (208 to 228 TFLOP/s, up to 1.37 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 78
+// (122), x 2,048 x 2,048 56 (79), x 2,048 x 8,192 204 (292). A split once by a kernel in front: the same (386 us and 384). Four waves of 64 rows: 455 for 370. G groups of WAVES waves take the segments of k in turn and the first adds up what the others hand it through LDS,
 // in ascending order.
 //
 // GLU: W holds gate rows, then up rows (N in all); every other 16 of the workgroup's columns are the ups of the 16 before, and C = silu(gate) * up. 1,021 rows x 8,192
