@@ -455,6 +455,27 @@ extern "C" long long ta_attention_f32_scratch(int batch, int nh, int max_blocks,
   return (long long)batch * nh * max_blocks * (dv + 2);
 }
 
+// Which kernels take these widths: 128 and 128, 64 and 64, both up to 64, any. Up to 64 by half the registers and LDS: 16 heads of 32 over 4, a prompt of
+// 1,021 76 us by the kernel for any and 55 by its own, 3,000 466 and 227.
+static int f32_widths(int dh, int dv) { return dh == 128 && dv == 128 ? 0 : dh == 64 && dv == 64 ? 1 : dh <= 64 && dv <= 64 ? 2 : 3; }
+
+// Waves for 16 rows by the blocks of 64 rows that the step has (half a block more a sequence), where SPLIT 4 keeps the CUs from idling and 2 the
+// longest rows from walking alone. Many short sequences gain nothing: their pages are few and every workgroup brings them again. us of SPLIT 1, 2, 4, heads of 128
+// over 4 kv heads: 2 + 34 blocks 22 / 16 / 14, 175 65 / 48 / 45, 4 x 50 to 300 tokens (190) 33 / 28 / 30, 4 x 400 (408) 63 / 58 / 67, 16 x 100 (432) 27 / 31 / 37, 8 x 300 (616) 63 / 67 / 78;
+// 32 heads of 64 over 8: 200 29 / 23 / 26, 512 100 / 68 / 91, 1,005 265 / 242 / 300, 1,500 493 / 492 / 626.
+// Heads of 16, whose pages cost little beside the barriers, not over several sequences (8 heads, 8 x 200 16 / 18, 8 x 300 21 / 24; 4 x 300 20 / 23; one of 1,021 53 / 44).
+static int f32_split(int batch, int max_qlen, int tokens, int group, int nkv, int widest) {
+  if (widest <= 16 && batch >= 4) return 1;
+  const long long rows = (long long)max_qlen * group, blocks = ((long long)tokens * group + 63) / 64 * nkv + (long long)batch * nkv / 2;
+  return rows > 65535 * 16 || blocks > (max_qlen >= 1000 ? 1024 : max_qlen >= 256 ? 512 : 256) ? 1 : blocks <= 180 ? 4 : 2;
+}
+
+// The prompts' kernel that ta_attention_f32 launches: f32_widths times 8 plus the waves for 16 rows; 0 for heads that it refuses.
+extern "C" int ta_attention_f32_form(int batch, int max_qlen, int tokens, int nh, int nkv, int dh, int dv) {
+  if (nh <= 0 || nkv <= 0 || nh % nkv != 0) return 0;
+  return f32_widths(dh, dv) * 8 + f32_split(batch, max_qlen, tokens, nh / nkv, nkv, dh > dv ? dh : dv);
+}
+
 // As ta_attention_generic_sink, float32, dh and dv multiples of 16 up to 128, rows that start on 16 bytes. parts:
 // scratch of ta_attention_f32_turn_scratch floats for steps in which every sequence brings one token or none (max_qlen 1), or
 // null: the kernel for prompts then serves these too, with the same bits. tokens: of all sequences, by which the prompts' kernel is split.
@@ -483,14 +504,14 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
   F32Attention p = {(const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table, cu_q, pos0,
                           sink, (const float*)gate, parts, q_stride, out_stride, max_blocks, nh, nkv, dh, dv, window,
                           sink_mode, gate_stride, gate_dv, keep, chunk, scale, softcap, 0, 0, 0, 0};
-  const int group = nh / nkv, most = dh > dv ? dh : dv;
-#define PICK(kernel, grid, ...)                                                                \
-  do {                                                                                         \
-    if (dh == 128 && dv == 128) kernel<8, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);   \
-    else if (dh == 64 && dv == 64) kernel<4, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p); \
-    else if (most <= 64) kernel<4, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);         \
-    else kernel<8, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);                         \
-  } while (0)
+  const int group = nh / nkv, widths = f32_widths(dh, dv);
+#define PICK(kernel, grid, ...)                                                         \
+  switch (widths) {                                                                     \
+    case 0: kernel<8, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p); break;         \
+    case 1: kernel<4, true, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p); break;         \
+    case 2: kernel<4, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p); break;        \
+    default: kernel<8, false, ##__VA_ARGS__><<<grid, 256, 0, stream>>>(p);              \
+  }
   if (max_qlen == 1 && parts != nullptr) {
     int kvs;
     f32_turn(batch, nh, nkv, max_blocks, dv, p.seqs, kvs);
@@ -500,20 +521,19 @@ extern "C" int ta_attention_f32(hipStream_t stream, const void* q, int q_stride,
         const int bs = batch - p.b0 < p.seqs ? batch - p.b0 : p.seqs, ks = nkv - p.kv0 < kvs ? nkv - p.kv0 : kvs;
         const long long rows = (long long)ks * ((group + 15) / 16) * bs;
         const int each = (int)((F32_PAGE_WGS + rows - 1) / rows), turn = each < 8 ? 8 : each;
-        PICK(attn_f32_pages_kernel, dim3(ks * ((group + 15) / 16), bs, max_blocks < turn ? max_blocks : turn));
+        PICK(attn_f32_pages_kernel, dim3(ks * ((group + 15) / 16), bs, max_blocks < turn ? max_blocks : turn))
         attn_f32_join_kernel<<<dim3(ks * group, bs), 128, 0, stream>>>(p);
       }
   } else {
-    // Waves for 16 rows by the blocks of 64 rows that the step has (half a block more a sequence), where SPLIT 4 keeps the CUs from idling and 2 the
-    // longest rows from walking alone. Many short sequences gain nothing: their pages are few and every workgroup brings them again. us of SPLIT 1, 2, 4, heads of 128
-    // over 4 kv heads: 2 + 34 blocks 22 / 16 / 14, 175 65 / 48 / 45, 4 x 50 to 300 tokens (190) 33 / 28 / 30, 4 x 400 (408) 63 / 58 / 67, 16 x 100 (432) 27 / 31 / 37, 8 x 300 (616) 63 / 67 / 78;
-    // 32 heads of 64 over 8: 200 29 / 23 / 26, 512 100 / 68 / 91, 1,005 265 / 242 / 300, 1,500 493 / 492 / 626.
-    const long long rows = (long long)max_qlen * group, blocks = ((long long)tokens * group + 63) / 64 * nkv + (long long)batch * nkv / 2;
-    const int most = max_qlen >= 1000 ? 1024 : max_qlen >= 256 ? 512 : 256;
-    const int split = rows > 65535 * 16 || blocks > most ? 1 : blocks <= 180 ? 4 : 2;
-    if (split == 4) PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 15) / 16), batch), 4);
-    else if (split == 2) PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 31) / 32), batch), 2);
-    else PICK(attn_f32_rows_kernel, dim3((unsigned)((rows + 63) / 64), nkv, batch), 1);
+    const long long rows = (long long)max_qlen * group;
+    const int split = f32_split(batch, max_qlen, tokens, group, nkv, dh > dv ? dh : dv);
+    if (split == 4) {
+      PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 15) / 16), batch), 4)
+    } else if (split == 2) {
+      PICK(attn_f32_rows_kernel, dim3(nkv, (unsigned)((rows + 31) / 32), batch), 2)
+    } else {
+      PICK(attn_f32_rows_kernel, dim3((unsigned)((rows + 63) / 64), nkv, batch), 1)
+    }
   }
 #undef PICK
   return ta_check_launch("ta_attention_f32");
