@@ -234,7 +234,8 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
     }
     return;
   }
-  bool bad = false;
+  uint64_t bad = 0;                                    // which of the lane's sums, without their bias, are not finite
+  static_assert(MT * NT * 4 <= 64, "a bit a result");
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + wave * 16 * MT + 16 * i + r;
@@ -245,22 +246,19 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
       f32x4 v = total[i][j];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        bad |= n + e < N && split_bad(v[e]);
+        bad |= (uint64_t)(n + e < N && split_bad(v[e])) << (i * NT * 4 + j * 4 + e);
         if (bias && n + e < N) v[e] += bias[n + e];
       }
       store(m, n, v);
     }
   }
-  if (!bad) return;
 #pragma unroll 1
-  for (int x = 0; x < MT * NT * 4; ++x) {              // what this lane has stored that is not finite
+  for (; bad; bad &= bad - 1) {
+    const int x = __ffsll((unsigned long long)bad) - 1;
     const int m = m0 + wave * 16 * MT + 16 * (x / (NT * 4)) + r, n = n0 + 16 * (x / 4 % NT) + 4 * kb + x % 4;
-    if (m >= M || n >= N) continue;
-    float* c = C + (size_t)m * ldc + n;
-    if (!split_bad(*c)) continue;
     const float* row = A + (size_t)m * lda;
     const float v = split_again([&](int k) { return row[k]; }, W + (size_t)n * ldw, K);
-    *c = bias ? v + bias[n] : v;
+    C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
   }
 }
 
