@@ -160,9 +160,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
   for (int e = 0; e < OUT; ++e) {
     const int at = (int)threadIdx.x + WAVES * 64 * e;
     const int m = m0 + at / COLS, n = n0 + at % COLS;
-    if (at >= ROWS * COLS || m >= M || n >= N) continue;
-    if (SPLIT && split_bad(total[e]))
-      total[e] = split_again([&](int k) { return to_f32(A[(size_t)m * lda + k]); }, reinterpret_cast<const float*>(W + (size_t)n * ldw), K);
+    const bool own = at < ROWS * COLS && m < M && n < N;
+    if constexpr (SPLIT) {
+      auto row = [&](int i, int k) { return (float)A[(size_t)i * lda + k]; };
+      total[e] = split_again(own && split_bad(total[e]), total[e], m, (const float*)(W + (size_t)n * ldw), K, row,
+                             [&](int i) { return split_undefined([&](int k) { return row(i, k); }, K); });
+    }
+    if (!own) continue;
     C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
   }
 }
@@ -189,6 +193,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
   constexpr int HALF = SIDE / 2;
   static_assert(WAVES * 64 >= SIDE * SIDE, "a thread an output");
   __shared__ __attribute__((aligned(16))) float part[2][TURN][SIDE * SIDE];
+  __shared__ int undefined[SIDE];                // of its rows, see split_undefined_once; a wave asks for its own only
+  if (threadIdx.x < SIDE) undefined[threadIdx.x] = 0;
   const int wave = threadIdx.x / TA_WAVE, lane = threadIdx.x % TA_WAVE;
   const int r = lane % 16, kb = lane / 16, col = r % SIDE;
   const int seg = PAIR ? 2 * wave + r / 8 : wave, segs = (K + SEG - 1) / SEG;
@@ -264,8 +270,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
       float total = 0.f;
       for (int s = 0; s < segs; ++s) total += to[s][threadIdx.x];
       const int n = (GLU ? HALF * tile + nn % HALF : SIDE * tile + nn);
-      if (split_bad(total) && m < M && n < n_out)
-        total = split_again([&](int k) { return A[(size_t)m * lda + k]; }, W + (size_t)(n + (GLU && nn >= HALF ? n_out : 0)) * ldw, K);
+      auto a_of = [&](int i, int k) { return A[(size_t)i * lda + k]; };
+      total = split_again(m < M && n < n_out && split_bad(total), total, m, W + (size_t)(n + (GLU && nn >= HALF ? n_out : 0)) * ldw, K, a_of,
+                          [&](int i) { return split_undefined_once(undefined, i, [&](int k) { return a_of(i, k); }, K); });
       if (bias && n < n_out) total += bias[n + (GLU && nn >= HALF ? n_out : 0)];
       if (GLU) {
         const float up = __shfl_xor(total, HALF, TA_WAVE);

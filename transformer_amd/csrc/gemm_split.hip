@@ -198,9 +198,43 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
     for (int e = 0; e < 4; ++e)
       if (n + e < n_out) c[e] = v[e];
   };
+  // What is not finite: bit i PER + 4 j + e of the lane's, of gates and ups one set each. Rows with an undefined number are left as they are.
+  constexpr int PER = GLU ? NT * 2 : NT * 4;           // results of one row tile
+  uint64_t bad[GLU ? 2 : 1] = {};
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        bad[GLU ? j % 2 : 0] |= (uint64_t)(m0 + wave * 16 * MT + 16 * i + r < M && n0 + 16 * (GLU ? j / 2 : j) + 4 * kb + e < n_out &&
+                                           split_bad(total[i][j][e])) << (i * PER + (GLU ? j / 2 : j) * 4 + e);
+  auto of_row = [&](int m) { return [=](int k) { return A[(size_t)m * lda + k]; }; };
+  uint64_t any = GLU ? bad[0] | bad[1 % (GLU ? 2 : 1)] : bad[0];
+  if (__ballot(any != 0) != 0)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const uint64_t own = (PER == 64 ? ~0ull : (1ull << PER) - 1) << (i * PER), lanes = __ballot((any & own) != 0);
+#pragma unroll 1
+      for (uint32_t rows = (lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xffff; rows; rows &= rows - 1) {
+        const int row = __builtin_ctz(rows);
+        if (!split_undefined(of_row(m0 + wave * 16 * MT + 16 * i + row), K)) continue;
+        if (r == row) any &= ~own, bad[0] &= ~own, bad[GLU ? 1 : 0] &= ~own;
+      }
+    }
+  // The others, by the wave one after the other: form(bit, lane, row, column).
+  auto again = [&](auto form) {
+    if (__ballot(any != 0) == 0) return;
+#pragma unroll 1
+    for (int x = 0; x < MT * PER; ++x)
+#pragma unroll 1
+      for (uint64_t lanes = __ballot((any >> x & 1) != 0); lanes; lanes &= lanes - 1) {
+        const int from = __builtin_ctzll(lanes);
+        form(x, from, m0 + wave * 16 * MT + 16 * (x / PER) + from % 16, n0 + 16 * (x % PER / 4) + 4 * (from / 16) + x % 4);
+      }
+  };
   if constexpr (GLU) {
-    // Gates and ups that are not finite are formed again: C holds the other of the two meanwhile.
-    uint32_t bad[2] = {0, 0};
+    // Of a gate and an up of which one is to be formed again C holds the other meanwhile.
     auto join = [&](float g, float u, int n) { return ta_glu(TaGlu{}, bias ? g + bias[n] : g, bias ? u + bias[n_out + n] : u); };
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -213,29 +247,23 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = total[i][2 * j][e], u = total[i][2 * j + 1][e];
-          const bool bg = n + e < n_out && split_bad(g), bu = n + e < n_out && split_bad(u);
-          bad[0] |= (uint32_t)bg << (i * NT * 2 + j * 4 + e);
-          bad[1] |= (uint32_t)bu << (i * NT * 2 + j * 4 + e);
-          v[e] = bg ? u : bu ? g : n + e < n_out ? join(g, u, n + e) : 0.f;
+          const int x = i * PER + j * 4 + e;
+          v[e] = bad[0] >> x & 1 ? u : bad[1] >> x & 1 ? g : n + e < n_out ? join(g, u, n + e) : 0.f;
         }
         store(m, n, v);
       }
     }
-#pragma unroll 1
-    for (uint32_t left = bad[0] | bad[1]; left; left &= left - 1) {
-      const int x = __ffs(left) - 1;
-      const int m = m0 + wave * 16 * MT + 16 * (x / (NT * 2)) + r, n = n0 + 16 * (x / 4 % (NT / 2)) + 4 * kb + x % 4;
+    again([&](int x, int from, int m, int n) {
+      const bool gate = __builtin_amdgcn_readlane((int)(bad[0] >> x & 1), from), up = __builtin_amdgcn_readlane((int)(bad[1] >> x & 1), from);
+      float g = 0.f, u = 0.f;
+      if (gate) g = split_dot(of_row(m), W + (size_t)n * ldw, K);
+      if (up) u = split_dot(of_row(m), W + (size_t)(n_out + n) * ldw, K);
+      if (lane != from) return;
       float* c = C + (size_t)m * ldc + n;
-      const float* row = A + (size_t)m * lda;
-      float g = *c, u = *c;
-      if (bad[0] >> x & 1) g = split_again([&](int k) { return row[k]; }, W + (size_t)n * ldw, K);
-      if (bad[1] >> x & 1) u = split_again([&](int k) { return row[k]; }, W + (size_t)(n_out + n) * ldw, K);
-      *c = join(g, u, n);
-    }
+      *c = join(gate ? g : *c, up ? u : *c, n);
+    });
     return;
   }
-  uint64_t bad = 0;                                    // which of the lane's sums, without their bias, are not finite
-  static_assert(MT * NT * 4 <= 64, "a bit a result");
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = m0 + wave * 16 * MT + 16 * i + r;
@@ -245,21 +273,15 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
       const int n = n0 + 16 * j + 4 * kb;
       f32x4 v = total[i][j];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        bad |= (uint64_t)(n + e < N && split_bad(v[e])) << (i * NT * 4 + j * 4 + e);
+      for (int e = 0; e < 4; ++e)
         if (bias && n + e < N) v[e] += bias[n + e];
-      }
       store(m, n, v);
     }
   }
-#pragma unroll 1
-  for (; bad; bad &= bad - 1) {
-    const int x = __ffsll((unsigned long long)bad) - 1;
-    const int m = m0 + wave * 16 * MT + 16 * (x / (NT * 4)) + r, n = n0 + 16 * (x / 4 % NT) + 4 * kb + x % 4;
-    const float* row = A + (size_t)m * lda;
-    const float v = split_again([&](int k) { return row[k]; }, W + (size_t)n * ldw, K);
-    C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
-  }
+  again([&](int, int from, int m, int n) {
+    const float v = split_dot(of_row(m), W + (size_t)n * ldw, K);
+    if (lane == from) C[(size_t)m * ldc + n] = bias ? v + bias[n] : v;
+  });
 }
 
 // us a step of 32 k (of all groups) when every CU has its workgroups: measured at 130 to 3,000 rows of 2,048 to 16,384 columns, k = 2,048

@@ -44,6 +44,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
   __shared__ __attribute__((aligned(16))) float ring[WAVES][PF][SLOT];
   __shared__ __attribute__((aligned(16))) float part[2][TURN][64];
   __shared__ float sq[8][WAVES / 2];
+  __shared__ int undefined[8];                   // of its rows, see split_undefined_once; one wave asks between two barriers
+  if (threadIdx.x < 8) undefined[threadIdx.x] = 0;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TA_WAVE), lane = threadIdx.x % TA_WAVE;
   const int r = lane % 16, kb = lane / 16, lrow = lane / 16, lpiece = lane % 16;
   const int n_out = GLU ? N / 2 : N, segs = (K + SEG - 1) / SEG;
@@ -168,18 +170,15 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
       const int m = lane / 8, nn = lane % 8, n = GLU ? 4 * tile + nn % 4 : 8 * tile + nn;
       float total = 0.f;
       for (int s = 0; s < segs; ++s) total += to[s][lane];
-      if (split_bad(total) && m < M && n < n_out) {
-        float rstd = 1.f;
-        if (NORM) {
-          float all = 0.f;
+      auto a_of = [&](int i, int k) {              // (of one row at a time: the factor is formed once)
+        if (!NORM) return A[(size_t)i * lda + k];
+        float all = 0.f;
 #pragma unroll
-          for (int i = 0; i < WAVES / 2; ++i) all += sq[m][i];
-          rstd = 1.0f / sqrtf(all / (float)K + nm.eps);
-        }
-        const float* row = A + (size_t)m * lda;
-        total = split_again([&](int k) { return NORM ? row[k] * rstd * nm.w[k] : row[k]; },
-                            W + (size_t)(n + (GLU && nn >= 4 ? n_out : 0)) * ldw, K);
-      }
+        for (int q = 0; q < WAVES / 2; ++q) all += sq[i][q];
+        return A[(size_t)i * lda + k] * (1.0f / sqrtf(all / (float)K + nm.eps)) * nm.w[k];
+      };
+      total = split_again(m < M && n < n_out && split_bad(total), total, m, W + (size_t)(n + (GLU && nn >= 4 ? n_out : 0)) * ldw, K, a_of,
+                          [&](int i) { return split_undefined_once(undefined, i, [&](int k) { return a_of(i, k); }, K); });
       if (bias && n < n_out) total += bias[n + (GLU && nn >= 4 ? n_out : 0)];
       if (GLU) {
         const float up = __shfl_xor(total, 4, TA_WAVE);
@@ -279,8 +278,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
       for (int s = 0; s < live; ++s) total += to[s][lane];
     }
   }
+  if (wave == 0) {
+    auto a_of = [&](int i, int k) { return A[(size_t)i * lda + k]; };
+    total = split_again(m < M && n < N && split_bad(total), total, m, W + (size_t)n * ldw, K, a_of,
+                        [&](int i) { return split_undefined([&](int k) { return a_of(i, k); }, K); });
+  }
   if (wave == 0 && m < M && n < N) {
-    if (split_bad(total)) total = split_again([&](int k) { return A[(size_t)m * lda + k]; }, W + (size_t)n * ldw, K);
     if (bias) total += bias[n];
     float* c = C + (size_t)m * ldc + n;
     *c = add ? *c + total : total;
