@@ -103,9 +103,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
     if constexpr (SPLIT) {
 #pragma unroll
       for (int i = 0; i < BC; i += 2) {
-        const Split8 w = split8<false>(wreg[set][i], wreg[set][i + 1]);
+        const Split8 w = split8(wreg[set][i], wreg[set][i + 1]);
 #pragma unroll
-        for (int t = 0; t < RT; ++t) acc[t] += split_block(w, split8<true>(areg[set][t][i], areg[set][t][i + 1]));
+        for (int t = 0; t < RT; ++t) acc[t] += split_block(w, split8(areg[set][t][i], areg[set][t][i + 1]));
       }
     } else {
 #pragma unroll
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
     const bool own = at < ROWS * COLS && m < M && n < N;
     if constexpr (SPLIT) {
       auto row = [&](int i, int k) { return (float)A[(size_t)i * lda + k]; };
-      total[e] = split_again(own && split_bad(total[e]), total[e], m, (const float*)(W + (size_t)n * ldw), K, row,
+      total[e] = split_again(own && split_bad(total[e]), total[e] * SPLIT_DOWN, m, (const float*)(W + (size_t)n * ldw), K, row,
                              [&](int i) { return split_undefined([&](int k) { return row(i, k); }, K); });
     }
     if (!own) continue;
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
     for (int i = 0; i < BC; ++i) to[i] = load_piece<float, true, false>(arow, k_of(c, i), K);
     if (KEEP)
 #pragma unroll
-      for (int i = 0; i < BC; i += 2) as[KEEP ? c : 0][i / 2] = split8<true>(to[i], to[i + 1]);
+      for (int i = 0; i < BC; i += 2) as[KEEP ? c : 0][i / 2] = split8(to[i], to[i + 1]);
   }
   const int m = threadIdx.x / SIDE, nn = threadIdx.x % SIDE;
   for (int turn = 0; tile < tiles; tile += gridDim.x, turn ^= 1) {
@@ -232,13 +232,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
     auto multiply = [&](int c) {
 #pragma unroll
       for (int i = 0; i < BC; i += 2) {
-        const Split8 wi = split8<false>(w[c % 2][i], w[c % 2][i + 1]);
+        const Split8 wi = split8(w[c % 2][i], w[c % 2][i + 1]);
         if (KEEP) {
           acc += split_block(wi, as[KEEP ? c : 0][i / 2]);
         } else {
           f32x4 x = a[KEEP ? 0 : c][i], y = a[KEEP ? 0 : c][i + 1];
           asm volatile("" : "+v"(x), "+v"(y));   // or the compiler splits all of A in front of the loop and has no registers for it
-          acc += split_block(wi, split8<true>(x, y));
+          acc += split_block(wi, split8(x, y));
         }
       }
     };
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_walk_kernel(const float* __re
       for (int s = 0; s < segs; ++s) total += to[s][threadIdx.x];
       const int n = (GLU ? HALF * tile + nn % HALF : SIDE * tile + nn);
       auto a_of = [&](int i, int k) { return A[(size_t)i * lda + k]; };
-      total = split_again(m < M && n < n_out && split_bad(total), total, m, W + (size_t)(n + (GLU && nn >= HALF ? n_out : 0)) * ldw, K, a_of,
+      total = split_again(m < M && n < n_out && split_bad(total), total * SPLIT_DOWN, m, W + (size_t)(n + (GLU && nn >= HALF ? n_out : 0)) * ldw, K, a_of,
                           [&](int i) { return split_undefined_once(undefined, i, [&](int k) { return a_of(i, k); }, K); });
       if (bias && n < n_out) total += bias[n + (GLU && nn >= HALF ? n_out : 0)];
       if (GLU) {

@@ -8,7 +8,7 @@ __device__ f32x4 split_zeros;      // where a piece past K is read from (never w
 // A workgroup owns 32 WAVES x 16 NT of C. A wave owns 32 of the rows: it reads them from memory in operand layout and splits them,
 // which no other wave needs; the columns' k are split once per workgroup, by all its waves, and go through LDS in operand layout,
 // 32 k at a time in two buffers, one barrier a step. The next step's operands are split between this step's products and what comes after them is
-// asked for right there. Bound by issue: 96 matrix instructions of 16 cycles, some 230 vector instructions and 30 of LDS a step of 32 k and wave. 1,021 x
+// asked for right there. Bound by issue: 96 matrix instructions of 16 cycles, some 250 vector instructions and 30 of LDS a step of 32 k and wave. 1,021 x
 // 16,384 x 2,048 301 to 330 us by card (208 to 228 TFLOP/s, up to 1.37 PFLOP/s of bfloat16; 535 to 610 in float32 tiles of 128 x 128 on the float32 matrix instructions), 1,021 x 3,072 x 2,048 78
 // (122), x 2,048 x 2,048 56 (79), x 2,048 x 8,192 204 (292). A split once by a kernel in front: the same (386 us and 384). Four waves of 64 rows: 455 for 370. G groups of WAVES waves take the segments of k in turn and the first adds up what the others hand it through LDS,
 // in ascending order.
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
     for (int i = 0; i < BRING; ++i) {
       const int f = wave + WAVES * i;
       if (NT % WAVES == 0 || f < NT) {
-        const Split8 w = split8<false>(win[i][0], win[i][1]);
+        const Split8 w = split8(win[i][0], win[i][1]);
         S[group][buf][0][f][lane] = w.h;
         S[group][buf][1][f][lane] = w.m;
         S[group][buf][2][f][lane] = w.l;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
   load_w(1);
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    a[0][i] = split8<true>(ain[i][0], ain[i][1]);
+    a[0][i] = split8(ain[i][0], ain[i][1]);
     load_a(i, 1);
   }
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -146,14 +146,14 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
 #pragma unroll
       for (int i = 0; i < MT; ++i)
         if (j == (NT > 4 ? 2 + 2 * i : 2 * i)) {
-          a[buf ^ 1][i] = split8<true>(ain[i][0], ain[i][1]);
+          a[buf ^ 1][i] = split8(ain[i][0], ain[i][1]);
           load_a(i, s + 2);
         }
-      // two products, then up to five of the vector instructions between them
+      // two products, then up to six of the vector instructions between them
 #pragma unroll
       for (int z = 0; z < 12; ++z) {
         __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 6, 0);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -204,11 +204,13 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+    for (int j = 0; j < NT; ++j) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         bad[GLU ? j % 2 : 0] |= (uint64_t)(m0 + wave * 16 * MT + 16 * i + r < M && n0 + 16 * (GLU ? j / 2 : j) + 4 * kb + e < n_out &&
                                            split_bad(total[i][j][e])) << (i * PER + (GLU ? j / 2 : j) * 4 + e);
+      total[i][j] *= SPLIT_DOWN;
+    }
   auto of_row = [&](int m) { return [=](int k) { return A[(size_t)m * lda + k]; }; };
   uint64_t any = GLU ? bad[0] | bad[1 % (GLU ? 2 : 1)] : bad[0];
   if (__ballot(any != 0) != 0)

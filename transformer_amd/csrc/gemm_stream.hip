@@ -157,8 +157,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
       slot = slot + 1 == PF ? 0 : slot + 1;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        if (first) as[2 * c + i] = split8<true>(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
-        acc += split_block(split8<false>(w[2 * i], w[2 * i + 1]), as[2 * c + i]);
+        if (first) as[2 * c + i] = split8(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
+        acc += split_block(split8(w[2 * i], w[2 * i + 1]), as[2 * c + i]);
       }
     }
     // a lane holds columns 4 kb .. + 3 of row r: of the products, the two squares on the diagonal are used
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
         for (int q = 0; q < WAVES / 2; ++q) all += sq[i][q];
         return A[(size_t)i * lda + k] * (1.0f / sqrtf(all / (float)K + nm.eps)) * nm.w[k];
       };
-      total = split_again(m < M && n < n_out && split_bad(total), total, m, W + (size_t)(n + (GLU && nn >= 4 ? n_out : 0)) * ldw, K, a_of,
+      total = split_again(m < M && n < n_out && split_bad(total), total * SPLIT_DOWN, m, W + (size_t)(n + (GLU && nn >= 4 ? n_out : 0)) * ldw, K, a_of,
                           [&](int i) { return split_undefined_once(undefined, i, [&](int k) { return a_of(i, k); }, K); });
       if (bias && n < n_out) total += bias[n + (GLU && nn >= 4 ? n_out : 0)];
       if (GLU) {
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
       request(slot);
       slot = slot + 1 == PF ? 0 : slot + 1;
 #pragma unroll
-      for (int i = 0; i < 4; i += 2) acc += split_block(split8<false>(w[i], w[i + 1]), split8<true>(a[i], a[i + 1]));
+      for (int i = 0; i < 4; i += 2) acc += split_block(split8(w[i], w[i + 1]), split8(a[i], a[i + 1]));
     }
     auto* to = part[round & 1];
     if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[2 * wave + r / 8][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
   }
   if (wave == 0) {
     auto a_of = [&](int i, int k) { return A[(size_t)i * lda + k]; };
-    total = split_again(m < M && n < N && split_bad(total), total, m, W + (size_t)n * ldw, K, a_of,
+    total = split_again(m < M && n < N && split_bad(total), total * SPLIT_DOWN, m, W + (size_t)n * ldw, K, a_of,
                         [&](int i) { return split_undefined([&](int k) { return a_of(i, k); }, K); });
   }
   if (wave == 0 && m < M && n < N) {

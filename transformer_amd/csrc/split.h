@@ -1,7 +1,8 @@
-// Products of 32-bit numbers on the 16-bit matrix instructions. A float32 x is the sum of three bfloat16, x = h + m + l, exactly
-// (24 bits in three times 8), and of the nine products of two such sums the six that matter are multiplied:
-// h h, h m, m h, m m, h l, l h; what is left out is 2^-24 of a product at the most, of either sign, and 2^-28 in the mean. v_mfma_f32_16x16x32_bf16 multiplies exactly and
-// takes denormals: 32 k of all six occupy a SIMD for 96 cycles where the float32 instructions need 256.
+// Products of 32-bit numbers on the 16-bit matrix instructions, by the published way of taking a number apart into shorter ones whose products are
+// exact (Ozaki's error-free transformation, Henry, Tang and Heinecke's three bfloat16 for a float32). A float32 x is the sum of three bfloat16,
+// x = h + m + l, exactly (24 bits in three times 8; subnormal numbers too, see SPLIT_UP), and of the nine products of two such sums the six that matter are
+// multiplied: h h, h m, m h, m m, h l, l h. What is left out is 2.9e-7 (2^-21.7) of a product at the most, of either sign. v_mfma_f32_16x16x32_bf16
+// multiplies exactly and takes subnormal numbers: 32 k of all six occupy a SIMD for 96 cycles where the float32 instructions need 256.
 //
 // The order of the sums, the same in every kernel that uses this, whatever M, N, the kernel or the tile:
 //   k is cut into segments of 256 and these into blocks of 32; a block's six products are a chain of instructions from zero, the
@@ -10,9 +11,10 @@
 // So a row of A gives the same bits alone or inside any batch. Segments let few rows be split over waves; they also round less.
 // Against 64 bits (rms of the difference over rms of the result; normal entries, k = 2,048 / 8,192) 1.0e-7 / 1.6e-7, where chains of
 // fused multiply-adds over segments of 256 give 2.9e-7 / 3.1e-7; positive entries 4.9e-8 / 7.8e-8 and 9.0e-8 / 8.7e-8; entries
-// spread over e^(2 normal) 1.0e-7 / 1.5e-7 and 2.9e-7 / 3.3e-7.
+// spread over e^(2 normal) 0.9e-7 / 1.2e-7 and 2.7e-7 / 2.8e-7; k = 64 5.0e-8 and 1.4e-7, 8 3.8e-8 and 5.4e-8. A product alone (k = 1, or a row with one entry
+// that is not zero) 3.8e-8, some 3e-7 at the most, where one rounding is 2.5e-8 and 6e-8.
 //
-// An operand that is infinite, undefined or rounds to an infinite bfloat16, and a sum that overflows on the way, give a result that
+// An operand that is infinite, undefined or above some 2^112, and a sum above 2^96 on the way, give a result that
 // is not finite here, never a wrong finite one; such a result is formed once more in fused multiply-adds, by a whole wave: lane i takes
 // k = i, 64 + i, ..., and the lanes are added up by halves. What a row with an undefined number gives is undefined already, so that a row is
 // looked through once and then left. 1,021 x 16,384 x 2,048: 350 us, with a NaN in one row 345, in every row 484, an infinity in one row 948 (8,400 for one
@@ -30,26 +32,30 @@ struct Split8 {
   bf16x8 h, m, l;
 };
 
-// A lane's 8 numbers of a block: x its k = 4 kb .. + 3, y its 16 + 4 kb .. + 3. h is a row's (ROUND) number to the nearest (half away from
-// zero) or a column's cut off after 8 bits, m what is left cut off again, l the rest, which fits. One operand is enough to round: what is
-// left out of a product is then of either sign. Plain instructions, 5.5 a number: v_cvt_pk_bf16_f32 takes as long as three of them, and
-// v_dot2_f32_bf16, which takes h away in one, holds up the matrix instructions (a tile of 256 x 128 over k = 8,192 590 us with it, 500 so).
-template <bool ROUND>
+// What is split is x 2^16, exactly, so that l has a bfloat16 down to the smallest float32 there is (bfloat16 ends at 2^-133: without, numbers
+// below 2^-110 would lose bits); a product is therefore 2^32 too large, and every kernel takes that out of its last sum.
+#define SPLIT_UP 65536.0f
+#define SPLIT_DOWN 0x1p-32f
+
+// A lane's 8 numbers of a block: x its k = 4 kb .. + 3, y its 16 + 4 kb .. + 3. h is within 2^-7 of the number on either side of it (cut off after 8 bits
+// behind a factor of 1 + 3 2^-10, which costs nothing beside the one above), m what is left cut off again, l the rest, which fits. Plain
+// instructions, 6.5 a number: v_cvt_pk_bf16_f32 takes as long as three of them, and v_dot2_f32_bf16, which takes h away in one, holds up
+// the matrix instructions (a tile of 256 x 128 over k = 8,192 590 us with it, 500 so).
 __device__ __forceinline__ Split8 split8(const f32x4& x, const f32x4& y) {
 #pragma clang fp contract(off)   // x and y may be products, which are rounded before they are split
   Split8 s;
   uint32_t *h = reinterpret_cast<uint32_t*>(&s.h), *m = reinterpret_cast<uint32_t*>(&s.m), *l = reinterpret_cast<uint32_t*>(&s.l);
-  auto rest = [](float v, uint32_t near) { return v - __uint_as_float(near & 0xffff0000u); };
+  auto cut = [](uint32_t v) { return __uint_as_float(v & 0xffff0000u); };
   auto tops = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float a = i < 2 ? x[2 * i] : y[2 * i - 4], b = i < 2 ? x[2 * i + 1] : y[2 * i - 3];
-    const uint32_t na = __float_as_uint(a) + (ROUND ? 0x8000u : 0u), nb = __float_as_uint(b) + (ROUND ? 0x8000u : 0u);
-    const float ra = rest(a, na), rb = rest(b, nb);
+    const uint32_t na = __float_as_uint(a * (SPLIT_UP * (1 + 0x3p-10f))), nb = __float_as_uint(b * (SPLIT_UP * (1 + 0x3p-10f)));
+    const float ra = __builtin_fmaf(a, SPLIT_UP, -cut(na)), rb = __builtin_fmaf(b, SPLIT_UP, -cut(nb));
     const uint32_t ma = __float_as_uint(ra), mb = __float_as_uint(rb);
     h[i] = tops(na, nb);
     m[i] = tops(ma, mb);
-    l[i] = tops(__float_as_uint(rest(ra, ma)), __float_as_uint(rest(rb, mb)));
+    l[i] = tops(__float_as_uint(ra - cut(ma)), __float_as_uint(rb - cut(mb)));
   }
   return s;
 }

@@ -2,8 +2,10 @@
 
 float32 engine: the hand-written products of csrc/gemm_simple.hip, gemm_stream.hip
 and gemm_split.hip, whose every output element is summed in one order that depends
-on k alone. All 24 bits of both operands are multiplied (csrc/split.h); no library
-and no reduced-precision matrix mode is involved anywhere in that path.
+on k alone. Both operands enter with all 24 bits, as three bfloat16 each; of the
+nine products of these the three smallest, 2.9e-7 of a product at the most, are
+left out (csrc/split.h, which states the measured errors: below those of chains
+of fused multiply-adds from k = 8 on). No library is involved anywhere in that path.
 
 bfloat16 engine: the vendor library through ``torch.mm`` (the reference's
 engine also hands its products to a library: the external ``mat_mul`` operator,
