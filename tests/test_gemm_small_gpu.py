@@ -32,7 +32,7 @@ def _run(a, w):
 def test_powers_of_two_pass_through(m, n, k):
     a, w = _draw(m, n, k)
     plain = _run(a, w)
-    for ea, ew in ((-120, 90), (90, -120), (-126, 20), (-60, -60)):
+    for ea, ew in ((-120, 90), (90, -120), (-126, 70), (-45, -45)):          # the last bits of a product stay above 2^-149: chains round alike
         assert torch.equal(_run(a * 2.0 ** ea, w * 2.0 ** ew), plain * 2.0 ** (ea + ew)), (ea, ew)
 
 

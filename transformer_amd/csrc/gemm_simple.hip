@@ -2,7 +2,7 @@
 // 32-bit path, and the fallback for storage types and shapes that no faster kernel takes.
 //
 // Every output element is summed in one order that depends on K and the types alone, whatever M, N, the kernel or the tile, so
-// a row of A gives the same bits alone or inside any batch. float32 by float32: split.h's. With a bfloat16 operand the products go to
+// a row of A gives the same bits alone or inside any batch. float32 by float32: split.h's. With a bfloat16 operand, and over a k of up to 32, the products go to
 // the float32 matrix instructions, which are chains of fused multiply-adds: v_mfma_f32_16x16x4_f32 and v_mfma_f32_32x32x2_f32 give the
 // bits of fmaf over their 4 (2) k-slots in ascending order, denormals included. Then
 //   k is cut into segments of 256 and these into blocks of 16; a segment's chain starts at zero and takes
@@ -12,7 +12,7 @@
 //
 // gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk (float32): the same for
 // wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns. gemm_tiles (a bfloat16
-// operand): a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS. Many rows of float32 are gemm_split.hip's, up to 8 of a long
+// operand, or a short k): a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS. Many rows of float32 are gemm_split.hip's, up to 8 of a long
 // enough matrix gemm_stream.hip's, with the same bits.
 #include "gemm_split.h"
 #include "gemm_stream.h"
@@ -55,8 +55,9 @@ __device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
 // SHORT: k does not fill a round of segments. A wave then ends where k does instead of multiplying zeros to the end of
 // its segment: 40 x 5,000 x 64 6.3 us (21 without), 1 x 5,000 x 768 6.9 (10.6). The test between the chunks costs
 // long k 2 to 4 % (8 x 16,384 x 4,096 74.6 us without it, 77.3 with).
+// CHAIN: float32 products over a short k (SHORT_K).
 // Eight waves take float32 products of 9 to 32 rows over a k of 4,096 and more whose workgroups leave the CUs half empty.
-template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool SHORT, bool VEC>
+template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool SHORT, bool VEC, bool CHAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __restrict__ A, int lda,
                                                                    const TW* __restrict__ W, int ldw,
                                                                    const float* __restrict__ bias,
@@ -64,7 +65,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
                                                                    long long sa, long long sw, long long sc) {
   static_assert(!PAIR || RT == 1, "two segments in one tile");
   static_assert(BC % 2 == 0, "blocks of split.h in pairs of 16 k");
-  constexpr bool SPLIT = sizeof(T) == 4 && sizeof(TW) == 4;
+  constexpr bool SPLIT = sizeof(T) == 4 && sizeof(TW) == 4 && !CHAIN;
   A += (size_t)blockIdx.z * sa;
   W += (size_t)blockIdx.z * sw;
   C += (size_t)blockIdx.z * sc;
@@ -320,7 +321,7 @@ static void walk(hipStream_t stream, const float* A, int lda, const float* W, in
 #undef WALK
 }
 
-// Many rows with a bfloat16 operand, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
+// Many rows with a bfloat16 operand, or any over a short k, bound by the matrix cores (a 32x32x2 instruction occupies its SIMD for 64 cycles and wants 512
 // bytes of operands). 4 waves in 2 x 2 share a tile of 64 TT x 64 TT; each owns TT x TT tiles of 32 x 32. 32 k at a
 // time go through registers, where they become float32, and LDS, double buffered: row by row in 8 pieces of 16 bytes, permuted by the row
 // number so that the eight lanes that are served together meet no bank twice. Half h of a wave multiplies pieces h and h + 2 of a block's
@@ -447,6 +448,11 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
   }
 }
 
+// float32 products over a k up to this stay on the float32 matrix instructions: a chain of so few fused multiply-adds rounds less than
+// the split's left out products and last sums (k = 1 2.5e-8 and 3.8e-8, 2 3.1e-8 and 4.0e-8, 4 4.0e-8 and 3.7e-8; entries of very different size
+// up to k = 16; 32 1.0e-7 and 4.2e-8).
+#define SHORT_K 32
+
 template <typename T, typename TW, typename TC, bool VEC>
 static void launch(hipStream_t stream, const void* A_, int lda, long long sa, const void* W_, int ldw, long long sw,
                    const float* bias, void* C_, int ldc, long long sc, int M, int N, int K, int batch) {
@@ -454,24 +460,34 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
   const TW* W = (const TW*)W_;
   TC* C = (TC*)C_;
   constexpr bool F32 = sizeof(T) == 4 && sizeof(TW) == 4;
+  // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
+  // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
+  // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
+  // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
+  auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
+  if (tiles(64) >= 192 && (F32 ? K <= SHORT_K : M > 64 || K <= 128)) {
+    if (tiles(128) >= 384)
+      gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+    else
+      gemm_tiles_kernel<T, TW, TC, 1, VEC><<<dim3((N + 63) / 64, (M + 63) / 64, batch), 256, 0, stream>>>(
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+    return;
+  }
+#define FEW_(WAVES, RT, BC, PAIR, SHORT, CHAIN)                                                                \
+  gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, SHORT, VEC, CHAIN>                                      \
+      <<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch), WAVES * 64, 0, stream>>>( \
+          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
   if constexpr (F32) {
-    if (const int form = ta_gemm_split_form(M, N, K, lda, ldw, batch, VEC)) {
-      ta_gemm_split(stream, form, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch, VEC);
+    if (K <= SHORT_K) {
+      if (M <= 8) FEW_(4, 1, 4, true, true, true);
+      else if (M <= 16) FEW_(4, 1, 4, false, true, true);
+      else if (M <= 32) FEW_(4, 2, 2, false, true, true);
+      else FEW_(4, 4, 2, false, true, true);
       return;
     }
-  } else {
-    // A tile's time does not depend on how many there are, so few tiles are better cut along k (2,048 columns over
-    // k = 8,192: 128 rows 85 us by few rows where 64 tiles take 187, 256 rows 170 against 187, 512 rows 187 by tiles
-    // against 340). Tiles of 128 take two workgroups on every CU to fill. Over a short k it is the start and the end that
-    // count: tiles for any rows (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2).
-    auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
-    if (tiles(64) >= 192 && (M > 64 || K <= 128)) {
-      if (tiles(128) >= 384)
-        gemm_tiles_kernel<T, TW, TC, 2, VEC><<<dim3((N + 127) / 128, (M + 127) / 128, batch), 256, 0, stream>>>(
-            A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
-      else
-        gemm_tiles_kernel<T, TW, TC, 1, VEC><<<dim3((N + 63) / 64, (M + 63) / 64, batch), 256, 0, stream>>>(
-            A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc);
+    if (const int form = ta_gemm_split_form(M, N, K, lda, ldw, batch, VEC)) {
+      ta_gemm_split(stream, form, A, lda, sa, W, ldw, sw, bias, C, ldc, sc, M, N, K, batch, VEC);
       return;
     }
   }
@@ -480,14 +496,10 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
     }
-#define FEW_(WAVES, RT, BC, PAIR, SHORT)                                                                       \
-  gemm_few_rows_kernel<T, TW, TC, WAVES, RT, BC, PAIR, SHORT, VEC>                                             \
-      <<<dim3((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch), WAVES * 64, 0, stream>>>( \
-          A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
 #define FEW(WAVES, RT, BC, PAIR)                                                                               \
   do {                                                                                                         \
-    if (K <= (WAVES * (PAIR ? 2 : 1) - 1) * SEG) FEW_(WAVES, RT, BC, PAIR, true);                              \
-    else FEW_(WAVES, RT, BC, PAIR, false);                                                                     \
+    if (K <= (WAVES * (PAIR ? 2 : 1) - 1) * SEG) FEW_(WAVES, RT, BC, PAIR, true, false);                       \
+    else FEW_(WAVES, RT, BC, PAIR, false, false);                                                              \
   } while (0)
   // four waves a workgroup and 16 KB on their way in each: several workgroups share a CU and fill each other's
   // starts and ends (16,384 x 2,048 at 16 rows: 38 us; 44 with eight waves and twice the loads)

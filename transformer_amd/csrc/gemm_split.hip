@@ -323,7 +323,7 @@ int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool ve
   const long long tiles = split_tiles(SPLIT_SMALL, M, N) * batch;
   const bool brief = K <= 128;
   if (tiles > 2147483640ll || (M <= 16 && !brief)) return 0;
-  // over a short k it is the start and the end that count (1 x 16,384 x 16 3.8 us, 7.2 by few rows; 32 products of 1 x 512 x 64 4.4 against 7.2)
+  // over a short k it is the start and the end that count (32 products of 1 x 512 x 64 4.4 us, 7.2 by few rows); up to 32 it is not taken here at all
   if (brief) return tiles < 192 ? 0 : tiles < 2 * SPLIT_CUS ? SPLIT_SMALL : SPLIT_PAIRED;
   int best = 0;
   double least = split_few_cost(M, N, K, batch);
