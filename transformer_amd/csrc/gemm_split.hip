@@ -1,5 +1,6 @@
 // C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits for many rows, on the 16-bit matrix instructions (split.h, which also states the
 // order of the sums: a row has the bits here that it has in the kernels for few rows).
+#include <type_traits>
 #include "split.h"
 #include "gemm_split.h"
 
@@ -16,7 +17,9 @@ __device__ f32x4 split_zeros;      // where a piece past K is read from (never w
 // GLU: W holds gate rows, then up rows (N in all); every other 16 of the workgroup's columns are the ups of the 16 before, and C = silu(gate) * up. 1,021 rows x 8,192
 // channels x 2,048 302 us, product and activation in turn 316; 2,000 rows 600 and 651; 3,000 x 14,336 x 4,096 3,400 and 3,477. Where the product goes by other
 // tiles (513 rows) it is their difference that would be lost.
-template <int WAVES, int NT, int G, bool VEC, bool WHOLE, bool GLU = false>
+//
+// FAR: rows further apart than offsets of 32 bits reach, in size_t.
+template <int WAVES, int NT, int G, bool VEC, bool WHOLE, bool GLU = false, bool FAR = false>
 __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W,
                                                                     int ldw, const float* __restrict__ bias, float* __restrict__ C,
                                                                     int ldc, int M, int N, int K, long long sa, long long sw,
@@ -42,18 +45,19 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
   const int steps = (rounds - 1) * (SEG / 32) + last;
   const char* abase = reinterpret_cast<const char*>(A + (size_t)m0 * lda);
   const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw);
-  uint32_t aoff[MT], woff[BRING];                      // rows past M or N read another row and feed what is never stored
+  typedef typename std::conditional<FAR, size_t, uint32_t>::type Offset;
+  Offset aoff[MT], woff[BRING];                         // rows past M or N read another row and feed what is never stored
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const int m = wave * 16 * MT + 16 * i + r;
-    aoff[i] = ((uint32_t)(m0 + m < M ? m : M - 1 - m0) * lda + 4 * kb) * 4;
+    aoff[i] = ((Offset)(m0 + m < M ? m : M - 1 - m0) * lda + 4 * kb) * 4;
   }
 #pragma unroll
   for (int i = 0; i < BRING; ++i) {
     const int f = wave + WAVES * i < NT ? wave + WAVES * i : NT - 1, n = 16 * (GLU ? f / 2 : f) + r;
-    woff[i] = ((uint32_t)((n0 + n < n_out ? n : n_out - 1 - n0) + (GLU && f % 2 ? n_out : 0)) * ldw + 4 * kb) * 4;
+    woff[i] = ((Offset)((n0 + n < n_out ? n : n_out - 1 - n0) + (GLU && f % 2 ? n_out : 0)) * ldw + 4 * kb) * 4;
   }
-  auto piece = [&](const char* base, uint32_t off, int b, int h) {
+  auto piece = [&](const char* base, Offset off, int b, int h) {
     const char* p = base + (size_t)b * 128 + off + 64 * h;
     if (VEC) {
       if (!WHOLE) p = b * 32 + 16 * h + 4 * kb < K ? p : reinterpret_cast<const char*>(&split_zeros);
@@ -294,8 +298,8 @@ struct SplitForm {
   int waves, nt, groups;
   float us;
 };
-constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f}, {8, 8, 1, 2.5f}, {4, 6, 2, 2.45f}, {4, 4, 2, 1.7f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}, {2, 4, 1, 0.f}};
-enum { SPLIT_PAIRED = 5, SPLIT_SMALL = 6, SPLIT_CUS = 256 };
+constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f}, {8, 8, 1, 2.5f}, {4, 6, 2, 2.45f}, {4, 4, 2, 1.7f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}, {2, 4, 1, 0.f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}};
+enum { SPLIT_GROUPS = 4, SPLIT_PAIRED = 5, SPLIT_SMALL = 6, SPLIT_FAR = 3, SPLIT_CUS = 256 };      // + SPLIT_FAR: the same, rows any distance apart
 
 static long long split_tiles(int form, int M, int N) {
   const SplitForm& f = SPLIT_FORMS[form];
@@ -318,27 +322,26 @@ static double split_few_cost(int M, int N, int K, int batch) {
   return (double)((groups + SPLIT_CUS - 1) / SPLIT_CUS) * rounds * (M <= 32 ? 7.0 : rounds > 1 ? 10.5 : 7.5);
 }
 
-int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool vec) {
-  if (lda > 4194303 || ldw > 4194303) return 0;        // rows of a tile by 32-bit offsets
+extern "C" int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool vec) {
   const long long tiles = split_tiles(SPLIT_SMALL, M, N) * batch;
-  const bool brief = K <= 128;
+  const bool brief = K <= 128, far = lda > 4194303 || ldw > 4194303;     // 256 rows by 32-bit offsets
   if (tiles > 2147483640ll || (M <= 16 && !brief)) return 0;
   // over a short k it is the start and the end that count (32 products of 1 x 512 x 64 4.4 us, 7.2 by few rows); up to 32 it is not taken here at all
-  if (brief) return tiles < 192 ? 0 : tiles < 2 * SPLIT_CUS ? SPLIT_SMALL : SPLIT_PAIRED;
+  if (brief) return tiles < 192 ? 0 : far ? SPLIT_PAIRED + SPLIT_FAR : tiles < 2 * SPLIT_CUS ? SPLIT_SMALL : SPLIT_PAIRED;
   int best = 0;
   double least = split_few_cost(M, N, K, batch);
-  for (int f = vec ? 1 : SPLIT_PAIRED; f <= SPLIT_PAIRED; ++f) {
+  for (int f = !vec ? SPLIT_PAIRED : far ? SPLIT_GROUPS : 1; f <= SPLIT_PAIRED; ++f) {
     const double cost = split_cost(f, M, N, K, batch) + 4.0;
     if (cost < least) best = f, least = cost;
   }
-  return best;
+  return best && far ? best + SPLIT_FAR : best;
 }
 
 void ta_gemm_split(hipStream_t stream, int form, const float* A, int lda, long long sa, const float* W, int ldw, long long sw,
                    const float* bias, float* C, int ldc, long long sc, int M, int N, int K, int batch, bool vec) {
   const int tiles = (int)split_tiles(form, M, N), tiles_m = (M + 32 * SPLIT_FORMS[form].waves - 1) / (32 * SPLIT_FORMS[form].waves);
-#define RUN_(WAVES, NT, G, VEC, WHOLE)                                                                        \
-  gemm_split_kernel<WAVES, NT, G, VEC, WHOLE><<<dim3((tiles + 7) / 8 * 8, batch), WAVES * G * 64, 0, stream>>>( \
+#define RUN_(WAVES, NT, G, VEC, ...)                                                                          \
+  gemm_split_kernel<WAVES, NT, G, VEC, __VA_ARGS__><<<dim3((tiles + 7) / 8 * 8, batch), WAVES * G * 64, 0, stream>>>( \
       A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc, tiles_m, tiles)
 #define RUN(WAVES, NT, G)                              \
   if (K % SEG == 0) RUN_(WAVES, NT, G, true, true);    \
@@ -352,6 +355,11 @@ void ta_gemm_split(hipStream_t stream, int form, const float* A, int lda, long l
     case 3: RUN(4, 4, 2); break;
     case 4: RUN(2, 4, 4); break;
     case 5: RUN_ANY(4, 4, 1); break;
+    case SPLIT_GROUPS + SPLIT_FAR: RUN_(2, 4, 4, true, false, false, true); break;
+    case SPLIT_PAIRED + SPLIT_FAR:
+      if (vec) RUN_(4, 4, 1, true, false, false, true);
+      else RUN_(4, 4, 1, false, false, false, true);
+      break;
     default: RUN_ANY(2, 4, 1); break;
   }
 #undef RUN_ANY
