@@ -1,7 +1,7 @@
 """A launch that fails is an error of the call that made it."""
 import pytest
 import torch
-from ctypes import c_int, c_void_p
+from ctypes import c_float, c_int, c_void_p
 
 from transformer_amd import kernels
 
@@ -19,3 +19,17 @@ def test_a_float32_product_without_a_device_fails(M, N, K, streams):
     assert rc != 0
     # a product handed on returns what the one that took it returns: its check takes the error, a second one finds none
     assert lib.ta_last_error().startswith(b"ta_gemm_stream" if streams else b"ta_gemm_simple"), lib.ta_last_error()
+
+
+def test_more_rows_than_a_launch_holds_are_refused():
+    """Before anything is launched: rounding the rows up to whole tiles must not pass the largest number."""
+    lib = kernels.library()
+    at, zero = c_void_p(1 << 20), c_float(0.0)
+    for rows in (2147483393, 2147483647):
+        assert lib.ta_gemm_glu(None, at, c_int(64), at, c_int(64), None, at, c_int(8192), c_int(rows), c_int(8192), c_int(64), c_int(0), zero, zero, zero) != 0
+        assert lib.ta_last_error().startswith(b"ta_gemm_glu: M=%d" % rows), lib.ta_last_error()
+        assert lib.ta_gemm_plain(None, at, c_int(64), at, c_int(64), at, c_int(256), c_int(rows), c_int(256), c_int(64), c_int(0)) != 0
+        assert lib.ta_last_error().startswith(b"ta_gemm_plain: M=%d" % rows), lib.ta_last_error()
+        assert not lib.ta_gemm_split_glu_takes(c_int(rows), c_int(8192), c_int(2048), c_int(2048), c_int(2048))
+        assert lib.ta_gemm_split_glu(None, at, c_int(2048), at, c_int(2048), None, at, c_int(8192), c_int(rows), c_int(8192), c_int(2048)) != 0
+        assert lib.ta_last_error().startswith(b"ta_gemm_split_glu: M=%d" % rows), lib.ta_last_error()

@@ -259,7 +259,7 @@ extern "C" int ta_gemm_glu_pays(int M, int n, int K) {
 // and shift, else gelu (tanh) or silu.
 extern "C" int ta_gemm_glu(hipStream_t stream, const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc, int M,
                            int n, int K, int gelu, float limit, float slope, float shift) {
-  TA_REQUIRE(M >= 0 && n > 0 && n <= 1073741823 && n % 4 == 0 && K > 0 && K % 64 == 0, "ta_gemm_glu: M=%d n=%d K=%d", M, n, K);
+  TA_REQUIRE(M >= 0 && M <= 2147483392 && n > 0 && n <= 1073741823 && n % 4 == 0 && K > 0 && K % 64 == 0, "ta_gemm_glu: M=%d n=%d K=%d", M, n, K);
   TA_REQUIRE(lda >= K && ldw >= K && ldc >= n && lda % 8 == 0 && ldw % 8 == 0 && ldc % 4 == 0 && lda <= 4194304 && ldw <= 4194304 &&
                  ((uintptr_t)A | (uintptr_t)W) % 16 == 0 && (uintptr_t)C % 8 == 0,
              "ta_gemm_glu: rows of %d, %d, %d or their start", lda, ldw, ldc);

@@ -370,7 +370,7 @@ void ta_gemm_split(hipStream_t stream, int form, const float* A, int lda, long l
 // Whether ta_gemm_split_glu takes the products of M rows with gates and ups (float32, rows on 16 bytes): where the product alone goes by
 // tiles of 256 x 128.
 extern "C" int ta_gemm_split_glu_takes(int M, int di, int K, int lda, int ldw) {
-  return M > 16 && di > 0 && di <= 1073741823 && K % 4 == 0 && ((long long)di + 64) * ldw < 1 << 30 &&
+  return M > 16 && M <= 65535 * 64 && di > 0 && di <= 1073741823 && K % 4 == 0 && ((long long)di + 64) * ldw < 1 << 30 &&
          ta_gemm_split_form(M, 2 * di, K, lda, ldw, 1, true) == 1;
 }
 
