@@ -1,0 +1,20 @@
+"""Which prompts' products go to the kernels for many bfloat16 rows: not those at which the vendor library was measured to be faster."""
+import pytest
+
+from ctypes import c_int
+
+from transformer_amd import kernels
+
+
+def _glu(m, n, k):
+    return bool(kernels.library().ta_gemm_glu_pays(c_int(m), c_int(n), c_int(k)))
+
+
+@pytest.mark.parametrize("m,n,k,takes", [
+    (384, 14336, 4096, False), (385, 14336, 4096, True), (512, 14336, 4096, True), (513, 14336, 4096, False), (640, 14336, 4096, False), (641, 14336, 4096, True),
+    (641, 8192, 4096, False), (768, 8192, 8192, False), (769, 8192, 4096, True), (700, 11008, 4096, True), (512, 8192, 4096, True),       # 192 tiles in three rows
+    (1025, 8192, 2048, False), (1280, 8192, 2048, False), (1281, 8192, 2048, True), (1100, 8192, 4096, True), (1024, 8192, 2048, True),    # a quarter of a second round
+    (1025, 14336, 2048, True), (8192, 16384, 2048, False), (8192, 16384, 4096, True), (1536, 16384, 2048, True), (7900, 16384, 2048, True),  # whole rounds only
+    (2048, 16384, 2048, False), (2011, 14336, 4096, True), (5000, 7996, 4096, False), (5000, 8002, 4096, False), (5000, 8192, 1984, False), (5000, 8192, 4100, False)])
+def test_gated(m, n, k, takes):
+    assert _glu(m, n, k) == takes

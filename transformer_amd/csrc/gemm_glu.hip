@@ -2,6 +2,7 @@
 // v_mfma_f32_16x16x32_bf16. The product with the activation behind it moves [M, 2 n] to memory and back; here gate and up of a channel meet in
 // a lane's registers, in float32.
 //
+// The schedule is the published one of eight waves on this chip, two to a SIMD that take turns at reading and multiplying ("ping-pong").
 // A workgroup of 8 waves, alone on its CU, owns 256 rows x 128 channels, wave (wm, wn) 128 rows and 32 channels of either kind in four quarters
 // of 64 x 32. 64 k of the operands lie in LDS, row by row in 8 pieces of 16 bytes, permuted by the row so that the lanes that are
 // served together meet no bank twice; they get there without passing through registers, in halves of 128 rows. A step of 64 k is four phases,
@@ -246,13 +247,21 @@ __global__ __launch_bounds__(512, 2) void gemm_glu_kernel(GluArgs p) {
 
 enum { GLU_CUS = 256 };
 
-// Where it gains over the library's product and the activation's kernel (us there and here), measured from 65 to 7,500 rows: wide matrices, except where
-// the last row of tiles is all but empty and there are few others. 14,336 channels over k = 4,096: 384 rows 88 / 93, 400 105 / 100, 512 105 / 102, 520 142 / 151, 640 148 /
-// 156, 700 161 / 156, 1,100 244 / 237, 2,060 399 / 384, 3,100 698 / 558, 7,500 1,361 / 1,271; 11,008 over 4,096: 512 88 / 92, 700 154 / 143, 1,600 339 / 251; 8,000 over 4,096: 449 68 / 65,
-// 1,281 250 / 153, 7,500 883 / 721; 8,192 over 2,048: 449 44 / 37, 1,030 84 / 85, 1,152 87 / 87, 2,011 123 / 117, 4,400 328 / 257; 28,672 over 8,192: 700 557 / 534, 2,060 1,442 / 1,447, 5,300 3,444 /
-// 3,392. Fewer channels either way: 5,632 over 2,048: 576 38 / 50, 830 55 / 47, 1,281 74 / 83, 2,011 98 / 94.
+// Where it gains over the library's product (hipBLASLt of ROCm 7) and the activation's kernel: wide matrices, by how full the rounds of tiles are. Measured at 76 numbers of
+// rows from 385 to 8,192 by 12 matrices (8,000 to 28,672 channels, k from 2,048 to 8,192), where it takes 1.11 times less in the mean. us there and here:
+//   two rows of tiles of which the second is over half full, and three or more: 14,336 channels over 4,096: 512 rows 105 / 102, 700 161 / 156, 1,100 244 / 237, 2,060 399 / 384,
+//   3,100 698 / 558, 7,500 1,361 / 1,271; 11,008 over 4,096: 700 154 / 143, 1,600 339 / 251; 8,000 over 4,096: 1,281 250 / 153; 22,016 over 4,096: 1,900 1.24 times.
+//   513 to 640 rows, whose third row of tiles is the half form's, lose 2 to 12 % at most widths (but gain 26 to 36 % at 22,016, 5 at 11,008);
+//   641 to 768 rows whose tiles leave a quarter of the CUs idle: 8,192 over 4,096 0.94 to 0.97 times, over 8,192 0.97 to 1.01 (8,000 over 4,096 would gain 2 to 8 %);
+//   over k below 4,096 a second round of up to a quarter (8,192 over 2,048: 1,025 to 1,100 rows 0.94 to 0.98, 1,152 to 1,280 1.00 to 1.03), and whole rounds only,
+//   four and more of them (16,384 over 2,048: 2,560 rows 0.98, 4,096 0.97, 5,632 0.96, 7,500 0.95, 8,192 0.90; 8,192 over 2,048 and 14,336 over 2,048: 8,192 rows 0.99, 1.00).
+// The worst that is left of 837: 11,008 over 4,096 769 rows 0.94 (145 / 154; 780 0.99, 820 1.06), 8,192 over 4,096 1,100 rows 0.96, 14,336 over 4,096 1,040 rows 0.97;
+// 400 rows, 28,672 over 8,192 at 2,060 and the like are ties. Fewer channels go either way: 5,632 over 2,048: 576 38 / 50, 830 55 / 47, 1,281 74 / 83, 2,011 98 / 94.
 extern "C" int ta_gemm_glu_pays(int M, int n, int K) {
-  return ((M > 384 && M <= 512) || M > 640) && n >= 8000 && n % 4 == 0 && K >= 2048 && K % 64 == 0;
+  if (M <= 384 || (M > 512 && M <= 640) || n < 8000 || n % 4 != 0 || K < 2048 || K % 64 != 0) return 0;
+  const long long tiles = ((long long)M + 255) / 256 * ((n + 127) / 128), rest = tiles % GLU_CUS;
+  if (M > 512 && M <= 768 && tiles <= 192) return 0;
+  return K >= 4096 || !((tiles > GLU_CUS && tiles <= GLU_CUS + GLU_CUS / 4) || (rest == 0 && tiles >= 4 * GLU_CUS));
 }
 
 // C [M, n] = act(A W[:n]^T + bias[:n]) * (A W[n:]^T + bias[n:]); the activation as in ta_gemm_mid: a limit above 0 the limited form with its slope
