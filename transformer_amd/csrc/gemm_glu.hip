@@ -286,15 +286,20 @@ extern "C" int ta_gemm_glu(hipStream_t stream, const void* A, int lda, const voi
 
 // The same as a plain product with a float32 result. It is the library's equal while it multiplies (and sums in the same order except where that one cuts k);
 // it gains where its rounds are full, and where the library cuts its last round along k and falls to half. us there and here (the product added to the stream):
-// 4,096 columns over k = 14,336: 1,600 rows 333 / 182, 2,011 195 / 199, 2,502 0.83 times the library's rate, 3,164 501 / 289, 3,400 309 / 295, 4,000 335 / 322, 4,500 424 / 473, 5,640 753 / 494, 8,159 676 / 653; over 8,192 3,274 1.06, 3,853
-// 1.04; over 4,096 3,400 106 / 101, 4,000 112 / 110, but 8,159 216 / 224; 8,192 columns over 14,336: 1,573 328 / 303, 2,868 720 / 524; 5,120 over 14,336: 1,166 321 / 171,
-// 4,829 814 / 525; over 4,096 2,942 108 / 104. Rounds that end nearly half full gain for a long k alone, more than two rounds nowhere, results in bfloat16 lose 3 to 5 % (5,000 rows x 6,144 over
-// 4,096 182 / 194).
+// 4,096 columns over k = 14,336: 1,600 rows 333 / 182, 2,502 0.83 times the library's rate, 3,164 501 / 289, 3,400 309 / 295, 4,000 335 / 322, 4,500 424 / 473, 5,640 753 / 494; over
+// 4,096 3,400 106 / 101, 4,000 112 / 110, but 8,159 216 / 224; 8,192 columns over 14,336: 1,573 328 / 303; 5,120 over 14,336: 1,166 321 / 171, 4,829 814 / 525; over 4,096 2,942 108 / 104.
+// Measured anew at 23 matrices, k = 4,096, 5,120, 8,192, 11,008, 12,288, 12,352, 13,824, 14,336, 16,384, 20,480 and 28,672, at up to 54 numbers of rows each. Two rounds or less, over a long k:
+//   full or from 208 tiles on: 0.98 to 1.75 times, mostly 1.03 (where the library keeps up) or 1.6 (where it falls); three rounds gain nowhere;
+//   nearly half full, 100 to 128 tiles: 1.0 to 1.9; 96 to 128 as the second round: 1.0 to 1.84, but 8,192 columns over 28,672 0.95 to 0.98; 96 alone 0.77 to 0.98, whatever
+//   the width; 128 over k above 12,288 0.98 (2,011 x 4,096 x 14,336 195 / 199).
+// Over k below 8,192 one nearly full round: 1.00 to 1.06 added, 1.05 to 1.09 stored (16,384 columns over 4,096 0.97 and 0.98). Results in bfloat16 lose 3 to 5 % (5,000 rows x 6,144 over 4,096 182 / 194).
 extern "C" int ta_gemm_plain_pays(int M, int n, int K) {
   if (M < 512 || n % 256 != 0 || K % 64 != 0 || K < 4096) return 0;
-  const long long tiles = (long long)(M + 255) / 256 * (n / 256), rest = tiles % GLU_CUS;
-  if (K < 8192) return tiles >= 208 && tiles <= GLU_CUS;
-  return tiles <= 2 * GLU_CUS && (rest == 0 || rest >= 208 || (rest >= 96 && rest <= (K <= 12288 ? 128 : 120)));
+  const long long tiles = ((long long)M + 255) / 256 * (n / 256), rest = tiles % GLU_CUS;
+  if (K < 8192) return n <= 8192 && tiles >= 208 && tiles <= GLU_CUS;
+  if (tiles > 2 * GLU_CUS) return 0;
+  if (rest == 0 || rest >= 208) return 1;
+  return rest >= (tiles < GLU_CUS ? 100 : 96) && rest <= (K <= 12288 ? 128 : 120) && (n < 8192 || K <= 14336);
 }
 
 // C [M, n] = A W^T, or C += A W^T, float32.
