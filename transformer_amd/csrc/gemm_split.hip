@@ -290,16 +290,20 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
   });
 }
 
-// us a step of 32 k (of all groups) when every CU has its workgroups: measured at 130 to 3,000 rows of 2,048 to 16,384 columns, k = 2,048
-// and 8,192. 256 x 128 reads and splits least per product but leaves CUs idle where there are few tiles: 1,021 x 16,384 x 2,048 330 to 380 us there,
-// 427 by 128 x 64, 483 by 128 x 96; 1,021 x 3,072 x 2,048 149, 107 and 82. Groups fill a CU that has a tile to itself: 1,021 x 2,048 x 8,192 268
-// by one group, 214 by two; 300 x 2,048 x 8,192 264, 187 and by four groups on 64 x 64 127. Two workgroups of 128 x 64 with one group share a CU.
+// us a step of 32 k (of all groups) and us a round of workgroups beside its steps, when every CU has one: fitted to all forms at 7 to 3,000 rows of 2,048 to 28,672
+// columns, k from 256 to 14,336, to 5 to 8 %. 256 x 128 reads and splits least per product but leaves CUs idle where there are few tiles: 16,384 x 2,048 at 1,021 rows
+// 310 us there and 390 by 128 x 64, at 130 rows 132 and 105; 4,096 x 1,024 at 700 rows 70 and 51. Groups fill a CU that has a tile to itself: 2,048 x 8,192 at 1,021 rows 214 us by two,
+// 6,144 x 8,192 at 64 rows 248 by one, 172 by two, 129 by four on 64 x 64. Two workgroups of 128 x 64 with one group share a CU.
+// Of 800 sizes the costs choose the fastest form to 0.6 % in the mean, 18 at the worst (8,192 x 1,024 at 33 rows: 21 us for 18).
 struct SplitForm {
   int waves, nt, groups;
-  float us;
+  float step, round;
 };
-constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f}, {8, 8, 1, 2.5f}, {4, 6, 2, 2.45f}, {4, 4, 2, 1.7f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}, {2, 4, 1, 0.f}, {2, 4, 4, 2.1f}, {4, 4, 1, 1.67f}};
+constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f, 0.f},      {8, 8, 1, 1.96f, 6.4f}, {4, 6, 2, 1.91f, 5.1f}, {4, 4, 2, 1.43f, 3.6f}, {2, 4, 4, 1.96f, 3.7f},
+                                     {4, 4, 1, 1.47f, 3.1f}, {2, 4, 1, 0.f, 0.f},    {2, 4, 4, 1.96f, 3.7f}, {4, 4, 1, 1.47f, 3.1f}};
 enum { SPLIT_GROUPS = 4, SPLIT_PAIRED = 5, SPLIT_SMALL = 6, SPLIT_FAR = 3, SPLIT_CUS = 256 };      // + SPLIT_FAR: the same, rows any distance apart
+#define SPLIT_LAUNCH 2.0        // us of a launch
+#define SPLIT_ALONE 0.94        // us a step of a SPLIT_PAIRED workgroup that has its CU to itself
 
 static long long split_tiles(int form, int M, int N) {
   const SplitForm& f = SPLIT_FORMS[form];
@@ -309,17 +313,19 @@ static double split_cost(int form, int M, int N, int K, int batch) {
   const SplitForm& f = SPLIT_FORMS[form];
   const long long tiles = split_tiles(form, M, N) * batch;
   const int segs = (K + SEG - 1) / SEG, steps = f.groups == 1 ? (K + 31) / 32 : (segs + f.groups - 1) / f.groups * (SEG / 32);
-  if (form != SPLIT_PAIRED) return (double)((tiles + SPLIT_CUS - 1) / SPLIT_CUS) * steps * f.us;
-  const long long rest = tiles % (2 * SPLIT_CUS);      // alone on its CU a workgroup takes 1.05 us a step
-  return (tiles / (2 * SPLIT_CUS) * f.us + (rest > SPLIT_CUS ? f.us : rest > 0 ? 1.05f : 0.f)) * steps;
+  const double round = (double)steps * f.step + f.round;
+  if (form != SPLIT_PAIRED) return SPLIT_LAUNCH + (double)((tiles + SPLIT_CUS - 1) / SPLIT_CUS) * round;
+  const long long rest = tiles % (2 * SPLIT_CUS);
+  return SPLIT_LAUNCH + (double)(tiles / (2 * SPLIT_CUS)) * round + (rest > SPLIT_CUS ? round : rest > 0 ? SPLIT_ALONE * steps + f.round : 0.0);
 }
 
-// the few-rows kernel's: a workgroup of 16 columns and 32 or 64 rows, four segments at a time
+// the few-rows kernel's: a workgroup of 16 columns and 32 or 64 rows, four segments at a time (12 % off in the mean). Over a short k several of its workgroups
+// share a CU evenly.
 static double split_few_cost(int M, int N, int K, int batch) {
-  const int rows = M <= 32 ? 32 : 64;
+  const int rows = M <= 32 ? 32 : 64, segs = (K + SEG - 1) / SEG;
   const long long groups = (long long)((N + 15) / 16) * ((M + rows - 1) / rows) * batch;
-  const int rounds = (K + 4 * SEG - 1) / (4 * SEG);
-  return (double)((groups + SPLIT_CUS - 1) / SPLIT_CUS) * rounds * (M <= 32 ? 7.0 : rounds > 1 ? 10.5 : 7.5);
+  const double share = segs > 4 ? (double)((groups + SPLIT_CUS - 1) / SPLIT_CUS) : groups / (double)SPLIT_CUS;
+  return 5.6 + (M <= 32 ? 5.1 : 8.4) * (share > 0.67 ? share : 0.67) * (segs < 4 ? segs / 4.0 : (segs + 3) / 4);
 }
 
 extern "C" int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool vec) {
@@ -331,7 +337,7 @@ extern "C" int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int bat
   int best = 0;
   double least = split_few_cost(M, N, K, batch);
   for (int f = !vec ? SPLIT_PAIRED : far ? SPLIT_GROUPS : 1; f <= SPLIT_PAIRED; ++f) {
-    const double cost = split_cost(f, M, N, K, batch) + 4.0;
+    const double cost = split_cost(f, M, N, K, batch);
     if (cost < least) best = f, least = cost;
   }
   return best && far ? best + SPLIT_FAR : best;
