@@ -47,8 +47,8 @@ __device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
 // of RT rows of A, which are operands as they are (a row's four lanes cover 64
 // bytes); while one chunk of BC blocks is multiplied the next is on its way. The waves take the segments in
 // turn and leave the partial tiles in LDS, where they are added in ascending order after every round.
-// float32, 2,048 columns over k = 8,192 at 9 / 16 / 32 / 64 rows 31 / 37 / 54 / 84 us (30 / 35 / 51 / 84 on the float32 matrix instructions:
-// from 32 rows on it is the splitting of A, once more for every 16 columns, that binds), 3,072 x 2,048 at 32 / 64 rows 15.2 / 21.8.
+// float32, 2,048 columns over k = 8,192 at 9 / 16 / 32 / 64 rows 32 / 38 / 55 / 85 us (31 / 36 / 52 / 86 on the float32 matrix instructions:
+// from 32 rows on it is the splitting of A, once more for every 16 columns, that binds), 3,072 x 2,048 at 32 / 64 rows 15.6 / 24.0.
 // PAIR (up to 8 rows): a matrix instruction multiplies two segments side by side, 8 columns of W each, of
 // whose 16 x 16 products the two squares on the diagonal are used. A workgroup then owns 8 columns: a matrix of
 // 2,048 rows keeps 256 CUs reading instead of 128.

@@ -6,8 +6,9 @@
 // 16 runs of 256 bytes, 4 KB, and every wave has a ring of its own of such chunks, up to 128 KB a CU on their way, that is
 // asked for across the ends of tiles. Operand layout straight from memory (gemm_walk, gemm_few_rows) touches half a line per row and
 // instruction: at 4 rows 16,384 x 2,048 gated 28.2 us there and 24.9 here (5.4 TB/s), 28,672 x 4,096 gated 88 and 80, 2,048 x 8,192 19.2 and 15.4,
-// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55 (on the float32 matrix instructions; splitting the operands costs a kernel 0.2 to 0.5
-// us more at its start and end: the four products of a layer of width 2,048 and 8,192, 1 / 4 / 8 rows, 57.6 / 60.2 / 64.3 us and 59.7 / 61.3 / 64.6).
+// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55 (on the float32 matrix instructions). Splitting the operands costs a kernel 0.3 to 0.9 us more
+// than those, in front of the first product and behind the last chunk: the four products of a layer of width 2,048 and 8,192 (3,072 and 2,048 x 2,048, 16,384 x 2,048 gated,
+// 2,048 x 8,192) at 1 / 4 / 8 rows 54.3 / 55.9 / 58.6 us and 56.7 / 57.7 / 60.6; it is what keeps a row's bits the same as among many, which gain more.
 //
 // A product may take the RMS norm in front of it (its workgroups form the rows' factors once more each, which costs 1 to 3 us
 // where the norm's own launch costs 4 to 5), and add its result to the residual stream where it stores it.
@@ -141,12 +142,18 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[i][e] = a[i][e] * rstd * g[i][e];
   }
-  Split8 as[CH * 2];                             // A, split where the first tile needs it
+  Split8 as[CH * 2];                             // A, split in front of the first tile's chunks
   int slot = 0, turn = 0;
   auto multiply = [&](int tile, bool first) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
+      if (first) {                               // while the chunk is on its way
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) as[2 * c + i] = split8(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       ta_wait_loads<(PF - 1) * 4>();
       f32x4 w[4];
 #pragma unroll
@@ -157,7 +164,6 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
       slot = slot + 1 == PF ? 0 : slot + 1;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        if (first) as[2 * c + i] = split8(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
         acc += split_block(split8(w[2 * i], w[2 * i + 1]), as[2 * c + i]);
       }
     }
