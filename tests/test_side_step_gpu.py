@@ -1,4 +1,4 @@
-"""The end of a block with a token side input in one kernel: against its kernels one by one, for a plain result in planes and for experts' rows,
+"""The end of a block with a token side input in one kernel: against its kernels one by one and against 64 bits, for a plain result in planes and for experts' rows,
 at the widths, side columns and numbers of tokens that it takes."""
 import pytest
 import torch
@@ -23,6 +23,25 @@ def _one_by_one(x, delta, w, eps, gate, side, proj, v, eps_side, w_next, eps_nex
     out = torch.empty(x.shape, device="cuda", dtype=torch.bfloat16)
     kernels.postnorm_add(x, y, v, eps_side, next_weight=w_next, next_eps=eps_next, out=out)
     return before, x, out
+
+
+def _exact(x, given, w, eps, gate, side, proj, v, eps_side, w_next, eps_next):
+    """In 64 bits from the operands on, nothing rounded: what the result's own add gives, the stream behind both, the next norm."""
+    norm = lambda t, gain, e: t * (t.square().mean(1, keepdim=True) + e).rsqrt() * gain.double()
+    if isinstance(given, kernels.RoutedRows):
+        g = given
+        pairs = g.pair_row.view(x.shape[0], g.top).long()
+        parts = torch.where((pairs >= 0)[..., None], g.rows.double()[pairs.clamp_min(0)], 0.0)
+        delta = (parts if g.weight is None else parts * g.weight.double()[..., None]).sum(1)
+        if g.shared is not None:
+            shared = g.shared.double() if g.shared.dim() == 2 else g.shared.double().sum(0)
+            delta = delta + (shared if g.shared_gate is None else shared * torch.sigmoid(g.shared_gate.double()))
+    else:
+        delta = given.double() if given.dim() == 2 else given.double().sum(0)
+    before = x.double() + norm(delta, w, eps)
+    g = torch.nn.functional.gelu(before @ gate.double().t(), approximate="tanh") * side.double()
+    after = before + norm(g @ proj.double().t(), v, eps_side)
+    return before, after, norm(after, w_next, eps_next)
 
 
 @pytest.mark.parametrize("nt,d,dim,kind", [(1, 512, 32, "plain"), (4, 2048, 64, "routed"), (64, 1024, 128, "routed"), (7, 4096, 64, "planes"),
@@ -51,6 +70,15 @@ def test_side_step(nt, d, dim, kind):
     assert bool(((got - want).norm(dim=1) <= 2.0 ** -8 * added + 1e-5 * want.norm(dim=1)).all())
     assert bool(((out.float() - want_out.float()).norm(dim=1) <= 2.0 ** -7 * want_out.float().norm(dim=1)).all())
     assert torch.equal(kernels.side_step(x0.clone(), given, *args[:-2]), got)          # without a norm behind it
+    # against 64 bits: the rows' and the gated columns' bfloat16 copies are 2^-9 off at the most each, and so is what the side input adds, in the
+    # norm over a row; the rest is 32 bits, and the next norm's rows are rounded once more
+    exact_before, exact, exact_out = _exact(x0, given, *args)
+    added = (exact - exact_before).norm(dim=1)
+    bound = 2.0 ** -8 * added + 1e-6 * exact.norm(dim=1)
+    assert bool(((got.double() - exact).norm(dim=1) <= bound).all())
+    assert bool(((out.double() - exact_out).norm(dim=1) <= (2.0 ** -9 + bound / exact.norm(dim=1)) * 1.01 * exact_out.norm(dim=1)).all())
+    # and no further from them than the kernels one by one, but for the closeness of two roundings
+    assert float((got.double() - exact).norm()) <= 1.5 * float((want.double() - exact).norm())
 
 
 def test_who_takes_it_and_what_it_refuses():
