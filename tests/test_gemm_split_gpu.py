@@ -8,13 +8,12 @@ from transformer_amd import kernels
 
 pytestmark = pytest.mark.gpu
 
-# form: rows, columns, k. 1: 256 x 128; 2, 3: 128 x 96 and 128 x 64 by two groups; 4: 64 x 64 by four; 5: 128 x 64, 6: 64 x 64 by one (short k); 0: the last number of
-# rows that stay with few rows. Of each form k of whole segments (which is code of its own), of whole blocks, ending inside a block, inside the segment of a later
+# form: rows, columns, k. 1: 256 x 128; 2, 3: 128 x 96 and 128 x 64 by two groups; 4: 64 x 64 by four; 5: 128 x 64, 6: 64 x 64 by one (short k); 0: few rows. Of each form k of whole segments (which is code of its own), of whole blocks, ending inside a block, inside the segment of a later
 # group, an odd number of blocks, and where a form takes them numbers of k that are no multiple of 4
 SHAPES = [(1, 1021, 4100, 512), (1, 1021, 16384, 512), (1, 1021, 8192, 2048), (1, 513, 16387, 264), (2, 1000, 3070, 1024), (2, 1021, 3000, 2048), (2, 900, 2050, 1796),
           (3, 1021, 2044, 2048), (3, 200, 5000, 1536), (3, 1021, 2044, 2044), (3, 500, 4090, 1300), (4, 130, 4100, 2048), (4, 130, 4100, 2000), (4, 40, 16000, 1540),
-          (4, 300, 2047, 772), (5, 700, 5000, 1024), (5, 257, 9000, 1292), (5, 129, 3000, 1056), (5, 65, 16400, 516), (5, 300, 9001, 1291), (5, 1100, 5570, 68),
-          (5, 1100, 5570, 67), (6, 3, 12300, 128), (6, 70, 12290, 36), (6, 70, 12290, 37), (0, 17, 33000, 2048)]
+          (4, 129, 3000, 1056), (5, 700, 5000, 1024), (5, 257, 9000, 1292), (5, 300, 9001, 1291), (5, 1100, 5570, 68), (5, 1100, 5570, 67), (5, 70, 12290, 36),
+          (2, 65, 16400, 516), (6, 300, 12290, 128), (6, 300, 12290, 127), (4, 300, 2047, 772), (0, 3, 12300, 128), (0, 17, 33000, 2048)]
 
 
 def _draw(m, n, k):

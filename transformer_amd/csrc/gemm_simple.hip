@@ -10,7 +10,7 @@
 //   segments' sums are added in ascending order.
 // The order inside a block is the one in which a lane that has read 4 consecutive k holds them: no operand is turned round.
 //
-// gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn. gemm_walk (float32): the same for
+// gemm_few_rows: 16 columns a workgroup, whose waves take segments in turn; gemm_blocks: blocks of a short k. gemm_walk (float32): the same for
 // wide matrices over a k of up to 4,096, where a workgroup keeps its rows of A and walks along the columns. gemm_tiles (a bfloat16
 // operand, or a short k): a tile of 128 x 128 or 64 x 64 a workgroup, operands through LDS. Many rows of float32 are gemm_split.hip's, up to 8 of a long
 // enough matrix gemm_stream.hip's, with the same bits.
@@ -52,11 +52,11 @@ __device__ __forceinline__ f32x4 load_piece(const T* row, int k, int K) {
 // PAIR (up to 8 rows): a matrix instruction multiplies two segments side by side, 8 columns of W each, of
 // whose 16 x 16 products the two squares on the diagonal are used. A workgroup then owns 8 columns: a matrix of
 // 2,048 rows keeps 256 CUs reading instead of 128.
-// SHORT: k does not fill a round of segments. A wave then ends where k does instead of multiplying zeros to the end of
+// SHORT: k does not fill a round of segments, or leaves half of the last one empty. A wave then ends where k does instead of multiplying zeros to the end of
 // its segment: 40 x 5,000 x 64 6.3 us (21 without), 1 x 5,000 x 768 6.9 (10.6). The test between the chunks costs
 // long k 2 to 4 % (8 x 16,384 x 4,096 74.6 us without it, 77.3 with).
 // CHAIN: float32 products over a short k (SHORT_K).
-// Eight waves take float32 products of 9 to 32 rows over a k of 4,096 and more whose workgroups leave the CUs half empty.
+// Four waves a workgroup, or eight (few_rows_waves).
 template <typename T, typename TW, typename TC, int WAVES, int RT, int BC, bool PAIR, bool SHORT, bool VEC, bool CHAIN>
 __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __restrict__ A, int lda,
                                                                    const TW* __restrict__ W, int ldw,
@@ -169,6 +169,89 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_few_rows_kernel(const T* __re
     }
     if (!own) continue;
     C[(size_t)m * ldc + n] = from_f32<TC>(bias ? total[e] + bias[n] : total[e]);
+  }
+}
+
+// Few rows over a k of up to 512 (up to 8 rows 1,280), float32: gemm_few_rows' tiles with the waves on blocks of 32 k instead of segments, so that a k of few segments
+// has all of them at work (splitting doubles what a wave has to do for a block, which a wave alone on its SIMD cannot hide).
+// Every block's tile goes to LDS (up to 64 KB), where a segment's blocks and the segments are added up in their order: the bits are the same. us of
+// gemm_few_rows on the float32 instructions, on the split and here: 2,048 x 256 at 4 / 16 / 32 / 64 rows 4.8 / 4.9 / 6.0 / 8.4, 5.7 / 5.8 / 7.4 / 10.1 and 4.3 / 4.6 / 5.3 / 7.1; 16,384 x 128 at
+// one row 7.0, 8.6, 5.3; 512 x 512 at 8 rows 4.9, 5.7, 4.7; 2,048 x 1,024 at one row 5.6, 6.4, 5.5.
+template <int WAVES, int RT, bool PAIR, bool VEC>
+__global__ __launch_bounds__(WAVES * 64) void gemm_blocks_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+                                                                 const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N,
+                                                                 int K, long long sa, long long sw, long long sc) {
+  static_assert(!PAIR || RT == 1, "two blocks in one tile");
+  A += (size_t)blockIdx.z * sa;
+  W += (size_t)blockIdx.z * sw;
+  C += (size_t)blockIdx.z * sc;
+  constexpr int COLS = PAIR ? 8 : 16, ROWS = PAIR ? 8 : 16 * RT, OUT = (ROWS * COLS + WAVES * 64 - 1) / (WAVES * 64);
+  constexpr int SIDE = PAIR ? 2 : 1;             // blocks that a matrix instruction multiplies side by side
+  extern __shared__ __attribute__((aligned(16))) float part[];       // [blocks, rounded up to SIDE][ROWS * COLS]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TA_WAVE), lane = threadIdx.x % TA_WAVE;
+  const int r = lane % 16, kb = lane / 16;
+  const int n0 = blockIdx.x * COLS, m0 = blockIdx.y * ROWS;
+  // rows past N or M read another row and feed outputs that are never stored
+  const float* wrow = W + (size_t)(n0 + r % COLS < N ? n0 + r % COLS : N - 1) * ldw;
+  const float* arow[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int m = m0 + 16 * i + r % (PAIR ? 8 : 16);
+    arow[i] = A + (size_t)(m < M ? m : m0) * lda;
+  }
+  const int blocks = (K + 31) / 32, steps = (blocks + SIDE - 1) / SIDE;
+  f32x4 w[2][2], a[2][RT][2];
+  auto load = [&](int set, int step) {
+    const int k0 = (step * SIDE + (PAIR ? r / 8 : 0)) * 32 + 4 * kb;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      w[set][h] = load_piece<float, VEC, (RT < 4)>(wrow, k0 + 16 * h, K);
+#pragma unroll
+      for (int t = 0; t < RT; ++t) a[set][t][h] = load_piece<float, VEC, false>(arow[t], k0 + 16 * h, K);
+    }
+  };
+  auto multiply = [&](int set, int step) {
+    const Split8 ws = split8(w[set][0], w[set][1]);
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      // a lane holds columns 4 kb .. + 3 of row r; of two blocks side by side the two squares on the diagonal are used
+      const f32x4 c = split_block(ws, split8(a[set][t][0], a[set][t][1]));
+      if (!PAIR) *reinterpret_cast<f32x4*>(&part[(step * RT + t) * 256 + r * 16 + 4 * kb]) = c;
+      else if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&part[(step * 2 + r / 8) * 64 + r % 8 * 8 + 4 * (kb % 2)]) = c;
+    }
+  };
+  load(0, wave);
+  for (int s = wave; s < steps; s += 2 * WAVES) {
+    load(1, s + WAVES);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0, s);
+    if (s + WAVES >= steps) break;
+    load(0, s + 2 * WAVES);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1, s + WAVES);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < OUT; ++e) {
+    const int at = (int)threadIdx.x + WAVES * 64 * e;
+    if (OUT * WAVES * 64 > ROWS * COLS && at / TA_WAVE * TA_WAVE >= ROWS * COLS) continue;       // whole waves
+    float total = 0.f;
+    for (int b0 = 0; b0 < blocks; b0 += SEG / 32) {
+      float sum = 0.f;
+      if (b0 + SEG / 32 <= blocks) {
+#pragma unroll
+        for (int b = 0; b < SEG / 32; ++b) sum += part[(b0 + b) * ROWS * COLS + at];
+      } else {
+        for (int b = b0; b < blocks; ++b) sum += part[b * ROWS * COLS + at];
+      }
+      total += sum;
+    }
+    const int m = m0 + at / COLS, n = n0 + at % COLS;
+    const bool own = m < M && n < N;
+    auto row = [&](int i, int k) { return A[(size_t)i * lda + k]; };
+    total = split_again(own && split_bad(total), total * SPLIT_DOWN, m, W + (size_t)n * ldw, K, row,
+                        [&](int i) { return split_undefined([&](int k) { return row(i, k); }, K); });
+    if (own) C[(size_t)m * ldc + n] = bias ? total + bias[n] : total;
   }
 }
 
@@ -306,7 +389,11 @@ static bool walk_pays(int M, int N, int K) {
 template <bool GLU>
 static void walk(hipStream_t stream, const float* A, int lda, const float* W, int ldw, const float* bias, float* C, int ldc,
                  int M, int N, int K) {
-  const int side = M <= 8 ? 8 : 16, tiles = (N + side - 1) / side, grid = walk_groups(M, K);
+  // Where the waves have many tiles and little of k each a second workgroup a CU, which splits while the first one waits (us with one, with two): 16,384 x 1,028 at 4 rows
+  // 23.0 and 19.1, 32,000 x 1,280 at one row 45 and 36, 5,000 x 1,028 10.1 and 9.0; 32,000 x 516 at 16 rows 21.1 and 18.9. But 32,000 x 1,500 44 and 43, 8,192 x 1,500 15.2 and 15.4,
+  // 3,000 x 1,280 (375 tiles) at 8 rows 8.8 and 9.8, 8,192 x 768 at 16 rows 9.6 and 10.9.
+  const int side = M <= 8 ? 8 : 16, tiles = (N + side - 1) / side, twice = tiles >= 2 * CUS && (M <= 8 ? K > 1024 && K <= 1408 : K <= 640);
+  const int most = walk_groups(M, K) * (twice ? 2 : 1), grid = tiles < most ? tiles : most;
 #define WALK(WAVES, OWN, PAIR) \
   gemm_walk_kernel<WAVES, OWN, PAIR, GLU><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles)
   if (M <= 8) {
@@ -453,6 +540,12 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles_kernel(const T* __restrict_
 // up to k = 16; 32 1.0e-7 and 4.2e-8).
 #define SHORT_K 32
 
+// Whether gemm_few_rows' waves look where k ends: less than a round of segments, or a last round of up to half of them behind at most three.
+static bool few_short(int K, int turn) {
+  const int segs = (K + SEG - 1) / SEG, rest = segs % turn;
+  return segs < turn || (rest != 0 && rest <= turn / 2 && segs < 4 * turn);
+}
+
 template <typename T, typename TW, typename TC, bool VEC>
 static void launch(hipStream_t stream, const void* A_, int lda, long long sa, const void* W_, int ldw, long long sw,
                    const float* bias, void* C_, int ldc, long long sc, int M, int N, int K, int batch) {
@@ -496,16 +589,38 @@ static void launch(hipStream_t stream, const void* A_, int lda, long long sa, co
       walk<false>(stream, A, lda, W, ldw, bias, C, ldc, M, N, K);
       return;
     }
+  // four waves a workgroup where there are many (4,096 x 48 at 130 rows, 768 workgroups, 7.3 us by eight and 6.3 by four; 8,192 x 384 at 16 rows, 512, 7.4 and 7.3)
+#define BLOCKS_(WAVES, RT, PAIR)                                                                               \
+  gemm_blocks_kernel<WAVES, RT, PAIR, VEC><<<grid, WAVES * 64, lds, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, sa, sw, sc)
+#define BLOCKS(RT, PAIR)                                                                                       \
+  do {                                                                                                         \
+    const dim3 grid((N + (PAIR ? 7 : 15)) / (PAIR ? 8 : 16), (M + 16 * RT - 1) / (16 * RT), batch);            \
+    const size_t lds = ((K + 31) / 32 + 1) / 2 * 2 * (PAIR ? 64 : 256 * RT) * sizeof(float);                   \
+    if ((long long)grid.x * grid.y * grid.z <= 640) BLOCKS_(8, RT, PAIR);                                      \
+    else BLOCKS_(4, RT, PAIR);                                                                                 \
+  } while (0)
+  if constexpr (F32)
+    if (const int rows = few_blocks_rows(M, N, K, batch)) {
+      if (rows == 8) BLOCKS(1, true);
+      else if (rows == 16) BLOCKS(1, false);
+      else if (rows == 32) BLOCKS(2, false);
+      else BLOCKS(4, false);
+      return;
+    }
+#undef BLOCKS
+#undef BLOCKS_
 #define FEW(WAVES, RT, BC, PAIR)                                                                               \
   do {                                                                                                         \
-    if (K <= (WAVES * (PAIR ? 2 : 1) - 1) * SEG) FEW_(WAVES, RT, BC, PAIR, true, false);                       \
+    if (few_short(K, WAVES * (PAIR ? 2 : 1))) FEW_(WAVES, RT, BC, PAIR, true, false);                          \
     else FEW_(WAVES, RT, BC, PAIR, false, false);                                                              \
   } while (0)
   // four waves a workgroup and 16 KB on their way in each: several workgroups share a CU and fill each other's
   // starts and ends (16,384 x 2,048 at 16 rows: 38 us; 44 with eight waves and twice the loads)
+  const bool eight = F32 && few_rows_waves(M, N, K, batch) == 8;
   if (M <= 8) FEW(4, 1, 4, true);
-  else if (M <= 16) { if (F32 && K >= 4096 && (N + 15) / 16 <= 256) FEW(8, 1, 4, false); else FEW(4, 1, 4, false); }
-  else if (M <= 32) { if (F32 && K >= 4096 && (N + 15) / 16 <= 256) FEW(8, 2, 2, false); else FEW(4, 2, 2, false); }
+  else if (M <= 16) { if (eight) FEW(8, 1, 4, false); else FEW(4, 1, 4, false); }
+  else if (M <= 32) { if (eight) FEW(8, 2, 2, false); else FEW(4, 2, 2, false); }
+  else if constexpr (F32) { if (eight) FEW(8, 4, 2, false); else FEW(4, 4, 2, false); }
   else FEW(4, 4, 2, false);
 #undef FEW_
 #undef FEW

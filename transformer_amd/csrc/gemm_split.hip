@@ -1,5 +1,6 @@
 // C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]) in 32 bits for many rows, on the 16-bit matrix instructions (split.h, which also states the
 // order of the sums: a row has the bits here that it has in the kernels for few rows).
+#include <math.h>
 #include <type_traits>
 #include "split.h"
 #include "gemm_split.h"
@@ -64,6 +65,12 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
       return *reinterpret_cast<const f32x4*>(p);
     }
     f32x4 v;
+    if (b * 32 + 32 <= K) {                            // 16 bytes from wherever they start (four loads of 4: 130 x 5,000 x 2,049 134 us)
+      typedef float any4 __attribute__((ext_vector_type(4), aligned(4)));
+      const any4 u = *reinterpret_cast<const any4*>(p);
+      v = f32x4{u[0], u[1], u[2], u[3]};
+      return v;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const char* q = b * 32 + 16 * h + 4 * kb + e < K ? p + 4 * e : reinterpret_cast<const char*>(&split_zeros);
@@ -300,7 +307,7 @@ struct SplitForm {
   float step, round;
 };
 constexpr SplitForm SPLIT_FORMS[] = {{0, 0, 0, 0.f, 0.f},      {8, 8, 1, 1.96f, 6.4f}, {4, 6, 2, 1.91f, 5.1f}, {4, 4, 2, 1.43f, 3.6f}, {2, 4, 4, 1.96f, 3.7f},
-                                     {4, 4, 1, 1.47f, 3.1f}, {2, 4, 1, 0.f, 0.f},    {2, 4, 4, 1.96f, 3.7f}, {4, 4, 1, 1.47f, 3.1f}};
+                                     {4, 4, 1, 1.47f, 3.1f}, {2, 4, 1, 1.02f, 3.6f}, {2, 4, 4, 1.96f, 3.7f}, {4, 4, 1, 1.47f, 3.1f}};
 enum { SPLIT_GROUPS = 4, SPLIT_PAIRED = 5, SPLIT_SMALL = 6, SPLIT_FAR = 3, SPLIT_CUS = 256 };      // + SPLIT_FAR: the same, rows any distance apart
 #define SPLIT_LAUNCH 2.0        // us of a launch
 #define SPLIT_ALONE 0.94        // us a step of a SPLIT_PAIRED workgroup that has its CU to itself
@@ -312,31 +319,47 @@ static long long split_tiles(int form, int M, int N) {
 static double split_cost(int form, int M, int N, int K, int batch) {
   const SplitForm& f = SPLIT_FORMS[form];
   const long long tiles = split_tiles(form, M, N) * batch;
-  const int segs = (K + SEG - 1) / SEG, steps = f.groups == 1 ? (K + 31) / 32 : (segs + f.groups - 1) / f.groups * (SEG / 32);
+  const int blocks = (K + 31) / 32, segs = (K + SEG - 1) / SEG, rounds = (segs + f.groups - 1) / f.groups;
+  const int last = segs - (rounds - 1) * f.groups > 1 ? SEG / 32 : blocks - (segs - 1) * (SEG / 32);        // as in the kernel
+  const int steps = f.groups == 1 ? blocks : (rounds - 1) * (SEG / 32) + last;
   const double round = (double)steps * f.step + f.round;
+  if (form == SPLIT_SMALL) {                           // up to four share a CU
+    const double share = (double)tiles / SPLIT_CUS, turns = share <= 4.0 ? (double)((tiles + SPLIT_CUS - 1) / SPLIT_CUS) : share;
+    return SPLIT_LAUNCH + steps * f.step + f.round + (turns - 1.0) * (0.37 * steps + 1.2);
+  }
   if (form != SPLIT_PAIRED) return SPLIT_LAUNCH + (double)((tiles + SPLIT_CUS - 1) / SPLIT_CUS) * round;
   const long long rest = tiles % (2 * SPLIT_CUS);
   return SPLIT_LAUNCH + (double)(tiles / (2 * SPLIT_CUS)) * round + (rest > SPLIT_CUS ? round : rest > 0 ? SPLIT_ALONE * steps + f.round : 0.0);
 }
 
-// the few-rows kernel's: a workgroup of 16 columns and 32 or 64 rows, four segments at a time (12 % off in the mean). Over a short k several of its workgroups
-// share a CU evenly.
+// what few rows take elsewhere. gemm_blocks: the blocks of a workgroup's waves one after the other, and all workgroups' work (10 % off in the mean).
+// gemm_few_rows: a workgroup's rounds of segments or all workgroups' work, whichever is more (14 %). What is chosen is 0.4 % from the fastest in the mean and 29 at the worst of 600 sizes.
 static double split_few_cost(int M, int N, int K, int batch) {
-  const int rows = M <= 32 ? 32 : 64, segs = (K + SEG - 1) / SEG;
-  const long long groups = (long long)((N + 15) / 16) * ((M + rows - 1) / rows) * batch;
-  const double share = segs > 4 ? (double)((groups + SPLIT_CUS - 1) / SPLIT_CUS) : groups / (double)SPLIT_CUS;
-  return 5.6 + (M <= 32 ? 5.1 : 8.4) * (share > 0.67 ? share : 0.67) * (segs < 4 ? segs / 4.0 : (segs + 3) / 4);
+  if (K <= SPLIT_BLOCKS_K) {
+    const int form = M <= 8 ? 0 : M <= 16 ? 1 : M <= 32 ? 2 : 3, rows = M <= 16 ? 16 : M <= 32 ? 32 : 64, cols = M <= 8 ? 8 : 16;
+    const double blocks = (K + 31) / 32 * (M <= 8 ? 0.5 : 1.0), share = (double)((N + cols - 1) / cols) * ((M + rows - 1) / rows) * batch / SPLIT_CUS;
+    constexpr double chain[4] = {0.7, 0.7, 1.1, 1.8}, each[4] = {0.116, 0.134, 0.183, 0.247};
+    return 2.3 + chain[form] * (int)((blocks + 7) / 8) + share * ((form == 3 ? 0.35 : 0.0) + each[form] * blocks);
+  }
+  const int segs = (K + SEG - 1) / SEG, rows = few_blocks_rows(M, N, K, batch), form = M <= 16 ? 0 : M <= 32 ? 1 : 2;
+  if (rows) {
+    const double share = (double)((N + 15) / 16) * ((M + rows - 1) / rows) * batch / SPLIT_CUS;
+    return 0.4 + (rows == 16 ? 1.2 : 1.9) * (((K + 31) / 32 + 7) / 8) + share * segs * (rows == 16 ? 0.62 : 0.47);
+  }
+  const int waves = few_rows_waves(M, N, K, batch), tile = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+  const double share = (double)((N + 15) / 16) * ((M + tile - 1) / tile) * batch / SPLIT_CUS;
+  constexpr double round4[3] = {3.8, 4.7, 8.5}, round8[3] = {7.5, 9.7, 14.7}, each[3] = {0.81, 1.42, 2.08};
+  const double chain = (waves == 4 ? round4 : round8)[form] * (segs < waves ? (double)segs / waves : (segs + waves - 1) / waves), work = (segs > 8 ? ceil(share) : share) * segs * each[form];        // (over a long k a last, partly filled round counts whole)
+  return 3.0 + cbrt(chain * chain * chain + work * work * work);
 }
 
+// Forms 1 to 4 only from k = 129 on, below which 5 and 6 start and end sooner; 6 only over a short k (12,300 x 48 at 300 rows 11.9 us, 15.3 by 5).
 extern "C" int ta_gemm_split_form(int M, int N, int K, int lda, int ldw, int batch, bool vec) {
-  const long long tiles = split_tiles(SPLIT_SMALL, M, N) * batch;
-  const bool brief = K <= 128, far = lda > 4194303 || ldw > 4194303;     // 256 rows by 32-bit offsets
-  if (tiles > 2147483640ll || (M <= 16 && !brief)) return 0;
-  // over a short k it is the start and the end that count (32 products of 1 x 512 x 64 4.4 us, 7.2 by few rows); up to 32 it is not taken here at all
-  if (brief) return tiles < 192 ? 0 : far ? SPLIT_PAIRED + SPLIT_FAR : tiles < 2 * SPLIT_CUS ? SPLIT_SMALL : SPLIT_PAIRED;
+  const bool far = lda > 4194303 || ldw > 4194303;     // 256 rows by 32-bit offsets
+  if (split_tiles(SPLIT_SMALL, M, N) * batch > 2147483640ll || (M <= 16 && K > SPLIT_BLOCKS_K)) return 0;
   int best = 0;
   double least = split_few_cost(M, N, K, batch);
-  for (int f = !vec ? SPLIT_PAIRED : far ? SPLIT_GROUPS : 1; f <= SPLIT_PAIRED; ++f) {
+  for (int f = !vec || K <= 128 ? SPLIT_PAIRED : far ? SPLIT_GROUPS : 1; f <= (K <= SPLIT_BLOCKS_K && !far ? SPLIT_SMALL : SPLIT_PAIRED); ++f) {
     const double cost = split_cost(f, M, N, K, batch);
     if (cost < least) best = f, least = cost;
   }
