@@ -1,4 +1,5 @@
-"""Which prompts' products go to the kernels for many bfloat16 rows: not those at which the vendor library was measured to be faster."""
+"""Which prompts' products go to the kernels for many bfloat16 rows, and which steps to the one for a token side input: not those at which the vendor
+library, or the kernels one by one, were measured to be faster."""
 import pytest
 
 from ctypes import c_int
@@ -31,3 +32,12 @@ def test_gated(m, n, k, takes):
     (816, 16384, 4096, False), (816, 16384, 16384, True), (8193, 4096, 14336, False), (4096, 4096, 8192, True), (3000, 4096, 14336, False), (3072, 2000, 8192, False)])
 def test_plain(m, n, k, takes):
     assert _plain(m, n, k) == takes
+
+
+@pytest.mark.parametrize("tokens,d,dim,plain,routed", [
+    (1, 4096, 32, True, True), (64, 512, 32, True, True), (65, 512, 32, False, False), (0, 512, 32, False, False), (4, 2048, 64, True, True), (4, 2560, 64, False, True),
+    (4, 4096, 64, False, False), (17, 4096, 64, True, True), (1, 1024, 128, False, True), (16, 2048, 128, False, False), (32, 2048, 128, True, True),
+    (32, 2560, 128, False, False), (64, 4096, 128, False, False), (4, 2048, 48, False, False), (4, 2000, 64, False, False), (4, 4608, 32, False, False)])
+def test_side_steps(tokens, d, dim, plain, routed):
+    pays = [bool(kernels.library().ta_side_step_pays(c_int(tokens), c_int(d), c_int(dim), c_int(r))) for r in (0, 1)]
+    assert pays == [plain, routed]

@@ -618,10 +618,17 @@ __global__ __launch_bounds__(1024) void side_step_kernel(SideStep p) {
   }
 }
 
-// Whether ta_side_step takes a step: one by one and here 17.5 / 15.8 us at one token, 17.6 / 13.7 at 4, 18.4 / 13.6 at 16, 26.8 / 13.5 at 32, 25.3 / 13.0 at 64;
-// beyond, every token's workgroup reads both matrices again, and a prompt's products share them.
-extern "C" int ta_side_step_pays(int nt, int d, int dim) {
-  return nt >= 1 && nt <= 64 && d % 512 == 0 && d <= SIDE_MAX_D && (dim == 32 || dim == 64 || dim == 128);
+// Whether ta_side_step takes a step (routed: experts' rows, whose sum is a kernel more one by one). us one by one and here, at 1 / 16 / 32 / 64 tokens, plain (routed): 32 side
+// columns 512 wide 10.2 / 11.3 / 17.6 / 18.3 and 7.8 / 8.1 / 8.1 / 8.2, 4,096 wide 14.6 / 17.0 / 21.4 / 21.8 and 11.3 / 11.6 / 11.9 / 12.1; 64 columns 2,048 wide 12.6 / 13.9 / 20.3 / 20.7 and
+// 10.7 / 11.6 / 11.7 / 11.7, 2,560 wide 13.3 / 15.5 / 19.3 / 21.1 and 13.7 / 14.4 / 14.4 / 14.3 (routed 15.6 / 17.0 and 14.4 / 15.2), 4,096 wide 15.5 / 17.4 / 21.6 / 24.6 and 16.8 / 17.7 / 17.6 / 17.4
+// (18.2 / 19.8 and 17.7 / 18.8, but 18.5 and 19.0 between). One CU takes in both matrices: 128 columns 1,024 wide 11.3 / 12.5 / 20.3 / 21.0 and 12.6 / 13.3 / 13.5 / 13.3 (13.1 / 14.6 and
+// 12.9 / 13.8), 2,048 wide 12.9 / 14.4 / 20.7 / 21.4 and 18.5 / 19.5 / 19.3 / 18.9, 4,096 wide 15.4 / 17.6 / 22.2 / 26.2 and 28.7 / 30.5 / 29.8 / 29.3. From 17 tokens on the products one
+// by one are other kernels'; beyond 64 every token's workgroup reads both matrices again, and a prompt's products share them.
+extern "C" int ta_side_step_pays(int nt, int d, int dim, int routed) {
+  if (nt < 1 || nt > 64 || d <= 0 || d % 512 != 0 || d > SIDE_MAX_D) return 0;
+  if (dim == 32) return 1;
+  if (dim == 64) return nt > 16 || d <= (routed ? 2560 : 2048);
+  return dim == 128 && (nt > 16 ? d <= 2048 : routed && d <= 1024);
 }
 
 // delta [planes, nt, d], or null and rows / top / pair_row / weight / shared [planes, nt, d] / shared_gate as in ta_moe_combine.

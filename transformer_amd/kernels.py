@@ -2250,11 +2250,12 @@ class RoutedRows:
         self.rows, self.top, self.pair_row, self.weight, self.shared, self.shared_gate = rows, int(top), pair_row, weight, shared, shared_gate
 
 
-def side_step_takes(rows: int, d: int, gate: torch.Tensor, proj: torch.Tensor) -> bool:
-    """Whether ``side_step`` takes a step of ``rows`` tokens of width d with these matrices."""
+def side_step_takes(rows: int, d: int, gate: torch.Tensor, proj: torch.Tensor, routed: bool = False) -> bool:
+    """Whether ``side_step`` is better for a step of ``rows`` tokens of width d with these matrices than its kernels one by one
+    (routed: behind a ``RoutedRows``)."""
     return gate.dtype == torch.bfloat16 and proj.dtype == torch.bfloat16 and gate.is_contiguous() and proj.is_contiguous() \
         and gate.data_ptr() % 16 == 0 and proj.data_ptr() % 16 == 0 \
-        and bool(library().ta_side_step_pays(c_int(rows), c_int(d), c_int(gate.shape[0])))
+        and bool(library().ta_side_step_pays(c_int(rows), c_int(d), c_int(gate.shape[0]), c_int(int(routed))))
 
 
 def side_step(x: torch.Tensor, delta, weight: torch.Tensor, eps: float, gate: torch.Tensor, side: torch.Tensor, proj: torch.Tensor,

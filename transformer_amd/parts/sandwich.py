@@ -44,10 +44,10 @@ class TokenSide(Part):
                             f"(columns {s.offset}..{s.offset + s.dim})")
         return rows[:, s.offset:s.offset + s.dim]
 
-    def takes_step(self, x) -> bool:
-        """Whether ``run_step`` takes this step: few bfloat16 tokens."""
+    def takes_step(self, x, routed) -> bool:
+        """Whether ``run_step`` takes this step (behind routed experts): few bfloat16 tokens, small matrices."""
         return self.dtype == torch.bfloat16 and \
-            kernels.side_step_takes(x.shape[0], x.shape[1], self.w["gate.weight"], self.w["proj.weight"])
+            kernels.side_step_takes(x.shape[0], x.shape[1], self.w["gate.weight"], self.w["proj.weight"], routed)
 
     def run_step(self, x, delta, weight, eps, ctx, next_norm=None, out=None):
         """The add in front (a sublayer's result normed with this weight and eps) and ``run`` in one kernel."""
@@ -161,9 +161,10 @@ class SandwichBlock(Part):
             add("1", delta, follow if last == "mixer" else None, True)
         else:
             add("1", delta, self.norm2, False)
-            step = self.side is not None and self.side.takes_step(x)
+            routed = isinstance(self.ffn, RoutedMLP)
+            step = self.side is not None and self.side.takes_step(x, routed)
             with span(ctx, "ffn"):
-                kw = {"combine": False} if step and isinstance(self.ffn, RoutedMLP) else {}
+                kw = {"combine": False} if step and routed else {}
                 delta, bias = self.ffn.run(h, ctx, **kw)
             if bias is not None:
                 raise PartError("a sandwich block's sublayers return no bias rows")
