@@ -6,9 +6,10 @@
 // 16 runs of 256 bytes, 4 KB, and every wave has a ring of its own of such chunks, up to 128 KB a CU on their way, that is
 // asked for across the ends of tiles. Operand layout straight from memory (gemm_walk, gemm_few_rows) touches half a line per row and
 // instruction: at 4 rows 16,384 x 2,048 gated 28.2 us there and 24.9 here (5.4 TB/s), 28,672 x 4,096 gated 88 and 80, 2,048 x 8,192 19.2 and 15.4,
-// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55 (on the float32 matrix instructions). Splitting the operands costs a kernel 0.3 to 0.9 us more
+// 4,096 x 14,336 64 and 47, 8,192 x 8,192 70 and 55 (on the float32 matrix instructions). Splitting the operands costs a kernel up to 0.9 us more
 // than those, in front of the first product and behind the last chunk: the four products of a layer of width 2,048 and 8,192 (3,072 and 2,048 x 2,048, 16,384 x 2,048 gated,
-// 2,048 x 8,192) at 1 / 4 / 8 rows 54.3 / 55.9 / 58.6 us and 56.7 / 57.7 / 60.6; it is what keeps a row's bits the same as among many, which gain more.
+// 2,048 x 8,192) at 1 / 4 / 8 rows 54.0 / 55.6 / 58.5 us on the float32 instructions, 57.7 / 58.2 / 60.8 with A split by every lane and 55.1 / 56.5 / 61.1 with half of it (HALF); it is what
+// keeps a row's bits the same as among many, which gain more.
 //
 // A product may take the RMS norm in front of it (its workgroups form the rows' factors once more each, which costs 1 to 3 us
 // where the norm's own launch costs 4 to 5), and add its result to the residual stream where it stores it.
@@ -33,7 +34,10 @@ struct StreamNorm {
 // workgroups of 4 waves a CU or one of 8. A (and the norm's weight and rows) come behind the first two chunks of W and in front of the
 // others: behind all of them they would be there only when those are, in front of all of them memory would wait for them (the norm's
 // rows by waves of their own: 16,384 x 2,048 33 us instead of 27).
-template <int WAVES, int PF, bool GLU, bool NORM, bool TAIL>
+//
+// HALF (up to 4 rows): rows 4 to 7 of the instruction hold the other half of rows 0 to 3, so that a lane reads, norms and splits half as much of A
+// and gets the rest from its neighbour; what those rows then multiply is never stored.
+template <int WAVES, int PF, bool GLU, bool NORM, bool TAIL, bool HALF>
 __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float* __restrict__ A, int lda,
                                                                  const float* __restrict__ W, int ldw,
                                                                  const float* __restrict__ bias, float* __restrict__ C, int ldc,
@@ -89,15 +93,16 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
 #pragma unroll
   for (int s = 0; s < EARLY; ++s) request(s);
 
-  // the lane's part of A, row r % 8, segment 2 wave + r / 8
-  const int m_a = r % 8 < M ? r % 8 : 0;
+  // the lane's part of A, row r % 8, segment 2 wave + r / 8, PIECES of a chunk's four from piece half on
+  constexpr int ROWS = HALF ? 4 : 8, PIECES = HALF ? 2 : 4;
+  const int m_a = r % ROWS < M ? r % ROWS : 0, half = HALF ? r / 4 % 2 * 2 : 0;
   const float* arow = A + (size_t)m_a * lda;
-  f32x4 a[CH * 4], g[NORM ? CH * 4 : 1], v[NORM ? 4 : 1][4];
+  f32x4 a[CH * PIECES], g[NORM ? CH * PIECES : 1], v[NORM ? ROWS / 2 : 1][4];
   constexpr int T = WAVES * 32;                  // threads a row: add_rmsnorm's, 4 vectors of 4 each
   const int side = threadIdx.x / T, at = threadIdx.x % T;
   if (NORM) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int p = 0; p < ROWS / 2; ++p)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int m = 2 * p + side, c = 4 * (at + u * T);
@@ -105,8 +110,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
       }
   }
 #pragma unroll
-  for (int i = 0; i < CH * 4; ++i) {
-    const int k = (2 * wave + r / 8) * SEG + i * BLK + 4 * kb;
+  for (int i = 0; i < CH * PIECES; ++i) {
+    const int k = (2 * wave + r / 8) * SEG + (i / PIECES * 4 + half + i % PIECES) * BLK + 4 * kb;
     a[i] = *(k < K ? reinterpret_cast<const f32x4*>(arow + k) : zeros);
     if (NORM) g[i] = *(k < K ? reinterpret_cast<const f32x4*>(nm.w + k) : zeros);
   }
@@ -114,7 +119,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
   // do not count those (a value that has been through an asm statement is waited for there).
   auto arrive = [](f32x4& x) { asm volatile("" : "+v"(x)); };
 #pragma unroll
-  for (int i = 0; i < CH * 4; ++i) {
+  for (int i = 0; i < CH * PIECES; ++i) {
     arrive(a[i]);
     if (NORM) arrive(g[i]);
     if (NORM) arrive(v[i / 4][i % 4]);
@@ -123,7 +128,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
   for (int s = EARLY; s < PF; ++s) request(s);
   if (NORM) {
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < ROWS / 2; ++p) {
       float ss = 0.f;
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -138,7 +143,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
     for (int i = 0; i < WAVES / 2; ++i) tot += sq[m_a][i];
     const float rstd = 1.0f / sqrtf(tot / (float)K + nm.eps);
 #pragma unroll
-    for (int i = 0; i < CH * 4; ++i)
+    for (int i = 0; i < CH * PIECES; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[i][e] = a[i][e] * rstd * g[i][e];
   }
@@ -151,7 +156,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const float*
       if (first) {                               // while the chunk is on its way
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) as[2 * c + i] = split8(a[4 * c + 2 * i], a[4 * c + 2 * i + 1]);
+        for (int i = 0; i < PIECES / 2; ++i) as[2 * c + i] = split8(a[PIECES * c + 2 * i], a[PIECES * c + 2 * i + 1]);
+        if (HALF) as[2 * c + 1] = split_next4(as[2 * c]);
         __builtin_amdgcn_sched_barrier(0);
       }
       ta_wait_loads<(PF - 1) * 4>();
@@ -255,6 +261,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
 #pragma unroll
   for (int s = 0; s < PF; ++s) request(s);
   const int arow = r / 8 * (2 * MR) + r % 8 % (2 * MR);
+  constexpr bool HALF = MR <= 2;                 // as above
+  const int half = HALF ? r / 4 % 2 * 2 : 0;
   const int m = lane / 8, n = 8 * blockIdx.x + lane % 8;
   float total = 0.f;
   int slot = 0;
@@ -267,14 +275,16 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_stream_long_kernel(const floa
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         w[i] = *reinterpret_cast<const f32x4*>(&ring[wave][slot][r * 64 + ((4 * i + kb) ^ r) * 4]);
-        a[i] = *reinterpret_cast<const f32x4*>(&ring[wave][slot][1024 + arow * 64 + ((4 * i + kb) ^ arow) * 4]);
+        if (i < 2 || !HALF) a[i] = *reinterpret_cast<const f32x4*>(&ring[wave][slot][1024 + arow * 64 + ((4 * (half + i) + kb) ^ arow) * 4]);
+        else a[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
       asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3])::"memory");
       asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])::"memory");
       request(slot);
       slot = slot + 1 == PF ? 0 : slot + 1;
-#pragma unroll
-      for (int i = 0; i < 4; i += 2) acc += split_block(split8(w[i], w[i + 1]), split8(a[i], a[i + 1]));
+      const Split8 first = split8(a[0], a[1]);
+      acc += split_block(split8(w[0], w[1]), first);
+      acc += split_block(split8(w[2], w[3]), HALF ? split_next4(first) : split8(a[2], a[3]));
     }
     auto* to = part[round & 1];
     if (kb / 2 == r / 8) *reinterpret_cast<f32x4*>(&to[2 * wave + r / 8][(r % 8) * 8 + 4 * (kb % 2)]) = acc;
@@ -343,11 +353,14 @@ extern "C" int ta_gemm_stream(hipStream_t stream, const float* A, int lda, const
   }
   const int most = K <= 2048 ? 512 : 256, grid = tiles < most ? tiles : most;
   const StreamNorm nm = {norm_w, eps};
+#define RUN_(WAVES, GLU, NORM, TAIL, HALF)                                                                        \
+  gemm_stream_kernel<WAVES, 4, GLU, NORM, TAIL, HALF><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles, add, nm)
 #define RUN(WAVES, GLU, NORM)                                                                                     \
-  if (K % (2 * WAVES * SEG) == 0)                                                                                 \
-    gemm_stream_kernel<WAVES, 4, GLU, NORM, false><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles, add, nm); \
-  else                                                                                                            \
-    gemm_stream_kernel<WAVES, 4, GLU, NORM, true><<<grid, WAVES * 64, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, tiles, add, nm)
+  if (K % (2 * WAVES * SEG) == 0) {                                                                               \
+    if (M <= 4) RUN_(WAVES, GLU, NORM, false, true); else RUN_(WAVES, GLU, NORM, false, false);                   \
+  } else {                                                                                                        \
+    if (M <= 4) RUN_(WAVES, GLU, NORM, true, true); else RUN_(WAVES, GLU, NORM, true, false);                     \
+  }
 #define PICK(WAVES)                                                                                        \
   do {                                                                                                     \
     if (glu) { if (norm_w) { RUN(WAVES, true, true); } else { RUN(WAVES, true, false); } }                 \
@@ -356,5 +369,6 @@ extern "C" int ta_gemm_stream(hipStream_t stream, const float* A, int lda, const
   if (K <= 2048) PICK(4); else PICK(8);
 #undef PICK
 #undef RUN
+#undef RUN_
   return ta_check_launch("ta_gemm_stream");
 }

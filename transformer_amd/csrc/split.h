@@ -31,6 +31,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct Split8 {
   bf16x8 h, m, l;
 };
+static_assert(sizeof(Split8) == 48, "twelve registers");
 
 // What is split is x 2^16, exactly, so that l has a bfloat16 down to the smallest float32 there is (bfloat16 ends at 2^-133: without, numbers
 // below 2^-110 would lose bits); a product is therefore 2^32 too large, and every kernel takes that out of its last sum.
@@ -58,6 +59,16 @@ __device__ __forceinline__ Split8 split8(const f32x4& x, const f32x4& y) {
     l[i] = tops(__float_as_uint(ra - cut(ma)), __float_as_uint(rb - cut(mb)));
   }
   return s;
+}
+
+// the numbers of the lane 4 further on in the row of 16
+__device__ __forceinline__ Split8 split_next4(const Split8& x) {
+  Split8 y;
+  const int *from = reinterpret_cast<const int*>(&x);
+  int* to = reinterpret_cast<int*>(&y);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) to[i] = __builtin_amdgcn_update_dpp(0, from[i], 0x104, 0xf, 0xf, true);
+  return y;
 }
 
 // step i (0 .. 5) of a block's chain
