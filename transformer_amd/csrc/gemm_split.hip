@@ -301,7 +301,7 @@ __global__ __launch_bounds__(WAVES * G * 64, 2) void gemm_split_kernel(const flo
 // columns, k from 256 to 14,336, to 5 to 8 %. 256 x 128 reads and splits least per product but leaves CUs idle where there are few tiles: 16,384 x 2,048 at 1,021 rows
 // 310 us there and 390 by 128 x 64, at 130 rows 132 and 105; 4,096 x 1,024 at 700 rows 70 and 51. Groups fill a CU that has a tile to itself: 2,048 x 8,192 at 1,021 rows 214 us by two,
 // 6,144 x 8,192 at 64 rows 248 by one, 172 by two, 129 by four on 64 x 64. Two workgroups of 128 x 64 with one group share a CU.
-// Of 800 sizes the costs choose the fastest form to 0.6 % in the mean, 18 at the worst (8,192 x 1,024 at 33 rows: 21 us for 18).
+// With split_few_cost they choose, of 633 sizes of 17 to 513 rows and k from 516, the fastest way to 0.5 % in the mean, 29 at the worst (16,384 x 516 at 17 rows: 20 us for 16).
 struct SplitForm {
   int waves, nt, groups;
   float step, round;
@@ -333,7 +333,7 @@ static double split_cost(int form, int M, int N, int K, int batch) {
 }
 
 // what few rows take elsewhere. gemm_blocks: the blocks of a workgroup's waves one after the other, and all workgroups' work (10 % off in the mean).
-// gemm_few_rows: a workgroup's rounds of segments or all workgroups' work, whichever is more (14 %). What is chosen is 0.4 % from the fastest in the mean and 29 at the worst of 600 sizes.
+// gemm_few_rows: a workgroup's rounds of segments or all workgroups' work, whichever is more (14 %).
 static double split_few_cost(int M, int N, int K, int batch) {
   if (K <= SPLIT_BLOCKS_K) {
     const int form = M <= 8 ? 0 : M <= 16 ? 1 : M <= 32 ? 2 : 3, rows = M <= 16 ? 16 : M <= 32 ? 32 : 64, cols = M <= 8 ? 8 : 16;
